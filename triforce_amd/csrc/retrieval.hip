@@ -56,6 +56,56 @@ __global__ __launch_bounds__(256) void retrieval_score_kernel(const h16* __restr
     }
 }
 
+// The same for chunks of CH rows (known at compile time): a group's next chunk is requested before the current one is summed up, so
+// that a few resident waves keep the stream going.  A plain read is fastest on this chip with about 32 KB in flight per CU and loses
+// 10-25 % at half or at several times that; the general kernel above holds 8 workgroups per CU with 8 KB per wave.
+template <int D, int CH>
+__global__ __launch_bounds__(256) void retrieval_score_ahead_kernel(const h16* __restrict__ k, int64_t stride_t,
+                                                                    int64_t stride_h, const h16* __restrict__ q,
+                                                                    h16* __restrict__ scores, int C) {
+    constexpr int LPR = D / 8, GPB = 256 / LPR;
+    const int h = blockIdx.y;
+    const int grp = threadIdx.x / LPR, li = threadIdx.x % LPR;
+    const h16* kb = k + (int64_t)h * stride_h + 8 * li;
+    float qf[8];
+    {
+        const half8 qv = load_half8(q + (int64_t)h * D + 8 * li);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) qf[e] = (float)qv[e];
+    }
+    const float inv = 1.0f / (float)CH;
+    const int step = gridDim.x * GPB;
+    auto fetch = [&](half8 (&r)[CH], int c) {                    // (past the end: the last chunk again, not used)
+        const h16* kp = kb + (int64_t)min(c, C - 1) * CH * stride_t;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) r[j] = load_half8_stream(kp + (int64_t)j * stride_t);
+    };
+    auto score = [&](const half8 (&r)[CH], int c) {
+        float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {                           // sequential fp32 accumulation over the chunk rows
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] += (float)r[j][e];
+        }
+        float dot = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot = fmaf(qf[e], (float)(h16)(acc[e] * inv), dot);
+#pragma unroll
+        for (int o = LPR / 2; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64);
+        if (li == 0 && c < C) scores[(int64_t)h * C + c] = (h16)dot;
+    };
+    half8 a[CH], b[CH];
+    const int c0 = blockIdx.x * GPB;                             // (uniform bound: the waves of a workgroup go together)
+    fetch(a, c0 + grp);
+    for (int c = c0; c < C; c += 2 * step) {
+        fetch(b, c + grp + step);
+        score(a, c + grp);
+        if (c + step >= C) break;
+        fetch(a, c + grp + 2 * step);
+        score(b, c + grp + step);
+    }
+}
+
 // ---- per-head top-k: full bitonic sort of (score, chunk) keys in LDS ------------------------
 __device__ __forceinline__ uint32_t sortable_fp16(uint32_t b) {
     return (b & 0x8000u) ? ((~b) & 0xFFFFu) : (b | 0x8000u);
@@ -96,81 +146,154 @@ __global__ __launch_bounds__(1024) void retrieval_topk_kernel(const uint16_t* __
 }
 
 // ---- per-head top-k, select-then-sort form ---------------------------------------------------
-// The keys are distinct 32-bit integers, so the m-th largest one is found EXACTLY by a 4-pass radix select
-// (8 bits per pass, one 256-bin LDS histogram each, integer atomics: deterministic), the m keys >= it are compacted
-// and only those are bitonic-sorted: for cfg2 (m = 511 of 15 615) 4 histogram passes + 45 passes over 512 keys
-// instead of 105 passes over 16 384 keys (213 us -> ~25 us per layer).  Same output, bit for bit, as the full sort.
+// The keys are distinct 32-bit integers, so the m-th largest one is found EXACTLY by a radix select (integer histograms in LDS:
+// deterministic), the m keys >= it are compacted and only those are sorted.  Same output, bit for bit, as the full sort.
+//
+// One workgroup per head; a latency chain, not a bandwidth one (15 615 keys are 31 KB), so every serial piece is what counts:
+//   * three passes of 11 / 11 / 10 bits instead of four of 8: 2 048 bins spread a head's scores (an fp16's sign, exponent and
+//     five mantissa bits) where 256 bins made the waves queue on a handful of LDS counters;
+//   * the bin that holds the m-th key is found by one wave with two 64-wide scans (one lane walking the bins from the top was
+//     the longest piece of the kernel);
+//   * bitonic stages below 64 exchange inside a wave, so 512 winners meet 6 barrier-separated stages of 45.
+// 32 heads x 15 616 chunks, m = 511: 46.9 -> 16.9 us.
+constexpr int kTopkBins = 2048;
+__device__ __forceinline__ int topk_bin(int b) { return b + (b >> 5); }      // (a lane sums 32 neighbouring bins: no bank twice)
+
+// The digit (of `bins` of them) at which the count from the top reaches `rem`, and what is left to find inside it.  One wave.
+__device__ __forceinline__ void topk_digit(const int* hist, int bins, int rem, int lane, int* digit, int* left) {
+    const int per = bins >> 6;                                           // 32 or 16
+    int own = 0;
+    for (int j = 0; j < per; ++j) own += hist[topk_bin(bins - 1 - (lane * per + j))];
+    int upto = own;                                                      // inclusive count of the lanes before (higher digits)
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(upto, o, 64);
+        if (lane >= o) upto += t;
+    }
+    const int owner = __ffsll((long long)__ballot(upto >= rem)) - 1;     // (rem <= keys in the histogram: some lane reaches it)
+    const int before = __shfl(upto - own, owner, 64);
+    const int cnt = lane < per ? hist[topk_bin(bins - 1 - (owner * per + lane))] : 0;
+    int in = cnt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(in, o, 64);
+        if (lane >= o) in += t;
+    }
+    const int at = __ffsll((long long)__ballot(before + in >= rem)) - 1;
+    *digit = bins - 1 - (owner * per + at);
+    *left = rem - before - __shfl(in - cnt, at, 64);
+}
+
+// E = winners per thread (the sort's size / 1024, at least 1): element e * 1024 + tid sits in register e of thread tid, so stages
+// below 64 are lane exchanges, stages of 1024 and more are register exchanges and only those between go through LDS.
+template <int E>
 __global__ __launch_bounds__(1024) void retrieval_topk_select_kernel(const uint16_t* __restrict__ scores,
                                                                       int32_t* __restrict__ idx, int C, int sets,
                                                                       int n, int mpow2) {
     extern __shared__ uint32_t smem_u[];
     uint32_t* keys = smem_u;                 // [n]   candidate keys (chunks 1..C-1)
-    uint32_t* sel = smem_u + n;              // [mpow2] the winners, then sorted in place
-    __shared__ int hist[256];
+    uint32_t* sel = smem_u + n;              // [mpow2] the winners
+    __shared__ int hist[kTopkBins + kTopkBins / 32];
     __shared__ uint32_t s_prefix;
     __shared__ int s_remaining, s_count;
-    const int h = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;
+    const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    constexpr int nt = 1024;
     const uint16_t* sc = scores + (int64_t)h * C;
     const int m = sets - 1;
+    int32_t* out = idx + (int64_t)h * sets;
+    if (tid == 0) out[0] = 0;
+    if (m == 0) return;
+#pragma unroll 8
     for (int i = tid; i < n; i += nt) {
         const int c = i + 1;
         keys[i] = (sortable_fp16(sc[c]) << 16) | (uint32_t)(65535 - (c & 0xFFFF));
     }
     for (int i = tid; i < mpow2; i += nt) sel[i] = 0u;                   // padding sorts last
     if (tid == 0) { s_prefix = 0u; s_remaining = m; s_count = 0; }
-    __syncthreads();
-    if (m > 0) {
-        for (int pass = 0; pass < 4; ++pass) {
-            const int shift = 24 - 8 * pass;
-            const uint32_t pmask = pass == 0 ? 0u : (0xFFFFFFFFu << (shift + 8));
-            if (tid < 256) hist[tid] = 0;
-            __syncthreads();
-            const uint32_t prefix = s_prefix;
-            for (int i = tid; i < n; i += nt) {
-                const uint32_t k = keys[i];
-                if ((k & pmask) == prefix) atomicAdd(&hist[(k >> shift) & 255u], 1);
-            }
-            __syncthreads();
-            if (tid == 0) {                                              // digit of the remaining-th largest key
-                int rem = s_remaining, b = 255, cum = 0;
-                for (; b > 0; --b) {
-                    if (cum + hist[b] >= rem) break;
-                    cum += hist[b];
-                }
-                s_remaining = rem - cum;
-                s_prefix = prefix | ((uint32_t)b << shift);
-            }
-            __syncthreads();
-        }
-        const uint32_t T = s_prefix;                                     // the m-th largest key (keys are distinct)
+    uint32_t prefix = 0u, known = 0u;                                    // the bits of the m-th key found so far
+#pragma unroll
+    for (int pass = 0; pass < 3; ++pass) {
+        const int shift = pass == 0 ? 21 : (pass == 1 ? 10 : 0), bins = pass == 2 ? 1024 : kTopkBins;
+        for (int i = tid; i < kTopkBins + kTopkBins / 32; i += nt) hist[i] = 0;
+        __syncthreads();
+#pragma unroll 4
         for (int i = tid; i < n; i += nt) {
             const uint32_t k = keys[i];
-            if (k >= T) {
-                const int p = atomicAdd(&s_count, 1);
-                if (p < mpow2) sel[p] = k;
+            if ((k & known) == prefix) atomicAdd(&hist[topk_bin((k >> shift) & (bins - 1))], 1);
+        }
+        __syncthreads();
+        if (tid < 64) {
+            int digit, left;
+            topk_digit(hist, bins, s_remaining, lane, &digit, &left);
+            if (tid == 0) {
+                s_remaining = left;
+                s_prefix = prefix | ((uint32_t)digit << shift);
             }
         }
         __syncthreads();
-        for (int kk = 2; kk <= mpow2; kk <<= 1) {
-            for (int j = kk >> 1; j > 0; j >>= 1) {
-                for (int i = tid; i < mpow2; i += nt) {
-                    const int ixj = i ^ j;
-                    if (ixj > i) {
-                        const bool desc = ((i & kk) == 0);
-                        const uint32_t a = sel[i], b = sel[ixj];
-                        if ((a < b) == desc) {
-                            sel[i] = b;
-                            sel[ixj] = a;
+        prefix = s_prefix;
+        known |= (uint32_t)(bins - 1) << shift;
+    }
+#pragma unroll 4
+    for (int i = tid; i < n; i += nt) {                                  // prefix is the m-th largest key (keys are distinct)
+        const uint32_t k = keys[i];
+        if (k >= prefix) {
+            const int p = atomicAdd(&s_count, 1);
+            if (p < mpow2) sel[p] = k;
+        }
+    }
+    __syncthreads();
+    uint32_t v[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) v[e] = e * nt + tid < mpow2 ? sel[e * nt + tid] : 0u;
+    for (int kk = 2; kk <= mpow2; kk <<= 1) {
+        int j = kk >> 1;
+        if constexpr (E > 1) {
+            for (; j >= nt; j >>= 1) {                                   // both elements of a pair sit in this thread
+                const int je = j / nt;
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+#pragma unroll
+                    for (int f = e + 1; f < E; ++f) {
+                        if ((e ^ f) == je) {
+                            const bool desc = ((e * nt + tid) & kk) == 0;
+                            const uint32_t a = v[e], b = v[f];
+                            v[e] = (a < b) == desc ? b : a;
+                            v[f] = (a < b) == desc ? a : b;
                         }
                     }
                 }
-                __syncthreads();
+            }
+        }
+        for (; j >= 64; j >>= 1) {                                       // other waves hold the partners
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                if (e * nt + tid < mpow2) sel[e * nt + tid] = v[e];
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = e * nt + tid;
+                if (i < mpow2) {
+                    const uint32_t b = sel[i ^ j];
+                    const bool larger = ((i & kk) == 0) == ((i & j) == 0);   // this place keeps the larger key of the pair
+                    v[e] = larger ? max(v[e], b) : min(v[e], b);
+                }
+            }
+        }
+        for (; j > 0; j >>= 1) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int i = e * nt + tid;
+                const uint32_t b = __shfl_xor(v[e], j, 64);
+                const bool larger = ((i & kk) == 0) == ((i & j) == 0);
+                v[e] = larger ? max(v[e], b) : min(v[e], b);
             }
         }
     }
-    int32_t* out = idx + (int64_t)h * sets;
-    if (tid == 0) out[0] = 0;
-    for (int i = tid; i < m; i += nt) out[1 + i] = 65535 - (int32_t)(sel[i] & 0xFFFFu);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+        if (e * nt + tid < m) out[1 + e * nt + tid] = 65535 - (int32_t)(v[e] & 0xFFFFu);
 }
 
 // ---- gather ---------------------------------------------------------------------------------
@@ -251,6 +374,18 @@ extern "C" int tf_retrieval_score(const void* k, int64_t stride_t, int64_t strid
 #endif
     if (gx > cap) gx = cap;
     if (gx < 1) gx = 1;
+    if (D == 128 && chunk == 8) {
+        // Workgroups per CU.  One (16 KB asked for ahead of 16 KB in use per wave quartet) is the best stream where every CU gets the
+        // same share and enough of it to pay for its start: 32 x 15 616 chunks 158.3 us at the general kernel's 8, 155.4 at two,
+        // 150.2 at one (6.81 TB/s); 40 heads (240 of 256 CUs with work) 198 / 194 / 199, 32 x 4 000 46.4 / 42.0 / 43.1,
+        // 32 x 1 000 12.6 / 12.1 / 13.0, 5 x 5 003 10.3 / 10.3 / 11.0.
+        const bool one = 256 % H == 0 && (int64_t)C * H >= (1 << 18);
+        const int room = one ? 256 : 512, few = H <= room ? room / H : 1;
+        hipLaunchKernelGGL((retrieval_score_ahead_kernel<128, 8>), dim3(gx < few ? gx : few, H), dim3(256), 0, st, (const h16*)k,
+                           stride_t, stride_h, (const h16*)q, (h16*)scores, C);
+        TF_LAUNCH_CHECK();
+        return TF_OK;
+    }
     if (D == 128)
         hipLaunchKernelGGL((retrieval_score_kernel<128>), dim3(gx, H), dim3(256), 0, st, (const h16*)k, stride_t,
                            stride_h, (const h16*)q, (h16*)scores, C, chunk);
@@ -263,27 +398,38 @@ extern "C" int tf_retrieval_score(const void* k, int64_t stride_t, int64_t strid
     return TF_OK;
 }
 
+template <int E>
+static int launch_topk_select(const void* scores, int32_t* idx, int C, int sets, int H, int mpow2, size_t lds, void* stream) {
+    if (lds > 48 * 1024) {
+        static bool raised = false;
+        if (!raised) {
+            hipError_t e = hipFuncSetAttribute((const void*)retrieval_topk_select_kernel<E>,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
+            if (e != hipSuccess) return (int)e;
+            raised = true;
+        }
+    }
+    hipLaunchKernelGGL((retrieval_topk_select_kernel<E>), dim3(H), dim3(1024), lds, (hipStream_t)stream,
+                       (const uint16_t*)scores, idx, C, sets, C - 1, mpow2);
+    TF_LAUNCH_CHECK();
+    return TF_OK;
+}
+
 extern "C" int tf_retrieval_topk(const void* scores, int32_t* idx, int C, int sets, int H, void* stream) {
     if (!scores || !idx || C < 2 || sets < 1 || sets > C || H < 1) return TF_EINVAL;
     if (C > 32768) return TF_ERANGE;
     // select-then-sort when candidates + winners fit in LDS together (always for the paper's shapes)
-    int mpow2 = 2;
+    int mpow2 = 64;
     while (mpow2 < sets - 1) mpow2 <<= 1;
     const size_t lds_sel = (size_t)((C - 1) + mpow2) * sizeof(uint32_t);
     if (lds_sel <= 150 * 1024 && mpow2 <= 8192) {
-        if (lds_sel > 48 * 1024) {
-            static bool raised_sel = false;
-            if (!raised_sel) {
-                hipError_t e = hipFuncSetAttribute((const void*)retrieval_topk_select_kernel,
-                                                   hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
-                if (e != hipSuccess) return (int)e;
-                raised_sel = true;
-            }
+        const int per_thread = mpow2 <= 1024 ? 1 : mpow2 / 1024;
+        switch (per_thread) {
+            case 1: return launch_topk_select<1>(scores, idx, C, sets, H, mpow2, lds_sel, stream);
+            case 2: return launch_topk_select<2>(scores, idx, C, sets, H, mpow2, lds_sel, stream);
+            case 4: return launch_topk_select<4>(scores, idx, C, sets, H, mpow2, lds_sel, stream);
+            default: return launch_topk_select<8>(scores, idx, C, sets, H, mpow2, lds_sel, stream);
         }
-        hipLaunchKernelGGL(retrieval_topk_select_kernel, dim3(H), dim3(1024), lds_sel, (hipStream_t)stream,
-                           (const uint16_t*)scores, idx, C, sets, C - 1, mpow2);
-        TF_LAUNCH_CHECK();
-        return TF_OK;
     }
     int npow2 = 2;
     while (npow2 < C - 1) npow2 <<= 1;
