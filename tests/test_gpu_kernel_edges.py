@@ -43,3 +43,52 @@ def test_retrieval_score_chunks_of_eight(H, C, token_major):
     # 128 fp32 products and sums, then one rounding to fp16
     bound = (mean * q[:, None].double()).abs().sum(-1) * 128 * 2.0 ** -24 + want.abs() * 2.0 ** -11 + 2.0 ** -24
     assert ((got.double() - want).abs() <= bound).all()
+
+
+def _attention64(q, k, v, scale):
+    """Causal attention of the last rows in float64: q (n, H, D), k / v (H, m, D) -> out and sum of weight x |value|, per head."""
+    n, m = q.shape[0], k.shape[1]
+    hidden = torch.arange(m, device=q.device)[None] > torch.arange(m - n, m, device=q.device)[:, None]
+    out, size = [], []
+    for h in range(q.shape[1]):
+        w = torch.softmax((q[:, h].double() @ k[h].double().T * scale).masked_fill(hidden, float("-inf")), -1)
+        out.append(w @ v[h].double())
+        size.append(w @ v[h].double().abs())
+    return torch.stack(out, 1), torch.stack(size, 1)
+
+
+# row blocks of 128: one row more, whole, one short; slabs of 64 keys: partial and whole; one split (output written by the kernel) and
+# several (merged); scores that rise with the key (the running maximum moves in every slab); rows H * D apart
+@pytest.mark.parametrize("n,past,H,token_major,rising", [(129, 0, 8, False, False), (256, 63, 8, False, True), (383, 1, 3, True, False), (200, 2000, 8, True, False),
+                                                         (1000, 129, 16, False, False), (2049, 0, 32, False, True), (4096, 5, 8, False, False),
+                                                         (130, 9000, 5, False, False)])
+def test_prefill_attention_blocks_and_splits(n, past, H, token_major, rising):
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n)
+    m, D, scale = past + n, 128, 0.08837890625
+    k, v = (torch.randn(m + 7, H, D, generator=g, device=DEV, dtype=torch.float16) for _ in range(2))
+    q = torch.randn(n, H, D, generator=g, device=DEV, dtype=torch.float16)
+    if rising:
+        k = (k + q.mean(0) * 20 * torch.linspace(0, 1, m + 7, device=DEV)[:, None, None]).half()
+    k[m:], v[m:] = float("nan"), float("nan")                   # behind the keys: never read
+    kc, vc = (t.transpose(0, 1) if token_major else t.transpose(0, 1).contiguous() for t in (k, v))
+    got = ops.attn_prefill(q, kc, vc, m, scale).view(n, H, D).double()
+    want, size = _attention64(q, kc[:, :m], vc[:, :m], scale)
+    # weights are rounded to fp16 (2^-11 of each, numerator and sum are not rounded alike), scores and sums are fp32
+    bound = 2.0 ** -10 * size + 2.0 ** -11 * want.abs() + 1e-6
+    assert ((got - want).abs() <= bound).all()
+
+
+def test_prefill_attention_rows_far_apart():
+    """Cache rows 2^25 elements apart: past the 32-bit offsets of a slab, so the chunk goes block by block."""
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(5)
+    n, m, D, gap = 130, 131, 128, 1 << 25
+    store = torch.empty((m - 1) * gap + 2 * D, device=DEV, dtype=torch.float16)
+    k, v = (store.as_strided((1, m, D), (D, gap, 1), at) for at in (0, D))
+    k.normal_(generator=g)
+    v.normal_(generator=g)
+    q = torch.randn(n, 1, D, generator=g, device=DEV, dtype=torch.float16)
+    got = ops.attn_prefill(q, k, v, m, 0.088).view(n, 1, D).double()
+    want, size = _attention64(q, k, v, 0.088)
+    assert ((got - want).abs() <= 2.0 ** -10 * size + 2.0 ** -11 * want.abs() + 1e-6).all()

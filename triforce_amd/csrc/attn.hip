@@ -1420,9 +1420,17 @@ __global__ __launch_bounds__(256, TREE ? TF_BLOCK_TREE_OCC : 2) void attn_block_
 // 424 TF/s), so K and V come in by LDS-DMA — `global_load_lds_dwordx4`: one instruction of a wave moves 64 x 16 B straight
 // into 1 KiB of LDS, lane-linear, no staging registers and no ds_write; the XOR swizzle of the layout is applied on the
 // SOURCE side (the lane that fills slot j of row r loads chunk j ^ f(r): the swizzles are involutions).
-// 1024-row chunk x 124 928 keys x 32 heads, same box (profiles/r03_prefill_slab_ab.jsonl): 792.7 -> 848.4 TF/s (+7 %; +10.5 %
-// on a slower box).  Splitting the softmax so that the compiler interleaves the next slab's QK^T MFMAs with this slab's exps
-// INSIDE one wave measured slower (820.5): what overlaps the matrix core with the VALU here is the other wave of the SIMD.
+// (1024-row chunk x 124 928 keys x 32 heads: 792.7 -> 848.4 TF/s, profiles/r03_prefill_slab_ab.jsonl.)
+// What bounds it: power first.  On random data the chip holds 1.67 GHz here (2.24 GHz in the merge kernel next to it; a library
+// GEMM of this type runs at 1.62 GHz), on zeros the same launch is 1.3 times as fast, and the matrix cores are busy 47 % of the
+// cycles.  So what counts is work that can be left out rather than overlap: the exponentials of a slab placed beside the next
+// slab's products by hand (907 TF/s), a wave priority for the products (925) and deeper or shallower fragment look-ahead (914-931)
+// are all within the noise of each other, while these helped (4096 rows x 65 536 keys x 32 heads):
+//   * addresses of the LDS-DMA from a scalar slab pointer and 32-bit lane offsets, fragment addresses by one XOR per tile, one
+//     code path for masked and unmasked slabs (scores outside set to -inf): 1 650 -> 1 000 VALU cycles per slab; 864 -> 915 TF/s;
+//   * fragments read 4 (K) and 8 (V) steps ahead in a fixed order: 915 -> 930;
+//   * one split (every chunk of more than 2 000 rows): the output is written here instead of partials for the merge kernel, and the
+//     longest row blocks start first: 3 100 rows without a past 205 -> 134 us, 4 096 rows behind 4 096 608 -> 486 us.
 // D = 128, chain (non-tree) form only; 0 = the shared body (attn_block_lds_body).
 #ifndef TF_PREFILL_AHEAD
 #define TF_PREFILL_AHEAD 1
@@ -1430,15 +1438,15 @@ __global__ __launch_bounds__(256, TREE ? TF_BLOCK_TREE_OCC : 2) void attn_block_
 template <int D>
 __device__ __forceinline__ void attn_prefill_ahead_body(
     const h16* __restrict__ q, const h16* __restrict__ k, const h16* __restrict__ v, int64_t stride_t,
-    int64_t stride_h, int sq, int sk, int H, float scale, int nsplit, float* __restrict__ ws, int split, int h,
-    int s_begin, int s_end) {
+    int64_t stride_h, int sq, int sk, int H, float scale, int nsplit, float* __restrict__ ws, h16* __restrict__ out, int split,
+    int h, int s_begin, int s_end) {
     static_assert(BlkLayout<D>::TR && BLK_SLAB == 64, "swizzled-K / transpose-read layout, 64-key slabs");
     constexpr int NC = D / 32, NT = D / 16, QT = 2, QR = 128, SLAB = BLK_SLAB, RS = BlkLayout<D>::RS;
     constexpr int VPR = D / 8, RPP = 256 / VPR, NPASS = SLAB / RPP;
     extern __shared__ __attribute__((aligned(16))) unsigned char blk_smem[];
     h16* sK = reinterpret_cast<h16*>(blk_smem);             // [2][SLAB * RS]
     h16* sVt = sK + 2 * BlkLayout<D>::K_HALFS;              // [2][SLAB * D]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, g = lane >> 4;
     const int qbase = wave * 32;
 
@@ -1458,59 +1466,88 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
     }
     const h16* kbase = k + (int64_t)h * stride_h;
     const h16* vbase = v + (int64_t)h * stride_h;
-    const TreeMask tm{nullptr, 0, 0, 0};
     const float scale_log2 = scale * 1.4426950408889634f;
     const int lr = tid / VPR, lc = tid % VPR;
     const int row_a = 8 * (li >> 2) + (li & 3);
 
-    // one slab (64 rows x 256 B) = 4 passes; pass p, wave w fills rows 16 p + 4 w .. + 3 (1 KiB, lane-linear)
+    // one slab (64 rows x 256 B) = 4 passes; pass p, wave w fills rows 16 p + 4 w .. + 3 (1 KiB, lane-linear).  The slab's first row
+    // is a scalar pointer; a lane adds its row's offset, cut at the slab's last key, and the chunk that the swizzle puts at its
+    // place (K's depends on the parity of p, V's does not): three 32-bit VALU operations per pass.  With the row index clamped and
+    // multiplied by the stride per lane, in 64 bits, addresses were 400 of the 1 650 VALU cycles of a slab.
+    const uint32_t row_bytes = 2 * (uint32_t)stride_t;                    // (the host takes strides past 2^25 another way: 63 rows stay below 2^32 bytes)
+    uint32_t row_off = (uint32_t)lr * row_bytes;
+    uint32_t chunk_k = 16 * (lc ^ ((lr & 3) | (((lr >> 3) & 3) << 2)));              // odd passes: XOR 8 chunks
+    uint32_t chunk_v = 16 * ((((lc >> 1) ^ ((lr & 3) | (((lr >> 3) & 1) << 2))) << 1) | (lc & 1));
     auto dma_slab = [&](const h16* base, h16* dst_buf, int slab, bool is_v) {
+        const char* first = reinterpret_cast<const char*>(base + (int64_t)slab * SLAB * stride_t);
+        const uint32_t last_off = (uint32_t)min(SLAB - 1, sk - 1 - slab * SLAB) * row_bytes;
 #pragma unroll
         for (int p = 0; p < NPASS; ++p) {
-            const int r = p * RPP + lr;                                   // lr = tid / 16: row within the pass
-            int key = slab * SLAB + r;
-            key = key < sk ? key : sk - 1;
-            int c;
-            if (!is_v) {
-                const int fk = (r & 3) | (((r >> 3) & 3) << 2);
-                c = lc ^ fk;
-            } else {
-                const int fv = (r & 3) | (((r >> 3) & 1) << 2);
-                c = (((lc >> 1) ^ fv) << 1) | (lc & 1);
-            }
-            const h16* src = base + (int64_t)key * stride_t + 8 * c;
-            h16* dst = dst_buf + (p * RPP + 4 * wave) * D;                // wave-uniform 1-KiB destination of this pass
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                             (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+            const uint32_t off = min(row_off + (uint32_t)(p * RPP) * row_bytes, last_off) + (is_v ? chunk_v : chunk_k ^ ((p & 1) * 128));
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(first + off),
+                                             (__attribute__((address_space(3))) void*)(dst_buf + (p * RPP + 4 * wave) * D), 16, 0, 0);
         }
     };
     auto fetch_k = [&](int slab, int buf) { dma_slab(kbase, sK + buf * BlkLayout<D>::K_HALFS, slab, false); };
     auto fetch_v = [&](int slab, int buf) { dma_slab(vbase, sVt + buf * BlkLayout<D>::V_HALFS, slab, true); };
+    // LDS places of a lane's fragments: the swizzles are XORs of bits that no other part of an address touches, so one place per
+    // buffer and one XOR per 32-wide chunk / 16-wide tile reach all of them; the rest are instruction offsets
+    int k_at = row_a * RS + 8 * (g ^ li);
+    int v_at = (8 * g + (li >> 2)) * D + 4 * (li & 3) + 16 * ((li >> 2) | ((g & 1) << 2));
+    // Fragments are requested a fixed distance ahead of their products, step by step: left to itself the scheduler moves all 16 (32)
+    // reads of a product to its front and spills a hundred registers.
+    auto pv = [&](const half8 (&pa)[QT], const half8 (&pb)[QT], int at) {
+        constexpr int STEPS = 2 * NT, AHEAD = 8;
+        half4 lo[AHEAD + 1], hi[AHEAD + 1];
+        auto read = [&](int n) {
+            const h16* src = sVt + (at ^ (16 * (n % NT))) + (n / NT) * 32 * D;
+            lo[n % (AHEAD + 1)] = lds_read_tr4(src);
+            hi[n % (AHEAD + 1)] = lds_read_tr4(src + 4 * D);
+        };
+#pragma unroll
+        for (int n = 0; n < AHEAD; ++n) read(n);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < STEPS; ++n) {
+            if (n + AHEAD < STEPS) read(n + AHEAD);
+            const half4 l = lo[n % (AHEAD + 1)], h = hi[n % (AHEAD + 1)];
+            const half8 vt = half8{l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]};
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt)
+                st.acc[qt][n % NT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt, n < NT ? pa[qt] : pb[qt], st.acc[qt][n % NT], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
     // both 32-key sub-steps of one slab: scores S^T[key][q] of tiles A / B (keys 4g..4g+3 of either half) per q-tile
-    auto qk_slab = [&](const h16* bk, f32x4 (&a0)[QT], f32x4 (&b0)[QT], f32x4 (&a1)[QT], f32x4 (&b1)[QT]) {
+    auto qk_slab = [&](int at, f32x4 (&a0)[QT], f32x4 (&b0)[QT], f32x4 (&a1)[QT], f32x4 (&b1)[QT], auto&& beside) {
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
             a0[qt] = f32x4{0.f, 0.f, 0.f, 0.f}; b0[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
             a1[qt] = f32x4{0.f, 0.f, 0.f, 0.f}; b1[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
+        constexpr int STEPS = 2 * NC, AHEAD = 4;
+        half8 ka[AHEAD + 1], kb[AHEAD + 1];
+        auto read = [&](int n) {
+            const h16* src = sK + (at ^ (32 * (n % NC))) + (n / NC) * 32 * RS;
+            ka[n % (AHEAD + 1)] = load_half8(src);
+            kb[n % (AHEAD + 1)] = load_half8(src + 4 * RS);
+        };
 #pragma unroll
-        for (int sub = 0; sub < 2; ++sub)
+        for (int n = 0; n < AHEAD; ++n) read(n);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const int kcol = 8 * ((4 * c + g) ^ li);
-                const half8 ka = load_half8(bk + (32 * sub + row_a) * RS + kcol);
-                const half8 kb = load_half8(bk + (32 * sub + row_a + 4) * RS + kcol);
+        for (int n = 0; n < STEPS; ++n) {
+            if (n + AHEAD < STEPS) read(n + AHEAD);
 #pragma unroll
-                for (int qt = 0; qt < QT; ++qt) {
-                    if (sub == 0) {
-                        a0[qt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, st.qf[qt][c], a0[qt], 0, 0, 0);
-                        b0[qt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb, st.qf[qt][c], b0[qt], 0, 0, 0);
-                    } else {
-                        a1[qt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, st.qf[qt][c], a1[qt], 0, 0, 0);
-                        b1[qt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb, st.qf[qt][c], b1[qt], 0, 0, 0);
-                    }
-                }
+            for (int qt = 0; qt < QT; ++qt) {
+                f32x4& a = n < NC ? a0[qt] : a1[qt];
+                f32x4& b = n < NC ? b0[qt] : b1[qt];
+                a = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[n % (AHEAD + 1)], st.qf[qt][n % NC], a, 0, 0, 0);
+                b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[n % (AHEAD + 1)], st.qf[qt][n % NC], b, 0, 0, 0);
             }
+            beside(n);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     };
 
     if (s_begin < s_end) {
@@ -1520,29 +1557,68 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
         fetch_k(min(s_begin + 1, s_end - 1), 1);
         __builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0): Q fragments and the prologue slabs have landed
         __syncthreads();
-        qk_slab(sK, c0a, c0b, c1a, c1b);
+        qk_slab(k_at, c0a, c0b, c1a, c1b, [](int) {});
         __syncthreads();                                     // every wave is done with K[s_begin] before iteration 0 overwrites it
         for (int sl = s_begin; sl < s_end; ++sl) {
             const int i = sl - s_begin;
+            // (opaque once per slab: the sums and XORs on these are one instruction each, hoisted out of the loop they would take
+            // some forty registers that the scores need)
+            asm("" : "+v"(row_off), "+v"(chunk_k), "+v"(chunk_v), "+v"(k_at), "+v"(v_at));
             fetch_k(min(sl + 2, s_end - 1), i & 1);          // K[sl + 2] over K[sl] (dead since the previous barrier), V[sl + 1]
             fetch_v(min(sl + 1, s_end - 1), (i + 1) & 1);    // over V[sl - 1]; unconditional: in flight under the MFMAs
-            const h16* bk_next = sK + ((i + 1) & 1) * BlkLayout<D>::K_HALFS;
-            const h16* bv = sVt + (i & 1) * BlkLayout<D>::V_HALFS;
+            const int k_next = k_at + ((i + 1) & 1) * BlkLayout<D>::K_HALFS;
             f32x4 n0a[QT], n0b[QT], n1a[QT], n1b[QT];
-            const int last = sl * SLAB + SLAB - 1;
-            if (last < sk && last <= sk - sq + qbase) {      // wave-uniform: the whole slab is visible to every row of the wave
-                half8 p0[QT], p1[QT], l0[QT], l1[QT];
-                qk_slab(bk_next, n0a, n0b, n1a, n1b);        // next slab's QK^T (past the end: finite garbage, never used)
-                lds_softmax_clear2<D, QT>(st, c0a, c0b, c1a, c1b, scale_log2, p0, p1, l0, l1);
-                lds_pv_tr<D, QT>(st, p0, l0, bv, 0, li, g);
-                lds_pv_tr<D, QT>(st, p1, l1, bv, 4, li, g);
-            } else {
-                qk_slab(bk_next, n0a, n0b, n1a, n1b);
-                const int key0 = sl * SLAB;
-                lds_softmax_pv<D, QT, false, true>(st, c0a, c0b, bv, 0, key0, sk, sq, scale_log2, li, g, qbase, tm);
-                if (key0 + 32 < sk)
-                    lds_softmax_pv<D, QT, false, true>(st, c1a, c1b, bv, 4, key0 + 32, sk, sq, scale_log2, li, g, qbase, tm);
+            const int key0 = sl * SLAB;
+            if (key0 + SLAB - 1 > sk - sq + qbase) {         // wave-uniform: some row of the wave does not see the whole slab
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) {
+                    const int qrow = qbase + qt * 16 + li, seen = (qrow < sq ? sk - sq + qrow : sk - 1) - key0 - 8 * g;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {            // exp2 of -inf minus any finite maximum is 0
+                        if (r > seen) c0a[qt][r] = -__builtin_inff();
+                        if (r + 4 > seen) c0b[qt][r] = -__builtin_inff();
+                        if (r + 32 > seen) c1a[qt][r] = -__builtin_inff();
+                        if (r + 36 > seen) c1b[qt][r] = -__builtin_inff();
+                    }
+                }
             }
+            float mnew[QT];
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) {
+                float tmax = c0a[qt][0];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) tmax = fmaxf(fmaxf(fmaxf(tmax, c0a[qt][r]), fmaxf(c0b[qt][r], c1a[qt][r])), c1b[qt][r]);
+                tmax = group_max4(tmax);
+                mnew[qt] = fmaxf(st.m[qt], tmax * scale_log2);
+                if (__builtin_amdgcn_ballot_w64(mnew[qt] != st.m[qt])) {
+                    const float alpha = __builtin_amdgcn_exp2f(st.m[qt] - mnew[qt]);
+                    st.l[qt] *= alpha;
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        st.acc[qt][t][0] *= alpha; st.acc[qt][t][1] *= alpha;
+                        st.acc[qt][t][2] *= alpha; st.acc[qt][t][3] *= alpha;
+                    }
+                    st.m[qt] = mnew[qt];
+                }
+            }
+            // The next slab's QK^T (past the end: finite garbage, never used) with this slab's exponentials beside it: four scores of
+            // a lane per four products, so that the matrix core works while the wave issues VALU operations
+            half8 p0[QT], p1[QT];
+            float psum[QT] = {};
+            qk_slab(k_next, n0a, n0b, n1a, n1b, [&](int n) {
+                const int qt = n / 4, quad = n % 4;
+                const f32x4& x = quad == 0 ? c0a[qt] : quad == 1 ? c0b[qt] : quad == 2 ? c1a[qt] : c1b[qt];
+                half8& dst = quad < 2 ? p0[qt] : p1[qt];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float e = __builtin_amdgcn_exp2f(fmaf(x[r], scale_log2, -mnew[qt]));
+                    psum[qt] += e;
+                    dst[4 * (quad & 1) + r] = (h16)e;
+                }
+            });
+            pv(p0, p1, v_at + (i & 1) * BlkLayout<D>::V_HALFS);
+#pragma unroll
+            for (int qt = 0; qt < QT; ++qt) st.l[qt] += psum[qt];
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
                 c0a[qt] = n0a[qt]; c0b[qt] = n0b[qt]; c1a[qt] = n1a[qt]; c1b[qt] = n1b[qt];
@@ -1552,6 +1628,26 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
         }
     }
 
+    if (nsplit == 1) {                                       // all keys were here: the merge's arithmetic with its one weight of 1
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+            float lsum = st.l[qt];
+            lsum += __shfl_xor(lsum, 16, 64);
+            lsum += __shfl_xor(lsum, 32, 64);
+            const float inv = 1.0f / lsum;
+            const int row = qbase + qt * 16 + li;
+            if (row >= sq) continue;
+            h16* o = out + ((int64_t)row * H + h) * D + 4 * g;
+#pragma unroll
+            for (int tt = 0; tt < NT; ++tt) {
+                half4 v;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = (h16)(st.acc[qt][tt][r] * inv);
+                *reinterpret_cast<half4*>(o + 16 * tt) = v;
+            }
+        }
+        return;
+    }
     float* ws_o = ws;
     float* ws_m = ws + (int64_t)H * nsplit * QR * D;
     float* ws_l = ws_m + (int64_t)H * nsplit * QR;
@@ -1581,14 +1677,15 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
 template <int D>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
     const h16* __restrict__ q, const h16* __restrict__ k, const h16* __restrict__ v, int64_t stride_t,
-    int64_t stride_h, int sq, int sk, int H, float scale, int nsplit, float* __restrict__ ws, int nrb, int rbg) {
+    int64_t stride_h, int sq, int sk, int H, float scale, int nsplit, float* __restrict__ ws, h16* __restrict__ out, int nrb,
+    int rbg) {
     const int id = blockIdx.x;
     const int pairs = H * nsplit;                                     // host guarantees pairs % 8 == 0
     const int xcd = id & 7, j = id >> 3;
     const int rb_lo = j % rbg, rest = j / rbg;
     const int pair = (rest % (pairs >> 3)) * 8 + xcd;
-    const int rb = rb_lo + rbg * (rest / (pairs >> 3));
-    if (rb >= nrb) return;
+    const int rb = nrb - 1 - (rb_lo + rbg * (rest / (pairs >> 3)));
+    if (rb < 0) return;
     const int h = pair / nsplit, split = pair - h * nsplit;
     const int r0 = rb * 128;
     const int rows = min(128, sq - r0);
@@ -1600,7 +1697,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
     float* ws_rb = ws + (int64_t)rb * H * nsplit * 128 * (D + 2);
     if constexpr (TF_PREFILL_AHEAD && BlkLayout<D>::TR)
         attn_prefill_ahead_body<D>(q + (int64_t)r0 * H * D, k, v, stride_t, stride_h, rows, sk_eff, H, scale, nsplit, ws_rb,
-                                   split, h, s_begin, min(nslabs, s_begin + sps));
+                                   out + (int64_t)r0 * H * D, split, h, s_begin, min(nslabs, s_begin + sps));
     else
         attn_block_lds_body<D, false>(q + (int64_t)r0 * H * D, k, v, stride_t, stride_h, rows, sk_eff, H, scale, nsplit, ws_rb,
                                       nullptr, 0, 0, 0, split, h, s_begin, min(nslabs, s_begin + sps));
@@ -2144,8 +2241,10 @@ static int launch_prefill(const void* q, const void* k, const void* v, void* out
     const int groups = (nrb + rbg - 1) / rbg;
     const int64_t blocks = (int64_t)H * nsplit * rbg * groups;
     hipLaunchKernelGGL((attn_prefill_kernel<D>), dim3((unsigned)blocks), dim3(256), blk_lds_bytes<D>(), st, (const h16*)q,
-                       (const h16*)k, (const h16*)v, stride_t, stride_h, sq, sk, H, scale, nsplit, ws, nrb, rbg);
+                       (const h16*)k, (const h16*)v, stride_t, stride_h, sq, sk, H, scale, nsplit, ws, (h16*)out, nrb,
+                       rbg);
     TF_LAUNCH_CHECK();
+    if (nsplit == 1 && TF_PREFILL_AHEAD && BlkLayout<D>::TR) return TF_OK;         // written by the kernel itself
     hipLaunchKernelGGL((attn_combine_rows_kernel<D>), dim3((sq * H + 3) / 4), dim3(256), 0, st, (const float*)ws,
                        (h16*)out, sq, H, nsplit, 128, 128);
     TF_LAUNCH_CHECK();
@@ -2163,6 +2262,15 @@ extern "C" int tf_attn_prefill(const void* q, const void* k, const void* v, void
     if ((stride_t % 8) || (stride_h % 8)) return TF_EINVAL;
     if (ws_floats < tf_attn_prefill_ws_floats(H, sq, D, nsplit)) return TF_ENOSPC;
     hipStream_t st = (hipStream_t)stream;
+    if (D == 128 && (stride_t < 0 || stride_t >= (1 << 25))) {   // rows 64 MB apart: the kernel's 32-bit slab offsets do not reach
+        for (int r0 = 0; r0 < sq; r0 += 128) {
+            const int rows = sq - r0 < 128 ? sq - r0 : 128;
+            const int rc = tf_attn_block((const h16*)q + (int64_t)r0 * H * D, k, v, (h16*)out + (int64_t)r0 * H * D, stride_t, stride_h, rows,
+                                         sk - (sq - r0 - rows), H, D, scale, nsplit < 32 ? nsplit : 32, ws, ws_floats, nullptr, 0, 0, 0, stream);
+            if (rc != TF_OK) return rc;
+        }
+        return TF_OK;
+    }
     if (D == 128) return launch_prefill<128>(q, k, v, out, stride_t, stride_h, sq, sk, H, scale, nsplit, ws, st);
     if (D == 64) return launch_prefill<64>(q, k, v, out, stride_t, stride_h, sq, sk, H, scale, nsplit, ws, st);
     return TF_EINVAL;
