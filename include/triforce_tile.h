@@ -6,7 +6,8 @@
  * to multiples of 32 with zeros unless a parameter is called "real".
  *
  * Packed weights: a [n, k] matrix is stored as [n/16][k/32][64][8]: piece (g*16 + i) of a 16x32 tile holds
- * w[16a + i][32b + 8g .. +7] - one wavefront load per tile.
+ * w[16a + i][32b + 8g .. +7] - one wavefront load per tile.  chunk_major: the same tiles as [k/32][n/16], so that neighbouring panels
+ * are neighbours in memory (what a launch with one workgroup per CU streams fastest).
  */
 #ifndef TRIFORCE_TILE_H
 #define TRIFORCE_TILE_H
@@ -67,6 +68,7 @@ typedef struct TflGemm {
     int32_t n_real, k_real, n_raw, n_scaled, ss_n, ss_ld;
     int32_t H, N, R, C, half, c_real, max_pos, cache_rows, vocab;
     float eps;
+    int32_t chunk_major;            /* packed weights as [k/32][n/16][64][8] (one group) */
 } TflGemm;
 
 int tfl_gemm(const TflGemm* a, int dtype, int epilogue, void* stream);

@@ -92,3 +92,51 @@ def test_prefill_attention_rows_far_apart():
     got = ops.attn_prefill(q, k, v, m, 0.088).view(n, 1, D).double()
     want, size = _attention64(q, k, v, 0.088)
     assert ((got - want).abs() <= 2.0 ** -10 * size + 2.0 ** -11 * want.abs() + 1e-6).all()
+
+
+def _bf(g, *shape, std=1.0):
+    return (torch.randn(*shape, generator=g, device=DEV) * std).to(torch.bfloat16)
+
+
+def _near(got, want, size, k, out_bits=0):
+    """fp32 sums of k exact products (k * 2^-24 of their magnitudes), and the output's own rounding."""
+    bound = size * k * 2.0 ** -24 + (want.abs() * 2.0 ** -out_bits if out_bits else 0) + 1e-6
+    assert ((got.double() - want).abs() <= bound).all()
+
+
+# panels of 16 outputs over 256 workgroups: whole shares, 4 / 8 / 12 rows left over (full and ragged), a share of one panel more, the
+# widest; chunks: fewer than the waves, odd, one per wave and more; batch rows around one and two row blocks
+@pytest.mark.parametrize("panels", [256, 257, 319, 330, 391, 460, 512, 700, 1076, 2000, 2048])
+@pytest.mark.parametrize("rows,k", [(1, 32), (3, 544), (16, 288), (17, 256), (32, 96), (33, 800)])
+def test_wide_gemm_shares(panels, rows, k):
+    from triforce_amd import ops_latent as ol, ops_tile as ot
+    g = torch.Generator(device=DEV).manual_seed(panels * 100 + rows)
+    n = 16 * panels
+    w, h = _bf(g, n, k, std=k ** -0.5), _bf(g, k // 8, rows, 8)
+    x = ot.act_rows(h)
+    wt = ot.TileWeight(w)
+    assert wt.chunk_major
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    _near(ot.linear_f32(h, wt, n - 5), want[:, :n - 5], size[:, :n - 5], k)
+    res = torch.randn(rows, n, generator=g, device=DEV)
+    got = res.clone()
+    copy = ol.add_linear(h, wt, got, want_copy=True)
+    _near(got, want + res.double(), size + res.double().abs(), k + 1)
+    assert torch.equal(ot.act_rows(copy), got.to(torch.bfloat16))
+    # gate | up: the outputs of one panel are an octet; errors of gate and up carry over with slopes below 1.13 and |gate|
+    out = ot.act_rows(ot.gelu_glu_linear(h, wt)).double()
+    v, s = (t.view(rows, panels, 2, 8) for t in (want, size))
+    glu = torch.nn.functional.gelu(v[:, :, 0], approximate="tanh") * v[:, :, 1]
+    bound = (1.13 * s[:, :, 0] * v[:, :, 1].abs() + s[:, :, 1] * v[:, :, 0].abs()) * (k + 16) * 2.0 ** -24 + glu.abs() * 2.0 ** -8 + 1e-6
+    assert ((out - glu.reshape(rows, -1)).abs() <= bound.reshape(rows, -1)).all()
+    # raw outputs with sums of squares in front, gelu behind: the left-over rows lie behind, or the raw part reaches into them
+    q_norm = 1.0 + 0.1 * torch.randn(64, generator=g, device=DEV)
+    for n_raw in (128, 16 * (panels - 1)):
+        act = ot.empty_act(rows, n - n_raw, torch.bfloat16, DEV)
+        raw, ss, xq = ol.input_projection(h, wt, n_raw, q_norm, act, 0)
+        _near(raw, want[:, :n_raw], size[:, :n_raw], k)
+        sums = raw.double().square().view(rows, -1, 16).sum(-1)
+        assert ((ss.double() - sums).abs() <= sums * 16 * 2.0 ** -24).all()
+        assert torch.equal(ot.act_rows(xq), (raw[:, :64] * q_norm).to(torch.bfloat16))
+        tail = torch.nn.functional.gelu(want[:, n_raw:], approximate="tanh")
+        _near(ot.act_rows(act), tail, size[:, n_raw:] * 1.13, k + 16, out_bits=8)

@@ -153,7 +153,7 @@ class TflGemm(_c.Structure):
                 + [(n, _i64) for n in ("ld_x", "x_oct", "x_group", "ld_t", "t_oct", "ld_f", "ld_gate", "ld_tok", "ld_kv")]
                 + [(n, _i32) for n in ("rows", "n", "k", "groups", "n_real", "k_real", "n_raw", "n_scaled", "ss_n", "ss_ld", "H", "N", "R", "C",
                                        "half", "c_real", "max_pos", "cache_rows", "vocab")]
-                + [("eps", _f32)])
+                + [("eps", _f32), ("chunk_major", _i32)])
 
 
 TILE_SIGNATURES = {
@@ -161,7 +161,7 @@ TILE_SIGNATURES = {
     "tfl_gemm": (_i32, [_c.POINTER(TflGemm), _i32, _i32, _vp]),
     "tfl_decode_prep": (_i32, [_vp, _vp, _i32, _i32, _vp, _vp, _vp, _i32, _vp]),
 }
-TILE_ABI_VERSION = 1
+TILE_ABI_VERSION = 2
 _tile = None
 
 # ---- libtriforce_latent.so (include/triforce_latent.h) ------------------------------------------------------------------

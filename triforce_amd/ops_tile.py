@@ -52,23 +52,27 @@ def grow(t, *shape):
     return out
 
 
-def pack_tiles(w):
-    """[.., n, k] -> MFMA operand order [.., n/16, k/32, 4 (k octet), 16 (row), 8]: one 16x32 tile is one wavefront load."""
+def pack_tiles(w, chunk_major=False):
+    """[.., n, k] -> MFMA operand order [.., n/16, k/32, 4 (k octet), 16 (row), 8]: one 16x32 tile is one wavefront load.
+    ``chunk_major``: the tiles as [.., k/32, n/16]."""
     n, k = w.shape[-2:]
     assert n % 16 == 0 and k % 32 == 0
     lead = w.shape[:-2]
     d = len(lead)
-    return w.reshape(*lead, n // 16, 16, k // 32, 4, 8).permute(*range(d), d, d + 2, d + 3, d + 1, d + 4).contiguous()
+    order = (d + 2, d) if chunk_major else (d, d + 2)
+    return w.reshape(*lead, n // 16, 16, k // 32, 4, 8).permute(*range(d), *order, d + 3, d + 1, d + 4).contiguous()
 
 
 class TileWeight:
     """A (groups of) [n, k] weight(s): packed for the skinny kernel and, unless ``packed_only``, row-major for the library GEMM
-    of the prefill."""
+    of the prefill.  Wide bfloat16 weights (a panel or more per CU) are packed chunk-major, which the one-workgroup-per-CU form of
+    the kernel streams, unless ``panel_major`` says that their epilogue has no such form (TFL_EPI_QUERY)."""
 
-    def __init__(self, w, packed_only=False):
+    def __init__(self, w, packed_only=False, panel_major=False):
         w3 = w if w.dim() == 3 else w.unsqueeze(0)
         self.groups, self.n, self.k = w3.shape
-        self.packed = pack_tiles(w3)
+        self.chunk_major = not panel_major and self.groups == 1 and w.dtype == torch.bfloat16 and self.n >= 256 * 16
+        self.packed = pack_tiles(w3, self.chunk_major)
         self.w = None if packed_only else w.contiguous()
         self.dtype, self.device = w.dtype, w.device
 
@@ -109,6 +113,7 @@ def _gemm(wt, x, epi, rows, **kw):
     a.wp, a.x = wt.packed.data_ptr(), x.data_ptr()
     a.rows, a.n, a.k, a.groups = rows, wt.n, wt.k, wt.groups
     a.x_oct = a.t_oct = 8
+    a.chunk_major = int(wt.chunk_major)
     for name, v in kw.items():
         setattr(a, name, v.data_ptr() if isinstance(v, torch.Tensor) else v)
     hip.check(hip.tile_lib().tfl_gemm(ctypes.byref(a), _CODE[wt.dtype], hip.TFL_EPI[epi], _stream()), "tfl_gemm " + epi)
