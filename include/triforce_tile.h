@@ -78,6 +78,11 @@ int tfl_gemm(const TflGemm* a, int dtype, int epilogue, void* stream);
 int tfl_decode_prep(int32_t* len, const int32_t* table, int table_ld, int table_cols, int32_t* pos, int32_t* slot, int32_t* klen,
                     int rows, void* stream);
 
+/* table[row * table_ld + column] = page for n (at most TFL_MAX_ENTRIES) host triples {row, column, page}: pages handed out between
+ * two decode steps.  The triples are kernel arguments (nothing is read after the call returns). */
+#define TFL_MAX_ENTRIES 64
+int tfl_set_pages(int32_t* table, int table_ld, int rows, int cols, const int32_t* entries, int n, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

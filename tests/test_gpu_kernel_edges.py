@@ -140,3 +140,18 @@ def test_wide_gemm_shares(panels, rows, k):
         assert torch.equal(ot.act_rows(xq), (raw[:, :64] * q_norm).to(torch.bfloat16))
         tail = torch.nn.functional.gelu(want[:, n_raw:], approximate="tanh")
         _near(ot.act_rows(act), tail, size[:, n_raw:] * 1.13, k + 16, out_bits=8)
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 200])
+def test_set_pages(n):
+    from triforce_amd import hip, ops_tile as ot
+    table = torch.zeros(7, 40, dtype=torch.int32, device=DEV)[:, :37]
+    places = torch.randperm(7 * 37, generator=torch.Generator().manual_seed(n))[:n].tolist()
+    ot.set_pages(table, [(p // 37, p % 37, 1000 + p) for p in places])
+    want = torch.zeros(7 * 37, dtype=torch.int32)
+    for p in places:
+        want[p] = 1000 + p
+    assert torch.equal(table.cpu(), want.view(7, 37))
+    for bad in ((7, 0, 1), (0, 37, 1), (-1, 0, 1)):
+        with pytest.raises(hip.TriforceHipError):
+            ot.set_pages(table, [bad])

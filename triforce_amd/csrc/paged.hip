@@ -23,3 +23,22 @@ extern "C" int tfl_decode_prep(int32_t* len, const int32_t* table, int table_ld,
     TFL_LAUNCH_CHECK();
     return TF_OK;
 }
+
+struct PageEntries { int32_t e[3 * TFL_MAX_ENTRIES]; };
+
+__global__ void set_pages_kernel(int32_t* __restrict__ table, int table_ld, const PageEntries entries, int n) {
+    const int j = threadIdx.x;
+    if (j < n) table[(int64_t)entries.e[3 * j] * table_ld + entries.e[3 * j + 1]] = entries.e[3 * j + 2];
+}
+
+extern "C" int tfl_set_pages(int32_t* table, int table_ld, int rows, int cols, const int32_t* entries, int n, void* stream) {
+    if (!table || !entries || rows < 1 || cols < 1 || table_ld < cols || n < 1 || n > TFL_MAX_ENTRIES) return TF_EINVAL;
+    PageEntries p;
+    for (int j = 0; j < n; ++j) {
+        if (entries[3 * j] < 0 || entries[3 * j] >= rows || entries[3 * j + 1] < 0 || entries[3 * j + 1] >= cols) return TF_EINVAL;
+        for (int i = 0; i < 3; ++i) p.e[3 * j + i] = entries[3 * j + i];
+    }
+    hipLaunchKernelGGL(set_pages_kernel, dim3(1), dim3(TFL_MAX_ENTRIES), 0, (hipStream_t)stream, table, table_ld, p, n);
+    TFL_LAUNCH_CHECK();
+    return TF_OK;
+}

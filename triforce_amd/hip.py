@@ -143,6 +143,7 @@ _lib = None
 
 # ---- libtriforce_tile.so (include/triforce_tile.h) ------------------------------------------------------------------
 TFL_PAGE = 64
+TFL_MAX_ENTRIES = 64
 TFL_EPI = {n: i for i, n in enumerate(("f32", "in", "query", "latent", "gated", "residual", "token", "glu"))}
 
 
@@ -159,6 +160,7 @@ class TflGemm(_c.Structure):
 TILE_SIGNATURES = {
     "tfl_tile_abi_version": (_i32, []),
     "tfl_gemm": (_i32, [_c.POINTER(TflGemm), _i32, _i32, _vp]),
+    "tfl_set_pages": (_i32, [_vp, _i32, _i32, _i32, _c.POINTER(_c.c_int32), _i32, _vp]),
     "tfl_decode_prep": (_i32, [_vp, _vp, _i32, _i32, _vp, _vp, _vp, _i32, _vp]),
 }
 TILE_ABI_VERSION = 2

@@ -604,16 +604,21 @@ class PagedCache(Cache):
         self.rows = [torch.zeros(self.n_pages * self.page, w, dtype=model.dtype, device=self.device) if w else None
                      for w in model.cache_widths()]
         model.prepare_positions(self.max_budget)
-        self.generation = 0                         # bumped when a page is handed out or taken back (device tables go stale)
+        self.generation = 0                         # bumped when a page is handed out or taken back
         self.free, self.pages, self.length = [], {}, {}
         self.free_seats, self.seat = [], {}
+        self.birth, self._births = {}, 0            # a number of its own for every sequence that ever lived here
+        self._by_seat = torch.zeros(self.max_batch, self.columns, dtype=torch.int32)    # pages of each seat's sequence, 0 behind
+        self._by_seat_np = self._by_seat.numpy()
         self.reset()
 
     # -- sequences -----------------------------------------------------------------------------
     def reset(self):
         self.free = list(range(self.n_pages - 1, -1, -1))
         self.free_seats = list(range(self.max_batch - 1, -1, -1))
-        self.pages, self.length, self.seat = {}, {}, {}
+        for s, seat in self.seat.items():
+            self._by_seat_np[seat, :len(self.pages[s])] = 0
+        self.pages, self.length, self.seat, self.birth = {}, {}, {}, {}
         self.generation += 1
 
     @property
@@ -630,9 +635,11 @@ class PagedCache(Cache):
 
     def release(self, seq):
         """The sequence is finished: its pages and its seat are free for others."""
-        self.free.extend(reversed(self.pages.pop(seq)))
-        self.free_seats.append(self.seat.pop(seq))
-        del self.length[seq]
+        pages, seat = self.pages.pop(seq), self.seat.pop(seq)
+        self.free.extend(reversed(pages))
+        self.free_seats.append(seat)
+        self._by_seat_np[seat, :len(pages)] = 0
+        del self.length[seq], self.birth[seq]
         self.generation += 1
 
     def extend(self, wants):
@@ -646,12 +653,17 @@ class PagedCache(Cache):
         for s, n in wants:
             if s not in self.length:
                 self.length[s], self.pages[s], self.seat[s] = 0, [], self.free_seats.pop()
+                self.birth[s] = self._births
+                self._births += 1
                 self.generation += 1
             self.length[s] += n
-            need = -(-self.length[s] // self.page) - len(self.pages[s])
-            for _ in range(need):
-                self.pages[s].append(self.free.pop())
-            if need:
+            pages = self.pages[s]
+            need = -(-self.length[s] // self.page) - len(pages)
+            if need > 0:
+                new = self.free[:-need - 1:-1]       # from the end, as single pops would
+                del self.free[-need:]
+                self._by_seat_np[self.seat[s], len(pages):len(pages) + need] = new
+                pages += new
                 self.generation += 1
 
     def cache_rows(self, seq, first, n):
@@ -680,11 +692,8 @@ class PagedCache(Cache):
 
     def tables(self, seqs):
         """(lengths int32 [B], page tables int32 [B, columns], seats int32 [B]) of some sequences, on the CPU; unused columns are 0."""
-        table = torch.zeros(len(seqs), self.columns, dtype=torch.int32)
-        for b, s in enumerate(seqs):
-            table[b, :len(self.pages[s])] = torch.tensor(self.pages[s], dtype=torch.int32)
-        return (torch.tensor([self.length[s] for s in seqs], dtype=torch.int32), table,
-                torch.tensor([self.seat[s] for s in seqs], dtype=torch.int32))
+        seats = torch.tensor([self.seat[s] for s in seqs], dtype=torch.int32)
+        return torch.tensor([self.length[s] for s in seqs], dtype=torch.int32), self._by_seat[seats.long()], seats
 
 
 class LatentCache(PagedCache):

@@ -147,6 +147,16 @@ def interleave_glu(gate, up):
     return torch.stack([gate.view(n // 8, 8, k), up.view(n // 8, 8, k)], 1).reshape(2 * n, k)
 
 
+def set_pages(table, entries):
+    """table[row, column] = page for every (row, column, page) of a host list; the entries travel as kernel arguments."""
+    _need(table)
+    _i32(table)
+    for at in range(0, len(entries), hip.TFL_MAX_ENTRIES):
+        part = entries[at:at + hip.TFL_MAX_ENTRIES]
+        flat = (ctypes.c_int32 * (3 * len(part)))(*(v for e in part for v in e))
+        hip.check(hip.tile_lib().tfl_set_pages(_p(table), table.stride(0), table.shape[0], table.shape[1], flat, len(part), _stream()), "tfl_set_pages")
+
+
 def decode_prep(lens, table, pos, slot, klen):
     _need(lens, table, pos, slot, klen)
     _i32(lens, table, pos, slot, klen)

@@ -13,18 +13,51 @@ from . import graph_infer
 
 class _DecodeBuffers:
     """Static device inputs of the decode step of B sequences.  ``lens`` advances on the device (ops_tile.decode_prep is part of
-    the step); the host uploads lengths, page tables and seats only when the set of sequences or their pages changed."""
+    the step); the host uploads lengths, page tables and seats when the set of sequences changed, in one asynchronous copy, and sends
+    pages that were handed out since as kernel arguments (at 32 sequences some sequence starts a page every other step: three
+    copies from pageable memory waited for the device each time, 0.3 ms of it idle)."""
 
     def __init__(self, cache, B):
         dev = cache.device
-        self.B = B
+        self.B, self.columns = B, cache.columns
         self.ids = torch.zeros(B, dtype=torch.int64, device=dev)
-        self.lens = torch.full((B,), -1, dtype=torch.int32, device=dev)             # -1: idle row
-        self.table = torch.zeros(B, cache.columns, dtype=torch.int32, device=dev)
+        image = torch.zeros(B * (2 + self.columns), dtype=torch.int32, device=dev)      # lengths | seats | table
+        self.lens, self.seat, self.table = self._parts(image)
+        self.lens.fill_(-1)                                                             # -1: idle row
+        self.seat.fill_(-1)
         self.pos, self.slot, self.klen = (torch.zeros(B, dtype=torch.int32, device=dev) for _ in range(3))
-        self.seat = torch.full((B,), -1, dtype=torch.int32, device=dev)
         self.batch = PagedBatch(True, self.pos, self.slot, table=self.table, klen=self.klen, seat=self.seat, max_len=cache.max_budget)
-        self.current = None                                     # (sequences, cache generation, lengths) the device holds
+        self.image, self.staged, self.sent = image, torch.zeros(image.shape, dtype=torch.int32, pin_memory=image.is_cuda), None
+        self.current, self.known = None, [0] * B                # (births, lengths) the device holds; pages of each row it knows
+
+    def _parts(self, flat):
+        return flat[:self.B], flat[self.B:2 * self.B], flat[2 * self.B:].view(self.B, self.columns)
+
+    def upload(self, cache, seqs):
+        """Everything of these sequences; the lengths without the token of this step."""
+        if self.sent is not None:
+            self.sent.synchronize()                             # (the last copy out of the staging memory is long done)
+        lens, seat, table = self._parts(self.staged)
+        n, t, s = cache.tables(seqs)
+        lens.copy_(n - 1)
+        seat.copy_(s)
+        table.copy_(t)
+        self.image.copy_(self.staged, non_blocking=True)
+        if self.image.is_cuda:
+            self.sent = torch.cuda.Event()
+            self.sent.record()
+        self.known = [len(cache.pages[q]) for q in seqs]
+
+    def add_pages(self, cache, seqs):
+        """The pages that were handed out to these sequences since the device last heard of them."""
+        new = []
+        for row, s in enumerate(seqs):
+            pages, k = cache.pages[s], self.known[row]
+            if len(pages) > k:
+                new += [(row, j, pages[j]) for j in range(k, len(pages))]
+                self.known[row] = len(pages)
+        if new:
+            ops_tile.set_pages(self.table, new)
 
 
 class _DecodeStep:
@@ -47,12 +80,12 @@ class _DecodeStep:
         b, c = self.buf, self.cache
         before = tuple(c.length.get(s, 0) for s in seqs)
         c.extend([(s, 1) for s in seqs])
-        if b.current != (tuple(seqs), c.generation, before):
-            lens, table, seat = c.tables(seqs)
-            b.table.copy_(table)
-            b.lens.copy_(lens - 1)
-            b.seat.copy_(seat)
-        b.current = (tuple(seqs), c.generation, tuple(n + 1 for n in before))
+        births = tuple(c.birth[s] for s in seqs)
+        if b.current != (births, before):
+            b.upload(c, seqs)
+        else:
+            b.add_pages(c, seqs)
+        b.current = (births, tuple(n + 1 for n in before))
         b.ids.copy_(ids)
         if self.graph is None:
             return self._run()
