@@ -115,7 +115,7 @@ def test_wide_gemm_shares(panels, rows, k):
     w, h = _bf(g, n, k, std=k ** -0.5), _bf(g, k // 8, rows, 8)
     x = ot.act_rows(h)
     wt = ot.TileWeight(w)
-    assert wt.chunk_major
+    wt.packed, wt.chunk_major = ot.pack_tiles(w, True), True            # (the layout that weights of a longer k come in)
     want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
     _near(ot.linear_f32(h, wt, n - 5), want[:, :n - 5], size[:, :n - 5], k)
     res = torch.randn(rows, n, generator=g, device=DEV)
@@ -155,3 +155,53 @@ def test_set_pages(n):
     for bad in ((7, 0, 1), (0, 37, 1), (-1, 0, 1)):
         with pytest.raises(hip.TriforceHipError):
             ot.set_pages(table, [bad])
+
+
+# the merge by waves (rows x heads from 128 on, at most 64 splits) and by workgroups; splits without a page, idle rows
+@pytest.mark.parametrize("rows,H,nsplit", [(4, 32, 2), (5, 32, 16), (4, 33, 17), (9, 16, 64), (4, 32, 65), (1, 32, 30), (130, 1, 3)])
+def test_latent_decode_merge(rows, H, nsplit):
+    from types import SimpleNamespace
+    from triforce_amd import ops_latent as ol
+    g = torch.Generator(device=DEV).manual_seed(rows * nsplit)
+    C, R, pages = 512, 64, 24
+    geom = SimpleNamespace(H=H, C=C, R=R)
+    lens = torch.tensor([0 if b % 7 == 6 else 1 + (b * 389) % (64 * 6) for b in range(rows)], dtype=torch.int32)
+    table = torch.randint(0, pages, (rows, 6), generator=torch.Generator().manual_seed(1), dtype=torch.int32)
+    cache, q = _bf(g, pages * 64, C + R), _bf(g, rows, H, C + R)
+    got = ol.attn_decode(q, cache, table.to(DEV), lens.to(DEV), geom, 0.05, 384, nsplit=nsplit).double()
+    for b in range(rows):
+        n = int(lens[b])
+        if n == 0:
+            assert not got[b].any()
+            continue
+        k = cache.view(pages, 64, C + R)[table[b].long().to(DEV)].reshape(-1, C + R)[:n].double()
+        w = torch.softmax(q[b].double() @ k.T * 0.05, -1)
+        want = w @ k[:, :C]
+        # weights as two bfloat16 (2^-16), fp32 scores of 576 products, fp32 sums, one rounding to bfloat16
+        bound = (2.0 ** -15 + 1e-4) * (w @ k[:, :C].abs()) + 2.0 ** -8 * want.abs() + 1e-6
+        assert ((got[b] - want).abs() <= bound).all()
+
+
+# rows in a workgroup's registers (16 waves up to 256 rows, four waves beyond) and the general form (wider than 4 096)
+@pytest.mark.parametrize("rows,width,real", [(1, 32, 30), (3, 4096, 4096), (256, 1056, 1040), (257, 4096, 4090), (300, 96, 96), (5, 4128, 4100)])
+@pytest.mark.parametrize("dtype,y32,parts", [(torch.bfloat16, False, "ys"), (torch.bfloat16, True, "y"), (torch.float32, True, "es"), (torch.bfloat16, False, "")])
+def test_finish_rows(rows, width, real, dtype, y32, parts):
+    from triforce_amd import ops_latent as ol
+    g = torch.Generator(device=DEV).manual_seed(rows + width)
+
+    def rand(*s):
+        t = torch.randn(*s, generator=g, device=DEV)
+        t[..., real:] = 0
+        return t
+    x, w, yw, step = rand(rows, width), rand(width), rand(width), rand(width)
+    y, embed, ids = rand(rows, width).to(torch.float32 if y32 else dtype), rand(50, width).to(dtype), torch.randint(0, 50, (rows,), generator=g, device=DEV)
+    want = embed[ids].double() if "e" in parts else x.double()
+    if "y" in parts:
+        want = want + y.double() / torch.sqrt(y.double().square().sum(-1, keepdim=True) / real + 1e-5) * yw.double()
+    if "s" in parts:
+        want = want + step.double()
+    h = ol.finish(x, w, 1e-5, real, dtype, **(dict(embed=embed, ids=ids) if "e" in parts else {}), **(dict(y=y, y_w=yw) if "y" in parts else {}),
+                  step=step if "s" in parts else None)
+    assert ((x.double() - want).abs() <= 2e-6 * (1 + want.abs())).all()
+    normed = want / torch.sqrt(want.square().sum(-1, keepdim=True) / real + 1e-5) * w.double()
+    assert ((h.double() - normed).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 0) * normed.abs() + 4e-6 * (1 + normed.abs())).all()

@@ -48,7 +48,7 @@ class LatentLayer:
         self.w_in = ol.TileWeight(torch.cat(parts))
         uq = mat("mix.uq").view(g.H, m.dim + m.rot_dim, m.q_rank)
         self.w_uq = ol.TileWeight(torch.cat([_grow(uq[:, :m.dim], g.H, g.N, g.Q), _grow(uq[:, m.dim:], g.H, g.R, g.Q)], 1)
-                                  .reshape(g.H * (g.N + g.R), g.Q), panel_major=True)
+                                  .reshape(g.H * (g.N + g.R), g.Q))
         uk = _grow(mat("mix.uk").view(g.H, m.dim, m.kv_rank), g.H, g.N, g.C)
         uv = _grow(mat("mix.uv").view(g.H, m.vdim, m.kv_rank), g.H, g.V, g.C)
         self.w_uk_t = ol.TileWeight(uk.transpose(1, 2).contiguous(), packed_only=True)          # decode: query -> latent

@@ -65,13 +65,14 @@ def pack_tiles(w, chunk_major=False):
 
 class TileWeight:
     """A (groups of) [n, k] weight(s): packed for the skinny kernel and, unless ``packed_only``, row-major for the library GEMM
-    of the prefill.  Wide bfloat16 weights (a panel or more per CU) are packed chunk-major, which the one-workgroup-per-CU form of
-    the kernel streams, unless ``panel_major`` says that their epilogue has no such form (TFL_EPI_QUERY)."""
+    of the prefill.  Wide and long bfloat16 weights (a panel or more per CU, k from 2 048 on) are packed chunk-major, which the
+    one-workgroup-per-CU form of the kernel streams; a shorter k is over before its look-ahead pays (4 096 x 256 at 32 rows 4.6 us with
+    a workgroup per panel, 6.4 with one per CU; 6 144 x 1 536 10.0 and 11.1)."""
 
-    def __init__(self, w, packed_only=False, panel_major=False):
+    def __init__(self, w, packed_only=False):
         w3 = w if w.dim() == 3 else w.unsqueeze(0)
         self.groups, self.n, self.k = w3.shape
-        self.chunk_major = not panel_major and self.groups == 1 and w.dtype == torch.bfloat16 and self.n >= 256 * 16
+        self.chunk_major = self.groups == 1 and w.dtype == torch.bfloat16 and self.n >= 256 * 16 and self.k >= 2048
         self.packed = pack_tiles(w3, self.chunk_major)
         self.w = None if packed_only else w.contiguous()
         self.dtype, self.device = w.dtype, w.device
