@@ -205,3 +205,37 @@ def test_finish_rows(rows, width, real, dtype, y32, parts):
     assert ((x.double() - want).abs() <= 2e-6 * (1 + want.abs())).all()
     normed = want / torch.sqrt(want.square().sum(-1, keepdim=True) / real + 1e-5) * w.double()
     assert ((h.double() - normed).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 0) * normed.abs() + 4e-6 * (1 + normed.abs())).all()
+
+
+# splits dealt over unequal rows (2 to 64 rows), one row and more than 64 rows (the same number each); idle rows, rows right behind a
+# chunk's edge; the sized attention and the general one
+@pytest.mark.parametrize("rows,nsplit", [(1, 7), (2, 1), (5, 3), (33, 4), (64, 2), (65, 3)])
+@pytest.mark.parametrize("D", [128, 96])
+def test_step_splits_over_rows(rows, nsplit, D):
+    from triforce_amd import ops_hybrid as oh
+    g = torch.Generator(device=DEV).manual_seed(rows * 10 + nsplit)
+    H, G, chunk, pages = 8, 2, 640, 40
+    lens = [0 if b % 9 == 5 else (chunk * (1 + b % 2) + 1 if b % 4 == 3 else 1 + (b * 331) % 1200) for b in range(rows)]
+    width = 2 * H * D + 2 * G * D
+    raw = torch.randn(rows, width, generator=g, device=DEV)
+    pool = _bf(g, pages * 64, G * 2 * D)
+    norm = torch.ones(D, device=DEV)
+    angle = torch.arange(2000, device=DEV)[:, None] * 0.01 * torch.arange(1, 9, device=DEV)
+
+    def operand(which, splits):
+        own = torch.stack([torch.randperm(pages, generator=torch.Generator().manual_seed(b))[:22].to(torch.int32) for b in which])
+        table = torch.arange(22 * len(which), dtype=torch.int32).view(len(which), 22).to(DEV)          # pages of its own: the step writes
+        cache = pool.view(pages, 64, -1)[own.reshape(-1).long().to(DEV)].reshape(-1, G * 2 * D).clone()
+        attn = dict(q_norm=norm, k_norm=norm, cos=angle.cos().float().contiguous(), sin=angle.sin().float().contiguous(), cache=cache, table=table,
+                    q_off=0, k_off=H * D, v_off=H * D + G * D, gate_off=H * D + 2 * G * D, half=8, max_pos=2000, H=H, G=G, D=D, D_real=D, V=D, chunk=chunk,
+                    scale=0.1, out_scale=1.0)
+        klen = torch.tensor([lens[b] for b in which], dtype=torch.int32, device=DEV)
+        step = oh.MixerStep(raw[list(which)].contiguous(), klen, 1e-5, torch.bfloat16, attn=attn, max_keys=1300, nsplit=splits)
+        return step.run().operand().permute(1, 0, 2).reshape(len(which), -1).double()
+    got = operand(range(rows), nsplit)
+    for b in range(rows):
+        alone = operand([b], 1)[0]
+        if lens[b] == 0:
+            assert not got[b].any()
+        # the same fp32 sums in another order, then one rounding to bfloat16 each
+        assert ((got[b] - alone).abs() <= 2.0 ** -7 * alone.abs() + 1e-5).all()

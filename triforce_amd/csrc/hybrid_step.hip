@@ -11,10 +11,73 @@
 
 template <typename T> struct StepCfg { static constexpr int PARTS = sizeof(T) == 2 ? 2 : 1; };
 
+// Which part of which row's keys a workgroup takes.  The launch has rows * nsplit slots per key / value head; rows of a batch see
+// different numbers of pages (and after a chunk's edge only a few), so up to 64 rows the slots are dealt by pages: the same number of
+// them, q, to every slot, row r having ceil(pages / q) slots in a row.  Every workgroup works it out from the rows' lengths (one
+// load, three reductions); the first one leaves each row's first slot and slots for the merge.  More rows: nsplit slots each.
+struct Slots { int row, first, pages, t0; };                  // the row that owns a slot (-1: none), its first slot, pages per slot, first page
+
+__device__ __forceinline__ int first_visible(int n, int chunk) { return n > 0 && chunk > 0 ? (n - 1) / chunk * chunk : 0; }
+
+__device__ __forceinline__ Slots find_slot(const int32_t* klen, int rows, int nsplit, int chunk, int slot, int32_t* info) {
+    const int lane = threadIdx.x & 63;
+    Slots f;
+    if (rows == 1 || rows > 64) {
+        f.row = slot / nsplit;
+        const int n = klen[f.row];
+        f.t0 = first_visible(n, chunk) / TFL_PAGE;
+        f.first = f.row * nsplit;
+        f.pages = n > 0 ? ((n - 1) / TFL_PAGE + 1 - f.t0 + nsplit - 1) / nsplit : 1;
+        return f;
+    }
+    const int n = lane < rows ? klen[lane] : 0, t0 = first_visible(n, chunk) / TFL_PAGE;
+    const int p = n > 0 ? (n - 1) / TFL_PAGE + 1 - t0 : 0;
+    int total = p, most = p;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        total += __shfl_xor(total, o, 64);
+        most = max(most, __shfl_xor(most, o, 64));
+    }
+    const int slots = rows * nsplit, least = max(1, (most + 255) / 256);                     // (the merge weighs 256 slots of a row)
+    // sum of ceil(p / q) <= total / q + rows: this q always fits, a smaller one often does
+    const int fits = max(least, slots > rows ? (total + slots - rows - 1) / (slots - rows) : most);
+    int q = max(least, (total + slots - 1) / slots), c = 0, upto = 0;
+    for (int k = 0;; ++k) {
+        if (k == 3 || q > fits) q = fits;
+        c = (p + q - 1) / q;
+        upto = c;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(upto, o, 64);
+            if (lane >= o) upto += t;
+        }
+        if (q == fits || __shfl(upto, 63, 64) <= slots) break;
+        ++q;
+    }
+    if (info && threadIdx.x < rows) {                         // (wave 0)
+        info[2 * lane] = upto - c;
+        info[2 * lane + 1] = c;
+    }
+    const uint64_t over = __ballot(upto > slot);
+    f.row = over ? __ffsll((long long)over) - 1 : -1;
+    const int at = over ? f.row : 0;
+    f.first = __shfl(upto - c, at, 64);
+    f.t0 = __shfl(t0, at, 64);
+    f.pages = q;
+    return f;
+}
+
+struct AttnStep : TfhAttnStep {
+    int slots;                                                // rows * nsplit
+    // ws: partial values [slots][H][V], maxima and sums [slots][H][2], first slot and slots of each row [rows][2]
+    __device__ __forceinline__ float* stats() const { return ws + (int64_t)slots * H * V; }
+    __device__ __forceinline__ int32_t* info() const { return reinterpret_cast<int32_t*>(ws + (int64_t)slots * H * (V + 2)); }
+};
+
 // ------------------------------------------------------------------------------------------------------------ attention
 // NTW: 16-wide value tiles per wave at most.
 template <typename T, int NTW>
-__device__ __forceinline__ void attn_part(const TfhAttnStep& a, const float* raw, int n, int row, int bid, float eps, char* smem) {
+__device__ __forceinline__ void attn_part(const AttnStep& a, const float* raw, int n, int row, int gh, int slot, int p_beg, int p_end, float eps, char* smem) {
     typedef typename El<T>::Frag Frag;
     constexpr int KT = TFL_PAGE, EPV = 16 / sizeof(T), PARTS = StepCfg<T>::PARTS, NT = 256, LDP = KT + EPV;
     const int D = a.D, V = a.V, dk = D >> 5, ldk = D + EPV, ldv = V + 2 * EPV;
@@ -25,22 +88,10 @@ __device__ __forceinline__ void attn_part(const TfhAttnStep& a, const float* raw
     float* red = (float*)(Ps + PARTS * 16 * LDP);             // [4][16]
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, i = lane & 15;
     const int hpg = a.H / a.G, tiles_h = (hpg + 15) >> 4;
-    const int split = bid % a.nsplit, gh = bid / a.nsplit, grp = gh / tiles_h, ht = gh - grp * tiles_h;
+    const int grp = gh / tiles_h, ht = gh - grp * tiles_h;
     const int h0 = grp * hpg + 16 * ht, nh = min(16, hpg - 16 * ht);
-    const int first_key = n > 0 && a.chunk > 0 ? (n - 1) / a.chunk * a.chunk : 0;
-    const int t0 = first_key / KT, t1 = n > 0 ? (n - 1) / KT + 1 : 0;
-    const int per = (t1 - t0 + a.nsplit - 1) / a.nsplit;
-    const int t_beg = min(t0 + split * per, t1), t_end = min(t1, t_beg + per);
-    const int rows = gridDim.y;
-    float* ml = a.ws + (int64_t)rows * a.H * a.nsplit * V;
-    if (t_beg >= t_end) {                                     // (idle rows, splits past the last page)
-        if (tid < nh) {
-            float* p = ml + (((int64_t)row * a.H + h0 + tid) * a.nsplit + split) * 2;
-            p[0] = NEG_INF;
-            p[1] = 0.f;
-        }
-        return;
-    }
+    const int first_key = first_visible(n, a.chunk), t_beg = p_beg, t_end = p_end;
+    float* ml = a.stats();
     const int32_t* tab = a.table + (int64_t)row * a.table_ld;
     const int64_t ld_c = (int64_t)a.G * (D + V);
     auto rows_of = [&](int t) {
@@ -154,7 +205,7 @@ __device__ __forceinline__ void attn_part(const TfhAttnStep& a, const float* raw
     if (g == 0) red[wave * 16 + i] = l_run;
     __syncthreads();
     if (i < nh) {
-        const int64_t at = ((int64_t)row * a.H + h0 + i) * a.nsplit + split;
+        const int64_t at = (int64_t)slot * a.H + h0 + i;
 #pragma unroll
         for (int x = 0; x < NTW; ++x) {
             const int col = 16 * (wave * NTW + x) + 4 * g;
@@ -170,40 +221,36 @@ __device__ __forceinline__ void attn_part(const TfhAttnStep& a, const float* raw
 // The same for known sizes, bfloat16: 32 * DK entries of query-key size, 16 * DV of value size.  The waves walk their own 32-key tiles
 // without a barrier: rows come from memory whole (the next tile's while this one is used), pass through a piece of LDS that only the wave
 // touches, and the result registers of a tile's two score products are the weight operand of its value products.  The waves meet once,
-// at the end.
+// at the end.  Keys and values of a tile pass through the same piece, one after the other: 41 KB a workgroup, so that with 168
+// registers three of them fit a CU and the recurrences' workgroups (all latency) run beside the attention's (all bandwidth) instead
+// of behind them.  What is left is a chain of some 12 us (launch, length, page, first rows, norms, merge of the waves) in front of and
+// behind the stream.  Step and merge, 41 KB and dealt slots against 77 KB and nsplit slots a row: 1 x 8 192 keys 23.7 -> 20.9 us, 8 x 4 096 51.3 ->
+// 46.9, 8 rows of 808 to 8 157 keys 59.1 -> 55.5, 32 around 3 000 139.5 -> 123.8.
 template <int DK, int DV>
 struct SizedStep {
-    static constexpr int KT = 32, D = 32 * DK, V = 16 * DV, LDK = D + 8, LDV = V + 16, TILE = KT * (LDK + LDV);
+    static constexpr int KT = 32, D = 32 * DK, V = 16 * DV, LDK = D + 8, LDV = V + 16, TILE = KT * (LDK > LDV ? LDK : LDV);
     static constexpr size_t LDS = sizeof(bf16) * (4 * TILE + 16 * LDK) + sizeof(float) * 128;
     static_assert(4 * 16 * V * sizeof(float) <= sizeof(bf16) * 4 * TILE, "the waves' results reuse the tiles");
 };
 
 template <int DK, int DV>
-__device__ __forceinline__ void attn_part_sized(const TfhAttnStep& a, const float* raw, int n, int row, int bid, float eps, char* smem) {
+__device__ __forceinline__ void attn_part_sized(const AttnStep& a, const float* raw, int n, int row, int gh, int slot, int p_beg, int p_end, float eps, char* smem) {
     typedef SizedStep<DK, DV> Z;
     constexpr int KT = Z::KT, D = Z::D, V = Z::V, LDK = Z::LDK, LDV = Z::LDV, KP = D / 8, VP = V / 8, NK = KT * KP / 64, NV = KT * VP / 64;
     static_assert(64 % KP == 0 && 64 % VP == 0, "whole rows per load");
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15;
-    bf16* Kt = (bf16*)smem + wave * Z::TILE;                  // this wave's [KT][LDK] and [KT][LDV]
-    bf16* Vt = Kt + KT * LDK;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int lane = tid & 63, g = lane >> 4, i = lane & 15;
+    bf16* Kt = (bf16*)smem + wave * Z::TILE;                  // this wave's [KT][LDK], then [KT][LDV]
+    bf16* Vt = Kt;
     bf16* Qs = (bf16*)smem + 4 * Z::TILE;                     // [16][LDK]
     float* red = (float*)(Qs + 16 * LDK);                     // [4][16] maxima, [4][16] sums
     const int hpg = a.H / a.G, tiles_h = (hpg + 15) >> 4;
-    const int split = bid % a.nsplit, gh = bid / a.nsplit, grp = gh / tiles_h, ht = gh - grp * tiles_h;
+    const int grp = gh / tiles_h, ht = gh - grp * tiles_h;
     const int h0 = grp * hpg + 16 * ht, nh = min(16, hpg - 16 * ht);
-    const int first_key = n > 0 && a.chunk > 0 ? (n - 1) / a.chunk * a.chunk : 0;
-    const int t0 = first_key / KT, t1 = n > 0 ? (n - 1) / KT + 1 : 0;
-    const int per = (t1 - t0 + a.nsplit - 1) / a.nsplit;
-    const int t_beg = min(t0 + split * per, t1), t_end = min(t1, t_beg + per);
-    float* ml = a.ws + (int64_t)gridDim.y * a.H * a.nsplit * V;
-    if (t_beg >= t_end) {                                     // (idle rows, splits past the last page)
-        if (tid < nh) {
-            float* p = ml + (((int64_t)row * a.H + h0 + tid) * a.nsplit + split) * 2;
-            p[0] = NEG_INF;
-            p[1] = 0.f;
-        }
-        return;
-    }
+    const int first_key = first_visible(n, a.chunk);
+    constexpr int PT = TFL_PAGE / KT;                         // tiles per page; the chunk may begin inside the first one
+    const int t_beg = max(p_beg * PT, first_key / KT), t_end = min(p_end * PT, (n - 1) / KT + 1);
+    float* ml = a.stats();
     const int32_t* tab = a.table + (int64_t)row * a.table_ld;
     const int64_t ld_c = (int64_t)a.G * (D + V);
     auto rows_of = [&](int t) {
@@ -211,17 +258,25 @@ __device__ __forceinline__ void attn_part_sized(const TfhAttnStep& a, const floa
         return (bf16*)a.cache + ((int64_t)(pg < 0 ? 0 : (pg >= a.n_pages ? (int)a.n_pages - 1 : pg)) * TFL_PAGE + t * KT % TFL_PAGE) * ld_c;
     };
     u32x4 prek[NK], prev[NV];
-    auto fetch = [&](int t) {
-        const bf16* base = rows_of(t);
+    const uint32_t row_bytes = 2 * (uint32_t)ld_c;            // (G * (D + V) elements: a tile stays far below 2^32 bytes)
+    auto fetch_k = [&](int t) {
+        const char* base = reinterpret_cast<const char*>(rows_of(t) + grp * D);
         const int left = n - 1 - t * KT;                      // rows behind the last key repeat it (masked)
 #pragma unroll
         for (int j = 0; j < NK; ++j)
-            prek[j] = *reinterpret_cast<const u32x4*>(base + (int64_t)min(lane / KP + j * (64 / KP), left) * ld_c + grp * D + 8 * (lane % KP));
+            prek[j] = *reinterpret_cast<const u32x4*>(base + ((uint32_t)min(lane / KP + j * (64 / KP), left) * row_bytes + 16u * (lane % KP)));
+    };
+    auto fetch_v = [&](int t) {
+        const char* base = reinterpret_cast<const char*>(rows_of(t) + a.G * D + grp * V);
+        const int left = n - 1 - t * KT;
 #pragma unroll
         for (int j = 0; j < NV; ++j)
-            prev[j] = *reinterpret_cast<const u32x4*>(base + (int64_t)min(lane / VP + j * (64 / VP), left) * ld_c + a.G * D + grp * V + 8 * (lane % VP));
+            prev[j] = *reinterpret_cast<const u32x4*>(base + ((uint32_t)min(lane / VP + j * (64 / VP), left) * row_bytes + 16u * (lane % VP)));
     };
-    if (t_beg + wave < t_end) fetch(t_beg + wave);
+    if (t_beg + wave < t_end) {
+        fetch_k(t_beg + wave);
+        fetch_v(t_beg + wave);
+    }
     const int p = min(n - 1, a.max_pos - 1);
     const float *cs = a.cos + (int64_t)p * a.half, *sn = a.sin + (int64_t)p * a.half;
     for (int r = wave; r < 16; r += 4) {
@@ -245,18 +300,14 @@ __device__ __forceinline__ void attn_part_sized(const TfhAttnStep& a, const floa
     for (int t = t_beg + wave; t < t_end; t += 4) {
         const int k0 = t * KT, fresh = n - 1 - k0;            // tile row of the new key (< KT: in this tile)
         const bool edge = fresh < KT;
+        asm("" : "+v"(lane), "+v"(g), "+v"(i));               // (opaque once per tile: hoisted addresses would take the registers)
 #pragma unroll
         for (int j = 0; j < NK; ++j) {
             const int r = lane / KP + j * (64 / KP);
             *reinterpret_cast<u32x4*>(Kt + r * LDK + 8 * (lane % KP)) = edge && r >= fresh ? u32x4{0, 0, 0, 0} : prek[j];
         }
-#pragma unroll
-        for (int j = 0; j < NV; ++j) {
-            const int r = lane / VP + j * (64 / VP);
-            *reinterpret_cast<u32x4*>(Vt + r * LDV + 8 * (lane % VP)) = edge && r >= fresh ? u32x4{0, 0, 0, 0} : prev[j];
-        }
+        bf16* dst = edge ? rows_of(t) + (int64_t)fresh * ld_c : nullptr;
         if (edge) {
-            bf16* dst = rows_of(t) + (int64_t)fresh * ld_c;
             const float* src = raw + a.k_off + grp * D;
             float k[4];
             head_norm_rotate([src](int e) { return src[e]; }, D, a.D_real, a.k_norm, eps, cs, sn, a.half, lane, k);
@@ -266,14 +317,9 @@ __device__ __forceinline__ void attn_part_sized(const TfhAttnStep& a, const floa
                     Kt[fresh * LDK + lane + 64 * j] = (bf16)k[j];
                     if (ht == 0) dst[grp * D + lane + 64 * j] = (bf16)k[j];
                 }
-            for (int e = lane; e < V; e += 64) {
-                const bf16 v = (bf16)raw[a.v_off + grp * V + e];
-                Vt[fresh * LDV + e] = v;
-                if (ht == 0) dst[a.G * D + grp * V + e] = v;
-            }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");            // (one wave's LDS accesses stay in order; so must the compiler)
-        if (t + 4 < t_end) fetch(t + 4);
+        if (t + 4 < t_end) fetch_k(t + 4);
         f32x4 s[2];
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
@@ -281,6 +327,21 @@ __device__ __forceinline__ void attn_part_sized(const TfhAttnStep& a, const floa
 #pragma unroll
             for (int c = 0; c < DK; ++c) s[kt] = El<bf16>::mma(load_frag(Kt + (16 * kt + i) * LDK + 32 * c + 8 * g), qf[c], s[kt]);
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");            // the keys are used up: the values take their place
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const int r = lane / VP + j * (64 / VP);
+            *reinterpret_cast<u32x4*>(Vt + r * LDV + 8 * (lane % VP)) = edge && r >= fresh ? u32x4{0, 0, 0, 0} : prev[j];
+        }
+        if (edge) {
+            for (int e = lane; e < V; e += 64) {
+                const bf16 v = (bf16)raw[a.v_off + grp * V + e];
+                Vt[fresh * LDV + e] = v;
+                if (ht == 0) dst[a.G * D + grp * V + e] = v;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (t + 4 < t_end) fetch_v(t + 4);
         float mx = NEG_INF;
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
@@ -307,10 +368,14 @@ __device__ __forceinline__ void attn_part_sized(const TfhAttnStep& a, const floa
                 lo[4 * kt + r] = (bf16)(w - (float)(bf16)w);
             }
         l_run = l_run * alpha + sum;
+        if (!__all(alpha == 1.0f)) {                          // (most tiles leave every maximum where it was)
+#pragma unroll
+            for (int d = 0; d < DV; ++d)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[d][r] *= alpha;
+        }
 #pragma unroll
         for (int d = 0; d < DV; ++d) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) o[d][r] *= alpha;
             const bf16x8 f = load_frag_t(Vt, LDV, 4 * g, 16 + 4 * g, 16 * d, i);
             o[d] = El<bf16>::mma(f, hi, o[d]);
             o[d] = El<bf16>::mma(f, lo, o[d]);
@@ -343,7 +408,7 @@ __device__ __forceinline__ void attn_part_sized(const TfhAttnStep& a, const floa
                 const float mw = red[w * 16 + i];
                 l += mw == NEG_INF ? 0.f : red[64 + w * 16 + i] * __builtin_amdgcn_exp2f((mw - m) * LOG2E);
             }
-            float* q = ml + (((int64_t)row * a.H + h0 + i) * a.nsplit + split) * 2;
+            float* q = ml + ((int64_t)slot * a.H + h0 + i) * 2;
             q[0] = m;
             q[1] = l;
         }
@@ -358,7 +423,7 @@ __device__ __forceinline__ void attn_part_sized(const TfhAttnStep& a, const floa
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] += x[r];
         }
-        *reinterpret_cast<f32x4*>(a.ws + (((int64_t)row * a.H + h0 + h) * a.nsplit + split) * V + c) = v;
+        *reinterpret_cast<f32x4*>(a.ws + ((int64_t)slot * a.H + h0 + h) * V + c) = v;
     }
 }
 
@@ -461,39 +526,53 @@ __device__ __forceinline__ void rec_part(const TfhRecStep& a, int slice, const f
     }
 }
 
-// attn_blocks first (they take longer), then the recurrence's.  DK > 0: the sized attention.
+// All rows' attention first (it takes longer), then the recurrences: attn_blocks and rec_blocks of them in all.  DK > 0: the sized
+// attention.
 template <typename T, int NTW, int DK, int DV>
-__global__ __launch_bounds__(256) void step_kernel(const TfhAttnStep a, const TfhRecStep r, int attn_blocks, int slice,
+__global__ __launch_bounds__(256, DK > 0 ? 3 : 1) void step_kernel(const AttnStep a, const TfhRecStep r, int attn_blocks, int rec_per_row, int slice, int rows,
                                                    const float* __restrict__ raw, int64_t ld_raw, const int32_t* __restrict__ klen, float eps) {
     extern __shared__ __align__(32) char smem[];
-    const int row = blockIdx.y, n = klen[row];
-    const float* rr = raw + (int64_t)row * ld_raw;
     if ((int)blockIdx.x >= attn_blocks) {
-        rec_part<T>(r, slice, rr, n, row, blockIdx.x - attn_blocks, smem);
-    } else if constexpr (DK > 0) {
-        attn_part_sized<DK, DV>(a, rr, n, row, blockIdx.x, eps, smem);
-    } else {
-        attn_part<T, NTW>(a, rr, n, row, blockIdx.x, eps, smem);
+        const int id = blockIdx.x - attn_blocks, row = id / rec_per_row;
+        rec_part<T>(r, slice, raw + (int64_t)row * ld_raw, klen[row], row, id - row * rec_per_row, smem);
+        return;
     }
+    const int gh = blockIdx.x / a.slots, slot = blockIdx.x - gh * a.slots;
+    const Slots f = find_slot(klen, rows, a.nsplit, a.chunk, slot, blockIdx.x == 0 ? a.info() : nullptr);
+    if (f.row < 0) return;
+    const int n = klen[f.row], p_beg = f.t0 + (slot - f.first) * f.pages, p_end = n > 0 ? min((n - 1) / TFL_PAGE + 1, p_beg + f.pages) : 0;
+    if (p_beg >= p_end) {                                     // (more than 64 rows: slots past the last page)
+        const int hpg = a.H / a.G, tiles_h = (hpg + 15) >> 4, grp = gh / tiles_h, h0 = grp * hpg + 16 * (gh - grp * tiles_h), tid = threadIdx.x;
+        if (tid < min(16, grp * hpg + hpg - h0)) {
+            float* p = a.stats() + ((int64_t)slot * a.H + h0 + tid) * 2;
+            p[0] = NEG_INF;
+            p[1] = 0.f;
+        }
+        return;
+    }
+    const float* rr = raw + (int64_t)f.row * ld_raw;
+    if constexpr (DK > 0) attn_part_sized<DK, DV>(a, rr, n, f.row, gh, slot, p_beg, p_end, eps, smem);
+    else attn_part<T, NTW>(a, rr, n, f.row, gh, slot, p_beg, p_end, eps, smem);
 }
 
 // ------------------------------------------------------------------------------------------------------------ operand
 template <typename T>
-__global__ __launch_bounds__(256) void step_out_kernel(const TfhAttnStep a, const TfhRecStep r, int attn_blocks, int groups,
+__global__ __launch_bounds__(256) void step_out_kernel(const AttnStep a, const TfhRecStep r, int attn_blocks, int groups,
                                                        const float* __restrict__ raw, int64_t ld_raw, T* __restrict__ act, int64_t ld_act,
                                                        int64_t act_oct, float eps) {
     __shared__ float wgt[256];
     __shared__ float red[8];
     __shared__ f32x4 acc[256];
-    const int row = blockIdx.y, tid = threadIdx.x, rows = gridDim.y;
+    const int row = blockIdx.y, tid = threadIdx.x;
     const float* rr = raw + (int64_t)row * ld_raw;
     T* dst = act + (int64_t)row * ld_act;
     if ((int)blockIdx.x < attn_blocks) {                      // one head: splits merged, output gate
-        const int head = blockIdx.x, V = a.V, ns = a.nsplit;
-        const int64_t at = ((int64_t)row * a.H + head) * ns;
-        const float* ml = a.ws + (int64_t)rows * a.H * ns * V + 2 * at;
-        const float ls = tid < ns ? ml[2 * tid + 1] : 0.f;
-        const float ms = ls > 0.f ? ml[2 * tid] : NEG_INF;
+        const bool dealt = gridDim.y > 1 && gridDim.y <= 64;
+        const int head = blockIdx.x, V = a.V, first = dealt ? a.info()[2 * row] : row * a.nsplit, ns = dealt ? a.info()[2 * row + 1] : a.nsplit;
+        const int64_t at = (int64_t)first * a.H + head;        // + s * H: slot s of the row
+        const float* ml = a.stats() + 2 * at;
+        const float ls = tid < ns ? ml[2 * (int64_t)tid * a.H + 1] : 0.f;
+        const float ms = ls > 0.f ? ml[2 * (int64_t)tid * a.H] : NEG_INF;
         float m = ms;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
@@ -510,7 +589,7 @@ __global__ __launch_bounds__(256) void step_out_kernel(const TfhAttnStep a, cons
             for (int s = gr; s < ns; s += ng) {
                 const float f = wgt[s];
                 if (f > 0.f) {                                // (an empty split's partial row was never written)
-                    const f32x4 z = *reinterpret_cast<const f32x4*>(a.ws + (at + s) * V + 4 * vq);
+                    const f32x4 z = *reinterpret_cast<const f32x4*>(a.ws + (at + (int64_t)s * a.H) * V + 4 * vq);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] = fmaf(z[e], f, v[e]);
                 }
@@ -519,7 +598,7 @@ __global__ __launch_bounds__(256) void step_out_kernel(const TfhAttnStep a, cons
         acc[tid] = v;
         __syncthreads();
         if (gr == 0) {
-            for (int k = 1; k < min(ng, ns); ++k) {
+            for (int k = 1; k < ng; ++k) {
                 const f32x4 z = acc[k * nq + vq];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] += z[e];
@@ -591,14 +670,16 @@ __global__ __launch_bounds__(256) void step_out_kernel(const TfhAttnStep a, cons
 
 extern "C" int64_t tfh_attn_step_ws_floats(int rows, int H, int V, int nsplit) {
     if (rows < 1 || H < 1 || V < 1 || nsplit < 1) return 0;
-    return (int64_t)rows * H * nsplit * (V + 2);
+    return (int64_t)rows * H * nsplit * (V + 2) + 2 * (int64_t)rows;
 }
 
-// Two workgroups per CU (512) as long as a split keeps a page of keys.
+// Two workgroups per CU (512), four splits a row where the batch is large (unequal rows are dealt by splits), as long as a split
+// keeps a page of keys.  us with the merge: 8 rows of 9 000 - 5 063 at 4 / 8 / 12 splits 58.4 / 55.5 / 56.2, 16 rows around 3 000 at 2 / 4 /
+// 8 92.8 / 68.8 / 72.4, 32 rows 141.7 / 123.8 / 126.4, one row of 8 192 at 16 / 32 / 64 / 128 22.4 / 20.2 / 20.9 / 26.4.
 extern "C" int tfh_attn_step_pick_nsplit(int rows, int H, int G, int max_keys) {
     if (rows < 1 || H < 1 || G < 1 || max_keys < 1) return 1;
     const int groups = G * ((H / G + 15) / 16);
-    int n = 512 / (rows * groups);
+    int n = 512 / (rows * groups) > 4 ? 512 / (rows * groups) : 4;
     const int cap = (max_keys + TFL_PAGE - 1) / TFL_PAGE;
     if (n > cap) n = cap;
     if (n > TFH_MAX_SPLIT) n = TFH_MAX_SPLIT;
@@ -642,7 +723,7 @@ static size_t step_lds(int dtype, const TfhAttnStep* a, const TfhRecStep* r) {
 }
 
 template <typename T, int NTW, int DK, int DV>
-static int launch_step(const TfhAttnStep& a, const TfhRecStep& r, int attn_blocks, int rec_blocks, int slice, size_t lds, const float* raw,
+static int launch_step(const AttnStep& a, const TfhRecStep& r, int attn_blocks, int rec_blocks, int slice, size_t lds, const float* raw,
                        int64_t ld_raw, const int32_t* klen, int rows, float eps, hipStream_t st) {
     auto k = step_kernel<T, NTW, DK, DV>;
     static bool attr = false;
@@ -652,7 +733,7 @@ static int launch_step(const TfhAttnStep& a, const TfhRecStep& r, int attn_block
         attr = true;
     }
     if constexpr (DK > 0) lds = SizedStep<DK, DV>::LDS > lds ? SizedStep<DK, DV>::LDS : lds;
-    hipLaunchKernelGGL(k, dim3(attn_blocks + rec_blocks, rows), dim3(256), lds, st, a, r, attn_blocks, slice, raw, ld_raw, klen, eps);
+    hipLaunchKernelGGL(k, dim3((unsigned)((int64_t)(attn_blocks + rec_blocks) * rows)), dim3(256), lds, st, a, r, attn_blocks * rows, rec_blocks, slice, rows, raw, ld_raw, klen, eps);
     TFL_LAUNCH_CHECK();
     return TF_OK;
 }
@@ -660,11 +741,12 @@ static int launch_step(const TfhAttnStep& a, const TfhRecStep& r, int attn_block
 extern "C" int tfh_step(const TfhAttnStep* pa, const TfhRecStep* pr, const float* raw, int64_t ld_raw, const int32_t* klen, int rows, float eps,
                         int dtype, void* stream) {
     if ((!pa && !pr) || !raw || !klen || rows < 1 || rows > 65535 || (ld_raw & 3) || (dtype != 0 && dtype != 1)) return TF_EINVAL;
-    TfhAttnStep a = {};
+    AttnStep a = {};
     TfhRecStep r = {};
     int ab = 0, rb = 0, slice = 64, rc;
     if (pa) {
-        a = *pa;
+        static_cast<TfhAttnStep&>(a) = *pa;
+        a.slots = rows * a.nsplit;
         if ((rc = check_attn(a, ld_raw)) != TF_OK) return rc;
         ab = a.G * ((a.H / a.G + 15) / 16) * a.nsplit;
     }
@@ -699,11 +781,12 @@ extern "C" int tfh_step_out(const TfhAttnStep* pa, const TfhRecStep* pr, const f
                             int64_t act_oct, int rows, float eps, int dtype, void* stream) {
     if ((!pa && !pr) || !raw || !act || rows < 1 || rows > 65535 || (ld_raw & 3) || ld_act < 8 || (ld_act & 7) || act_oct < 8 || (act_oct & 7)
         || (dtype != 0 && dtype != 1)) return TF_EINVAL;
-    TfhAttnStep a = {};
+    AttnStep a = {};
     TfhRecStep r = {};
     int ab = 0, groups = 0, rc;
     if (pa) {
-        a = *pa;
+        static_cast<TfhAttnStep&>(a) = *pa;
+        a.slots = rows * a.nsplit;
         if ((rc = check_attn(a, ld_raw)) != TF_OK) return rc;
         ab = a.H;
     }
