@@ -78,6 +78,13 @@ int tfl_gemm(const TflGemm* a, int dtype, int epilogue, void* stream);
 int tfl_decode_prep(int32_t* len, const int32_t* table, int table_ld, int table_cols, int32_t* pos, int32_t* slot, int32_t* klen,
                     int rows, void* stream);
 
+/* float32 products of many rows on the bfloat16 matrix cores (csrc/split_gemm.hip): out[m*ld_out + n] = sum over k of x[m*ld_x + k] * w[n*k_total + k].
+ * n % 16 == 0, k % 32 == 0, 16-byte aligned pointers and rows; k is cut into `splits` parts (0: the library's choice).
+ * ws: tfl_split_gemm_ws_floats floats for the same sizes and splits. */
+int64_t tfl_split_gemm_ws_floats(int rows, int n, int k, int splits);
+int tfl_split_gemm(const float* w, const float* x, int64_t ld_x, float* out, int64_t ld_out, float* ws, int64_t ws_floats, int rows, int n, int k,
+                   int splits, void* stream);
+
 /* table[row * table_ld + column] = page for n (at most TFL_MAX_ENTRIES) host triples {row, column, page}: pages handed out between
  * two decode steps.  The triples are kernel arguments (nothing is read after the call returns). */
 #define TFL_MAX_ENTRIES 64

@@ -239,3 +239,38 @@ def test_step_splits_over_rows(rows, nsplit, D):
             assert not got[b].any()
         # the same fp32 sums in another order, then one rounding to bfloat16 each
         assert ((got[b] - alone).abs() <= 2.0 ** -7 * alone.abs() + 1e-5).all()
+
+
+# float32 on the bfloat16 matrix cores: below and above a tile of 256 x 128, waves without rows, parts of k of unequal length and empty ones
+@pytest.mark.parametrize("rows,n,k,splits", [(1, 16, 32, 1), (17, 272, 96, 2), (128, 256, 64, 3), (129, 528, 1056, 5), (257, 48, 4096, 8), (700, 2064, 1536, 0),
+                                             (64, 2304, 4096, 1), (300, 16, 32, 0)])
+def test_split_float32_product(rows, n, k, splits):
+    from triforce_amd import ops_tile as ot
+    g = torch.Generator(device=DEV).manual_seed(rows + n)
+    wide = torch.randn(rows, k + 36, generator=g, device=DEV)
+    w = torch.randn(n, k, generator=g, device=DEV) * torch.exp2(torch.randint(-12, 12, (n, 1), generator=g, device=DEV).float())
+    for x in (wide[:, :k], wide[:, 4:k + 4], wide[:, 1:k + 1]):                       # a copy where rows are not 16-byte aligned
+        want = x.double() @ w.double().T
+        # six sums per 32 columns, each rounded once: a walk of 6 k / 32 steps of at most 2^-24 (and the sum of the parts) of the size that
+        # a product of independent values has; a lost lower plane would leave 2^-17 of it
+        size = x.double().norm() * w.double().norm(dim=1) / k ** 0.5
+        err = (ot.split_linear(x, w, splits).double() - want).norm(dim=0) / size
+        assert err.max() <= 2.0 ** -24 * (6 * k / 32) ** 0.5 + 2.0 ** -22
+
+
+@pytest.mark.parametrize("splits", [1, 2])
+def test_split_float32_extremes(splits):
+    from triforce_amd import ops_tile as ot
+    g = torch.Generator(device=DEV).manual_seed(splits)
+    x, w = torch.randn(200, 64, generator=g, device=DEV), torch.randn(272, 64, generator=g, device=DEV).bfloat16().float()
+    x[3, 5], x[4, 6], x[5, 7], x[6, 8], x[6, 9] = float("inf"), -float("inf"), float("nan"), float("inf"), -float("inf")
+    x[130], x[131], x[132], x[133] = 0, x[131] * 1e-30, x[132] * 1e-36, x[133] * 1e36
+    x[134, 1:] *= 1e-38
+    w[7, 3], w[8, 3] = float("inf"), float("nan")
+    want = x.double() @ w.double().T
+    got = ot.split_linear(x, w, splits).double()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+    ok = torch.isfinite(want)
+    bound = 64 * 2.0 ** -24 * (x.double().abs().nan_to_num(0, 0, 0) @ w.double().abs().nan_to_num(0, 0, 0).T) + 64 * 2.0 ** -149
+    assert ((got - want).abs()[ok] <= bound[ok]).all()

@@ -19,7 +19,7 @@ HYBRID_LIB_PATH = os.path.join(LIB_DIR, "libtriforce_hybrid.so")
 SOURCES = ["attn.hip", "retrieval.hip", "elementwise.hip", "sampling.hip", "offload.hip", "gemv.hip", "allreduce.hip", "draft.hip", "draft_persist.hip", "topp_multi.hip", "abi.hip"]
 LIBRARIES = {
     "core": (LIB_PATH, SOURCES, ["common.h", "tree_mask.h", "select_common.h"], ["triforce_hip.h"]),
-    "tile": (TILE_LIB_PATH, ["tile_gemm.hip", "paged.hip"], ["tile_common.h"], ["triforce_tile.h"]),
+    "tile": (TILE_LIB_PATH, ["tile_gemm.hip", "split_gemm.hip", "paged.hip"], ["tile_common.h"], ["triforce_tile.h"]),
     "latent": (LATENT_LIB_PATH, ["latent_attn.hip", "latent_ops.hip"], ["tile_common.h"], ["triforce_tile.h", "triforce_latent.h"]),
     "hybrid": (HYBRID_LIB_PATH, ["hybrid_rec.hip", "hybrid_attn.hip", "hybrid_step.hip", "hybrid_ops.hip"], ["tile_common.h", "hybrid_common.h"],
                ["triforce_tile.h", "triforce_hybrid.h"]),

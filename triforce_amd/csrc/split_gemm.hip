@@ -1,0 +1,260 @@
+// float32 products of many rows (prefill) on the bfloat16 matrix cores: y = x . W^T.
+//
+// A float32 is exactly the sum of three bfloat16 (its 24 bits of mantissa cut into 8 + 8 + 8; cutting, not rounding, so that nothing
+// overflows), and six of the nine products of two such sums carry everything down to 2^-24 of a product: with h, m, l the three parts,
+// hh + hm + mh + mm + hl + lh; what is left out (ml, lm, ll) is below 2^-23 * 2^-8 of it.  Each product of bfloat16 is exact in the
+// matrix core and the sums are fp32, over k in steps of 32 where the fp32 instruction takes 4: the error against 64 bits is that of a
+// product on the fp32 instruction or less (normal values, 4 096 outputs: 700 x 4 096 1.1e-6 -> 4.4e-7, 700 x 15 104 2.1e-6 -> 7.2e-7, 2 048 x
+// 15 104 without parts 2.2e-6 -> 2.1e-6).  Six bf16 instructions take 3/8 of the cycles of the eight fp32 ones that cover the same
+// 16 x 16 x 32.
+//
+// 256 outputs x 128 rows per workgroup, eight waves of 64 x 64: per step of 32 a wave reads 24 KB from LDS for 96 products (1 536 cycles),
+// half of what LDS delivers.  x is cut once by a kernel in front, into planes in MFMA order ([rows/16][k/32][3][64 lanes][8]: a fragment is one
+// contiguous KiB that goes to LDS by DMA); a weight is used by one workgroup per 128 rows and is cut on its way to LDS, beside the products.
+// (Cut at load time
+// into planes, weights cost 6 bytes beside the 4 and gain 3 to 8 %: 22 016 x 4 096 at 700 rows 706 us against 730.  The cut between the
+// products instead of behind them waits for x's DMA before each store to LDS: 22 016 x 4 096 at 2 048 rows 1 830 -> 2 230 us.)
+//
+// Bound by the power of the matrix cores (1.6 to 1.7 GHz under these products, as bf16 GEMMs) and by rounds of tiles.  fp32 GEMM before ->
+// now, x's cut and the sum of parts included: 700 rows, 22 016 x 4 096 940 -> 750 us, 18 784 x 4 096 900 -> 590, 4 096 x 15 104 680 -> 460;
+// 2 048 rows, 22 016 x 4 096 2 600 -> 1 800 (205 TFLOP/s).
+//
+// A result that is not finite (an infinity times a zero lower part would be NaN) or below 2^-50 (whose smallest products may have left
+// fp32's range, and the lower parts of its factors bfloat16's) is computed again in plain fp32.
+#include "tile_common.h"
+
+#define SPLIT_KC 512                   // columns of x that one workgroup cuts
+
+__device__ __forceinline__ void cut_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
+    constexpr uint32_t HIGH = 0x07060302u;                    // the upper halves of both
+    const uint32_t ha = __builtin_bit_cast(uint32_t, a), hb = __builtin_bit_cast(uint32_t, b);
+    h = __builtin_amdgcn_perm(hb, ha, HIGH);
+    a -= __builtin_bit_cast(float, ha & 0xFFFF0000u);
+    b -= __builtin_bit_cast(float, hb & 0xFFFF0000u);
+    const uint32_t ma = __builtin_bit_cast(uint32_t, a), mb = __builtin_bit_cast(uint32_t, b);
+    m = __builtin_amdgcn_perm(mb, ma, HIGH);
+    a -= __builtin_bit_cast(float, ma & 0xFFFF0000u);
+    b -= __builtin_bit_cast(float, mb & 0xFFFF0000u);
+    l = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), HIGH);
+}
+
+// Eight values into the three planes of a fragment.
+__device__ __forceinline__ void cut_store(const f32x4 (&v)[2], bf16* dst) {
+    u32x4 out[3];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        uint32_t h, m, l;
+        cut_pair(v[e >> 1][2 * (e & 1)], v[e >> 1][2 * (e & 1) + 1], h, m, l);
+        out[0][e] = h;
+        out[1][e] = m;
+        out[2][e] = l;
+    }
+#pragma unroll
+    for (int z = 0; z < 3; ++z) *reinterpret_cast<u32x4*>(dst + 512 * z) = out[z];
+}
+
+// One workgroup: 16 rows, SPLIT_KC columns.
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, int64_t ld, int rows, int k, bf16* __restrict__ planes) {
+    const int panel = blockIdx.x, tid = threadIdx.x, lane = tid & 63, chunks = k >> 5, row = 16 * panel + (lane & 15);
+    const int c_end = min(chunks, (int)(blockIdx.y + 1) * (SPLIT_KC / 32));
+    for (int c = blockIdx.y * (SPLIT_KC / 32) + (tid >> 6); c < c_end; c += 4) {
+        f32x4 v[2] = {};
+        if (row < rows) {
+            const f32x4* src = reinterpret_cast<const f32x4*>(x + (int64_t)row * ld + 32 * c + 8 * (lane >> 4));
+            v[0] = src[0];
+            v[1] = src[1];
+        }
+        cut_store(v, planes + ((int64_t)panel * chunks + c) * 1536 + lane * 8);
+    }
+}
+
+struct SplitGemm {
+    const float* w;
+    const bf16* xp;
+    const float* x;
+    float* out;
+    float* ws;
+    int64_t ld_x, ld_out;
+    int rows, n, k, splits;
+};
+
+__device__ __forceinline__ void mend(const SplitGemm& a, int row, int n, f32x4& v) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float s = __builtin_fabsf(v[e]);
+        if (s == 0.f || (s >= 0x1p-50f && s < __builtin_inff())) continue;
+        const float* x = a.x + (int64_t)row * a.ld_x;
+        const float* w = a.w + (int64_t)(n + e) * a.k;
+        float p = 0.f;
+        for (int c = 0; c < a.k && p == p; ++c) p = fmaf(x[c], w[c], p);
+        v[e] = p;
+    }
+}
+
+// MT 16-row tiles of x per wave; waves: 4 x 64 outputs, 2 x 16 MT rows.
+template <int MT>
+__global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
+    constexpr int NP = 16, XP = 2 * MT, PER = 3 * XP / 8, BUF = 3 * (NP + XP) * 512;
+    static_assert(3 * XP % 8 == 0, "the waves bring in the same number of fragments");
+    extern __shared__ __align__(16) bf16 tiles[];             // [2][NP + XP][3][512]
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15;
+    const int wn = wave & 3, wm = wave >> 2, chunks = a.k >> 5;
+    // workgroups go round-robin over the 8 XCDs: each takes an eighth of the tiles, the row tiles of one column tile one after the other, which
+    // share its weights in L2
+    const int mts = (a.rows + 32 * MT - 1) / (32 * MT), tiles_all = (a.n + 255) / 256 * mts, xcd = blockIdx.x & 7;
+    const int id = (int)((int64_t)tiles_all * xcd >> 3) + (blockIdx.x >> 3);
+    if (id >= (int)((int64_t)tiles_all * (xcd + 1) >> 3)) return;
+    const int nt = id / mts, mt0 = id % mts;
+    const int per = (chunks + a.splits - 1) / a.splits, c_beg = blockIdx.y * per, c_end = min(chunks, c_beg + per);
+    const int xpan = (a.rows + 15) >> 4;
+    const bf16* src[PER];                                     // this wave's fragments of x: scalar pointers to their first chunk
+#pragma unroll
+    for (int f = 0; f < PER; ++f) {
+        const int p = (wave * PER + f) / 3, z = (wave * PER + f) % 3;
+        src[f] = a.xp + (int64_t)min(mt0 * XP + p, xpan - 1) * chunks * 1536 + z * 512;
+    }
+    const float* wsrc[2];                                     // this lane's eight weights of two panels
+#pragma unroll
+    for (int f = 0; f < 2; ++f) wsrc[f] = a.w + (int64_t)min(nt * 256 + 16 * (wave + 8 * f) + i, a.n - 1) * a.k + 8 * g;
+    f32x4 staged[2][2];
+    auto fetch_x = [&](int c, int buf) {
+#pragma unroll
+        for (int f = 0; f < PER; ++f)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[f] + (int64_t)c * 1536 + lane * 8),
+                                             (__attribute__((address_space(3))) void*)(tiles + buf * BUF + (3 * NP + wave * PER + f) * 512), 16, 0, 0);
+    };
+    auto fetch_w = [&](int c) {
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) staged[f][h] = *reinterpret_cast<const f32x4*>(wsrc[f] + 32 * c + 4 * h);
+    };
+    auto put_w = [&](int buf) {
+#pragma unroll
+        for (int f = 0; f < 2; ++f) cut_store(staged[f], tiles + buf * BUF + (wave + 8 * f) * 1536 + lane * 8);
+    };
+    const bool live = mt0 * XP + wm * MT < xpan;              // a wave without rows leaves the matrix core to its neighbour
+    f32x4 acc[4][MT];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (c_beg < c_end) {
+        fetch_x(c_beg, 0);
+        fetch_w(c_beg);
+        put_w(0);
+        fetch_w(min(c_beg + 1, c_end - 1));
+        __builtin_amdgcn_s_waitcnt(0x0F74);                   // vmcnt(4): all but the weights just asked for
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+    }
+    for (int c = c_beg; c < c_end; ++c) {
+        const int buf = (c - c_beg) & 1;
+        fetch_x(min(c + 1, c_end - 1), buf ^ 1);              // in flight under this step's products
+        if (live) {
+            const bf16* wt = tiles + buf * BUF + wn * 4 * 1536 + lane * 8;
+            const bf16* xt = tiles + buf * BUF + (NP + wm * MT) * 1536 + lane * 8;
+            bf16x8 w[4][3];
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int z = 0; z < 3; ++z) w[t][z] = load_frag(wt + (3 * t + z) * 512);
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                bf16x8 x[3];
+#pragma unroll
+                for (int z = 0; z < 3; ++z) x[z] = load_frag(xt + (3 * m + z) * 512);
+                constexpr int WZ[6] = {2, 0, 1, 1, 0, 0}, XZ[6] = {0, 2, 1, 0, 1, 0};          // small products first
+#pragma unroll
+                for (int q = 0; q < 6; ++q)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][WZ[q]], x[XZ[q]], acc[t][m], 0, 0, 0);
+            }
+        }
+        put_w(buf ^ 1);
+        fetch_w(min(c + 2, c_end - 1));
+        __builtin_amdgcn_s_waitcnt(0x0F74);                   // this wave's part of the next step is in LDS before the barrier
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+    }
+    float* y = a.splits > 1 ? a.ws + (int64_t)blockIdx.y * a.rows * a.n : a.out;
+    const int64_t ld = a.splits > 1 ? a.n : a.ld_out;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int row = mt0 * 32 * MT + 16 * (wm * MT + m) + i;
+        if (row >= a.rows) continue;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int n = nt * 256 + 64 * wn + 16 * t + 4 * g;
+            if (n >= a.n) continue;
+            if (a.splits == 1) mend(a, row, n, acc[t][m]);
+            *reinterpret_cast<f32x4*>(y + (int64_t)row * ld + n) = acc[t][m];
+        }
+    }
+}
+
+// The parts of a split k, summed in order.
+__global__ __launch_bounds__(256) void split_sum_kernel(const SplitGemm a) {
+    const int row = blockIdx.x, n = 4 * (blockIdx.y * 256 + threadIdx.x);
+    if (n >= a.n) return;
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int z = 0; z < a.splits; ++z) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(a.ws + ((int64_t)z * a.rows + row) * a.n + n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] += v[e];
+    }
+    mend(a, row, n, s);
+    *reinterpret_cast<f32x4*>(a.out + (int64_t)row * a.ld_out + n) = s;
+}
+
+template <int MT>
+static int launch_split_gemm(const SplitGemm& a, hipStream_t st) {
+    constexpr int LDS = 2 * 3 * (16 + 2 * MT) * 1024;
+    const hipError_t e = hipFuncSetAttribute((const void*)split_gemm_kernel<MT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if (e != hipSuccess) return (int)e;
+    const int tiles = (a.n + 255) / 256 * ((a.rows + 32 * MT - 1) / (32 * MT));
+    hipLaunchKernelGGL(split_gemm_kernel<MT>, dim3((tiles + 7) / 8 * 8, a.splits), dim3(512), LDS, st, a);
+    TFL_LAUNCH_CHECK();
+    if (a.splits > 1) {
+        hipLaunchKernelGGL(split_sum_kernel, dim3(a.rows, (a.n + 1023) / 1024), dim3(256), 0, st, a);
+        TFL_LAUNCH_CHECK();
+    }
+    return TF_OK;
+}
+
+static int64_t split_planes(int rows, int k) { return (int64_t)((rows + 15) / 16) * (k / 32) * 1536 * 2 / 4; }      // in floats
+
+// Parts of k: rounds of 256 workgroups, each with the fill of its pipe (4 steps of 32), against what the parts cost on their way through memory
+// (a written and read 128 x 256 part as much as 8 steps).  256 rows, 12 320 x 4 096: 267 us without parts, 159 with two, 171 with four;
+// 700 rows, 4 096 x 8 192: 514, 296 with two, 262 with five, 265 with eight.
+static int pick_parts(int rows, int n, int k) {
+    const int64_t tiles = (int64_t)((n + 255) / 256) * ((rows + 127) / 128);
+    int best = 1;
+    double least = 0;
+    for (int s = 1; s <= 8 && (s == 1 || s * 512 <= k); ++s) {
+        const double t = (double)((tiles * s + 255) / 256) * (1.0 / s + 4.0 / (k / 32)) + (s > 1 ? 8.0 * (double)s * tiles / 256 / (k / 32) : 0);
+        if (s == 1 || t < least) { best = s; least = t; }
+    }
+    return best;
+}
+
+extern "C" int64_t tfl_split_gemm_ws_floats(int rows, int n, int k, int splits) {
+    if (rows < 1 || rows > (1 << 24) || n < 16 || k < 32 || splits < 0 || splits > 64) return 0;
+    if (splits == 0) splits = pick_parts(rows, n, k);
+    return split_planes(rows, k) + (splits > 1 ? (int64_t)splits * rows * n : 0);
+}
+
+extern "C" int tfl_split_gemm(const float* w, const float* x, int64_t ld_x, float* out, int64_t ld_out, float* ws, int64_t ws_floats, int rows, int n,
+                              int k, int splits, void* stream) {
+    if (!w || !x || !out || !ws || rows < 1 || rows > (1 << 24) || n < 16 || (n & 15) || k < 32 || (k & 31) || ld_x < k || (ld_x & 3) || ld_out < n
+        || (ld_out & 3) || splits < 0 || splits > 64) return TF_EINVAL;
+    if (((uintptr_t)w | (uintptr_t)x | (uintptr_t)out | (uintptr_t)ws) & 15) return TF_EINVAL;
+    if (splits == 0) splits = pick_parts(rows, n, k);
+    if (ws_floats < tfl_split_gemm_ws_floats(rows, n, k, splits)) return TF_ENOSPC;
+    hipLaunchKernelGGL(split_rows_kernel, dim3((rows + 15) / 16, (k + SPLIT_KC - 1) / SPLIT_KC), dim3(256), 0, (hipStream_t)stream, x, ld_x, rows, k,
+                       (bf16*)ws);
+    TFL_LAUNCH_CHECK();
+    const SplitGemm a = {w, (const bf16*)ws, x, out, ws + split_planes(rows, k), ld_x, ld_out, rows, n, k, splits};
+    return launch_split_gemm<4>(a, (hipStream_t)stream);
+}

@@ -160,6 +160,8 @@ class TflGemm(_c.Structure):
 TILE_SIGNATURES = {
     "tfl_tile_abi_version": (_i32, []),
     "tfl_gemm": (_i32, [_c.POINTER(TflGemm), _i32, _i32, _vp]),
+    "tfl_split_gemm_ws_floats": (_i64, [_i32, _i32, _i32, _i32]),
+    "tfl_split_gemm": (_i32, [_vp, _vp, _i64, _vp, _i64, _vp, _i64, _i32, _i32, _i32, _i32, _vp]),
     "tfl_set_pages": (_i32, [_vp, _i32, _i32, _i32, _c.POINTER(_c.c_int32), _i32, _vp]),
     "tfl_decode_prep": (_i32, [_vp, _vp, _i32, _i32, _vp, _vp, _vp, _i32, _vp]),
 }

@@ -90,7 +90,7 @@ class LatentLayer:
         if ck is None:
             ck = ol.gather_rows(cache_rows, batch.key_rows)              # earlier portions' rows and the ones just stored
         q = self.w_uq.matmul(cq)
-        kv = torch.nn.functional.linear(ck[:, :g.C], self.w_ukv)
+        kv = ol.linear_rows(ck[:, :g.C], self.w_ukv)
         ol.attn_prefill(q, kv, ck, batch.seq, batch.max_new, batch.pos, rope, y[:, g.gate_off:], act, g, self.scale)
         d = self.w_out.matmul(act)
         xt = ol.residual(d, x, want_copy=bool(self.side_dim))

@@ -7,7 +7,7 @@ tensors.  Call these as ``ops_latent.<name>(...)``.
 import torch
 
 from . import hip
-from .ops_tile import (_CODE, PAGE, TileWeight, _f32, _gemm, _i32, _lay, _need, _p, _stream, _tail, act_rows, decode_prep, empty_act,  # noqa: F401
+from .ops_tile import (_CODE, PAGE, TileWeight, _f32, _gemm, _i32, _lay, _need, _p, _stream, _tail, act_rows, decode_prep, empty_act, linear_rows,  # noqa: F401
                        linear_f32, pack_tiles, pad32)
 
 def input_projection(h, wt, n_raw, q_norm, act, act_off):
