@@ -274,3 +274,79 @@ def test_split_float32_extremes(splits):
     ok = torch.isfinite(want)
     bound = 64 * 2.0 ** -24 * (x.double().abs().nan_to_num(0, 0, 0) @ w.double().abs().nan_to_num(0, 0, 0).T) + 64 * 2.0 ** -149
     assert ((got - want).abs()[ok] <= bound[ok]).all()
+
+
+def _flash_want(q, k, v, lo, hi, scale):
+    """float64 attention of q [n, d] with keys lo .. hi of every row: (result, the same sums with |v|)."""
+    s = (q.double() @ k.double().T) * scale
+    at = torch.arange(k.shape[0], device=DEV)
+    s = s.masked_fill((at < lo[:, None]) | (at > hi[:, None]), -float("inf"))
+    p = torch.softmax(s, 1)
+    return p @ v.double(), p @ v.double().abs()
+
+
+# around a wave's 16 and 32 rows, a workgroup's 128, a tile's 64 keys; chunks that begin inside a tile and inside a workgroup; strange
+# values behind the last key
+@pytest.mark.parametrize("news,pasts,chunk", [([1], [0], 8192), ([127, 33], [1, 64], 8192), ([129, 16], [63, 500], 8192), ([300], [190], 100),
+                                              ([257, 128, 2], [0, 127, 1000], 640), ([65], [0], 1)])
+@pytest.mark.parametrize("H,G", [(8, 2), (3, 3)])
+def test_chunked_prefill_tiles(news, pasts, chunk, H, G):
+    from types import SimpleNamespace as NS
+    from triforce_amd import ops_hybrid as oh
+    g = torch.Generator(device=DEV).manual_seed(sum(news) + H)
+    geom = NS(q_off=0, gate_off=H * 128, H=H, G=G, D=128, V=128, row=G * 256, chunk=chunk, scale=0.11)
+    y, out = _bf(g, sum(news), 2 * H * 128), torch.full((sum(news), H * 128), 9.0, dtype=torch.bfloat16, device=DEV)
+    pages = [(n + p + 63) // 64 for n, p in zip(news, pasts)]
+    cache = _bf(g, (sum(pages) + 1) * 64, G * 256)
+    own = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(1)).to(torch.int32)
+    table, seq, at, tok = torch.zeros(len(news), max(pages), dtype=torch.int32), [], 0, 0
+    for b, (n, p) in enumerate(zip(news, pasts)):
+        table[b, :pages[b]] = own[at:at + pages[b]]
+        cache.view(-1, 64, G * 256)[int(own[at + pages[b] - 1]), (n + p - 1) % 64 + 1:] = float("nan")
+        seq.append([tok, n, p, 0])
+        at, tok = at + pages[b], tok + n
+    batch = NS(table=table.to(DEV), seq=torch.tensor(seq, dtype=torch.int32, device=DEV), max_new=max(news))
+    oh.attn_prefill(y, geom, cache, batch, out, 0.7)
+    for b, (t0, n, p, _) in enumerate(seq):
+        rows = cache.view(-1, 64, G * 256)[table[b, :pages[b]].long().to(DEV)].reshape(-1, G * 256)[:n + p]
+        hi = p + torch.arange(n, device=DEV)
+        for h in range(H):
+            kv = h // (H // G)
+            want, size = _flash_want(y[t0:t0 + n, 128 * h:128 * h + 128], rows[:, 128 * kv:128 * kv + 128], rows[:, 128 * (G + kv):128 * (G + kv) + 128],
+                                     hi // chunk * chunk, hi, 0.11)
+            s = 0.7 * torch.sigmoid(y[t0:t0 + n, 128 * (H + h):128 * (H + h) + 128].double())
+            # every weight rounded to bfloat16 (2^-9 of it), the result too
+            assert ((out[t0:t0 + n, 128 * h:128 * h + 128].double() - s * want).abs() <= 2.0 ** -8 * s * (want.abs() + size) + 1e-6).all()
+
+
+# as above; the last one: long enough, and a whole round, for workgroups of 256 rows
+@pytest.mark.parametrize("news,pasts,H", [([1], [0], 8), ([127, 33], [1, 64], 8), ([129, 16], [63, 500], 3), ([257, 128, 2], [0, 127, 1000], 8), ([300, 40], [16400, 16400], 52)])
+@pytest.mark.parametrize("half", [32, 5, 0])
+def test_latent_prefill_tiles(news, pasts, H, half):
+    from types import SimpleNamespace as NS
+    from triforce_amd import ops_latent as ol
+    g = torch.Generator(device=DEV).manual_seed(sum(news) + H)
+    tq, tk = sum(news), sum(news) + sum(pasts)
+    geom = NS(H=H, N=128, R=64, V=128, C=64)
+    q, kv, ck, gate = _bf(g, tq, H * 192), _bf(g, tk, H * 256), _bf(g, tk, 128), _bf(g, tq, H * 128)
+    out = torch.full((tq, H * 128), 9.0, dtype=torch.bfloat16, device=DEV)
+    angle = torch.rand(20000, max(half, 1), generator=g, device=DEV)
+    rope = NS(cos=angle.cos().contiguous(), sin=angle.sin().contiguous(), half=half, max_pos=20000)
+    seq, pos, a, b = [], [], 0, 0
+    for n, p in zip(news, pasts):
+        seq.append([a, n, b, n + p])
+        pos += range(p, p + n)
+        a, b = a + n, b + n + p
+    pos = torch.tensor(pos, dtype=torch.int32, device=DEV)
+    ol.attn_prefill(q, kv, ck, torch.tensor(seq, dtype=torch.int32, device=DEV), max(news), pos, rope, gate, out, geom, 0.08)
+    turned = q.view(tq, H, 192).clone()
+    even, odd = q.view(tq, H, 192)[..., 128:128 + 2 * half:2].float(), q.view(tq, H, 192)[..., 129:129 + 2 * half:2].float()
+    cos, sin = rope.cos[pos.long(), None, :half], rope.sin[pos.long(), None, :half]
+    turned[..., 128:128 + 2 * half:2], turned[..., 129:129 + 2 * half:2] = (even * cos - odd * sin).bfloat16(), (odd * cos + even * sin).bfloat16()
+    for t0, n, k0, nk in seq:
+        hi = nk - n + torch.arange(n, device=DEV)
+        for h in sorted({0, H // 2, H - 1}):
+            k = torch.cat([kv[k0:k0 + nk, 128 * h:128 * h + 128], ck[k0:k0 + nk, 64:]], 1)
+            want, size = _flash_want(turned[t0:t0 + n, h], k, kv[k0:k0 + nk, 128 * (H + h):128 * (H + h) + 128], hi * 0, hi, 0.08)
+            s = torch.sigmoid(gate[t0:t0 + n, 128 * h:128 * h + 128].double())
+            assert ((out[t0:t0 + n, 128 * h:128 * h + 128].double() - s * want).abs() <= 2.0 ** -8 * s * (want.abs() + size) + 1e-6).all()

@@ -20,8 +20,8 @@ SOURCES = ["attn.hip", "retrieval.hip", "elementwise.hip", "sampling.hip", "offl
 LIBRARIES = {
     "core": (LIB_PATH, SOURCES, ["common.h", "tree_mask.h", "select_common.h"], ["triforce_hip.h"]),
     "tile": (TILE_LIB_PATH, ["tile_gemm.hip", "split_gemm.hip", "paged.hip"], ["tile_common.h"], ["triforce_tile.h"]),
-    "latent": (LATENT_LIB_PATH, ["latent_attn.hip", "latent_ops.hip"], ["tile_common.h"], ["triforce_tile.h", "triforce_latent.h"]),
-    "hybrid": (HYBRID_LIB_PATH, ["hybrid_rec.hip", "hybrid_attn.hip", "hybrid_step.hip", "hybrid_ops.hip"], ["tile_common.h", "hybrid_common.h"],
+    "latent": (LATENT_LIB_PATH, ["latent_attn.hip", "latent_ops.hip"], ["tile_common.h", "flash_tile.h"], ["triforce_tile.h", "triforce_latent.h"]),
+    "hybrid": (HYBRID_LIB_PATH, ["hybrid_rec.hip", "hybrid_attn.hip", "hybrid_step.hip", "hybrid_ops.hip"], ["tile_common.h", "flash_tile.h", "hybrid_common.h"],
                ["triforce_tile.h", "triforce_hybrid.h"]),
 }
 # -amdgpu-kernarg-preload-count: the leading pointer / scalar kernel arguments (up to 14 dwords) arrive in SGPRs with the

@@ -6,10 +6,10 @@
 // wave w takes keys 16w .. 16w+15.  The weights go to LDS as [head][key] and every wave then accumulates its share of the
 // latent columns, O^T = C^T P^T, with the transposed operand read straight from the key-major page (ds_read_b64_tr_b16).
 //
-// Prefill (attn_prefill_kernel): keys and values up-projected once per chunk, flash attention with 16 * QT query rows per wave,
-// the waves of a workgroup sharing the key / value tile.  Also transposed: the S^T result registers of two 16-key tiles ARE the P operand of
+// Prefill (attn_prefill_kernel): keys and values up-projected once per chunk, flash attention with 16 query rows per wave (2 x 16 in
+// attn_prefill_sized_kernel), the waves of a workgroup sharing the key / value tile.  Also transposed: the S^T result registers of two 16-key tiles ARE the P operand of
 // one PV product (the value operand is read with the matching key order), so the weights never leave the registers.
-#include "tile_common.h"
+#include "flash_tile.h"
 
 #define NEG_INF (-__builtin_inff())
 #define LOG2E 1.4426950408889634f
@@ -564,39 +564,21 @@ extern "C" int tfl_attn_decode(const void* q, const void* cache, int n_pages, co
 }
 
 // --------------------------------------------------------------------------------------------------------------- prefill
-// A 64-row section of PR 16-byte pieces per row, spread over NT threads, to / from registers pre[AT ..].
-template <int NT, int PR, int AT, typename T, int N>
-__device__ __forceinline__ void fetch_section(u32x4 (&pre)[N], const T* base, int64_t ld, int left, int tid) {
-    const int r0 = tid / PR, c = tid % PR;
-#pragma unroll
-    for (int j = 0; j < 64 * PR / NT; ++j)
-        if (AT + j < N) pre[AT + j] = *reinterpret_cast<const u32x4*>(base + (int64_t)min(r0 + j * (NT / PR), left) * ld + 8 * c);
-}
-template <int NT, int PR, int AT, typename T, int N>
-__device__ __forceinline__ void put_section(const u32x4 (&pre)[N], T* base, int ld, int tid) {
-    const int r0 = tid / PR, c = tid % PR;
-#pragma unroll
-    for (int j = 0; j < 64 * PR / NT; ++j)
-        if (AT + j < N) *reinterpret_cast<u32x4*>(base + (r0 + j * (NT / PR)) * ld + 8 * c) = pre[AT + j];
-}
-
-// NWV waves, KT keys per tile, QT 16-row query tiles per wave, up to DK 32-wide chunks of query-key size (NC unrotated ones first) and DV
-// 16-wide tiles of value size.  EXACT: the sizes are exactly NCX, DK, DV (no bounds in the inner loops, register look-ahead).
-template <typename T, int NWV, int KT, int QT, int DK, int DV, int NCX>
-__global__ __launch_bounds__(64 * NWV, NWV / 4) void attn_prefill_kernel(const T* __restrict__ q, const T* __restrict__ kv, const T* __restrict__ ck,
+// Four waves of 16 query rows, KT keys per tile, up to DK 32-wide chunks of query-key size and DV 16-wide tiles of value size.
+template <typename T, int KT, int DK, int DV>
+__global__ __launch_bounds__(256, 1) void attn_prefill_kernel(const T* __restrict__ q, const T* __restrict__ kv, const T* __restrict__ ck,
                                                            const int32_t* __restrict__ seq, const int32_t* __restrict__ pos,
                                                            const float* __restrict__ cosb, const float* __restrict__ sinb,
                                                            int half, int max_pos, const T* __restrict__ gate, int64_t ld_gate,
                                                            T* __restrict__ out, int64_t ld_out, int tq, int tk, int H, int N, int R,
                                                            int V, int C, float scale) {
     typedef typename El<T>::Frag Frag;
-    constexpr bool EXACT = NCX > 0;
-    constexpr int EPV = 16 / sizeof(T), PADE = EPV, PADV = 2 * EPV, QB = 16 * NWV * QT, NT = 64 * NWV;
+    constexpr int EPV = 16 / sizeof(T), PADE = EPV, PADV = 2 * EPV, QB = 64, NT = 256;
     extern __shared__ __align__(16) char smem[];
-    const int nc = EXACT ? NCX : N >> 5, dk = EXACT ? DK : (N + R) >> 5, dv = EXACT ? DV : V >> 4;
+    const int nc = N >> 5, dk = (N + R) >> 5, dv = V >> 4;
     const int D = 32 * dk, ldk = D + PADE, ldv = 16 * dv + PADV;
-    T* Ks = (T*)smem;                                         // [1 or 2][KT][ldk], then the values [KT][ldv]
-    T* Vs = Ks + (EXACT ? 2 : 1) * KT * ldk;
+    T* Ks = (T*)smem;                                         // [KT][ldk], then the values [KT][ldv]
+    T* Vs = Ks + KT * ldk;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, i = lane & 15;
     // workgroups go round-robin over the 8 XCDs: all query blocks of a head sit on one of them and share its L2, longest first
     const int nqb = gridDim.x / H, id = blockIdx.x;
@@ -609,112 +591,70 @@ __global__ __launch_bounds__(64 * NWV, NWV / 4) void attn_prefill_kernel(const T
     const int past = nk - nq;
     const int64_t ld_kv = (int64_t)H * (N + V), ld_ck = C + R;
 
-    Frag qf[QT][DK];
-    int qpos[QT];                                             // key index of the lane's own query token
+    Frag qf[DK];
+    const int j = qb + 16 * wave + i, qpos = past + j;        // the lane's own query token: its row, its key index
+    const int64_t tok = q_at + min(j, nq - 1);
+    const T* src = q + (tok * H + h) * (int64_t)(N + R) + 8 * g;
+    int p = pos[tok];
+    p = p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-        const int j = qb + 16 * (wave * QT + t) + i;
-        qpos[t] = past + j;
-        const int64_t tok = q_at + min(j, nq - 1);
-        const T* src = q + (tok * H + h) * (int64_t)(N + R) + 8 * g;
-        int p = pos[tok];
-        p = p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
+    for (int c = 0; c < DK; ++c) {
+        if (c >= dk) { qf[c] = Frag{}; continue; }
+        Frag f = load_frag(src + 32 * c);
+        if (c >= nc) {
+            const int pr = (c - nc) * 16 + 4 * g;
 #pragma unroll
-        for (int c = 0; c < DK; ++c) {
-            if (!EXACT && c >= dk) { qf[t][c] = Frag{}; continue; }
-            Frag f = load_frag(src + 32 * c);
-            if (c >= nc) {
-                const int pr = (c - nc) * 16 + 4 * g;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (pr + e < half) {
-                        const float cs = cosb[(int64_t)p * half + pr + e], sn = sinb[(int64_t)p * half + pr + e];
-                        const float u = (float)f[2 * e], v = (float)f[2 * e + 1];
-                        f[2 * e] = (T)(u * cs - v * sn);
-                        f[2 * e + 1] = (T)(v * cs + u * sn);
-                    }
-            }
-            qf[t][c] = f;
+            for (int e = 0; e < 4; ++e)
+                if (pr + e < half) {
+                    const float cs = cosb[(int64_t)p * half + pr + e], sn = sinb[(int64_t)p * half + pr + e];
+                    const float u = (float)f[2 * e], v = (float)f[2 * e + 1];
+                    f[2 * e] = (T)(u * cs - v * sn);
+                    f[2 * e + 1] = (T)(v * cs + u * sn);
+                }
         }
+        qf[c] = f;
     }
-    f32x4 o[QT][DV];
-    float m_run[QT], l_run[QT];
+    f32x4 o[DV];
+    float m_run = NEG_INF, l_run = 0.f;
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-        m_run[t] = NEG_INF;
-        l_run[t] = 0.f;
-#pragma unroll
-        for (int d = 0; d < DV; ++d) o[t][d] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int d = 0; d < DV; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int last_q = min(qb + QB, nq) - 1;                  // last query row of the workgroup
     const int ntiles = (past + last_q) / KT + 1;
-    const int first_qpos = past + qb + 16 * wave * QT;        // the wave's first row: tiles that end before it need no mask
-    [[maybe_unused]] const int kn = N / EPV, kr = R / EPV, vn = V / EPV, ppr = kn + kr + vn;   // 16-byte pieces per key
-    // EXACT: two tiles in LDS and one in registers.  A tile is NJ pieces per thread; piece j of a section is row
-    // (tid / pieces per row) + j * step of it
-    constexpr int RCX = EXACT ? DK - NCX : 1, NKX = EXACT ? NCX : 1, VCX = EXACT ? DV / 2 : 1;
-    constexpr int NJ = EXACT ? 4 * (NKX + RCX + VCX) / NWV : 1;
-    static_assert(!EXACT || (KT == 64 && (4 * NKX) % NWV == 0 && (4 * RCX) % NWV == 0 && (4 * VCX) % NWV == 0), "piece split");
-    u32x4 pre[NJ];
-    auto fetch = [&](int t) {
-        const T* kv_t = kv + (int64_t)(k_at + t * KT) * ld_kv;
-        const T* ck_t = ck + (int64_t)(k_at + t * KT) * ld_ck + C;
-        const int left = nk - t * KT - 1;                     // rows past the last key repeat it (masked)
-        fetch_section<NT, 4 * NKX, 0>(pre, kv_t + (int64_t)h * N, ld_kv, left, tid);
-        fetch_section<NT, 4 * RCX, 4 * NKX / NWV>(pre, ck_t, ld_ck, left, tid);
-        fetch_section<NT, 4 * VCX, 4 * (NKX + RCX) / NWV>(pre, kv_t + (int64_t)H * N + (int64_t)h * V, ld_kv, left, tid);
-    };
-    auto put = [&](int t) {
-        T* kt = Ks + (t & 1) * KT * ldk;
-        put_section<NT, 4 * NKX, 0>(pre, kt, ldk, tid);
-        put_section<NT, 4 * RCX, 4 * NKX / NWV>(pre, kt + 32 * NKX, ldk, tid);
-        put_section<NT, 4 * VCX, 4 * (NKX + RCX) / NWV>(pre, Vs + (t & 1) * KT * ldv, ldv, tid);
-    };
-    if constexpr (EXACT) {
-        fetch(0);
-        put(0);
-        if (ntiles > 1) fetch(1);
-        __syncthreads();
-    }
+    const int first_qpos = past + qb + 16 * wave;             // the wave's first row: tiles that end before it need no mask
+    const int kn = N / EPV, kr = R / EPV, vn = V / EPV, ppr = kn + kr + vn;   // 16-byte pieces per key
     for (int t = 0; t < ntiles; ++t) {
         const int k0 = t * KT;
-        const T* Kt = EXACT ? Ks + (t & 1) * KT * ldk : Ks;
-        const T* Vt = EXACT ? Vs + (t & 1) * KT * ldv : Vs;
-        if constexpr (!EXACT) {
-            for (int p = tid; p < KT * ppr; p += NT) {
-                const int key = p / ppr;
-                int c = p - key * ppr;
-                const int64_t kk = k_at + min(k0 + key, nk - 1);
-                const T* src;
-                T* dst;
-                if (c < kn) {
-                    src = kv + kk * ld_kv + (int64_t)h * N + EPV * c;
-                    dst = Ks + key * ldk + EPV * c;
-                } else if (c < kn + kr) {
-                    c -= kn;
-                    src = ck + kk * ld_ck + C + EPV * c;
-                    dst = Ks + key * ldk + N + EPV * c;
-                } else {
-                    c -= kn + kr;
-                    src = kv + kk * ld_kv + (int64_t)H * N + (int64_t)h * V + EPV * c;
-                    dst = Vs + key * ldv + EPV * c;
-                }
-                *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(src);
+        for (int p = tid; p < KT * ppr; p += NT) {
+            const int key = p / ppr;
+            int c = p - key * ppr;
+            const int64_t kk = k_at + min(k0 + key, nk - 1);
+            const T* src;
+            T* dst;
+            if (c < kn) {
+                src = kv + kk * ld_kv + (int64_t)h * N + EPV * c;
+                dst = Ks + key * ldk + EPV * c;
+            } else if (c < kn + kr) {
+                c -= kn;
+                src = ck + kk * ld_ck + C + EPV * c;
+                dst = Ks + key * ldk + N + EPV * c;
+            } else {
+                c -= kn + kr;
+                src = kv + kk * ld_kv + (int64_t)H * N + (int64_t)h * V + EPV * c;
+                dst = Vs + key * ldv + EPV * c;
             }
-            __syncthreads();
+            *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(src);
         }
-        f32x4 s[KT / 16][QT];
+        __syncthreads();
+        f32x4 s[KT / 16];
 #pragma unroll
         for (int kt = 0; kt < KT / 16; ++kt) {
-#pragma unroll
-            for (int u = 0; u < QT; ++u) s[kt][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-            const T* kp = Kt + (16 * kt + i) * ldk + 8 * g;
+            s[kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const T* kp = Ks + (16 * kt + i) * ldk + 8 * g;
 #pragma unroll
             for (int c = 0; c < DK; ++c) {
-                if (EXACT || c < dk) {
+                if (c < dk) {
                     const Frag a = load_frag(kp + 32 * c);
-#pragma unroll
-                    for (int u = 0; u < QT; ++u) s[kt][u] = El<T>::mma(a, qf[u][c], s[kt][u]);
+                    s[kt] = El<T>::mma(a, qf[c], s[kt]);
                 }
             }
         }
@@ -722,73 +662,143 @@ __global__ __launch_bounds__(64 * NWV, NWV / 4) void attn_prefill_kernel(const T
 #pragma unroll
             for (int kt = 0; kt < KT / 16; ++kt)
 #pragma unroll
-                for (int u = 0; u < QT; ++u)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (k0 + 16 * kt + 4 * g + r > qpos[u]) s[kt][u][r] = NEG_INF;
+                for (int r = 0; r < 4; ++r)
+                    if (k0 + 16 * kt + 4 * g + r > qpos) s[kt][r] = NEG_INF;
         }
-        Frag pf[QT][KT / 32];
+        Frag pf[KT / 32];
+        float mx = NEG_INF;
 #pragma unroll
-        for (int u = 0; u < QT; ++u) {
-            float mx = NEG_INF;
+        for (int kt = 0; kt < KT / 16; ++kt)
 #pragma unroll
-            for (int kt = 0; kt < KT / 16; ++kt)
+            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = fmaxf(m_run, mx * scale);                        // (scale > 0; key 0 is visible to every row: finite from tile 0 on)
+        const float alpha = __builtin_amdgcn_exp2f((m_run - mx) * LOG2E), sc = scale * LOG2E, mb = mx * LOG2E;
+        m_run = mx;
+        float sum = 0.f;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][u][r]);
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            mx = fmaxf(m_run[u], mx * scale);                 // (scale > 0; key 0 is visible to every row: finite from tile 0 on)
-            const float alpha = __builtin_amdgcn_exp2f((m_run[u] - mx) * LOG2E), sc = scale * LOG2E, mb = mx * LOG2E;
-            m_run[u] = mx;
-            float sum = 0.f;
+        for (int kt = 0; kt < KT / 16; ++kt)
 #pragma unroll
-            for (int kt = 0; kt < KT / 16; ++kt)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float p = __builtin_amdgcn_exp2f(fmaf(s[kt][u][r], sc, -mb));
-                    sum += p;
-                    pf[u][kt >> 1][(kt & 1) * 4 + r] = (T)p;
-                }
-            l_run[u] = l_run[u] * alpha + sum;
-            if (!__all(alpha == 1.0f)) {                      // (most tiles leave every maximum where it was)
-#pragma unroll
-                for (int d = 0; d < DV; ++d)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) o[u][d][r] *= alpha;
+            for (int r = 0; r < 4; ++r) {
+                const float p = __builtin_amdgcn_exp2f(fmaf(s[kt][r], sc, -mb));
+                sum += p;
+                pf[kt >> 1][(kt & 1) * 4 + r] = (T)p;
             }
-        }
-        if constexpr (EXACT) {
-            if (t + 1 < ntiles) put(t + 1);
-            if (t + 2 < ntiles) fetch(t + 2);
+        l_run = l_run * alpha + sum;
+        if (!__all(alpha == 1.0f)) {                          // (most tiles leave every maximum where it was)
+#pragma unroll
+            for (int d = 0; d < DV; ++d)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[d][r] *= alpha;
         }
 #pragma unroll
         for (int d = 0; d < DV; ++d) {
-            if (EXACT || d < dv) {
+            if (d < dv) {
 #pragma unroll
                 for (int c = 0; c < KT / 32; ++c) {
-                    const Frag a = load_frag_t(Vt, ldv, 32 * c + 4 * g, 32 * c + 16 + 4 * g, 16 * d, i);
-#pragma unroll
-                    for (int u = 0; u < QT; ++u) o[u][d] = El<T>::mma(a, pf[u][c], o[u][d]);
+                    const Frag a = load_frag_t(Vs, ldv, 32 * c + 4 * g, 32 * c + 16 + 4 * g, 16 * d, i);
+                    o[d] = El<T>::mma(a, pf[c], o[d]);
                 }
             }
         }
         __syncthreads();
     }
+    float l = l_run;
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (j >= nq) return;
+    const float inv = 1.0f / l;
 #pragma unroll
-    for (int u = 0; u < QT; ++u) {
-        const int j = qb + 16 * (wave * QT + u) + i;
-        float l = l_run[u];
-        l += __shfl_xor(l, 16, 64);
-        l += __shfl_xor(l, 32, 64);
+    for (int d = 0; d < DV; ++d) {
+        if (d >= dv) continue;
+        const int col = h * V + 16 * d + 4 * g;
+        const f32x4 z = load_quad(gate + tok * ld_gate + col);
+        f32x4 v = o[d];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] *= inv * sigmoid(z[r]);
+        store_quad(out + tok * ld_out + col, v);
+    }
+}
+
+// Keys of 128 + 64 and values of 128 in bfloat16, on the loop of flash_tile.h: 80 KB of LDS, two workgroups of 128 query rows per CU (or one of 256).
+// Workgroups go round-robin over the 8 XCDs: a head's query blocks sit on one of them and share its L2, the longest of all heads first.
+// 32 heads, against one workgroup of 256 rows per CU with tiles staged in registers and one product at a time: 4 096 rows 302 -> 243 us, behind
+// 4 096 keys 597 -> 568 (907 TFLOP/s), 6 x 666 rows 111 -> 92, 3 x 700 rows behind 4 096 401 -> 335.
+template <int NWV>
+__global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_sized_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kv, const bf16* __restrict__ ck,
+                                                                    const int32_t* __restrict__ seq, const int32_t* __restrict__ pos,
+                                                                    const float* __restrict__ cosb, const float* __restrict__ sinb, int half,
+                                                                    int max_pos, const bf16* __restrict__ gate, int64_t ld_gate,
+                                                                    bf16* __restrict__ out, int64_t ld_out, int tq, int tk, int H, int C,
+                                                                    float scale) {
+    typedef FlashTile<2, NWV> Flash;
+    constexpr int N = 128, R = 64, V = 128, QB = Flash::ROWS, KT = Flash::KT;
+    extern __shared__ __align__(16) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, i = lane & 15;
+    const int nqb = gridDim.x / H, id = blockIdx.x;
+    const bool by_xcd = (H & 7) == 0;
+    const int hx = by_xcd ? H >> 3 : H, j_ = by_xcd ? id >> 3 : id, h = by_xcd ? (j_ % hx) * 8 + (id & 7) : j_ % hx;
+    const int32_t* sq = seq + 4 * blockIdx.y;
+    const int q_at = sq[0], nq = sq[1], k_at = sq[2], nk = sq[3];
+    const int qb = (nqb - 1 - j_ / hx) * QB;
+    if (qb >= nq || nq < 1 || nk < nq || q_at < 0 || k_at < 0 || q_at + nq > tq || k_at + nk > tk) return;
+    const int past = nk - nq;
+    const int64_t ld_kv = (int64_t)H * (N + V), ld_ck = C + R;
+
+    Flash f;
+    int hi[2], lo[2] = {0, 0};                                // last key that the lane's own query token sees
+    auto load = [&] {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int j = min(qb + 32 * wave + 16 * u + i, nq - 1);
+            hi[u] = past + j;
+            const int64_t tok = q_at + j;
+            const bf16* src = q + (tok * H + h) * (int64_t)(N + R) + 8 * g;
+            int p = pos[tok];
+            p = p < 0 ? 0 : (p >= max_pos ? max_pos - 1 : p);
+#pragma unroll
+            for (int c = 0; c < 6; ++c) {
+                bf16x8 v = load_frag(src + 32 * c);
+                if (c >= 4 && half > 0) {
+                    const int pr = (c - 4) * 16 + 4 * g;
+                    float cs[4], sn[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {             // (all loads at once: behind the condition each waited for the one before)
+                        const int64_t at = (int64_t)p * half + min(pr + e, half - 1);
+                        cs[e] = cosb[at];
+                        sn[e] = sinb[at];
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float a = (float)v[2 * e], b = (float)v[2 * e + 1];
+                        const bf16 x = (bf16)(a * cs[e] - b * sn[e]), y = (bf16)(b * cs[e] + a * sn[e]);
+                        v[2 * e] = pr + e < half ? x : v[2 * e];
+                        v[2 * e + 1] = pr + e < half ? y : v[2 * e + 1];
+                    }
+                }
+                f.q[u][c] = v;
+            }
+        }
+    };
+    const int wave_first = past + qb + 32 * wave;             // the wave's first row: tiles that end before it need no mask
+    f.run(smem, 0, (past + min(qb + QB, nq) - 1) / KT + 1, (uint32_t)ld_kv, (uint32_t)ld_ck, scale, lo, hi, load,
+          [&](int t) {
+              const bf16* base = kv + (int64_t)(k_at + t * KT) * ld_kv;
+              return typename Flash::Tile{base + h * N, ck + (int64_t)(k_at + t * KT) * ld_ck + C, base + (int64_t)H * N + h * V, min(KT, nk - t * KT) - 1};
+          },
+          [&](int k0) { return k0 + KT - 1 <= wave_first; });
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int j = qb + 32 * wave + 16 * u + i;
+        const float inv = 1.0f / f.weight(u);
         if (j >= nq) continue;
-        const float inv = 1.0f / l;
         const int64_t tok = q_at + j;
 #pragma unroll
-        for (int d = 0; d < DV; ++d) {
-            if (!EXACT && d >= dv) continue;
+        for (int d = 0; d < 8; ++d) {
             const int col = h * V + 16 * d + 4 * g;
             const f32x4 z = load_quad(gate + tok * ld_gate + col);
-            f32x4 v = o[u][d];
+            f32x4 v = f.acc[u][d];
 #pragma unroll
             for (int r = 0; r < 4; ++r) v[r] *= inv * sigmoid(z[r]);
             store_quad(out + tok * ld_out + col, v);
@@ -796,21 +806,36 @@ __global__ __launch_bounds__(64 * NWV, NWV / 4) void attn_prefill_kernel(const T
     }
 }
 
-template <typename T, int NWV, int KT, int QT, int DK, int DV, int NCX>
+template <int NWV>
+static int launch_prefill_sized(const void* q, const void* kv, const void* ck, const int32_t* seq, int nseq, int max_new, const int32_t* pos,
+                                const float* cosb, const float* sinb, int half, int max_pos, const void* gate, int64_t ld_gate, void* out,
+                                int64_t ld_out, int tq, int tk, int H, int C, float scale, hipStream_t st) {
+    typedef FlashTile<2, NWV> Flash;
+    auto k = attn_prefill_sized_kernel<NWV>;
+    const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, Flash::LDS);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL(k, dim3((unsigned)((max_new + Flash::ROWS - 1) / Flash::ROWS * H), nseq), dim3(64 * NWV), Flash::LDS, st, (const bf16*)q,
+                       (const bf16*)kv, (const bf16*)ck, seq, pos, cosb, sinb, half, max_pos, (const bf16*)gate, ld_gate, (bf16*)out, ld_out, tq, tk, H,
+                       C, scale);
+    TFL_LAUNCH_CHECK();
+    return TF_OK;
+}
+
+template <typename T, int KT, int DK, int DV>
 static int launch_prefill(const void* q, const void* kv, const void* ck, const int32_t* seq, int nseq, int max_new, const int32_t* pos,
                           const float* cosb, const float* sinb, int half, int max_pos, const void* gate, int64_t ld_gate, void* out,
                           int64_t ld_out, int tq, int tk, int H, int N, int R, int V, int C, float scale, hipStream_t st) {
     const int pad = 16 / (int)sizeof(T);
-    const size_t lds = (NCX > 0 ? 2 : 1) * sizeof(T) * KT * (size_t)(N + R + V + 3 * pad);
+    const size_t lds = sizeof(T) * KT * (size_t)(N + R + V + 3 * pad);
     if (lds > 160 * 1024) return TF_ERANGE;
-    auto k = attn_prefill_kernel<T, NWV, KT, QT, DK, DV, NCX>;
+    auto k = attn_prefill_kernel<T, KT, DK, DV>;
     static bool attr = false;
     if (!attr) {
         const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e != hipSuccess) return (int)e;
         attr = true;
     }
-    hipLaunchKernelGGL(k, dim3((max_new + 16 * NWV * QT - 1) / (16 * NWV * QT) * H, nseq), dim3(64 * NWV), lds, st, (const T*)q, (const T*)kv, (const T*)ck,
+    hipLaunchKernelGGL(k, dim3((max_new + 63) / 64 * H, nseq), dim3(256), lds, st, (const T*)q, (const T*)kv, (const T*)ck,
                        seq, pos, cosb, sinb, half, max_pos, (const T*)gate, ld_gate, (T*)out, ld_out, tq, tk, H, N, R, V, C, scale);
     TFL_LAUNCH_CHECK();
     return TF_OK;
@@ -825,26 +850,32 @@ extern "C" int tfl_attn_prefill(const void* q, const void* kv, const void* ck, c
     if (half < 0 || 2 * half > R || max_pos < 1 || (half && (!cosb || !sinb)) || !(scale > 0.f)) return TF_EINVAL;
     if ((ld_gate & 3) || (ld_out & 3) || ld_gate < (int64_t)H * V || ld_out < (int64_t)H * V) return TF_EINVAL;
     hipStream_t st = (hipStream_t)stream;
-#define GO(T, NWV, KT, QT, DK, DV, NCX)                                                                                               \
-    return launch_prefill<T, NWV, KT, QT, DK, DV, NCX>(q, kv, ck, seq, nseq, max_new, pos, cosb, sinb, half, max_pos, gate, ld_gate, \
+#define GO(T, KT, DK, DV)                                                                                                             \
+    return launch_prefill<T, KT, DK, DV>(q, kv, ck, seq, nseq, max_new, pos, cosb, sinb, half, max_pos, gate, ld_gate, \
                                                   out, ld_out, tq, tk, H, N, R, V, C, scale, st)
+#define SIZED_ARGS q, kv, ck, seq, nseq, max_new, pos, cosb, sinb, half, max_pos, gate, ld_gate, out, ld_out, tq, tk, H, C, scale, st
     const int D = N + R;
     if (dtype == 0) {
-        if (N == 128 && R == 64 && V == 128) {                   // 256 query rows per workgroup where that still fills the chip
-            if ((int64_t)((max_new + 255) / 256) * H * nseq >= 256) GO(bf16, 8, 64, 2, 6, 8, 4);
-            GO(bf16, 4, 64, 2, 6, 8, 4);
+        if (N == 128 && R == 64 && V == 128 && C <= 1 << 24) {   // (63 rows of either stay below 2^32 bytes)
+            // 256 rows per workgroup read half as much, which tells where the keys of all heads come from memory (from 16 384 per sequence), but
+            // only with whole rounds of 256: 2 048 rows behind 20 000 keys 879 -> 853 us, 4 096 1 812 -> 1 758; behind 10 000 471 -> 478,
+            // 2 500 behind 20 000 1 322 -> 1 568
+            const int64_t wide = (int64_t)((max_new + 255) / 256) * H * nseq;
+            if (tk / nseq >= 16384 && (wide + 255) / 256 * 256 - wide < 48) return launch_prefill_sized<8>(SIZED_ARGS);
+            return launch_prefill_sized<4>(SIZED_ARGS);
         }
-        if (D <= 96 && V <= 64) GO(bf16, 4, 64, 1, 3, 4, 0);
-        if (D <= 192 && V <= 128) GO(bf16, 4, 64, 1, 6, 8, 0);
-        if (D <= 384 && V <= 256) GO(bf16, 4, 64, 1, 12, 16, 0);
+        if (D <= 96 && V <= 64) GO(bf16, 64, 3, 4);
+        if (D <= 192 && V <= 128) GO(bf16, 64, 6, 8);
+        if (D <= 384 && V <= 256) GO(bf16, 64, 12, 16);
         return TF_ERANGE;
     }
     if (dtype == 1) {
-        if (D <= 96 && V <= 64) GO(float, 4, 32, 1, 3, 4, 0);
-        if (D <= 192 && V <= 128) GO(float, 4, 32, 1, 6, 8, 0);
-        if (D <= 384 && V <= 256) GO(float, 4, 32, 1, 12, 16, 0);
+        if (D <= 96 && V <= 64) GO(float, 32, 3, 4);
+        if (D <= 192 && V <= 128) GO(float, 32, 6, 8);
+        if (D <= 384 && V <= 256) GO(float, 32, 12, 16);
         return TF_ERANGE;
     }
 #undef GO
+#undef SIZED_ARGS
     return TF_EINVAL;
 }
