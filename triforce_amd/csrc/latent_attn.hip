@@ -486,12 +486,14 @@ extern "C" int64_t tfl_attn_decode_ws_floats(int rows, int H, int C, int nsplit)
     return nsplit == 1 ? 0 : (int64_t)rows * H * nsplit * (C + 2);
 }
 
-// One workgroup per CU (256) as long as a split keeps at least two pages of keys.
+// One workgroup per CU (256) as long as a split keeps at least two pages of keys, or one of up to 16: there the second page costs more
+// (2.4 us) than its partial rows (one row, attention and merge: 500 keys 16.7 -> 14.3 us, 1 000 16.8 -> 14.6; 4 000 keys 18.2 either way, two rows of
+// 4 000 19.7 against 20.7).
 extern "C" int tfl_attn_decode_pick_nsplit(int rows, int H, int max_len) {
     if (rows < 1 || H < 1 || max_len < 1) return 1;
     const int groups = H <= 16 ? 1 : (H + 31) / 32;
     int n = 256 / (rows * groups);
-    const int cap = (max_len + 2 * TFL_PAGE - 1) / (2 * TFL_PAGE);
+    const int pages = (max_len + TFL_PAGE - 1) / TFL_PAGE, cap = pages <= 16 ? pages : (pages + 1) / 2;
     if (n > cap) n = cap;
     if (n > TFL_MAX_SPLIT) n = TFL_MAX_SPLIT;
     return n < 1 ? 1 : n;
