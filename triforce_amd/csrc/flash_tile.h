@@ -31,7 +31,7 @@ template <int KR, int NWV> struct FlashTile {
         const float sc = scale * 1.4426950408889634f;
 #pragma unroll
         for (int u = 0; u < QT; ++u) {
-            m[u] = -1e30f;
+            m[u] = -__FLT_MAX__;
             l[u] = 0.f;
 #pragma unroll
             for (int d = 0; d < NT; ++d) acc[u][d] = f32x4{0.f, 0.f, 0.f, 0.f};
