@@ -724,7 +724,8 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(const T* __restric
 }
 
 // Keys of 128 + 64 and values of 128 in bfloat16, on the loop of flash_tile.h: 80 KB of LDS, two workgroups of 128 query rows per CU (or one of 256).
-// Workgroups go round-robin over the 8 XCDs: a head's query blocks sit on one of them and share its L2, the longest of all heads first.
+// Workgroups go round-robin over the 8 XCDs: a head's query blocks sit on one of them and share its L2, the last blocks of all sequences and
+// heads first (sequence by sequence six of 222 to 1 333 rows take 106 us, not 98).
 // 32 heads, against one workgroup of 256 rows per CU with tiles staged in registers and one product at a time: 4 096 rows 302 -> 243 us, behind
 // 4 096 keys 597 -> 568 (907 TFLOP/s), 6 x 666 rows 111 -> 92, 3 x 700 rows behind 4 096 401 -> 335.
 template <int NWV>
@@ -738,12 +739,11 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_sized_kernel(const b
     constexpr int N = 128, R = 64, V = 128, QB = Flash::ROWS, KT = Flash::KT;
     extern __shared__ __align__(16) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, i = lane & 15;
-    const int nqb = gridDim.x / H, id = blockIdx.x;
+    const int id = blockIdx.x, qb = (gridDim.y - 1 - blockIdx.y) * QB;
     const bool by_xcd = (H & 7) == 0;
     const int hx = by_xcd ? H >> 3 : H, j_ = by_xcd ? id >> 3 : id, h = by_xcd ? (j_ % hx) * 8 + (id & 7) : j_ % hx;
-    const int32_t* sq = seq + 4 * blockIdx.y;
+    const int32_t* sq = seq + 4 * (j_ / hx);
     const int q_at = sq[0], nq = sq[1], k_at = sq[2], nk = sq[3];
-    const int qb = (nqb - 1 - j_ / hx) * QB;
     if (qb >= nq || nq < 1 || nk < nq || q_at < 0 || k_at < 0 || q_at + nq > tq || k_at + nk > tk) return;
     const int past = nk - nq;
     const int64_t ld_kv = (int64_t)H * (N + V), ld_ck = C + R;
@@ -816,7 +816,7 @@ static int launch_prefill_sized(const void* q, const void* kv, const void* ck, c
     auto k = attn_prefill_sized_kernel<NWV>;
     const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, Flash::LDS);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(k, dim3((unsigned)((max_new + Flash::ROWS - 1) / Flash::ROWS * H), nseq), dim3(64 * NWV), Flash::LDS, st, (const bf16*)q,
+    hipLaunchKernelGGL(k, dim3((unsigned)(H * nseq), (max_new + Flash::ROWS - 1) / Flash::ROWS), dim3(64 * NWV), Flash::LDS, st, (const bf16*)q,
                        (const bf16*)kv, (const bf16*)ck, seq, pos, cosb, sinb, half, max_pos, (const bf16*)gate, ld_gate, (bf16*)out, ld_out, tq, tk, H,
                        C, scale);
     TFL_LAUNCH_CHECK();
@@ -858,7 +858,8 @@ extern "C" int tfl_attn_prefill(const void* q, const void* kv, const void* ck, c
 #define SIZED_ARGS q, kv, ck, seq, nseq, max_new, pos, cosb, sinb, half, max_pos, gate, ld_gate, out, ld_out, tq, tk, H, C, scale, st
     const int D = N + R;
     if (dtype == 0) {
-        if (N == 128 && R == 64 && V == 128 && C <= 1 << 24) {   // (63 rows of either stay below 2^32 bytes)
+        if (N == 128 && R == 64 && V == 128 && C <= 1 << 24 && (int64_t)H * nseq <= 1 << 30 && max_new <= 1 << 22) {       // (63 rows of
+                                                                 // either stay below 2^32 bytes)
             // 256 rows per workgroup read half as much, which tells where the keys of all heads come from memory (from 16 384 per sequence), but
             // only with whole rounds of 256: 2 048 rows behind 20 000 keys 879 -> 853 us, 4 096 1 812 -> 1 758; behind 10 000 471 -> 478,
             // 2 500 behind 20 000 1 322 -> 1 568
