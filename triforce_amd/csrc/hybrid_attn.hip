@@ -8,10 +8,10 @@
 #include "flash_tile.h"
 #include "hybrid_common.h"
 
-// Workgroups go round-robin over the 8 XCDs: the query blocks of a key / value head stay on one of them (its heads side by side), the last blocks
-// of all sequences and heads first (sequence by sequence six of 222 to 1 333 rows take 82 us, not 73).  32 heads on 8, against workgroups of 256 rows with tiles staged in
-// registers, head by head: 4 096 rows 276 -> 197 us, 3 904 behind 4 096 531 -> 478 (810 TFLOP/s), 4 096 behind 6 000 with a chunk's edge at 8 192
-// 569 -> 453, 6 x 1 000 behind 500 in chunks of 640 140 -> 94.
+// Workgroups go round-robin over the 8 XCDs: the query blocks of a key / value head stay on one of them (its heads side by side), the last
+// blocks of all sequences and heads first (sequence by sequence six of 222 to 1 333 rows take 82 us, not 73).  32 heads on 8, against
+// workgroups of 256 rows with tiles staged in registers, head by head: 4 096 rows 276 -> 197 us, 3 904 behind 4 096 531 -> 478 (810
+// TFLOP/s), 4 096 behind 6 000 with a chunk's edge at 8 192 569 -> 453, 6 x 1 000 behind 500 in chunks of 640 140 -> 94.
 __global__ __launch_bounds__(256, 2) void attn_chunk_sized_kernel(const bf16* __restrict__ q, int64_t ld_q, const bf16* __restrict__ cache, int n_pages,
                                                                   const int32_t* __restrict__ table, int table_ld, const int32_t* __restrict__ seq,
                                                                   const bf16* __restrict__ gate, int64_t ld_gate, bf16* __restrict__ out,
