@@ -116,3 +116,29 @@ _Zk: ; @_Zk
     for k, v in topp.items():
         assert v["arrivals"] == 2 and v["arrivals_without_drain"] == 0 and v["fences"] == 0, (k, v)
         assert v["sc1_loads"] >= 20 and v["sc1_stores"] >= 8 and v["vgpr_spills"] == 0 and v["vgprs"] <= 128, (k, v)
+
+
+def test_split_product_drains_its_lds_dma_before_every_barrier():
+    """The waves of split_gemm_kernel read tiles that other waves' DMA brought to LDS.  Each path from a DMA to a barrier has to pass a
+    drain that the source asks for; a counted wait (all but the four youngest loads) would hold only for one order of the loads."""
+    synthetic = """
+_Zk: ; @_Zk
+\tglobal_load_lds_dwordx4 v[0:1], off
+\tglobal_load_dwordx4 v[4:7], v[8:9], off
+\ts_cbranch_scc1 .LBB0_2
+\t;;#ASMSTART
+\ts_waitcnt vmcnt(0)
+\t;;#ASMEND
+.LBB0_2:
+\ts_waitcnt vmcnt(0)
+\ts_barrier
+\ts_endpgm
+.Lfunc_end0:
+"""
+    assert isa_lint.undrained_dma(synthetic)["_Zk"] == dict(dma=1, undrained_barriers=1)
+    assert isa_lint.undrained_dma(synthetic.replace("\ts_cbranch_scc1 .LBB0_2\n", ""))["_Zk"] == dict(dma=1, undrained_barriers=0)
+    from triforce_amd.build import FLAGS
+    extra = [f for f in FLAGS if f == "-mllvm" or f.startswith("-amdgpu-")]
+    shapes = isa_lint.undrained_dma(isa_lint.compile_to_asm(os.path.join(CSRC, "split_gemm.hip"), extra=extra))
+    kernels = {k: v for k, v in shapes.items() if "split_gemm_kernel" in k}
+    assert kernels and all(v["dma"] >= 6 and v["undrained_barriers"] == 0 for v in kernels.values()), shapes

@@ -207,3 +207,45 @@ def handoff_shape(text):
         if m.group(1) in out:
             out[m.group(1)].update(vgprs=int(m.group(2)), vgpr_spills=int(m.group(3)))
     return out
+
+
+# ---- fourth check: LDS-DMA in front of a barrier that other waves read behind (csrc/split_gemm.hip) ---------------------------
+# global_load_lds writes LDS behind the wave's back and counts in vmcnt.  Waits that the compiler inserts follow its own idea of what
+# aliases, and a counted wait (vmcnt(4)) holds only as long as the scheduler keeps the loads' order.  undrained_dma() walks every
+# path of a kernel and counts the barriers that some path reaches with a DMA issued since the last `s_waitcnt vmcnt(0)` that the SOURCE
+# wrote (inline asm).
+def undrained_dma(text):
+    out = {}
+    for m in re.finditer(r"^(_Z\w+):\s*;\s*@\1\n([\s\S]*?)\n\.Lfunc_end\d+:", text, re.M):
+        insts, labels, inasm = [], {}, False
+        for line in m.group(2).split("\n"):
+            t = line.strip()
+            lab = re.match(r"^(\.LBB\w+):", t)
+            if "ASMSTART" in t or "ASMEND" in t:
+                inasm = "ASMSTART" in t
+            elif lab:
+                labels[lab.group(1)] = len(insts)
+            elif t and t[0] not in ";.":
+                insts.append((t, inasm))
+        dma, bad, seen, work = sum(t.startswith("global_load_lds") for t, _ in insts), set(), set(), [(0, False)]
+        while work:
+            at, pending = work.pop()
+            while at < len(insts) and (at, pending) not in seen:
+                seen.add((at, pending))
+                t, own = insts[at]
+                if t.startswith("global_load_lds"):
+                    pending = True
+                elif own and t.startswith("s_waitcnt") and "vmcnt(0)" in t:
+                    pending = False
+                elif t.startswith("s_barrier") and pending:
+                    bad.add(at)
+                elif t.startswith("s_endpgm"):
+                    break
+                jump = re.match(r"^s_c?branch\w*\s+(\.LBB\w+)", t)
+                if jump:
+                    work.append((labels[jump.group(1)], pending))
+                    if t.startswith("s_branch"):
+                        break
+                at += 1
+        out[m.group(1)] = dict(dma=dma, undrained_barriers=len(bad))
+    return out

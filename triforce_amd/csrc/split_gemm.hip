@@ -133,6 +133,15 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
 #pragma unroll
         for (int f = 0; f < 2; ++f) cut_store(staged[f], tiles + buf * BUF + (wave + 8 * f) * 1536 + lane * 8);
     };
+    // What makes a step's tiles visible to the other waves: this wave's DMA has landed (nothing may be in flight but the weights asked for
+    // behind it, which stay in flight over the barrier), its LDS stores are done, and no access crosses the barrier.  Both are compiler
+    // fences too: an access to LDS may not move over them, whatever order the scheduler likes.
+    auto landed = [&] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+    auto meet = [&] {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
     const bool live = mt0 * XP + wm * MT < xpan;              // a wave without rows leaves the matrix core to its neighbour
     f32x4 acc[4][MT];
 #pragma unroll
@@ -143,10 +152,9 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
         fetch_x(c_beg, 0);
         fetch_w(c_beg);
         put_w(0);
+        landed();
         fetch_w(min(c_beg + 1, c_end - 1));
-        __builtin_amdgcn_s_waitcnt(0x0F74);                   // vmcnt(4): all but the weights just asked for
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
+        meet();
     }
     for (int c = c_beg; c < c_end; ++c) {
         const int buf = (c - c_beg) & 1;
@@ -172,10 +180,9 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
             }
         }
         put_w(buf ^ 1);
+        landed();
         fetch_w(min(c + 2, c_end - 1));
-        __builtin_amdgcn_s_waitcnt(0x0F74);                   // this wave's part of the next step is in LDS before the barrier
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
+        meet();
     }
     float* y = a.splits > 1 ? a.ws + (int64_t)blockIdx.y * a.rows * a.n : a.out;
     const int64_t ld = a.splits > 1 ? a.n : a.ld_out;
