@@ -258,6 +258,51 @@ def test_split_float32_product(rows, n, k, splits):
         assert err.max() <= 2.0 ** -24 * (6 * k / 32) ** 0.5 + 2.0 ** -22
 
 
+# products that stand alone (a row of x with one entry): every bit of both factors counts, in every place of a step of 32
+@pytest.mark.parametrize("splits", [1, 2])
+def test_split_float32_single_products(splits):
+    from triforce_amd import ops_tile as ot
+    g = torch.Generator(device=DEV).manual_seed(splits)
+    k, n = 64, 512
+    a = torch.rand(k, generator=g, device=DEV) + 1
+    w = (torch.rand(n, k, generator=g, device=DEV) + 1) * (torch.randint(0, 2, (n, k), generator=g, device=DEV) * 2 - 1)
+    a[::2], w[::3] = 1.0 + 65535 * 2.0 ** -23, 1.0 + 65535 * 2.0 ** -23               # (what cutting loses most of)
+    got, want = ot.split_linear(torch.diag(a), w, splits).double(), a.double()[:, None] * w.double().T
+    # left out: ml + lm of 2^-25 each and ll; the small products' sum and the last addition are rounded, 2^-24 and less
+    assert ((got - want).abs() <= 2.25 * 2.0 ** -24 * want.abs()).all()
+
+
+def _factors(kind, rows, n, k):
+    g = torch.Generator(device=DEV).manual_seed(k)
+    x, w = torch.randn(rows, k, generator=g, device=DEV), torch.randn(n, k, generator=g, device=DEV)
+    if kind == "uniform":
+        return torch.rand(rows, k, generator=g, device=DEV) + 1, torch.rand(n, k, generator=g, device=DEV) + 1
+    return {"normal": (x, w), "absolute": (x.abs(), w.abs()), "mean one": (x + 1, w + 1), "mixed": (x.abs(), w)}[kind]
+
+
+# sums of one sign and of a mean: what a running sum swallows does not average out
+@pytest.mark.parametrize("k,splits", [(15104, 1), (15104, 0), (4096, 1), (1024, 3)])
+@pytest.mark.parametrize("kind", ["normal", "absolute", "mean one", "uniform", "mixed"])
+def test_split_float32_sums(k, splits, kind):
+    from triforce_amd import ops_tile as ot
+    x, w = _factors(kind, 160, 256, k)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    # k / 32 roundings of a running sum, 2^-24 of it each and independent; five of them for the largest of 40 960 results
+    assert ((ot.split_linear(x, w, splits).double() - want).abs() / size).max() <= 5 * 2.0 ** -24 * (1 + (k / 32 / 3) ** 0.5)
+
+
+# where these products are taken, they are no further off than the library's on the fp32 instruction
+@pytest.mark.parametrize("rows,n,k", [(256, 1136, 15104), (272, 4112, 4096), (1030, 4096, 1024), (300, 512, 65536)])
+@pytest.mark.parametrize("kind", ["normal", "absolute", "mean one", "uniform", "mixed"])
+def test_split_float32_against_the_instruction(rows, n, k, kind):
+    from triforce_amd import ops_tile as ot
+    x, w = _factors(kind, rows, n, k)
+    want, library = x.double() @ w.double().T, torch.nn.functional.linear(x, w)
+    got = ot.linear_rows(x, w)
+    assert torch.equal(got, ot.split_linear(x, w))
+    assert (got.double() - want).norm() <= (library.double() - want).norm()
+
+
 @pytest.mark.parametrize("splits", [1, 2])
 def test_split_float32_extremes(splits):
     from triforce_amd import ops_tile as ot

@@ -1,12 +1,17 @@
 // float32 products of many rows (prefill) on the bfloat16 matrix cores: y = x . W^T.
 //
-// A float32 is exactly the sum of three bfloat16 (its 24 bits of mantissa cut into 8 + 8 + 8; cutting, not rounding, so that nothing
-// overflows), and six of the nine products of two such sums carry everything down to 2^-24 of a product: with h, m, l the three parts,
-// hh + hm + mh + mm + hl + lh; what is left out (ml, lm, ll) is below 2^-23 * 2^-8 of it.  Each product of bfloat16 is exact in the
-// matrix core and the sums are fp32, over k in steps of 32 where the fp32 instruction takes 4: the error against 64 bits is that of a
-// product on the fp32 instruction or less (normal values, 4 096 outputs: 700 x 4 096 1.1e-6 -> 4.4e-7, 700 x 15 104 2.1e-6 -> 7.2e-7, 2 048 x
-// 15 104 without parts 2.2e-6 -> 2.1e-6).  Six bf16 instructions take 3/8 of the cycles of the eight fp32 ones that cover the same
-// 16 x 16 x 32.
+// The products of Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision Computations"
+// (ARITH 2019): a float32 is exactly the sum of three bfloat16 h + m + l, each the nearest to what is left (|m| <= 2^-8 and |l| <= 2^-17 of the
+// value, of either sign), and six of the nine products of two such sums, hh + hm + mh + mm + hl + lh, leave out at most 2^-24 of a product
+// (ml + lm, 2^-25 each, and ll), without a preferred sign.  Products of bfloat16 are exact in the matrix core and the sums are fp32, hh in
+// an accumulator of its own: beside a large sum the five small products of a step would fall below its last place, step after step, and
+// with parts that are cut instead of rounded always towards zero.
+// Error against 64 bits, relative 2-norm, fp32 instruction -> cut parts in one accumulator -> this:
+//   700 rows of k = 4 096   normals 1.1e-6 -> 7.1e-7 -> 2.7e-7, their absolute values 9.9e-7 -> 3.2e-6 -> 1.8e-7;
+//   700 rows of k = 15 104  normals 2.1e-6 -> 9.2e-7 -> 3.4e-7, absolute values 1.7e-6 -> 5.8e-6 -> 1.2e-7, normals of mean 1
+//   1.5e-6 -> 4.7e-6 -> 1.4e-7, uniform in 1 .. 2 1.6e-6 -> 8.4e-6 -> 1.4e-7.
+// (Rounded parts in one accumulator: 9.1e-7, 2.2e-7, 2.5e-7, 2.3e-7.  The accuracy costs 1 to 2 %: 22 016 x 4 096 at 700 rows 730 -> 740 us.)
+// Six bf16 instructions take 3/8 of the cycles of the eight fp32 ones that cover the same 16 x 16 x 32.
 //
 // 256 outputs x 128 rows per workgroup, eight waves of 64 x 64: per step of 32 a wave reads 24 KB from LDS for 96 products (1 536 cycles),
 // half of what LDS delivers.  x is cut once by a kernel in front, into planes in MFMA order ([rows/16][k/32][3][64 lanes][8]: a fragment is one
@@ -26,16 +31,14 @@
 #define SPLIT_KC 512                   // columns of x that one workgroup cuts
 
 __device__ __forceinline__ void cut_pair(float a, float b, uint32_t& h, uint32_t& m, uint32_t& l) {
-    constexpr uint32_t HIGH = 0x07060302u;                    // the upper halves of both
-    const uint32_t ha = __builtin_bit_cast(uint32_t, a), hb = __builtin_bit_cast(uint32_t, b);
-    h = __builtin_amdgcn_perm(hb, ha, HIGH);
-    a -= __builtin_bit_cast(float, ha & 0xFFFF0000u);
-    b -= __builtin_bit_cast(float, hb & 0xFFFF0000u);
-    const uint32_t ma = __builtin_bit_cast(uint32_t, a), mb = __builtin_bit_cast(uint32_t, b);
-    m = __builtin_amdgcn_perm(mb, ma, HIGH);
-    a -= __builtin_bit_cast(float, ma & 0xFFFF0000u);
-    b -= __builtin_bit_cast(float, mb & 0xFFFF0000u);
-    l = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), HIGH);
+    typedef bf16 Pair __attribute__((ext_vector_type(2)));
+    h = __builtin_bit_cast(uint32_t, Pair{(bf16)a, (bf16)b});
+    a -= __builtin_bit_cast(float, h << 16);
+    b -= __builtin_bit_cast(float, h & 0xFFFF0000u);
+    m = __builtin_bit_cast(uint32_t, Pair{(bf16)a, (bf16)b});
+    a -= __builtin_bit_cast(float, m << 16);
+    b -= __builtin_bit_cast(float, m & 0xFFFF0000u);
+    l = __builtin_bit_cast(uint32_t, Pair{(bf16)a, (bf16)b});
 }
 
 // Eight values into the three planes of a fragment.
@@ -143,11 +146,11 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
         asm volatile("" ::: "memory");
     };
     const bool live = mt0 * XP + wm * MT < xpan;              // a wave without rows leaves the matrix core to its neighbour
-    f32x4 acc[4][MT];
+    f32x4 acc[4][MT], low[4][MT];                             // hh and the five small products
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int m = 0; m < MT; ++m) acc[t][m] = low[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (c_beg < c_end) {
         fetch_x(c_beg, 0);
         fetch_w(c_beg);
@@ -172,11 +175,14 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
                 bf16x8 x[3];
 #pragma unroll
                 for (int z = 0; z < 3; ++z) x[z] = load_frag(xt + (3 * m + z) * 512);
-                constexpr int WZ[6] = {2, 0, 1, 1, 0, 0}, XZ[6] = {0, 2, 1, 0, 1, 0};          // small products first
+                constexpr int WZ[6] = {2, 0, 1, 1, 0, 0}, XZ[6] = {0, 2, 1, 0, 1, 0};          // smallest first
 #pragma unroll
                 for (int q = 0; q < 6; ++q)
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][WZ[q]], x[XZ[q]], acc[t][m], 0, 0, 0);
+                    for (int t = 0; t < 4; ++t) {
+                        f32x4& s = q < 5 ? low[t][m] : acc[t][m];
+                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][WZ[q]], x[XZ[q]], s, 0, 0, 0);
+                    }
             }
         }
         put_w(buf ^ 1);
@@ -194,6 +200,8 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
         for (int t = 0; t < 4; ++t) {
             const int n = nt * 256 + 64 * wn + 16 * t + 4 * g;
             if (n >= a.n) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[t][m][e] += low[t][m][e];
             if (a.splits == 1) mend(a, row, n, acc[t][m]);
             *reinterpret_cast<f32x4*>(y + (int64_t)row * ld + n) = acc[t][m];
         }

@@ -152,9 +152,9 @@ def linear_rows(x, w):
     """x . W^T over many rows (prefill), w [n, k] contiguous: the library GEMM, and for large float32 products split_linear.  Its tiles
     are 256 x 128: from 256 rows and 2^32 multiply-adds on it is the faster one (256 x 4 096 x 4 096 73 -> 61 us, 2 048 x 2 048 x 1 024
     70 -> 63, 700 x 22 016 x 4 096 940 -> 750), below that it leaves CUs idle (300 x 6 144 x 1 536 51 -> 55, 64 x 22 016 x 4 096
-    115 -> 133)."""
+    115 -> 133).  Up to k = 65 536 its error is a tenth to a half of the library's; at 2^20, with as few parts, the two are equal."""
     rows, (n, k) = x.shape[0], w.shape
-    if x.dtype == torch.float32 and 256 <= rows <= 1 << 24 and rows * n * k >= 1 << 32 and n % 16 == 0 and k % 32 == 0 \
+    if x.dtype == torch.float32 and 256 <= rows <= 1 << 24 and rows * n * k >= 1 << 32 and n % 16 == 0 and k % 32 == 0 and k <= 1 << 16 \
             and w.data_ptr() % 16 == 0:
         return split_linear(x, w)
     return F.linear(x, w)
