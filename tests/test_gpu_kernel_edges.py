@@ -303,6 +303,22 @@ def test_split_float32_against_the_instruction(rows, n, k, kind):
     assert (got.double() - want).norm() <= (library.double() - want).norm()
 
 
+# every pair of scales, down to denormal factors: results of ordinary size from a tiny factor and a huge one, tiny and huge results
+@pytest.mark.parametrize("splits", [1, 2])
+def test_split_float32_scales(splits):
+    from triforce_amd import ops_tile as ot
+    g = torch.Generator(device=DEV).manual_seed(splits)
+    k = 64
+    scales = torch.tensor([-147, -140, -126, -120, -112, -100, -64, -24, 0, 30, 64, 79, 81, 100, 106, 120], device=DEV)
+    x, w = torch.randn(256, k, generator=g, device=DEV, dtype=torch.float64), torch.randn(256, k, generator=g, device=DEV, dtype=torch.float64)
+    x, w = ((t * torch.exp2(scales.repeat(16)[:, None].double())).float() for t in (x, w))
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    got = ot.split_linear(x, w, splits).double()
+    ok = size < 2.0 ** 127                                       # (above, a partial sum may overflow in one order and not in another)
+    assert torch.isfinite(got[ok]).all() and not torch.isnan(got[want.abs() > 2.0 ** 129]).any()
+    assert ((got - want).abs()[ok] <= (k * 2.0 ** -24 * size + k * 2.0 ** -149)[ok]).all()
+
+
 @pytest.mark.parametrize("splits", [1, 2])
 def test_split_float32_extremes(splits):
     from triforce_amd import ops_tile as ot
