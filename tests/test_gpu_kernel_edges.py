@@ -336,6 +336,29 @@ def test_split_float32_extremes(splits):
     bound = 64 * 2.0 ** -24 * (x.double().abs().nan_to_num(0, 0, 0) @ w.double().abs().nan_to_num(0, 0, 0).T) + 64 * 2.0 ** -149
     assert ((got - want).abs()[ok] <= bound[ok]).all()
 
+@pytest.mark.parametrize("rows,n,k", [(700, 8192, 4096), (300, 4096, 15104)])                    # whole k, parts of it
+def test_split_float32_strange_rows_cost_no_walk(rows, n, k):
+    """Results that are not finite are computed again by whole waves, rows with a NaN not at all; a thread for each result took 5 and
+    38 times as long as the whole product here."""
+    from triforce_amd import ops_tile as ot
+    x, w = torch.randn(rows, k, device=DEV), torch.randn(n, k, device=DEV)
+
+    def fastest():
+        spans = []
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            ot.split_linear(x, w)
+            b.record()
+            b.synchronize()
+            spans.append(a.elapsed_time(b))
+        return min(spans)
+    plain = fastest()
+    x[rows // 2, 7] = float("inf")
+    assert fastest() < 4 * plain
+    x[:, k - 3] = float("nan")
+    assert fastest() < 1.5 * plain
+
 
 def _flash_want(q, k, v, lo, hi, scale):
     """float64 attention of q [n, d] with keys lo .. hi of every row: (result, the same sums with |v|)."""

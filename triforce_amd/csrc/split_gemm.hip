@@ -27,7 +27,9 @@
 // Range: both operands are cut at 2^24 times their value, so the last bit of the smallest float32 (2^-149) is still a normal bfloat16 and no
 // product of parts that counts leaves fp32's range below; results are multiplied by 2^-48.  Above, a factor from 2^104 or a sum from 2^80
 // on becomes infinite on the way; such a result, and one that is not finite because a factor is not (an infinity times a zero part is NaN),
-// is computed again in plain fp32.  (The scaling is 16 of some 200 VALU operations per step: 22 016 x 4 096 at 700 rows 740 -> 752 us.)
+// is computed again in plain fp32, the 16 x 16 tile that it lies in by its wave on the fp32 instruction; rows of x with a NaN, which is what
+// an infinity leaves behind in a model, are marked when they are cut and keep their NaN results.  One infinite row of 700 in front of
+// 22 016 x 4 096 costs 770 -> 1 040 us, of 300 in front of 4 096 x 15 104 265 -> 530 (by a thread per result 4 200 and 9 900).  (The scaling is 16 of some 200 VALU operations per step: 22 016 x 4 096 at 700 rows 740 -> 752 us.)
 #include "tile_common.h"
 
 #define SPLIT_KC 512                   // columns of x that one workgroup cuts
@@ -61,10 +63,13 @@ __device__ __forceinline__ void cut_store(const f32x4 (&v)[2], bf16* dst) {
     for (int z = 0; z < 3; ++z) *reinterpret_cast<u32x4*>(dst + 512 * z) = out[z];
 }
 
-// One workgroup: 16 rows, SPLIT_KC columns.
-__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, int64_t ld, int rows, int k, bf16* __restrict__ planes) {
+// One workgroup: 16 rows, SPLIT_KC columns.  nans[row][part]: the row has a NaN in this part of k.
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, int64_t ld, int rows, int k, bf16* __restrict__ planes,
+                                                         int32_t* __restrict__ nans) {
+    __shared__ int found[4][16];
     const int panel = blockIdx.x, tid = threadIdx.x, lane = tid & 63, chunks = k >> 5, row = 16 * panel + (lane & 15);
     const int c_end = min(chunks, (int)(blockIdx.y + 1) * (SPLIT_KC / 32));
+    int nan = 0;
     for (int c = blockIdx.y * (SPLIT_KC / 32) + (tid >> 6); c < c_end; c += 4) {
         f32x4 v[2] = {};
         if (row < rows) {
@@ -72,8 +77,15 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
             v[0] = src[0];
             v[1] = src[1];
         }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) nan |= v[e >> 2][e & 3] != v[e >> 2][e & 3];
         cut_store(v, planes + ((int64_t)panel * chunks + c) * 1536 + lane * 8);
     }
+    nan |= __shfl_xor(nan, 16, 64);
+    nan |= __shfl_xor(nan, 32, 64);
+    if (lane < 16) found[tid >> 6][lane] = nan;
+    __syncthreads();
+    if (tid < 16 && row < rows) nans[(int64_t)row * gridDim.y + blockIdx.y] = found[0][tid] | found[1][tid] | found[2][tid] | found[3][tid];
 }
 
 struct SplitGemm {
@@ -81,21 +93,53 @@ struct SplitGemm {
     const bf16* xp;
     const float* x;
     float* out;
-    float* ws;
+    float* ws;                                                // [splits][rows][n]
+    const int32_t* nans;
     int64_t ld_x, ld_out;
     int rows, n, k, splits;
 };
 
-__device__ __forceinline__ void mend(const SplitGemm& a, int row, int n, f32x4& v) {
+__host__ __device__ __forceinline__ int split_parts(int k) { return (k + SPLIT_KC - 1) / SPLIT_KC; }
+
+// Results row0 + i, n0 + 4 g .. + 3 of a wave's 16 x 16 tile: those that are not finite, again on the fp32 instruction (whole tile, one wave).
+__device__ __forceinline__ void mend(const SplitGemm& a, int row0, int n0, f32x4& v) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
+    bool lost[4], any = false;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        if (__builtin_fabsf(v[e]) < __builtin_inff()) continue;
-        const float* x = a.x + (int64_t)row * a.ld_x;
-        const float* w = a.w + (int64_t)(n + e) * a.k;
-        float p = 0.f;
-        for (int c = 0; c < a.k && p == p; ++c) p = fmaf(x[c], w[c], p);
-        v[e] = p;
+        lost[e] = row0 + i < a.rows && !(__builtin_fabsf(v[e]) < __builtin_inff());
+        any = any || lost[e];
     }
+    if (!__any(any)) return;
+    if (any) {
+        const int parts = split_parts(a.k);
+        int nan = 0;
+        for (int z = 0; z < parts; ++z) nan |= a.nans[(int64_t)(row0 + i) * parts + z];
+        any = nan == 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lost[e] = lost[e] && any;
+    }
+    if (!__any(any)) return;
+    const float* x = a.x + (int64_t)min(row0 + i, a.rows - 1) * a.ld_x + 4 * g;
+    const float* w = a.w + (int64_t)(n0 + i) * a.k + 4 * g;
+    f32x4 p = {0.f, 0.f, 0.f, 0.f};
+    constexpr int U = 8;                                      // steps of 16 asked for at once: the loads are the chain
+    for (int c = 0; c < a.k; c += 16 * U) {
+        f32x4 xc[U], wc[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {                         // (k in any order, the same for both; past the end: the last step again, not used)
+            xc[u] = *reinterpret_cast<const f32x4*>(x + min(c + 16 * u, a.k - 16));
+            wc[u] = *reinterpret_cast<const f32x4*>(w + min(c + 16 * u, a.k - 16));
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (c + 16 * u < a.k) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) p = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[u][e], xc[u][e], p, 0, 0, 0);
+            }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = lost[e] ? p[e] : v[e];
 }
 
 // MT 16-row tiles of x per wave; waves: 4 x 64 outputs, 2 x 16 MT rows.
@@ -198,33 +242,35 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
     const int64_t ld = a.splits > 1 ? a.n : a.ld_out;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        const int row = mt0 * 32 * MT + 16 * (wm * MT + m) + i;
-        if (row >= a.rows) continue;
+        const int row0 = mt0 * 32 * MT + 16 * (wm * MT + m);
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const int n = nt * 256 + 64 * wn + 16 * t + 4 * g;
-            if (n >= a.n) continue;
+            const int n0 = nt * 256 + 64 * wn + 16 * t;
+            if (row0 >= a.rows || n0 >= a.n) continue;
+            f32x4 v;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[t][m][e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE));
-            if (a.splits == 1) mend(a, row, n, acc[t][m]);
-            *reinterpret_cast<f32x4*>(y + (int64_t)row * ld + n) = acc[t][m];
+            for (int e = 0; e < 4; ++e) v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE));
+            if (a.splits == 1) mend(a, row0, n0, v);
+            if (row0 + i < a.rows) *reinterpret_cast<f32x4*>(y + (int64_t)(row0 + i) * ld + n0 + 4 * g) = v;
         }
     }
 }
 
-// The parts of a split k, summed in order.
+// The parts of a split k, summed in order: a wave takes a 16 x 16 tile, a workgroup four side by side.
 __global__ __launch_bounds__(256) void split_sum_kernel(const SplitGemm a) {
-    const int row = blockIdx.x, n = 4 * (blockIdx.y * 256 + threadIdx.x);
-    if (n >= a.n) return;
+    const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15, cols = (a.n + 63) >> 6;
+    const int row0 = 16 * (int)(blockIdx.x / cols), n0 = 64 * (int)(blockIdx.x % cols) + 16 * (threadIdx.x >> 6);
+    if (n0 >= a.n) return;
+    const int64_t at = (int64_t)min(row0 + i, a.rows - 1) * a.n + n0 + 4 * g;
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
     for (int z = 0; z < a.splits; ++z) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(a.ws + ((int64_t)z * a.rows + row) * a.n + n);
+        const f32x4 v = *reinterpret_cast<const f32x4*>(a.ws + (int64_t)z * a.rows * a.n + at);
 #pragma unroll
         for (int e = 0; e < 4; ++e) s[e] += v[e];
     }
-    mend(a, row, n, s);
-    *reinterpret_cast<f32x4*>(a.out + (int64_t)row * a.ld_out + n) = s;
+    mend(a, row0, n0, s);
+    if (row0 + i < a.rows) *reinterpret_cast<f32x4*>(a.out + (int64_t)(row0 + i) * a.ld_out + n0 + 4 * g) = s;
 }
 
 template <int MT>
@@ -236,13 +282,15 @@ static int launch_split_gemm(const SplitGemm& a, hipStream_t st) {
     hipLaunchKernelGGL(split_gemm_kernel<MT>, dim3((tiles + 7) / 8 * 8, a.splits), dim3(512), LDS, st, a);
     TFL_LAUNCH_CHECK();
     if (a.splits > 1) {
-        hipLaunchKernelGGL(split_sum_kernel, dim3(a.rows, (a.n + 1023) / 1024), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((int64_t)((a.rows + 15) / 16) * ((a.n + 63) / 64))), dim3(256), 0, st, a);
         TFL_LAUNCH_CHECK();
     }
     return TF_OK;
 }
 
-static int64_t split_planes(int rows, int k) { return (int64_t)((rows + 15) / 16) * (k / 32) * 1536 * 2 / 4; }      // in floats
+// In floats: x's planes, and one mark per row and part of k (16-byte pieces).
+static int64_t split_planes(int rows, int k) { return (int64_t)((rows + 15) / 16) * (k / 32) * 1536 * 2 / 4; }
+static int64_t split_marks(int rows, int k) { return ((int64_t)rows * split_parts(k) + 3) / 4 * 4; }
 
 // Parts of k: rounds of 256 workgroups, each with the fill of its pipe (4 steps of 32), against what the parts cost on their way through memory
 // (a written and read 128 x 256 part as much as 8 steps).  256 rows, 12 320 x 4 096: 267 us without parts, 159 with two, 171 with four;
@@ -261,7 +309,7 @@ static int pick_parts(int rows, int n, int k) {
 extern "C" int64_t tfl_split_gemm_ws_floats(int rows, int n, int k, int splits) {
     if (rows < 1 || rows > (1 << 24) || n < 16 || k < 32 || splits < 0 || splits > 64) return 0;
     if (splits == 0) splits = pick_parts(rows, n, k);
-    return split_planes(rows, k) + (splits > 1 ? (int64_t)splits * rows * n : 0);
+    return split_planes(rows, k) + split_marks(rows, k) + (splits > 1 ? (int64_t)splits * rows * n : 0);
 }
 
 extern "C" int tfl_split_gemm(const float* w, const float* x, int64_t ld_x, float* out, int64_t ld_out, float* ws, int64_t ws_floats, int rows, int n,
@@ -271,9 +319,9 @@ extern "C" int tfl_split_gemm(const float* w, const float* x, int64_t ld_x, floa
     if (((uintptr_t)w | (uintptr_t)x | (uintptr_t)out | (uintptr_t)ws) & 15) return TF_EINVAL;
     if (splits == 0) splits = pick_parts(rows, n, k);
     if (ws_floats < tfl_split_gemm_ws_floats(rows, n, k, splits)) return TF_ENOSPC;
-    hipLaunchKernelGGL(split_rows_kernel, dim3((rows + 15) / 16, (k + SPLIT_KC - 1) / SPLIT_KC), dim3(256), 0, (hipStream_t)stream, x, ld_x, rows, k,
-                       (bf16*)ws);
+    int32_t* nans = (int32_t*)(ws + split_planes(rows, k));
+    hipLaunchKernelGGL(split_rows_kernel, dim3((rows + 15) / 16, split_parts(k)), dim3(256), 0, (hipStream_t)stream, x, ld_x, rows, k, (bf16*)ws, nans);
     TFL_LAUNCH_CHECK();
-    const SplitGemm a = {w, (const bf16*)ws, x, out, ws + split_planes(rows, k), ld_x, ld_out, rows, n, k, splits};
+    const SplitGemm a = {w, (const bf16*)ws, x, out, ws + split_planes(rows, k) + split_marks(rows, k), nans, ld_x, ld_out, rows, n, k, splits};
     return launch_split_gemm<4>(a, (hipStream_t)stream);
 }
