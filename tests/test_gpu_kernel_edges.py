@@ -359,6 +359,31 @@ def test_split_float32_strange_rows_cost_no_walk(rows, n, k):
     x[:, k - 3] = float("nan")
     assert fastest() < 1.5 * plain
 
+def test_large_float32_products_that_something_follows():
+    """Gradients, tangents, transforms, autocast and other shapes go through the library, which takes part in them."""
+    from torch.autograd import forward_ad
+    from triforce_amd import ops_tile as ot
+    F = torch.nn.functional
+    g = torch.Generator(device=DEV).manual_seed(4)
+    w, x = torch.randn(4096, 4096, generator=g, device=DEV), torch.randn(256, 4096, generator=g, device=DEV)
+    wt = ot.TileWeight(w)
+    assert torch.equal(wt.matmul(x), ot.split_linear(x, w))                    # (nothing follows: the kernel)
+    assert wt.matmul(x.view(256, 1, 4096)).shape == (256, 1, 4096)
+    y = wt.matmul(x.clone().requires_grad_())
+    assert y.requires_grad and torch.equal(y, F.linear(x, w))
+    with torch.no_grad():
+        assert torch.equal(wt.matmul(x.clone().requires_grad_()), ot.split_linear(x, w))
+    with forward_ad.dual_level():
+        t = forward_ad.unpack_dual(wt.matmul(forward_ad.make_dual(x, torch.ones_like(x)))).tangent
+    assert torch.equal(t, F.linear(torch.ones_like(x), w))
+    both = torch.func.vmap(wt.matmul)(torch.stack([x, 2 * x]))
+    assert both.shape == (2, 256, 4096) and torch.allclose(both[0], F.linear(x, w), rtol=1e-4, atol=1e-3)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert wt.matmul(x).dtype == torch.bfloat16
+    with pytest.raises(RuntimeError):
+        ot.linear_rows(x[:, :4064], w)
+
+
 
 def _flash_want(q, k, v, lo, hi, scale):
     """float64 attention of q [n, d] with keys lo .. hi of every row: (result, the same sums with |v|)."""

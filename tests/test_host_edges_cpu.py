@@ -394,3 +394,18 @@ def test_topp_candidate_cut_always_contains_the_crossing():
                 tau = int(np.floor(np.float64(np.float32(top_p)) * np.float64(Z)))
                 cand = (m != 0) & (e.view(np.uint32) >= cutpat)
                 assert int(m[cand].sum()) > tau, (V, top_p, int(m[cand].sum()), tau)
+
+
+def test_large_float32_products_stay_the_librarys_off_the_device():
+    """ops_tile.linear_rows: the kernel for many rows takes plain device tensors only."""
+    import torch
+    from triforce_amd import ops_tile as ot
+    g = torch.Generator().manual_seed(3)
+    w = torch.randn(2048, 2048, generator=g)
+    x = torch.randn(1024, 2048, generator=g)
+    assert x.numel() * w.shape[0] >= 1 << 32
+    want = torch.nn.functional.linear(x, w)
+    assert torch.equal(ot.linear_rows(x, w), want)
+    assert torch.equal(ot.TileWeight(w).matmul(x), want)
+    assert ot.linear_rows(x.view(512, 2, 2048), w).shape == (512, 2, 2048)
+    assert ot.linear_rows(x.to("meta"), w.to("meta")).shape == (1024, 2048)

@@ -8,6 +8,7 @@ import ctypes
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import hip
 
@@ -154,10 +155,20 @@ def linear_rows(x, w):
     70 -> 63, 700 x 22 016 x 4 096 940 -> 750), below that it leaves CUs idle (300 x 6 144 x 1 536 51 -> 55, 64 x 22 016 x 4 096
     115 -> 133).  Up to k = 65 536 its error is a tenth to a half of the library's; at 2^20, with as few parts, the two are equal."""
     rows, (n, k) = x.shape[0], w.shape
-    if x.dtype == torch.float32 and 256 <= rows <= 1 << 24 and rows * n * k >= 1 << 32 and n % 16 == 0 and k % 32 == 0 and k <= 1 << 16 \
+    if x.dtype == w.dtype == torch.float32 and x.dim() == 2 and x.shape[1] == k and 256 <= rows <= 1 << 24 and rows * n * k >= 1 << 32 \
+            and n % 16 == 0 and k % 32 == 0 and k <= 1 << 16 and x.device == w.device and _unwatched(x, w) and w.is_contiguous() \
             and w.data_ptr() % 16 == 0:
         return split_linear(x, w)
     return F.linear(x, w)
+
+
+def _unwatched(*ts):
+    """Device tensors that no derivative, transform, trace or autocast follows: a launch behind torch's back would be lost on them."""
+    if torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() \
+            or torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    return all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) and not (t.requires_grad and torch.is_grad_enabled())
+               and forward_ad.unpack_dual(t).tangent is None for t in ts)
 
 
 def split_linear(x, w, splits=0):
