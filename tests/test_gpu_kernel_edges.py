@@ -142,6 +142,68 @@ def test_wide_gemm_shares(panels, rows, k):
         _near(ot.act_rows(act), tail, size[:, n_raw:] * 1.13, k + 16, out_bits=8)
 
 
+# what the packing rule says is what the kernel does: the two forms sum in different orders, so the layout's own form is the one whose
+# bits a weight that was packed by the rule has; and both forms read either layout
+@pytest.mark.parametrize("panels,raw", [(255, 0), (256, 0), (257, 16), (257, 4112), (330, 4096), (330, 4112), (452, 7232), (2047, 0), (2048, 0), (2049, 0), (2300, 64)])
+def test_weight_layout_follows_the_kernel(panels, raw):
+    from triforce_amd import ops_latent as ol, ops_tile as ot
+    g = torch.Generator(device=DEV).manual_seed(panels)
+    n, k, rows = 16 * panels, 2048, 3
+    w, h = _bf(g, n, k, std=k ** -0.5), _bf(g, k // 8, rows, 8)
+    x = ot.act_rows(h)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    rule, other = ot.TileWeight(w, packed_only=True, raw=raw), ot.TileWeight(w, packed_only=True, raw=raw)
+    other.chunk_major = not rule.chunk_major
+    other.packed = ot.pack_tiles(w, True) if other.chunk_major else ot.pack_tiles(w.unsqueeze(0))
+    q_norm = torch.ones(16, device=DEV)
+
+    def outputs(wt):
+        if raw:
+            act = ot.empty_act(rows, max(n - raw, 16), torch.bfloat16, DEV)
+            return ol.input_projection(h, wt, raw, q_norm, act, 0)[0]
+        return ot.linear_f32(h, wt, n)
+    a, b = outputs(rule), outputs(other)
+    for got in (a, b):
+        _near(got, want[:, :got.shape[1]], size[:, :got.shape[1]], k)
+    assert rule.chunk_major == ot.shares_panels(n, k, raw) == (not torch.equal(a, b))          # (same bits: the same form on both layouts)
+    if not raw:                                                  # the other epilogues of more panels than the form takes
+        wt = rule if rule.chunk_major else other
+        res = torch.randn(rows, n, generator=g, device=DEV)
+        got = res.clone()
+        ol.add_linear(h, wt, got)
+        _near(got, want + res.double(), size + res.double().abs(), k + 1)
+        v, s = (t.view(rows, panels, 2, 8) for t in (want, size))
+        glu = torch.nn.functional.gelu(v[:, :, 0], approximate="tanh") * v[:, :, 1]
+        bound = (1.13 * s[:, :, 0] * v[:, :, 1].abs() + s[:, :, 1] * v[:, :, 0].abs()) * (k + 16) * 2.0 ** -24 + glu.abs() * 2.0 ** -8 + 1e-6
+        assert ((ot.act_rows(ot.gelu_glu_linear(h, wt)).double() - glu.reshape(rows, -1)).abs() <= bound.reshape(rows, -1)).all()
+
+
+# weights of products without the one-workgroup-per-CU form: panel by panel, whatever their size; chunk-major ones give the same bits
+def test_query_and_token_weights_in_both_layouts():
+    from types import SimpleNamespace as NS
+    from triforce_amd import ops_latent as ol, ops_tile as ot
+    g = torch.Generator(device=DEV).manual_seed(6)
+    geom, rows = NS(H=32, N=128, R=64, C=64, Q=2048, q_real=2048, c_real=64, row=128), 5
+    raw = torch.randn(rows, 2048 + 128, generator=g, device=DEV)
+    ss = raw.view(rows, -1, 16).square().sum(-1).contiguous()
+    angle = torch.rand(50, 32, generator=g, device=DEV)
+    rope = NS(cos=angle.cos().contiguous(), sin=angle.sin().contiguous(), half=32, max_pos=50)
+    at = torch.arange(rows, dtype=torch.int32, device=DEV)
+    wq, wg, h = _bf(g, 32 * 192, 2048), _bf(g, 4096, 2048), _bf(g, 256, rows, 8)
+    table, ids = _bf(g, 9, 4096), torch.arange(rows, device=DEV)
+    out = []
+    for chunk_major in (False, True):
+        a, b = ot.TileWeight(wq, per_panel=True), ot.TileWeight(wg, per_panel=True)
+        assert not a.chunk_major and not b.chunk_major and ot.TileWeight(wg).chunk_major
+        if chunk_major:
+            for t, w in ((a, wq), (b, wg)):
+                t.packed, t.chunk_major = ot.pack_tiles(w, True), True
+        cache = torch.zeros(128, 128, dtype=torch.bfloat16, device=DEV)
+        qn, q = ol.query_and_append(h, raw, ss, a, geom, torch.ones(64, device=DEV), 1e-5, rope, at, at, cache)
+        out.append((qn, q[..., 64:], cache, ol.token_gate_linear(h, b, table, ids, 4096)))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
 @pytest.mark.parametrize("n", [1, 64, 65, 200])
 def test_set_pages(n):
     from triforce_amd import hip, ops_tile as ot

@@ -45,10 +45,10 @@ class LatentLayer:
                  _grow(mat("mix.g").view(g.H, m.vdim, width), g.H, g.V, W).reshape(g.H * g.V, W)]
         if F:
             parts.append(_grow(mat("mlp.up"), F, W))
-        self.w_in = ol.TileWeight(torch.cat(parts))
+        self.w_in = ol.TileWeight(torch.cat(parts), raw=g.n_raw)
         uq = mat("mix.uq").view(g.H, m.dim + m.rot_dim, m.q_rank)
         self.w_uq = ol.TileWeight(torch.cat([_grow(uq[:, :m.dim], g.H, g.N, g.Q), _grow(uq[:, m.dim:], g.H, g.R, g.Q)], 1)
-                                  .reshape(g.H * (g.N + g.R), g.Q))
+                                  .reshape(g.H * (g.N + g.R), g.Q), per_panel=True)
         uk = _grow(mat("mix.uk").view(g.H, m.dim, m.kv_rank), g.H, g.N, g.C)
         uv = _grow(mat("mix.uv").view(g.H, m.vdim, m.kv_rank), g.H, g.V, g.C)
         self.w_uk_t = ol.TileWeight(uk.transpose(1, 2).contiguous(), packed_only=True)          # decode: query -> latent
@@ -60,7 +60,7 @@ class LatentLayer:
         self.w_out = ol.TileWeight(torch.cat(out, 1))
         self.norm1, self.q_norm, self.kv_norm = vec("norm1", W), vec("mix.dq.norm", g.Q), vec("mix.dkv.norm", g.C)
         if D:
-            self.side_gate = ol.TileWeight(_grow(mat("side.gate"), D, W))
+            self.side_gate = ol.TileWeight(_grow(mat("side.gate"), D, W), per_panel=True)
             self.side_proj = ol.TileWeight(_grow(mat("side.proj"), W, D))
             self.side_norm = vec("side.norm", W)
 

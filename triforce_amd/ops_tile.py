@@ -64,16 +64,27 @@ def pack_tiles(w, chunk_major=False):
     return w.reshape(*lead, n // 16, 16, k // 32, 4, 8).permute(*range(d), *order, d + 3, d + 1, d + 4).contiguous()
 
 
+def shares_panels(n, k, raw=0):
+    """Does the one-workgroup-per-CU form of the skinny kernel (share_gemm in csrc/tile_gemm.hip) take n outputs in bfloat16, the first
+    ``raw`` of them with sums of squares?  A panel or more per CU and at most eight; left-over panels are dealt in fours of rows, where
+    sums of squares need whole ones.  k from 2 048 on: a shorter one is over before the form's look-ahead pays (4 096 x 256 at 32
+    rows 4.6 us with a workgroup per panel, 6.4 with one per CU; 6 144 x 1 536 10.0 and 11.1)."""
+    panels = n // 16
+    whole, left = panels // 256, panels % 256
+    return k >= 2048 and 256 <= panels <= 2048 and (left == 0 or left > 192 or 256 * whole * 16 >= raw)
+
+
 class TileWeight:
     """A (groups of) [n, k] weight(s): packed for the skinny kernel and, unless ``packed_only``, row-major for the library GEMM
-    of the prefill.  Wide and long bfloat16 weights (a panel or more per CU, k from 2 048 on) are packed chunk-major, which the
-    one-workgroup-per-CU form of the kernel streams; a shorter k is over before its look-ahead pays (4 096 x 256 at 32 rows 4.6 us with
-    a workgroup per panel, 6.4 with one per CU; 6 144 x 1 536 10.0 and 11.1)."""
+    of the prefill.  Weights of the one-workgroup-per-CU form are packed chunk-major, the layout it streams; the workgroup-per-panel form
+    reads that one too, but up to 10 % slower (128 256 x 4 096 at 8 rows 171 -> 181 us, a projection of 17 216 with 16 480 raw 27.4 -> 30.1
+    at one row), so its weights stay panel by panel.  ``raw``: outputs of an input projection that come with sums of squares; ``per_panel``:
+    the weight of a product that only the workgroup-per-panel form has (query, token gate)."""
 
-    def __init__(self, w, packed_only=False):
+    def __init__(self, w, packed_only=False, raw=0, per_panel=False):
         w3 = w if w.dim() == 3 else w.unsqueeze(0)
         self.groups, self.n, self.k = w3.shape
-        self.chunk_major = self.groups == 1 and w.dtype == torch.bfloat16 and self.n >= 256 * 16 and self.k >= 2048
+        self.chunk_major = self.groups == 1 and w.dtype == torch.bfloat16 and not per_panel and shares_panels(self.n, self.k, raw)
         self.packed = pack_tiles(w3, self.chunk_major)
         self.w = None if packed_only else w.contiguous()
         self.dtype, self.device = w.dtype, w.device
