@@ -142,3 +142,17 @@ _Zk: ; @_Zk
     shapes = isa_lint.undrained_dma(isa_lint.compile_to_asm(os.path.join(CSRC, "split_gemm.hip"), extra=extra))
     kernels = {k: v for k, v in shapes.items() if "split_gemm_kernel" in k}
     assert kernels and all(v["dma"] >= 6 and v["undrained_barriers"] == 0 for v in kernels.values()), shapes
+
+
+def test_every_prefill_attention_kernel_takes_the_split_of_its_weights():
+    """TF_BLOCK_P_SPLIT=1 feeds a second half of every weight to the value product: each prefill kernel then has more products."""
+    import re
+
+    def products(defines):
+        text = isa_lint.compile_to_asm(os.path.join(CSRC, "attn.hip"), defines)
+        assert isa_lint.lint_asm(text) == []
+        bodies = re.findall(r"^(_Z\w*attn_prefill_kernel\w+):\s*;\s*@\1\n([\s\S]*?)\n\.Lfunc_end\d+:", text, re.M)
+        return {name: len(re.findall(r"^\s+v_mfma_", body, re.M)) for name, body in bodies}
+    plain, split = products(()), products(("TF_BLOCK_P_SPLIT=1",))
+    assert len(plain) == 2 and plain.keys() == split.keys()
+    assert all(split[k] > 1.3 * plain[k] for k in plain), (plain, split)

@@ -134,9 +134,9 @@ __device__ __forceinline__ float group_max4(float v) {
 #ifndef TF_ATTN_P_SPLIT
 #define TF_ATTN_P_SPLIT 1
 #endif
-// The same hi + lo feed in the block / prefill / tree kernels (pair_softmax_pv, lds_softmax_*) and in the 68M draft's
-// rope-on-read kernel: TF_BLOCK_P_SPLIT / TF_DRAFT_P_SPLIT.  Measured in round 4 (tools/prefill_psplit_ab.py,
-// profiles/r04_psplit_block_ab.jsonl) — see the note there for what ships and why.
+// The same hi + lo feed in the block / prefill / tree kernels (pair_softmax_pv, lds_softmax_*, pv of the D = 128 prefill) and in
+// the 68M draft's rope-on-read kernel: TF_BLOCK_P_SPLIT / TF_DRAFT_P_SPLIT.  What ships and why: tools/prefill_psplit_ab.py,
+// profiles/r04_psplit_block_ab.jsonl.  (512 rows behind 7 680 keys, 8 heads of 128: outputs not correctly rounded 39.6 % at 0, 0.2 % at 1.)
 #ifndef TF_BLOCK_P_SPLIT
 #define TF_BLOCK_P_SPLIT 0
 #endif
@@ -1496,7 +1496,7 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
     int v_at = (8 * g + (li >> 2)) * D + 4 * (li & 3) + 16 * ((li >> 2) | ((g & 1) << 2));
     // Fragments are requested a fixed distance ahead of their products, step by step: left to itself the scheduler moves all 16 (32)
     // reads of a product to its front and spills a hundred registers.
-    auto pv = [&](const half8 (&pa)[QT], const half8 (&pb)[QT], int at) {
+    auto pv = [&](const half8 (&pa)[QT], const half8 (&pb)[QT], const half8 (&la)[QT], const half8 (&lb)[QT], int at) {
         constexpr int STEPS = 2 * NT, AHEAD = 8;
         half4 lo[AHEAD + 1], hi[AHEAD + 1];
         auto read = [&](int n) {
@@ -1513,8 +1513,12 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
             const half4 l = lo[n % (AHEAD + 1)], h = hi[n % (AHEAD + 1)];
             const half8 vt = half8{l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]};
 #pragma unroll
-            for (int qt = 0; qt < QT; ++qt)
+            for (int qt = 0; qt < QT; ++qt) {
                 st.acc[qt][n % NT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt, n < NT ? pa[qt] : pb[qt], st.acc[qt][n % NT], 0, 0, 0);
+#if TF_BLOCK_P_SPLIT > 0
+                st.acc[qt][n % NT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt, n < NT ? la[qt] : lb[qt], st.acc[qt][n % NT], 0, 0, 0);
+#endif
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -1603,7 +1607,7 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
             }
             // The next slab's QK^T (past the end: finite garbage, never used) with this slab's exponentials beside it: four scores of
             // a lane per four products, so that the matrix core works while the wave issues VALU operations
-            half8 p0[QT], p1[QT];
+            half8 p0[QT], p1[QT], l0[QT], l1[QT];            // (l0, l1: TF_BLOCK_P_SPLIT's remainders)
             float psum[QT] = {};
             qk_slab(k_next, n0a, n0b, n1a, n1b, [&](int n) {
                 const int qt = n / 4, quad = n % 4;
@@ -1614,9 +1618,12 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
                     const float e = __builtin_amdgcn_exp2f(fmaf(x[r], scale_log2, -mnew[qt]));
                     psum[qt] += e;
                     dst[4 * (quad & 1) + r] = (h16)e;
+#if TF_BLOCK_P_SPLIT > 0
+                    (quad < 2 ? l0[qt] : l1[qt])[4 * (quad & 1) + r] = (h16)(e - (float)(h16)e);
+#endif
                 }
             });
-            pv(p0, p1, v_at + (i & 1) * BlkLayout<D>::V_HALFS);
+            pv(p0, p1, l0, l1, v_at + (i & 1) * BlkLayout<D>::V_HALFS);
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) st.l[qt] += psum[qt];
 #pragma unroll
