@@ -301,6 +301,27 @@ def test_step_splits_over_rows(rows, nsplit, D):
             assert not got[b].any()
         # the same fp32 sums in another order, then one rounding to bfloat16 each
         assert ((got[b] - alone).abs() <= 2.0 ** -7 * alone.abs() + 1e-5).all()
+        if lens[b] == 0:
+            continue
+        # and against plain attention: the new token's key and value behind the row's pages, its chunk alone
+        n, at = lens[b], (lens[b] - 1) // chunk * chunk
+        own = torch.randperm(pages, generator=torch.Generator().manual_seed(b))[:22]
+        old = pool.view(pages, 64, -1)[own.to(DEV)].reshape(-1, G * 2 * D)[at:n - 1]
+
+        def turned(x):                                           # norm, then pairs (e, e + 8) by the position's angle
+            x = x / torch.sqrt(x.square().mean(-1, keepdim=True) + 1e-5)
+            c, s = angle[n - 1].cos(), angle[n - 1].sin()
+            return torch.cat([x[:, :8] * c - x[:, 8:16] * s, x[:, 8:16] * c + x[:, :8] * s, x[:, 16:]], 1).bfloat16().double()
+        q, k = turned(raw[b, :H * D].view(H, D)), turned(raw[b, H * D:H * D + G * D].view(G, D))
+        v = raw[b, H * D + G * D:H * D + 2 * G * D].view(G, D).bfloat16().double()
+        keys = torch.cat([old[:, :G * D].double().view(-1, G, D), k[None]])
+        vals = torch.cat([old[:, G * D:].double().view(-1, G, D), v[None]])
+        gate = torch.sigmoid(raw[b, H * D + 2 * G * D:].double()).view(H, D)
+        for h in range(H):
+            w = torch.softmax(keys[:, h // (H // G)] @ q[h] * 0.1, 0)
+            want, size = gate[h] * (w @ vals[:, h // (H // G)]), gate[h] * (w @ vals[:, h // (H // G)].abs())
+            # the result's rounding to bfloat16; an entry of q or k that rounds the other way moves a score by 2^-8 * 4 * 4 * 0.1 at most
+            assert ((got[b, h * D:h * D + D] - want).abs() <= 2.0 ** -8 * want.abs() + (2.0 ** -15 + 0.00625) * size + 1e-6).all()
 
 
 # float32 on the bfloat16 matrix cores: below and above a tile of 256 x 128, waves without rows, parts of k of unequal length and empty ones
