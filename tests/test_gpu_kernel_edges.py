@@ -79,6 +79,18 @@ def test_prefill_attention_blocks_and_splits(n, past, H, token_major, rising):
     assert ((got - want).abs() <= bound).all()
 
 
+# every key alike, rows that do not see all of their last slab: a hidden score of minus infinity times 0 is no number
+@pytest.mark.parametrize("n,past,H", [(130, 0, 8), (200, 2000, 8), (2049, 0, 32)])
+def test_prefill_attention_scale_of_zero(n, past, H):
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n)
+    k, v = (torch.randn(H, past + n, 128, generator=g, device=DEV, dtype=torch.float16) for _ in range(2))
+    q = torch.randn(n, H, 128, generator=g, device=DEV, dtype=torch.float16)
+    got = ops.attn_prefill(q, k, v, past + n, 0.0).view(n, H, 128).double()
+    want, size = _attention64(q, k, v, 0.0)
+    assert ((got - want).abs() <= 2.0 ** -10 * size + 2.0 ** -11 * want.abs() + 1e-6).all()
+
+
 def test_prefill_attention_rows_far_apart():
     """Cache rows 2^25 elements apart: past the 32-bit offsets of a slab, so the chunk goes block by block."""
     from triforce_amd import ops

@@ -2269,7 +2269,9 @@ extern "C" int tf_attn_prefill(const void* q, const void* k, const void* v, void
     if ((stride_t % 8) || (stride_h % 8)) return TF_EINVAL;
     if (ws_floats < tf_attn_prefill_ws_floats(H, sq, D, nsplit)) return TF_ENOSPC;
     hipStream_t st = (hipStream_t)stream;
-    if (D == 128 && (stride_t < 0 || stride_t >= (1 << 25))) {   // rows 64 MB apart: the kernel's 32-bit slab offsets do not reach
+    // Block by block: rows 64 MB apart, which the kernel's 32-bit slab offsets do not reach, and a scale that is not positive (its masks are
+    // scores of minus infinity in front of the scale: times 0 they are no numbers)
+    if (D == 128 && (stride_t < 0 || stride_t >= (1 << 25) || !(scale > 0.f))) {
         for (int r0 = 0; r0 < sq; r0 += 128) {
             const int rows = sq - r0 < 128 ? sq - r0 : 128;
             const int rc = tf_attn_block((const h16*)q + (int64_t)r0 * H * D, k, v, (h16*)out + (int64_t)r0 * H * D, stride_t, stride_h, rows,
