@@ -160,6 +160,17 @@ class _Model:
         return 64
 
 
+def test_step_splits_by_rows():
+    """Splits per row of the decode step: one workgroup per CU for a row alone (two cost 5 to 12 %), two for more, above 16 splits in whole
+    sixteens; more than 64 rows, which share nothing, take three (four cost 5 % at 128 rows of 1 000 keys)."""
+    from triforce_amd import hip
+    L = hip.hybrid_lib()
+    pick = [L.tfh_attn_step_pick_nsplit(rows, 32, 8, 8256) for rows in (1, 2, 3, 4, 5, 8, 12, 16, 64, 65, 128, 1000)]
+    assert pick == [32, 32, 16, 16, 12, 8, 5, 4, 4, 3, 3, 3]
+    assert [L.tfh_attn_step_pick_nsplit(1, 16, g, 100000) for g in (1, 2, 4)] == [256, 128, 64]
+    assert [L.tfh_attn_step_pick_nsplit(2, 32, 8, n) for n in (64, 65, 700)] == [1, 2, 11]
+
+
 def test_cache_pages_and_seats():
     c = HybridCache(_Model(), max_budget=200, max_batch=3)
     assert [None if r is None else tuple(r.shape) for r in c.rows] == [(384, 64), None, (384, 96)]

@@ -673,13 +673,17 @@ extern "C" int64_t tfh_attn_step_ws_floats(int rows, int H, int V, int nsplit) {
     return (int64_t)rows * H * nsplit * (V + 2) + 2 * (int64_t)rows;
 }
 
-// Two workgroups per CU (512), four splits a row where the batch is large (unequal rows are dealt by splits), as long as a split
-// keeps a page of keys.  us with the merge: 8 rows of 9 000 - 5 063 at 4 / 8 / 12 splits 58.4 / 55.5 / 56.2, 16 rows around 3 000 at 2 / 4 /
-// 8 92.8 / 68.8 / 72.4, 32 rows 141.7 / 123.8 / 126.4, one row of 8 192 at 16 / 32 / 64 / 128 22.4 / 20.2 / 20.9 / 26.4.
+// Two workgroups per CU (512) - one (256) for a row alone -, above 16 splits a row in whole sixteens, as long as a split keeps a page of keys; at
+// least four splits a row up to 64 rows, whose unequal lengths are dealt by splits, and three where they are not.  us with the merge,
+// recurrences beside it, caches from memory: one row of 300 / 3 000 / 8 000 keys at 32 splits 13.6 / 15.1 / 15.8, at 64 14.6 / 16.9 / 17.9; three
+// of 1 000 at 16 / 21 16.9 / 20.0; 16 rows of 3 000 at 4 / 8 / 16 65.9 / 66.6 / 74.1; 128 rows of 1 000 at 1 / 2 / 3 / 4 / 8 240 / 245 / 243 / 258 /
+// 277, of 3 000 426 / 431 / 431 / 429 / 446, 65 rows of up to 8 000 325 / 264 / 252 / 246 / 254.
 extern "C" int tfh_attn_step_pick_nsplit(int rows, int H, int G, int max_keys) {
     if (rows < 1 || H < 1 || G < 1 || max_keys < 1) return 1;
-    const int groups = G * ((H / G + 15) / 16);
-    int n = 512 / (rows * groups) > 4 ? 512 / (rows * groups) : 4;
+    const int groups = G * ((H / G + 15) / 16), least = rows <= 64 ? 4 : 3;
+    int n = (rows == 1 ? 256 : 512) / (rows * groups);
+    if (n > 16) n &= ~15;
+    if (n < least) n = least;
     const int cap = (max_keys + TFL_PAGE - 1) / TFL_PAGE;
     if (n > cap) n = cap;
     if (n > TFH_MAX_SPLIT) n = TFH_MAX_SPLIT;
