@@ -216,6 +216,32 @@ def test_query_and_token_weights_in_both_layouts():
     assert all(torch.equal(a, b) for a, b in zip(*out))
 
 
+# seven panels per CU in two row blocks, whole and with rows left over: right, and no slower than the wider eight-panel form
+def test_wide_gemm_of_seven_panels():
+    from triforce_amd import ops_tile as ot
+    g = torch.Generator(device=DEV).manual_seed(7)
+    k, rows, spans = 4096, 33, {}
+    for panels in (1700, 1792, 1900):
+        h, ws, out = _bf(g, k // 8, rows - 1, 8), [], torch.empty(rows - 1, 16 * panels, device=DEV)
+        for _ in range(2):                                       # (470 MB: from memory each time)
+            w = _bf(g, 16 * panels, k, std=k ** -0.5)
+            ws.append(ot.TileWeight(w, packed_only=True))
+        assert ws[0].chunk_major
+        h33 = _bf(g, k // 8, rows, 8)
+        x = ot.act_rows(h33)
+        _near(ot.linear_f32(h33, ws[1], 16 * panels), x.double() @ w.double().T, x.double().abs() @ w.double().abs().T, k)
+        spans[panels] = []
+        for i in range(12):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for j in range(4):
+                ot.linear_f32(h, ws[j % 2], 16 * panels, out)
+            b.record()
+            b.synchronize()
+            spans[panels].append(a.elapsed_time(b))
+    assert min(spans[1700]) < min(spans[1900]) and min(spans[1792]) < min(spans[1900]), spans
+
+
 @pytest.mark.parametrize("n", [1, 64, 65, 200])
 def test_set_pages(n):
     from triforce_amd import hip, ops_tile as ot

@@ -393,7 +393,9 @@ __global__ __launch_bounds__(512, 2) void share_gemm_kernel(const TflGemm a, con
 template <typename T, int EPI, int P, bool TAIL, int MT>
 static int launch_share_rows(const TflGemm& a, int tail_rows, int tail_per, hipStream_t st) {
     constexpr int NP = P + (TAIL ? 1 : 0), LDS = 8 * NP * MT * 64 * (int)sizeof(f32x4);
-    constexpr int U = NP == 1 ? 4 : NP * MT <= 12 ? 2 : 1;           // (measured: 1, 2 and 4 for every form)
+    // Chunks asked for ahead: what the registers hold (seven panels and two row blocks 221; with one chunk ahead 1 792 panels of 4 096 took 51.8
+    // us at 32 rows, more than 2 048 do, and 41.1 with two; eight panels and two row blocks would spill).
+    constexpr int U = NP == 1 ? 4 : NP * MT <= 14 ? 2 : 1;
     static_assert(LDS <= 160 * 1024, "one workgroup's partial tiles");
     if (LDS > 64 * 1024) {
         const hipError_t e = hipFuncSetAttribute((const void*)share_gemm_kernel<T, EPI, P, TAIL, MT, U>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
