@@ -60,7 +60,9 @@ __global__ __launch_bounds__(256) void finish_kernel(const T* __restrict__ embed
 // The same for rows that fit a workgroup's registers (HOLD quads per thread of NW waves): everything is asked for at once and nothing
 // is read twice, where the form above makes three passes whose loads wait for each other.  A decode row is a latency chain:
 // sixteen waves with one quad a thread; a prompt's rows are a stream: four waves with four.  Rows of 4 096: 1 row 5.1 ->
-// 3.9 us, 32 rows 5.4 -> 4.1, 4 000 rows 40.6 -> 33.4 (5.9 TB/s).
+// 3.9 us, 32 rows 5.4 -> 4.1, 4 000 rows 40.6 -> 33.4 (5.9 TB/s).  Narrow rows take no more waves than they have quads (4 000 rows of 192 with four
+// times four 8.6 us, with one wave 4.3, in the form above 6.7); 4 000 rows of 1 025 to 2 048, which leave half the four quads empty, are
+// faster above (2 048 16.5 us and 18.6).
 template <typename T, typename Y, int NW, int HOLD>
 __global__ __launch_bounds__(64 * NW) void finish_row_kernel(const T* __restrict__ embed, const int64_t* __restrict__ ids, int vocab,
                                                              const Y* __restrict__ y, int64_t ld_y, const float* __restrict__ y_w,
@@ -136,7 +138,9 @@ extern "C" int tfl_finish(const void* embed, const int64_t* ids, int vocab, cons
 #define ARGS(T, Y) 0, st, (const T*)embed, ids, vocab, (const Y*)y, ld_y, y_w, step, norm_w, x, (T*)h, ld_h, h_oct, width, width_real, eps
 #define GO(T, Y)                                                                                                                              \
     do {                                                                                                                                      \
-        if (width > 4096) hipLaunchKernelGGL((finish_kernel<T, Y>), dim3(rows), dim3(256), ARGS(T, Y));                                       \
+        if (width > 4096 || (width > 1024 && width <= 2048 && rows > 1024)) hipLaunchKernelGGL((finish_kernel<T, Y>), dim3(rows), dim3(256), ARGS(T, Y)); \
+        else if (width <= 256) hipLaunchKernelGGL((finish_row_kernel<T, Y, 1, 1>), dim3(rows), dim3(64), ARGS(T, Y));                          \
+        else if (width <= 1024) hipLaunchKernelGGL((finish_row_kernel<T, Y, 4, 1>), dim3(rows), dim3(256), ARGS(T, Y));                        \
         else if (rows <= 256) hipLaunchKernelGGL((finish_row_kernel<T, Y, 16, 1>), dim3(rows), dim3(1024), ARGS(T, Y));  /* a row per CU */    \
         else hipLaunchKernelGGL((finish_row_kernel<T, Y, 4, 4>), dim3(rows), dim3(256), ARGS(T, Y));                                          \
     } while (0)
