@@ -56,8 +56,10 @@ int tfl_attn_prefill(const void* q, const void* kv, const void* ck, const int32_
 
 /* One query token per sequence over the paged latent cache: q [rows][H][C + R] (keys are the cached rows themselves, values
  * their first C entries), len[row] keys (<= 0: output 0), page table [rows][table_ld].  out [rows][H][C] (T).
- * ws: tfl_attn_decode_ws_floats floats when nsplit > 1. */
+ * ws: tfl_attn_decode_ws_floats floats when nsplit > 1.  tfl_attn_decode_splits: the nsplit to take for rows of up to max_len keys
+ * (tfl_attn_decode_pick_nsplit: for bfloat16 rows of 512 + 64). */
 int64_t tfl_attn_decode_ws_floats(int rows, int H, int C, int nsplit);
+int tfl_attn_decode_splits(int rows, int H, int C, int R, int max_len, int dtype);
 int tfl_attn_decode_pick_nsplit(int rows, int H, int max_len);
 int tfl_attn_decode(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len,
                     void* out, float* ws, int64_t ws_floats, int rows, int H, int C, int R, float scale, int nsplit, int dtype,

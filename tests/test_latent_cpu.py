@@ -67,6 +67,26 @@ def test_bad_arguments_are_refused_before_any_launch():
                 assert 1 <= s <= 256 and (s == 1 or s <= math.ceil(n / 128))
 
 
+def test_decode_splits_by_form():
+    """Two pages: one split where the merge costs more than the second page; float32 (one workgroup of 16 heads per CU): single pages only
+    where they are no more rounds of 256 workgroups than pairs."""
+    from triforce_amd import hip
+    _, L = hip.tile_lib(), hip.latent_lib()
+    splits = L.tfl_attn_decode_splits
+    for rows in (1, 7, 64, 128):
+        for heads in (1, 16, 33, 128):
+            assert [splits(rows, heads, 512, 64, n, 0) for n in (1, 64, 65, 128)] == [1, 1, 1, 1]
+            for n in (129, 1024, 1025, 40000):
+                assert splits(rows, heads, 512, 64, n, 0) == L.tfl_attn_decode_pick_nsplit(rows, heads, n) == max(1, min(
+                    256 // (rows * (-(-heads // 32))), -(-n // 64) if n <= 1024 else -(-n // 128), 256))
+    assert [splits(rows, 16, 256, 32, 128, 0) for rows in (1, 64, 65, 128)] == [2, 2, 1, 1]
+    assert [splits(rows, 32, 256, 32, 128, 0) for rows in (1, 32, 33)] == [2, 2, 1]
+    assert [splits(rows, 16, 512, 64, 128, 1) for rows in (1, 128, 129)] == [2, 2, 1]
+    assert [splits(rows, 32, 512, 64, 768, 1) for rows in (10, 11, 12, 21, 22)] == [12, 6, 6, 6, 11]
+    assert splits(0, 16, 512, 64, 128, 0) == splits(1, 0, 512, 64, 128, 0) == splits(1, 16, 512, 64, 0, 0) == 1
+    assert splits(1 << 30, 1 << 20, 512, 64, 1 << 30, 1) == 1
+
+
 # ---- configuration and registry -------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("name", sorted(H.CONFIGS))
 def test_config_round_trip_and_layer_order(name):

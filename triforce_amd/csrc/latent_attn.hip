@@ -488,16 +488,25 @@ extern "C" int64_t tfl_attn_decode_ws_floats(int rows, int H, int C, int nsplit)
 
 // One workgroup per CU (256) as long as a split keeps at least two pages of keys, or one of up to 16: there the second page costs more
 // (2.4 us) than its partial rows (one row, attention and merge: 500 keys 16.7 -> 14.3 us, 1 000 16.8 -> 14.6; 4 000 keys 18.2 either way, two rows of
-// 4 000 19.7 against 20.7).
-extern "C" int tfl_attn_decode_pick_nsplit(int rows, int H, int max_len) {
+// 4 000 19.7 against 20.7).  Two pages are one split where the second one costs less than the merge: always in the form of known sizes (32 heads,
+// one row 12.7 us against 14.1, 64 rows 13.6 against 19.7), in the other bfloat16 forms from 65 workgroups of 16 heads on (256 | 32, 16 heads, 96 rows
+// 11.5 against 12.4; 32 rows 11.5 against 10.6), never in float32 (55 against 35).  Float32 takes 16 heads per workgroup, one to a CU: single pages
+// only where they are no more rounds of 256 than pairs would be (32 heads, 12 rows of 12 pages 86.5 us against 92.8).
+extern "C" int tfl_attn_decode_splits(int rows, int H, int C, int R, int max_len, int dtype) {
     if (rows < 1 || H < 1 || max_len < 1) return 1;
-    const int groups = H <= 16 ? 1 : (H + 31) / 32;
-    int n = 256 / (rows * groups);
-    const int pages = (max_len + TFL_PAGE - 1) / TFL_PAGE, cap = pages <= 16 ? pages : (pages + 1) / 2;
-    if (n > cap) n = cap;
+    const int groups = H <= 16 ? 1 : (H + 31) / 32, pages = (max_len + TFL_PAGE - 1) / TFL_PAGE, pairs = (pages + 1) / 2;
+    const int64_t tiles = (int64_t)rows * ((H + 15) / 16);
+    const int room = (int)(256 / ((int64_t)rows * groups));
+    int n = pages < room ? pages : room;
+    const bool twice = dtype == 1 && tiles * n > 256 && tiles * pairs <= 256;
+    const bool merge = pages == 2 && dtype == 0 && ((C == 512 && R == 64) || tiles > 64);
+    if ((pages > 16 || twice || merge) && n > pairs) n = pairs;
     if (n > TFL_MAX_SPLIT) n = TFL_MAX_SPLIT;
     return n < 1 ? 1 : n;
 }
+
+// The same for the form of known sizes.
+extern "C" int tfl_attn_decode_pick_nsplit(int rows, int H, int max_len) { return tfl_attn_decode_splits(rows, H, 512, 64, max_len, 0); }
 
 template <typename T, int NW, int HT, int NTW>
 static int launch_latent(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len,

@@ -180,6 +180,7 @@ LATENT_SIGNATURES = {
     "tfl_attn_prefill": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _vp, _vp, _vp, _i32, _i32, _vp, _i64, _vp, _i64, _i32, _i32, _i32,
                                 _i32, _i32, _i32, _i32, _f32, _i32, _vp]),
     "tfl_attn_decode_ws_floats": (_i64, [_i32, _i32, _i32, _i32]),
+    "tfl_attn_decode_splits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32]),
     "tfl_attn_decode_pick_nsplit": (_i32, [_i32, _i32, _i32]),
     "tfl_attn_decode": (_i32, [_vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _vp]),
 }

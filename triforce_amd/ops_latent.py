@@ -179,7 +179,7 @@ def attn_decode(q, cache, table, klen, g, scale, max_len, nsplit=None):
     assert cache.is_contiguous() and cache.shape[0] % PAGE == 0 and table.shape[0] == rows and table.stride(1) == 1 and klen.numel() == rows
     L = hip.latent_lib()
     if nsplit is None:
-        nsplit = L.tfl_attn_decode_pick_nsplit(rows, g.H, int(max_len))
+        nsplit = L.tfl_attn_decode_splits(rows, g.H, g.C, g.R, int(max_len), _CODE[q.dtype])
     n_ws = L.tfl_attn_decode_ws_floats(rows, g.H, g.C, nsplit)
     ws = torch.empty(n_ws, dtype=torch.float32, device=q.device) if n_ws else None
     out = torch.empty(rows, g.H, g.C, dtype=q.dtype, device=q.device)
