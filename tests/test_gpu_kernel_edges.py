@@ -615,3 +615,11 @@ def test_latent_prefill_tiles(news, pasts, H, half):
             want, size = _flash_want(turned[t0:t0 + n, h], k, kv[k0:k0 + nk, 128 * (H + h):128 * (H + h) + 128], hi * 0, hi, 0.08)
             s = torch.sigmoid(gate[t0:t0 + n, 128 * h:128 * h + 128].double())
             assert ((out[t0:t0 + n, 128 * h:128 * h + 128].double() - s * want).abs() <= 2.0 ** -8 * s * (want.abs() + size) + 1e-6).all()
+
+
+# more keys than the caches hold and more than one round of workgroups: sequence by sequence, in blocks of 128 and of 256 rows; heads that
+# do not divide over the XCDs; blocks of 256 rows for a few rows behind many keys
+@pytest.mark.parametrize("news,pasts,H", [([700, 130, 257], [6000, 5500, 5000], 40), ([700, 130, 257], [6000, 5500, 5000], 39),
+                                          ([700, 130, 257, 513], [4200, 3500, 3000, 2500], 64), ([222, 130], [1500, 1700], 128)])
+def test_latent_prefill_by_sequence(news, pasts, H):
+    test_latent_prefill_tiles(news, pasts, H, 32)

@@ -11,6 +11,15 @@
 #pragma once
 #include "tile_common.h"
 
+// Which (sequence, head, query block) the workgroup at (at, row) takes of a grid of width (sequences times heads) x blocks.  Row by row, all
+// sequences and heads of a row side by side; by_seq: in the same linear order sequence by sequence, then block by block, heads side by side.
+struct SeqBlock { int seq, head, block; };
+__device__ __forceinline__ SeqBlock seq_block(int at, int width, int heads, int row, int blocks, bool by_seq) {
+    if (!by_seq) return SeqBlock{at / heads, at % heads, row};
+    const int l = row * width + at, rest = l / heads;
+    return SeqBlock{rest / blocks, l % heads, rest % blocks};
+}
+
 template <int KR, int NWV> struct FlashTile {
     static constexpr int KT = 64, QT = 2, NC = 4 + KR, NT = 8, D = 128, ROWS = 32 * NWV, STEP = 4 * NWV;
     static constexpr int K_ELEMS = KT * D, R_ELEMS = KT * 32 * KR, LDS = 2 * (2 * K_ELEMS + R_ELEMS) * 2;      // bytes

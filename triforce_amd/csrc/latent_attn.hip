@@ -734,7 +734,9 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(const T* __restric
 
 // Keys of 128 + 64 and values of 128 in bfloat16, on the loop of flash_tile.h: 80 KB of LDS, two workgroups of 128 query rows per CU (or one of 256).
 // Workgroups go round-robin over the 8 XCDs: a head's query blocks sit on one of them and share its L2, the last blocks of all sequences and
-// heads first (sequence by sequence six of 222 to 1 333 rows take 106 us, not 98).
+// heads first (sequence by sequence six of 222 to 1 333 rows take 106 us, not 98).  That reads every key once per query block from wherever it
+// lies, so with more keys than the chip's caches hold (256 MB; from 5 * 2^17 keys times heads, 320 MB, on) and more than one round of workgroups the order is sequence
+// by sequence, a block's heads side by side: 32 heads, 16 x 500 rows behind 4 096 keys 1 028 -> 875 us, 16 x 1 333 behind 2 000 1 900 -> 1 557.
 // 32 heads, against one workgroup of 256 rows per CU with tiles staged in registers and one product at a time: 4 096 rows 302 -> 243 us, behind
 // 4 096 keys 597 -> 568 (907 TFLOP/s), 6 x 666 rows 111 -> 92, 3 x 700 rows behind 4 096 401 -> 335.
 template <int NWV>
@@ -743,15 +745,17 @@ __global__ __launch_bounds__(64 * NWV, 2) void attn_prefill_sized_kernel(const b
                                                                     const float* __restrict__ cosb, const float* __restrict__ sinb, int half,
                                                                     int max_pos, const bf16* __restrict__ gate, int64_t ld_gate,
                                                                     bf16* __restrict__ out, int64_t ld_out, int tq, int tk, int H, int C,
-                                                                    float scale) {
+                                                                    float scale, int by_seq) {
     typedef FlashTile<2, NWV> Flash;
     constexpr int N = 128, R = 64, V = 128, QB = Flash::ROWS, KT = Flash::KT;
     extern __shared__ __align__(16) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, i = lane & 15;
-    const int id = blockIdx.x, qb = (gridDim.y - 1 - blockIdx.y) * QB;
     const bool by_xcd = (H & 7) == 0;
-    const int hx = by_xcd ? H >> 3 : H, j_ = by_xcd ? id >> 3 : id, h = by_xcd ? (j_ % hx) * 8 + (id & 7) : j_ % hx;
-    const int32_t* sq = seq + 4 * (j_ / hx);
+    const int hx = by_xcd ? H >> 3 : H, x = by_xcd ? blockIdx.x & 7 : 0;
+    const int at = by_xcd ? blockIdx.x >> 3 : blockIdx.x;     // the XCD's own workgroups, in order
+    const SeqBlock o = seq_block(at, by_xcd ? gridDim.x >> 3 : gridDim.x, hx, blockIdx.y, gridDim.y, by_seq);
+    const int h = by_xcd ? o.head * 8 + x : o.head, qb = (gridDim.y - 1 - o.block) * QB;
+    const int32_t* sq = seq + 4 * o.seq;
     const int q_at = sq[0], nq = sq[1], k_at = sq[2], nk = sq[3];
     if (qb >= nq || nq < 1 || nk < nq || q_at < 0 || k_at < 0 || q_at + nq > tq || k_at + nk > tk) return;
     const int past = nk - nq;
@@ -822,12 +826,15 @@ static int launch_prefill_sized(const void* q, const void* kv, const void* ck, c
                                 const float* cosb, const float* sinb, int half, int max_pos, const void* gate, int64_t ld_gate, void* out,
                                 int64_t ld_out, int tq, int tk, int H, int C, float scale, hipStream_t st) {
     typedef FlashTile<2, NWV> Flash;
+    const int blocks = (max_new + Flash::ROWS - 1) / Flash::ROWS;
+    const int64_t all = (int64_t)H * nseq * blocks;
+    const bool by_seq = (int64_t)tk * H >= 5 << 17 && all > 2048 / NWV && all < 1 << 30;
     auto k = attn_prefill_sized_kernel<NWV>;
     const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, Flash::LDS);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(k, dim3((unsigned)(H * nseq), (max_new + Flash::ROWS - 1) / Flash::ROWS), dim3(64 * NWV), Flash::LDS, st, (const bf16*)q,
+    hipLaunchKernelGGL(k, dim3((unsigned)(H * nseq), blocks), dim3(64 * NWV), Flash::LDS, st, (const bf16*)q,
                        (const bf16*)kv, (const bf16*)ck, seq, pos, cosb, sinb, half, max_pos, (const bf16*)gate, ld_gate, (bf16*)out, ld_out, tq, tk, H,
-                       C, scale);
+                       C, scale, (int)by_seq);
     TFL_LAUNCH_CHECK();
     return TF_OK;
 }
@@ -869,11 +876,12 @@ extern "C" int tfl_attn_prefill(const void* q, const void* kv, const void* ck, c
     if (dtype == 0) {
         if (N == 128 && R == 64 && V == 128 && C <= 1 << 24 && (int64_t)H * nseq <= 1 << 30 && max_new <= 1 << 22) {       // (63 rows of
                                                                  // either stay below 2^32 bytes)
-            // 256 rows per workgroup read half as much, which tells where the keys of all heads come from memory (from 16 384 per sequence), but
-            // only with whole rounds of 256: 2 048 rows behind 20 000 keys 879 -> 853 us, 4 096 1 812 -> 1 758; behind 10 000 471 -> 478,
-            // 2 500 behind 20 000 1 322 -> 1 568
+            // 256 rows per workgroup read half as much, which tells where the keys of all heads come from memory (from 16 384 per sequence) or
+            // are many to a query (8 and more; a causal prompt of 222 rows 27 % slower), but only with whole rounds of 256: 2 048 rows behind 20 000
+            // keys 879 -> 853 us, 4 096 1 812 -> 1 758; 32 heads, 16 x 130 behind 4 096 466 -> 410, 8 heads, 32 x 222 behind 10 000 545 -> 477; behind
+            // 10 000 471 -> 478, 2 500 behind 20 000 1 322 -> 1 568
             const int64_t wide = (int64_t)((max_new + 255) / 256) * H * nseq;
-            if (tk / nseq >= 16384 && (wide + 255) / 256 * 256 - wide < 48) return launch_prefill_sized<8>(SIZED_ARGS);
+            if ((tk / nseq >= 16384 || (tk / 8 >= tq && max_new > 128)) && (wide + 255) / 256 * 256 - wide < 48) return launch_prefill_sized<8>(SIZED_ARGS);
             return launch_prefill_sized<4>(SIZED_ARGS);
         }
         if (D <= 96 && V <= 64) GO(bf16, 64, 3, 4);
