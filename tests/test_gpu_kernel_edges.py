@@ -623,3 +623,12 @@ def test_latent_prefill_tiles(news, pasts, H, half):
                                           ([700, 130, 257, 513], [4200, 3500, 3000, 2500], 64), ([222, 130], [1500, 1700], 128)])
 def test_latent_prefill_by_sequence(news, pasts, H):
     test_latent_prefill_tiles(news, pasts, H, 32)
+
+
+# the same over the paged cache, where the kernel itself adds up the visible keys: on either side of its line, chunks that hide most of
+# them, more sequences than a wave has lanes
+@pytest.mark.parametrize("news,pasts,chunk,H,G", [([700, 130, 257, 513], [2500, 1000, 2000, 2300], 8192, 32, 32), ([700, 130, 257, 513], [4000, 3000, 2500, 2300], 8192, 23, 23),
+                                                  ([700, 130, 257, 513], [4000, 3000, 2500, 2300], 600, 32, 32), ([130] + [1, 3] * 35, [1900] * 71, 8192, 8, 2),
+                                                  ([700, 130, 257, 513], [3000, 1500, 1400, 691], 8192, 32, 32), ([700, 130, 257, 513], [3000, 1500, 1400, 692], 8192, 32, 32)])
+def test_chunked_prefill_by_sequence(news, pasts, chunk, H, G):
+    test_chunked_prefill_tiles(news, pasts, chunk, H, G)

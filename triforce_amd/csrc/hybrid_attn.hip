@@ -9,20 +9,32 @@
 #include "hybrid_common.h"
 
 // Workgroups go round-robin over the 8 XCDs: the query blocks of a key / value head stay on one of them (its heads side by side), the last
-// blocks of all sequences and heads first (sequence by sequence six of 222 to 1 333 rows take 82 us, not 73).  32 heads on 8, against
+// blocks of all sequences and heads first (sequence by sequence six of 222 to 1 333 rows take 82 us, not 73).  That reads every key once per
+// query block from wherever it lies: with more keys than the caches keep for it (2^18 visible keys times key / value heads, 128 MB) and more
+// than one round of workgroups (the caller's by_seq) the order is sequence by sequence, a block's heads side by side: 32 heads on 32, 16 x
+// 1 333 rows behind 2 000 keys 1 668 -> 1 299 us, 32 x 700 behind 500 723 -> 550; 8 on 2, 32 x 700 behind 4 096 552 -> 522.  32 heads on 8, against
 // workgroups of 256 rows with tiles staged in registers, head by head: 4 096 rows 276 -> 197 us, 3 904 behind 4 096 531 -> 478 (810
 // TFLOP/s), 4 096 behind 6 000 with a chunk's edge at 8 192 569 -> 453, 6 x 1 000 behind 500 in chunks of 640 140 -> 94.
 __global__ __launch_bounds__(256, 2) void attn_chunk_sized_kernel(const bf16* __restrict__ q, int64_t ld_q, const bf16* __restrict__ cache, int n_pages,
                                                                   const int32_t* __restrict__ table, int table_ld, const int32_t* __restrict__ seq,
                                                                   const bf16* __restrict__ gate, int64_t ld_gate, bf16* __restrict__ out,
-                                                                  int64_t ld_out, int tokens, int H, int G, int chunk, float scale, float out_scale) {
+                                                                  int64_t ld_out, int tokens, int H, int G, int chunk, float scale, float out_scale,
+                                                                  int nseq, int by_seq) {
     typedef FlashTile<0, 4> Flash;
     constexpr int D = 128, QB = Flash::ROWS, KT = Flash::KT;
     extern __shared__ __align__(16) char smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, i = lane & 15;
-    const int id = blockIdx.x, qb = (gridDim.y - 1 - blockIdx.y) * QB;
+    if (by_seq) {                                             // (the lengths are on the device: every wave adds them up)
+        int64_t keys = 0;
+        for (int s = lane; s < nseq; s += 64) keys += max(0, seq[4 * s + 1]) + max(0, chunk > 0 ? seq[4 * s + 2] % chunk : seq[4 * s + 2]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) keys += __shfl_xor(keys, o, 64);
+        by_seq = __builtin_amdgcn_readfirstlane(keys * G >= 1 << 18);     // (scalar, and with it every tile address)
+    }
     const bool by_xcd = (H & 7) == 0;
-    const int hx = by_xcd ? H >> 3 : H, j_ = by_xcd ? id >> 3 : id, h = (by_xcd ? (id & 7) * hx : 0) + j_ % hx, b = j_ / hx;
+    const int hx = by_xcd ? H >> 3 : H, at = by_xcd ? blockIdx.x >> 3 : blockIdx.x;      // the XCD's own workgroups, in order
+    const SeqBlock o = seq_block(at, by_xcd ? gridDim.x >> 3 : gridDim.x, hx, blockIdx.y, gridDim.y, by_seq);
+    const int h = (by_xcd ? (blockIdx.x & 7) * hx : 0) + o.head, b = o.seq, qb = (gridDim.y - 1 - o.block) * QB;
     const int32_t* sq = seq + 4 * b;
     const int q_at = sq[0], nq = sq[1], past = sq[2];
     if (qb >= nq || nq < 1 || past < 0 || q_at < 0 || q_at + nq > tokens) return;
@@ -240,11 +252,13 @@ extern "C" int tfh_attn_prefill(const void* q, int64_t ld_q, const void* cache, 
     if (dtype == 0) {
         if (D == 128 && V == 128 && G <= 1 << 16 && (int64_t)H * nseq <= 1 << 30 && max_new <= 1 << 22) {       // (63 cache rows stay below 2^32 bytes)
             constexpr int LDS = FlashTile<0, 4>::LDS;
+            const int blocks = (max_new + 127) / 128;
+            const bool by_seq = nseq > 1 && (int64_t)H * nseq * blocks > 512 && (int64_t)H * nseq * blocks < 1 << 30;
             const hipError_t e = hipFuncSetAttribute((const void*)attn_chunk_sized_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
             if (e != hipSuccess) return (int)e;
-            hipLaunchKernelGGL(attn_chunk_sized_kernel, dim3((unsigned)(H * nseq), (max_new + 127) / 128), dim3(256), LDS, st, (const bf16*)q, ld_q,
+            hipLaunchKernelGGL(attn_chunk_sized_kernel, dim3((unsigned)(H * nseq), blocks), dim3(256), LDS, st, (const bf16*)q, ld_q,
                                (const bf16*)cache, (int)n_pages, table, table_ld, seq, (const bf16*)gate, ld_gate, (bf16*)out, ld_out, tokens, H, G,
-                               chunk, scale, out_scale);
+                               chunk, scale, out_scale, nseq, (int)by_seq);
             TFL_LAUNCH_CHECK();
             return TF_OK;
         }
