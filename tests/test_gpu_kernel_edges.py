@@ -45,6 +45,13 @@ def test_retrieval_score_chunks_of_eight(H, C, token_major):
     assert ((got.double() - want).abs() <= bound).all()
 
 
+# three and four rounds of chunks and a little (the general kernel, up to its 2 048 workgroups), whole rounds, nearly four
+@pytest.mark.parametrize("H,C,token_major", [(32, 769, False), (32, 800, True), (32, 768, False), (32, 921, False), (32, 1000, False), (40, 600, False), (40, 801, False),
+                                             (64, 450, True), (7, 3700, False)])
+def test_retrieval_score_rounds(H, C, token_major):
+    test_retrieval_score_chunks_of_eight(H, C, token_major)
+
+
 def _attention64(q, k, v, scale):
     """Causal attention of the last rows in float64: q (n, H, D), k / v (H, m, D) -> out and sum of weight x |value|, per head."""
     n, m = q.shape[0], k.shape[1]

@@ -381,10 +381,17 @@ extern "C" int tf_retrieval_score(const void* k, int64_t stride_t, int64_t strid
         // 32 x 1 000 12.6 / 12.1 / 13.0, 5 x 5 003 10.3 / 10.3 / 11.0.
         const bool one = 256 % H == 0 && (int64_t)C * H >= (1 << 18);
         const int room = one ? 256 : 512, few = H <= room ? room / H : 1;
-        hipLaunchKernelGGL((retrieval_score_ahead_kernel<128, 8>), dim3(gx < few ? gx : few, H), dim3(256), 0, st, (const h16*)k,
-                           stride_t, stride_h, (const h16*)q, (h16*)scores, C);
-        TF_LAUNCH_CHECK();
-        return TF_OK;
+        // Three or four rounds and a little: the general kernel has every chunk on its way at once, a last round here is nearly a round
+        // (32 x 800, 3.1 rounds, 9.9 us there against 10.5, 40 x 600 9.5 against 10.4, 64 x 450, 3.5 rounds, 11.0 against 11.7; 40 x 700, 3.6
+        // rounds, 10.7 both; 32 x 600, 2.3 rounds, 8.4 and 8.7 from memory, 7.7 and 7.4 from the caches; more workgroups here 11.4 for 32 x 800).
+        const int round = few * gpb, whole = C / round, rest = C - whole * round;
+        const bool at_once = (int64_t)H * ((C + gpb - 1) / gpb) <= 2048 && whole >= 3 && rest > 0 && 5 * rest < 3 * round;
+        if (!at_once) {
+            hipLaunchKernelGGL((retrieval_score_ahead_kernel<128, 8>), dim3(gx < few ? gx : few, H), dim3(256), 0, st, (const h16*)k,
+                               stride_t, stride_h, (const h16*)q, (h16*)scores, C);
+            TF_LAUNCH_CHECK();
+            return TF_OK;
+        }
     }
     if (D == 128)
         hipLaunchKernelGGL((retrieval_score_kernel<128>), dim3(gx, H), dim3(256), 0, st, (const h16*)k, stride_t,
