@@ -409,3 +409,17 @@ def test_large_float32_products_stay_the_librarys_off_the_device():
     assert torch.equal(ot.TileWeight(w).matmul(x), want)
     assert ot.linear_rows(x.view(512, 2, 2048), w).shape == (512, 2, 2048)
     assert ot.linear_rows(x.to("meta"), w.to("meta")).shape == (1024, 2048)
+
+
+def test_float32_parts_fit_an_xcd():
+    """Parts of k that the library picks: the workgroups of no XCD (32 CUs, an eighth of the 256 x 128 tiles, rounded up) run one round more
+    than all of them together need."""
+    from triforce_amd import hip
+    L = hip.tile_lib()
+    for rows, n, k in ((700, 1536, 6144), (700, 2560, 4096), (640, 1536, 6144), (300, 4096, 4096), (3100, 1536, 6144), (256, 12320, 4096)):
+        tiles = -(-n // 256) * -(-rows // 128)
+        auto = L.tfl_split_gemm_ws_floats(rows, n, k, 0)
+        parts = [s for s in range(1, 9) if L.tfl_split_gemm_ws_floats(rows, n, k, s) == auto]
+        assert len(parts) == 1, (rows, n, k, parts)
+        rounds = -(--(-tiles // 8) * parts[0] // 32)
+        assert rounds == -(-tiles * parts[0] // 256), (rows, n, k, parts, rounds)

@@ -10,7 +10,8 @@
 //   700 rows of k = 4 096   normals 1.1e-6 -> 7.1e-7 -> 2.7e-7, their absolute values 9.9e-7 -> 3.2e-6 -> 1.8e-7;
 //   700 rows of k = 15 104  normals 2.1e-6 -> 9.2e-7 -> 3.4e-7, absolute values 1.7e-6 -> 5.8e-6 -> 1.2e-7, normals of mean 1
 //   1.5e-6 -> 4.7e-6 -> 1.4e-7, uniform in 1 .. 2 1.6e-6 -> 8.4e-6 -> 1.4e-7.
-// (Rounded parts in one accumulator: 9.1e-7, 2.2e-7, 2.5e-7, 2.3e-7.  The accuracy costs 1 to 2 %: 22 016 x 4 096 at 700 rows 730 -> 740 us.)
+// (Rounded parts in one accumulator: 9.1e-7, 2.2e-7, 2.5e-7, 2.3e-7.  The accuracy costs 1 to 2 % where a CU has many steps, up to 6 % in short parts: 22 016 x 4 096 at 700
+// rows 730 -> 740 us.)
 // Six bf16 instructions take 3/8 of the cycles of the eight fp32 ones that cover the same 16 x 16 x 32.
 //
 // 256 outputs x 128 rows per workgroup, eight waves of 64 x 64: per step of 32 a wave reads 24 KB from LDS for 96 products (1 536 cycles),
@@ -292,15 +293,16 @@ static int launch_split_gemm(const SplitGemm& a, hipStream_t st) {
 static int64_t split_planes(int rows, int k) { return (int64_t)((rows + 15) / 16) * (k / 32) * 1536 * 2 / 4; }
 static int64_t split_marks(int rows, int k) { return ((int64_t)rows * split_parts(k) + 3) / 4 * 4; }
 
-// Parts of k: rounds of 256 workgroups, each with the fill of its pipe (4 steps of 32), against what the parts cost on their way through memory
-// (a written and read 128 x 256 part as much as 8 steps).  256 rows, 12 320 x 4 096: 267 us without parts, 159 with two, 171 with four;
-// 700 rows, 4 096 x 8 192: 514, 296 with two, 262 with five, 265 with eight.
+// Parts of k: rounds of workgroups, each with the fill of its pipe (4 steps of 32), against what the parts cost on their way through memory
+// (a written and read 128 x 256 part as much as 8 steps).  Rounds are an XCD's: it has 32 CUs and its eighth of the tiles, rounded up (36 tiles in
+// seven parts are 252 workgroups, but 35 on some XCDs: 700 rows, 1 536 x 6 144 in seven 119 us, in six 95).  256 rows, 12 320 x 4 096: 267 us
+// without parts, 159 with two, 171 with four; 700 rows, 4 096 x 8 192: 514, 296 with two, 262 with five, 265 with eight.
 static int pick_parts(int rows, int n, int k) {
-    const int64_t tiles = (int64_t)((n + 255) / 256) * ((rows + 127) / 128);
+    const int64_t tiles = (int64_t)((n + 255) / 256) * ((rows + 127) / 128), per_xcd = (tiles + 7) / 8;
     int best = 1;
     double least = 0;
     for (int s = 1; s <= 8 && (s == 1 || s * 512 <= k); ++s) {
-        const double t = (double)((tiles * s + 255) / 256) * (1.0 / s + 4.0 / (k / 32)) + (s > 1 ? 8.0 * (double)s * tiles / 256 / (k / 32) : 0);
+        const double t = (double)((per_xcd * s + 31) / 32) * (1.0 / s + 4.0 / (k / 32)) + (s > 1 ? 8.0 * (double)s * tiles / 256 / (k / 32) : 0);
         if (s == 1 || t < least) { best = s; least = t; }
     }
     return best;
