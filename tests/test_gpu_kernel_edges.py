@@ -455,7 +455,7 @@ def test_split_float32_sums(k, splits, kind):
 
 
 # where these products are taken, they are no further off than the library's on the fp32 instruction
-@pytest.mark.parametrize("rows,n,k", [(256, 1136, 15104), (272, 4112, 4096), (1030, 4096, 1024), (300, 512, 65536)])
+@pytest.mark.parametrize("rows,n,k", [(512, 1136, 15104), (272, 4112, 4096), (1030, 4096, 1024), (1152, 512, 65536)])
 @pytest.mark.parametrize("kind", ["normal", "absolute", "mean one", "uniform", "mixed"])
 def test_split_float32_against_the_instruction(rows, n, k, kind):
     from triforce_amd import ops_tile as ot
@@ -464,6 +464,18 @@ def test_split_float32_against_the_instruction(rows, n, k, kind):
     got = ot.linear_rows(x, w)
     assert torch.equal(got, ot.split_linear(x, w))
     assert (got.double() - want).norm() <= (library.double() - want).norm()
+
+
+# few results of a long k, and a short k: the library's; on the other side of either line the split kernel's, in parts that fit an XCD
+@pytest.mark.parametrize("rows,n,k,split", [(256, 1136, 15104, False), (1024, 512, 8192, False), (1040, 512, 8192, True), (1030, 65536, 64, False),
+                                            (700, 65536, 96, True), (700, 1536, 6144, True)])
+def test_float32_products_by_shape(rows, n, k, split):
+    from triforce_amd import ops_tile as ot
+    x, w = _factors("normal", rows, n, k)
+    got = ot.linear_rows(x, w)
+    assert torch.equal(got, ot.split_linear(x, w) if split else torch.nn.functional.linear(x, w))
+    want, size = x[:64].double() @ w[-48:].double().T, x[:64].double().norm(dim=1)[:, None] * w[-48:].double().norm(dim=1)
+    assert ((got[:64, -48:].double() - want).abs() <= 2e-6 * size).all()
 
 
 # every pair of scales, down to denormal factors: results of ordinary size from a tiny factor and a huge one, tiny and huge results
