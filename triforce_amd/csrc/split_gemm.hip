@@ -143,11 +143,9 @@ __device__ __forceinline__ void mend(const SplitGemm& a, int row0, int n0, f32x4
     for (int e = 0; e < 4; ++e) v[e] = lost[e] ? p[e] : v[e];
 }
 
-// MT 16-row tiles of x per wave; waves: 4 x 64 outputs, 2 x 16 MT rows.
-template <int MT>
+// Waves: 4 x 64 outputs, 2 x 64 rows (MT 16-row tiles of x each); every wave brings PER fragments of x in.
 __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
-    constexpr int NP = 16, XP = 2 * MT, PER = 3 * XP / 8, BUF = 3 * (NP + XP) * 512;
-    static_assert(3 * XP % 8 == 0, "the waves bring in the same number of fragments");
+    constexpr int MT = 4, NP = 16, XP = 2 * MT, PER = 3 * XP / 8, BUF = 3 * (NP + XP) * 512;
     extern __shared__ __align__(16) bf16 tiles[];             // [2][NP + XP][3][512]
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15;
     const int wn = wave & 3, wm = wave >> 2, chunks = a.k >> 5;
@@ -274,13 +272,12 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const SplitGemm a) {
     if (row0 + i < a.rows) *reinterpret_cast<f32x4*>(a.out + (int64_t)(row0 + i) * a.ld_out + n0 + 4 * g) = s;
 }
 
-template <int MT>
 static int launch_split_gemm(const SplitGemm& a, hipStream_t st) {
-    constexpr int LDS = 2 * 3 * (16 + 2 * MT) * 1024;
-    const hipError_t e = hipFuncSetAttribute((const void*)split_gemm_kernel<MT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    constexpr int LDS = 2 * 3 * (16 + 8) * 1024;              // two buffers of 16 panels of weights and 8 of x, in three parts
+    const hipError_t e = hipFuncSetAttribute((const void*)split_gemm_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e != hipSuccess) return (int)e;
-    const int tiles = (a.n + 255) / 256 * ((a.rows + 32 * MT - 1) / (32 * MT));
-    hipLaunchKernelGGL(split_gemm_kernel<MT>, dim3((tiles + 7) / 8 * 8, a.splits), dim3(512), LDS, st, a);
+    const int tiles = (a.n + 255) / 256 * ((a.rows + 127) / 128);
+    hipLaunchKernelGGL(split_gemm_kernel, dim3((tiles + 7) / 8 * 8, a.splits), dim3(512), LDS, st, a);
     TFL_LAUNCH_CHECK();
     if (a.splits > 1) {
         hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((int64_t)((a.rows + 15) / 16) * ((a.n + 63) / 64))), dim3(256), 0, st, a);
@@ -325,5 +322,5 @@ extern "C" int tfl_split_gemm(const float* w, const float* x, int64_t ld_x, floa
     hipLaunchKernelGGL(split_rows_kernel, dim3((rows + 15) / 16, split_parts(k)), dim3(256), 0, (hipStream_t)stream, x, ld_x, rows, k, (bf16*)ws, nans);
     TFL_LAUNCH_CHECK();
     const SplitGemm a = {w, (const bf16*)ws, x, out, ws + split_planes(rows, k) + split_marks(rows, k), nans, ld_x, ld_out, rows, n, k, splits};
-    return launch_split_gemm<4>(a, (hipStream_t)stream);
+    return launch_split_gemm(a, (hipStream_t)stream);
 }

@@ -604,10 +604,12 @@ class PagedCache(Cache):
         self.rows = [torch.zeros(self.n_pages * self.page, w, dtype=model.dtype, device=self.device) if w else None
                      for w in model.cache_widths()]
         model.prepare_positions(self.max_budget)
-        self.generation = 0                         # bumped when a page is handed out or taken back
+        self.generation = 0                         # counts pages handed out and sequences taken back, for a caller's own tables
         self.free, self.pages, self.length = [], {}, {}
         self.free_seats, self.seat = [], {}
-        self.birth, self._births = {}, 0            # a number of its own for every sequence that ever lived here
+        # a number of its own for every sequence that ever lived here: while a birth lasts its pages only grow, so births and lengths
+        # say what a device copy of the tables holds
+        self.birth, self._births = {}, 0
         self._by_seat = torch.zeros(self.max_batch, self.columns, dtype=torch.int32)    # pages of each seat's sequence, 0 behind
         self._by_seat_np = self._by_seat.numpy()
         self.reset()
