@@ -121,6 +121,8 @@ typedef struct TfhRecStep {
 } TfhRecStep;
 
 int64_t tfh_attn_step_ws_floats(int rows, int H, int V, int nsplit);
+/* The nsplit to take for rows that see up to max_keys keys (tfh_attn_step_pick_nsplit: for bfloat16 heads of 128). */
+int tfh_attn_step_splits(int rows, int H, int G, int D, int V, int max_keys, int dtype);
 int tfh_attn_step_pick_nsplit(int rows, int H, int G, int max_keys);
 /* Both parts of a layer's mixer in one launch, either may be NULL: norm / rotation / cache append / attention over the splits of the
  * visible keys; convolution / decay / state update / read-out. */

@@ -171,6 +171,24 @@ def test_step_splits_by_rows():
     assert [L.tfh_attn_step_pick_nsplit(2, 32, 8, n) for n in (64, 65, 700)] == [1, 2, 11]
 
 
+def test_step_splits_by_form():
+    """The rule for heads of 128 in bfloat16 is theirs alone: others take their splits as they come, eight from 16 rows on, and from 32 on three
+    where two workgroups or fewer fit a CU."""
+    from triforce_amd import hip
+    L = hip.hybrid_lib()
+    for rows in (1, 2, 3, 16, 64, 65):
+        for n in (1, 64, 5000, 131072):
+            assert L.tfh_attn_step_splits(rows, 32, 8, 128, 128, n, 0) == L.tfh_attn_step_pick_nsplit(rows, 32, 8, n)
+    rows = (1, 2, 3, 5, 8, 15, 16, 31, 32, 64, 65, 128)
+    assert [L.tfh_attn_step_splits(r, 32, 8, 64, 64, 100000, 0) for r in rows] == [64, 32, 21, 12, 8, 4, 4, 4, 4, 4, 4, 4]
+    for D, dtype in ((96, 0), (64, 1)):
+        assert [L.tfh_attn_step_splits(r, 32, 8, D, D, 100000, dtype) for r in rows] == [64, 32, 21, 12, 8, 4, 8, 8, 4, 4, 4, 4]
+    for D, dtype in ((256, 0), (160, 0), (128, 1), (96, 1)):
+        assert [L.tfh_attn_step_splits(r, 32, 8, D, D, 100000, dtype) for r in rows] == [64, 32, 21, 12, 8, 4, 8, 8, 3, 3, 3, 3]
+    assert [L.tfh_attn_step_splits(20, 32, 8, 96, 96, n, 0) for n in (1, 65, 449)] == [1, 2, 8]
+    assert L.tfh_attn_step_splits(1 << 30, 1 << 15, 1 << 15, 96, 96, 100, 1) == 2
+
+
 def test_cache_pages_and_seats():
     c = HybridCache(_Model(), max_budget=200, max_batch=3)
     assert [None if r is None else tuple(r.shape) for r in c.rows] == [(384, 64), None, (384, 96)]

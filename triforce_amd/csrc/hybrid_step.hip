@@ -673,22 +673,35 @@ extern "C" int64_t tfh_attn_step_ws_floats(int rows, int H, int V, int nsplit) {
     return (int64_t)rows * H * nsplit * (V + 2) + 2 * (int64_t)rows;
 }
 
-// Two workgroups per CU (512) - one (256) for a row alone -, above 16 splits a row in whole sixteens, as long as a split keeps a page of keys; at
-// least four splits a row up to 64 rows, whose unequal lengths are dealt by splits, and three where they are not.  us with the merge,
-// recurrences beside it, caches from memory: one row of 300 / 3 000 / 8 000 keys at 32 splits 13.6 / 15.1 / 15.8, at 64 14.6 / 16.9 / 17.9; three
-// of 1 000 at 16 / 21 16.9 / 20.0; 16 rows of 3 000 at 4 / 8 / 16 65.9 / 66.6 / 74.1; 128 rows of 1 000 at 1 / 2 / 3 / 4 / 8 240 / 245 / 243 / 258 /
-// 277, of 3 000 426 / 431 / 431 / 429 / 446, 65 rows of up to 8 000 325 / 264 / 252 / 246 / 254.
-extern "C" int tfh_attn_step_pick_nsplit(int rows, int H, int G, int max_keys) {
+static bool sized_step(int D, int V, int dtype) { return dtype == 0 && V == D && (D == 64 || D == 128); }
+
+// Two workgroups per CU (512), at least four splits a row up to 64 rows, whose unequal lengths are dealt by splits, as long as a split keeps a
+// page of keys.  us with the merge, recurrences beside it, caches from memory:
+//   * the sized attention of 128: one workgroup per CU for a row alone, above 16 splits a row in whole sixteens, three splits above 64 rows.  One row
+//     of 300 / 3 000 / 8 000 keys at 32 splits 13.6 / 15.1 / 15.8, at 64 14.6 / 16.9 / 17.9; three of 1 000 at 16 / 21 16.9 / 20.0; 16 rows
+//     of 3 000 at 4 / 8 / 16 65.9 / 66.6 / 74.1; 128 rows of 1 000 at 1 / 2 / 3 / 4 / 8 240 / 245 / 243 / 258 / 277, of 3 000 426 / 431 / 431 / 429 /
+//     446, 65 rows of up to 8 000 325 / 264 / 252 / 246 / 254;
+//   * of 64, and the general one: splits as they come (bfloat16 heads of 96, one row of 30 000 keys at 32 / 64 89 / 59; of 256, five rows at 16 / 25
+//     705 / 463);
+//   * the general one, 16 to 31 rows: at least eight (16 rows of 8 000 to 4 000 keys, float32 heads of 128 at 4 / 6 / 8 / 16 830 / 694 / 674 / 737,
+//     bfloat16 of 96 198 / 125 / 106 / 116); from 32 rows on three where two workgroups or fewer fit a CU (float32 heads of 128, 48 rows of 1 000 to 500
+//     keys at 1 / 2 / 3 / 4 384 / 395 / 365 / 400, 128 rows of 300 488 / 544 / 524 / 664), four where more do.
+extern "C" int tfh_attn_step_splits(int rows, int H, int G, int D, int V, int max_keys, int dtype) {
     if (rows < 1 || H < 1 || G < 1 || max_keys < 1) return 1;
-    const int groups = G * ((H / G + 15) / 16), least = rows <= 64 ? 4 : 3;
-    int n = (rows == 1 ? 256 : 512) / (rows * groups);
-    if (n > 16) n &= ~15;
+    const bool sized = sized_step(D, V, dtype), full = sized && D == 128, large = (int64_t)(D + V) * (dtype ? 4 : 2) >= 640;
+    const int groups = G * ((H / G + 15) / 16);
+    const int least = full ? (rows <= 64 ? 4 : 3) : sized ? 4 : rows < 16 ? 4 : rows < 32 ? 8 : large ? 3 : 4;
+    int n = (int)((rows == 1 && full ? 256 : 512) / ((int64_t)rows * groups));
+    if (full && n > 16) n &= ~15;
     if (n < least) n = least;
     const int cap = (max_keys + TFL_PAGE - 1) / TFL_PAGE;
     if (n > cap) n = cap;
     if (n > TFH_MAX_SPLIT) n = TFH_MAX_SPLIT;
     return n < 1 ? 1 : n;
 }
+
+// The same for bfloat16 heads of 128.
+extern "C" int tfh_attn_step_pick_nsplit(int rows, int H, int G, int max_keys) { return tfh_attn_step_splits(rows, H, G, 128, 128, max_keys, 0); }
 
 static int check_attn(const TfhAttnStep& a, int64_t ld_raw) {
     if (!a.q_norm || !a.k_norm || !a.cache || !a.table || !a.ws || a.n_pages < 1 || a.n_pages > (1 << 30) || a.table_ld < 1) return TF_EINVAL;
@@ -762,7 +775,7 @@ extern "C" int tfh_step(const TfhAttnStep* pa, const TfhRecStep* pr, const float
     }
     hipStream_t st = (hipStream_t)stream;
 #define GO(T, NTW, DK, DV) return launch_step<T, NTW, DK, DV>(a, r, ab, rb, slice, lds, raw, ld_raw, klen, rows, eps, st)
-    if (dtype == 0 && pa && a.V == a.D && (a.D == 64 || a.D == 128)) {
+    if (pa && sized_step(a.D, a.V, dtype)) {
         const size_t lds = step_lds(dtype, nullptr, pr);
         if (a.D == 64) GO(bf16, 1, 2, 4);
         GO(bf16, 2, 4, 8);

@@ -228,6 +228,7 @@ HYBRID_SIGNATURES = {
     "tfh_group_norm": (_i32, [_vp, _i64, _vp, _i64, _i32, _vp, _i32, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _f32, _i32, _vp]),
     "tfh_glu": (_i32, [_vp, _vp, _i32, _i32, _i32, _vp]),
     "tfh_attn_step_ws_floats": (_i64, [_i32, _i32, _i32, _i32]),
+    "tfh_attn_step_splits": (_i32, [_i32, _i32, _i32, _i32, _i32, _i32, _i32]),
     "tfh_attn_step_pick_nsplit": (_i32, [_i32, _i32, _i32, _i32]),
     "tfh_step": (_i32, [_c.POINTER(TfhAttnStep), _c.POINTER(TfhRecStep), _vp, _i64, _vp, _i32, _f32, _i32, _vp]),
     "tfh_step_out": (_i32, [_c.POINTER(TfhAttnStep), _c.POINTER(TfhRecStep), _vp, _i64, _vp, _i64, _i64, _i32, _f32, _i32, _vp]),

@@ -159,7 +159,8 @@ class MixerStep:
             a = self.attn = self._fill(hip.TfhAttnStep(), attn)
             assert attn["cache"].dtype == dtype and attn["cache"].is_contiguous() and attn["table"].stride(1) == 1 and attn["table"].shape[0] == rows
             a.n_pages, a.table_ld = attn["cache"].shape[0] // PAGE, attn["table"].stride(0)
-            a.nsplit = nsplit or _lib().tfh_attn_step_pick_nsplit(rows, a.H, a.G, min(max_keys, a.chunk + PAGE) if a.chunk else max_keys)
+            a.nsplit = nsplit or _lib().tfh_attn_step_splits(rows, a.H, a.G, a.D, a.V, min(max_keys, a.chunk + PAGE) if a.chunk else max_keys,
+                                                             _CODE[dtype])
             ws = torch.empty(_lib().tfh_attn_step_ws_floats(rows, a.H, a.V, a.nsplit), dtype=torch.float32, device=raw.device)
             a.ws = ws.data_ptr()
             self.keep.append(ws)
