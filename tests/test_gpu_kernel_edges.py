@@ -161,6 +161,12 @@ def test_wide_gemm_shares(panels, rows, k):
         _near(ot.act_rows(act), tail, size[:, n_raw:] * 1.13, k + 16, out_bits=8)
 
 
+# rests that are taken as a panel of their own, in some epilogues only, and the last that are not
+@pytest.mark.parametrize("panels,rows,k", [(384, 3, 96), (385, 17, 64), (640, 16, 96), (704, 33, 64), (705, 2, 64), (960, 17, 64), (961, 1, 96), (1984, 5, 64)])
+def test_wide_gemm_rests(panels, rows, k):
+    test_wide_gemm_shares(panels, rows, k)
+
+
 # what the packing rule says is what the kernel does: the two forms sum in different orders, so the layout's own form is the one whose
 # bits a weight that was packed by the rule has; and both forms read either layout
 @pytest.mark.parametrize("panels,raw", [(255, 0), (256, 0), (257, 16), (257, 4112), (330, 4096), (330, 4112), (452, 7232), (2047, 0), (2048, 0), (2049, 0), (2300, 64)])

@@ -420,7 +420,12 @@ static int share_gemm(const TflGemm& a, hipStream_t st) {
     const int panels = a.n >> 4, whole = panels / 256, left = (panels - 256 * whole) * 16, per = (left + 1023) / 1024 * 4;
     if (!a.chunk_major || panels < 256) return TF_ERANGE;
     if (EPI == TFL_EPI_IN && per > 0 && per < 16 && 256 * whole * 16 < a.n_raw) return TF_ERANGE;      // sums of squares need whole panels
-    if (per == 0 || per == 16) switch (per == 0 ? whole : whole + 1) {
+    // Rests of 9 to 12 rows a workgroup, and of 5 to 8 beside one panel of gate | up, cost as much as a panel of their own or more (gate | up deals
+    // them in pairs of rows, 32 bytes each): whole panels on fewer CUs.  us at one row, K 4 096, gate | up: 448 panels 13.0 panel by panel, 16.3
+    // with a rest, 12.9 on 224 CUs; 688 17.8, 21.9, 16.7; other outputs 448 12.5, 12.7, 12.5; 688 17.0, 18.3, 16.1; 900 21.7, 21.3 and, as 1 024,
+    // 22.7.
+    const bool up = per == 16 || (per == 12 && (EPI == TFL_EPI_GLU || whole <= 2)) || (per == 8 && EPI == TFL_EPI_GLU && whole == 1);
+    if (per == 0 || up) switch (up ? whole + 1 : whole) {
         case 1: return launch_share<T, EPI, 1, false>(a, 0, 0, st);
         case 2: return launch_share<T, EPI, 2, false>(a, 0, 0, st);
         case 3: return launch_share<T, EPI, 3, false>(a, 0, 0, st);
