@@ -1421,9 +1421,10 @@ __global__ __launch_bounds__(256, TREE ? TF_BLOCK_TREE_OCC : 2) void attn_block_
 // into 1 KiB of LDS, lane-linear, no staging registers and no ds_write; the XOR swizzle of the layout is applied on the
 // SOURCE side (the lane that fills slot j of row r loads chunk j ^ f(r): the swizzles are involutions).
 // (1024-row chunk x 124 928 keys x 32 heads: 792.7 -> 848.4 TF/s, profiles/r03_prefill_slab_ab.jsonl.)
-// What bounds it: power first.  On random data the chip holds 1.67 GHz here (2.24 GHz in the merge kernel next to it; a library
-// GEMM of this type runs at 1.62 GHz), on zeros the same launch is 1.3 times as fast, and the matrix cores are busy 47 % of the
-// cycles.  So what counts is work that can be left out rather than overlap: the exponentials of a slab placed beside the next
+// What bounds it: what the products and everything between them draw.  On random data the chip holds 1.67 GHz here (2.24 GHz in the
+// merge kernel next to it; a library GEMM of this type runs at 1.62 GHz), on zeros the same launch is 1.3 times as fast, and the matrix
+// cores are busy 47 % of the cycles, those of the GEMM 79 %.  So what counts is work that can be left out rather than overlap: the
+// exponentials of a slab placed beside the next
 // slab's products by hand (907 TF/s), a wave priority for the products (925) and deeper or shallower fragment look-ahead (914-931)
 // are all within the noise of each other, while these helped (4096 rows x 65 536 keys x 32 heads):
 //   * addresses of the LDS-DMA from a scalar slab pointer and 32-bit lane offsets, fragment addresses by one XOR per tile, one

@@ -5,7 +5,8 @@
 // V tiles in LDS the loop holds K one tile ahead of V: step t runs QK^T(t + 1) beside the exponentials of tile t, then PV(t).  One barrier
 // per step.  K and V come in by LDS-DMA (no staging registers, no ds_write); the XOR swizzle that keeps the fragments' reads free of bank
 // conflicts is applied where the DMA reads from.  Two workgroups per CU fill each other's waits.
-// Bound by the power of the matrix cores; in front of that by VALU work (exponentials, addresses).  So: tile pointers are scalar, a lane adds 32-bit
+// Bound by what the products and the VALU work between them (exponentials, addresses) draw together: the matrix cores are busy less than half
+// of the cycles, at the clock of a GEMM.  So: tile pointers are scalar, a lane adds 32-bit
 // offsets; fragments are reached by one XOR; masked and unmasked tiles take one path; fragments are read 4 (K) and 8 (V) steps ahead in a
 // fixed order (left to itself the scheduler moves all reads to the front and spills).
 #pragma once

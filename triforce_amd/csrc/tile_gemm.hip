@@ -420,6 +420,10 @@ static int share_gemm(const TflGemm& a, hipStream_t st) {
     const int panels = a.n >> 4, whole = panels / 256, left = (panels - 256 * whole) * 16, per = (left + 1023) / 1024 * 4;
     if (!a.chunk_major || panels < 256) return TF_ERANGE;
     if (EPI == TFL_EPI_IN && per > 0 && per < 16 && 256 * whole * 16 < a.n_raw) return TF_ERANGE;      // sums of squares need whole panels
+    // One panel and a rest of up to 4 rows, from the third (gate | up) or fifth row block on: every block reads the rest again at the price of a
+    // panel.  300 panels, K 4 096, gate | up, 64 / 128 / 256 rows here 26.5 / 48.6 / 92.9 us, panel by panel 25.1 / 39.9 / 76.4; other outputs
+    // 23.5 / 44.5 / 86.8 and 25.6 / 41.8 / 80.8
+    if (whole == 1 && per == 4 && a.rows > (EPI == TFL_EPI_GLU ? 32 : 64)) return TF_ERANGE;
     // Rests of 9 to 12 rows a workgroup, and of 5 to 8 beside one panel of gate | up, cost as much as a panel of their own or more (gate | up deals
     // them in pairs of rows, 32 bytes each): whole panels on fewer CUs.  us at one row, K 4 096, gate | up: 448 panels 13.0 panel by panel, 16.3
     // with a rest, 12.9 on 224 CUs; 688 17.8, 21.9, 16.7; other outputs 448 12.5, 12.7, 12.5; 688 17.0, 18.3, 16.1; 900 21.7, 21.3 and, as 1 024,
