@@ -255,6 +255,16 @@ int tf_rope_append(const void* qkv, int64_t qkv_row_stride, const void* cos, con
                    int64_t stride_t, int64_t stride_h, int slot0, const int32_t* slot0_dev,
                    int rows, int H, int D, int rotate_k, void* stream);
 int tf_silu_mul(const void* gate_up, void* out, int rows, int I, void* stream);
+/* tf_rows_gemm: fp16 products of many rows (csrc/rows_gemm.h): out[m*ld_out + n] = sum over k of x[m*ld_x + k] * w[n*k_total + k], or with form
+ * TF_ROWS_SILU_HALVES, w = [gate rows | up rows], out[m*ld_out + n] = fp16(silu(gate n)) * up n for n < n_total/2 (both rounded to fp16 first:
+ * tf_silu_mul of the product).  n % 16 == 0 (32 with a gated unit), k % 64 == 0, ld_x and ld_out % 8 == 0, 16-byte aligned pointers,
+ * x and w below 4 GiB.  shape, splits: the tile and the parts of k, tf_rows_gemm_plan's or any other of 0 .. TF_ROWS_SHAPES - 1 with a step
+ * of 64 for every part; the plan returns the floats of ws they need (parts * rows * n from two parts on). */
+#define TF_ROWS_SHAPES 8
+enum { TF_ROWS_PLAIN = 0, TF_ROWS_SILU_HALVES = 1 };
+int64_t tf_rows_gemm_plan(int rows, int n, int k, int32_t* shape, int32_t* splits);
+int tf_rows_gemm(const void* x, int64_t ld_x, const void* w, void* out, int64_t ld_out, float* ws, int64_t ws_floats, int rows, int n, int k,
+                 int form, int shape, int splits, void* stream);
 /* tf_embed_rows: x = embed_tokens(input_ids) (models/modeling_llama.py:342, TP_llama.py:206) for the n <= 32 rows of a
  * decode forward, written in an explicit activation layout (see tf_skinny_gemm_act): element (m, k) at
  * out[m * out_sm + (k / 8) * out_sk + k % 8].  embed [vocab][hidden] fp16, ids [n] int64 (clamped to the vocabulary). */

@@ -85,6 +85,17 @@ int64_t tfl_split_gemm_ws_floats(int rows, int n, int k, int splits);
 int tfl_split_gemm(const float* w, const float* x, int64_t ld_x, float* out, int64_t ld_out, float* ws, int64_t ws_floats, int rows, int n, int k,
                    int splits, void* stream);
 
+/* bfloat16 products of many rows (csrc/rows_gemm.h): out[m*ld_out + n] = sum over k of x[m*ld_x + k] * w[n*k_total + k], or with form
+ * TFL_ROWS_GELU_EIGHTS, w being blocks of 8 gate rows | 8 up rows, out[m*ld_out + n] = gelu_tanh(gate n) * up n for n < n_total/2.
+ * n % 16 == 0 (32 with a gated unit), k % 64 == 0, ld_x and ld_out % 8 == 0, 16-byte aligned pointers, x and w below 4 GiB.
+ * shape, splits: the tile and the parts of k, tfl_rows_gemm_plan's or any other of 0 .. TFL_ROWS_SHAPES - 1 with a step of 64 for every part;
+ * the plan returns the floats of ws they need (parts * rows * n from two parts on). */
+#define TFL_ROWS_SHAPES 8
+enum { TFL_ROWS_PLAIN = 0, TFL_ROWS_GELU_EIGHTS = 2 };
+int64_t tfl_rows_gemm_plan(int rows, int n, int k, int32_t* shape, int32_t* splits);
+int tfl_rows_gemm(const void* x, int64_t ld_x, const void* w, void* out, int64_t ld_out, float* ws, int64_t ws_floats, int rows, int n, int k,
+                  int form, int shape, int splits, void* stream);
+
 /* table[row * table_ld + column] = page for n (at most TFL_MAX_ENTRIES) host triples {row, column, page}: pages handed out between
  * two decode steps.  The triples are kernel arguments (nothing is read after the call returns). */
 #define TFL_MAX_ENTRIES 64

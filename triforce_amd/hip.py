@@ -43,6 +43,8 @@ SIGNATURES = {
     "tf_kv_gather_rows": (_i32, [_vp, _vp, _i64, _i64, _i64, _i32, _vp, _i32, _i32, _i32, _i32, _vp]),
     "tf_tree_accept": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i32, _f32, _vp, _vp]),
     "tf_sample_without_replacement": (_i32, [_vp, _vp, _vp, _i32, _i32, _i32, _f32, _vp]),
+    "tf_rows_gemm_plan": (_i64, [_i32, _i32, _i32, _c.POINTER(_c.c_int32), _c.POINTER(_c.c_int32)]),
+    "tf_rows_gemm": (_i32, [_vp, _i64, _vp, _vp, _i64, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _vp]),
     "tf_rmsnorm": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i32, _f32, _vp]),
     "tf_rope_append": (_i32, [_vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _vp, _i32, _i32, _i32, _i32, _vp]),
     "tf_silu_mul": (_i32, [_vp, _vp, _i32, _i32, _vp]),
@@ -162,6 +164,8 @@ TILE_SIGNATURES = {
     "tfl_gemm": (_i32, [_c.POINTER(TflGemm), _i32, _i32, _vp]),
     "tfl_split_gemm_ws_floats": (_i64, [_i32, _i32, _i32, _i32]),
     "tfl_split_gemm": (_i32, [_vp, _vp, _i64, _vp, _i64, _vp, _i64, _i32, _i32, _i32, _i32, _vp]),
+    "tfl_rows_gemm_plan": (_i64, [_i32, _i32, _i32, _c.POINTER(_c.c_int32), _c.POINTER(_c.c_int32)]),
+    "tfl_rows_gemm": (_i32, [_vp, _i64, _vp, _vp, _i64, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _vp]),
     "tfl_set_pages": (_i32, [_vp, _i32, _i32, _i32, _c.POINTER(_c.c_int32), _i32, _vp]),
     "tfl_decode_prep": (_i32, [_vp, _vp, _i32, _i32, _vp, _vp, _vp, _i32, _vp]),
 }

@@ -3,7 +3,7 @@ state-space recurrence, or gated linear attention) on the HIP ops (ops_hybrid).
 
 Decode form of a layer (one token per sequence, any number of sequences): eight launches - [streams, norm] [input projections]
 [mixer: attention splits and state updates side by side] [merge, norms, gates] [output projection] [streams, norm] [gated unit] [down].
-Prefill form: library GEMMs between the row kernels, the paged attention and the segmented recurrence.
+Prefill form: products of many rows (ops_rows) between the row kernels, the paged attention and the segmented recurrence.
 """
 import zlib
 
@@ -245,7 +245,8 @@ class GatedFeedForward:
         return oh.linear_f32(oh.gelu_glu_linear(h, self.w_gu), self.w_down, self.w_down.n)
 
     def prefill(self, h):
-        return self.w_down.matmul(oh.glu(self.w_gu.matmul(h)))
+        act = self.w_gu.glu_matmul(h)
+        return self.w_down.matmul(oh.glu(self.w_gu.matmul(h)) if act is None else act)
 
 
 def one_plus(w, n):

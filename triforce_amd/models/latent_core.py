@@ -2,7 +2,8 @@
 
 Decode form of a layer (one token per sequence, any number of sequences): ten launches - [norm] [input projections, gelu]
 [query up-projection + cache append] [query to latent] [attention, merge] [latent to value, gate] [output + feed-forward down,
-residual] [token gate] [token projection].  Prefill form: library GEMMs between the row kernels and the up-projected attention.
+residual] [token gate] [token projection].  Prefill form: products of many rows (ops_rows) between the row
+kernels and the up-projected attention.
 """
 import zlib
 

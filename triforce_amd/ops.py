@@ -15,7 +15,7 @@ import functools
 import torch
 import torch.nn.functional as F
 
-from . import hip
+from . import hip, ops_rows
 
 _HALF = torch.float16
 
@@ -341,7 +341,7 @@ def can_fuse_rows(rows, embed, *ws):
 
 def linear(x, w, out_f32=False, ln=None, eps=0.0, resid=None, out=None, ss_in=None, ss_out=None):
     """y = x . W^T, fp16 with fp32 accumulation — the reference's nn.Linear / F.linear.  <=32 rows against a
-    PackedLinear run the hand-written weight-streaming kernel; larger blocks (prefill) go to hipBLASLt.
+    PackedLinear run the hand-written weight-streaming kernel; larger blocks (prefill) go to ops_rows.linear.
     Fused forms of the skinny kernel (only valid when ``can_fuse``): ``ln`` = RMSNorm weight applied to x first
     (h = ln * fp16(x * rsqrt(mean(x^2)+eps))), ``resid`` = fp16 residual added to the fp16 result, ``out`` = where
     to write (may be ``resid`` itself); ``ss_out`` (N/16, 32) fp32 receives the per-panel sums of squares of the
@@ -377,13 +377,13 @@ def linear(x, w, out_f32=False, ln=None, eps=0.0, resid=None, out=None, ss_in=No
     assert ln is None and resid is None and out is None and ss_in is None and ss_out is None, \
         "fused linear needs the skinny kernel (ops.can_fuse)"
     assert not isinstance(x, Act), "k-octet-major activations exist only on the skinny decode path"
-    y = F.linear(x, _w(w))
+    y = ops_rows.linear(x, _w(w))
     return y.float() if out_f32 else y
 
 
 def mlp_act(h, wgu, ln=None, eps=0.0, ss_in=None):
     """fp16(silu(gate(h))) * up(h) for a fused gate|up weight: one kernel for <=32 rows (optionally with the
-    RMSNorm of h folded in, ``ln``), GEMM + silu_mul otherwise.  An Act input gives an Act output."""
+    RMSNorm of h folded in, ``ln``), the product of many rows with the unit in its epilogue (or GEMM + silu_mul) otherwise.  An Act input gives an Act output."""
     M = h.shape[0]
     if isinstance(wgu, PackedLinear) and wgu.parts is not None and wgu.split == 2 and M <= SKINNY_MAX_ROWS \
             and h.is_cuda:
@@ -401,7 +401,10 @@ def mlp_act(h, wgu, ln=None, eps=0.0, ss_in=None):
                   "tf_skinny_gemm_swiglu_act")
         return act
     assert ln is None and not isinstance(h, Act), "fused mlp_act needs the skinny kernel (ops.can_fuse)"
-    return silu_mul(F.linear(h, _w(wgu)))
+    w = _w(wgu)
+    if ops_rows.takes(h, w, ops_rows.SILU_HALVES):
+        return ops_rows.product(h, w, ops_rows.SILU_HALVES)
+    return silu_mul(F.linear(h, w))
 
 
 def ss_buffer(hidden, device):

@@ -1,0 +1,80 @@
+"""Products of many rows in 16 bits (prefill) over the C ABI: x . W^T and x . W^T with a gated unit behind it, float16 by libtriforce_hip.so,
+bfloat16 by libtriforce_tile.so (csrc/rows_gemm.h).
+
+Same rules as ops.py: torch owns the memory and the stream.  What the kernel does not take, and what a derivative, transform or trace
+follows, goes to torch.
+"""
+import ctypes
+import functools
+
+import torch
+import torch.nn.functional as F
+from torch.autograd import forward_ad
+
+from . import hip
+
+PLAIN, SILU_HALVES, GELU_EIGHTS = 0, 1, 2
+_FORMS = {torch.float16: (PLAIN, SILU_HALVES), torch.bfloat16: (PLAIN, GELU_EIGHTS)}
+
+
+def unwatched(*ts):
+    """Device tensors that no derivative, transform, trace or autocast follows: a launch behind torch's back would be lost on them."""
+    if torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() \
+            or torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    return all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) and not (t.requires_grad and torch.is_grad_enabled())
+               and forward_ad.unpack_dual(t).tangent is None for t in ts)
+
+
+def takes(x, w, form=PLAIN):
+    """Does the kernel take x [rows, k] . w [n, k]^T as it stands?  (entry() of csrc/rows_gemm.h)"""
+    if x.dim() != 2 or w.dim() != 2 or x.dtype != w.dtype or form not in _FORMS.get(x.dtype, ()):
+        return False
+    (rows, k), n = x.shape, w.shape[0]
+    ld = x.stride(0)
+    return (w.shape[1] == k and rows >= 1 and n >= 16 and n % (16 if form == PLAIN else 32) == 0 and k >= 64 and k % 64 == 0 and x.stride(1) == 1
+            and ld >= k and ld % 8 == 0 and rows * ld < 1 << 31 and n * k < 1 << 31 and n < 1 << 26 and rows * n < 1 << 37 and w.is_contiguous()
+            and x.device == w.device and unwatched(x, w) and x.device.index == torch.cuda.current_device() and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def library_fills(rows, n):
+    """Do tiles of 256 x 256 fill whole rounds of the 256 CUs?  There the library's kernel is the faster one, for a plain product: 4 096 x 4 096 x
+    4 096 93.9 us against 98.5, 4 096 x 12 288 282 against 293, 8 000 x 4 096 x 11 008 480 against 487; where they do not, the other way
+    round (3 100 x 12 288 x 4 096 256 against 245, 3 100 x 22 016 547 against 425)."""
+    tiles = -(-rows // 256) * -(-n // 256)
+    return tiles % 256 == 0 and 100 * rows * n >= 97 * 65536 * tiles
+
+
+@functools.lru_cache(maxsize=4096)
+def _plan(dtype, rows, n, k):
+    shape, splits = ctypes.c_int32(), ctypes.c_int32()
+    f = hip.lib().tf_rows_gemm_plan if dtype == torch.float16 else hip.tile_lib().tfl_rows_gemm_plan
+    floats = f(rows, n, k, ctypes.byref(shape), ctypes.byref(splits))
+    if floats < 0:
+        hip.check(floats, "rows_gemm_plan")
+    return shape.value, splits.value, floats
+
+
+def product(x, w, form=PLAIN, plan=None):
+    """The kernel's product.  plan = (shape, splits): another than its own choice."""
+    (rows, k), n = x.shape, w.shape[0]
+    if plan is None:
+        shape, splits, floats = _plan(x.dtype, rows, n, k)
+    else:
+        shape, splits = plan
+        floats = splits * rows * n if splits > 1 else 0
+    n_out = n if form == PLAIN else n // 2
+    out = torch.empty(rows, n_out, dtype=x.dtype, device=x.device)
+    ws = torch.empty(floats, dtype=torch.float32, device=x.device) if floats else None
+    f, name = (hip.lib().tf_rows_gemm, "tf_rows_gemm") if x.dtype == torch.float16 else (hip.tile_lib().tfl_rows_gemm, "tfl_rows_gemm")
+    hip.check(f(x.data_ptr(), x.stride(0), w.data_ptr(), out.data_ptr(), n_out, ws.data_ptr() if floats else None, floats, rows, n, k, form, shape, splits,
+                torch.cuda.current_stream().cuda_stream), name)
+    return out
+
+
+def linear(x, w):
+    """x . W^T, w [n, k] contiguous.  Up to 32 rows only large weights are the kernel's: 18 784 x 4 096 at 16 rows 67 -> 38 us, 4 096 x 11 008 29 -> 23,
+    but 4 096 x 4 096 11.0 -> 11.7, 256 x 4 096 7.8 -> 10.0 (at 40 rows 12.6 -> 12.3 and 11.3 -> 9.8)."""
+    if (x.shape[0] > 32 or w.numel() > 1 << 25) and takes(x, w) and not library_fills(x.shape[0], w.shape[0]):
+        return product(x, w)
+    return F.linear(x, w)

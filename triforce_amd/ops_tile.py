@@ -7,10 +7,8 @@ gfx950 kernels on torch's current stream; no CPU path exists.  The element type 
 import ctypes
 
 import torch
-import torch.nn.functional as F
-from torch.autograd import forward_ad
 
-from . import hip
+from . import hip, ops_rows
 
 PAGE = hip.TFL_PAGE
 _CODE = {torch.bfloat16: 0, torch.float32: 1}
@@ -97,6 +95,11 @@ class TileWeight:
         assert self.groups == 1 and x.dtype == self.dtype
         return linear_rows(x, self.w)
 
+    def glu_matmul(self, x):
+        """gelu_tanh(gate) * up of x . W^T over many rows in bfloat16, the weight interleave_glu(gate, up); None where it is not one launch."""
+        assert self.groups == 1 and x.dtype == self.dtype
+        return ops_rows.product(x, self.w, ops_rows.GELU_EIGHTS) if ops_rows.takes(x, self.w, ops_rows.GELU_EIGHTS) else None
+
 
 def empty_act(rows, k, dtype, device):
     """Octet-major activation block [k/8, rows, 8] (include/triforce_tile.h); a 2-D tensor is a row-major one."""
@@ -161,27 +164,18 @@ def interleave_glu(gate, up):
 
 
 def linear_rows(x, w):
-    """x . W^T over many rows (prefill), w [n, k] contiguous: the library GEMM, and for large float32 products split_linear.  Its tiles
-    are 256 x 128: from 256 rows and 2^32 multiply-adds on it is the faster one (256 x 4 096 x 4 096 73 -> 61 us, 2 048 x 2 048 x 1 024
+    """x . W^T over many rows (prefill), w [n, k] contiguous: in 16 bits ops_rows.linear, in float32 the library GEMM, and for large products
+    split_linear.  Its tiles are 256 x 128: from 256 rows and 2^32 multiply-adds on it is the faster one (256 x 4 096 x 4 096 73 -> 61 us, 2 048 x 2 048 x 1 024
     70 -> 63, 700 x 22 016 x 4 096 940 -> 750), below that it leaves CUs idle (300 x 6 144 x 1 536 51 -> 55, 64 x 22 016 x 4 096
     115 -> 133), as with few results of a long k, whose parts are eight at most (2^19 results: 385 x 1 136 x 15 104 117 -> 145, 512 x 1 136
     162 -> 150), and with k below 96 the cut and the results are all there is (1 030 x 65 536 x 64 110 -> 116).  Up to k = 65 536 its error is a
     tenth to a half of the library's; at 2^20, with as few parts, the two are equal."""
     rows, (n, k) = x.shape[0], w.shape
     if x.dtype == w.dtype == torch.float32 and x.dim() == 2 and x.shape[1] == k and 256 <= rows <= 1 << 24 and rows * n * k >= 1 << 32 \
-            and rows * n > 1 << 19 and n % 16 == 0 and k % 32 == 0 and 96 <= k <= 1 << 16 and x.device == w.device and _unwatched(x, w) \
+            and rows * n > 1 << 19 and n % 16 == 0 and k % 32 == 0 and 96 <= k <= 1 << 16 and x.device == w.device and ops_rows.unwatched(x, w) \
             and w.is_contiguous() and w.data_ptr() % 16 == 0:
         return split_linear(x, w)
-    return F.linear(x, w)
-
-
-def _unwatched(*ts):
-    """Device tensors that no derivative, transform, trace or autocast follows: a launch behind torch's back would be lost on them."""
-    if torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() \
-            or torch._C._functorch.peek_interpreter_stack() is not None:
-        return False
-    return all(t.is_cuda and type(t) in (torch.Tensor, torch.nn.Parameter) and not (t.requires_grad and torch.is_grad_enabled())
-               and forward_ad.unpack_dual(t).tangent is None for t in ts)
+    return ops_rows.linear(x, w)
 
 
 def split_linear(x, w, splits=0):
