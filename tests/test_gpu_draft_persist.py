@@ -221,3 +221,36 @@ def test_one_launch_draft_lost_arrival_times_out_poisons_and_recovers(sd68, monk
     finally:
         L.tf_draft_persist_tune(1, 0)
         L.tf_draft_persist_tune(0, old_ms)
+
+
+@torch.inference_mode()
+def test_engine_draft_step_in_one_launch_equals_its_graph(sd68, monkeypatch):
+    """graph_draft_inference over device tokens launches the step itself, everything else replays the graph: the same rows, bit for bit, in a
+    tensor of the caller's own."""
+    from triforce_amd.models.cache import FlashSimpleCache, RetrievalCache
+    from triforce_amd.models.modeling_llama import LlamaForCausalLM
+    from triforce_amd.utils.graph_infer import GraphInferenceEngine
+    m, c = _build(sd68, _cfg(), True, monkeypatch)
+    target = LlamaForCausalLM(zoo.config("tiny")).init_random(0)
+    small = RetrievalCache(target, max_budget=64, prefill=64, gamma=GAMMA, chunk_size=8)
+    ge = GraphInferenceEngine(target, FlashSimpleCache(target, 64), small, m, c)
+    ge.initialize_cuda_graph(GAMMA, probs=True, temperature=0.6, top_p=0.9, verbose=False, capture_target=False)
+    gen = torch.Generator().manual_seed(3)
+    c.k.copy_(torch.randn(c.k.shape, generator=gen))
+    c.v.copy_(torch.randn(c.v.shape, generator=gen))
+    for off in range(GAMMA + 3):
+        ids = torch.randint(3, 32000, (1, off + 1), generator=gen).to(DEV)
+        assert ge._draft_is_one_launch(ids, off)
+        fn, k = ge.callables[off], c.k.clone()
+        want = fn(ids)
+        k_want = c.k.clone()
+        c.k.copy_(k)
+        got = ge.graph_draft_inference(ids, gamma_offset=off)
+        assert torch.equal(got, want) and torch.equal(c.k, k_want)
+        assert got.data_ptr() != fn.output.data_ptr() and got.data_ptr() != ge.graph_draft_inference(ids, gamma_offset=off).data_ptr()
+        strided = torch.stack([ids, ids], 2)[:, :, 0]
+        for other in (ids.cpu(), ids.int(), strided):
+            if other is strided and off == 0:
+                continue
+            assert not ge._draft_is_one_launch(other, off)
+            assert torch.equal(ge.graph_draft_inference(other, gamma_offset=off), want)

@@ -93,6 +93,12 @@ class LlamaForCausalLM:
             self._native_cache_ref = c                                  # keeps id(c) from being recycled
         return self._native_cache_struct
 
+    def one_launch(self, c, gamma_offset):
+        """Is a speculative step of gamma_offset + 1 tokens on the cache ``c`` one launch (ops.DraftPersist)?"""
+        n = gamma_offset + 1
+        return (n <= min(ops.SKINNY_MAX_ROWS, c.gamma + 3) and self._native_model() is not None and self._persist is not None and ops.DRAFT_PERSIST
+                and ops.draft_persist_supported(self._native, n, gamma_offset + c.start_size + c.recent_size + 1))
+
     def forward(self, input_ids, kv_cache, graph_cache=None, gamma_offset=-1, probs=None):
         """``probs`` = (temperature, top_p): also return the top-p probability row of the last token (out.probs)."""
         W = self.weights
