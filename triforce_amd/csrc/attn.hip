@@ -1421,15 +1421,17 @@ __global__ __launch_bounds__(256, TREE ? TF_BLOCK_TREE_OCC : 2) void attn_block_
 // into 1 KiB of LDS, lane-linear, no staging registers and no ds_write; the XOR swizzle of the layout is applied on the
 // SOURCE side (the lane that fills slot j of row r loads chunk j ^ f(r): the swizzles are involutions).
 // (1024-row chunk x 124 928 keys x 32 heads: 792.7 -> 848.4 TF/s, profiles/r03_prefill_slab_ab.jsonl.)
-// What bounds it: what the products and everything between them draw.  On random data the chip holds 1.67 GHz here (2.24 GHz in the
-// merge kernel next to it; a library GEMM of this type runs at 1.62 GHz), on zeros the same launch is 1.3 times as fast, and the matrix
-// cores are busy 47 % of the cycles, those of the GEMM 79 %.  So what counts is work that can be left out rather than overlap: the
-// exponentials of a slab placed beside the next
-// slab's products by hand (907 TF/s), a wave priority for the products (925) and deeper or shallower fragment look-ahead (914-931)
-// are all within the noise of each other, while these helped (4096 rows x 65 536 keys x 32 heads):
-//   * addresses of the LDS-DMA from a scalar slab pointer and 32-bit lane offsets, fragment addresses by one XOR per tile, one
-//     code path for masked and unmasked slabs (scores outside set to -inf): 1 650 -> 1 000 VALU cycles per slab; 864 -> 915 TF/s;
-//   * fragments read 4 (K) and 8 (V) steps ahead in a fixed order: 915 -> 930;
+// What bounds it: a wave issues its products (1 024 cycles a slab), some 170 other VALU operations (32 of them exponentials of 16 cycles) and 100
+// scalar and LDS operations one after the other, two waves of a SIMD overlap by half, and the chip is at its power limit while they do:
+// matrix cores busy 50 % of the cycles at 1.82 GHz, on zeros the same launch is 1.3 times as fast.  So what counts is work that can be
+// left out: the exponentials of a slab placed beside the next slab's products by hand, a wave priority for the products and deeper or
+// shallower fragment look-ahead are all within the noise of each other, while these helped (4096 rows x 65 536 keys x 32 heads):
+//   * addresses of the LDS-DMA from a scalar slab pointer and 32-bit lane offsets, one code path for masked and unmasked slabs (scores outside
+//     set to -inf): 864 -> 915 TF/s; fragments read 4 (K) and 8 (V) steps ahead in a fixed order: 930;
+//   * the lane offsets and the twelve LDS places of its fragments kept in registers, the maxima of the next slab beside the products with V, by
+//     instructions of three operands, and the sums rescaled in place: 224 -> 170 VALU operations a slab, 930 -> 959 TF/s (3 100 rows without
+//     a past 136 -> 132 us, 700 rows 22.0 -> 21.4, 1 024 rows x 20 000 408 -> 394).  Two slabs per turn, so that buffers are instruction
+//     offsets too, moves 64 sums between registers in every second slab instead;
 //   * one split (every chunk of more than 2 000 rows): the output is written here instead of partials for the merge kernel, and the
 //     longest row blocks start first: 3 100 rows without a past 205 -> 134 us, 4 096 rows behind 4 096 608 -> 486 us.
 // D = 128, chain (non-tree) form only; 0 = the shared body (attn_block_lds_body).
@@ -1445,8 +1447,7 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
     constexpr int NC = D / 32, NT = D / 16, QT = 2, QR = 128, SLAB = BLK_SLAB, RS = BlkLayout<D>::RS;
     constexpr int VPR = D / 8, RPP = 256 / VPR, NPASS = SLAB / RPP;
     extern __shared__ __attribute__((aligned(16))) unsigned char blk_smem[];
-    h16* sK = reinterpret_cast<h16*>(blk_smem);             // [2][SLAB * RS]
-    h16* sVt = sK + 2 * BlkLayout<D>::K_HALFS;              // [2][SLAB * D]
+    // K [2][SLAB * RS], V [2][SLAB * D]
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, g = lane >> 4;
     const int qbase = wave * 32;
@@ -1472,36 +1473,53 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
     const int row_a = 8 * (li >> 2) + (li & 3);
 
     // one slab (64 rows x 256 B) = 4 passes; pass p, wave w fills rows 16 p + 4 w .. + 3 (1 KiB, lane-linear).  The slab's first row
-    // is a scalar pointer; a lane adds its row's offset, cut at the slab's last key, and the chunk that the swizzle puts at its
-    // place (K's depends on the parity of p, V's does not): three 32-bit VALU operations per pass.  With the row index clamped and
-    // multiplied by the stride per lane, in 64 bits, addresses were 400 of the 1 650 VALU cycles of a slab.
+    // is a scalar pointer, a lane's eight offsets from it stay in registers; the last slab's rows are cut at the last key.
     const uint32_t row_bytes = 2 * (uint32_t)stride_t;                    // (the host takes strides past 2^25 another way: 63 rows stay below 2^32 bytes)
-    uint32_t row_off = (uint32_t)lr * row_bytes;
-    uint32_t chunk_k = 16 * (lc ^ ((lr & 3) | (((lr >> 3) & 3) << 2)));              // odd passes: XOR 8 chunks
-    uint32_t chunk_v = 16 * ((((lc >> 1) ^ ((lr & 3) | (((lr >> 3) & 1) << 2))) << 1) | (lc & 1));
-    auto dma_slab = [&](const h16* base, h16* dst_buf, int slab, bool is_v) {
-        const char* first = reinterpret_cast<const char*>(base + (int64_t)slab * SLAB * stride_t);
-        const uint32_t last_off = (uint32_t)min(SLAB - 1, sk - 1 - slab * SLAB) * row_bytes;
+    const uint32_t chunk_k = 16 * (lc ^ ((lr & 3) | (((lr >> 3) & 3) << 2)));        // odd passes: XOR 8 chunks
+    const uint32_t chunk_v = 16 * ((((lc >> 1) ^ ((lr & 3) | (((lr >> 3) & 1) << 2))) << 1) | (lc & 1));
+    uint32_t off_k[NPASS], off_v[NPASS];
 #pragma unroll
-        for (int p = 0; p < NPASS; ++p) {
-            const uint32_t off = min(row_off + (uint32_t)(p * RPP) * row_bytes, last_off) + (is_v ? chunk_v : chunk_k ^ ((p & 1) * 128));
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(first + off),
-                                             (__attribute__((address_space(3))) void*)(dst_buf + (p * RPP + 4 * wave) * D), 16, 0, 0);
+    for (int p = 0; p < NPASS; ++p) {
+        off_k[p] = (uint32_t)(lr + p * RPP) * row_bytes + (chunk_k ^ ((p & 1) * 128));
+        off_v[p] = (uint32_t)(lr + p * RPP) * row_bytes + chunk_v;
+    }
+    auto dma = [&](const char* src, uint32_t off, int dst) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src + off),
+                                         (__attribute__((address_space(3))) void*)(blk_smem + dst + 1024 * wave), 16, 0, 0);
+    };
+    auto fetch = [&](const h16* base, const uint32_t (&off)[NPASS], int dst, int slab, bool is_v) {
+        const char* first = reinterpret_cast<const char*>(base + (int64_t)slab * SLAB * stride_t);
+        const int last = sk - 1 - slab * SLAB;
+        if (last >= SLAB - 1) {
+#pragma unroll
+            for (int p = 0; p < NPASS; ++p) dma(first, off[p], dst + p * RPP * 2 * D);
+        } else {
+#pragma unroll
+            for (int p = 0; p < NPASS; ++p)
+                dma(first, (uint32_t)min(lr + p * RPP, last) * row_bytes + (is_v ? chunk_v : chunk_k ^ ((p & 1) * 128)), dst + p * RPP * 2 * D);
         }
     };
-    auto fetch_k = [&](int slab, int buf) { dma_slab(kbase, sK + buf * BlkLayout<D>::K_HALFS, slab, false); };
-    auto fetch_v = [&](int slab, int buf) { dma_slab(vbase, sVt + buf * BlkLayout<D>::V_HALFS, slab, true); };
-    // LDS places of a lane's fragments: the swizzles are XORs of bits that no other part of an address touches, so one place per
-    // buffer and one XOR per 32-wide chunk / 16-wide tile reach all of them; the rest are instruction offsets
-    int k_at = row_a * RS + 8 * (g ^ li);
-    int v_at = (8 * g + (li >> 2)) * D + 4 * (li & 3) + 16 * ((li >> 2) | ((g & 1) << 2));
+    constexpr int K_BYTES = 2 * BlkLayout<D>::K_HALFS, V_BYTES = 2 * BlkLayout<D>::V_HALFS, V_BASE = 2 * K_BYTES;
+    auto fetch_k = [&](int slab, int buf) { fetch(kbase, off_k, buf * K_BYTES, slab, false); };
+    auto fetch_v = [&](int slab, int buf) { fetch(vbase, off_v, V_BASE + buf * V_BYTES, slab, true); };
+    // LDS places of a lane's fragments, in bytes: the swizzles are XORs of bits that no other part of an address touches, one place per
+    // 32-wide chunk of K and 16-wide tile of V; halves of a slab and the second row block are instruction offsets, the buffers
+    // one addition per place and slab
+    typedef __attribute__((address_space(3))) const char* Lds;
+    Lds k_at[NC], v_at[NT];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) k_at[c] = (Lds)blk_smem + (2 * (row_a * RS + 8 * (g ^ li)) ^ (64 * c));
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        v_at[t] = (Lds)blk_smem + V_BASE + (2 * ((8 * g + (li >> 2)) * D + 4 * (li & 3) + 16 * ((li >> 2) | ((g & 1) << 2))) ^ (32 * t));
+    f32x4 s[4][QT];                                          // scores of this slab: tiles A, B of keys 0 .. 31, of 32 .. 63
     // Fragments are requested a fixed distance ahead of their products, step by step: left to itself the scheduler moves all 16 (32)
     // reads of a product to its front and spills a hundred registers.
-    auto pv = [&](const half8 (&pa)[QT], const half8 (&pb)[QT], const half8 (&la)[QT], const half8 (&lb)[QT], int at) {
+    auto pv = [&](const half8 (&pa)[2][QT], const half8 (&pl)[2][QT], auto&& beside) {
         constexpr int STEPS = 2 * NT, AHEAD = 8;
         half4 lo[AHEAD + 1], hi[AHEAD + 1];
         auto read = [&](int n) {
-            const h16* src = sVt + (at ^ (16 * (n % NT))) + (n / NT) * 32 * D;
+            const h16* src = (const h16*)(v_at[n % NT] + (n / NT) * 64 * D);
             lo[n % (AHEAD + 1)] = lds_read_tr4(src);
             hi[n % (AHEAD + 1)] = lds_read_tr4(src + 4 * D);
         };
@@ -1515,25 +1533,22 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
             const half8 vt = half8{l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]};
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
-                st.acc[qt][n % NT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt, n < NT ? pa[qt] : pb[qt], st.acc[qt][n % NT], 0, 0, 0);
+                st.acc[qt][n % NT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt, pa[n / NT][qt], st.acc[qt][n % NT], 0, 0, 0);
 #if TF_BLOCK_P_SPLIT > 0
-                st.acc[qt][n % NT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt, n < NT ? la[qt] : lb[qt], st.acc[qt][n % NT], 0, 0, 0);
+                st.acc[qt][n % NT] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vt, pl[n / NT][qt], st.acc[qt][n % NT], 0, 0, 0);
 #endif
             }
+            beside(n);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
-    // both 32-key sub-steps of one slab: scores S^T[key][q] of tiles A / B (keys 4g..4g+3 of either half) per q-tile
-    auto qk_slab = [&](int at, f32x4 (&a0)[QT], f32x4 (&b0)[QT], f32x4 (&a1)[QT], f32x4 (&b1)[QT], auto&& beside) {
-#pragma unroll
-        for (int qt = 0; qt < QT; ++qt) {
-            a0[qt] = f32x4{0.f, 0.f, 0.f, 0.f}; b0[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
-            a1[qt] = f32x4{0.f, 0.f, 0.f, 0.f}; b1[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
+    // both 32-key halves of one slab: scores S^T[key][q] of tiles A / B (keys 4g..4g+3 of either half) per q-tile
+    auto qk = [&](f32x4 (&x)[4][QT], auto&& beside) {
         constexpr int STEPS = 2 * NC, AHEAD = 4;
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
         half8 ka[AHEAD + 1], kb[AHEAD + 1];
         auto read = [&](int n) {
-            const h16* src = sK + (at ^ (32 * (n % NC))) + (n / NC) * 32 * RS;
+            const h16* src = (const h16*)(k_at[n % NC] + (n / NC) * 64 * RS);
             ka[n % (AHEAD + 1)] = load_half8(src);
             kb[n % (AHEAD + 1)] = load_half8(src + 4 * RS);
         };
@@ -1545,92 +1560,111 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
             if (n + AHEAD < STEPS) read(n + AHEAD);
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
-                f32x4& a = n < NC ? a0[qt] : a1[qt];
-                f32x4& b = n < NC ? b0[qt] : b1[qt];
-                a = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[n % (AHEAD + 1)], st.qf[qt][n % NC], a, 0, 0, 0);
-                b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[n % (AHEAD + 1)], st.qf[qt][n % NC], b, 0, 0, 0);
+                f32x4 &a = x[2 * (n / NC)][qt], &b = x[2 * (n / NC) + 1][qt];
+                a = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[n % (AHEAD + 1)], st.qf[qt][n % NC], n % NC ? a : zero, 0, 0, 0);
+                b = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[n % (AHEAD + 1)], st.qf[qt][n % NC], n % NC ? b : zero, 0, 0, 0);
             }
             beside(n);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
+    // scores that a row does not see: exp2 of -inf minus any finite maximum is 0
+    auto hide = [&](int key0, f32x4 (&x)[4][QT]) {
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+            const int qrow = qbase + qt * 16 + li, seen = (qrow < sq ? sk - sq + qrow : sk - 1) - key0 - 8 * g;
+#pragma unroll
+            for (int z = 0; z < 4; ++z)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (32 * (z >> 1) + 4 * (z & 1) + r > seen) x[z][qt][r] = -__builtin_inff();
+        }
+    };
+    // the largest of a slab's scores, one of eight steps per query tile; the last one across the lanes
+    auto largest = [&](const f32x4 (&x)[4][QT], float (&top)[QT], int n) {
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+            if (n == 0) top[qt] = vmax3_raw(x[0][qt][0], x[0][qt][1], x[0][qt][2]);
+            else if (n < 7) top[qt] = vmax3_raw(top[qt], x[(2 * n + 1) >> 2][qt][(2 * n + 1) & 3], x[(2 * n + 2) >> 2][qt][(2 * n + 2) & 3]);
+            else top[qt] = group_max4(vmax_raw(top[qt], x[3][qt][3]));
+        }
+    };
 
     if (s_begin < s_end) {
-        f32x4 c0a[QT], c0b[QT], c1a[QT], c1b[QT];            // scores of the CURRENT slab
+        float top[QT];
         fetch_k(s_begin, 0);
         fetch_v(s_begin, 0);
         fetch_k(min(s_begin + 1, s_end - 1), 1);
         __builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0): Q fragments and the prologue slabs have landed
         __syncthreads();
-        qk_slab(k_at, c0a, c0b, c1a, c1b, [](int) {});
+        qk(s, [](int) {});
+        asm volatile("s_nop 15" ::: "memory");               // (largest() reads products in inline asm, which the compiler does not guard)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < 8; ++n) largest(s, top, n);
         __syncthreads();                                     // every wave is done with K[s_begin] before iteration 0 overwrites it
         for (int sl = s_begin; sl < s_end; ++sl) {
-            const int i = sl - s_begin;
-            // (opaque once per slab: the sums and XORs on these are one instruction each, hoisted out of the loop they would take
-            // some forty registers that the scores need)
-            asm("" : "+v"(row_off), "+v"(chunk_k), "+v"(chunk_v), "+v"(k_at), "+v"(v_at));
-            fetch_k(min(sl + 2, s_end - 1), i & 1);          // K[sl + 2] over K[sl] (dead since the previous barrier), V[sl + 1]
-            fetch_v(min(sl + 1, s_end - 1), (i + 1) & 1);    // over V[sl - 1]; unconditional: in flight under the MFMAs
-            const int k_next = k_at + ((i + 1) & 1) * BlkLayout<D>::K_HALFS;
-            f32x4 n0a[QT], n0b[QT], n1a[QT], n1b[QT];
-            const int key0 = sl * SLAB;
-            if (key0 + SLAB - 1 > sk - sq + qbase) {         // wave-uniform: some row of the wave does not see the whole slab
+            const int buf = (sl - s_begin) & 1;
+            // (opaque once per slab: widened to 64 bits outside the loop they would take a register more each)
 #pragma unroll
-                for (int qt = 0; qt < QT; ++qt) {
-                    const int qrow = qbase + qt * 16 + li, seen = (qrow < sq ? sk - sq + qrow : sk - 1) - key0 - 8 * g;
+            for (int p = 0; p < NPASS; ++p) asm("" : "+v"(off_k[p]), "+v"(off_v[p]));
+            fetch_k(min(sl + 2, s_end - 1), buf);              // K[sl + 2] over K[sl] (dead since the previous barrier), V[sl + 1]
+            fetch_v(min(sl + 1, s_end - 1), buf ^ 1);              // over V[sl - 1]; unconditional: in flight under the MFMAs
+            if (sl * SLAB + SLAB - 1 > sk - sq + qbase) {    // wave-uniform: some row of the wave does not see the whole slab
+                hide(sl * SLAB, s);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {            // exp2 of -inf minus any finite maximum is 0
-                        if (r > seen) c0a[qt][r] = -__builtin_inff();
-                        if (r + 4 > seen) c0b[qt][r] = -__builtin_inff();
-                        if (r + 32 > seen) c1a[qt][r] = -__builtin_inff();
-                        if (r + 36 > seen) c1b[qt][r] = -__builtin_inff();
-                    }
-                }
+                for (int n = 0; n < 8; ++n) largest(s, top, n);
             }
             float mnew[QT];
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) {
-                float tmax = c0a[qt][0];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) tmax = fmaxf(fmaxf(fmaxf(tmax, c0a[qt][r]), fmaxf(c0b[qt][r], c1a[qt][r])), c1b[qt][r]);
-                tmax = group_max4(tmax);
-                mnew[qt] = fmaxf(st.m[qt], tmax * scale_log2);
+                mnew[qt] = fmaxf(st.m[qt], top[qt] * scale_log2);
                 if (__builtin_amdgcn_ballot_w64(mnew[qt] != st.m[qt])) {
                     const float alpha = __builtin_amdgcn_exp2f(st.m[qt] - mnew[qt]);
                     st.l[qt] *= alpha;
+                    // (in place, and only seen here: with results of its own the path without a rescale copies all 64 sums.  The products
+                    // that wrote them lie before the barrier.)
 #pragma unroll
-                    for (int t = 0; t < NT; ++t) {
-                        st.acc[qt][t][0] *= alpha; st.acc[qt][t][1] *= alpha;
-                        st.acc[qt][t][2] *= alpha; st.acc[qt][t][3] *= alpha;
-                    }
+                    for (int t = 0; t < NT; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            float x = st.acc[qt][t][r];
+                            asm("v_mul_f32 %0, %1, %0" : "+v"(x) : "v"(alpha));
+                            st.acc[qt][t][r] = x;
+                        }
                     st.m[qt] = mnew[qt];
                 }
             }
             // The next slab's QK^T (past the end: finite garbage, never used) with this slab's exponentials beside it: four scores of
             // a lane per four products, so that the matrix core works while the wave issues VALU operations
-            half8 p0[QT], p1[QT], l0[QT], l1[QT];            // (l0, l1: TF_BLOCK_P_SPLIT's remainders)
+            half8 p[2][QT], pl[2][QT];                       // (pl: TF_BLOCK_P_SPLIT's remainders)
             float psum[QT] = {};
-            qk_slab(k_next, n0a, n0b, n1a, n1b, [&](int n) {
-                const int qt = n / 4, quad = n % 4;
-                const f32x4& x = quad == 0 ? c0a[qt] : quad == 1 ? c0b[qt] : quad == 2 ? c1a[qt] : c1b[qt];
-                half8& dst = quad < 2 ? p0[qt] : p1[qt];
+            f32x4 next[4][QT];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) k_at[c] += buf ? -K_BYTES : K_BYTES;
+            qk(next, [&](int n) {
+                const int qt = n / 4, z = n % 4;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const float e = __builtin_amdgcn_exp2f(fmaf(x[r], scale_log2, -mnew[qt]));
+                    const float e = __builtin_amdgcn_exp2f(fmaf(s[z][qt][r], scale_log2, -mnew[qt]));
                     psum[qt] += e;
-                    dst[4 * (quad & 1) + r] = (h16)e;
+                    p[z >> 1][qt][4 * (z & 1) + r] = (h16)e;
 #if TF_BLOCK_P_SPLIT > 0
-                    (quad < 2 ? l0[qt] : l1[qt])[4 * (quad & 1) + r] = (h16)(e - (float)(h16)e);
+                    pl[z >> 1][qt][4 * (z & 1) + r] = (h16)(e - (float)(h16)e);
 #endif
                 }
             });
-            pv(p0, p1, l0, l1, v_at + (i & 1) * BlkLayout<D>::V_HALFS);
+            pv(p, pl, [&](int n) {                      // the next slab's maxima (of all its keys) beside the products with V
+                if (n >= 2 && n < 10) largest(next, top, n - 2);
+            });
 #pragma unroll
             for (int qt = 0; qt < QT; ++qt) st.l[qt] += psum[qt];
 #pragma unroll
-            for (int qt = 0; qt < QT; ++qt) {
-                c0a[qt] = n0a[qt]; c0b[qt] = n0b[qt]; c1a[qt] = n1a[qt]; c1b[qt] = n1b[qt];
-            }
+            for (int n = 0; n < NT; ++n) v_at[n] += buf ? -V_BYTES : V_BYTES;
+#pragma unroll
+            for (int z = 0; z < 4; ++z)
+#pragma unroll
+                for (int qt = 0; qt < QT; ++qt) s[z][qt] = next[z][qt];
             __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0): this wave's DMA writes are in LDS before the barrier
             __syncthreads();
         }
