@@ -1,0 +1,86 @@
+"""Latent attention of single tokens with a product beside it in the same launch, against fp64 and against the two launched apart."""
+import pytest
+import torch
+
+from tests.test_gpu_latent import Geom, _paged, f, octets, rnd
+
+pytestmark = pytest.mark.gpu
+SCALE = 1.5 * 576 ** -0.5
+
+
+def _block(rows, n, k0, k, seed):
+    from triforce_amd import ops_latent as ol
+    act = rnd(rows, k0 + k, seed=seed, dtype=torch.bfloat16)
+    w = rnd(n, k0 + k, seed=seed + 1, dtype=torch.bfloat16, scale=(k0 + k) ** -0.5)
+    wt = ol.TileWeight(w, packed_only=True)
+    assert wt.chunk_major
+    return act, w, wt, rnd(rows, n, seed=seed + 2)
+
+
+# lens, heads, n, k0, k, (workers, panels each, splits): as many workers as splits and fewer, two panels and four, a last workgroup with
+# fewer panels, rows of no key, one row, the borders of 16 and 32 rows
+CASES = [([500], 20, 4096, 64, 2048, None), ([1], 32, 4096, 32, 4096, None), ([0], 17, 4096, 32, 4096, None),
+         ([0, 1], 20, 4096, 4096, 3072, None), ([64, 65, 63, 4000, 0, 128, 129, 700], 20, 4096, 4096, 11008, None),
+         ([2000] * 16, 20, 4096, 96, 2176, None), ([129] * 17, 32, 4096, 96, 2176, (170, 3, 20)),
+         ([7 * b * b for b in range(32)], 20, 4096, 4096, 2048, (170, 3, 10)), ([1030, 5], 20, 4112, 32, 2080, (4, 2, 2)),
+         ([1030, 5, 300], 20, 4112, 32, 2080, (6, 3, 3)), ([1030, 5, 300], 18, 6160, 32, 2080, (200, 4, 128)),
+         ([3000] * 20, 18, 4112, 32, 2048, (40, 4, 2))]
+
+
+@pytest.mark.parametrize("lens,heads,n,k0,k,plan", CASES, ids=[f"{len(c[0])}x{c[1]}-{c[2]}x{c[4]}-{c[5]}" for c in CASES])
+def test_attention_beside_a_product(lens, heads, n, k0, k, plan):
+    from triforce_amd import ops_latent as ol
+    rows = len(lens)
+    cache, table, keys = _paged(lens, 512, 64, torch.bfloat16, 5)
+    q = rnd(rows, heads, 576, seed=1, dtype=torch.bfloat16)
+    klen = torch.tensor(lens, dtype=torch.int32, device=q.device)
+    act, w, wt, x = _block(rows, n, k0, k, 7)
+    g = Geom(heads, 32, 64, 32, 512, 32)
+    plan = plan or (128, 2, max(2, min(128, 256 // rows)))
+    got = x.clone()
+    out = ol.attn_decode_beside(q, cache, table, klen, g, SCALE, plan, octets(act), wt, got, k0)
+    down = act[:, k0:].double() @ w[:, k0:].double().T
+    # fp32 sums of exact products: error below (chunks of 32 + waves) ulp of the sum of magnitudes
+    mag = act[:, k0:].double().abs() @ w[:, k0:].double().abs().T + x.double().abs()
+    assert bool(((got.double() - (x.double() + down)).abs() <= mag * 2.0 ** -23 * 16).all())
+    for b, v in enumerate(lens):
+        if v == 0:
+            assert bool((out[b] == 0).all())
+            continue
+        kb = f(keys[b])
+        want = torch.softmax(f(q[b]) @ kb.T * SCALE, -1) @ kb[:, :512]
+        torch.testing.assert_close(f(out[b]), want, atol=1e-2, rtol=1e-2)
+    apart = f(ol.attn_decode(q, cache, table, klen, g, SCALE, max(max(lens), 1)))
+    torch.testing.assert_close(f(out), apart, atol=2.0 ** -8, rtol=2.0 ** -7)          # two roundings to bfloat16 of nearly equal sums
+    xt = ol.add_linear(octets(act), wt, got, want_copy=True, k=k0)
+    total = x.double() + act.double() @ w.double().T
+    mag += act.double().abs() @ w.double().abs().T
+    assert bool(((got.double() - total).abs() <= mag * 2.0 ** -23 * 16).all())
+    assert torch.equal(xt.permute(1, 0, 2).reshape(rows, n), got.bfloat16())
+
+
+def test_replays_in_a_graph():
+    """Lengths that change between replays: the deal of the splits is made on the device."""
+    from triforce_amd import ops_latent as ol
+    lens = [700, 64, 1, 2000]
+    cache, table, keys = _paged(lens, 512, 64, torch.bfloat16, 6)
+    q = rnd(4, 20, 576, seed=1, dtype=torch.bfloat16)
+    klen = torch.tensor(lens, dtype=torch.int32, device=q.device)
+    act, w, wt, x = _block(4, 4096, 4096, 2048, 9)
+    octs, g = octets(act), Geom(20, 32, 64, 32, 512, 32)
+    plan = (128, 2, 64)
+    keep = torch.zeros_like(x)
+    run = lambda into: ol.attn_decode_beside(q, cache, table, klen, g, SCALE, plan, octs, wt, into, 4096)      # noqa: E731
+    run(keep)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run(keep)
+    for short in ([700, 64, 1, 2000], [1, 0, 1, 1999], [65, 33, 0, 64], [700, 64, 1, 2000]):
+        klen.copy_(torch.tensor(short, dtype=torch.int32))
+        keep.zero_()
+        graph.replay()
+        fresh = torch.zeros_like(x)
+        want = run(fresh)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(keep, fresh)

@@ -60,6 +60,16 @@ def test_bad_arguments_are_refused_before_any_launch():
     assert T.tfl_gemm(ctypes.byref(a), 0, 0, None) == -22
     assert L.tfl_attn_decode(1, 1, 1, 1, 1, 1, 1, None, 0, 1, 1, 48, 32, 1.0, 1, 0, None) == -22        # latent not padded
     assert L.tfl_attn_decode(1, 1, 1, 1, 1, 1, 1, None, 0, 1, 1, 64, 32, 1.0, 4, 0, None) == -28        # no workspace
+    def beside(rows=1, heads=20, splits=8, workers=16, panels=2, ws=1 << 30, **kw):
+        for key, v in dict(dict(rows=rows, n=4096, k=2048, groups=1, chunk_major=1, ld_x=8, x_oct=8, ld_f=4096, out_t=None), **kw).items():
+            setattr(a, key, v)
+        a.wp = a.x = a.out_f = 1 << 20
+        return L.tfl_attn_decode_beside(1, 1, 1, 1, 1, 1, 1, 1, ws, rows, heads, 1.0, splits, workers, panels, ctypes.byref(a), None)
+    assert beside(ws=20 * 8 * 514 - 1) == -28
+    for bad in (dict(rows=33, workers=200), dict(rows=0), dict(heads=16), dict(heads=33), dict(splits=1), dict(splits=129), dict(workers=1),
+                dict(workers=256), dict(panels=1), dict(panels=5), dict(n=4100), dict(k=2056), dict(groups=2), dict(chunk_major=0), dict(ld_x=12),
+                dict(x_oct=4), dict(ld_f=4092), dict(out_t=1 << 20)):
+        assert beside(**bad) == -22, bad
     for rows in (1, 3, 64):
         for heads in (1, 16, 33, 128):
             for n in (1, 64, 5000, 131072):
@@ -85,6 +95,25 @@ def test_decode_splits_by_form():
     assert [splits(rows, 32, 512, 64, 768, 1) for rows in (10, 11, 12, 21, 22)] == [12, 6, 6, 6, 11]
     assert splits(0, 16, 512, 64, 128, 0) == splits(1, 0, 512, 64, 128, 0) == splits(1, 16, 512, 64, 0, 0) == 1
     assert splits(1 << 30, 1 << 20, 512, 64, 1 << 30, 1) == 1
+
+
+def test_plan_of_attention_beside_a_product():
+    """Whatever the sizes: a plan's groups of panels and its workers share 256 CUs, two workers a row at least, splits the kernel takes."""
+    from triforce_amd import ops_latent as ol
+    seen = set()
+    for rows in (0, 1, 5, 8, 17, 32, 33):
+        for heads in (16, 17, 20, 32, 33):
+            for pages in (0, 1, 31, 64, 500, 1500, 2016, 100000, 1 << 21):
+                for n, k in ((4096, 11008), (4096, 2016), (4080, 11008), (8192, 8192), (8208, 8192), (6160, 2080)):
+                    plan = ol.beside_plan(rows, heads, 512, 64, pages, n, k)
+                    if plan is None:
+                        continue
+                    workers, each, splits = plan
+                    assert 1 <= rows <= 32 and 16 < heads <= 32 and 256 <= n // 16 <= 512 and k >= 2048 and 2 <= each <= 4
+                    assert workers >= 2 * rows and workers + -(-n // 16 // each) <= 256 and 2 <= splits <= 128
+                    seen.add((each, n))
+    assert {(2, 4096), (3, 4096), (4, 4096), (4, 8192)} <= seen
+    assert ol.beside_plan(1, 20, 512, 32, 64, 4096, 11008) is None and ol.beside_plan(1, 20, 256, 64, 64, 4096, 11008) is None
 
 
 # ---- configuration and registry -------------------------------------------------------------------------------------------

@@ -10,6 +10,7 @@
 // attn_prefill_sized_kernel), the waves of a workgroup sharing the key / value tile.  Also transposed: the S^T result registers of two 16-key tiles ARE the P operand of
 // one PV product (the value operand is read with the matching key order), so the weights never leave the registers.
 #include "flash_tile.h"
+#include "share_gemm.h"
 
 #define NEG_INF (-__builtin_inff())
 #define LOG2E 1.4426950408889634f
@@ -301,24 +302,16 @@ static int launch_merge(const float* ws, void* out, int rows, int H, int C, int 
 // registers, and accumulates CT / (4 HT) of the latent tiles for all heads.  Two pages in LDS: the next one is written and the one
 // after it requested while the current one is used, so a page costs two barriers and the stream never waits for the arithmetic.
 template <int HT, int WC, int CT>
-__global__ __launch_bounds__(256 * HT, HT) void attn_latent_sized_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache,
-                                                                         int n_pages, const int32_t* __restrict__ table, int table_ld,
-                                                                         const int32_t* __restrict__ len, bf16* __restrict__ out,
-                                                                         float* __restrict__ ws, int H, float scale, int nsplit,
-                                                                         int rows) {
+__device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages,
+                                                       const int32_t* __restrict__ tab, int n, bf16* __restrict__ out,
+                                                       float* __restrict__ ws, int H, float scale, int nsplit, int rows, int row, int h0,
+                                                       int split, int t_beg, int t_end, char* smem) {
     constexpr int NT = 256 * HT, W = 32 * WC, C = 16 * CT, LDK = W + 8, LDP = 64 + 8, NTW = CT / (4 * HT), NPRE = 64 * (W / 8) / NT;
     static_assert(CT % (4 * HT) == 0 && 64 * (W / 8) % NT == 0, "tile split");
-    extern __shared__ __align__(16) char smem[];
     bf16* Kt = (bf16*)smem;                                   // [2][64][LDK]
     bf16* Ps = Kt + 2 * 64 * LDK;                             // [2 (value, remainder)][16 HT][LDP]
     float* red = (float*)(Ps + 2 * 16 * HT * LDP);            // [4][16 HT]
-    const int split = blockIdx.x, h0 = blockIdx.y * 16 * HT, row = blockIdx.z;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, i = lane & 15, ks = wave & 3, ht = wave >> 2;
-    const int n = len[row];
-    const int ntiles = n > 0 ? (n + 63) / 64 : 0;
-    const int per = (ntiles + nsplit - 1) / nsplit;
-    const int t_beg = min(split * per, ntiles), t_end = min(ntiles, t_beg + per);
-    const int32_t* tab = table + (int64_t)row * table_ld;
 
     bf16x8 qf[WC];
     {
@@ -479,6 +472,71 @@ __global__ __launch_bounds__(256 * HT, HT) void attn_latent_sized_kernel(const b
     }
 }
 
+template <int HT, int WC, int CT>
+__global__ __launch_bounds__(256 * HT, HT) void attn_latent_sized_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache,
+                                                                         int n_pages, const int32_t* __restrict__ table, int table_ld,
+                                                                         const int32_t* __restrict__ len, bf16* __restrict__ out,
+                                                                         float* __restrict__ ws, int H, float scale, int nsplit,
+                                                                         int rows) {
+    extern __shared__ __align__(16) char smem[];
+    const int split = blockIdx.x, row = blockIdx.z, n = len[row];
+    const int ntiles = n > 0 ? (n + 63) / 64 : 0;
+    const int per = (ntiles + nsplit - 1) / nsplit;
+    const int t_beg = min(split * per, ntiles), t_end = min(ntiles, t_beg + per);
+    attn_latent_sized_body<HT, WC, CT>(q, cache, n_pages, table + (int64_t)row * table_ld, n, out, ws, H, scale, nsplit, rows, row,
+                                       blockIdx.y * 16 * HT, split, t_beg, t_end, smem);
+}
+
+// The same attention on the first `workers` workgroups, and a product that waits for nothing of it on the others: out_f += x . W^T, P panels of
+// W each.  A workgroup of either kind has a CU to itself (two pages in LDS), so the two share the chip by CUs: attention asks for 30 bytes a ns
+// and CU behind 10 us of start, the product for up to 50.
+// Splits are dealt: as many pages each, 2 at least where a row has more than 16, as make the splits of all rows fit the workers; a row has
+// nsplit at most, with as many pages each as that takes.  Statistics of splits that a row does not have are zero, which the merge skips.
+// us, 20 heads, attention, merge and the output product (shorter by 11 008 of its 15 104), apart -> so: a row of 64 pages 36.6 -> 31.1, 32 rows of 48
+// 61.9 -> 59.9; of a whole step of 48 layer runs, one row of 4 000 keys 4 987 -> 4 668, 32 rows 7 500 -> 7 335.
+template <int P, int MT>
+__global__ __launch_bounds__(512, 2) void attn_latent_beside_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages,
+                                                                    const int32_t* __restrict__ table, int table_ld, const int32_t* __restrict__ len,
+                                                                    float* __restrict__ ws, int H, float scale, int nsplit, int rows, int workers,
+                                                                    const TflGemm g) {
+    extern __shared__ __align__(16) char smem[];
+    if ((int)blockIdx.x >= workers) {
+        share_gemm_body<bf16, TFL_EPI_RESIDUAL, P, false, MT, 2>(g, 0, 0, blockIdx.x - workers, 0, smem);
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    const int pages = lane < rows ? max(1, (len[min(lane, rows - 1)] + 63) >> 6) : 0;        // (a row without keys has one empty split)
+    int total = pages, most = pages;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        total += __shfl_xor(total, o, 64);
+        most = max(most, __shfl_xor(most, o, 64));
+    }
+    int per = max((total + workers - 1) / workers, most > 16 ? 2 : 1), mine, end;
+    for (;; ++per) {                                          // (with `most` pages a split there are as many splits as rows)
+        mine = lane < rows ? min(nsplit, (pages + per - 1) / per) : 0;
+        end = mine;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(end, o, 64);
+            if (lane >= o) end += v;
+        }
+        if (per >= most || __shfl(end, 63, 64) <= workers) break;
+    }
+    const int row = __popcll(__builtin_amdgcn_ballot_w64(end <= (int)blockIdx.x));            // (lanes past the rows end where the last row does)
+    if (row >= rows) return;
+    const int have = __shfl(mine, row, 64), split = (int)blockIdx.x - (__shfl(end, row, 64) - have), n = len[row];
+    const int ntiles = n > 0 ? (n + 63) >> 6 : 0, each = (ntiles + have - 1) / have;
+    const int t_beg = min(split * each, ntiles), t_end = min(ntiles, t_beg + each);
+    if (split == have - 1)
+        for (int s = have + (int)threadIdx.x / 32; s < nsplit; s += 16) {
+            const int head = threadIdx.x & 31;
+            if (head < H) ws[(int64_t)rows * H * nsplit * 512 + (((int64_t)row * H + head) * nsplit + s) * 2 + 1] = 0.f;
+        }
+    attn_latent_sized_body<2, 18, 32>(q, cache, n_pages, table + (int64_t)row * table_ld, n, nullptr, ws, H, scale, nsplit, rows, row, 0, split, t_beg,
+                                      t_end, smem);
+}
+
 #define TFL_MAX_SPLIT 256
 
 extern "C" int64_t tfl_attn_decode_ws_floats(int rows, int H, int C, int nsplit) {
@@ -572,6 +630,75 @@ extern "C" int tfl_attn_decode(const void* q, const void* cache, int n_pages, co
     }
 #undef GO
     return TF_EINVAL;
+}
+
+// How the CUs are shared between the attention of `pages` pages in all and a product of n outputs of k, or 0 workers where the two are better one
+// after the other.  The product takes up to half of the CUs, which draw all that memory gives (48 bytes a ns each).  us of a graph of both and the
+// rest of the output product, 20 heads, n 4096, k 11 008 of 15 104, apart -> beside on 128 CUs | 86 | 64:
+//   pages a row   1           8           16          32                  48                        64                        96
+//    1 row    29.0->30.1  32.7->30.3  32.8->30.7  35.7->30.5|36.9     36.4->31.0|37.7           36.6->31.1|37.7           37.4->31.7|38.1
+//    8 rows   29.9->33.4  34.2->34.3  35.8->36.0  39.0->36.5|43.8     40.3->37.8|44.8           41.5->37.7|45.0           45.1->44.4|46.6|52.1
+//   32 rows   39.1->44.5  46.0->46.7  49.8->47.3  56.3->52.2|55.6     61.9->63.6|59.9|63.3      67.2->75.1|68.7|64.5
+// A row of activations costs both sides 0.3 us (each group of panels reads all of x), a page 3 us of an attention on the whole chip and 2.8 behind 15
+// of one on part of it, a merge of splits 5.
+static int beside_plan(int rows, int H, int64_t pages, int n, int k, int* panels_each) {
+    const int panels = n >> 4;
+    if (rows < 1 || rows > 32 || H <= 16 || H > 32 || pages < 1 || pages > (1 << 20) || panels < 256 || panels > 512 || k < 2048) return 0;
+    const int row = (int)((pages + rows - 1) / rows), ns = tfl_attn_decode_splits(rows, H, 512, 64, row * TFL_PAGE, 0);
+    const double bytes = 2.0 * n * k, x = 0.3 * rows * k / 11008.0;
+    double least = bytes / 6.2e6 + 4.5 + 3.0 * ((row + ns - 1) / ns) + 0.9 * x - (ns == 1 ? 5.0 : 0.0) - 1.5;       // (apart)
+    int workers = 0;
+    for (int p = 2; p <= 4; ++p) {
+        const int g = (panels + p - 1) / p, a = 256 - g;
+        if (g > 128) continue;
+        const double t = fmax(5.0 + bytes / g / 50e3 + x, 15.0 + 2.8 * (double)((pages + a - 1) / a));
+        if (t < least) { least = t; workers = a; *panels_each = p; }
+    }
+    return workers;
+}
+
+extern "C" int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages, int n, int k, int32_t* panels_each, int32_t* nsplit) {
+    if (!panels_each || !nsplit || C != 512 || R != 64) return 0;
+    int p = 0;
+    const int a = beside_plan(rows, H, pages, n, k, &p);
+    *panels_each = p;
+    *nsplit = rows < 1 ? 0 : 2 * a / rows < 128 ? 2 * a / rows : 128;
+    return a;
+}
+
+template <int P, int MT>
+static int launch_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, float* ws, int rows, int H,
+                         float scale, int nsplit, int workers, const TflGemm& g, hipStream_t st) {
+    constexpr int LDS = 2 * 64 * (32 * 18 + 8) * (int)sizeof(bf16) + 2 * 32 * (64 + 8) * (int)sizeof(bf16) + 4 * 32 * (int)sizeof(float);
+    static_assert(LDS <= 160 * 1024 && 8 * P * MT * 64 * (int)sizeof(f32x4) <= LDS, "LDS");
+    const hipError_t e = hipFuncSetAttribute((const void*)attn_latent_beside_kernel<P, MT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL((attn_latent_beside_kernel<P, MT>), dim3(workers + ((g.n >> 4) + P - 1) / P), dim3(512), LDS, st, (const bf16*)q, (const bf16*)cache,
+                       n_pages, table, table_ld, len, ws, H, scale, nsplit, rows, workers, g);
+    TFL_LAUNCH_CHECK();
+    return TF_OK;
+}
+
+extern "C" int tfl_attn_decode_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out,
+                                      float* ws, int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int panels_each,
+                                      const TflGemm* product, void* stream) {
+    if (!q || !cache || !table || !len || !out || !ws || !product || rows < 1 || rows > 32 || H <= 16 || H > 32 || n_pages < 1 || table_ld < 1) return TF_EINVAL;
+    if (nsplit < 2 || nsplit > 128 || workers < 2 * rows || workers > 255) return TF_EINVAL;
+    if (ws_floats < tfl_attn_decode_ws_floats(rows, H, 512, nsplit)) return TF_ENOSPC;
+    const TflGemm g = *product;
+    if (!g.wp || !g.x || !g.out_f || g.out_t || g.rows != rows || g.n < 16 || (g.n & 15) || g.k < 32 || (g.k & 31) || g.groups != 1 || g.chunk_major != 1
+        || (g.ld_x & 7) || g.ld_x < 8 || g.x_oct < 8 || (g.x_oct & 7) || g.ld_f < g.n || (g.ld_f & 3)) return TF_EINVAL;
+    hipStream_t st = (hipStream_t)stream;
+    int rc = TF_EINVAL;
+#define GO(P) rc = rows <= 16 ? launch_beside<P, 1>(q, cache, n_pages, table, table_ld, len, ws, rows, H, scale, nsplit, workers, g, st) \
+                              : launch_beside<P, 2>(q, cache, n_pages, table, table_ld, len, ws, rows, H, scale, nsplit, workers, g, st)
+    switch (panels_each) {
+        case 2: GO(2); break;
+        case 3: GO(3); break;
+        case 4: GO(4); break;
+    }
+#undef GO
+    return rc == TF_OK ? launch_merge<bf16>(ws, out, rows, H, 512, nsplit, st) : rc;
 }
 
 // --------------------------------------------------------------------------------------------------------------- prefill

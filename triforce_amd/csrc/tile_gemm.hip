@@ -15,6 +15,7 @@
 //   GLU       panels of 8 gate | 8 up rows: gelu(gate) * up
 //   F32       the sums themselves
 #include "tile_common.h"
+#include "share_gemm.h"
 
 #ifndef TFL_PAIR_MIN
 #define TFL_PAIR_MIN 420     // panel pairs from which two panels share a workgroup
@@ -223,171 +224,10 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
     }
 }
 
-// What one lane does with four finished outputs n .. n+3 of batch row m (`s`); panel-wide parts (sums of squares, gate | up pairs) are
-// its caller's.
-template <typename T, int EPI>
-__device__ __forceinline__ void finish_quad(const TflGemm& a, int m, int n, f32x4 s) {
-    if constexpr (EPI == TFL_EPI_F32) {
-        float* y = a.out_f + (int64_t)m * a.ld_f + n;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (n + r < a.n_real) y[r] = s[r];
-    } else if constexpr (EPI == TFL_EPI_RESIDUAL) {
-        f32x4* y = reinterpret_cast<f32x4*>(a.out_f + (int64_t)m * a.ld_f + n);
-        f32x4 o = *y;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] += s[r];
-        *y = o;
-        if (a.out_t) store_quad((T*)a.out_t + (int64_t)m * a.ld_t + (n >> 3) * a.t_oct + (n & 7), o);
-    } else {                                                 // IN behind its raw part
-        static_assert(EPI == TFL_EPI_IN, "quad epilogues");
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[r] = gelu_tanh(s[r]);
-        const int k = n - a.n_raw;
-        store_quad((T*)a.out_t + (int64_t)m * a.ld_t + (k >> 3) * a.t_oct + (k & 7), s);
-    }
-}
-
-// IN's raw part: outputs n .. n+3 of a panel that all lanes of the wave hold (g = quad of the panel, i = row).
-template <typename T>
-__device__ __forceinline__ void finish_raw(const TflGemm& a, int m, bool live, int pin, int n, int g, f32x4 s) {
-    float q = s[0] * s[0] + s[1] * s[1] + s[2] * s[2] + s[3] * s[3];
-    q += __shfl_xor(q, 16, 64);
-    q += __shfl_xor(q, 32, 64);
-    if (!live) return;
-    *reinterpret_cast<f32x4*>(a.out_f + (int64_t)m * a.ld_f + n) = s;
-    if (n < a.n_scaled) {
-        const f32x4 w = *reinterpret_cast<const f32x4*>(a.norm_w + n);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[r] *= w[r];
-        store_quad((T*)a.out_t2 + (int64_t)m * 8 + (n >> 3) * (8 * (int64_t)a.rows) + (n & 7), s);
-    }
-    if (g == 0) a.ss_out[(int64_t)m * a.ss_ld + pin] = q;
-}
-
-// The wide outputs: one workgroup per CU, each with P whole panels and tail_per more rows (0, 4, 8 or 12) of what 256 workgroups
-// leave over, over weights packed chunk-major.  Bound by the weight stream.  Three things held the workgroup-per-panel form back:
-//   * a few CUs with one panel more than the rest: 1 028 panels of 4 096 took 1.9 us (1 row) to 6.7 us (32 rows) longer than 1 024.
-//     Here all CUs have the same share to within four rows; the rows left over are MFMA tiles whose upper rows repeat the
-//     last one (the same addresses, no traffic), for gate | up panels dealt in quads of two gate and the same two up rows;
-//   * every workgroup read all of x (256 KB at 32 rows: twice the weights' bytes, from L2) and asked for it right before its use: here
-//     once per CU, and U chunks ahead like the weights;
-//   * one private stream per wave, panels a power of two apart: chunk-major, the chip reads one moving window per wave index.  (The same
-//     kernel on panel-major weights is slower than the old form up to 8 rows: 28.4 us at 1 076 panels.)
-// us before -> now at 1 / 8 / 32 rows, K 4 096: 256 panels 10.5 / 10.4 / 11.9 -> 7.8 / 8.1 / 10.7, 512: 13.9 / 14.8 / 20.5 -> 12.9 / 12.8 /
-// 15.6, 1 076: 27.9 / 29.2 / 39.5 -> 26.1 / 26.3 / 29.2, 1 376: 34.2 / 34.7 / 41.9 -> 31.2 / 31.6 / 34.8, 2 000: 44.6 / 45.9 / 56.5 -> 43.4 /
-// 43.6 / 46.1 (6.0 TB/s); 256 panels of 15 104: 26.9 / 28.7 / 36.5 -> 21.2 / 22.2 / 32.9 (5.8 TB/s).
 template <typename T, int EPI, int P, bool TAIL, int MT, int U>
 __global__ __launch_bounds__(512, 2) void share_gemm_kernel(const TflGemm a, const int tail_rows, const int tail_per) {
-    typedef typename El<T>::Frag Frag;
-    constexpr int WAVES = 8, NP = P + (TAIL ? 1 : 0), CUS = 256;
     extern __shared__ __align__(16) char share_smem[];
-    f32x4 (*part)[NP * MT][64] = reinterpret_cast<f32x4 (*)[NP * MT][64]>(share_smem);
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15;
-    const int npan = a.n >> 4, panel0 = blockIdx.x * P, m0 = blockIdx.y * 16 * MT;
-    const int chunks = a.k >> 5, per = (chunks + WAVES - 1) / WAVES;
-    const int c_beg = wave * per, n_own = min(chunks, c_beg + per) - c_beg;
-    // (the waves' ranges start K/8 chunks apart, a power of two for most K: in step they would ask the same few channels)
-    const int rot = n_own > 0 ? 2 * wave % n_own : 0;
-    const int64_t wstep = (int64_t)npan * 512;               // one chunk of all panels
-    const T* wp[NP];
-#pragma unroll
-    for (int p = 0; p < P; ++p) wp[p] = (const T*)a.wp + min(panel0 + p, npan - 1) * 512 + lane * 8;
-    if constexpr (TAIL) {
-        const int row = min(min((int)blockIdx.x * tail_per + i, (int)blockIdx.x * tail_per + tail_per - 1), tail_rows - 1);
-        int slot = row & 15;
-        if constexpr (EPI == TFL_EPI_GLU) slot = ((slot >> 2) << 1) + (slot & 1) + ((slot & 2) << 2);
-        wp[P] = (const T*)a.wp + (CUS * P + (row >> 4)) * 512 + g * 128 + slot * 8;
-    }
-    const T* xp[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) xp[t] = (const T*)a.x + (int64_t)min(m0 + 16 * t + i, a.rows - 1) * a.ld_x + g * a.x_oct;
-    const int64_t xstep = 4 * a.x_oct;
-    f32x4 acc[NP][MT];
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) acc[p][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto load = [&](Frag (&w)[U][NP], Frag (&x)[U][MT], int c0) {         // (past the end: the last chunk again, not used)
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            int c = min(c0 + u, n_own - 1) + rot;
-            c = c_beg + (c >= n_own ? c - n_own : c);
-#pragma unroll
-            for (int p = 0; p < NP; ++p) w[u][p] = load_frag_stream(wp[p] + wstep * c);
-#pragma unroll
-            for (int t = 0; t < MT; ++t) x[u][t] = load_frag(xp[t] + xstep * c);
-        }
-    };
-    auto multiply = [&](const Frag (&w)[U][NP], const Frag (&x)[U][MT], int c0) {
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (c0 + u < n_own) {
-#pragma unroll
-                for (int p = 0; p < NP; ++p)
-#pragma unroll
-                    for (int t = 0; t < MT; ++t) acc[p][t] = El<T>::mma(w[u][p], x[u][t], acc[p][t]);
-            }
-    };
-    if (n_own > 0) {
-        Frag wa[U][NP], xa[U][MT], wb[U][NP], xb[U][MT];
-        load(wa, xa, 0);
-        for (int c0 = 0; c0 < n_own; c0 += 2 * U) {
-            load(wb, xb, c0 + U);
-            multiply(wa, xa, c0);
-            if (c0 + U >= n_own) break;
-            load(wa, xa, c0 + 2 * U);
-            multiply(wb, xb, c0 + U);
-        }
-    }
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-        for (int t = 0; t < MT; ++t) part[wave][p * MT + t][lane] = acc[p][t];
-    __syncthreads();
-    for (int j = wave; j < NP * MT; j += WAVES) {            // row block t of tile p: the waves' sums, in wave order
-        const int p = j / MT, t = j - p * MT, m = m0 + 16 * t + i;
-        f32x4 s = part[0][j][lane];
-#pragma unroll
-        for (int w = 1; w < WAVES; ++w) {
-            const f32x4 o = part[w][j][lane];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) s[r] += o[r];
-        }
-        const bool live = m < a.rows;
-        if (!TAIL || p < P) {
-            const int panel = panel0 + p, n = 16 * panel + 4 * g;
-            if (panel >= npan) continue;
-            if constexpr (EPI == TFL_EPI_GLU) {              // lanes g < 2 hold gate rows, g + 2 the same outputs' up rows
-                f32x4 up;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(s[r], 32, 64);
-                if (live && g < 2) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) s[r] = gelu_tanh(s[r]) * up[r];
-                    store_quad((T*)a.out_t + (int64_t)m * a.ld_t + panel * a.t_oct + 4 * g, s);
-                }
-            } else {
-                if constexpr (EPI == TFL_EPI_IN) {
-                    if (16 * panel < a.n_raw) {
-                        finish_raw<T>(a, m, live, panel, n, g, s);
-                        continue;
-                    }
-                }
-                if (live) finish_quad<T, EPI>(a, m, n, s);
-            }
-        } else {
-            const int row = blockIdx.x * tail_per + 4 * g;   // first of this lane's four left-over rows
-            if (!live || 4 * g >= tail_per || row >= tail_rows) continue;
-            if constexpr (EPI == TFL_EPI_GLU) {              // gate, gate, up, up of outputs 2q, 2q + 1 of a panel's octet
-                typedef T Pair __attribute__((ext_vector_type(2)));
-                const Pair y = {(T)(gelu_tanh(s[0]) * s[2]), (T)(gelu_tanh(s[1]) * s[3])};
-                *reinterpret_cast<Pair*>((T*)a.out_t + (int64_t)m * a.ld_t + (CUS * P + (row >> 4)) * a.t_oct + ((row & 15) >> 1)) = y;
-            } else {
-                finish_quad<T, EPI>(a, m, 16 * CUS * P + row, s);
-            }
-        }
-    }
+    share_gemm_body<T, EPI, P, TAIL, MT, U>(a, tail_rows, tail_per, blockIdx.x, blockIdx.y, share_smem);
 }
 
 template <typename T, int EPI, int P, bool TAIL, int MT>

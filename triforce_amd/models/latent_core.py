@@ -1,9 +1,9 @@
 """Weights and the per-layer compute of a latent-attention decoder on the HIP ops (ops_latent).
 
 Decode form of a layer (one token per sequence, any number of sequences): ten launches - [norm] [input projections, gelu]
-[query up-projection + cache append] [query to latent] [attention, merge] [latent to value, gate] [output + feed-forward down,
-residual] [token gate] [token projection].  Prefill form: products of many rows (ops_rows) between the row
-kernels and the up-projected attention.
+[query up-projection + cache append] [query to latent] [attention (beside it, on CUs of its own, feed-forward down), merge]
+[latent to value, gate] [output (+ feed-forward down), residual] [token gate] [token projection].  Prefill form: products of many
+rows (ops_rows) between the row kernels and the up-projected attention.
 """
 import zlib
 
@@ -75,9 +75,15 @@ class LatentLayer:
         raw, ss, xq = ol.input_projection(h, self.w_in, g.n_raw, self.q_norm, act, g.H * g.V)
         qn, q = ol.query_and_append(xq, raw, ss, self.w_uq, g, self.kv_norm, eps, rope, batch.pos, batch.slot, cache_rows)
         ol.query_to_latent(qn, self.w_uk_t, q, g)
-        o = ol.attn_decode(q, cache_rows, batch.table, batch.klen, g, self.scale, batch.max_len)
+        own = g.H * g.V                                       # act: the attention's columns, then the feed-forward's, which wait for nothing of it
+        plan = ol.beside_plan(ids.numel(), g.H, g.C, g.R, -(-batch.max_len // ol.PAGE), self.w_out.n, self.w_out.k - own) \
+            if self.ff and self.w_out.chunk_major and h.dtype == torch.bfloat16 else None
+        if plan is None:
+            o = ol.attn_decode(q, cache_rows, batch.table, batch.klen, g, self.scale, batch.max_len)
+        else:
+            o = ol.attn_decode_beside(q, cache_rows, batch.table, batch.klen, g, self.scale, plan, act, self.w_out, x, own)
         ol.latent_to_value(o, self.w_uv, raw, g.gate_off, act, g)
-        xt = ol.add_linear(act, self.w_out, x, want_copy=bool(self.side_dim))
+        xt = ol.add_linear(act, self.w_out, x, want_copy=bool(self.side_dim), k=None if plan is None else own)
         if not self.side_dim:
             return None
         return ol.linear_f32(ol.token_gate_linear(xt, self.side_gate, side_table, ids, self.side_dim), self.side_proj, self.width)

@@ -4,6 +4,9 @@ Same rules as ops.py: torch owns the memory and the stream, every function valid
 gfx950 kernels on torch's current stream; no CPU path exists.  The element type is bfloat16 or float32 and follows the
 tensors.  Call these as ``ops_latent.<name>(...)``.
 """
+import ctypes
+import functools
+
 import torch
 
 from . import hip
@@ -68,14 +71,16 @@ def latent_to_value(ol, wt, raw, gate_off, act, g):
           ld_t=act_ld, t_oct=act_oct)
 
 
-def add_linear(act, wt, x, want_copy=False):
-    """x (fp32) += act . W^T; returns the sum as an octet-major block of act's type when ``want_copy``."""
+def add_linear(act, wt, x, want_copy=False, k=None):
+    """x (fp32) += act . W^T, over the first ``k`` columns of both if given (chunk-major weights); returns the sum as an octet-major
+    block of act's type when ``want_copy``."""
     _need(act, x)
     _f32(x)
-    rows, k, ld, octet = _lay(act)
-    assert act.dtype == wt.dtype and k == wt.k and x.shape == (rows, wt.n) and x.is_contiguous()
+    rows, have, ld, octet = _lay(act)
+    assert act.dtype == wt.dtype and have == wt.k and x.shape == (rows, wt.n) and x.is_contiguous()
+    assert k is None or (wt.chunk_major and 0 < k <= have and k % 32 == 0)
     xt = empty_act(rows, wt.n, wt.dtype, x.device) if want_copy else None
-    _gemm(wt, act, "residual", rows, ld_x=ld, x_oct=octet, out_f=x, ld_f=x.stride(0),
+    _gemm(wt, act, "residual", rows, ld_x=ld, x_oct=octet, out_f=x, ld_f=x.stride(0), k=have if k is None else k,
           **(dict(out_t=xt, ld_t=8, t_oct=8 * rows) if want_copy else {}))
     return xt
 
@@ -185,4 +190,36 @@ def attn_decode(q, cache, table, klen, g, scale, max_len, nsplit=None):
     out = torch.empty(rows, g.H, g.C, dtype=q.dtype, device=q.device)
     hip.check(L.tfl_attn_decode(_p(q), _p(cache), cache.shape[0] // PAGE, _p(table), table.stride(0), _p(klen), _p(out), _p(ws), n_ws,
                                 rows, g.H, g.C, g.R, float(scale), nsplit, _CODE[q.dtype], _stream()), "tfl_attn_decode")
+    return out
+
+
+@functools.lru_cache(maxsize=1024)
+def beside_plan(rows, H, C, R, pages, n, k):
+    """(workers, panels each, splits) of attn_decode_beside for rows with ``pages`` pages in all and a product of n outputs of k, None where the
+    two are better launched apart."""
+    each, nsplit = ctypes.c_int32(), ctypes.c_int32()
+    workers = hip.latent_lib().tfl_attn_beside_plan(rows, H, C, R, pages, n, k, ctypes.byref(each), ctypes.byref(nsplit))
+    return (workers, each.value, nsplit.value) if workers > 0 else None
+
+
+def attn_decode_beside(q, cache, table, klen, g, scale, plan, act, wt, x, k0):
+    """attn_decode of bfloat16 rows of 512 + 64 with x += act . W^T over the columns from k0 on in the same launch."""
+    _need(q, cache, table, klen, act, x)
+    _i32(table, klen)
+    _f32(x)
+    rows, (workers, each, nsplit) = q.shape[0], plan
+    assert q.dtype == cache.dtype == act.dtype == wt.dtype == torch.bfloat16 and q.is_contiguous() and q.shape[1:] == (g.H, 576) and (g.C, g.R) == (512, 64)
+    assert cache.is_contiguous() and cache.shape[1] == 576 and cache.shape[0] % PAGE == 0
+    assert table.shape[0] == rows and table.stride(1) == 1 and klen.numel() == rows
+    assert act.dim() == 3 and act.is_contiguous() and act.shape[:2] == (wt.k // 8, rows) and x.shape == (rows, wt.n) and x.is_contiguous()
+    assert wt.chunk_major and 0 <= k0 < wt.k and k0 % 32 == 0
+    L = hip.latent_lib()
+    ws = torch.empty(L.tfl_attn_decode_ws_floats(rows, g.H, g.C, nsplit), dtype=torch.float32, device=q.device)
+    out = torch.empty(rows, g.H, g.C, dtype=q.dtype, device=q.device)
+    a = hip.TflGemm()
+    a.wp, a.x, a.out_f = wt.packed.data_ptr() + 2 * k0 * wt.n, act[k0 // 8:].data_ptr(), x.data_ptr()
+    a.rows, a.n, a.k, a.groups, a.chunk_major, a.ld_f = rows, wt.n, wt.k - k0, 1, 1, x.stride(0)
+    a.ld_x, a.x_oct, a.t_oct = 8, 8 * rows, 8
+    hip.check(L.tfl_attn_decode_beside(_p(q), _p(cache), cache.shape[0] // PAGE, _p(table), table.stride(0), _p(klen), _p(out), _p(ws), ws.numel(), rows, g.H,
+                                       float(scale), nsplit, workers, each, ctypes.byref(a), _stream()), "tfl_attn_decode_beside")
     return out
