@@ -427,6 +427,27 @@ def test_split_float32_product(rows, n, k, splits):
         assert err.max() <= 2.0 ** -24 * (6 * k / 32) ** 0.5 + 2.0 ** -22
 
 
+# more tiles than CUs: whole rounds of whole tiles and the steps of the others shared by an XCD's CUs; k of no whole eights of steps, ragged last
+# tiles, XCDs with one shared tile and with none, few sharers
+@pytest.mark.parametrize("rows,n,k", [(1040, 7680, 1024), (1100, 7664, 1056), (700, 12320, 1536), (896, 9472, 2048), (2050, 4112, 4064)])
+def test_split_float32_shared_tiles(rows, n, k):
+    from triforce_amd import hip
+    from triforce_amd import ops_tile as ot
+    size_of = hip.tile_lib().tfl_split_gemm_ws_floats
+    assert size_of(rows, n, k, 0) not in [size_of(rows, n, k, s) for s in range(1, 9)]
+    g = torch.Generator(device=DEV).manual_seed(rows + n)
+    x, w = torch.randn(rows, k, generator=g, device=DEV), torch.randn(n, k, generator=g, device=DEV)
+    want, size = x.double() @ w.double().T, x.double().norm() * w.double().norm(dim=1) / k ** 0.5
+    got = ot.split_linear(x, w)
+    assert ((got.double() - want).norm(dim=0) / size).max() <= 2.0 ** -24 * (6 * k / 32) ** 0.5 + 2.0 ** -22         # (as above)
+    assert ((got.double() - want).abs() / (x.double().abs() @ w.double().abs().T)).max() <= 5 * 2.0 ** -24 * (1 + (k / 32 / 3) ** 0.5)
+    assert torch.equal(got, ot.split_linear(x, w))
+    x[rows - 1, 5], x[3, k - 1], w[n - 1, k // 2] = float("inf"), float("nan"), -float("inf")
+    got, plain = ot.split_linear(x, w), ot.split_linear(x, w, 1)
+    assert torch.equal(torch.isnan(got), torch.isnan(plain)) and torch.equal(got[torch.isinf(plain)], plain[torch.isinf(plain)])
+    assert torch.isfinite(got[torch.isfinite(plain)]).all()
+
+
 # products that stand alone (a row of x with one entry): every bit of both factors counts, in every place of a step of 32
 @pytest.mark.parametrize("splits", [1, 2])
 def test_split_float32_single_products(splits):

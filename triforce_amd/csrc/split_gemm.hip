@@ -22,7 +22,7 @@
 // products instead of behind them waits for x's DMA before each store to LDS: 22 016 x 4 096 at 2 048 rows 1 830 -> 2 230 us.)
 //
 // Bound by the power of the matrix cores (1.6 to 1.7 GHz under these products, as bf16 GEMMs) and by rounds of tiles.  fp32 GEMM before ->
-// now, x's cut and the sum of parts included: 700 rows, 22 016 x 4 096 940 -> 750 us, 18 784 x 4 096 900 -> 590, 4 096 x 15 104 680 -> 460;
+// now, x's cut and the sum of parts included: 700 rows, 22 016 x 4 096 940 -> 635 us, 18 784 x 4 096 900 -> 570, 4 096 x 15 104 680 -> 460;
 // 2 048 rows, 22 016 x 4 096 2 600 -> 1 800 (205 TFLOP/s).
 //
 // Range: both operands are cut at 2^24 times their value, so the last bit of the smallest float32 (2^-149) is still a normal bfloat16 and no
@@ -94,11 +94,36 @@ struct SplitGemm {
     const bf16* xp;
     const float* x;
     float* out;
-    float* ws;                                                // [splits][rows][n]
+    float* ws;                                                // [8 XCDs][slots][128 rows][256 outputs]
     const int32_t* nans;
     int64_t ld_x, ld_out;
-    int rows, n, k, splits;
+    int rows, n, k;
+    int whole, splits, sharers, slots;                        // see Share; slots of an XCD
 };
+
+// An XCD's tiles (an eighth of all): the first `whole` of them have a workgroup each.  The steps of the others stand in a line, which is cut among
+// the XCD's `sharers` evenly, at eights of steps, or, without sharers, tile by tile into `splits` parts.  A sharer has a part of one tile or of
+// two; the parts in their order along the line are numbered by sharer + tile, the slots of ws by part.
+struct Share {
+    int first, own, rest, sharers, chunks, parts;             // of one XCD: its tiles, those of one workgroup, the others, who shares them; parts of a tile or 0
+    __device__ __forceinline__ int cut(int q) const {         // (32 sharers of up to 2^24 steps)
+        const uint32_t s = q, n = sharers, p = parts;
+        if (parts) return (int)(s / p * chunks + s % p * chunks / p);
+        return s < n ? (int)(s * (uint32_t)(rest * chunks) / n & ~7u) : rest * chunks;
+    }
+};
+__device__ __forceinline__ Share share_of(int tiles, int chunks, int whole, int splits, int sharers, int xcd) {
+    const int first = (int)((int64_t)tiles * xcd >> 3), all = (int)((int64_t)tiles * (xcd + 1) >> 3) - first, own = min(all, whole), rest = all - own;
+    const int parts = min(splits, chunks);                    // (a step at least to each part, an eight to each sharer)
+    return Share{first, own, rest, sharers > 0 ? min(sharers, rest * chunks >> 3) : rest * parts, chunks, sharers > 0 ? 0 : parts};
+}
+constexpr int SLOT = 128 * 256;                               // floats of a part in ws
+static int split_tiles(int rows, int n) { return (n + 255) / 256 * ((rows + 127) / 128); }
+// Slots of an XCD.
+static int split_slots(int tiles, int whole, int splits, int sharers) {
+    const int rest = (tiles + 7) / 8 - whole;
+    return rest > 0 ? (sharers > 0 ? sharers : rest * splits) + rest - 1 : 0;
+}
 
 __host__ __device__ __forceinline__ int split_parts(int k) { return (k + SPLIT_KC - 1) / SPLIT_KC; }
 
@@ -151,21 +176,19 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
     const int wn = wave & 3, wm = wave >> 2, chunks = a.k >> 5;
     // workgroups go round-robin over the 8 XCDs: each takes an eighth of the tiles, the row tiles of one column tile one after the other, which
     // share its weights in L2
-    const int mts = (a.rows + 32 * MT - 1) / (32 * MT), tiles_all = (a.n + 255) / 256 * mts, xcd = blockIdx.x & 7;
-    const int id = (int)((int64_t)tiles_all * xcd >> 3) + (blockIdx.x >> 3);
-    if (id >= (int)((int64_t)tiles_all * (xcd + 1) >> 3)) return;
-    const int nt = id / mts, mt0 = id % mts;
-    const int per = (chunks + a.splits - 1) / a.splits, c_beg = blockIdx.y * per, c_end = min(chunks, c_beg + per);
+    const int mts = (a.rows + 32 * MT - 1) / (32 * MT), xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const Share share = share_of((a.n + 255) / 256 * mts, chunks, a.whole, a.splits, a.sharers, xcd);
+    int q = j - share.own;
+    if (q >= share.sharers) return;
+    if (q >= 0 && a.sharers == 0) q = q % share.rest * share.parts + q / share.rest;     // (the same part of all tiles together)
+    int beg = 0, end = chunks;                                // of the line of shared tiles, or of this workgroup's own tile
+    if (q >= 0) {
+        beg = share.cut(q);
+        end = share.cut(q + 1);
+    }
     const int xpan = (a.rows + 15) >> 4;
     const bf16* src[PER];                                     // this wave's fragments of x: scalar pointers to their first chunk
-#pragma unroll
-    for (int f = 0; f < PER; ++f) {
-        const int p = (wave * PER + f) / 3, z = (wave * PER + f) % 3;
-        src[f] = a.xp + (int64_t)min(mt0 * XP + p, xpan - 1) * chunks * 1536 + z * 512;
-    }
     const float* wsrc[2];                                     // this lane's eight weights of two panels
-#pragma unroll
-    for (int f = 0; f < 2; ++f) wsrc[f] = a.w + (int64_t)min(nt * 256 + 16 * (wave + 8 * f) + i, a.n - 1) * a.k + 8 * g;
     f32x4 staged[2][2];
     auto fetch_x = [&](int c, int buf) {
 #pragma unroll
@@ -192,6 +215,16 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    do {
+    const int r = beg / chunks, c_beg = beg - r * chunks, c_end = min(chunks, c_beg + end - beg), id = share.first + (q < 0 ? j : share.own + r);
+    const int nt = id / mts, mt0 = id % mts;
+#pragma unroll
+    for (int f = 0; f < PER; ++f) {
+        const int p = (wave * PER + f) / 3, z = (wave * PER + f) % 3;
+        src[f] = a.xp + (int64_t)min(mt0 * XP + p, xpan - 1) * chunks * 1536 + z * 512;
+    }
+#pragma unroll
+    for (int f = 0; f < 2; ++f) wsrc[f] = a.w + (int64_t)min(nt * 256 + 16 * (wave + 8 * f) + i, a.n - 1) * a.k + 8 * g;
     const bool live = mt0 * XP + wm * MT < xpan;              // a wave without rows leaves the matrix core to its neighbour
     f32x4 acc[4][MT], low[4][MT];                             // hh and the five small products
 #pragma unroll
@@ -237,34 +270,51 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
         fetch_w(min(c + 2, c_end - 1));
         meet();
     }
-    float* y = a.splits > 1 ? a.ws + (int64_t)blockIdx.y * a.rows * a.n : a.out;
-    const int64_t ld = a.splits > 1 ? a.n : a.ld_out;
+    // a part goes to its slot, a row of 256 behind the other
+    float* part = q < 0 ? nullptr : a.ws + ((int64_t)xcd * a.slots + q + r) * SLOT;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        const int row0 = mt0 * 32 * MT + 16 * (wm * MT + m);
+        const int in_row = 16 * (wm * MT + m), row0 = mt0 * 32 * MT + in_row;
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const int n0 = nt * 256 + 64 * wn + 16 * t;
+            const int in_n = 64 * wn + 16 * t, n0 = nt * 256 + in_n;
             if (row0 >= a.rows || n0 >= a.n) continue;
             f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE));
-            if (a.splits == 1) mend(a, row0, n0, v);
-            if (row0 + i < a.rows) *reinterpret_cast<f32x4*>(y + (int64_t)(row0 + i) * ld + n0 + 4 * g) = v;
+            if (part) {
+                *reinterpret_cast<f32x4*>(part + 256 * (in_row + i) + in_n + 4 * g) = v;
+            } else {
+                mend(a, row0, n0, v);
+                if (row0 + i < a.rows) *reinterpret_cast<f32x4*>(a.out + (int64_t)(row0 + i) * a.ld_out + n0 + 4 * g) = v;
+            }
         }
     }
+    beg += c_end - c_beg;
+    } while (beg < end);
 }
 
-// The parts of a split k, summed in order: a wave takes a 16 x 16 tile, a workgroup four side by side.
+// The parts of shared tiles, summed in order: a wave takes a 16 x 16 tile, a workgroup four side by side.
 __global__ __launch_bounds__(256) void split_sum_kernel(const SplitGemm a) {
-    const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15, cols = (a.n + 63) >> 6;
-    const int row0 = 16 * (int)(blockIdx.x / cols), n0 = 64 * (int)(blockIdx.x % cols) + 16 * (threadIdx.x >> 6);
-    if (n0 >= a.n) return;
-    const int64_t at = (int64_t)min(row0 + i, a.rows - 1) * a.n + n0 + 4 * g;
+    const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15, mts = (a.rows + 127) / 128, tiles = (a.n + 255) / 256 * mts;
+    const int xcd = blockIdx.x & 7, r = blockIdx.x >> 8, at = blockIdx.x >> 3 & 31;          // (32 pieces of a tile)
+    const Share share = share_of(tiles, a.k >> 5, a.whole, a.splits, a.sharers, xcd);
+    if (r >= share.rest) return;
+    const int id = share.first + share.own + r, in_row = 16 * (at >> 2), in_n = 64 * (at & 3) + 16 * (threadIdx.x >> 6);
+    const int row0 = id % mts * 128 + in_row, n0 = id / mts * 256 + in_n;
+    if (row0 >= a.rows || n0 >= a.n) return;
+    int q = r * share.parts, parts = share.parts;
+    if (!parts) {
+        q = r * share.sharers / share.rest;                   // its first part begins in it, or reaches into it from the tile before
+        while (q > 0 && share.cut(q) > r * share.chunks) --q;
+        while (share.cut(q + 1) <= r * share.chunks) ++q;
+        for (parts = 1; q + parts < share.sharers && share.cut(q + parts) < (r + 1) * share.chunks;) ++parts;
+    }
+    const float* src = a.ws + ((int64_t)xcd * a.slots + q + r) * SLOT + 256 * (in_row + i) + in_n + 4 * g;
     f32x4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-    for (int z = 0; z < a.splits; ++z) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(a.ws + (int64_t)z * a.rows * a.n + at);
+    for (int z = 0; z < parts; ++z) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(src + (int64_t)z * SLOT);
 #pragma unroll
         for (int e = 0; e < 4; ++e) s[e] += v[e];
     }
@@ -276,11 +326,11 @@ static int launch_split_gemm(const SplitGemm& a, hipStream_t st) {
     constexpr int LDS = 2 * 3 * (16 + 8) * 1024;              // two buffers of 16 panels of weights and 8 of x, in three parts
     const hipError_t e = hipFuncSetAttribute((const void*)split_gemm_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e != hipSuccess) return (int)e;
-    const int tiles = (a.n + 255) / 256 * ((a.rows + 127) / 128);
-    hipLaunchKernelGGL(split_gemm_kernel, dim3((tiles + 7) / 8 * 8, a.splits), dim3(512), LDS, st, a);
+    const int each = (split_tiles(a.rows, a.n) + 7) / 8, own = each < a.whole ? each : a.whole, rest = each - own;
+    hipLaunchKernelGGL(split_gemm_kernel, dim3(8 * (own + (rest == 0 ? 0 : a.sharers > 0 ? a.sharers : rest * a.splits))), dim3(512), LDS, st, a);
     TFL_LAUNCH_CHECK();
-    if (a.splits > 1) {
-        hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)((int64_t)((a.rows + 15) / 16) * ((a.n + 63) / 64))), dim3(256), 0, st, a);
+    if (rest > 0) {
+        hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)rest * 256), dim3(256), 0, st, a);
         TFL_LAUNCH_CHECK();
     }
     return TF_OK;
@@ -290,25 +340,45 @@ static int launch_split_gemm(const SplitGemm& a, hipStream_t st) {
 static int64_t split_planes(int rows, int k) { return (int64_t)((rows + 15) / 16) * (k / 32) * 1536 * 2 / 4; }
 static int64_t split_marks(int rows, int k) { return ((int64_t)rows * split_parts(k) + 3) / 4 * 4; }
 
-// Parts of k: rounds of workgroups, each with the fill of its pipe (4 steps of 32), against what the parts cost on their way through memory
+struct Parts { int whole, splits, sharers; };
+
+// How k is cut: rounds of workgroups, each with the fill of its pipe (4 steps of 32), against what the parts cost on their way through memory
 // (a written and read 128 x 256 part as much as 8 steps).  Rounds are an XCD's: it has 32 CUs and its eighth of the tiles, rounded up (36 tiles in
 // seven parts are 252 workgroups, but 35 on some XCDs: 700 rows, 1 536 x 6 144 in seven 119 us, in six 95).  256 rows, 12 320 x 4 096: 267 us
 // without parts, 159 with two, 171 with four; 700 rows, 4 096 x 8 192: 514, 296 with two, 262 with five, 265 with eight.
-static int pick_parts(int rows, int n, int k) {
-    const int64_t tiles = (int64_t)((n + 255) / 256) * ((rows + 127) / 128), per_xcd = (tiles + 7) / 8;
-    int best = 1;
+// From 32 tiles an XCD on: whole rounds of whole tiles, and the steps of the others shared by all CUs, 8 or more to each.  A last round of few tiles,
+// or parts of all tiles instead (516 tiles of 22 016 x 4 096 at 700 rows in two parts, 2.5 rounds and 250 MB of parts): 755 -> 635 us; 12 320
+// outputs 425 -> 375, 300 rows of 22 016 400 -> 335, 1 000 rows of 18 784 805 -> 750.  Below, sharing gains nothing over whole tiles on fewer
+// CUs, which run at a higher clock (256 rows of 22 016, 172 tiles: 317 us alone, 327 shared).
+static Parts pick_parts(int rows, int n, int k) {
+    const int tiles = split_tiles(rows, n), per_xcd = (tiles + 7) / 8;
+    const double chunks = k / 32;
+    Parts best{0, 1, 0};
     double least = 0;
     for (int s = 1; s <= 8 && (s == 1 || s * 512 <= k); ++s) {
-        const double t = (double)((per_xcd * s + 31) / 32) * (1.0 / s + 4.0 / (k / 32)) + (s > 1 ? 8.0 * (double)s * tiles / 256 / (k / 32) : 0);
-        if (s == 1 || t < least) { best = s; least = t; }
+        const double t = (double)(((int64_t)per_xcd * s + 31) / 32) * (1.0 / s + 4.0 / chunks) + (s > 1 ? 8.0 * (double)s * tiles / 256 / chunks : 0);
+        if (s == 1 || t < least) { best.splits = s; least = t; }
     }
+    for (int w = per_xcd >> 5; w > 0 && w >= (per_xcd >> 5) - 1; --w) {
+        const int rest = per_xcd - 32 * w;
+        const int64_t line = (int64_t)rest * (k / 32);
+        if (rest == 0 || line < 16 || line > 1 << 24) continue;
+        const int sharers = (int)(line / 8 < 32 ? line / 8 : 32);
+        const double t = w * (1.0 + 4.0 / chunks) + rest / (double)sharers + (rest > 1 ? 8.0 : 4.0) / chunks + 8.0 * (sharers + rest) / 32 / chunks + 3.0 / chunks;
+        if (t < least) { best = Parts{32 * w, 1, sharers}; least = t; }
+    }
+    if (best.sharers == 0 && best.splits == 1) best.whole = 1 << 28;
     return best;
+}
+
+static Parts given_parts(int rows, int n, int k, int splits) {
+    return splits == 0 ? pick_parts(rows, n, k) : Parts{splits == 1 ? 1 << 28 : 0, splits, 0};
 }
 
 extern "C" int64_t tfl_split_gemm_ws_floats(int rows, int n, int k, int splits) {
     if (rows < 1 || rows > (1 << 24) || n < 16 || k < 32 || splits < 0 || splits > 64) return 0;
-    if (splits == 0) splits = pick_parts(rows, n, k);
-    return split_planes(rows, k) + split_marks(rows, k) + (splits > 1 ? (int64_t)splits * rows * n : 0);
+    const Parts p = given_parts(rows, n, k, splits);
+    return split_planes(rows, k) + split_marks(rows, k) + (int64_t)8 * split_slots(split_tiles(rows, n), p.whole, p.splits, p.sharers) * SLOT;
 }
 
 extern "C" int tfl_split_gemm(const float* w, const float* x, int64_t ld_x, float* out, int64_t ld_out, float* ws, int64_t ws_floats, int rows, int n,
@@ -316,11 +386,12 @@ extern "C" int tfl_split_gemm(const float* w, const float* x, int64_t ld_x, floa
     if (!w || !x || !out || !ws || rows < 1 || rows > (1 << 24) || n < 16 || (n & 15) || k < 32 || (k & 31) || ld_x < k || (ld_x & 3) || ld_out < n
         || (ld_out & 3) || splits < 0 || splits > 64) return TF_EINVAL;
     if (((uintptr_t)w | (uintptr_t)x | (uintptr_t)out | (uintptr_t)ws) & 15) return TF_EINVAL;
-    if (splits == 0) splits = pick_parts(rows, n, k);
+    const Parts p = given_parts(rows, n, k, splits);
     if (ws_floats < tfl_split_gemm_ws_floats(rows, n, k, splits)) return TF_ENOSPC;
     int32_t* nans = (int32_t*)(ws + split_planes(rows, k));
     hipLaunchKernelGGL(split_rows_kernel, dim3((rows + 15) / 16, split_parts(k)), dim3(256), 0, (hipStream_t)stream, x, ld_x, rows, k, (bf16*)ws, nans);
     TFL_LAUNCH_CHECK();
-    const SplitGemm a = {w, (const bf16*)ws, x, out, ws + split_planes(rows, k) + split_marks(rows, k), nans, ld_x, ld_out, rows, n, k, splits};
+    const SplitGemm a = {w, (const bf16*)ws, x, out, ws + split_planes(rows, k) + split_marks(rows, k), nans, ld_x, ld_out, rows, n, k, p.whole, p.splits, p.sharers,
+                         split_slots(split_tiles(rows, n), p.whole, p.splits, p.sharers)};
     return launch_split_gemm(a, (hipStream_t)stream);
 }
