@@ -68,10 +68,14 @@ int tfl_attn_decode(const void* q, const void* cache, int n_pages, const int32_t
 /* The same for bfloat16 rows of 512 + 64, 17 to 32 heads and up to 32 rows, with a product in the same launch that needs nothing of it:
  * product->out_f += x . W^T (TFL_EPI_RESIDUAL without out_t, chunk-major weights; include/triforce_tile.h).  workers CUs do the attention, its
  * splits dealt over the rows' pages (at most nsplit, 2 .. 128, of a row); the others take panels_each panels (2 .. 4) of the product.
- * tfl_attn_beside_plan: workers, panels_each and nsplit for rows with `pages` pages in all, 0 where the two are better launched apart. */
-int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages, int n, int k, int32_t* panels_each, int32_t* nsplit);
+ * out NULL: the splits stay in ws, for tfl_latent_value.
+ * tfl_attn_beside_plan: workers, panels_each and nsplit for rows with `pages` pages in all, 0 where the two are better launched apart; parts: how
+ * many splits all rows have together. */
+int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages, int n, int k, int32_t* panels_each, int32_t* nsplit, int32_t* parts);
 int tfl_attn_decode_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out, float* ws,
                            int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int panels_each, const TflGemm* product, void* stream);
+/* TFL_EPI_GATED in bfloat16 (include/triforce_tile.h; k 512, up to 4 rows) of what the splits in ws merge to: product->x is not read. */
+int tfl_latent_value(const float* ws, int64_t ws_floats, int nsplit, const TflGemm* product, void* stream);
 
 #ifdef __cplusplus
 }

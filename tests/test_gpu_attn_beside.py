@@ -38,7 +38,7 @@ def test_attention_beside_a_product(lens, heads, n, k0, k, plan):
     g = Geom(heads, 32, 64, 32, 512, 32)
     plan = plan or (128, 2, max(2, min(128, 256 // rows)))
     got = x.clone()
-    out = ol.attn_decode_beside(q, cache, table, klen, g, SCALE, plan, octets(act), wt, got, k0)
+    out = ol.attn_decode_beside(q, cache, table, klen, g, SCALE, plan + (False,), octets(act), wt, got, k0)
     down = act[:, k0:].double() @ w[:, k0:].double().T
     # fp32 sums of exact products: error below (chunks of 32 + waves) ulp of the sum of magnitudes
     mag = act[:, k0:].double().abs() @ w[:, k0:].double().abs().T + x.double().abs()
@@ -59,6 +59,33 @@ def test_attention_beside_a_product(lens, heads, n, k0, k, plan):
     assert torch.equal(xt.permute(1, 0, 2).reshape(rows, n), got.bfloat16())
 
 
+# as many splits as the kernel takes, rows of one and of none beside them, an odd number of rows; V of one panel and of eight
+@pytest.mark.parametrize("lens,heads,V,plan", [([4000], 20, 128, (128, 2, 128)), ([0], 17, 16, (128, 2, 128)), ([130, 0, 1, 700], 20, 48, (128, 2, 64)),
+                                               ([8000], 32, 128, (128, 2, 128)), ([65] * 4, 20, 128, (8, 3, 2)), ([3000, 2500, 7], 20, 128, (170, 3, 113))])
+def test_value_of_unmerged_splits(lens, heads, V, plan):
+    from triforce_amd import ops_latent as ol
+    rows = len(lens)
+    cache, table, keys = _paged(lens, 512, 64, torch.bfloat16, 5)
+    q = rnd(rows, heads, 576, seed=1, dtype=torch.bfloat16)
+    klen = torch.tensor(lens, dtype=torch.int32, device=q.device)
+    act, w, wt, x = _block(rows, 4096, 32, 2048, 7)
+    g = Geom(heads, 32, 64, V, 512, 32)
+    raw, w_uv = rnd(rows, heads * V + 16, seed=3), rnd(heads, V, 512, seed=4, dtype=torch.bfloat16, scale=512 ** -0.5)
+    value = ol.TileWeight(w_uv, packed_only=True)
+    got, want = ol.empty_act(rows, heads * V, torch.bfloat16, q.device), ol.empty_act(rows, heads * V, torch.bfloat16, q.device)
+    splits = ol.attn_decode_beside(q, cache, table, klen, g, SCALE, plan + (True,), octets(act), wt, x.clone(), 32)
+    ol.latent_to_value(splits, value, raw, 16, got, g)
+    merged = ol.attn_decode_beside(q, cache, table, klen, g, SCALE, plan + (False,), octets(act), wt, x.clone(), 32)
+    ol.latent_to_value(merged, value, raw, 16, want, g)
+    flat, gate = (f(t.permute(1, 0, 2).reshape(rows, heads, V)) for t in (got, want)), torch.sigmoid(raw[:, 16:]).view(rows, heads, V)
+    got, want = flat
+    exact = torch.einsum("rhc,hvc->rhv", f(merged), f(w_uv)) * gate
+    size = torch.einsum("rhc,hvc->rhv", f(merged).abs(), f(w_uv).abs()) * gate
+    # the merged row is rounded to bfloat16 either way, from sums in another order (now and then to the neighbour, 2^-8 of an entry), and the result
+    assert ((got - exact).abs() <= 2.0 ** -8 * exact.abs() + 2.0 ** -8 * size / 8 + 1e-6).all()
+    assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * size / 8 + 1e-6).all()
+
+
 def test_replays_in_a_graph():
     """Lengths that change between replays: the deal of the splits is made on the device."""
     from triforce_amd import ops_latent as ol
@@ -68,7 +95,7 @@ def test_replays_in_a_graph():
     klen = torch.tensor(lens, dtype=torch.int32, device=q.device)
     act, w, wt, x = _block(4, 4096, 4096, 2048, 9)
     octs, g = octets(act), Geom(20, 32, 64, 32, 512, 32)
-    plan = (128, 2, 64)
+    plan = (128, 2, 64, False)
     keep = torch.zeros_like(x)
     run = lambda into: ol.attn_decode_beside(q, cache, table, klen, g, SCALE, plan, octs, wt, into, 4096)      # noqa: E731
     run(keep)

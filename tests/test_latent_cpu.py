@@ -70,6 +70,15 @@ def test_bad_arguments_are_refused_before_any_launch():
                 dict(workers=256), dict(panels=1), dict(panels=5), dict(n=4100), dict(k=2056), dict(groups=2), dict(chunk_major=0), dict(ld_x=12),
                 dict(x_oct=4), dict(ld_f=4092), dict(out_t=1 << 20)):
         assert beside(**bad) == -22, bad
+    def value(splits=8, ws=1 << 30, **kw):
+        for key, v in dict(dict(rows=1, n=128, k=512, groups=20, chunk_major=0, ld_t=8, t_oct=8, ld_gate=2560), **kw).items():
+            setattr(a, key, v)
+        a.wp = a.gate = a.out_t = 1 << 20
+        return L.tfl_latent_value(1, ws, splits, ctypes.byref(a), None)
+    assert value(ws=20 * 8 * 514 - 1) == -28
+    for bad in (dict(rows=5), dict(rows=0), dict(splits=1), dict(splits=129), dict(k=480), dict(n=24), dict(groups=0), dict(chunk_major=1), dict(ld_t=4),
+                dict(t_oct=4), dict(ld_gate=2558), dict(ld_gate=2552)):
+        assert value(**bad) == -22, bad
     for rows in (1, 3, 64):
         for heads in (1, 16, 33, 128):
             for n in (1, 64, 5000, 131072):
@@ -108,7 +117,8 @@ def test_plan_of_attention_beside_a_product():
                     plan = ol.beside_plan(rows, heads, 512, 64, pages, n, k)
                     if plan is None:
                         continue
-                    workers, each, splits = plan
+                    workers, each, splits, later = plan
+                    assert not later or rows <= 4
                     assert 1 <= rows <= 32 and 16 < heads <= 32 and 256 <= n // 16 <= 512 and k >= 2048 and 2 <= each <= 4
                     assert workers >= 2 * rows and workers + -(-n // 16 // each) <= 256 and 2 <= splits <= 128
                     seen.add((each, n))

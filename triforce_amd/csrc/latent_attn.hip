@@ -657,12 +657,17 @@ static int beside_plan(int rows, int H, int64_t pages, int n, int k, int* panels
     return workers;
 }
 
-extern "C" int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages, int n, int k, int32_t* panels_each, int32_t* nsplit) {
-    if (!panels_each || !nsplit || C != 512 || R != 64) return 0;
+extern "C" int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages, int n, int k, int32_t* panels_each, int32_t* nsplit, int32_t* parts) {
+    if (!panels_each || !nsplit || !parts || C != 512 || R != 64) return 0;
     int p = 0;
     const int a = beside_plan(rows, H, pages, n, k, &p);
     *panels_each = p;
     *nsplit = rows < 1 ? 0 : 2 * a / rows < 128 ? 2 * a / rows : 128;
+    *parts = 0;
+    if (a > 0) {                                              // (as the kernel deals them when all rows have as many pages)
+        const int64_t per = (pages + a - 1) / a, least = pages > 16 * rows ? 2 : 1, all = (pages + rows) / (per > least ? per : least) + rows;
+        *parts = (int32_t)(all < a ? all : a);
+    }
     return a;
 }
 
@@ -682,7 +687,7 @@ static int launch_beside(const void* q, const void* cache, int n_pages, const in
 extern "C" int tfl_attn_decode_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out,
                                       float* ws, int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int panels_each,
                                       const TflGemm* product, void* stream) {
-    if (!q || !cache || !table || !len || !out || !ws || !product || rows < 1 || rows > 32 || H <= 16 || H > 32 || n_pages < 1 || table_ld < 1) return TF_EINVAL;
+    if (!q || !cache || !table || !len || !ws || !product || rows < 1 || rows > 32 || H <= 16 || H > 32 || n_pages < 1 || table_ld < 1) return TF_EINVAL;
     if (nsplit < 2 || nsplit > 128 || workers < 2 * rows || workers > 255) return TF_EINVAL;
     if (ws_floats < tfl_attn_decode_ws_floats(rows, H, 512, nsplit)) return TF_ENOSPC;
     const TflGemm g = *product;
@@ -698,7 +703,112 @@ extern "C" int tfl_attn_decode_beside(const void* q, const void* cache, int n_pa
         case 4: GO(4); break;
     }
 #undef GO
-    return rc == TF_OK ? launch_merge<bf16>(ws, out, rows, H, 512, nsplit, st) : rc;
+    return rc == TF_OK && out ? launch_merge<bf16>(ws, out, rows, H, 512, nsplit, st) : rc;
+}
+
+// The merge of the splits in front of latent to value: out = (merged . W_head^T) * sigmoid(gate) for up to 4 rows of 512 latents, one panel of
+// values to a workgroup.  Each of a head's workgroups merges for itself, from L2: that costs less than a launch between the two as long as the
+// splits are few.  The panel's weights and gates come in under it.  One row of 4 000 keys (32 splits): merge 4.7 and product 4.5 -> 5.8 us, a step of
+// 48 layer runs 4 666 -> 4 568.  us of a graph of the attention beside its product and this, merge launched -> here (splits of all rows): 1 row
+// 26.5 -> 24.9 (16), 27.2 -> 25.2 (32), 29.7 -> 28.9 (80); 2 rows 27.4 -> 26.9 (32), 28.7 -> 28.0 (64), 30.8 -> 31.2 (100); 4 rows 31.9 -> 30.6 (64);
+// 8 rows 32.0 -> 35.5 (64).
+constexpr int VALUE_ROWS = 4;
+__global__ __launch_bounds__(512) void latent_value_kernel(const float* __restrict__ ws, int nsplit, const TflGemm a) {
+    __shared__ float weight[VALUE_ROWS][128];
+    __shared__ int count[VALUE_ROWS];
+    __shared__ __align__(16) float sums[4][VALUE_ROWS][512];
+    __shared__ __align__(16) bf16 merged[VALUE_ROWS][512 + 8];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15;
+    const int ppg = a.n >> 4, head = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / ppg), panel = (blockIdx.x >> 3) % ppg;        // (a head on one XCD)
+    if (head >= a.groups) return;
+    const int col = head * a.n + 16 * panel + 4 * g, quad = tid & 127, grp = tid >> 7;
+    const float* src = ws + (int64_t)head * nsplit * 512 + 4 * quad;
+    const int64_t row_step = (int64_t)a.groups * nsplit * 512;
+    bf16x8 w[2];
+    f32x4 z[8];                                               // splits grp, grp + 4, .. of the first row: asked for before it is known which there are
+#pragma unroll
+    for (int u = 0; u < 8; ++u) z[u] = *reinterpret_cast<const f32x4*>(src + (int64_t)min(grp + 4 * u, nsplit - 1) * 512);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) w[u] = load_frag_stream((const bf16*)a.wp + ((int64_t)(head * ppg + panel) * 16 + 2 * wave + u) * 512 + lane * 8);
+    f32x4 gate = {0.f, 0.f, 0.f, 0.f};
+    if (wave == 0 && i < a.rows) gate = *reinterpret_cast<const f32x4*>(a.gate + (int64_t)i * a.ld_gate + col);
+    if (wave < a.rows) {
+        const float* ml = ws + (int64_t)a.rows * a.groups * nsplit * 512 + ((int64_t)wave * a.groups + head) * nsplit * 2;
+        float l[2], m[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int s = lane + 64 * h;
+            l[h] = s < nsplit ? ml[2 * s + 1] : 0.f;
+            m[h] = l[h] > 0.f ? ml[2 * s] : NEG_INF;          // (an empty split: its partial row is not read either)
+        }
+        float most = fmaxf(m[0], m[1]), all = 0.f;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o, 64));
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            m[h] = l[h] > 0.f ? exp2f((m[h] - most) * LOG2E) : 0.f;
+            all += m[h] * l[h];
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) all += __shfl_xor(all, o, 64);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) weight[wave][lane + 64 * h] = all > 0.f ? m[h] / all : 0.f;
+        const uint64_t low = __builtin_amdgcn_ballot_w64(l[0] > 0.f), high = __builtin_amdgcn_ballot_w64(l[1] > 0.f);
+        if (lane == 0) count[wave] = high ? 128 - __builtin_clzll(high) : low ? 64 - __builtin_clzll(low) : 0;
+    }
+    __syncthreads();
+    for (int r = 0; r < a.rows; ++r) {
+        const int n = count[r], next = r + 1 < a.rows ? count[r + 1] : 0;
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        for (int s0 = grp;; s0 += 32) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const float x = s0 + 4 * u < n ? weight[r][s0 + 4 * u] : 0.f;
+                if (x > 0.f)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = fmaf(z[u][e], x, v[e]);
+            }
+            if (s0 + 32 >= n) break;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) z[u] = *reinterpret_cast<const f32x4*>(src + r * row_step + (int64_t)min(s0 + 32 + 4 * u, n - 1) * 512);
+        }
+        if (next > 0)
+#pragma unroll
+            for (int u = 0; u < 8; ++u) z[u] = *reinterpret_cast<const f32x4*>(src + (r + 1) * row_step + (int64_t)min(grp + 4 * u, next - 1) * 512);
+        *reinterpret_cast<f32x4*>(&sums[grp][r][4 * quad]) = v;
+    }
+    __syncthreads();
+    for (int r = 0; r < a.rows; ++r) merged[r][tid] = (bf16)(sums[0][r][tid] + sums[1][r][tid] + sums[2][r][tid] + sums[3][r][tid]);
+    __syncthreads();
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        bf16x8 x = {};
+        if (i < a.rows) x = load_frag(&merged[i][32 * (2 * wave + u) + 8 * g]);
+        acc = El<bf16>::mma(w[u], x, acc);
+    }
+    f32x4 (*part)[64] = reinterpret_cast<f32x4 (*)[64]>(sums);
+    part[wave][lane] = acc;
+    __syncthreads();
+    if (wave || i >= a.rows) return;
+#pragma unroll
+    for (int v = 1; v < 8; ++v)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += part[v][lane][e];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] *= sigmoid(gate[e]);
+    store_quad((bf16*)a.out_t + (int64_t)i * a.ld_t + (col >> 3) * a.t_oct + (col & 7), acc);
+}
+
+extern "C" int tfl_latent_value(const float* ws, int64_t ws_floats, int nsplit, const TflGemm* p, void* stream) {
+    if (!ws || !p || !p->wp || !p->gate || !p->out_t || nsplit < 2 || nsplit > 128) return TF_EINVAL;
+    const TflGemm a = *p;
+    if (a.rows < 1 || a.rows > VALUE_ROWS || a.n < 16 || (a.n & 15) || a.k != 512 || a.groups < 1 || a.chunk_major || a.t_oct < 8 || (a.t_oct & 7) || a.ld_t < 8
+        || (a.ld_t & 7) || a.ld_gate < (int64_t)a.groups * a.n || (a.ld_gate & 3)) return TF_EINVAL;
+    if (ws_floats < tfl_attn_decode_ws_floats(a.rows, a.groups, 512, nsplit)) return TF_ENOSPC;
+    hipLaunchKernelGGL(latent_value_kernel, dim3((a.n >> 4) * ((a.groups + 7) / 8 * 8)), dim3(512), 0, (hipStream_t)stream, ws, nsplit, a);
+    TFL_LAUNCH_CHECK();
+    return TF_OK;
 }
 
 // --------------------------------------------------------------------------------------------------------------- prefill

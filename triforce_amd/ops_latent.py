@@ -62,11 +62,17 @@ def query_to_latent(qn, wt, q, g):
 
 
 def latent_to_value(ol, wt, raw, gate_off, act, g):
-    """Columns h*V .. of the activation block act = (ol[:, h] . Wuv_h^T) * sigmoid(gate)."""
-    _need(ol, raw, act)
+    """Columns h*V .. of the activation block act = (ol[:, h] . Wuv_h^T) * sigmoid(gate).  ``ol``: a tensor, or Splits that it merges."""
+    _need(ol.ws if isinstance(ol, Splits) else ol, raw, act)
     rows, (act_rows_, act_k, act_ld, act_oct) = ol.shape[0], _lay(act)
     assert (wt.groups, wt.n, wt.k) == (g.H, g.V, g.C) and ol.dtype == act.dtype == wt.dtype and act_rows_ == rows and act_k >= g.H * g.V
     assert raw.shape[1] >= gate_off + g.H * g.V
+    if isinstance(ol, Splits):
+        a = hip.TflGemm()
+        a.wp, a.gate, a.out_t, a.ld_gate, a.ld_t, a.t_oct = wt.packed.data_ptr(), raw[:, gate_off:].data_ptr(), act.data_ptr(), raw.stride(0), act_ld, act_oct
+        a.rows, a.n, a.k, a.groups, a.chunk_major = rows, wt.n, wt.k, wt.groups, int(wt.chunk_major)
+        hip.check(hip.latent_lib().tfl_latent_value(_p(ol.ws), ol.ws.numel(), ol.nsplit, ctypes.byref(a), _stream()), "tfl_latent_value")
+        return
     _gemm(wt, ol, "gated", rows, ld_x=g.H * g.C, x_group=g.C, gate=raw[:, gate_off:], ld_gate=raw.stride(0), out_t=act,
           ld_t=act_ld, t_oct=act_oct)
 
@@ -193,21 +199,31 @@ def attn_decode(q, cache, table, klen, g, scale, max_len, nsplit=None):
     return out
 
 
+VALUE_ROWS, VALUE_PARTS = 4, 80      # up to which latent_to_value merges the splits itself, see latent_value_kernel
+
+
 @functools.lru_cache(maxsize=1024)
 def beside_plan(rows, H, C, R, pages, n, k):
-    """(workers, panels each, splits) of attn_decode_beside for rows with ``pages`` pages in all and a product of n outputs of k, None where the
-    two are better launched apart."""
-    each, nsplit = ctypes.c_int32(), ctypes.c_int32()
-    workers = hip.latent_lib().tfl_attn_beside_plan(rows, H, C, R, pages, n, k, ctypes.byref(each), ctypes.byref(nsplit))
-    return (workers, each.value, nsplit.value) if workers > 0 else None
+    """(workers, panels each, splits, does latent_to_value merge them) of attn_decode_beside for rows with ``pages`` pages in all and a
+    product of n outputs of k, None where the two are better launched apart."""
+    each, nsplit, parts = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
+    workers = hip.latent_lib().tfl_attn_beside_plan(rows, H, C, R, pages, n, k, ctypes.byref(each), ctypes.byref(nsplit), ctypes.byref(parts))
+    return (workers, each.value, nsplit.value, rows <= VALUE_ROWS and parts.value <= VALUE_PARTS) if workers > 0 else None
+
+
+class Splits:
+    """What attn_decode_beside leaves to latent_to_value: unmerged splits of [rows, H, C]."""
+
+    def __init__(self, ws, nsplit, shape, dtype):
+        self.ws, self.nsplit, self.shape, self.dtype, self.is_cuda = ws, nsplit, shape, dtype, ws.is_cuda
 
 
 def attn_decode_beside(q, cache, table, klen, g, scale, plan, act, wt, x, k0):
-    """attn_decode of bfloat16 rows of 512 + 64 with x += act . W^T over the columns from k0 on in the same launch."""
+    """attn_decode of bfloat16 rows of 512 + 64 with x += act . W^T over the columns from k0 on in the same launch.  Splits as the plan says."""
     _need(q, cache, table, klen, act, x)
     _i32(table, klen)
     _f32(x)
-    rows, (workers, each, nsplit) = q.shape[0], plan
+    rows, (workers, each, nsplit, later) = q.shape[0], plan
     assert q.dtype == cache.dtype == act.dtype == wt.dtype == torch.bfloat16 and q.is_contiguous() and q.shape[1:] == (g.H, 576) and (g.C, g.R) == (512, 64)
     assert cache.is_contiguous() and cache.shape[1] == 576 and cache.shape[0] % PAGE == 0
     assert table.shape[0] == rows and table.stride(1) == 1 and klen.numel() == rows
@@ -215,11 +231,11 @@ def attn_decode_beside(q, cache, table, klen, g, scale, plan, act, wt, x, k0):
     assert wt.chunk_major and 0 <= k0 < wt.k and k0 % 32 == 0
     L = hip.latent_lib()
     ws = torch.empty(L.tfl_attn_decode_ws_floats(rows, g.H, g.C, nsplit), dtype=torch.float32, device=q.device)
-    out = torch.empty(rows, g.H, g.C, dtype=q.dtype, device=q.device)
+    out = None if later else torch.empty(rows, g.H, g.C, dtype=q.dtype, device=q.device)
     a = hip.TflGemm()
     a.wp, a.x, a.out_f = wt.packed.data_ptr() + 2 * k0 * wt.n, act[k0 // 8:].data_ptr(), x.data_ptr()
     a.rows, a.n, a.k, a.groups, a.chunk_major, a.ld_f = rows, wt.n, wt.k - k0, 1, 1, x.stride(0)
     a.ld_x, a.x_oct, a.t_oct = 8, 8 * rows, 8
     hip.check(L.tfl_attn_decode_beside(_p(q), _p(cache), cache.shape[0] // PAGE, _p(table), table.stride(0), _p(klen), _p(out), _p(ws), ws.numel(), rows, g.H,
                                        float(scale), nsplit, workers, each, ctypes.byref(a), _stream()), "tfl_attn_decode_beside")
-    return out
+    return Splits(ws, nsplit, (rows, g.H, g.C), q.dtype) if later else out
