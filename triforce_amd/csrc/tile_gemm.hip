@@ -73,6 +73,18 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
     for (int p = 0; p < P; ++p)
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[p][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // QUERY: the producer's sums of squares are asked for here and added behind the products
+    constexpr int SSU = EPI == TFL_EPI_QUERY ? 12 : 1;
+    [[maybe_unused]] float2 sums[SSU];
+    [[maybe_unused]] const float2* ss = nullptr;
+    if constexpr (EPI == TFL_EPI_QUERY) {
+        if (wave < MT) {
+            ss = reinterpret_cast<const float2*>(a.ss_in + (int64_t)min(m0 + 16 * wave + i, a.rows - 1) * a.ss_ld);
+#pragma unroll
+            for (int u = 0; u < SSU; ++u) sums[u] = ss[min(g + 4 * u, a.ss_n / 2 - 1)];
+        }
+        asm volatile("" ::: "memory");
+    }
     if (c_beg < c_end) {
         Frag w[P][U], wn[P][U];
         load_w(w, c_beg);
@@ -110,10 +122,12 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
     float inv = 1.f;
     if constexpr (EPI == TFL_EPI_QUERY) {                    // scale of row m from the producer's per-panel sums of squares
         if (wave < MT) {
-            const float2* ss = reinterpret_cast<const float2*>(a.ss_in + (int64_t)min(m0 + 16 * wave + i, a.rows - 1) * a.ss_ld);
             float q = 0.f;
-#pragma unroll 8
-            for (int p = g; p < a.ss_n / 2; p += 4) {
+#pragma unroll
+            for (int u = 0; u < SSU; ++u)
+                if (g + 4 * u < a.ss_n / 2) q += sums[u].x + sums[u].y;
+#pragma unroll 4
+            for (int p = g + 4 * SSU; p < a.ss_n / 2; p += 4) {
                 const float2 v = ss[p];
                 q += v.x + v.y;
             }
