@@ -448,6 +448,15 @@ def test_split_float32_shared_tiles(rows, n, k):
     assert torch.isfinite(got[torch.isfinite(plain)]).all()
 
 
+# whole tiles of a product that would be cut in three parts of k otherwise: their running sums are as short
+def test_split_float32_shared_tiles_are_as_exact_as_parts():
+    from triforce_amd import ops_tile as ot
+    x, w = _factors("absolute", 700, 12320, 4096)
+    want = x.double() @ w.double().T
+    far = [(ot.split_linear(x, w, s).double() - want).norm() for s in (0, 3, 1)]
+    assert far[0] <= 1.02 * far[1] and far[1] < 0.5 * far[2]
+
+
 # products that stand alone (a row of x with one entry): every bit of both factors counts, in every place of a step of 32
 @pytest.mark.parametrize("splits", [1, 2])
 def test_split_float32_single_products(splits):

@@ -22,7 +22,7 @@
 // products instead of behind them waits for x's DMA before each store to LDS: 22 016 x 4 096 at 2 048 rows 1 830 -> 2 230 us.)
 //
 // Bound by the power of the matrix cores (1.6 to 1.7 GHz under these products, as bf16 GEMMs) and by rounds of tiles.  fp32 GEMM before ->
-// now, x's cut and the sum of parts included: 700 rows, 22 016 x 4 096 940 -> 635 us, 18 784 x 4 096 900 -> 570, 4 096 x 15 104 680 -> 460;
+// now, x's cut and the sum of parts included: 700 rows, 22 016 x 4 096 940 -> 665 us, 18 784 x 4 096 900 -> 565, 4 096 x 15 104 680 -> 460;
 // 2 048 rows, 22 016 x 4 096 2 600 -> 1 800 (205 TFLOP/s).
 //
 // Range: both operands are cut at 2^24 times their value, so the last bit of the smallest float32 (2^-149) is still a normal bfloat16 and no
@@ -99,6 +99,7 @@ struct SplitGemm {
     int64_t ld_x, ld_out;
     int rows, n, k;
     int whole, splits, sharers, slots;                        // see Share; slots of an XCD
+    int fold;                                                 // steps that are added up in registers
 };
 
 // An XCD's tiles (an eighth of all): the first `whole` of them have a workgroup each.  The steps of the others stand in a line, which is cut among
@@ -168,7 +169,8 @@ __device__ __forceinline__ void mend(const SplitGemm& a, int row0, int n0, f32x4
     for (int e = 0; e < 4; ++e) v[e] = lost[e] ? p[e] : v[e];
 }
 
-// Waves: 4 x 64 outputs, 2 x 64 rows (MT 16-row tiles of x each); every wave brings PER fragments of x in.
+// Waves: 4 x 64 outputs, 2 x 64 rows (MT 16-row tiles of x each); every wave brings PER fragments of x in.  FOLDS: a.fold is below a tile's steps.
+template <bool FOLDS>
 __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
     constexpr int MT = 4, NP = 16, XP = 2 * MT, PER = 3 * XP / 8, BUF = 3 * (NP + XP) * 512;
     extern __shared__ __align__(16) bf16 tiles[];             // [2][NP + XP][3][512]
@@ -226,11 +228,36 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
 #pragma unroll
     for (int f = 0; f < 2; ++f) wsrc[f] = a.w + (int64_t)min(nt * 256 + 16 * (wave + 8 * f) + i, a.n - 1) * a.k + 8 * g;
     const bool live = mt0 * XP + wm * MT < xpan;              // a wave without rows leaves the matrix core to its neighbour
+    float* part = q < 0 ? nullptr : a.ws + ((int64_t)xcd * a.slots + q + r) * SLOT;           // a row of 256 behind the other
     f32x4 acc[4][MT], low[4][MT];                             // hh and the five small products
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int m = 0; m < MT; ++m) acc[t][m] = low[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // f of this lane's places in the result, or in the part's slot
+    const int lines = q < 0 ? a.rows : 1 << 30;
+    bool lost = false;                                        // a result that is not finite
+    auto each = [&](auto&& f) {
+        int at = lane;
+        if constexpr (FOLDS) asm volatile("" : "+v"(at));     // (places made ahead of the steps would take registers from them)
+        const int g = at >> 4, i = at & 15;
+        float* y = q < 0 ? a.out : part;
+        const int64_t ld = q < 0 ? a.ld_out : 256;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int in_row = 16 * (wm * MT + m), row0 = mt0 * 32 * MT + in_row;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int in_n = 64 * wn + 16 * t;
+                if constexpr (FOLDS) {                        // one after the other: what is there would take a step's registers
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (row0 >= a.rows || nt * 256 + in_n >= a.n) continue;
+                f(m, t, reinterpret_cast<f32x4*>(y + (q < 0 ? row0 + i : in_row + i) * ld + (q < 0 ? nt * 256 : 0) + in_n + 4 * g), row0, i);
+            }
+        }
+    };
     if (c_beg < c_end) {
         fetch_x(c_beg, 0);
         fetch_w(c_beg);
@@ -239,7 +266,8 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
         fetch_w(min(c_beg + 1, c_end - 1));
         meet();
     }
-    for (int c = c_beg; c < c_end; ++c) {
+    for (int c = c_beg;;) {
+    for (const int stop = FOLDS ? min(c_end, c + a.fold) : c_end; c < stop; ++c) {
         const int buf = (c - c_beg) & 1;
         fetch_x(min(c + 1, c_end - 1), buf ^ 1);              // in flight under this step's products
         if (live) {
@@ -270,26 +298,32 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
         fetch_w(min(c + 2, c_end - 1));
         meet();
     }
-    // a part goes to its slot, a row of 256 behind the other
-    float* part = q < 0 ? nullptr : a.ws + ((int64_t)xcd * a.slots + q + r) * SLOT;
+    if constexpr (!FOLDS) break;
+    each([&](int m, int t, f32x4* y, int row0, int i) {       // sums go to the result, or to a part's slot, and to what is there
+        f32x4 v, have = {0.f, 0.f, 0.f, 0.f};
+        if (c > c_beg + a.fold && row0 + i < lines) have = *y;
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int in_row = 16 * (wm * MT + m), row0 = mt0 * 32 * MT + in_row;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int in_n = 64 * wn + 16 * t, n0 = nt * 256 + in_n;
-            if (row0 >= a.rows || n0 >= a.n) continue;
-            f32x4 v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE));
-            if (part) {
-                *reinterpret_cast<f32x4*>(part + 256 * (in_row + i) + in_n + 4 * g) = v;
-            } else {
-                mend(a, row0, n0, v);
-                if (row0 + i < a.rows) *reinterpret_cast<f32x4*>(a.out + (int64_t)(row0 + i) * a.ld_out + n0 + 4 * g) = v;
-            }
+        for (int e = 0; e < 4; ++e) {
+            v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE)) + have[e];
+            lost = lost || !(__builtin_fabsf(v[e]) < __builtin_inff());
         }
+        acc[t][m] = low[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (row0 + i < lines) *y = v;
+    });
+    if (c >= c_end) break;
     }
+    if (!FOLDS || (q < 0 && __any(lost)))
+        each([&](int m, int t, f32x4* y, int row0, int i) {
+            f32x4 v = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (!FOLDS) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE));
+            } else if (row0 + i < lines) {
+                v = *y;
+            }
+            if (q < 0) mend(a, row0, nt * 256 + 64 * wn + 16 * t, v);
+            if (row0 + i < lines) *y = v;
+        });
     beg += c_end - c_beg;
     } while (beg < end);
 }
@@ -324,10 +358,11 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const SplitGemm a) {
 
 static int launch_split_gemm(const SplitGemm& a, hipStream_t st) {
     constexpr int LDS = 2 * 3 * (16 + 8) * 1024;              // two buffers of 16 panels of weights and 8 of x, in three parts
-    const hipError_t e = hipFuncSetAttribute((const void*)split_gemm_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    const auto kernel = a.fold < a.k >> 5 ? split_gemm_kernel<true> : split_gemm_kernel<false>;
+    const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e != hipSuccess) return (int)e;
     const int each = (split_tiles(a.rows, a.n) + 7) / 8, own = each < a.whole ? each : a.whole, rest = each - own;
-    hipLaunchKernelGGL(split_gemm_kernel, dim3(8 * (own + (rest == 0 ? 0 : a.sharers > 0 ? a.sharers : rest * a.splits))), dim3(512), LDS, st, a);
+    hipLaunchKernelGGL(kernel, dim3(8 * (own + (rest == 0 ? 0 : a.sharers > 0 ? a.sharers : rest * a.splits))), dim3(512), LDS, st, a);
     TFL_LAUNCH_CHECK();
     if (rest > 0) {
         hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)rest * 256), dim3(256), 0, st, a);
@@ -340,39 +375,42 @@ static int launch_split_gemm(const SplitGemm& a, hipStream_t st) {
 static int64_t split_planes(int rows, int k) { return (int64_t)((rows + 15) / 16) * (k / 32) * 1536 * 2 / 4; }
 static int64_t split_marks(int rows, int k) { return ((int64_t)rows * split_parts(k) + 3) / 4 * 4; }
 
-struct Parts { int whole, splits, sharers; };
+struct Parts { int whole, splits, sharers, fold; };
 
 // How k is cut: rounds of workgroups, each with the fill of its pipe (4 steps of 32), against what the parts cost on their way through memory
 // (a written and read 128 x 256 part as much as 8 steps).  Rounds are an XCD's: it has 32 CUs and its eighth of the tiles, rounded up (36 tiles in
 // seven parts are 252 workgroups, but 35 on some XCDs: 700 rows, 1 536 x 6 144 in seven 119 us, in six 95).  256 rows, 12 320 x 4 096: 267 us
 // without parts, 159 with two, 171 with four; 700 rows, 4 096 x 8 192: 514, 296 with two, 262 with five, 265 with eight.
 // From 32 tiles an XCD on: whole rounds of whole tiles, and the steps of the others shared by all CUs, 8 or more to each.  A last round of few tiles,
-// or parts of all tiles instead (516 tiles of 22 016 x 4 096 at 700 rows in two parts, 2.5 rounds and 250 MB of parts): 755 -> 635 us; 12 320
-// outputs 425 -> 375, 300 rows of 22 016 400 -> 335, 1 000 rows of 18 784 805 -> 750.  Below, sharing gains nothing over whole tiles on fewer
-// CUs, which run at a higher clock (256 rows of 22 016, 172 tiles: 317 us alone, 327 shared).
+// or parts of all tiles instead (516 tiles of 22 016 x 4 096 at 700 rows in two parts, 2.5 rounds and 250 MB of parts): 755 -> 665 us; 12 320
+// outputs 425 -> 402, 1 000 rows of them 565 -> 509, 300 rows of 22 016 402 -> 365, 1 500 1 437 -> 1 288.  Below, sharing gains nothing over whole
+// tiles on fewer CUs, which run at a higher clock (256 rows of 22 016, 172 tiles: 317 us alone, 327 shared).
+// A running sum of all steps is further off than the parts that k would be in otherwise (absolute values, 4 096 columns: 3.5e-7, two parts 1.8e-7,
+// three 1.1e-7), so it goes to the result as often (`fold`), at 4 steps' cost each: 700 rows of 22 016 637 -> 665 us, error as in two parts.
 static Parts pick_parts(int rows, int n, int k) {
     const int tiles = split_tiles(rows, n), per_xcd = (tiles + 7) / 8;
     const double chunks = k / 32;
-    Parts best{0, 1, 0};
+    Parts best{0, 1, 0, k / 32};
     double least = 0;
     for (int s = 1; s <= 8 && (s == 1 || s * 512 <= k); ++s) {
         const double t = (double)(((int64_t)per_xcd * s + 31) / 32) * (1.0 / s + 4.0 / chunks) + (s > 1 ? 8.0 * (double)s * tiles / 256 / chunks : 0);
         if (s == 1 || t < least) { best.splits = s; least = t; }
     }
+    const int parts = best.splits, fold = (k / 32 + parts - 1) / parts;
     for (int w = per_xcd >> 5; w > 0 && w >= (per_xcd >> 5) - 1; --w) {
         const int rest = per_xcd - 32 * w;
         const int64_t line = (int64_t)rest * (k / 32);
         if (rest == 0 || line < 16 || line > 1 << 24) continue;
         const int sharers = (int)(line / 8 < 32 ? line / 8 : 32);
-        const double t = w * (1.0 + 4.0 / chunks) + rest / (double)sharers + (rest > 1 ? 8.0 : 4.0) / chunks + 8.0 * (sharers + rest) / 32 / chunks + 3.0 / chunks;
-        if (t < least) { best = Parts{32 * w, 1, sharers}; least = t; }
+        const double t = w * (1.0 + 4.0 * parts / chunks) + rest / (double)sharers + (rest > 1 ? 8.0 : 4.0) / chunks + 8.0 * (sharers + rest) / 32 / chunks + 3.0 / chunks;
+        if (t < least) { best = Parts{32 * w, 1, sharers, fold}; least = t; }
     }
     if (best.sharers == 0 && best.splits == 1) best.whole = 1 << 28;
     return best;
 }
 
 static Parts given_parts(int rows, int n, int k, int splits) {
-    return splits == 0 ? pick_parts(rows, n, k) : Parts{splits == 1 ? 1 << 28 : 0, splits, 0};
+    return splits == 0 ? pick_parts(rows, n, k) : Parts{splits == 1 ? 1 << 28 : 0, splits, 0, k / 32};
 }
 
 extern "C" int64_t tfl_split_gemm_ws_floats(int rows, int n, int k, int splits) {
@@ -392,6 +430,6 @@ extern "C" int tfl_split_gemm(const float* w, const float* x, int64_t ld_x, floa
     hipLaunchKernelGGL(split_rows_kernel, dim3((rows + 15) / 16, split_parts(k)), dim3(256), 0, (hipStream_t)stream, x, ld_x, rows, k, (bf16*)ws, nans);
     TFL_LAUNCH_CHECK();
     const SplitGemm a = {w, (const bf16*)ws, x, out, ws + split_planes(rows, k) + split_marks(rows, k), nans, ld_x, ld_out, rows, n, k, p.whole, p.splits, p.sharers,
-                         split_slots(split_tiles(rows, n), p.whole, p.splits, p.sharers)};
+                         split_slots(split_tiles(rows, n), p.whole, p.splits, p.sharers), p.fold};
     return launch_split_gemm(a, (hipStream_t)stream);
 }

@@ -76,7 +76,7 @@ class LatentLayer:
         qn, q = ol.query_and_append(xq, raw, ss, self.w_uq, g, self.kv_norm, eps, rope, batch.pos, batch.slot, cache_rows)
         ol.query_to_latent(qn, self.w_uk_t, q, g)
         own = g.H * g.V                                       # act: the attention's columns, then the feed-forward's, which wait for nothing of it
-        # (max_len is the cache's capacity; contexts that grow to it are half to all of it long.  32 rows of 1 500 to 3 000 keys, planned for
+        # (max_len is the cache's capacity; contexts that grow to it are half to all of it long.  32 rows of 2 000 to 4 000 keys, planned for
         # all pages 7 309 us a step, for three quarters 7 225)
         plan = ol.beside_plan(ids.numel(), g.H, g.C, g.R, -(-3 * batch.max_len // (4 * ol.PAGE)), self.w_out.n, self.w_out.k - own) \
             if self.ff and self.w_out.chunk_major and h.dtype == torch.bfloat16 else None
