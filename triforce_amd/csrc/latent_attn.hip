@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256 * HT, HT) void attn_latent_sized_kernel(const b
 // Splits are dealt: as many pages each, 2 at least where a row has more than 16, as make the splits of all rows fit the workers; a row has
 // nsplit at most, with as many pages each as that takes.  Statistics of splits that a row does not have are zero, which the merge skips.
 // us, 20 heads, attention, merge and the output product (shorter by 11 008 of its 15 104), apart -> so: a row of 64 pages 36.6 -> 31.1, 32 rows of 48
-// 61.9 -> 59.9; of a whole step of 48 layer runs, one row of 4 000 keys 4 987 -> 4 668, 32 rows 7 500 -> 7 335.
+// 61.9 -> 59.9; of eight steps of six layer runs, one row of 4 000 keys 4 987 -> 4 668, 32 rows 7 500 -> 7 335.
 template <int P, int MT>
 __global__ __launch_bounds__(512, 2) void attn_latent_beside_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages,
                                                                     const int32_t* __restrict__ table, int table_ld, const int32_t* __restrict__ len,
@@ -708,8 +708,8 @@ extern "C" int tfl_attn_decode_beside(const void* q, const void* cache, int n_pa
 
 // The merge of the splits in front of latent to value: out = (merged . W_head^T) * sigmoid(gate) for up to 4 rows of 512 latents, one panel of
 // values to a workgroup.  Each of a head's workgroups merges for itself, from L2: that costs less than a launch between the two as long as the
-// splits are few.  The panel's weights and gates come in under it.  One row of 4 000 keys (32 splits): merge 4.7 and product 4.5 -> 5.8 us, a step of
-// 48 layer runs 4 666 -> 4 568.  us of a graph of the attention beside its product and this, merge launched -> here (splits of all rows): 1 row
+// splits are few.  The panel's weights and gates come in under it.  One row of 4 000 keys (32 splits): merge 4.7 and product 4.5 -> 5.8 us, eight
+// steps of six layer runs 4 666 -> 4 568.  us of a graph of the attention beside its product and this, merge launched -> here (splits of all rows): 1 row
 // 26.5 -> 24.9 (16), 27.2 -> 25.2 (32), 29.7 -> 28.9 (80); 2 rows 27.4 -> 26.9 (32), 28.7 -> 28.0 (64), 30.8 -> 31.2 (100); 4 rows 31.9 -> 30.6 (64);
 // 8 rows 32.0 -> 35.5 (64).
 constexpr int VALUE_ROWS = 4;

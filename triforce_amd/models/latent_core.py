@@ -77,7 +77,7 @@ class LatentLayer:
         ol.query_to_latent(qn, self.w_uk_t, q, g)
         own = g.H * g.V                                       # act: the attention's columns, then the feed-forward's, which wait for nothing of it
         # (max_len is the cache's capacity; contexts that grow to it are half to all of it long.  32 rows of 2 000 to 4 000 keys, planned for
-        # all pages 7 309 us a step, for three quarters 7 225)
+        # all pages, 7 309 us for eight steps of six layer runs, for three quarters 7 225)
         plan = ol.beside_plan(ids.numel(), g.H, g.C, g.R, -(-3 * batch.max_len // (4 * ol.PAGE)), self.w_out.n, self.w_out.k - own) \
             if self.ff and self.w_out.chunk_major and h.dtype == torch.bfloat16 else None
         if plan is None:
