@@ -223,8 +223,8 @@ def stage_latencies(ge, args, device):
     ids = torch.full((1, gamma + 1), 100, dtype=torch.long, device=device)
     pos = torch.arange(S, S + gamma + 1, device=device).unsqueeze(0)
     # draft step: the replay the loop issues (inner-iteration graphs and the catch-up forward run the draft over the shared
-    # token buffer: no input copy, no output clone); `draft_step_with_io_us` is graph_draft_inference with both (two more
-    # launches: the figure quoted as draft_step_us up to round 5)
+    # token buffer: no input copy, no output clone); `draft_step_with_io_us` is graph_draft_inference, over the caller's tokens into
+    # a fresh row: one launch without the graph where the draft runs as one, the replay between two copies otherwise
     with_io = _timed(lambda: ge.graph_draft_inference(ids[:, :3], gamma_offset=2), 20)
     if getattr(ge, "tok_buf", None) is not None and hasattr(ge, "replay_draft"):
         with torch.inference_mode():                           # (the engine's static buffers are inference tensors)
@@ -738,8 +738,8 @@ def main():
         "form": "one launch: tf_draft_forward_68m_persist, 256 co-resident workgroups, arrival counters + READY flags"
                 if dp is not None else "13-launch chain: tf_draft_forward_68m",
         "error_word": dp.error() if dp is not None else None,
-        "draft_step_us_is": "the hipGraph replay the loop issues (shared token buffer); draft_step_with_io_us adds the input "
-                            "copy and the output clone of graph_draft_inference (what rounds 1-5 quoted as draft_step_us)"}
+        "draft_step_us_is": "the hipGraph replay the loop issues (shared token buffer); draft_step_with_io_us is "
+                            "graph_draft_inference: one launch over the caller's tokens into a fresh row"}
     if kind == "aligned":
         # the headline is CONDITIONAL on a dial: say so next to it (trained checkpoints are not available offline)
         result["value_note"] = (f"configured-acceptance scenario: synthetic weights {wlabel} SET the draft->retrieval and "
