@@ -121,3 +121,13 @@ def test_captured_with_parts_of_k():
         torch.cuda.synchronize()
         assert torch.equal(y, want)
         assert torch.equal(ops_rows.linear(x, w), want)
+
+
+def test_wide_products_of_some_rows_are_the_librarys(monkeypatch):
+    taken = []
+    monkeypatch.setattr(ops_rows, "product", lambda x, w: taken.append(x.shape[0]) or F.linear(x, w))
+    w = torch.zeros(24592, 64, dtype=torch.float16, device="cuda")
+    for rows in (100, 101, 199, 200):
+        ops_rows.linear(torch.zeros(rows, 64, dtype=torch.float16, device="cuda"), w)
+        ops_rows.linear(torch.zeros(rows, 64, dtype=torch.float16, device="cuda"), w[:24576])
+    assert taken == [100, 100, 101, 199, 200, 200]

@@ -14,7 +14,7 @@
 //   22 016 x 4 096:  130 rows 51 -> 55, 700 140 -> 141, 1 500 294 -> 236, 3 100 547 -> 425, 4 096 654 -> 556, 8 000 1 152 -> 1 027
 //   4 096 x 11 008:  130 rows 49 -> 34, 700  89 ->  71, 1 500 129 -> 122, 3 100 221 -> 210, 4 096 243 -> 247, 8 000   480 -> 487
 //   4 096 x 4 096:   130 rows 18 -> 13, 700  31 ->  33, 1 500  50 ->  50, 3 100  84 ->  80, 4 096  94 ->  99, 8 000   185 -> 191
-// At 100 to 350 rows plan() can miss the library's time by up to a fifth (12 288 x 4 096, 220 rows: 40 -> 49; the best tile there takes 40).
+// At 200 to 300 rows of 12 288 x 4 096 the library is still up to 8 % faster (255 rows: 43 -> 47).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -338,7 +338,8 @@ constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 struct Plan { int shape, splits; };
 
 // The bytes each operand needs at 6.5 TB/s; the steps of a CU's tiles, one or two at a time; parts of k are written and read at 4 TB/s by
-// another launch.  XCDs take an eighth of the tiles each, and their 32 CUs whole ones.
+// another launch.  XCDs take an eighth of the tiles each, and their 32 CUs whole ones.  Small tiles in number are bound by what they read from L2,
+// 17 TB/s (12 288 x 4 096: 190 rows 47 -> 41 us by another tile, 255 rows 53 -> 47, 350 rows 62 -> 57; 4 096 x 11 008, 255 rows 51 -> 42).
 inline Plan plan(int rows, int n, int k) {
     const int nk = k >> 6;
     const double mem = (2.0 * n * k + 2.0 * rows * k + 2.0 * rows * n) / 6.5e6;
@@ -347,13 +348,14 @@ inline Plan plan(int rows, int n, int k) {
     for (int s = 0; s < N_SHAPES; ++s) {
         const Shape& h = SHAPES[s];
         const int64_t tiles = (int64_t)((rows + h.rows - 1) / h.rows) * ((n + h.cols - 1) / h.cols);
+        const double l2 = h.per_cu > 1 ? (double)tiles * nk * (h.rows + h.cols) * 128 / 17e6 : 0.0;
         for (int z = 1; z <= 16; ++z) {
             const int per = (nk + z - 1) / z;
             if (z > 1 && ((z - 1) * per >= nk || per < 4 || tiles * z > 410 * h.per_cu || (int64_t)z * rows * n > (int64_t)1 << 28)) continue;
             const int64_t a_cu = ((tiles * z + 7) / 8 + 31) / 32, full = a_cu / h.per_cu;
             const double fully = per * (double)fmaxf(h.per_cu * h.step, h.least) + h.per_cu * h.tile;
             const double work = full * fully + (a_cu > full * h.per_cu ? per * (double)fmaxf(h.step, h.least) + h.tile : 0.0);
-            const double t = cbrt(work * work * work + mem * mem * mem) + (z > 1 ? 3.0 + z * 4.0 * rows * n / 4.3e6 : 0.0);
+            const double t = cbrt(work * work * work + mem * mem * mem + l2 * l2 * l2) + (z > 1 ? 3.0 + z * 4.0 * rows * n / 4.3e6 : 0.0);
             if ((s == 0 && z == 1) || t < least) { least = t; best = Plan{s, z}; }
         }
     }

@@ -75,6 +75,8 @@ def product(x, w, form=PLAIN, plan=None):
 def linear(x, w):
     """x . W^T, w [n, k] contiguous.  Up to 32 rows only large weights are the kernel's: 18 784 x 4 096 at 16 rows 67 -> 38 us, 4 096 x 11 008 29 -> 23,
     but 4 096 x 4 096 11.0 -> 11.7, 256 x 4 096 7.8 -> 10.0 (at 40 rows 12.6 -> 12.3 and 11.3 -> 9.8)."""
-    if (x.shape[0] > 32 or w.numel() > 1 << 25) and takes(x, w) and not library_fills(x.shape[0], w.shape[0]):
+    rows, n = x.shape[0], w.shape[0]
+    # (logits of a portion's last rows are the library's at 100 to 200 rows: 32 000 x 4 096, 128 rows 63 us against 72, 190 70 / 73, 220 77 / 74)
+    if (rows > 32 or w.numel() > 1 << 25) and not (100 < rows < 200 and n > 24576) and takes(x, w) and not library_fills(rows, n):
         return product(x, w)
     return F.linear(x, w)
