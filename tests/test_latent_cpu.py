@@ -126,6 +126,14 @@ def test_plan_of_attention_beside_a_product():
     assert ol.beside_plan(1, 20, 512, 32, 64, 4096, 11008) is None and ol.beside_plan(1, 20, 256, 64, 64, 4096, 11008) is None
 
 
+# rows, pages in all -> panels each: where one division was the fastest by 3 % or more (32 heads, 4 096 x 11 008)
+@pytest.mark.parametrize("rows,pages,each", [(1, 4, 2), (1, 64, 2), (1, 192, 2), (2, 114, 2), (4, 204, 2), (8, 54, 2), (8, 258, 2), (12, 438, 2), (16, 592, 2),
+                                             (24, 596, 2), (24, 1192, 3), (32, 32, 2), (32, 784, 2), (32, 1184, 3), (12, 870, 3), (24, 1788, 4)])
+def test_plan_picks_what_was_measured_fastest(rows, pages, each):
+    from triforce_amd import ops_latent as ol
+    assert ol.beside_plan(rows, 32, 512, 64, pages, 4096, 11008)[1] == each
+
+
 # ---- configuration and registry -------------------------------------------------------------------------------------------
 @pytest.mark.parametrize("name", sorted(H.CONFIGS))
 def test_config_round_trip_and_layer_order(name):

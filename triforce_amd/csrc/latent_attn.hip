@@ -492,8 +492,8 @@ __global__ __launch_bounds__(256 * HT, HT) void attn_latent_sized_kernel(const b
 // and CU behind 10 us of start, the product for up to 50.
 // Splits are dealt: as many pages each, 2 at least where a row has more than 16, as make the splits of all rows fit the workers; a row has
 // nsplit at most, with as many pages each as that takes.  Statistics of splits that a row does not have are zero, which the merge skips.
-// us, 20 heads, attention, merge and the output product (shorter by 11 008 of its 15 104), apart -> so: a row of 64 pages 36.6 -> 31.1, 32 rows of 48
-// 61.9 -> 59.9; of eight steps of six layer runs, one row of 4 000 keys 4 987 -> 4 668, 32 rows 7 500 -> 7 335.
+// us, 32 heads, attention, merge, value and the output product (shorter by 11 008 of its 15 104), apart -> so: a row of 64 pages 42.3 -> 35.4, 32 rows
+// with 1 184 pages 72.6 -> 64.0 (more beside beside_plan); of eight steps of six layer runs, one row of 4 000 keys 4 987 -> 4 668, 32 rows 7 500 -> 7 225.
 template <int P, int MT>
 __global__ __launch_bounds__(512, 2) void attn_latent_beside_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages,
                                                                     const int32_t* __restrict__ table, int table_ld, const int32_t* __restrict__ len,
@@ -633,25 +633,31 @@ extern "C" int tfl_attn_decode(const void* q, const void* cache, int n_pages, co
 }
 
 // How the CUs are shared between the attention of `pages` pages in all and a product of n outputs of k, or 0 workers where the two are better one
-// after the other.  The product takes up to half of the CUs, which draw all that memory gives (48 bytes a ns each).  us of a graph of both and the
-// rest of the output product, 20 heads, n 4096, k 11 008 of 15 104, apart -> beside on 128 CUs | 86 | 64:
-//   pages a row   1           8           16          32                  48                        64                        96
-//    1 row    29.0->30.1  32.7->30.3  32.8->30.7  35.7->30.5|36.9     36.4->31.0|37.7           36.6->31.1|37.7           37.4->31.7|38.1
-//    8 rows   29.9->33.4  34.2->34.3  35.8->36.0  39.0->36.5|43.8     40.3->37.8|44.8           41.5->37.7|45.0           45.1->44.4|46.6|52.1
-//   32 rows   39.1->44.5  46.0->46.7  49.8->47.3  56.3->52.2|55.6     61.9->63.6|59.9|63.3      67.2->75.1|68.7|64.5
-// A row of activations costs both sides 0.3 us (each group of panels reads all of x), a page 3 us of an attention on the whole chip and 2.8 behind 15
-// of one on part of it, a merge of splits 5.
+// after the other.  The product takes up to half of the CUs, which draw all that memory gives (39 bytes a ns each with their start).  us of a graph of
+// the attention, its merge, latent to value and the whole output product (32 heads, n 4096, k 11 008 of 15 104, rows half to all as long as the longest),
+// apart -> beside with the product on 128 CUs | 86 | 64:
+//   pages in all   one each               ~200                       ~600                      ~1 200                    ~2 400
+//    1 row    34.4->32.5|39.2|44.4   46.9->37.5|44.2|49.2      50.9->44.3|47.0|52.0 (512)
+//    8 rows   39.9->39.4|46.7|51.7   44.6->42.3|49.3|54.2      50.5->47.4|51.8|56.5      60.2->62.4|58.9|58.8      77.2->91.5|81.0|76.9 (6 rows)
+//   16 rows   45.4->42.2|50.5|56.2   46.9->45.5|53.0|57.7      53.1->46.7|54.8|59.5      62.7->61.3|59.4|61.4      77.1->90.4|81.8|76.7
+//   32 rows   57.4->53.0|59.2|65.4   55.8->54.4|60.7|66.6      61.8->54.9|62.7|68.4      72.6->68.5|64.0|70.3      87.1->97.4|84.4|82.4
+// The constants are fitted to these and to 530 other points (20 and 32 heads, 1 to 32 rows, 1 to 512 pages a row, n 4 096 to 8 192, k 2 048 to 16 384): what
+// they pick is 1.003 of the best on average, at most 1.03 of the two apart from k 4 096 on and 1.06 below.  At k 16 384 the product's half of the CUs is by
+// far the longer side: with fewer than 32 pages each, 8 to 32 rows took up to 1.09 of the two apart, with more 0.92 to 0.96.  A page costs 3.9 us of an
+// attention on the whole chip and 4.4 of one on part of it, a row of activations 0.5 in either form (each group of panels reads all of x).
 static int beside_plan(int rows, int H, int64_t pages, int n, int k, int* panels_each) {
     const int panels = n >> 4;
     if (rows < 1 || rows > 32 || H <= 16 || H > 32 || pages < 1 || pages > (1 << 20) || panels < 256 || panels > 512 || k < 2048) return 0;
-    const int row = (int)((pages + rows - 1) / rows), ns = tfl_attn_decode_splits(rows, H, 512, 64, row * TFL_PAGE, 0);
-    const double bytes = 2.0 * n * k, x = 0.3 * rows * k / 11008.0;
-    double least = bytes / 6.2e6 + 4.5 + 3.0 * ((row + ns - 1) / ns) + 0.9 * x - (ns == 1 ? 5.0 : 0.0) - 1.5;       // (apart)
+    if (k > 12288 && rows > 4 && pages < 32 * rows) return 0;
+    const int row = (int)((pages + rows - 1) / rows), ns = tfl_attn_decode_splits(rows, H, 512, 64, (int)pages * TFL_PAGE, 0);
+    const double bytes = 2.0 * n * k, heads = H / 32.0, x = rows * k / 11008.0;
+    double least = bytes / 6.2e6 + 13.35 + 3.9 * ((row + ns - 1) / ns) - 0.11 * rows + 0.47 * x + 0.005 * heads * rows * ns;        // (apart)
     int workers = 0;
     for (int p = 2; p <= 4; ++p) {
         const int g = (panels + p - 1) / p, a = 256 - g;
         if (g > 128) continue;
-        const double t = fmax(5.0 + bytes / g / 50e3 + x, 15.0 + 2.8 * (double)((pages + a - 1) / a));
+        const double product = 5.5 + bytes / g / 39e3 + 0.51 * x, attention = 7.85 + 4.45 * (double)pages / a + 2.0 * p;
+        const double t = fmax(product, attention) + (0.064 + 0.03 * heads) * rows + 0.005 * heads * (double)(pages < a ? pages : a);
         if (t < least) { least = t; workers = a; *panels_each = p; }
     }
     return workers;

@@ -199,16 +199,21 @@ def attn_decode(q, cache, table, klen, g, scale, max_len, nsplit=None):
     return out
 
 
-VALUE_ROWS, VALUE_PARTS = 4, 80      # up to which latent_to_value merges the splits itself, see latent_value_kernel
+def _value_merges(rows, H, nsplit, parts):
+    """Does latent_to_value merge the splits of attn_decode_beside itself (latent_value_kernel) or a launch in front of it?  us of a layer's attention,
+    value and output product, launch -> itself: one row 35.4 -> 33.3 (64 pages), 40.0 -> 39.4 (256); two 36.4 -> 35.5 (46 splits), 36.7 -> 35.9 (60),
+    38.2 -> 39.0 (88); three rows the same to 1 %; four rows of 32 heads, whose merge is a wave for 128 columns (launch_merge: from 128 heads
+    on, up to 64 splits), 40.3 -> 38.8 with 64 splits a row, with 85 48.2 -> 50.4; four of 20 heads 35.2 -> 36.1."""
+    return rows == 1 or (rows == 2 and parts <= 72) or (rows <= 4 and rows * H >= 128 and nsplit <= 64)
 
 
 @functools.lru_cache(maxsize=1024)
 def beside_plan(rows, H, C, R, pages, n, k):
-    """(workers, panels each, splits, does latent_to_value merge them) of attn_decode_beside for rows with ``pages`` pages in all and a
+    """(workers, panels each, splits, does latent_to_value merge them) of attn_decode_beside for rows that hold ``pages`` pages in all and a
     product of n outputs of k, None where the two are better launched apart."""
     each, nsplit, parts = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
     workers = hip.latent_lib().tfl_attn_beside_plan(rows, H, C, R, pages, n, k, ctypes.byref(each), ctypes.byref(nsplit), ctypes.byref(parts))
-    return (workers, each.value, nsplit.value, rows <= VALUE_ROWS and parts.value <= VALUE_PARTS) if workers > 0 else None
+    return (workers, each.value, nsplit.value, _value_merges(rows, H, nsplit.value, parts.value)) if workers > 0 else None
 
 
 class Splits:
