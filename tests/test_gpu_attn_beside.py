@@ -86,6 +86,42 @@ def test_value_of_unmerged_splits(lens, heads, V, plan):
     assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * size / 8 + 1e-6).all()
 
 
+@pytest.mark.parametrize("plan", [(128, 2, 64), (170, 3, 85)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_values_that_are_not_finite(bad, plan):
+    """A query and a cached row with such a value give what the two launches apart give, and other rows and heads what they give without."""
+    from triforce_amd import ops_latent as ol
+    lens, heads, V = [700, 130, 64, 300], 32, 32
+    cache, table, keys = _paged(lens, 512, 64, torch.bfloat16, 5)
+    q = rnd(4, heads, 576, seed=1, dtype=torch.bfloat16)
+    klen = torch.tensor(lens, dtype=torch.int32, device=q.device)
+    act, w, wt, x = _block(4, 4096, 1024, 2048, 7)
+    g, octs = Geom(heads, 32, 64, V, 512, 32), octets(act)
+    raw, value = rnd(4, heads * V, seed=3), ol.TileWeight(rnd(heads, V, 512, seed=4, dtype=torch.bfloat16, scale=512 ** -0.5), packed_only=True)
+
+    def run(q, cache, later):
+        got, sums = ol.empty_act(4, heads * V, torch.bfloat16, q.device), x.clone()
+        o = ol.attn_decode_beside(q, cache, table, klen, g, SCALE, plan + (later,), octs, wt, sums, 1024)
+        ol.latent_to_value(o, value, raw, 0, got, g)
+        return (None if later else o), got.permute(1, 0, 2).reshape(4, heads, V), sums
+    clean = {later: run(q, cache, later) for later in (False, True)}
+    q2, cache2 = q.clone(), cache.clone()
+    q2[0, 3, 17] = bad                                     # one head of row 0, and every head of row 2 through its first page
+    cache2[int(table[2, 0]) * 64 + 5, 11] = bad
+    apart = ol.attn_decode(q2, cache2, table, klen, g, SCALE, max(lens))
+    spoilt = torch.zeros(4, heads, dtype=torch.bool, device=q.device)
+    spoilt[0, 3] = spoilt[2] = True
+    for later in (False, True):
+        merged, values, sums = run(q2, cache2, later)
+        assert torch.equal(sums, clean[later][2]) and torch.equal(values[~spoilt], clean[later][1][~spoilt])
+        if merged is not None:
+            assert torch.equal(merged[~spoilt], clean[later][0][~spoilt])
+            assert torch.equal(merged.isnan(), apart.isnan()) and torch.equal(merged.isinf(), apart.isinf())
+            together = values.isnan()
+        else:
+            assert torch.equal(values.isnan(), together)
+
+
 def test_replays_in_a_graph():
     """Lengths that change between replays: the deal of the splits is made on the device."""
     from triforce_amd import ops_latent as ol
@@ -111,3 +147,46 @@ def test_replays_in_a_graph():
         want = run(fresh)
         torch.cuda.synchronize()
         assert torch.equal(out, want) and torch.equal(keep, fresh)
+
+
+def _model():
+    from tests import latent_helpers as lh
+    from triforce_amd.models.config_befidra import BefidraConfig
+    from triforce_amd.models.modeling_befidra import BefidraForCausalLM
+    cfg = lh.config(96, 4096, [(lh.mixer(17, 32, 64, 32, 64, 512), 11008)])
+    return BefidraForCausalLM(BefidraConfig.from_dict(cfg)).init_random(3)
+
+
+def _filled(model, budget, lens, graphs):
+    from triforce_amd.utils.batch_infer import BatchInferenceEngine
+    e = BatchInferenceEngine(model, model.make_cache(budget, max_batch=len(lens)), use_graphs=graphs)
+    e.kv_cache.extend([(s, n) for s, n in enumerate(lens)])
+    for s, n in enumerate(lens):
+        for block in e.kv_cache.rows:
+            block[e.kv_cache.cache_rows(s, 0, n).long().cuda()] = rnd(n, block.shape[1], seed=s, dtype=block.dtype)
+    return e
+
+
+@pytest.mark.parametrize("lens", [[200], [700, 90, 300, 64, 1, 500, 250, 63], [130 * b for b in range(1, 33)]], ids=lambda v: str(len(v)))
+def test_steps_do_not_depend_on_the_room_in_the_cache(lens):
+    """A server's cache is larger than its load: the same launches, and the same bits, as in a cache that is full."""
+    model = _model()
+    tight, roomy = (_filled(model, n, lens, True) for n in (sum(lens) + 8 * len(lens), 400000))
+    names, ids = list(range(len(lens))), torch.arange(len(lens)) % 96
+    for t in range(3):
+        assert torch.equal(tight.decode(names, ids + t), roomy.decode(names, ids + t))
+    forms = [list(e._steps[len(lens)].graphs) for e in (tight, roomy)]
+    assert forms[0] == forms[1] and forms[0][0][0] is not None
+
+
+def test_a_graph_for_each_form_of_the_step():
+    """Few pages and many in turn, by replays and eagerly: the same logits, and a graph for each form, whichever rows are live."""
+    model = _model()
+    lens = [60 + 3 * b for b in range(8)] + [8000 - 16 * b for b in range(8)]
+    graphs, eager = (_filled(model, sum(lens) + 1000, lens, g) for g in (True, False))
+    few, many = list(range(8)), list(range(8, 16))
+    for t, names in enumerate((few, many, few, few, many, few)):
+        ids = (torch.arange(8) * 7 + t) % 96
+        assert torch.equal(graphs.decode(names, ids), eager.decode(names, ids)), t
+    forms = list(graphs._steps[8].graphs)
+    assert forms == [model.decode_form(8, sum(n // 64 + 1 for n in ls)) for ls in (lens[:8], lens[8:])] and len(set(forms)) == 2

@@ -68,6 +68,15 @@ class LatentLayer:
     def weights(self):
         return [self.w_in, self.w_uq, self.w_uk_t, self.w_uv, self.w_out] + ([self.side_gate, self.side_proj] if self.side_dim else [])
 
+    def beside(self, rows, pages):
+        """How attention and the feed-forward's half of the output product share the chip in a decode step of rows that hold ``pages`` pages in
+        all (ops_latent.beside_plan); None: one after the other, as where nobody knows the pages.  (What they hold, not what the cache could:
+        for the product a CU too few costs more than a page's attention on one CU more.)"""
+        g = self.geom
+        if pages is None or not self.ff or not self.w_out.chunk_major or self.w_out.dtype != torch.bfloat16:
+            return None
+        return ol.beside_plan(rows, g.H, g.C, g.R, pages, self.w_out.n, self.w_out.k - g.H * g.V)
+
     # -- the two forms of a layer: h (normed input), x (fp32 residual, updated) -> y (token-side output, added by the next norm) ----
     def decode(self, h, x, ids, side_table, batch, rope, cache_rows, eps):
         g = self.geom
@@ -76,10 +85,7 @@ class LatentLayer:
         qn, q = ol.query_and_append(xq, raw, ss, self.w_uq, g, self.kv_norm, eps, rope, batch.pos, batch.slot, cache_rows)
         ol.query_to_latent(qn, self.w_uk_t, q, g)
         own = g.H * g.V                                       # act: the attention's columns, then the feed-forward's, which wait for nothing of it
-        # (max_len is the cache's capacity; contexts that grow to it are half to all of it long.  32 rows of 2 000 to 4 000 keys, planned for
-        # all pages, 7 309 us for eight steps of six layer runs, for three quarters 7 225)
-        plan = ol.beside_plan(ids.numel(), g.H, g.C, g.R, -(-3 * batch.max_len // (4 * ol.PAGE)), self.w_out.n, self.w_out.k - own) \
-            if self.ff and self.w_out.chunk_major and h.dtype == torch.bfloat16 else None
+        plan = self.beside(ids.numel(), batch.pages)
         if plan is None:
             o = ol.attn_decode(q, cache_rows, batch.table, batch.klen, g, self.scale, batch.max_len)
         else:
@@ -113,7 +119,7 @@ class LatentWeights:
 
     def __init__(self, cfg, device, dtype):
         self.cfg, self.device, self.dtype = cfg, torch.device(device), dtype
-        self.layers = []
+        self.layers, self.kinds = [], []          # kinds: a layer of every set of sizes
         self.embed = self.logits = self.final_norm = self.side_embed = self.step = None
         self.capture = None       # list -> the forward appends the residual stream after every layer run (comparisons)
 
@@ -150,7 +156,12 @@ class LatentWeights:
             self.side_embed = get("side.embed").to(self.dtype).contiguous()
         self.layers = [LatentLayer(s, c.hidden_size, c.side_dim, lambda n, i=i: get(f"l{i}." + n), self.dtype)
                        for i, s in enumerate(c.layers)]
+        self.kinds = list({(L.geom.H, L.geom.V, L.geom.C, L.geom.R, L.ff, L.w_out.n): L for L in self.layers}.values())
         return self
+
+    def decode_form(self, rows, pages):
+        """What a decode step's launches depend on besides the number of rows: equal for steps that one captured graph serves."""
+        return tuple(L.beside(rows, pages) for L in self.kinds)
 
     def load_state_dict(self, sd):
         want = self.shapes()

@@ -70,6 +70,10 @@ class BefidraForCausalLM:
             self._rope = {k: RotaryTable(s, n, self.device) for k, s in specs.items()}
 
     # -- forward -----------------------------------------------------------------------------
+    def decode_form(self, rows, pages):
+        """Key of the decode step's launches for ``rows`` sequences that hold ``pages`` cache pages in all."""
+        return self.weights.decode_form(rows, pages)
+
     @torch.inference_mode()
     def __call__(self, input_ids, kv_cache=None, graph_cache=None, position_ids=None, **_):
         return self.forward(input_ids, kv_cache)

@@ -1,7 +1,7 @@
 """Engine for targets that are served autoregressively in batches (models with ``forward_batch``): prompts are prefilled
-together as one packed batch, then the sequences advance in lockstep, one token each, through one captured hipGraph per batch
-size.  It has the surface the decode loops drive (``engine``, ``inference``, ``decode_step``, ``clear_kv``) plus ``step`` for
-batches of named sequences."""
+together as one packed batch, then the sequences advance in lockstep, one token each, through captured hipGraphs: one per batch
+size, and where the best launches depend on how much context there is, a few.  It has the surface the decode loops drive
+(``engine``, ``inference``, ``decode_step``, ``clear_kv``) plus ``step`` for batches of named sequences."""
 import os
 
 import torch
@@ -22,13 +22,18 @@ class _DecodeBuffers:
         self.B, self.columns = B, cache.columns
         self.ids = torch.zeros(B, dtype=torch.int64, device=dev)
         image = torch.zeros(B * (2 + self.columns), dtype=torch.int32, device=dev)      # lengths | seats | table
-        self.lens, self.seat, self.table = self._parts(image)
-        self.lens.fill_(-1)                                                             # -1: idle row
-        self.seat.fill_(-1)
+        self.lens, self.seat, self.table = self._parts(image)                           # (length or seat -1: idle row)
         self.pos, self.slot, self.klen = (torch.zeros(B, dtype=torch.int32, device=dev) for _ in range(3))
         self.batch = PagedBatch(True, self.pos, self.slot, table=self.table, klen=self.klen, seat=self.seat, max_len=cache.max_budget)
         self.image, self.staged, self.sent = image, torch.zeros(image.shape, dtype=torch.int32, pin_memory=image.is_cuda), None
         self.current, self.known = None, [0] * B                # (births, lengths) the device holds; pages of each row it knows
+        self.idle()
+
+    def idle(self):
+        """No row is a sequence's: nothing is stored, and everything is sent again afterwards."""
+        self.lens.fill_(-1)
+        self.seat.fill_(-1)
+        self.current = None
 
     def _parts(self, flat):
         return flat[:self.B], flat[self.B:2 * self.B], flat[2 * self.B:].view(self.B, self.columns)
@@ -61,13 +66,20 @@ class _DecodeBuffers:
 
 
 class _DecodeStep:
-    """The lockstep decode forward of B sequences: eager, or captured once and replayed."""
+    """The lockstep decode forward of B sequences: eager, or captured and replayed.  How the launches share the chip may depend on how
+    many pages the sequences hold: there is a graph for each of the model's ``decode_form``s (a handful), captured when a step first asks for
+    it, as the first one is for a new B."""
 
     def __init__(self, model, cache, B, use_graph):
-        self.model, self.cache, self.buf = model, cache, _DecodeBuffers(cache, B)
-        self.graph = self.logits = None
-        if use_graph:                                           # warm-up and capture run on idle rows: nothing is stored
-            self.graph, self.logits = graph_infer._capture(self._run, (), None, 2)
+        self.model, self.cache, self.buf, self.use_graph = model, cache, _DecodeBuffers(cache, B), use_graph
+        self.graphs = {}                                        # form -> (graph, logits), in one pool: of these only one runs at a time
+
+    def _graph(self, form):
+        if form not in self.graphs:                             # warm-up and capture run on idle rows: nothing is stored
+            self.buf.idle()
+            pool = next(iter(self.graphs.values()))[0].pool() if self.graphs else None
+            self.graphs[form] = graph_infer._capture(self._run, (), pool, 2)
+        return self.graphs[form]
 
     def _run(self):
         b = self.buf
@@ -79,6 +91,8 @@ class _DecodeStep:
         until the next call."""
         b, c = self.buf, self.cache
         before = tuple(c.length.get(s, 0) for s in seqs)
+        b.batch.pages = sum(n // c.page + 1 for n in before)    # with this step's token
+        graph, logits = self._graph(self.model.decode_form(b.B, b.batch.pages)) if self.use_graph else (None, None)
         c.extend([(s, 1) for s in seqs])
         births = tuple(c.birth[s] for s in seqs)
         if b.current != (births, before):
@@ -87,10 +101,10 @@ class _DecodeStep:
             b.add_pages(c, seqs)
         b.current = (births, tuple(n + 1 for n in before))
         b.ids.copy_(ids)
-        if self.graph is None:
+        if graph is None:
             return self._run()
-        self.graph.replay()
-        return self.logits
+        graph.replay()
+        return logits
 
 
 class BatchInferenceEngine:
