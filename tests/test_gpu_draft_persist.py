@@ -254,3 +254,9 @@ def test_engine_draft_step_in_one_launch_equals_its_graph(sd68, monkeypatch):
                 continue
             assert not ge._draft_is_one_launch(other, off)
             assert torch.equal(ge.graph_draft_inference(other, gamma_offset=off), want)
+    # what the launch needs besides the tokens was settled when the graph was captured: a call asks the model and the library nothing more
+    for name in ("forward", "one_launch", "_native_model", "_native_cache"):
+        monkeypatch.setattr(m, name, None)
+    monkeypatch.setattr(ops, "draft_persist_supported", None)
+    ids = torch.tensor([[5, 900, 31999]], device=DEV)
+    assert torch.equal(ge.graph_draft_inference(ids, gamma_offset=2), ge.callables[2](ids))

@@ -93,11 +93,15 @@ class LlamaForCausalLM:
             self._native_cache_ref = c                                  # keeps id(c) from being recycled
         return self._native_cache_struct
 
-    def one_launch(self, c, gamma_offset):
-        """Is a speculative step of gamma_offset + 1 tokens on the cache ``c`` one launch (ops.DraftPersist)?"""
-        n = gamma_offset + 1
-        return (n <= min(ops.SKINNY_MAX_ROWS, c.gamma + 3) and self._native_model() is not None and self._persist is not None and ops.DRAFT_PERSIST
-                and ops.draft_persist_supported(self._native, n, gamma_offset + c.start_size + c.recent_size + 1))
+    def one_launch(self, c, gamma_offset, probs):
+        """The speculative step of gamma_offset + 1 tokens on the cache ``c`` as one launch over these weights (ops.DraftStep), None where it is
+        more than one."""
+        n, kv_len, W = gamma_offset + 1, gamma_offset + c.start_size + c.recent_size + 1, self.weights
+        if n > min(ops.SKINNY_MAX_ROWS, c.gamma + 3) or self._native_model() is None or self._persist is None or not ops.DRAFT_PERSIST \
+                or not ops.draft_persist_supported(self._native, n, kv_len):
+            return None
+        keep = (c, W.embed, tuple(W.ln1), tuple(W.wqkv), tuple(W.wo), tuple(W.ln2), tuple(W.wgu), tuple(W.wd), W.norm, W.lm_head, self.cos, self.sin)
+        return ops.DraftStep(self._native, self._native_cache(c), self._persist, n, c.spec_slot, kv_len, probs, keep)
 
     def forward(self, input_ids, kv_cache, graph_cache=None, gamma_offset=-1, probs=None):
         """``probs`` = (temperature, top_p): also return the top-p probability row of the last token (out.probs)."""

@@ -749,6 +749,33 @@ def draft_forward(model, cache, ids, slot0, kv_len, probs=None, persist=None):
     return logits, p
 
 
+class DraftStep:
+    """draft_forward's one launch with everything but the tokens settled, as a captured graph has it: n tokens into slot0 .. of one cache, kv_len
+    keys, the top-p row of the last token (``probs``) or its logits.  ``keep``: what the structs point into.  A call is two allocations and
+    the launch (16 us of the host's time through the model's forward)."""
+
+    def __init__(self, model, cache, persist, n, slot0, kv_len, probs, keep):
+        self.device, self.shape, self.vocab, self.probs = persist.ctl.device, (1, n), model.vocab, probs
+        self.keep = (model, cache, persist, keep)
+        T, top_p = probs if probs is not None else (1.0, 1.0)
+        self.fn = hip.lib().tf_draft_forward_68m_persist
+        self.head = ctypes.byref(model), ctypes.byref(cache)
+        self.sizes = n, int(slot0), int(kv_len)
+        self.tail = float(T), float(top_p), _ptr(persist.ws), persist.ws.numel(), _ptr(persist.ctl)
+
+    def takes(self, ids):
+        """Tokens that the launch can read where they are."""
+        return (isinstance(ids, torch.Tensor) and ids.shape == self.shape and ids.dtype == torch.int64 and ids.device == self.device
+                and ids.is_contiguous() and self.device.index == torch.cuda.current_device())
+
+    def __call__(self, ids):
+        logits = torch.empty(*self.shape, self.vocab, dtype=torch.float32, device=self.device)
+        p = torch.empty(self.vocab, dtype=torch.float32, device=self.device) if self.probs is not None else None
+        hip.check(self.fn(*self.head, ids.data_ptr(), *self.sizes, logits.data_ptr(), None if p is None else p.data_ptr(), *self.tail,
+                          torch.cuda.current_stream().cuda_stream), "tf_draft_forward_68m_persist")
+        return logits if p is None else p
+
+
 def attn_rope_on_read(q, k_layer, v_layer, cos, sin, kv_len, scale):
     """Draft attention: cached keys are un-rotated and rotated on read with positions 0..kv_len-1."""
     _dev(q, k_layer, v_layer, cos, sin)
