@@ -123,11 +123,14 @@ def test_captured_with_parts_of_k():
         assert torch.equal(ops_rows.linear(x, w), want)
 
 
-def test_wide_products_of_some_rows_are_the_librarys(monkeypatch):
+def test_products_that_the_library_is_faster_at_are_the_librarys(monkeypatch):
+    """Plain products and gated units at sizes that were timed (the rule itself: test_sizes_of_the_kernel_and_of_the_library)."""
     taken = []
-    monkeypatch.setattr(ops_rows, "product", lambda x, w: taken.append(x.shape[0]) or F.linear(x, w))
-    w = torch.zeros(24592, 64, dtype=torch.float16, device="cuda")
-    for rows in (100, 101, 199, 200):
-        ops_rows.linear(torch.zeros(rows, 64, dtype=torch.float16, device="cuda"), w)
-        ops_rows.linear(torch.zeros(rows, 64, dtype=torch.float16, device="cuda"), w[:24576])
-    assert taken == [100, 100, 101, 199, 200, 200]
+    monkeypatch.setattr(ops_rows, "product", lambda x, w, form=ops_rows.PLAIN: taken.append((x.shape[0], form)) or F.linear(x, w))
+    w = torch.zeros(12288, 4096, dtype=torch.float16, device="cuda")
+    for rows in (33, 112, 650, 1300):
+        x = torch.zeros(rows, 4096, dtype=torch.float16, device="cuda")
+        ops_rows.linear(x, w)
+        assert (ops_rows.glu_linear(x, w, ops_rows.SILU_HALVES) is None) == (rows == 112)
+        assert ops_rows.glu_linear(x, w, ops_rows.GELU_EIGHTS) is None
+    assert taken == [(33, 0), (33, 1), (650, 1), (1300, 0), (1300, 1)]

@@ -328,34 +328,35 @@ template <typename T, int FORM> __global__ __launch_bounds__(256) void rows_sum_
 }
 
 // Tiles: rows, outputs, workgroups that share a CU, and in us what a step costs where a CU is full and at least, and what a tile costs besides.
-// Fitted to 16 products of 768 .. 27 648 outputs at 23 counts of rows from 40 to 6 000, every tile and every number of parts of each timed: the
-// one picked is 1.02 of the best on average.  (Tiles of 160 x 64, 96 x 128 and 128 x 128 were the best of all nowhere by more than 1 %.)
+// Fitted to 24 products of 256 .. 32 000 outputs and 256 .. 15 104 columns at 57 counts of rows from 33 to 8 000, weights from memory, every tile with
+// 1 to 16 parts of each timed: the one picked is 1.006 of the best on average, more than 1.05 in one of 18.  (Tiles of 160 x 64, 96 x 128 and 128 x 128 were
+// the best of all nowhere by more than 1 %.)
 struct Shape { int rows, cols, per_cu; float step, least, tile; };
-constexpr Shape SHAPES[] = {{256, 256, 1, 1.269f, 0.60f, 3.2f}, {224, 256, 1, 1.141f, 0.60f, 2.0f}, {192, 256, 1, 1.119f, 0.60f, 1.7f}, {160, 256, 1, 1.009f, 0.60f, 1.2f},
-                            {128, 256, 1, 0.542f, 0.77f, 1.2f}, {64, 128, 2, 0.302f, 0.28f, 0.5f}, {96, 64, 2, 0.248f, 0.07f, 0.4f}, {64, 64, 2, 0.165f, 0.01f, 0.6f}};
+constexpr Shape SHAPES[] = {{256, 256, 1, 1.268f, 0.60f, 7.1f}, {224, 256, 1, 1.173f, 0.60f, 4.5f}, {192, 256, 1, 1.108f, 0.60f, 4.6f}, {160, 256, 1, 1.044f, 0.60f, 2.4f},
+                            {128, 256, 1, 0.542f, 0.79f, 2.8f}, {64, 128, 2, 0.323f, 0.28f, 0.07f}, {96, 64, 2, 0.241f, 0.07f, 0.18f}, {64, 64, 2, 0.179f, 0.03f, 0.17f}};
 constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 struct Plan { int shape, splits; };
 
-// The bytes each operand needs at 6.5 TB/s; the steps of a CU's tiles, one or two at a time; parts of k are written and read at 4 TB/s by
+// The bytes each operand needs at 7.1 TB/s; the steps of a CU's tiles, one or two at a time; parts of k are written and read at 4 TB/s by
 // another launch.  XCDs take an eighth of the tiles each, and their 32 CUs whole ones.  Small tiles in number are bound by what they read from L2,
-// 17 TB/s (12 288 x 4 096: 190 rows 47 -> 41 us by another tile, 255 rows 53 -> 47, 350 rows 62 -> 57; 4 096 x 11 008, 255 rows 51 -> 42).
+// 20 TB/s (12 288 x 4 096: 190 rows 47 -> 41 us by another tile, 255 rows 53 -> 47, 350 rows 62 -> 57; 4 096 x 11 008, 255 rows 51 -> 42).
 inline Plan plan(int rows, int n, int k) {
     const int nk = k >> 6;
-    const double mem = (2.0 * n * k + 2.0 * rows * k + 2.0 * rows * n) / 6.5e6;
+    const double mem = (2.0 * n * k + 2.0 * rows * k + 2.0 * rows * n) / 7.1e6;
     Plan best{0, 1};
     double least = 0;
     for (int s = 0; s < N_SHAPES; ++s) {
         const Shape& h = SHAPES[s];
         const int64_t tiles = (int64_t)((rows + h.rows - 1) / h.rows) * ((n + h.cols - 1) / h.cols);
-        const double l2 = h.per_cu > 1 ? (double)tiles * nk * (h.rows + h.cols) * 128 / 17e6 : 0.0;
+        const double l2 = h.per_cu > 1 ? (double)tiles * nk * (h.rows + h.cols) * 128 / 20e6 : 0.0;
         for (int z = 1; z <= 16; ++z) {
             const int per = (nk + z - 1) / z;
             if (z > 1 && ((z - 1) * per >= nk || per < 4 || tiles * z > 410 * h.per_cu || (int64_t)z * rows * n > (int64_t)1 << 28)) continue;
             const int64_t a_cu = ((tiles * z + 7) / 8 + 31) / 32, full = a_cu / h.per_cu;
             const double fully = per * (double)fmaxf(h.per_cu * h.step, h.least) + h.per_cu * h.tile;
             const double work = full * fully + (a_cu > full * h.per_cu ? per * (double)fmaxf(h.step, h.least) + h.tile : 0.0);
-            const double t = cbrt(work * work * work + mem * mem * mem + l2 * l2 * l2) + (z > 1 ? 3.0 + z * 4.0 * rows * n / 4.3e6 : 0.0);
+            const double t = cbrt(work * work * work + mem * mem * mem + l2 * l2 * l2) + (z > 1 ? 2.55 + z * (0.18 + 4.0 * rows * n / 4.2e6) : 0.0);
             if ((s == 0 && z == 1) || t < least) { least = t; best = Plan{s, z}; }
         }
     }

@@ -383,7 +383,8 @@ def linear(x, w, out_f32=False, ln=None, eps=0.0, resid=None, out=None, ss_in=No
 
 def mlp_act(h, wgu, ln=None, eps=0.0, ss_in=None):
     """fp16(silu(gate(h))) * up(h) for a fused gate|up weight: one kernel for <=32 rows (optionally with the
-    RMSNorm of h folded in, ``ln``), the product of many rows with the unit in its epilogue (or GEMM + silu_mul) otherwise.  An Act input gives an Act output."""
+    RMSNorm of h folded in, ``ln``), the product of many rows with the unit in its epilogue (or GEMM + silu_mul) otherwise.
+    An Act input gives an Act output."""
     M = h.shape[0]
     if isinstance(wgu, PackedLinear) and wgu.parts is not None and wgu.split == 2 and M <= SKINNY_MAX_ROWS \
             and h.is_cuda:
@@ -402,9 +403,8 @@ def mlp_act(h, wgu, ln=None, eps=0.0, ss_in=None):
         return act
     assert ln is None and not isinstance(h, Act), "fused mlp_act needs the skinny kernel (ops.can_fuse)"
     w = _w(wgu)
-    if ops_rows.takes(h, w, ops_rows.SILU_HALVES):
-        return ops_rows.product(h, w, ops_rows.SILU_HALVES)
-    return silu_mul(F.linear(h, w))
+    act = ops_rows.glu_linear(h, w, ops_rows.SILU_HALVES)
+    return silu_mul(F.linear(h, w)) if act is None else act
 
 
 def ss_buffer(hidden, device):

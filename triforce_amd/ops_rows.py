@@ -38,11 +38,28 @@ def takes(x, w, form=PLAIN):
 
 
 def library_fills(rows, n):
-    """Do tiles of 256 x 256 fill whole rounds of the 256 CUs?  There the library's kernel is the faster one, for a plain product: 4 096 x 4 096 x
-    4 096 93.9 us against 98.5, 4 096 x 12 288 282 against 293, 8 000 x 4 096 x 11 008 480 against 487; where they do not, the other way
-    round (3 100 x 12 288 x 4 096 256 against 245, 3 100 x 22 016 547 against 425)."""
+    """Do tiles of 256 x 256 fill whole rounds of the 256 CUs?  There the library's kernel is the faster one, for a plain product of more than
+    1 152 columns: 4 096 x 4 096 x 4 096 93.9 us against 98.5, 4 096 x 12 288 282 against 293, 8 000 x 4 096 x 11 008 480 against 487 (but
+    4 096 x 8 192 x 512 41 against 38); where they do not, the other way round (3 100 x 12 288 x 4 096 256 against 245, 3 100 x 22 016
+    547 against 425)."""
     tiles = -(-rows // 256) * -(-n // 256)
     return tiles % 256 == 0 and 100 * rows * n >= 97 * 65536 * tiles
+
+
+def library_is_faster(rows, n, k, form=PLAIN):
+    """Is the library's product (and the unit's launch behind it) the faster one from 33 rows on?  The kernel's time over the library's, of 24 products of
+    256 .. 32 000 outputs and 256 .. 15 104 columns at 57 counts of rows up to 8 000, weights from memory:
+      * up to 1 152 columns 0.4 to 1.05;  from 9 600 on 0.45 to 1.0 up to 2 000 rows (4 096 x 11 008, 700 rows 88 -> 71 us) and 0.6 to 1.1 above;
+      * between, with a gated unit 0.63 to 1.03, but from 65 to 160 rows 1.02 to 1.2 (22 016 x 4 096, 100 rows 48 -> 51 us; 27 648 x 5 120 0.92 to 1.04);
+      * between, plain, up to 2^32 multiply-adds 0.56 to 1.07 (4 096 x 4 096, 160 rows 26 -> 18 us); from 6e10 on 0.62 to 1.1 (12 288 x 4 096, 6 000 rows
+        566 -> 462); from one to the other 0.99 on average, 0.6 to 1.25 case by case: the library's tiles are the better ones where they fill
+        one round of the CUs (4 096 x 4 096, 768 rows 36 -> 41; 12 288 x 4 096, 112 rows 31.5 -> 35.5), and the only ones it had there before;
+      * few outputs: its own parts of k serve 512 to 2 048 (768 x 3 072, 100 rows 7.6 -> 9.2 us), not fewer (256 x 4 096, 100 rows 11.3 -> 9.2)."""
+    if k <= 1152:
+        return False
+    if form != PLAIN:
+        return 64 < rows <= 160 and k <= 9600
+    return library_fills(rows, n) or (k <= 9600 and n > 512 and (n < 2048 or 1 << 32 < rows * n * k < 60e9))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -75,8 +92,11 @@ def product(x, w, form=PLAIN, plan=None):
 def linear(x, w):
     """x . W^T, w [n, k] contiguous.  Up to 32 rows only large weights are the kernel's: 18 784 x 4 096 at 16 rows 67 -> 38 us, 4 096 x 11 008 29 -> 23,
     but 4 096 x 4 096 11.0 -> 11.7, 256 x 4 096 7.8 -> 10.0 (at 40 rows 12.6 -> 12.3 and 11.3 -> 9.8)."""
-    rows, n = x.shape[0], w.shape[0]
-    # (logits of a portion's last rows are the library's at 100 to 200 rows: 32 000 x 4 096, 128 rows 63 us against 72, 190 70 / 73, 220 77 / 74)
-    if (rows > 32 or w.numel() > 1 << 25) and not (100 < rows < 200 and n > 24576) and takes(x, w) and not library_fills(rows, n):
+    if takes(x, w) and (x.shape[0] > 32 or w.numel() > 1 << 25) and not library_is_faster(x.shape[0], *w.shape):
         return product(x, w)
     return F.linear(x, w)
+
+
+def glu_linear(x, w, form):
+    """The gated unit ``form`` of x . W^T in one launch, None where it is not one or the product and the unit apart are faster."""
+    return product(x, w, form) if takes(x, w, form) and not library_is_faster(x.shape[0], *w.shape, form) else None

@@ -98,7 +98,7 @@ class TileWeight:
     def glu_matmul(self, x):
         """gelu_tanh(gate) * up of x . W^T over many rows in bfloat16, the weight interleave_glu(gate, up); None where it is not one launch."""
         assert self.groups == 1 and x.dtype == self.dtype
-        return ops_rows.product(x, self.w, ops_rows.GELU_EIGHTS) if ops_rows.takes(x, self.w, ops_rows.GELU_EIGHTS) else None
+        return ops_rows.glu_linear(x, self.w, ops_rows.GELU_EIGHTS)
 
 
 def empty_act(rows, k, dtype, device):
