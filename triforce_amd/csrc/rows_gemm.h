@@ -41,8 +41,8 @@ template <> struct El<__bf16> {
     static __device__ __forceinline__ void add(Frag a, Frag b, f32x4& c) { c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
     static __device__ __forceinline__ void add_in_place(Frag a, Frag b, f32x4& c) { asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b)); }
 };
-// Twelve wait states between products and what else touches their sums: a product of 16 cycles needs at most eight.  Behind the products of a
-// step, inside their loop, so that no copy of a sum can come first.
+// Twelve wait states between products and what else touches their sums: behind a 16 x 16 x 32 product (eight passes) eleven are needed.  Behind the
+// products of a step, inside their loop, so that no copy of a sum can come first.
 __device__ __forceinline__ void hold() {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_nop 11" ::: "memory");
