@@ -90,6 +90,31 @@ def test_infinities_and_nan_stay_in_their_rows():
         assert float((y[rest].double() - clean[rest].double()).abs().max()) < 4e-3 and bool(y[rest].isfinite().all())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("plan", [(0, 1), (4, 1), (4, 2), (7, 1), (7, 3)])
+def test_values_that_are_not_finite_through_the_units(dtype, plan):
+    """Infinities, NaN and sums beyond the type's range: as the library's product and the unit's own launch treat them, and other rows untouched."""
+    from triforce_amd import ops, ops_hybrid
+    unit = ops_rows.SILU_HALVES if dtype == torch.float16 else ops_rows.GELU_EIGHTS
+    x, w = _operands(300, 512, 320, dtype)
+    plain, clean = ops_rows.product(x, w, plan=plan), ops_rows.product(x, w, unit, plan=plan)
+    bad = x.clone()
+    big = 6e4 if dtype == torch.float16 else 3e38
+    bad[17, 3], bad[40, 300], bad[90, 5], bad[200] = float("inf"), float("nan"), -float("inf"), big * torch.sign(x[200])
+    rows = [17, 40, 90, 200]
+    rest = [i for i in range(300) if i not in rows]
+    y, got = ops_rows.product(bad, w, plan=plan), ops_rows.product(bad, w, unit, plan=plan)
+    assert torch.equal(y[rest], plain[rest]) and torch.equal(got[rest], clean[rest])
+    assert bool(y[40].isnan().all()) and not bool((y[17].isfinite() | y[90].isfinite()).any()) and bool(got[40].isnan().all())
+    library = F.linear(bad, w)
+    apart = ops.silu_mul(library) if unit == ops_rows.SILU_HALVES else ops_hybrid.glu(library)
+    for a, b in ((y[[17, 40, 90]], library[[17, 40, 90]]), (got[[17, 40, 90]], apart[[17, 40, 90]])):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isposinf(), b.isposinf()) and torch.equal(a.isneginf(), b.isneginf())
+    # the unit of the kernel's own sums, where they leave the type's range or do not
+    own = ops.silu_mul(y) if unit == ops_rows.SILU_HALVES else ops_hybrid.glu(y)
+    assert torch.equal(got[200].isnan(), own[200].isnan()) and torch.equal(got[200].isinf(), own[200].isinf())
+
+
 def test_what_the_kernel_does_not_take_is_torchs():
     for dtype in (torch.float16, torch.bfloat16):
         x, w = _operands(96, 256, 256, dtype)
