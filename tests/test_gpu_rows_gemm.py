@@ -148,14 +148,15 @@ def test_captured_with_parts_of_k():
         assert torch.equal(ops_rows.linear(x, w), want)
 
 
-def test_products_that_the_library_is_faster_at_are_the_librarys(monkeypatch):
-    """Plain products and gated units at sizes that were timed (the rule itself: test_sizes_of_the_kernel_and_of_the_library)."""
+def test_products_that_are_the_librarys(monkeypatch):
+    """linear at sizes that were timed (the rule itself: test_sizes_of_the_kernel_and_of_the_library)."""
     taken = []
-    monkeypatch.setattr(ops_rows, "product", lambda x, w, form=ops_rows.PLAIN: taken.append((x.shape[0], form)) or F.linear(x, w))
-    w = torch.zeros(12288, 4096, dtype=torch.float16, device="cuda")
-    for rows in (33, 112, 650, 1300):
+    monkeypatch.setattr(ops_rows, "product", lambda x, w, form=ops_rows.PLAIN: taken.append((x.shape[0], w.shape[0], form)) or F.linear(x, w))
+    wide, narrow = (torch.zeros(n, 4096, dtype=torch.float16, device="cuda") for n in (32000, 768))
+    for rows in (40, 128, 700):
         x = torch.zeros(rows, 4096, dtype=torch.float16, device="cuda")
-        ops_rows.linear(x, w)
-        assert (ops_rows.glu_linear(x, w, ops_rows.SILU_HALVES) is None) == (rows == 112)
-        assert ops_rows.glu_linear(x, w, ops_rows.GELU_EIGHTS) is None
-    assert taken == [(33, 0), (33, 1), (650, 1), (1300, 0), (1300, 1)]
+        ops_rows.linear(x, wide)
+        ops_rows.linear(x, narrow)
+        ops_rows.glu_linear(x, wide, ops_rows.SILU_HALVES)
+        assert ops_rows.glu_linear(x, wide, ops_rows.GELU_EIGHTS) is None
+    assert taken == [(40, 32000, 0), (40, 32000, 1), (128, 32000, 1), (700, 32000, 0), (700, 768, 0), (700, 32000, 1)]

@@ -60,14 +60,13 @@ def test_the_librarys_sizes():
     assert not ops_rows.library_fills(4096, 22016) and not ops_rows.library_fills(3900, 4096)
 
 
-# rows, n, k, form -> is the library's product the faster one: sizes where one of the two was by 5 % or more
-@pytest.mark.parametrize("rows,n,k,form,library", [(112, 12288, 4096, 0, True), (384, 12320, 4096, 0, True), (768, 4096, 4096, 0, True), (560, 15360, 5120, 0, True),
-                                                   (128, 32000, 4096, 0, True), (512, 6144, 1536, 0, True), (100, 768, 3072, 0, True), (100, 22016, 4096, 1, True),
-                                                   (160, 4096, 4096, 0, False), (160, 5120, 5120, 0, False), (6000, 12288, 4096, 0, False),
-                                                   (2048, 18784, 4096, 0, False), (700, 4096, 11008, 0, False), (160, 4096, 15104, 0, False), (100, 256, 4096, 0, False),
-                                                   (700, 2304, 768, 0, False), (4096, 8192, 512, 0, False), (33, 22016, 4096, 1, False), (1500, 22016, 4096, 2, False)])
-def test_sizes_of_the_kernel_and_of_the_library(rows, n, k, form, library):
-    assert ops_rows.library_is_faster(rows, n, k, form) == library
+# is the library's product the one to take: sizes on either side of each line
+@pytest.mark.parametrize("rows,n,k,library", [(128, 32000, 4096, True), (160, 32000, 5120, True), (96, 32000, 4096, False), (193, 32000, 4096, False), (128, 27648, 4096, False),
+                                              (64, 768, 3072, True), (320, 768, 3072, True), (700, 768, 3072, False), (64, 512, 4096, False), (64, 2048, 4096, False),
+                                              (64, 768, 1152, False), (4096, 4096, 4096, True), (4096, 8192, 512, False), (3100, 4096, 4096, False),
+                                              (112, 12288, 4096, False), (700, 4096, 11008, False)])
+def test_sizes_of_the_kernel_and_of_the_library(rows, n, k, library):
+    assert ops_rows.library_is_faster(rows, n, k) == library
 
 
 @functools.lru_cache(maxsize=None)

@@ -46,20 +46,19 @@ def library_fills(rows, n):
     return tiles % 256 == 0 and 100 * rows * n >= 97 * 65536 * tiles
 
 
-def library_is_faster(rows, n, k, form=PLAIN):
-    """Is the library's product (and the unit's launch behind it) the faster one from 33 rows on?  The kernel's time over the library's, of 24 products of
-    256 .. 32 000 outputs and 256 .. 15 104 columns at 57 counts of rows up to 8 000, weights from memory:
-      * up to 1 152 columns 0.4 to 1.05;  from 9 600 on 0.45 to 1.0 up to 2 000 rows (4 096 x 11 008, 700 rows 88 -> 71 us) and 0.6 to 1.1 above;
-      * between, with a gated unit 0.63 to 1.03, but from 65 to 160 rows 1.02 to 1.2 (22 016 x 4 096, 100 rows 48 -> 51 us; 27 648 x 5 120 0.92 to 1.04);
-      * between, plain, up to 2^32 multiply-adds 0.56 to 1.07 (4 096 x 4 096, 160 rows 26 -> 18 us); from 6e10 on 0.62 to 1.1 (12 288 x 4 096, 6 000 rows
-        566 -> 462); from one to the other 0.99 on average, 0.6 to 1.25 case by case: the library's tiles are the better ones where they fill
-        one round of the CUs (4 096 x 4 096, 768 rows 36 -> 41; 12 288 x 4 096, 112 rows 31.5 -> 35.5), and the only ones it had there before;
-      * few outputs: its own parts of k serve 512 to 2 048 (768 x 3 072, 100 rows 7.6 -> 9.2 us), not fewer (256 x 4 096, 100 rows 11.3 -> 9.2)."""
-    if k <= 1152:
-        return False
-    if form != PLAIN:
-        return 64 < rows <= 160 and k <= 9600
-    return library_fills(rows, n) or (k <= 9600 and n > 512 and (n < 2048 or 1 << 32 < rows * n * k < 60e9))
+def library_is_faster(rows, n, k):
+    """Is the library's kernel the one to take for a plain product, from 33 rows on?  On the device alone the two are within 10 % of each other at most sizes
+    (24 products of 256 .. 32 000 outputs and 256 .. 15 104 columns at 57 counts of rows up to 8 000, weights from memory: this kernel 0.87 of the
+    library's time on average, more than 1.05 of it in one of nine).  A call of the library is 7 us of the host's time more, and some 50 where
+    its sizes are new, as a prompt's mostly are: forwards of 80 and 300 tokens with the library's products wherever those were the faster
+    ones 1 054 -> 1 197 and 1 430 -> 1 483 us (kemurax, four layers), of 550 and 1 700 tokens 1 244 -> 1 264 and 2 787 -> 2 812 (llama).  So it is
+    taken where it gains more than that, or inside graphs:
+      * whole rounds of tiles of 256 x 256, see library_fills;
+      * 513 to 2 047 outputs of more than 1 152 columns, few tiles behind parts of k: 768 x 3 072 (the 68M draft's chunks) at 64 rows 7.1 us against
+        8.9, 320 rows 8.8 / 10.4, but 700 13.8 / 11.3 (fewer outputs are again this kernel's: 256 x 4 096, 100 rows 11.3 / 9.2);
+      * 97 to 192 rows of 240 MB of weights and more (logits), where tiles of 128 rows leave half of the CUs without one: 32 000 x 4 096, 100 rows
+        62.7 / 69, 128 62 / 72, 160 65 / 74, x 5 120 68 / 76, 70 / 80, 76 / 90; 72 rows 62 / 58, 220 rows 71 / 71."""
+    return k > 1152 and (library_fills(rows, n) or (512 < n < 2048 and rows <= 512) or (96 < rows <= 192 and n * k >= 120e6))
 
 
 @functools.lru_cache(maxsize=4096)
@@ -98,5 +97,6 @@ def linear(x, w):
 
 
 def glu_linear(x, w, form):
-    """The gated unit ``form`` of x . W^T in one launch, None where it is not one or the product and the unit apart are faster."""
-    return product(x, w, form) if takes(x, w, form) and not library_is_faster(x.shape[0], *w.shape, form) else None
+    """The gated unit ``form`` of x . W^T in one launch, None where it is not one.  (65 to 160 rows of 22 016 x 4 096 are 2 to 4 us more than the library's
+    product and the unit's launch, 48 -> 51, whose calls cost the host 16 more.)"""
+    return product(x, w, form) if takes(x, w, form) else None
