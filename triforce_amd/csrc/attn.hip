@@ -1421,15 +1421,15 @@ __global__ __launch_bounds__(256, TREE ? TF_BLOCK_TREE_OCC : 2) void attn_block_
 // into 1 KiB of LDS, lane-linear, no staging registers and no ds_write; the XOR swizzle of the layout is applied on the
 // SOURCE side (the lane that fills slot j of row r loads chunk j ^ f(r): the swizzles are involutions).
 // (1024-row chunk x 124 928 keys x 32 heads: 792.7 -> 848.4 TF/s, profiles/r03_prefill_slab_ab.jsonl.)
-// What bounds it: a wave issues its products (1 024 cycles a slab), some 170 other VALU operations (32 of them exponentials of 16 cycles) and 100
+// What bounds it: a wave issues its products (1 024 cycles a slab), some 176 other VALU operations (32 of them exponentials of 16 cycles) and 100
 // scalar and LDS operations one after the other, two waves of a SIMD overlap by half, and the chip is at its power limit while they do:
-// matrix cores busy 50 % of the cycles at 1.82 GHz, on zeros the same launch is 1.3 times as fast.  So what counts is work that can be
+// matrix cores busy 50 % of the cycles at 1.83 GHz, on zeros the same launch is 1.3 times as fast.  So what counts is work that can be
 // left out: the exponentials of a slab placed beside the next slab's products by hand, a wave priority for the products and deeper or
 // shallower fragment look-ahead are all within the noise of each other, while these helped (4096 rows x 65 536 keys x 32 heads):
 //   * addresses of the LDS-DMA from a scalar slab pointer and 32-bit lane offsets, one code path for masked and unmasked slabs (scores outside
 //     set to -inf): 864 -> 915 TF/s; fragments read 4 (K) and 8 (V) steps ahead in a fixed order: 930;
 //   * the lane offsets and the twelve LDS places of its fragments kept in registers, the maxima of the next slab beside the products with V, by
-//     instructions of three operands, and the sums rescaled in place: 224 -> 170 VALU operations a slab, 930 -> 959 TF/s (3 100 rows without
+//     instructions of three operands, and the sums rescaled in place: 220 -> 176 VALU operations a slab, 930 -> 959 TF/s (3 100 rows without
 //     a past 136 -> 132 us, 700 rows 22.0 -> 21.4, 1 024 rows x 20 000 408 -> 394).  Two slabs per turn, so that buffers are instruction
 //     offsets too, moves 64 sums between registers in every second slab instead;
 //   * one split (every chunk of more than 2 000 rows): the output is written here instead of partials for the merge kernel, and the

@@ -8,13 +8,13 @@
 // may then begin before the waves have met.  No branch lies between the products of two steps (a test for the end of the tile there: 266 ->
 // 250), so steps are counted in runs, and the loads run on into the next tile while this one is finished.
 //
-// Bound by power: at 8 000 x 12 288 x 4 096 the matrix cores are busy 75 % of the cycles at 1.82 GHz (the library's kernel: 83 % at 1.71, 0.97 of
-// the time), and other orders of reads, loads and meeting points give the same time to 1 %.  Four waves of 128 x 128 instead of eight of 128 x 64
+// Bound by power: at 8 000 x 12 288 x 4 096 the matrix cores are busy 77 % of the cycles at 1.79 GHz (the library's kernel: 81 % at 1.71, 0.97 to 1.0
+// of the time), and other orders of reads, loads and meeting points give the same time to 1 %.  Four waves of 128 x 128 instead of eight of 128 x 64
 // read a third less from LDS: as fast, and cooler.  Against the library's product (us, weights from memory; plan() picks tile and parts):
 //   22 016 x 4 096:  130 rows 51 -> 55, 700 140 -> 141, 1 500 294 -> 236, 3 100 547 -> 425, 4 096 654 -> 556, 8 000 1 152 -> 1 027
 //   4 096 x 11 008:  130 rows 49 -> 34, 700  89 ->  71, 1 500 129 -> 122, 3 100 221 -> 210, 4 096 243 -> 247, 8 000   480 -> 487
 //   4 096 x 4 096:   130 rows 18 -> 13, 700  31 ->  33, 1 500  50 ->  50, 3 100  84 ->  80, 4 096  94 ->  99, 8 000   185 -> 191
-// At 200 to 300 rows of 12 288 x 4 096 the library is still up to 8 % faster (255 rows: 43 -> 47).
+// Where the library is still the faster one, and where it is taken: library_is_faster() of ops_rows.py.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <math.h>

@@ -82,10 +82,6 @@ class KemuraxForCausalLM:
         return self._rope[spec.mixer.left.rot.key()] if spec.mixer.type == "parallel" else None
 
     # -- forward -----------------------------------------------------------------------------
-    def decode_form(self, rows, pages):
-        """One set of launches, whatever the sequences hold."""
-        return None
-
     @torch.inference_mode()
     def __call__(self, input_ids, kv_cache=None, graph_cache=None, position_ids=None, **_):
         return self.forward(input_ids, kv_cache)

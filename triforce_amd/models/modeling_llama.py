@@ -6,8 +6,8 @@ build (:226-238), same numerics.
 
 A decode-sized forward (<= 32 rows) is 6 launches per layer, all hand-written: qkv GEMM (RMSNorm prologue,
 RoPE + KV-append epilogue), split-KV MFMA attention + merge, o GEMM (+residual), gate|up GEMM (RMSNorm prologue,
-SwiGLU epilogue), down GEMM (+residual).  Prefill chunks (128 rows) run hipBLASLt GEMMs with the stand-alone
-RMSNorm / RoPE-append / SwiGLU kernels and the 128-row block attention.
+SwiGLU epilogue), down GEMM (+residual).  Prefill chunks (up to 4 096 rows) run the products of many rows (ops_rows, gate|up
+with the SwiGLU epilogue) between the stand-alone RMSNorm / RoPE-append kernels and the 128-row block attention.
 """
 import torch
 

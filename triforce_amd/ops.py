@@ -141,7 +141,7 @@ def _ensure_sg_workspace(device):
 
 class PackedLinear:
     """A weight matrix with (on a HIP device) its pre-packed copy for the skinny decode GEMM.  ``w`` stays
-    available for the >32-row prefill GEMMs (hipBLASLt).  ``split`` = number of equal row blocks that were
+    available for the >32-row prefill GEMMs (ops_rows).  ``split`` = number of equal row blocks that were
     fused (2 for gate|up) — each block is packed on its own so the SwiGLU kernel can pair them.  ``rope=(H, D)``
     marks a fused q|k|v weight: a second packed copy in rotary-pair row order feeds tf_skinny_qkv_rope."""
 

@@ -73,8 +73,8 @@ def shares_panels(n, k, raw=0):
 
 
 class TileWeight:
-    """A (groups of) [n, k] weight(s): packed for the skinny kernel and, unless ``packed_only``, row-major for the library GEMM
-    of the prefill.  Weights of the one-workgroup-per-CU form are packed chunk-major, the layout it streams; the workgroup-per-panel form
+    """A (groups of) [n, k] weight(s): packed for the skinny kernel and, unless ``packed_only``, row-major for the prefill's products
+    of many rows (linear_rows).  Weights of the one-workgroup-per-CU form are packed chunk-major, the layout it streams; the workgroup-per-panel form
     reads that one too, but up to 10 % slower (128 256 x 4 096 at 8 rows 171 -> 181 us, a projection of 17 216 with 16 480 raw 27.4 -> 30.1
     at one row), so its weights stay panel by panel.  ``raw``: outputs of an input projection that come with sums of squares; ``per_panel``:
     the weight of a product that only the workgroup-per-panel form has (query, token gate)."""
@@ -166,7 +166,7 @@ def interleave_glu(gate, up):
 def linear_rows(x, w):
     """x . W^T over many rows (prefill), w [n, k] contiguous: in 16 bits ops_rows.linear, in float32 the library GEMM, and for large products
     split_linear.  Its tiles are 256 x 128: from 256 rows and 2^32 multiply-adds on it is the faster one (256 x 4 096 x 4 096 73 -> 61 us, 2 048 x 2 048 x 1 024
-    70 -> 63, 700 x 22 016 x 4 096 940 -> 750), below that it leaves CUs idle (300 x 6 144 x 1 536 51 -> 55, 64 x 22 016 x 4 096
+    70 -> 63, 700 x 22 016 x 4 096 940 -> 665), below that it leaves CUs idle (300 x 6 144 x 1 536 51 -> 55, 64 x 22 016 x 4 096
     115 -> 133), as with few results of a long k, whose parts are eight at most (2^19 results: 385 x 1 136 x 15 104 117 -> 145, 512 x 1 136
     162 -> 150), and with k below 96 the cut and the results are all there is (1 030 x 65 536 x 64 110 -> 116).  Up to k = 65 536 its error is a
     tenth to a half of the library's; at 2^20, with as few parts, the two are equal."""
