@@ -62,9 +62,11 @@ def test_the_librarys_sizes():
 
 # is the library's product the one to take: sizes on either side of each line
 @pytest.mark.parametrize("rows,n,k,library", [(128, 32000, 4096, True), (160, 32000, 5120, True), (96, 32000, 4096, False), (193, 32000, 4096, False), (128, 27648, 4096, False),
-                                              (64, 768, 3072, True), (320, 768, 3072, True), (700, 768, 3072, False), (64, 512, 4096, False), (64, 2048, 4096, False),
-                                              (64, 768, 1152, False), (4096, 4096, 4096, True), (4096, 8192, 512, False), (3100, 4096, 4096, False),
-                                              (112, 12288, 4096, False), (700, 4096, 11008, False)])
+                                              (128, 28672, 8192, True), (128, 128256, 4096, False), (128, 40960, 4096, False), (128, 8192, 28672, False), (128, 16384, 16384, False),
+                                              (64, 768, 3072, True), (320, 768, 3072, True), (321, 768, 3072, False), (64, 512, 4096, False), (64, 1536, 4096, False),
+                                              (64, 768, 1536, False), (64, 640, 8192, False), (4096, 4096, 4096, True), (4096, 4096, 1152, False), (4096, 8192, 512, False),
+                                              (512, 32768, 4096, False), (1024, 16384, 4096, False), (3100, 4096, 4096, False), (112, 12288, 4096, False),
+                                              (700, 4096, 11008, False)])
 def test_sizes_of_the_kernel_and_of_the_library(rows, n, k, library):
     assert ops_rows.library_is_faster(rows, n, k) == library
 

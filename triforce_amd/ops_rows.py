@@ -52,13 +52,18 @@ def library_is_faster(rows, n, k):
     library's time on average, more than 1.05 of it in one of nine).  A call of the library is 7 us of the host's time more, and some 50 where
     its sizes are new, as a prompt's mostly are: forwards of 80 and 300 tokens with the library's products wherever those were the faster
     ones 1 054 -> 1 197 and 1 430 -> 1 483 us (kemurax, four layers), of 550 and 1 700 tokens 1 244 -> 1 264 and 2 787 -> 2 812 (llama).  So it is
-    taken where it gains more than that, or inside graphs:
-      * whole rounds of tiles of 256 x 256, see library_fills;
-      * 513 to 2 047 outputs of more than 1 152 columns, few tiles behind parts of k: 768 x 3 072 (the 68M draft's chunks) at 64 rows 7.1 us against
-        8.9, 320 rows 8.8 / 10.4, but 700 13.8 / 11.3 (fewer outputs are again this kernel's: 256 x 4 096, 100 rows 11.3 / 9.2);
-      * 97 to 192 rows of 240 MB of weights and more (logits), where tiles of 128 rows leave half of the CUs without one: 32 000 x 4 096, 100 rows
-        62.7 / 69, 128 62 / 72, 160 65 / 74, x 5 120 68 / 76, 70 / 80, 76 / 90; 72 rows 62 / 58, 220 rows 71 / 71."""
-    return k > 1152 and (library_fills(rows, n) or (512 < n < 2048 and rows <= 512) or (96 < rows <= 192 and n * k >= 120e6))
+    taken where it gains more than that, or inside graphs (this kernel's time over the library's):
+      * whole rounds of tiles of 256 x 256, see library_fills: 1.02 to 1.10 from 2 048 rows and 1 280 columns on; at 512 and 1 024 rows 0.83 to 1.02, and of
+        512 columns 0.98;
+      * a few tiles with parts of k that cost more than they bring: 576 x 4 096, 1 024 x 4 096 and 768 x 3 072 (the 68M draft's chunks of 64 rows, 7.1 us
+        against 8.9) 0.9 to 1.25 up to 320 rows; on either side of these 512 x 2 048 and 768 x 1 536 1.0 to 1.05, 1 536 x 4 096 0.82 to 1.07, 1 280 x
+        5 120 0.73 to 0.9, 640 x 8 192 0.7 to 1.06, and all of them 0.8 to 1.0 at 600 rows;
+      * 97 to 192 rows of 234 MB of weights and more (logits), where tiles of 128 x 256 leave half of the CUs without one: 32 000 x 4 096 1.0 to 1.27 (62 us
+        against 72), x 5 120 0.8 to 1.19, 28 672 x 4 096 1.05 to 1.21, x 8 192 1.08 to 1.13, 24 576 x 5 120 1.01 to 1.13, 16 384 x 8 192 1.13 to 1.28; but
+        18 784 x 6 144 0.91 to 1.03, 40 960 x 3 072 and 49 152 x 4 096 0.94 to 1.08, 128 256 x 4 096 0.68 to 0.82 and 8 192 x 28 672 0.36 to 0.51."""
+    if rows >= 2048:
+        return k > 1152 and library_fills(rows, n)
+    return (rows <= 320 and 512 < n <= 1024 and 2048 <= k <= 4096) or (96 < rows <= 192 and 16384 <= n <= 32768 and k <= 9600 and n * k >= 117e6)
 
 
 @functools.lru_cache(maxsize=4096)
@@ -91,7 +96,7 @@ def product(x, w, form=PLAIN, plan=None):
 def linear(x, w):
     """x . W^T, w [n, k] contiguous.  Up to 32 rows only large weights are the kernel's: 18 784 x 4 096 at 16 rows 67 -> 38 us, 4 096 x 11 008 29 -> 23,
     but 4 096 x 4 096 11.0 -> 11.7, 256 x 4 096 7.8 -> 10.0 (at 40 rows 12.6 -> 12.3 and 11.3 -> 9.8)."""
-    if takes(x, w) and (x.shape[0] > 32 or w.numel() > 1 << 25) and not library_is_faster(x.shape[0], *w.shape):
+    if (x.shape[0] > 32 or w.numel() > 1 << 25) and takes(x, w) and not library_is_faster(x.shape[0], *w.shape):
         return product(x, w)
     return F.linear(x, w)
 
