@@ -151,7 +151,7 @@ def test_captured_with_parts_of_k():
 def test_products_that_are_the_librarys(monkeypatch):
     """linear at sizes that were timed (the rule itself: test_sizes_of_the_kernel_and_of_the_library)."""
     taken = []
-    monkeypatch.setattr(ops_rows, "product", lambda x, w, form=ops_rows.PLAIN: taken.append((x.shape[0], w.shape[0], form)) or F.linear(x, w))
+    monkeypatch.setattr(ops_rows, "product", lambda x, w, form=ops_rows.PLAIN, plan=None: taken.append((x.shape[0], w.shape[0], form)) or F.linear(x, w))
     wide, narrow = (torch.zeros(n, 4096, dtype=torch.float16, device="cuda") for n in (32000, 768))
     for rows in (40, 128, 700):
         x = torch.zeros(rows, 4096, dtype=torch.float16, device="cuda")

@@ -76,6 +76,12 @@ def _plan(dtype, rows, n, k):
     return shape.value, splits.value, floats
 
 
+@functools.lru_cache(maxsize=4096)
+def _choice(dtype, rows, k, n):
+    """linear's plan of the kernel, None where the library is taken.  (One look-up: at 50 rows a forward waits for the host.)"""
+    return None if library_is_faster(rows, n, k) else _plan(dtype, rows, n, k)[:2]
+
+
 def product(x, w, form=PLAIN, plan=None):
     """The kernel's product.  plan = (shape, splits): another than its own choice."""
     (rows, k), n = x.shape, w.shape[0]
@@ -96,8 +102,10 @@ def product(x, w, form=PLAIN, plan=None):
 def linear(x, w):
     """x . W^T, w [n, k] contiguous.  Up to 32 rows only large weights are the kernel's: 18 784 x 4 096 at 16 rows 67 -> 38 us, 4 096 x 11 008 29 -> 23,
     but 4 096 x 4 096 11.0 -> 11.7, 256 x 4 096 7.8 -> 10.0 (at 40 rows 12.6 -> 12.3 and 11.3 -> 9.8)."""
-    if (x.shape[0] > 32 or w.numel() > 1 << 25) and takes(x, w) and not library_is_faster(x.shape[0], *w.shape):
-        return product(x, w)
+    if (x.shape[0] > 32 or w.numel() > 1 << 25) and takes(x, w):
+        plan = _choice(x.dtype, *x.shape, w.shape[0])
+        if plan is not None:
+            return product(x, w, PLAIN, plan)
     return F.linear(x, w)
 
 
