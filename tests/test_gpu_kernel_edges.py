@@ -86,6 +86,21 @@ def test_prefill_attention_blocks_and_splits(n, past, H, token_major, rising):
     assert ((got - want).abs() <= bound).all()
 
 
+# keys and values on either side of 256 MB (8 heads: 65 536 keys), row blocks that are no multiple of eight, splits
+@pytest.mark.parametrize("n,past,H", [(1100, 64436, 8), (1100, 64437, 8), (2500, 63100, 8), (1409, 20000, 32)])
+def test_prefill_attention_order_of_row_blocks(n, past, H):
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n)
+    k, v = (torch.randn(H, past + n, 128, generator=g, device=DEV, dtype=torch.float16) for _ in range(2))
+    q = torch.randn(n, H, 128, generator=g, device=DEV, dtype=torch.float16)
+    got = ops.attn_prefill(q, k, v, past + n, 0.088).view(n, H, 128).double()
+    for rows in (slice(0, 64), slice(n - 140, n)):              # (the first rows and those of the last blocks)
+        seen = past + n - (n - rows.stop)
+        want, size = _attention64(q[rows], k[:, :seen], v[:, :seen], 0.088)
+        assert ((got[rows] - want).abs() <= 2.0 ** -10 * size + 2.0 ** -11 * want.abs() + 1e-6).all()
+    assert torch.isfinite(got).all()
+
+
 # every key alike, rows that do not see all of their last slab: a hidden score of minus infinity times 0 is no number
 @pytest.mark.parametrize("n,past,H", [(130, 0, 8), (200, 2000, 8), (2049, 0, 32)])
 def test_prefill_attention_scale_of_zero(n, past, H):

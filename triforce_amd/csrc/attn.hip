@@ -1713,7 +1713,7 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
 // Launching the blocks one by one streams the KV cache from HBM once per 128 rows (128 flop per byte: an 800 TF/s
 // ceiling at 6.3 TB/s, and the 125K-token prefill ran at ~490).  Here the row blocks that read the SAME key range run at
 // the same time on the SAME XCD, so all but one of them hit that XCD's L2: workgroup ids are laid out as
-//   id % 8 = XCD (hardware round-robin),  (id / 8) % RBG = row block within a group of RBG <= 8,  id / (8 RBG) = the rest,
+//   id % 8 = XCD (hardware round-robin),  (id / 8) % RBG = row block within a group of RBG (launch_prefill),  id / (8 RBG) = the rest,
 // and a (split, head) pair is pinned to XCD pair % 8.  Every row block uses the key partition of the full sk, so its
 // splits cover the same slabs as its neighbours'; splits past a block's causal edge write a neutral partial.
 template <int D>
@@ -2279,7 +2279,13 @@ static int launch_prefill(const void* q, const void* k, const void* v, void* out
         if (e != hipSuccess) return (int)e;
         attr_set = true;
     }
-    const int nrb = (sq + 127) / 128, rbg = nrb < 8 ? nrb : 8;
+    // Row blocks that run side by side.  Eight, the longest first, leave the shortest tail; but every eight read the keys and values again,
+    // past 256 MB of them from memory and not from the Infinity Cache, and what that draws the matrix cores lack: 4 096 rows x 65 536 keys
+    // x 32 heads 4 380 -> 4 020 us at 1.8 -> 2.0 GHz (L2-resident keys: 4 080, no data at all: 3 340).  So all of them there.  By keys (us, 8 ->
+    // all): 32 heads 12 288 684 -> 703, 16 384 (268 MB) 950 -> 938, 32 768 2 060 -> 1 973; 40 heads 12 288 (252 MB) 852 -> 896, 16 384 1 211
+    // -> 1 194; 1 400 rows x 20 000 x 32 heads 519 -> 503.
+    const bool from_memory = (int64_t)H * sk * D * 4 > (int64_t)256 << 20;
+    const int nrb = (sq + 127) / 128, rbg = nrb < 8 || from_memory ? nrb : 8;
     const int groups = (nrb + rbg - 1) / rbg;
     const int64_t blocks = (int64_t)H * nsplit * rbg * groups;
     hipLaunchKernelGGL((attn_prefill_kernel<D>), dim3((unsigned)blocks), dim3(256), blk_lds_bytes<D>(), st, (const h16*)q,
