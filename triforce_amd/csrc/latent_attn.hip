@@ -297,156 +297,244 @@ static int launch_merge(const float* ws, void* out, int rows, int H, int C, int 
     return TF_OK;
 }
 
-// The same attention for a known row size (WC chunks of 32, the first CT 16-wide tiles of it latent), bfloat16, HT head tiles of
-// 16 per workgroup and four waves per head tile: wave (ht, ks) scores keys 16 ks .. of its head tile with the queries held in
-// registers, and accumulates CT / (4 HT) of the latent tiles for all heads.  Two pages in LDS: the next one is written and the one
-// after it requested while the current one is used, so a page costs two barriers and the stream never waits for the arithmetic.
-template <int HT, int WC, int CT>
-__device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages,
-                                                       const int32_t* __restrict__ tab, int n, bf16* __restrict__ out,
-                                                       float* __restrict__ ws, int H, float scale, int nsplit, int rows, int row, int h0,
-                                                       int split, int t_beg, int t_end, char* smem) {
-    constexpr int NT = 256 * HT, W = 32 * WC, C = 16 * CT, LDK = W + 8, LDP = 64 + 8, NTW = CT / (4 * HT), NPRE = 64 * (W / 8) / NT;
-    static_assert(CT % (4 * HT) == 0 && 64 * (W / 8) % NT == 0, "tile split");
-    bf16* Kt = (bf16*)smem;                                   // [2][64][LDK]
-    bf16* Ps = Kt + 2 * 64 * LDK;                             // [2 (value, remainder)][16 HT][LDP]
-    float* red = (float*)(Ps + 2 * 16 * HT * LDP);            // [4][16 HT]
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, i = lane & 15, ks = wave & 3, ht = wave >> 2;
+// The same attention for rows of 512 + 64 in bfloat16, up to 32 heads per workgroup.  Half pages (32 keys) stream through four places in LDS,
+// where LDS-DMA brings them two ahead of their use.  Waves 0 .. 3 score a half page (16 keys x 16 heads each, queries in registers) while waves
+// 4 .. 7 multiply the one before it with its weights (128 of the latent columns each, all heads): one barrier a half page.
+// The weights' reference is a head's largest score of the first half page, and stays: weights go in as value and remainder, whose precision
+// does not depend on the scale, and nothing overflows before a score is 2^100 above it.  Then the reference follows and the sums are scaled.
+// A place holds rows of 1 152 bytes; inside every 128 bytes the pieces of 16 are XORed by swap(row), which leaves the row reads of the scores and
+// the transposing reads of the values without bank conflicts.
+// Bound by what two half pages under way (74 KB a CU) draw, 5.5 TB/s, behind some 9 us of start and end.  Eight waves that took a page together, scored it,
+// met, weighed it, met and multiplied it needed 2.6 us a page from L2 and 3.8 from memory, with the maxima and the scaling in every page; this 2.05 and
+// 3.4.  us with the merge, 32 heads, keys from memory, before -> now: 32 rows of 24 / 48 / 96 pages 28.2 / 40.0 / 62.7 -> 25.5 / 34.8 / 55.1, 8 of 48 / 192
+// 22.3 / 38.3 -> 19.3 / 34.3, one of 64 / 512 18.1 / 28.3 -> 14.3 / 25.7.  More loads under way (one word of each line, 4 to 8 half pages ahead): 62 -> 71
+// to 77.
+struct LatentTile {
+    static constexpr int KT = 32, W = 576, C = 512, H = 32, BYTES = KT * W * 2, RING = 4, LDP = KT + 8, PARTS = 2;
+    static constexpr int P_ELEMS = PARTS * H * LDP, RED = RING * BYTES + 2 * P_ELEMS * 2, LDS = RED + 4 * (2 * H + H + 2);
+};
+static_assert(LatentTile::LDS <= 160 * 1024, "LDS");
 
-    bf16x8 qf[WC];
-    {
-        const int head = h0 + 16 * ht + i;
-        const bf16* src = q + ((int64_t)row * H + min(head, H - 1)) * W + 8 * g;
-#pragma unroll
-        for (int c = 0; c < WC; ++c) {
-            qf[c] = load_frag(src + 32 * c);
-            if (head >= H) qf[c] = bf16x8{};
+// All waves are here, this one's LDS accesses are done and all but the LEFT youngest of its loads have landed.
+template <int LEFT> __device__ __forceinline__ void meet() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070 | (LEFT & 15) | (LEFT >> 4 << 14));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// (everything but the pointers is the same in all lanes)
+__device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages, const int32_t* __restrict__ tab,
+                                                       int n, bf16* __restrict__ out, float* __restrict__ ws, int H, float scale, int nsplit, int rows,
+                                                       int row, int h0, int split, int t_beg, int t_end, char* smem) {
+    typedef LatentTile Z;
+    constexpr int W = Z::W, C = Z::C, LDP = Z::LDP, ROW = 2 * W, PIECES = W / 8, LOADS = Z::BYTES / 4096;
+    constexpr float GROW = 100.0f;
+    typedef __attribute__((address_space(3))) const char* Lds;
+    typedef __attribute__((address_space(3))) bf16x4* Lds4;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15, part = wave & 3;
+    const uint32_t lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+    bf16* Ps = (bf16*)(smem + Z::RING * Z::BYTES);            // [2 half pages][2 (value, remainder)][32 heads][LDP]
+    float* red = (float*)(smem + Z::RED);                     // [2][32]: by 16 keys
+    float* ref = red + 2 * Z::H;                              // [32]
+    volatile int* grow = (volatile int*)(ref + Z::H);         // [2 half pages]: (a fast wave may set the next one's before a slow one has read this one's)
+    const int keys = max(0, min(n, 64 * t_end) - 64 * t_beg), nt = (keys + Z::KT - 1) / Z::KT;         // of this split
+    auto swap = [](int r) { return (r >> 2 & 1) | (r >> 1 & 1) << 1 | (r >> 3 & 1) << 2; };
+
+    if (wave < 4) {                                           // ---- scores and weights
+        const int ks = part & 1, head = 16 * (part >> 1) + i; // this wave's keys, a lane's head
+        float* ml = ws + (int64_t)rows * H * nsplit * C + (((int64_t)row * H + h0 + head) * nsplit + split) * 2;
+        const bool writes = nsplit > 1 && ks == 0 && g == 0 && h0 + head < H;
+        if (nt == 0) {
+            if (writes) {
+                ml[0] = NEG_INF;
+                ml[1] = 0.f;
+            }
+            return;
         }
-    }
-    u32x4 pre[NPRE];
-    auto page_of = [&](int t) {
-        const int pg = tab[t];
-        return pg < 0 ? 0 : (pg >= n_pages ? n_pages - 1 : pg);
-    };
-    auto fetch = [&](int pg) {
-        const bf16* base = cache + (int64_t)pg * (64 * W) + tid * 8;
+        // loads: pieces tid + 256 u of a half page; the ids of 64 pages at a time in the lanes
+        uint32_t off[LOADS];
+        int ids = 0, window = 0;
+        auto place = [&](int u, int last) {
+            const int p = tid + 256 * u, r = p / PIECES, c = p - PIECES * r;
+            return (uint32_t)min(r, last) * ROW + 16 * ((c & ~7) | ((c ^ swap(r)) & 7));
+        };
+        auto page_ids = [&] { ids = t_beg + 64 * window + lane < t_end ? tab[t_beg + 64 * window + lane] : 0; };
+        auto fetch = [&](int j) {                             // (past the end: the last one again, not used)
+            const int c = min(j, nt - 1), t = c >> 1, left = keys - 1 - Z::KT * c;
+            if (t >> 6 != window) {
+                window = t >> 6;
+                page_ids();
+            }
+            const int pg = __builtin_amdgcn_readlane(ids, t & 63);
+            const char* src = (const char*)(cache + (int64_t)(pg < 0 ? 0 : (pg >= n_pages ? n_pages - 1 : pg)) * (64 * W)) + (c & 1) * Z::BYTES;
+            const uint32_t dst = lds + (j & 3) * Z::BYTES + 1024 * part;
 #pragma unroll
-        for (int j = 0; j < NPRE; ++j) pre[j] = *reinterpret_cast<const u32x4*>(base + j * NT * 8);
-    };
-    auto put = [&](int t) {
-        bf16* dst = Kt + (t & 1) * 64 * LDK;
-        const bool edge = 64 * t + 64 > n;
+            for (int u = 0; u < LOADS; ++u) {                 // (nothing else here uses M0)
+                const uint32_t at = __builtin_amdgcn_readfirstlane(dst + 4096 * u), o = left >= Z::KT - 1 ? off[u] : place(u, left);
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(o), "s"(src) : "memory");
+            }
+        };
+        page_ids();
 #pragma unroll
-        for (int j = 0; j < NPRE; ++j) {
-            const int p = tid + j * NT, r = p / (W / 8), c = p - r * (W / 8);
-            u32x4 v = pre[j];
-            if (edge && 64 * t + r >= n) v = u32x4{0, 0, 0, 0};     // rows past the end: never let stale contents into 0 * x
-            *reinterpret_cast<u32x4*>(dst + r * LDK + 8 * c) = v;
-        }
-    };
-    f32x4 o[HT][NTW];
-    float m_run[HT], l_run = 0.f;
+        for (int u = 0; u < LOADS; ++u) off[u] = place(u, Z::KT - 1);
+        fetch(0);
+        fetch(1);
+        fetch(2);
+        bf16x8 qf[W / 32];
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};                       // scores of the half page whose weights are not used yet
+        float m, l = 0.f, sum = 0.f;                          // sum: of those weights
+        auto frag = [&](uint32_t at, int c) { return *(const __attribute__((address_space(3))) bf16x8*)((Lds)(uintptr_t)(at ^ (64 * (c & 1))) + 128 * (c >> 1)); };
+        const uint32_t k_at = lds + (16 * ks + i) * ROW + 16 * (g ^ swap(i));
+        auto scores = [&](int j) {
+            f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
+            const uint32_t at = k_at + (j & 3) * Z::BYTES;
 #pragma unroll
-    for (int h = 0; h < HT; ++h) {
-        m_run[h] = NEG_INF;
+            for (int c = 0; c < W / 32; c += 2) {
+                a = El<bf16>::mma(frag(at, c), qf[c], a);
+                b = El<bf16>::mma(frag(at, c + 1), qf[c + 1], b);
+            }
 #pragma unroll
-        for (int x = 0; x < NTW; ++x) o[h][x] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    int pg_next = 0;
-    if (t_beg < t_end) {
-        fetch(page_of(t_beg));
-        if (t_beg + 1 < t_end) pg_next = page_of(t_beg + 1);
-        put(t_beg);
-        if (t_beg + 1 < t_end) fetch(pg_next);
-        if (t_beg + 2 < t_end) pg_next = page_of(t_beg + 2);
-        __syncthreads();
-    }
-    for (int t = t_beg; t < t_end; ++t) {
-        const bf16* K = Kt + (t & 1) * 64 * LDK;
-        const int k0 = 64 * t;
-        f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = s0;
-        const bf16* kp = K + (16 * ks + i) * LDK + 8 * g;
-#pragma unroll
-        for (int c = 0; c < WC; c += 2) {
-            s0 = El<bf16>::mma(load_frag(kp + 32 * c), qf[c], s0);
-            if (c + 1 < WC) s1 = El<bf16>::mma(load_frag(kp + 32 * (c + 1)), qf[c + 1], s1);
-        }
-        float mx = NEG_INF;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            s0[r] = k0 + 16 * ks + 4 * g + r < n ? (s0[r] + s1[r]) * scale : NEG_INF;
-            mx = fmaxf(mx, s0[r]);
-        }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        if (g == 0) red[ks * 16 * HT + 16 * ht + i] = mx;
-        __syncthreads();                                      // maxima are in; everyone is done with the previous page and weights
-        float alpha[HT];
-#pragma unroll
-        for (int h = 0; h < HT; ++h) {
-            float m = m_run[h];
-#pragma unroll
-            for (int w = 0; w < 4; ++w) m = fmaxf(m, red[w * 16 * HT + 16 * h + i]);
-            alpha[h] = __builtin_amdgcn_exp2f((m_run[h] - m) * LOG2E);   // (the page's first key is visible: m is finite)
-            m_run[h] = m;
-        }
-        {
-            float m = m_run[0], al = alpha[0];
-#pragma unroll
-            for (int h = 1; h < HT; ++h)
-                if (ht == h) { m = m_run[h]; al = alpha[h]; }
+            for (int r = 0; r < 4; ++r) s[r] = Z::KT * j + 16 * ks + 4 * g + r < keys ? (a[r] + b[r]) * scale : NEG_INF;
+        };
+        auto largest = [&] {                                  // of these 16 keys, into red
+            float x = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+            x = fmaxf(x, __shfl_xor(x, 16, 64));
+            x = fmaxf(x, __shfl_xor(x, 32, 64));
+            if (g == 0) red[Z::H * ks + head] = x;
+        };
+        auto weights = [&](int j) {
             f32x4 p, lo;
-            float sum = 0.f;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                p[r] = __builtin_amdgcn_exp2f((s0[r] - m) * LOG2E);
-                sum += p[r];
+                p[r] = __builtin_amdgcn_exp2f((s[r] - m) * LOG2E);
                 lo[r] = p[r] - (float)(bf16)p[r];
             }
-            l_run = l_run * al + sum;
-            bf16* dst = Ps + (16 * ht + i) * LDP + 16 * ks + 4 * g;
+            sum = (p[0] + p[1]) + (p[2] + p[3]);
+            bf16* dst = Ps + (j & 1) * Z::P_ELEMS + head * LDP + 16 * ks + 4 * g;
             store_quad(dst, p);
-            store_quad(dst + 16 * HT * LDP, lo);
-        }
-        if (t + 1 < t_end) {
-            put(t + 1);
-            if (t + 2 < t_end) fetch(pg_next);
-            if (t + 3 < t_end) pg_next = page_of(t + 3);
-        }
-        __syncthreads();                                      // weights and the next page are in
+            store_quad(dst + Z::H * LDP, lo);
+        };
+        meet<2 * LOADS>();                                    // the first half page, and the queries in the last place
+        const uint32_t q_at = lds + 3 * Z::BYTES + head * ROW + 16 * (g ^ swap(head));
 #pragma unroll
-        for (int h = 0; h < HT; ++h)
-#pragma unroll
-            for (int x = 0; x < NTW; ++x)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o[h][x][r] *= alpha[h];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            bf16x8 b[HT][2];
-#pragma unroll
-            for (int h = 0; h < HT; ++h)
-#pragma unroll
-                for (int z = 0; z < 2; ++z) b[h][z] = load_frag(Ps + (z * 16 * HT + 16 * h + i) * LDP + 32 * c + 8 * g);
-#pragma unroll
-            for (int x = 0; x < NTW; ++x) {
-                const bf16x8 a = load_frag_t(K, LDK, 32 * c + 8 * g, 32 * c + 8 * g + 4, 16 * (wave * NTW + x), i);
-#pragma unroll
-                for (int z = 0; z < 2; ++z)
-#pragma unroll
-                    for (int h = 0; h < HT; ++h) o[h][x] = El<bf16>::mma(a, b[h][z], o[h][x]);
+        for (int c = 0; c < W / 32; ++c) qf[c] = frag(q_at, c);
+        scores(0);
+        largest();
+        meet<63>();
+        m = fmaxf(red[head], red[Z::H + head]);               // (the first key is visible: finite)
+        if (ks == 0 && g == 0) ref[head] = m;
+        weights(0);
+        meet<LOADS>();
+        for (int j = 1; j <= nt; ++j) {
+            const int grown = grow[(j - 1) & 1];
+            if (j < nt) fetch(j + 2);
+            if (__builtin_amdgcn_readfirstlane(grown)) {      // the half page before this one needs another reference
+                largest();
+                meet<63>();
+                const float to = fmaxf(m, fmaxf(red[head], red[Z::H + head]));
+                l *= __builtin_amdgcn_exp2f((m - to) * LOG2E);
+                m = to;
+                weights(j - 1);
+                meet<63>();
+                if (ks == 0 && g == 0) ref[head] = m;
             }
+            l += sum;
+            if (j < nt) {
+                scores(j);
+                const float top = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+                if (__builtin_amdgcn_ballot_w64((top - m) * LOG2E > GROW)) {
+                    if (lane == 0) grow[j & 1] = 1;
+                }
+                weights(j);
+            }
+            meet<LOADS>();
         }
+        l += __shfl_xor(l, 16, 64);
+        l += __shfl_xor(l, 32, 64);
+        if (g == 0) red[Z::H * ks + head] = l;
+        meet<0>();                                            // (no load is under way when the LDS is given back)
+        if (writes) {
+            ml[0] = m;
+            ml[1] = red[head] + red[Z::H + head];
+        }
+        return;
     }
-    __syncthreads();
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
-    if (g == 0) red[ks * 16 * HT + 16 * ht + i] = l_run;
-    __syncthreads();
+
+    // ---- values
+    constexpr int HT = 2, NTW = 8;                            // head tiles, a wave's 16-wide tiles of the latent
+    f32x4 o[HT][NTW];
+#pragma unroll
+    for (int h = 0; h < HT; ++h)
+#pragma unroll
+        for (int x = 0; x < NTW; ++x) o[h][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (nt > 0) {
+        const int t4 = tid - 256;
+        u32x4 z[LOADS];
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u) {
+            const int p = t4 + 256 * u, r = p / PIECES, c = p - PIECES * r;
+            z[u] = *reinterpret_cast<const u32x4*>(q + ((int64_t)row * H + min(h0 + r, H - 1)) * W + 8 * c);
+            if (h0 + r >= H) z[u] = u32x4{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int u = 0; u < LOADS; ++u) {
+            const int p = t4 + 256 * u, r = p / PIECES, c = p - PIECES * r;
+            *reinterpret_cast<u32x4*>(smem + 3 * Z::BYTES + r * ROW + 16 * ((c & ~7) | ((c ^ swap(r)) & 7))) = z[u];
+        }
+        if (t4 < 2) grow[t4] = 0;
+        const int vrow = 8 * g + (i >> 2);
+        const uint32_t v_at = lds + vrow * ROW + 256 * part + 16 * (((i & 3) >> 1) ^ swap(vrow)) + 8 * (i & 1);
+        meet<63>();
+        meet<63>();
+        meet<63>();
+        for (int j = 1; j <= nt; ++j) {
+            const int grown = grow[(j - 1) & 1];
+            bf16x8 b[HT][2];
+            auto read_p = [&] {
+                const bf16* src = Ps + ((j - 1) & 1) * Z::P_ELEMS + i * LDP + 8 * g;
+#pragma unroll
+                for (int h = 0; h < HT; ++h)
+#pragma unroll
+                    for (int y = 0; y < 2; ++y) b[h][y] = load_frag(src + (Z::H * y + 16 * h) * LDP);
+            };
+            read_p();
+            if (__builtin_amdgcn_readfirstlane(grown)) {
+                meet<63>();
+#pragma unroll
+                for (int h = 0; h < HT; ++h) {
+                    const float was = ref[16 * h + i], to = fmaxf(was, fmaxf(red[16 * h + i], red[Z::H + 16 * h + i]));
+                    const float f = __builtin_amdgcn_exp2f((was - to) * LOG2E);
+#pragma unroll
+                    for (int x = 0; x < NTW; ++x)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) o[h][x][r] *= f;
+                }
+                if (t4 == 0) grow[(j - 1) & 1] = 0;
+                meet<63>();
+                read_p();
+            }
+            const uint32_t base = v_at + ((j - 1) & 3) * Z::BYTES;
+#pragma unroll
+            for (int x = 0; x < NTW; ++x) {                   // keys 8 g .. + 3 and + 4 .. + 7 of 16 columns
+                const uint32_t at = base ^ (32 * (x & 3));
+                const bf16x4 u = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((Lds4)(uintptr_t)(at + 128 * (x >> 2)));
+                const bf16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((Lds4)(uintptr_t)((at ^ 16) + 128 * (x >> 2) + 4 * ROW));
+                const bf16x8 a = __builtin_shufflevector(u, v, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+                for (int y = 0; y < 2; ++y)
+#pragma unroll
+                    for (int h = 0; h < HT; ++h) o[h][x] = El<bf16>::mma(a, b[h][y], o[h][x]);
+            }
+            meet<63>();
+        }
+        meet<63>();
+    }
 #pragma unroll
     for (int h = 0; h < HT; ++h) {
         const int head = h0 + 16 * h + i;
         if (head >= H) continue;
-        const float l = red[16 * h + i] + red[16 * HT + 16 * h + i] + red[32 * HT + 16 * h + i] + red[48 * HT + 16 * h + i];
+        const float l = nt > 0 ? red[16 * h + i] + red[Z::H + 16 * h + i] : 0.f;
         if (nsplit == 1) {
             const float inv = l > 0.f ? 1.0f / l : 0.f;
 #pragma unroll
@@ -454,54 +542,47 @@ __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ 
                 f32x4 v = o[h][x];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) v[r] *= inv;
-                store_quad(out + ((int64_t)row * H + head) * C + 16 * (wave * NTW + x) + 4 * g, v);
+                store_quad(out + ((int64_t)row * H + head) * C + 128 * part + 16 * x + 4 * g, v);
             }
-        } else {
-            const int64_t at = ((int64_t)row * H + head) * nsplit + split;
-            if (l > 0.f) {                                    // (the partial row of an empty split is not read either)
+        } else if (l > 0.f) {                                 // (the partial row of an empty split is not read either)
+            float* dst = ws + (((int64_t)row * H + head) * nsplit + split) * C + 128 * part + 4 * g;
 #pragma unroll
-                for (int x = 0; x < NTW; ++x)
-                    *reinterpret_cast<f32x4*>(ws + at * C + 16 * (wave * NTW + x) + 4 * g) = o[h][x];
-            }
-            if (wave == 0 && g == 0) {
-                float* ml = ws + (int64_t)rows * H * nsplit * C + at * 2;
-                ml[0] = m_run[h];
-                ml[1] = l;
-            }
+            for (int x = 0; x < NTW; ++x) *reinterpret_cast<f32x4*>(dst + 16 * x) = o[h][x];
         }
     }
 }
 
-template <int HT, int WC, int CT>
-__global__ __launch_bounds__(256 * HT, HT) void attn_latent_sized_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache,
-                                                                         int n_pages, const int32_t* __restrict__ table, int table_ld,
-                                                                         const int32_t* __restrict__ len, bf16* __restrict__ out,
-                                                                         float* __restrict__ ws, int H, float scale, int nsplit,
-                                                                         int rows) {
+__global__ __launch_bounds__(512, 2) void attn_latent_sized_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages,
+                                                                   const int32_t* __restrict__ table, int table_ld, const int32_t* __restrict__ len,
+                                                                   bf16* __restrict__ out, float* __restrict__ ws, int H, float scale, int nsplit, int rows) {
     extern __shared__ __align__(16) char smem[];
     const int split = blockIdx.x, row = blockIdx.z, n = len[row];
     const int ntiles = n > 0 ? (n + 63) / 64 : 0;
     const int per = (ntiles + nsplit - 1) / nsplit;
     const int t_beg = min(split * per, ntiles), t_end = min(ntiles, t_beg + per);
-    attn_latent_sized_body<HT, WC, CT>(q, cache, n_pages, table + (int64_t)row * table_ld, n, out, ws, H, scale, nsplit, rows, row,
-                                       blockIdx.y * 16 * HT, split, t_beg, t_end, smem);
+    attn_latent_sized_body(q, cache, n_pages, table + (int64_t)row * table_ld, n, out, ws, H, scale, nsplit, rows, row, blockIdx.y * 32, split, t_beg,
+                           t_end, smem);
 }
 
 // The same attention on the first `workers` workgroups, and a product that waits for nothing of it on the others: out_f += x . W^T, P panels of
-// W each.  A workgroup of either kind has a CU to itself (two pages in LDS), so the two share the chip by CUs: attention asks for 30 bytes a ns
-// and CU behind 10 us of start, the product for up to 50.
+// W each.  A workgroup of either kind has a CU to itself (two pages in LDS), so the two share the chip by CUs: attention draws up to 35 bytes a ns
+// and CU behind 8 us of start, the product up to 50.
 // Splits are dealt: as many pages each, 2 at least where a row has more than 16, as make the splits of all rows fit the workers; a row has
 // nsplit at most, with as many pages each as that takes.  Statistics of splits that a row does not have are zero, which the merge skips.
-// us, 32 heads, attention, merge, value and the output product (shorter by 11 008 of its 15 104), apart -> so: a row of 64 pages 42.3 -> 35.4, 32 rows
-// with 1 184 pages 72.6 -> 64.0 (more beside beside_plan); of eight steps of six layer runs, one row of 4 000 keys 4 987 -> 4 668, 32 rows 7 500 -> 7 225.
+// us, 32 heads, attention, merge, value and the output product (shorter by 11 008 of its 15 104), apart -> so: a row of 64 pages 38.2 -> 33.2, 32 rows
+// with 1 184 pages 67.1 -> 64.8 (more beside beside_plan).
 template <int P, int MT>
 __global__ __launch_bounds__(512, 2) void attn_latent_beside_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages,
                                                                     const int32_t* __restrict__ table, int table_ld, const int32_t* __restrict__ len,
                                                                     float* __restrict__ ws, int H, float scale, int nsplit, int rows, int workers,
                                                                     const TflGemm g) {
     extern __shared__ __align__(16) char smem[];
-    if ((int)blockIdx.x >= workers) {
-        share_gemm_body<bf16, TFL_EPI_RESIDUAL, P, false, MT, 2>(g, 0, 0, blockIdx.x - workers, 0, smem);
+    // which of the two start first: on 128 CUs the product is the longer side up to 1 200 pages (one row of 64 pages 33.4 -> 33.2 us with it first, 32
+    // rows of 1 568 61.6 -> 61.2), on 86 and 64 it is slower for it (40.0 -> 41.5, 45.1 -> 45.7)
+    constexpr bool FIRST = P == 2;
+    const int me = (int)blockIdx.x - (FIRST ? (int)gridDim.x - workers : 0), group = (int)blockIdx.x - (FIRST ? 0 : workers);
+    if (FIRST ? me < 0 : group >= 0) {
+        share_gemm_body<bf16, TFL_EPI_RESIDUAL, P, false, MT, 2>(g, 0, 0, group, 0, smem);
         return;
     }
     const int lane = threadIdx.x & 63;
@@ -523,9 +604,9 @@ __global__ __launch_bounds__(512, 2) void attn_latent_beside_kernel(const bf16* 
         }
         if (per >= most || __shfl(end, 63, 64) <= workers) break;
     }
-    const int row = __popcll(__builtin_amdgcn_ballot_w64(end <= (int)blockIdx.x));            // (lanes past the rows end where the last row does)
+    const int row = __popcll(__builtin_amdgcn_ballot_w64(end <= me));            // (lanes past the rows end where the last row does)
     if (row >= rows) return;
-    const int have = __shfl(mine, row, 64), split = (int)blockIdx.x - (__shfl(end, row, 64) - have), n = len[row];
+    const int have = __builtin_amdgcn_readlane(mine, row), split = me - (__builtin_amdgcn_readlane(end, row) - have), n = len[row];
     const int ntiles = n > 0 ? (n + 63) >> 6 : 0, each = (ntiles + have - 1) / have;
     const int t_beg = min(split * each, ntiles), t_end = min(ntiles, t_beg + each);
     if (split == have - 1)
@@ -533,7 +614,7 @@ __global__ __launch_bounds__(512, 2) void attn_latent_beside_kernel(const bf16* 
             const int head = threadIdx.x & 31;
             if (head < H) ws[(int64_t)rows * H * nsplit * 512 + (((int64_t)row * H + head) * nsplit + s) * 2 + 1] = 0.f;
         }
-    attn_latent_sized_body<2, 18, 32>(q, cache, n_pages, table + (int64_t)row * table_ld, n, nullptr, ws, H, scale, nsplit, rows, row, 0, split, t_beg,
+    attn_latent_sized_body(q, cache, n_pages, table + (int64_t)row * table_ld, n, nullptr, ws, H, scale, nsplit, rows, row, 0, split, t_beg,
                                       t_end, smem);
 }
 
@@ -586,22 +667,14 @@ static int launch_latent(const void* q, const void* cache, int n_pages, const in
     return nsplit > 1 ? launch_merge<T>(ws, out, rows, H, C, nsplit, st) : TF_OK;
 }
 
-template <int HT, int WC, int CT>
-static int launch_latent_sized(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len,
-                               void* out, float* ws, int rows, int H, float scale, int nsplit, hipStream_t st) {
-    constexpr size_t lds = 2 * 64 * (32 * WC + 8) * sizeof(bf16) + 2 * 16 * HT * (64 + 8) * sizeof(bf16) + 4 * 16 * HT * sizeof(float);
-    static_assert(lds <= 160 * 1024, "LDS");
-    auto k = attn_latent_sized_kernel<HT, WC, CT>;
-    static bool attr = false;
-    if (!attr) {
-        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return (int)e;
-        attr = true;
-    }
-    hipLaunchKernelGGL(k, dim3(nsplit, (H + 16 * HT - 1) / (16 * HT), rows), dim3(256 * HT), lds, st, (const bf16*)q, (const bf16*)cache,
+static int launch_latent_sized(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out, float* ws,
+                               int rows, int H, float scale, int nsplit, hipStream_t st) {
+    const hipError_t e = hipFuncSetAttribute((const void*)attn_latent_sized_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LatentTile::LDS);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL(attn_latent_sized_kernel, dim3(nsplit, (H + 31) / 32, rows), dim3(512), LatentTile::LDS, st, (const bf16*)q, (const bf16*)cache,
                        n_pages, table, table_ld, len, (bf16*)out, ws, H, scale, nsplit, rows);
     TFL_LAUNCH_CHECK();
-    return nsplit > 1 ? launch_merge<bf16>(ws, out, rows, H, 16 * CT, nsplit, st) : TF_OK;
+    return nsplit > 1 ? launch_merge<bf16>(ws, out, rows, H, LatentTile::C, nsplit, st) : TF_OK;
 }
 
 extern "C" int tfl_attn_decode(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len,
@@ -614,10 +687,7 @@ extern "C" int tfl_attn_decode(const void* q, const void* cache, int n_pages, co
 #define GO(T, NW, HT, NTW) \
     return launch_latent<T, NW, HT, NTW>(q, cache, n_pages, table, table_ld, len, out, ws, rows, H, C, R, scale, nsplit, st)
     if (dtype == 0) {
-        if (C == 512 && R == 64) {
-            if (H <= 16) return launch_latent_sized<1, 18, 32>(q, cache, n_pages, table, table_ld, len, out, ws, rows, H, scale, nsplit, st);
-            return launch_latent_sized<2, 18, 32>(q, cache, n_pages, table, table_ld, len, out, ws, rows, H, scale, nsplit, st);
-        }
+        if (C == 512 && R == 64) return launch_latent_sized(q, cache, n_pages, table, table_ld, len, out, ws, rows, H, scale, nsplit, st);
         if (C <= 128) { if (H <= 16) GO(bf16, 4, 1, 2); GO(bf16, 4, 2, 2); }
         if (C <= 512) { if (H <= 16) GO(bf16, 4, 1, 8); GO(bf16, 4, 2, 8); }
         if (C <= 1024) GO(bf16, 2, 1, 32);
@@ -636,15 +706,15 @@ extern "C" int tfl_attn_decode(const void* q, const void* cache, int n_pages, co
 // after the other.  The product takes up to half of the CUs, which draw all that memory gives (39 bytes a ns each with their start).  us of a graph of
 // the attention, its merge, latent to value and the whole output product (32 heads, n 4096, k 11 008 of 15 104, rows half to all as long as the longest),
 // apart -> beside with the product on 128 CUs | 86 | 64:
-//   pages in all   one each               ~200                       ~600                      ~1 200                    ~2 400
-//    1 row    34.4->32.5|39.2|44.4   46.9->37.5|44.2|49.2      50.9->44.3|47.0|52.0 (512)
-//    8 rows   39.9->39.4|46.7|51.7   44.6->42.3|49.3|54.2      50.5->47.4|51.8|56.5      60.2->62.4|58.9|58.8      77.2->91.5|81.0|76.9 (6 rows)
-//   16 rows   45.4->42.2|50.5|56.2   46.9->45.5|53.0|57.7      53.1->46.7|54.8|59.5      62.7->61.3|59.4|61.4      77.1->90.4|81.8|76.7
-//   32 rows   57.4->53.0|59.2|65.4   55.8->54.4|60.7|66.6      61.8->54.9|62.7|68.4      72.6->68.5|64.0|70.3      87.1->97.4|84.4|82.4
-// The constants are fitted to these and to 530 other points (20 and 32 heads, 1 to 32 rows, 1 to 512 pages a row, n 4 096 to 8 192, k 2 048 to 16 384): what
-// they pick is 1.003 of the best on average, at most 1.03 of the two apart from k 4 096 on and 1.06 below.  At k 16 384 the product's half of the CUs is by
-// far the longer side: with fewer than 32 pages each, 8 to 32 rows took up to 1.09 of the two apart, with more 0.92 to 0.96.  A page costs 3.9 us of an
-// attention on the whole chip and 4.4 of one on part of it, a row of activations 0.5 in either form (each group of panels reads all of x).
+//   pages in all   one each                ~200                  ~600                  ~1 200                  ~2 350
+//    1 row    31.2->32.6|39.1|44.4   42.8->37.8|44.4|49.3   48.0->41.8|47.0|51.5 (512)
+//    8 rows   37.2->39.7|46.4|51.7   42.1->43.4|50.5|54.5   46.5->45.9|51.9|56.4   53.7->50.8|53.9|59.5   68.7->70.0|64.3|67.6 (16 rows)
+//   16 rows   42.7->42.0|50.2|55.9   44.8->46.1|53.0|57.7   48.9->47.9|55.4|59.8   56.6->50.3|56.4|62.0
+//   32 rows   54.9->53.7|59.8|65.2   54.2->55.1|60.9|66.7   58.7->55.2|63.1|68.4   67.1->57.0|64.8|70.8   79.4->74.4|68.4|75.4
+// The constants were fitted (530 points: 20 and 32 heads, 1 to 32 rows, 1 to 512 pages a row, n 4 096 to 8 192, k 2 048 to 16 384) to the attention before
+// this one, whose page took a CU 4.4 us beside the product and 3.9 on the whole chip, where this one's takes 2.2 and 2.7.  They hold up to some 30 pages
+// a row; behind that they leave the product fewer CUs than it would like (32 rows, 1 200 to 1 600 pages in all: 64.8 and 66.4 on 86, 57.0 and 61.4 on 128).
+// At k 16 384 the product's half of the CUs is by far the longer side.  A row of activations costs 0.5 in either form (each group of panels reads all of x).
 static int beside_plan(int rows, int H, int64_t pages, int n, int k, int* panels_each) {
     const int panels = n >> 4;
     if (rows < 1 || rows > 32 || H <= 16 || H > 32 || pages < 1 || pages > (1 << 20) || panels < 256 || panels > 512 || k < 2048) return 0;
@@ -680,8 +750,8 @@ extern "C" int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages
 template <int P, int MT>
 static int launch_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, float* ws, int rows, int H,
                          float scale, int nsplit, int workers, const TflGemm& g, hipStream_t st) {
-    constexpr int LDS = 2 * 64 * (32 * 18 + 8) * (int)sizeof(bf16) + 2 * 32 * (64 + 8) * (int)sizeof(bf16) + 4 * 32 * (int)sizeof(float);
-    static_assert(LDS <= 160 * 1024 && 8 * P * MT * 64 * (int)sizeof(f32x4) <= LDS, "LDS");
+    constexpr int LDS = LatentTile::LDS;
+    static_assert(8 * P * MT * 64 * (int)sizeof(f32x4) <= LDS, "LDS");
     const hipError_t e = hipFuncSetAttribute((const void*)attn_latent_beside_kernel<P, MT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e != hipSuccess) return (int)e;
     hipLaunchKernelGGL((attn_latent_beside_kernel<P, MT>), dim3(workers + ((g.n >> 4) + P - 1) / P), dim3(512), LDS, st, (const bf16*)q, (const bf16*)cache,
