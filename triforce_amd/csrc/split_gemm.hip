@@ -21,9 +21,14 @@
 // into planes, weights cost 6 bytes beside the 4 and gain 3 to 8 %: 22 016 x 4 096 at 700 rows 706 us against 730.  The cut between the
 // products instead of behind them waits for x's DMA before each store to LDS: 22 016 x 4 096 at 2 048 rows 1 830 -> 2 230 us.)
 //
-// Bound by the power of the matrix cores (1.6 to 1.7 GHz under these products, as bf16 GEMMs) and by rounds of tiles.  fp32 GEMM before ->
-// now, x's cut and the sum of parts included: 700 rows, 22 016 x 4 096 940 -> 665 us, 18 784 x 4 096 900 -> 565, 4 096 x 15 104 680 -> 460;
-// 2 048 rows, 22 016 x 4 096 2 600 -> 1 800 (205 TFLOP/s).
+// Bound by the power of the matrix cores (1.6 to 1.7 GHz under these products, as bf16 GEMMs), by what a step costs beside its products (all
+// operands zero, at full clock: 22 016 x 4 096 at 700 rows 613 -> 567 us) and by rounds of tiles.  A matrix core draws less where a product goes to the sum
+// that the one before it went to (registers alone, bf16 normals: 2 110 TFLOP/s with another sum each time, 2 226 in twos, 2 350 in fours, 2 395 in
+// eights), so the five small products of a result follow each other, and a row tile's parts are read during the products of the one before: 700 rows,
+// 22 016 x 4 096 665 -> 613 us, 18 784 x 4 096 567 -> 537, 4 096 x 15 104 481 -> 460, 4 096 x 8 192 266 -> 256; 2 048 rows of 22 016 1 719 -> 1 642
+// (225 TFLOP/s); 256 rows of 12 320 158 -> 156.  (In two halves, four waves cutting their weights in front of the products and four behind: nothing.)
+// The fp32 instruction, x's cut and the sum of parts included: 700 rows, 22 016 x 4 096 940 us, 18 784 x 4 096 900, 4 096 x 15 104 680; 2 048 rows,
+// 22 016 x 4 096 2 600.
 //
 // Range: both operands are cut at 2^24 times their value, so the last bit of the smallest float32 (2^-149) is still a normal bfloat16 and no
 // product of parts that counts leaves fp32's range below; results are multiplied by 2^-48.  Above, a factor from 2^104 or a sum from 2^80
@@ -278,18 +283,23 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
             for (int t = 0; t < 4; ++t)
 #pragma unroll
                 for (int z = 0; z < 3; ++z) w[t][z] = load_frag(wt + (3 * t + z) * 512);
+            bf16x8 x[2][3];
+            auto read_x = [&](int m) {
+#pragma unroll
+                for (int z = 0; z < 3; ++z) x[m & 1][z] = load_frag(xt + (3 * m + z) * 512);
+            };
+            read_x(0);
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-                bf16x8 x[3];
-#pragma unroll
-                for (int z = 0; z < 3; ++z) x[z] = load_frag(xt + (3 * m + z) * 512);
                 constexpr int WZ[6] = {2, 0, 1, 1, 0, 0}, XZ[6] = {0, 2, 1, 0, 1, 0};          // smallest first
+                if (m + 1 < MT) read_x(m + 1);
 #pragma unroll
-                for (int q = 0; q < 6; ++q)
+                for (int t = 0; t < 4; ++t)
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) {
+                    for (int q = 0; q < 6; ++q) {
                         f32x4& s = q < 5 ? low[t][m] : acc[t][m];
-                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][WZ[q]], x[XZ[q]], s, 0, 0, 0);
+                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][WZ[q]], x[m & 1][XZ[q]], s, 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);    // (left to itself the scheduler deals them out among the sums)
                     }
             }
         }
