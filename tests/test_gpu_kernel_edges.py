@@ -442,6 +442,21 @@ def test_split_float32_product(rows, n, k, splits):
         assert err.max() <= 2.0 ** -24 * (6 * k / 32) ** 0.5 + 2.0 ** -22
 
 
+# row tiles of up to 64 rows and of more, waves with some of their panels and with none, one step and two of a tile or part
+@pytest.mark.parametrize("k,splits", [(32, 1), (64, 2), (64, 1), (352, 3), (4096, 0)])
+@pytest.mark.parametrize("rows,n", [(16, 16), (64, 304), (65, 208), (192, 256), (193, 80), (330, 1040)])
+def test_split_float32_ragged_tiles(rows, n, k, splits):
+    from triforce_amd import ops_tile as ot
+    g = torch.Generator(device=DEV).manual_seed(rows + n + k)
+    x, w = torch.randn(rows, k, generator=g, device=DEV), torch.randn(n, k, generator=g, device=DEV)
+    got, want = ot.split_linear(x, w, splits).double(), x.double() @ w.double().T
+    # every result for itself: six sums per 32 columns, a walk of at most 2^-24 a step of the size of what has been added up
+    assert ((got - want).abs() / (x.double().abs() @ w.double().abs().T)).max() <= 5 * 2.0 ** -24 * (1 + (k / 32 / 3) ** 0.5)
+    x[rows - 1, k - 1], w[n - 1, 0] = float("inf"), -float("inf")
+    odd, rest = ot.split_linear(x, w, splits).double(), (slice(0, rows - 1), slice(0, n - 1))
+    assert torch.equal(odd[rest], got[rest]) and not torch.isfinite(odd[rows - 1]).any() and not torch.isfinite(odd[:, n - 1]).any()
+
+
 # more tiles than CUs: whole rounds of whole tiles and the steps of the others shared by an XCD's CUs; k of no whole eights of steps, ragged last
 # tiles, XCDs with one shared tile and with none, few sharers
 @pytest.mark.parametrize("rows,n,k", [(1040, 7680, 1024), (1100, 7664, 1056), (700, 12320, 1536), (896, 9472, 2048), (2050, 4112, 4064)])

@@ -14,19 +14,21 @@
 // rows 730 -> 740 us.)
 // Six bf16 instructions take 3/8 of the cycles of the eight fp32 ones that cover the same 16 x 16 x 32.
 //
-// 256 outputs x 128 rows per workgroup, eight waves of 64 x 64: per step of 32 a wave reads 24 KB from LDS for 96 products (1 536 cycles),
-// half of what LDS delivers.  x is cut once by a kernel in front, into planes in MFMA order ([rows/16][k/32][3][64 lanes][8]: a fragment is one
-// contiguous KiB that goes to LDS by DMA); a weight is used by one workgroup per 128 rows and is cut on its way to LDS, beside the products.
+// 256 outputs x 128 rows per workgroup, four waves of 64 x 128, one per SIMD: per step of 32 a wave reads 36 KB from LDS for 192 products (3 170
+// cycles), a third of what LDS delivers.  x is cut once by a kernel in front, into planes in MFMA order ([rows/16][k/32][3][64 lanes][8]: a fragment is one
+// contiguous KiB that goes to LDS by DMA); a weight is used by one workgroup per 128 rows and is cut on its way to LDS, between the products.
 // (Cut at load time
-// into planes, weights cost 6 bytes beside the 4 and gain 3 to 8 %: 22 016 x 4 096 at 700 rows 706 us against 730.  The cut between the
-// products instead of behind them waits for x's DMA before each store to LDS: 22 016 x 4 096 at 2 048 rows 1 830 -> 2 230 us.)
+// into planes, weights cost 6 bytes beside the 4 and gain 3 to 8 %.)  A wave issues one operation in five cycles and a product takes sixteen, so two
+// operations behind every product cost nothing and five behind every third product do: the cut goes in eighths, 128 of them behind 144 products
+// (in thirds 2 048 rows of 22 016 1 565 -> 1 665 us, two products at a time 1 645).  Weights asked for in whole lines of 128 bytes, an eighth of the
+// rows a load, need twice the stores to LDS: 1 565 -> 1 577; asked for four steps ahead into L2 as well, 1 644.
 //
-// Bound by the power of the matrix cores (1.6 to 1.7 GHz under these products, as bf16 GEMMs), by what a step costs beside its products (all
-// operands zero, at full clock: 22 016 x 4 096 at 700 rows 613 -> 567 us) and by rounds of tiles.  A matrix core draws less where a product goes to the sum
+// Bound by the power of the matrix cores (1.6 to 1.7 GHz under these products, as bf16 GEMMs; all operands zero, at full clock, 22 016 x 4 096 at 700
+// rows takes 536 us), by what a step costs beside its products and by rounds of tiles.  A matrix core draws less where a product goes to the sum
 // that the one before it went to (registers alone, bf16 normals: 2 110 TFLOP/s with another sum each time, 2 226 in twos, 2 350 in fours, 2 395 in
-// eights), so the five small products of a result follow each other, and a row tile's parts are read during the products of the one before: 700 rows,
-// 22 016 x 4 096 665 -> 613 us, 18 784 x 4 096 567 -> 537, 4 096 x 15 104 481 -> 460, 4 096 x 8 192 266 -> 256; 2 048 rows of 22 016 1 719 -> 1 642
-// (225 TFLOP/s); 256 rows of 12 320 158 -> 156.  (In two halves, four waves cutting their weights in front of the products and four behind: nothing.)
+// eights), so the five small products of a result follow each other.  700 rows, each product to another sum in eight waves of 64 x 64 -> in fives -> four
+// waves: 22 016 x 4 096 665 -> 613 -> 588 us, 18 784 x 4 096 567 -> 537 -> 512, 4 096 x 15 104 481 -> 456 -> 427, 4 096 x 8 192 266 -> 256 -> 247; 2 048
+// rows of 22 016 1 719 -> 1 632 -> 1 563 (236 TFLOP/s); 256 rows of 12 320 158 -> 156 -> 149.
 // The fp32 instruction, x's cut and the sum of parts included: 700 rows, 22 016 x 4 096 940 us, 18 784 x 4 096 900, 4 096 x 15 104 680; 2 048 rows,
 // 22 016 x 4 096 2 600.
 //
@@ -37,6 +39,7 @@
 // an infinity leaves behind in a model, are marked when they are cut and keep their NaN results.  One infinite row of 700 in front of
 // 22 016 x 4 096 costs 770 -> 1 040 us, of 300 in front of 4 096 x 15 104 265 -> 530 (by a thread per result 4 200 and 9 900).  (The scaling is 16 of some 200 VALU operations per step: 22 016 x 4 096 at 700 rows 740 -> 752 us.)
 #include "tile_common.h"
+#include <type_traits>
 
 #define SPLIT_KC 512                   // columns of x that one workgroup cuts
 #define SPLIT_SCALE 0x1p24f            // of either operand
@@ -67,6 +70,24 @@ __device__ __forceinline__ void cut_store(const f32x4 (&v)[2], bf16* dst) {
     }
 #pragma unroll
     for (int z = 0; z < 3; ++z) *reinterpret_cast<u32x4*>(dst + 512 * z) = out[z];
+}
+
+// 16 bytes a lane from `from` + off to LDS at `to` + 16 * lane.  Not counted by the compiler, which behind its own form waits for all reads of
+// LDS that are under way wherever one is needed: see meet().
+__device__ __forceinline__ void lds_dma(bf16* to, uint32_t off, const bf16* from) {
+    const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)to;
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(off), "s"(from) : "memory");
+}
+
+// A product without the compiler's say in where its sum goes: it moves some of 256 registers of sums through others in every step.  It does not
+// see then what the matrix core still has to read or write: see hold().
+__device__ __forceinline__ void add_in_place(bf16x8 a, bf16x8 b, f32x4& c) { asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b)); }
+// Twelve wait states between products and what else touches their sums: behind a 16 x 16 x 32 product (eight passes) eleven are needed.  Behind the
+// products of a step, inside their loop, so that no copy of a sum can come first.
+__device__ __forceinline__ void hold() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 11" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // One workgroup: 16 rows, SPLIT_KC columns.  nans[row][part]: the row has a NaN in this part of k.
@@ -174,16 +195,24 @@ __device__ __forceinline__ void mend(const SplitGemm& a, int row0, int n0, f32x4
     for (int e = 0; e < 4; ++e) v[e] = lost[e] ? p[e] : v[e];
 }
 
-// Waves: 4 x 64 outputs, 2 x 64 rows (MT 16-row tiles of x each); every wave brings PER fragments of x in.  FOLDS: a.fold is below a tile's steps.
+// f(0), f(1), .. f(N - 1), their arguments known to the compiler.
+template <int N, int I = 0, class F> __device__ __forceinline__ void upto(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        upto<N, I + 1>(f);
+    }
+}
+
+// Waves: 4 x 64 outputs, one per SIMD, each with all 128 rows.  FOLDS: a.fold is below a tile's steps.
 template <bool FOLDS>
-__global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
-    constexpr int MT = 4, NP = 16, XP = 2 * MT, PER = 3 * XP / 8, BUF = 3 * (NP + XP) * 512;
-    extern __shared__ __align__(16) bf16 tiles[];             // [2][NP + XP][3][512]
+__global__ __launch_bounds__(256, 1) void split_gemm_kernel(const SplitGemm a) {
+    constexpr int MT = 8, NP = 16, PER = 3 * MT / 4, BUF = 3 * (NP + MT) * 512;
+    extern __shared__ __align__(16) bf16 tiles[];             // [2][NP + MT][3][512]
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15;
-    const int wn = wave & 3, wm = wave >> 2, chunks = a.k >> 5;
+    const int chunks = a.k >> 5;
     // workgroups go round-robin over the 8 XCDs: each takes an eighth of the tiles, the row tiles of one column tile one after the other, which
     // share its weights in L2
-    const int mts = (a.rows + 32 * MT - 1) / (32 * MT), xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int mts = (a.rows + 16 * MT - 1) / (16 * MT), xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
     const Share share = share_of((a.n + 255) / 256 * mts, chunks, a.whole, a.splits, a.sharers, xcd);
     int q = j - share.own;
     if (q >= share.sharers) return;
@@ -195,32 +224,31 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
     }
     const int xpan = (a.rows + 15) >> 4;
     const bf16* src[PER];                                     // this wave's fragments of x: scalar pointers to their first chunk
-    const float* wsrc[2];                                     // this lane's eight weights of two panels
-    f32x4 staged[2][2];
-    auto fetch_x = [&](int c, int buf) {
+    const float* wsrc[4];                                     // this lane's eight weights of four panels
+    f32x4 staged[4][2];
+    auto fetch_x = [&](int f, int c, int buf) { lds_dma(tiles + buf * BUF + (3 * NP + wave * PER + f) * 512, 16u * lane, src[f] + (int64_t)c * 1536); };
+    auto fetch_w = [&](int f, int c) {
 #pragma unroll
-        for (int f = 0; f < PER; ++f)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[f] + (int64_t)c * 1536 + lane * 8),
-                                             (__attribute__((address_space(3))) void*)(tiles + buf * BUF + (3 * NP + wave * PER + f) * 512), 16, 0, 0);
+        for (int h = 0; h < 2; ++h) staged[f][h] = *reinterpret_cast<const f32x4*>(wsrc[f] + 32 * c + 4 * h);
     };
-    auto fetch_w = [&](int c) {
-#pragma unroll
-        for (int f = 0; f < 2; ++f)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) staged[f][h] = *reinterpret_cast<const f32x4*>(wsrc[f] + 32 * c + 4 * h);
-    };
-    auto put_w = [&](int buf) {
-#pragma unroll
-        for (int f = 0; f < 2; ++f) cut_store(staged[f], tiles + buf * BUF + (wave + 8 * f) * 1536 + lane * 8);
-    };
-    // What makes a step's tiles visible to the other waves: this wave's DMA has landed (nothing may be in flight but the weights asked for
-    // behind it, which stay in flight over the barrier), its LDS stores are done, and no access crosses the barrier.  Both are compiler
-    // fences too: an access to LDS may not move over them, whatever order the scheduler likes.
+    bf16x8 w[4][3], x[2][3];
+    auto read_w = [&](int t, int z, int buf) { w[t][z] = load_frag(tiles + buf * BUF + (3 * (4 * wave + t) + z) * 512 + lane * 8); };
+    auto read_x = [&](int m, int z, int buf) { x[m & 1][z] = load_frag(tiles + buf * BUF + (3 * (NP + m) + z) * 512 + lane * 8); };
+    // What makes a step's tiles visible to the other waves: this wave's DMA has landed (nothing may be in flight but weights asked for behind
+    // it, which stay in flight over the barrier), its LDS stores are done, and no access crosses the barrier.  Both are compiler fences too: an access
+    // to LDS may not move over them, whatever order the scheduler likes.
     auto landed = [&] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
     auto meet = [&] {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
+    };
+    f32x4 acc[4][MT], low[4][MT];                             // hh and the five small products
+    auto clear = [&] {
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) acc[t][m] = low[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
     };
     do {
     const int r = beg / chunks, c_beg = beg - r * chunks, c_end = min(chunks, c_beg + end - beg), id = share.first + (q < 0 ? j : share.own + r);
@@ -228,111 +256,153 @@ __global__ __launch_bounds__(512, 2) void split_gemm_kernel(const SplitGemm a) {
 #pragma unroll
     for (int f = 0; f < PER; ++f) {
         const int p = (wave * PER + f) / 3, z = (wave * PER + f) % 3;
-        src[f] = a.xp + (int64_t)min(mt0 * XP + p, xpan - 1) * chunks * 1536 + z * 512;
+        src[f] = a.xp + (int64_t)min(mt0 * MT + p, xpan - 1) * chunks * 1536 + z * 512;
     }
 #pragma unroll
-    for (int f = 0; f < 2; ++f) wsrc[f] = a.w + (int64_t)min(nt * 256 + 16 * (wave + 8 * f) + i, a.n - 1) * a.k + 8 * g;
-    const bool live = mt0 * XP + wm * MT < xpan;              // a wave without rows leaves the matrix core to its neighbour
+    for (int f = 0; f < 4; ++f) wsrc[f] = a.w + (int64_t)min(nt * 256 + 16 * (wave + 4 * f) + i, a.n - 1) * a.k + 8 * g;
     float* part = q < 0 ? nullptr : a.ws + ((int64_t)xcd * a.slots + q + r) * SLOT;           // a row of 256 behind the other
-    f32x4 acc[4][MT], low[4][MT];                             // hh and the five small products
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[t][m] = low[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // f of this lane's places in the result, or in the part's slot
-    const int lines = q < 0 ? a.rows : 1 << 30;
+    clear();
+    // f of this lane's places in a row of the result, or of the part's slot, one row tile after the other
+    const int lines = q < 0 ? a.rows : 1 << 30, panels = min(4, (a.n - nt * 256 - 64 * wave) >> 4);
     bool lost = false;                                        // a result that is not finite
     auto each = [&](auto&& f) {
         int at = lane;
-        if constexpr (FOLDS) asm volatile("" : "+v"(at));     // (places made ahead of the steps would take registers from them)
+        asm volatile("" : "+v"(at));                          // (places made ahead of the steps would take registers from them)
         const int g = at >> 4, i = at & 15;
-        float* y = q < 0 ? a.out : part;
+        float* y = (q < 0 ? a.out + nt * 256 : part) + 64 * wave + 4 * g;
         const int64_t ld = q < 0 ? a.ld_out : 256;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            const int in_row = 16 * (wm * MT + m), row0 = mt0 * 32 * MT + in_row;
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int in_n = 64 * wn + 16 * t;
-                if constexpr (FOLDS) {                        // one after the other: what is there would take a step's registers
-                    asm volatile("" ::: "memory");
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                if (row0 >= a.rows || nt * 256 + in_n >= a.n) continue;
-                f(m, t, reinterpret_cast<f32x4*>(y + (q < 0 ? row0 + i : in_row + i) * ld + (q < 0 ? nt * 256 : 0) + in_n + 4 * g), row0, i);
-            }
+            const int row0 = mt0 * 16 * MT + 16 * m;
+            asm volatile("" ::: "memory");                    // (sums and places of all rows, read ahead, would take all registers)
+            __builtin_amdgcn_sched_barrier(0);
+            if (row0 < a.rows) f(m, reinterpret_cast<f32x4*>(y + (q < 0 ? row0 + i : 16 * m + i) * ld), row0, row0 + i < lines);
         }
     };
+    // Steps c .. stop - 1 over the first LIVE row tiles.  While step c is multiplied the weights of c + 1 are cut, between its products, and those of
+    // c + 2 asked for, as soon as x of c + 1 has landed.  The waves meet in front of the last row tile, whose x is in registers: from there on x of c + 2
+    // may come in over this step's, and w and x of c + 1 are read behind their last use.
+    auto run = [&](auto live, int& c, int stop) __attribute__((always_inline)) {
+        constexpr int LIVE = decltype(live)::value, CUTS = 4 * (LIVE - 2);     // (cut behind the first CUTS results)
+        for (; c < stop; ++c) {
+            const int buf = (c - c_beg) & 1;
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_nop 1" ::: "memory");             // (between zeros and copies, which the loop may begin with, and the products that read them)
+            __builtin_amdgcn_sched_barrier(0);
+            float va = 0.f, vb = 0.f;
+            u32x4 out[3];
+            // an eighth of the cut of a pair: two operations at most, what the matrix core leaves room for behind a product
+            uint32_t ha, hb;
+            auto cut = [&](auto at) __attribute__((always_inline)) {
+                constexpr int p = decltype(at)::value / 8, f = p / 4, e = p % 4, z = decltype(at)::value % 8;
+                if constexpr (z == 0) {
+                    va = staged[f][e >> 1][2 * (e & 1)] * SPLIT_SCALE;
+                    vb = staged[f][e >> 1][2 * (e & 1) + 1] * SPLIT_SCALE;
+                    asm volatile("" ::"v"(va), "v"(vb));
+                } else if constexpr (z == 1 || z == 4 || z == 7) {
+                    typedef bf16 Pair __attribute__((ext_vector_type(2)));
+                    constexpr int y = z / 3;
+                    uint32_t v = __builtin_bit_cast(uint32_t, Pair{(bf16)va, (bf16)vb});
+                    asm("" : "+v"(v));
+                    out[y][e] = v;
+                    if constexpr (e == 3) *reinterpret_cast<u32x4*>(tiles + (buf ^ 1) * BUF + (wave + 4 * f) * 1536 + 512 * y + lane * 8) = out[y];
+                    if constexpr (f == 0 && e == 3 && y == 2) landed();                  // (x of the next step, asked for behind the last barrier)
+                    if constexpr (e == 3 && y == 2) fetch_w(f, min(c + 2, c_end - 1));
+                } else if constexpr (z == 2 || z == 5) {
+                    ha = out[z / 3][e] << 16;
+                    hb = out[z / 3][e] & 0xFFFF0000u;
+                    asm volatile("" ::"v"(ha), "v"(hb));
+                } else {
+                    va -= __builtin_bit_cast(float, ha);
+                    vb -= __builtin_bit_cast(float, hb);
+                    asm volatile("" ::"v"(va), "v"(vb));
+                }
+            };
+            upto<24 * LIVE>([&](auto at) __attribute__((always_inline)) {
+                constexpr int s = decltype(at)::value % 6, t = decltype(at)::value / 6 % 4, m = decltype(at)::value / 24;
+                constexpr int WZ[6] = {2, 0, 1, 1, 0, 0}, XZ[6] = {0, 2, 1, 0, 1, 0};          // smallest first
+                constexpr int P = decltype(at)::value, FIRST = P < 6 * CUTS ? 128 * P / (6 * CUTS) : 0, N = P < 6 * CUTS ? 128 * (P + 1) / (6 * CUTS) - FIRST : 0;
+                if constexpr (m == LIVE - 1 && t == 0 && s == 0) meet();
+                if constexpr (s < 5) add_in_place(w[t][WZ[s]], x[m & 1][XZ[s]], low[t][m]);
+                else add_in_place(w[t][WZ[s]], x[m & 1][XZ[s]], acc[t][m]);
+                __builtin_amdgcn_sched_barrier(0);
+                upto<N>([&](auto n) __attribute__((always_inline)) { cut(std::integral_constant<int, FIRST + decltype(n)::value>()); });
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (t < 3 && s == 0) read_x(m + 1 < LIVE ? m + 1 : 0, t, m + 1 < LIVE ? buf : buf ^ 1);
+                if constexpr (m + 1 == LIVE && t > 0 && (s & 1) == 0) read_w(t - 1, s / 2, buf ^ 1);
+                if constexpr (m + 1 == LIVE && t == 0) fetch_x(s, min(c + 2, c_end - 1), buf);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+#pragma unroll
+            for (int z = 0; z < 3; ++z) read_w(3, z, buf ^ 1);
+            hold();
+        }
+    };
+    const bool half = xpan - mt0 * MT <= MT / 2;
     if (c_beg < c_end) {
-        fetch_x(c_beg, 0);
-        fetch_w(c_beg);
-        put_w(0);
+#pragma unroll
+        for (int f = 0; f < PER; ++f) fetch_x(f, c_beg, 0);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) fetch_w(f, c_beg);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) cut_store(staged[f], tiles + (wave + 4 * f) * 1536 + lane * 8);
         landed();
-        fetch_w(min(c_beg + 1, c_end - 1));
+#pragma unroll
+        for (int f = 0; f < 4; ++f) fetch_w(f, min(c_beg + 1, c_end - 1));
         meet();
+#pragma unroll
+        for (int f = 0; f < PER; ++f) fetch_x(f, min(c_beg + 1, c_end - 1), 1);
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int z = 0; z < 3; ++z) read_w(t, z, 0);
+#pragma unroll
+        for (int z = 0; z < 3; ++z) read_x(0, z, 0);
     }
     for (int c = c_beg;;) {
-    for (const int stop = FOLDS ? min(c_end, c + a.fold) : c_end; c < stop; ++c) {
-        const int buf = (c - c_beg) & 1;
-        fetch_x(min(c + 1, c_end - 1), buf ^ 1);              // in flight under this step's products
-        if (live) {
-            const bf16* wt = tiles + buf * BUF + wn * 4 * 1536 + lane * 8;
-            const bf16* xt = tiles + buf * BUF + (NP + wm * MT) * 1536 + lane * 8;
-            bf16x8 w[4][3];
+    const int stop = FOLDS ? min(c_end, c + a.fold) : c_end;
+    if (half) run(std::integral_constant<int, MT / 2>(), c, stop);
+    else run(std::integral_constant<int, MT>(), c, stop);
+    if constexpr (!FOLDS) break;
+    each([&](int m, f32x4* y, int, bool live) {               // sums go to the result, or to a part's slot, and to what is there
+        f32x4 have[4] = {};
+        if (c > c_beg + a.fold && live)
 #pragma unroll
             for (int t = 0; t < 4; ++t)
+                if (t < panels) have[t] = y[4 * t];
 #pragma unroll
-                for (int z = 0; z < 3; ++z) w[t][z] = load_frag(wt + (3 * t + z) * 512);
-            bf16x8 x[2][3];
-            auto read_x = [&](int m) {
+        for (int t = 0; t < 4; ++t) {
+            asm volatile("" : "+a"(acc[t][m]), "+a"(low[t][m]));
+            f32x4 v;
 #pragma unroll
-                for (int z = 0; z < 3; ++z) x[m & 1][z] = load_frag(xt + (3 * m + z) * 512);
-            };
-            read_x(0);
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                constexpr int WZ[6] = {2, 0, 1, 1, 0, 0}, XZ[6] = {0, 2, 1, 0, 1, 0};          // smallest first
-                if (m + 1 < MT) read_x(m + 1);
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int q = 0; q < 6; ++q) {
-                        f32x4& s = q < 5 ? low[t][m] : acc[t][m];
-                        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][WZ[q]], x[m & 1][XZ[q]], s, 0, 0, 0);
-                        __builtin_amdgcn_sched_barrier(0);    // (left to itself the scheduler deals them out among the sums)
-                    }
+            for (int e = 0; e < 4; ++e) {
+                v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE)) + have[t][e];
+                lost = lost || (t < panels && !(__builtin_fabsf(v[e]) < __builtin_inff()));
             }
+            if (t < panels && live) y[4 * t] = v;
         }
-        put_w(buf ^ 1);
-        landed();
-        fetch_w(min(c + 2, c_end - 1));
-        meet();
-    }
-    if constexpr (!FOLDS) break;
-    each([&](int m, int t, f32x4* y, int row0, int i) {       // sums go to the result, or to a part's slot, and to what is there
-        f32x4 v, have = {0.f, 0.f, 0.f, 0.f};
-        if (c > c_beg + a.fold && row0 + i < lines) have = *y;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE)) + have[e];
-            lost = lost || !(__builtin_fabsf(v[e]) < __builtin_inff());
-        }
-        acc[t][m] = low[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (row0 + i < lines) *y = v;
     });
     if (c >= c_end) break;
+    clear();
     }
+    landed();
+    meet();                                                   // nothing is on its way to LDS, and nobody reads it
     if (!FOLDS || (q < 0 && __any(lost)))
-        each([&](int m, int t, f32x4* y, int row0, int i) {
-            f32x4 v = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (!FOLDS) {
+        each([&](int m, f32x4* y, int row0, bool live) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE));
-            } else if (row0 + i < lines) {
-                v = *y;
+            for (int t = 0; t < 4; ++t) {
+                f32x4 v = {0.f, 0.f, 0.f, 0.f};
+                if (t >= panels) continue;
+                if constexpr (!FOLDS) {
+                    asm volatile("" : "+a"(acc[t][m]), "+a"(low[t][m]));
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE));
+                } else if (live) {
+                    v = y[4 * t];
+                }
+                if (q < 0) mend(a, row0, nt * 256 + 64 * wave + 16 * t, v);
+                if (live) y[4 * t] = v;
             }
-            if (q < 0) mend(a, row0, nt * 256 + 64 * wn + 16 * t, v);
-            if (row0 + i < lines) *y = v;
         });
     beg += c_end - c_beg;
     } while (beg < end);
@@ -372,7 +442,7 @@ static int launch_split_gemm(const SplitGemm& a, hipStream_t st) {
     const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e != hipSuccess) return (int)e;
     const int each = (split_tiles(a.rows, a.n) + 7) / 8, own = each < a.whole ? each : a.whole, rest = each - own;
-    hipLaunchKernelGGL(kernel, dim3(8 * (own + (rest == 0 ? 0 : a.sharers > 0 ? a.sharers : rest * a.splits))), dim3(512), LDS, st, a);
+    hipLaunchKernelGGL(kernel, dim3(8 * (own + (rest == 0 ? 0 : a.sharers > 0 ? a.sharers : rest * a.splits))), dim3(256), LDS, st, a);
     TFL_LAUNCH_CHECK();
     if (rest > 0) {
         hipLaunchKernelGGL(split_sum_kernel, dim3((unsigned)rest * 256), dim3(256), 0, st, a);
