@@ -37,7 +37,8 @@
 // on becomes infinite on the way; such a result, and one that is not finite because a factor is not (an infinity times a zero part is NaN),
 // is computed again in plain fp32, the 16 x 16 tile that it lies in by its wave on the fp32 instruction; rows of x with a NaN, which is what
 // an infinity leaves behind in a model, are marked when they are cut and keep their NaN results.  One infinite row of 700 in front of
-// 22 016 x 4 096 costs 770 -> 1 040 us, of 300 in front of 4 096 x 15 104 265 -> 530 (by a thread per result 4 200 and 9 900).  (The scaling is 16 of some 200 VALU operations per step: 22 016 x 4 096 at 700 rows 740 -> 752 us.)
+// 22 016 x 4 096 costs 600 -> 1 070 us, of 300 in front of 4 096 x 15 104 236 -> 665 (by a thread per result 4 200 and 9 900).  The kernel stores all
+// sums first and walks through a wave's tiles again where one was odd: thirty-two walks in line cost every launch 4 %.  (The scaling is 16 of some 200 VALU operations per step: 22 016 x 4 096 at 700 rows 740 -> 752 us.)
 #include "tile_common.h"
 #include <type_traits>
 
@@ -262,21 +263,41 @@ __global__ __launch_bounds__(256, 1) void split_gemm_kernel(const SplitGemm a) {
     for (int f = 0; f < 4; ++f) wsrc[f] = a.w + (int64_t)min(nt * 256 + 16 * (wave + 4 * f) + i, a.n - 1) * a.k + 8 * g;
     float* part = q < 0 ? nullptr : a.ws + ((int64_t)xcd * a.slots + q + r) * SLOT;           // a row of 256 behind the other
     clear();
-    // f of this lane's places in a row of the result, or of the part's slot, one row tile after the other
     const int lines = q < 0 ? a.rows : 1 << 30, panels = min(4, (a.n - nt * 256 - 64 * wave) >> 4);
-    bool lost = false;                                        // a result that is not finite
-    auto each = [&](auto&& f) {
+    float odd = 0.f;                                          // NaN behind a result that is not finite
+    // this lane's places in row 0 of the result, or of the part's slot, and of the row tiles behind it
+    float* y0 = (q < 0 ? a.out + nt * 256 : part) + 64 * wave;
+    const int64_t ld = q < 0 ? a.ld_out : 256;
+    auto place = [&](int m, int at) { return reinterpret_cast<f32x4*>(y0 + ((q < 0 ? mt0 * 16 * MT : 0) + 16 * m + (at & 15)) * ld + 4 * (at >> 4)); };
+    // Sums go to the result, or to a part's slot, and to what is there.
+    auto put = [&](bool more) __attribute__((always_inline)) {
         int at = lane;
         asm volatile("" : "+v"(at));                          // (places made ahead of the steps would take registers from them)
-        const int g = at >> 4, i = at & 15;
-        float* y = (q < 0 ? a.out + nt * 256 : part) + 64 * wave + 4 * g;
-        const int64_t ld = q < 0 ? a.ld_out : 256;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const int row0 = mt0 * 16 * MT + 16 * m;
             asm volatile("" ::: "memory");                    // (sums and places of all rows, read ahead, would take all registers)
             __builtin_amdgcn_sched_barrier(0);
-            if (row0 < a.rows) f(m, reinterpret_cast<f32x4*>(y + (q < 0 ? row0 + i : 16 * m + i) * ld), row0, row0 + i < lines);
+            if (row0 >= a.rows) break;
+            f32x4* y = place(m, at);
+            const bool live = row0 + (at & 15) < lines;
+            f32x4 have[4] = {};
+            if (FOLDS && more && live)
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (t < panels) have[t] = y[4 * t];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                asm volatile("" : "+a"(acc[t][m]), "+a"(low[t][m]));
+                f32x4 v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE));
+                    if constexpr (FOLDS) v[e] += have[t][e];
+                    odd = fmaf(v[e], 0.f, odd);
+                }
+                if (t < panels && live) y[4 * t] = v;
+            }
         }
     };
     // Steps c .. stop - 1 over the first LIVE row tiles.  While step c is multiplied the weights of c + 1 are cut, between its products, and those of
@@ -363,47 +384,22 @@ __global__ __launch_bounds__(256, 1) void split_gemm_kernel(const SplitGemm a) {
     const int stop = FOLDS ? min(c_end, c + a.fold) : c_end;
     if (half) run(std::integral_constant<int, MT / 2>(), c, stop);
     else run(std::integral_constant<int, MT>(), c, stop);
-    if constexpr (!FOLDS) break;
-    each([&](int m, f32x4* y, int, bool live) {               // sums go to the result, or to a part's slot, and to what is there
-        f32x4 have[4] = {};
-        if (c > c_beg + a.fold && live)
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-                if (t < panels) have[t] = y[4 * t];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            asm volatile("" : "+a"(acc[t][m]), "+a"(low[t][m]));
-            f32x4 v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE)) + have[t][e];
-                lost = lost || (t < panels && !(__builtin_fabsf(v[e]) < __builtin_inff()));
-            }
-            if (t < panels && live) y[4 * t] = v;
-        }
-    });
-    if (c >= c_end) break;
+    put(c > c_beg + a.fold);
+    if (!FOLDS || c >= c_end) break;
     clear();
     }
     landed();
     meet();                                                   // nothing is on its way to LDS, and nobody reads it
-    if (!FOLDS || (q < 0 && __any(lost)))
-        each([&](int m, f32x4* y, int row0, bool live) {
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                f32x4 v = {0.f, 0.f, 0.f, 0.f};
-                if (t >= panels) continue;
-                if constexpr (!FOLDS) {
-                    asm volatile("" : "+a"(acc[t][m]), "+a"(low[t][m]));
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = (acc[t][m][e] + low[t][m][e]) * (1.f / (SPLIT_SCALE * SPLIT_SCALE));
-                } else if (live) {
-                    v = y[4 * t];
-                }
-                if (q < 0) mend(a, row0, nt * 256 + 64 * wave + 16 * t, v);
-                if (live) y[4 * t] = v;
-            }
-        });
+    if (q < 0 && __any(odd != 0.f))
+#pragma unroll 1
+        for (int e = 0; e < 4 * MT; ++e) {
+            const int row0 = mt0 * 16 * MT + 16 * (e >> 2), t = e & 3;
+            if (row0 >= a.rows || t >= panels) continue;
+            f32x4 *y = place(e >> 2, lane) + 4 * t, v = {0.f, 0.f, 0.f, 0.f};
+            if (row0 + i < lines) v = *y;
+            mend(a, row0, nt * 256 + 64 * wave + 16 * t, v);
+            if (row0 + i < lines) *y = v;
+        }
     beg += c_end - c_beg;
     } while (beg < end);
 }

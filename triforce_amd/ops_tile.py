@@ -165,10 +165,10 @@ def interleave_glu(gate, up):
 
 def linear_rows(x, w):
     """x . W^T over many rows (prefill), w [n, k] contiguous: in 16 bits ops_rows.linear, in float32 the library GEMM, and for large products
-    split_linear.  Its tiles are 256 x 128: from 256 rows and 2^32 multiply-adds on it is the faster one (256 x 4 096 x 4 096 73 -> 61 us, 2 048 x 2 048 x 1 024
-    70 -> 63, 700 x 22 016 x 4 096 940 -> 665), below that it leaves CUs idle (300 x 6 144 x 1 536 51 -> 55, 64 x 22 016 x 4 096
-    115 -> 133), as with few results of a long k, whose parts are eight at most (2^19 results: 385 x 1 136 x 15 104 117 -> 145, 512 x 1 136
-    162 -> 150), and with k below 96 the cut and the results are all there is (1 030 x 65 536 x 64 110 -> 116).  Up to k = 65 536 its error is a
+    split_linear.  Its tiles are 256 x 128: from 256 rows and 2^32 multiply-adds on it is the faster one (256 x 4 096 x 4 096 87 -> 68 us, 2 048 x 2 048 x 1 024
+    68 -> 65, 700 x 22 016 x 4 096 917 -> 590), below that it leaves CUs idle (300 x 6 144 x 1 536 47 -> 52, 64 x 22 016 x 4 096
+    117 -> 124), as with few results of a long k, whose parts are eight at most (2^19 results: 385 x 1 136 x 15 104 117 -> 135, 512 x 1 136
+    160 -> 143), and with k below 96 the cut and the results are all there is (1 030 x 65 536 x 64 111 -> 127; of 96 151 -> 159, but 3 000 x 16 384 97 -> 93).  Up to k = 65 536 its error is a
     tenth to a half of the library's; at 2^20, with as few parts, the two are equal."""
     rows, (n, k) = x.shape[0], w.shape
     if x.dtype == w.dtype == torch.float32 and x.dim() == 2 and x.shape[1] == k and 256 <= rows <= 1 << 24 and rows * n * k >= 1 << 32 \
