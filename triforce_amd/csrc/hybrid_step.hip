@@ -8,6 +8,7 @@
 //               S = decay S + k v^T, o = S^T q.
 // step_out_kernel makes the operand of the output projection: attention merged over the splits and gated, recurrence normed and gated.
 #include "hybrid_common.h"
+#include <type_traits>
 
 template <typename T> struct StepCfg { static constexpr int PARTS = sizeof(T) == 2 ? 2 : 1; };
 
@@ -34,10 +35,13 @@ __device__ __forceinline__ Slots find_slot(const int32_t* klen, int rows, int ns
     const int p = n > 0 ? (n - 1) / TFL_PAGE + 1 - t0 : 0;
     int total = p, most = p;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        total += __shfl_xor(total, o, 64);
-        most = max(most, __shfl_xor(most, o, 64));
-    }
+    for (int o = 32; o > 0; o >>= 1)
+        if (o < rows) {                                       // (lanes from `rows` on hold zeros)
+            total += __shfl_xor(total, o, 64);
+            most = max(most, __shfl_xor(most, o, 64));
+        }
+    total = __builtin_amdgcn_readfirstlane(total);            // (one number for the wave, and known to be: see attn_part_sized)
+    most = __builtin_amdgcn_readfirstlane(most);
     const int slots = rows * nsplit, least = max(1, (most + 255) / 256);                     // (the merge weighs 256 slots of a row)
     // sum of ceil(p / q) <= total / q + rows: this q always fits, a smaller one often does
     const int fits = max(least, slots > rows ? (total + slots - rows - 1) / (slots - rows) : most);
@@ -47,22 +51,23 @@ __device__ __forceinline__ Slots find_slot(const int32_t* klen, int rows, int ns
         c = (p + q - 1) / q;
         upto = c;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(upto, o, 64);
-            if (lane >= o) upto += t;
-        }
-        if (q == fits || __shfl(upto, 63, 64) <= slots) break;
+        for (int o = 1; o < 64; o <<= 1)
+            if (o < rows) {
+                const int t = __shfl_up(upto, o, 64);
+                if (lane >= o) upto += t;
+            }
+        if (q == fits || __builtin_amdgcn_readlane(upto, rows - 1) <= slots) break;
         ++q;
     }
     if (info && threadIdx.x < rows) {                         // (wave 0)
         info[2 * lane] = upto - c;
         info[2 * lane + 1] = c;
     }
-    const uint64_t over = __ballot(upto > slot);
+    const uint64_t over = __ballot(lane < rows && upto > slot);
     f.row = over ? __ffsll((long long)over) - 1 : -1;
     const int at = over ? f.row : 0;
-    f.first = __shfl(upto - c, at, 64);
-    f.t0 = __shfl(t0, at, 64);
+    f.first = __builtin_amdgcn_readlane(upto - c, at);
+    f.t0 = __builtin_amdgcn_readlane(t0, at);
     f.pages = q;
     return f;
 }
@@ -218,6 +223,49 @@ __device__ __forceinline__ void attn_part(const AttnStep& a, const float* raw, i
     }
 }
 
+// head_norm_rotate() of D entries (64 or 128) in two parts, loads and arithmetic.
+template <int D> struct HeadFactors {                         // this lane's weights of the norm, and its angles
+    float w[D / 64], pw[D / 64], cs[D / 64], sn[D / 64];
+    __device__ __forceinline__ void load(const float* norm, const float* c, const float* s, int half, int lane) {
+#pragma unroll
+        for (int j = 0; j < D / 64; ++j) {
+            const int e = lane + 64 * j;
+            w[j] = norm[e];
+            pw[j] = cs[j] = sn[j] = 0.f;
+            if (half > 0) {                                   // (no tables without a rotated part)
+                const int pe = e < half ? e + half : max(e - half, 0), p = min(e < half ? e : e - half, half - 1);
+                pw[j] = norm[pe];
+                cs[j] = c[p];
+                sn[j] = s[p];
+            }
+        }
+    }
+};
+template <int D> struct HeadEntries {                         // raw entries, and those of the other half of a rotated pair
+    float v[D / 64], pv[D / 64];
+    __device__ __forceinline__ void load(const float* src, int half, int lane) {
+#pragma unroll
+        for (int j = 0; j < D / 64; ++j) {
+            const int e = lane + 64 * j;
+            v[j] = src[e];
+            pv[j] = src[e < half ? e + half : max(e - half, 0)];
+        }
+    }
+    __device__ __forceinline__ void norm_rotate(const HeadFactors<D>& f, int D_real, float eps, int half, int lane, float (&o)[D / 64]) const {
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < D / 64; ++j) ss = fmaf(v[j], v[j], ss);
+        ss = wave_sum64(ss);
+        const float inv = 1.0f / sqrtf(ss / (float)D_real + eps);
+#pragma unroll
+        for (int j = 0; j < D / 64; ++j) {
+            const int e = lane + 64 * j;
+            const float u = v[j] * inv * f.w[j], t = pv[j] * inv * f.pw[j];
+            o[j] = e < half ? u * f.cs[j] - t * f.sn[j] : e < 2 * half ? u * f.cs[j] + t * f.sn[j] : u;
+        }
+    }
+};
+
 // The same for known sizes, bfloat16: 32 * DK entries of query-key size, 16 * DV of value size.  The waves walk their own 32-key tiles
 // without a barrier: rows come from memory whole (the next tile's while this one is used), pass through a piece of LDS that only the wave
 // touches, and the result registers of a tile's two score products are the weight operand of its value products.  The waves meet once,
@@ -253,10 +301,34 @@ __device__ __forceinline__ void attn_part_sized(const AttnStep& a, const float* 
     float* ml = a.stats();
     const int32_t* tab = a.table + (int64_t)row * a.table_ld;
     const int64_t ld_c = (int64_t)a.G * (D + V);
+    int ids_from = p_beg, ids = tab[min(p_beg + lane, p_end - 1)];                       // of 64 pages
     auto rows_of = [&](int t) {
-        const int pg = tab[t * KT / TFL_PAGE];
+        const int page = t * KT / TFL_PAGE;
+        if (page >= ids_from + 64) {
+            ids_from = page;
+            ids = tab[min(page + lane, p_end - 1)];
+            asm volatile("" : "+v"(ids));                     // (waited for here: behind the branch all loads would be)
+        }
+        const int pg = __builtin_amdgcn_readlane(ids, page - ids_from);
         return (bf16*)a.cache + ((int64_t)(pg < 0 ? 0 : (pg >= a.n_pages ? (int)a.n_pages - 1 : pg)) * TFL_PAGE + t * KT % TFL_PAGE) * ld_c;
     };
+    // What the norms and the new key need is asked for first: loads return in the order that they were asked for.
+    const int p = min(n - 1, a.max_pos - 1);
+    HeadFactors<D> qw, kw;
+    HeadEntries<D> qr[4], kr;
+    qw.load(a.q_norm, a.cos + (int64_t)p * a.half, a.sin + (int64_t)p * a.half, a.half, lane);
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+        if (wave + 4 * h < nh) qr[h].load(raw + a.q_off + (h0 + wave + 4 * h) * D, a.half, lane);
+    const int t_new = (n - 1) / KT;                           // the new key's tile, and whose it is
+    const bool newest = t_new < t_end && ((t_new - t_beg) & 3) == wave;
+    float vr[V / 64] = {};
+    if (newest) {
+        kw.load(a.k_norm, a.cos + (int64_t)p * a.half, a.sin + (int64_t)p * a.half, a.half, lane);
+        kr.load(raw + a.k_off + grp * D, a.half, lane);
+#pragma unroll
+        for (int j = 0; j < V / 64; ++j) vr[j] = raw[a.v_off + grp * V + lane + 64 * j];
+    }
     u32x4 prek[NK], prev[NV];
     const uint32_t row_bytes = 2 * (uint32_t)ld_c;            // (G * (D + V) elements: a tile stays far below 2^32 bytes)
     auto fetch_k = [&](int t) {
@@ -273,21 +345,28 @@ __device__ __forceinline__ void attn_part_sized(const AttnStep& a, const float* 
         for (int j = 0; j < NV; ++j)
             prev[j] = *reinterpret_cast<const u32x4*>(base + ((uint32_t)min(lane / VP + j * (64 / VP), left) * row_bytes + 16u * (lane % VP)));
     };
+    __builtin_amdgcn_sched_barrier(0);
     if (t_beg + wave < t_end) {
         fetch_k(t_beg + wave);
         fetch_v(t_beg + wave);
     }
-    const int p = min(n - 1, a.max_pos - 1);
-    const float *cs = a.cos + (int64_t)p * a.half, *sn = a.sin + (int64_t)p * a.half;
-    for (int r = wave; r < 16; r += 4) {
-        float o[4] = {0.f, 0.f, 0.f, 0.f};
-        if (r < nh) {
-            const float* src = raw + a.q_off + (h0 + r) * D;
-            head_norm_rotate([src](int e) { return src[e]; }, D, a.D_real, a.q_norm, eps, cs, sn, a.half, lane, o);
-        }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (lane + 64 * j < D) Qs[r * LDK + lane + 64 * j] = (bf16)o[j];
+    for (int h = 0; h < 4; ++h) {
+        const int r = wave + 4 * h;
+        float o[D / 64] = {};
+        if (r < nh) qr[h].norm_rotate(qw, a.D_real, eps, a.half, lane, o);
+#pragma unroll
+        for (int j = 0; j < D / 64; ++j) Qs[r * LDK + lane + 64 * j] = (bf16)o[j];
+    }
+    bf16 k_new[D / 64] = {}, v_new[V / 64] = {};              // of the new key
+    if (newest) {
+        float o[D / 64];
+        kr.norm_rotate(kw, a.D_real, eps, a.half, lane, o);
+#pragma unroll
+        for (int j = 0; j < D / 64; ++j) k_new[j] = (bf16)o[j];
+#pragma unroll
+        for (int j = 0; j < V / 64; ++j) v_new[j] = (bf16)vr[j];
     }
     __syncthreads();
     bf16x8 qf[DK];
@@ -297,9 +376,12 @@ __device__ __forceinline__ void attn_part_sized(const AttnStep& a, const float* 
 #pragma unroll
     for (int d = 0; d < DV; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = NEG_INF, l_run = 0.f;
-    for (int t = t_beg + wave; t < t_end; t += 4) {
+    // One tile, and the next one's loads.  The last one apart: only it can hold the new key, and loads behind a condition would be waited for as if
+    // they had been left out.
+    auto step = [&](int t, auto last) __attribute__((always_inline)) {
+        constexpr bool LAST = decltype(last)::value;
         const int k0 = t * KT, fresh = n - 1 - k0;            // tile row of the new key (< KT: in this tile)
-        const bool edge = fresh < KT;
+        const bool edge = LAST && fresh < KT;
         asm("" : "+v"(lane), "+v"(g), "+v"(i));               // (opaque once per tile: hoisted addresses would take the registers)
 #pragma unroll
         for (int j = 0; j < NK; ++j) {
@@ -308,18 +390,14 @@ __device__ __forceinline__ void attn_part_sized(const AttnStep& a, const float* 
         }
         bf16* dst = edge ? rows_of(t) + (int64_t)fresh * ld_c : nullptr;
         if (edge) {
-            const float* src = raw + a.k_off + grp * D;
-            float k[4];
-            head_norm_rotate([src](int e) { return src[e]; }, D, a.D_real, a.k_norm, eps, cs, sn, a.half, lane, k);
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (lane + 64 * j < D) {
-                    Kt[fresh * LDK + lane + 64 * j] = (bf16)k[j];
-                    if (ht == 0) dst[grp * D + lane + 64 * j] = (bf16)k[j];
-                }
+            for (int j = 0; j < D / 64; ++j) {
+                Kt[fresh * LDK + lane + 64 * j] = k_new[j];
+                if (ht == 0) dst[grp * D + lane + 64 * j] = k_new[j];
+            }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");            // (one wave's LDS accesses stay in order; so must the compiler)
-        if (t + 4 < t_end) fetch_k(t + 4);
+        if constexpr (!LAST) fetch_k(t + 4);
         f32x4 s[2];
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
@@ -334,21 +412,21 @@ __device__ __forceinline__ void attn_part_sized(const AttnStep& a, const float* 
             *reinterpret_cast<u32x4*>(Vt + r * LDV + 8 * (lane % VP)) = edge && r >= fresh ? u32x4{0, 0, 0, 0} : prev[j];
         }
         if (edge) {
-            for (int e = lane; e < V; e += 64) {
-                const bf16 v = (bf16)raw[a.v_off + grp * V + e];
-                Vt[fresh * LDV + e] = v;
-                if (ht == 0) dst[a.G * D + grp * V + e] = v;
+#pragma unroll
+            for (int j = 0; j < V / 64; ++j) {
+                Vt[fresh * LDV + lane + 64 * j] = v_new[j];
+                if (ht == 0) dst[a.G * D + grp * V + lane + 64 * j] = v_new[j];
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        if (t + 4 < t_end) fetch_v(t + 4);
+        if constexpr (!LAST) fetch_v(t + 4);
         float mx = NEG_INF;
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int k = k0 + 16 * kt + 4 * g + r;
-                s[kt][r] = k < n && k >= first_key ? s[kt][r] * a.scale : NEG_INF;
+                s[kt][r] = (!LAST || k < n) && k >= first_key ? s[kt][r] * a.scale : NEG_INF;
                 mx = fmaxf(mx, s[kt][r]);
             }
         mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -381,6 +459,11 @@ __device__ __forceinline__ void attn_part_sized(const AttnStep& a, const float* 
             o[d] = El<bf16>::mma(f, lo, o[d]);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    };
+    if (t_beg + wave < t_end) {
+        int t = t_beg + wave;
+        for (; t + 4 < t_end; t += 4) step(t, std::false_type());
+        step(t, std::true_type());
     }
     l_run += __shfl_xor(l_run, 16, 64);
     l_run += __shfl_xor(l_run, 32, 64);
