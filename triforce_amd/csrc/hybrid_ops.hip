@@ -19,6 +19,22 @@ __global__ __launch_bounds__(64 * NW) void connect_kernel(const T* __restrict__ 
     __shared__ float cf[S * S + 2 * S];                      // mix | out | in
     const int row = blockIdx.x, nq = width >> 2;
     float* xr = x + (int64_t)row * streams * width;
+    const Y* yr = y ? y + (int64_t)row * ld_y : nullptr;
+    // Few rows are bound by round trips: what a thread's first quad needs is asked for together with the coefficients (8 rows of 4 x 4 096
+    // 6.0 -> 5.0 us).  More rows are bound by memory, and more
+    // streams do not fit the registers.
+    constexpr bool EARLY = NW == 16 && S <= 4;
+    f32x4 x0[S], y0 = {0.f, 0.f, 0.f, 0.f}, w0 = {0.f, 0.f, 0.f, 0.f};
+    auto streams_of = [&](f32x4 (&v)[S], int q) {
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            v[s] = s < streams ? *reinterpret_cast<const f32x4*>(xr + (int64_t)s * width + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    if (EARLY && (int)threadIdx.x < nq) {
+        if (!embed) streams_of(x0, threadIdx.x);
+        if (yr) y0 = load_quad(yr + 4 * threadIdx.x);
+        w0 = *reinterpret_cast<const f32x4*>(norm_w + 4 * threadIdx.x);
+    }
     for (int t = threadIdx.x; t < S * S; t += NT) {
         const int s = t / S, d = t - s * S;
         cf[t] = y && s < streams && d < streams ? mix[s * streams + d] : 0.f;
@@ -55,15 +71,18 @@ __global__ __launch_bounds__(64 * NW) void connect_kernel(const T* __restrict__ 
             ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
         }
     } else {
-        const Y* yr = y ? y + (int64_t)row * ld_y : nullptr;
         for (int q = threadIdx.x; q < nq; q += NT) {
+            const bool have = EARLY && q == (int)threadIdx.x;
             f32x4 v[S];
+            if (have) {
 #pragma unroll
-            for (int s = 0; s < S; ++s)
-                v[s] = s < streams ? *reinterpret_cast<const f32x4*>(xr + (int64_t)s * width + 4 * q) : f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int s = 0; s < S; ++s) v[s] = x0[s];
+            } else {
+                streams_of(v, q);
+            }
             f32x4 u = {0.f, 0.f, 0.f, 0.f};
             if (yr) {
-                const f32x4 z = load_quad(yr + 4 * q);
+                const f32x4 z = have ? y0 : load_quad(yr + 4 * q);
 #pragma unroll
                 for (int t = 0; t < S; ++t) {
                     const float o = cf[S * S + t], g = cf[S * S + S + t];
@@ -96,7 +115,7 @@ __global__ __launch_bounds__(64 * NW) void connect_kernel(const T* __restrict__ 
     const float inv = 1.0f / sqrtf(ss / (float)width_real + eps);
     for (int q = threadIdx.x; q < nq; q += NT) {              // (each thread reads back what it wrote itself)
         f32x4 u = *reinterpret_cast<const f32x4*>(us + 4 * q);
-        const f32x4 w = *reinterpret_cast<const f32x4*>(norm_w + 4 * q);
+        const f32x4 w = EARLY && q == (int)threadIdx.x ? w0 : *reinterpret_cast<const f32x4*>(norm_w + 4 * q);
 #pragma unroll
         for (int r = 0; r < 4; ++r) u[r] = u[r] * inv * w[r];
         store_quad(h + (int64_t)row * ld_h + (q >> 1) * h_oct + 4 * (q & 1), u);

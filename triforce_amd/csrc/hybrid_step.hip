@@ -651,11 +651,19 @@ __global__ __launch_bounds__(256) void step_out_kernel(const AttnStep a, const T
     T* dst = act + (int64_t)row * ld_act;
     if ((int)blockIdx.x < attn_blocks) {                      // one head: splits merged, output gate
         const bool dealt = gridDim.y > 1 && gridDim.y <= 64;
-        const int head = blockIdx.x, V = a.V, first = dealt ? a.info()[2 * row] : row * a.nsplit, ns = dealt ? a.info()[2 * row + 1] : a.nsplit;
+        const int head = blockIdx.x, V = a.V, first = dealt ? min(a.info()[2 * row], a.slots - 1) : row * a.nsplit, ns = dealt ? a.info()[2 * row + 1] : a.nsplit;
         const int64_t at = (int64_t)first * a.H + head;        // + s * H: slot s of the row
         const float* ml = a.stats() + 2 * at;
-        const float ls = tid < ns ? ml[2 * (int64_t)tid * a.H + 1] : 0.f;
-        const float ms = ls > 0.f ? ml[2 * (int64_t)tid * a.H] : NEG_INF;
+        const int nq = V >> 2, ng = 256 / nq, vq = tid % nq, gr = tid / nq, c = head * V + 4 * vq;
+        // Bound by round trips: gate and first partial rows are asked for together with the statistics, whose two halves come at once.
+        constexpr int U = 2;
+        f32x4 z0[U], zg = {0.f, 0.f, 0.f, 0.f};
+        const int last = max(ns, 1) - 1;
+#pragma unroll
+        for (int u = 0; u < U; ++u) z0[u] = *reinterpret_cast<const f32x4*>(a.ws + (at + (int64_t)min(gr + u * ng, last) * a.H) * V + 4 * vq);
+        if (gr == 0) zg = *reinterpret_cast<const f32x4*>(rr + a.gate_off + c);
+        const float m_have = ml[2 * (int64_t)min(tid, last) * a.H], l_have = ml[2 * (int64_t)min(tid, last) * a.H + 1];
+        const float ls = tid < ns ? l_have : 0.f, ms = ls > 0.f ? m_have : NEG_INF;
         float m = ms;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
@@ -666,10 +674,18 @@ __global__ __launch_bounds__(256) void step_out_kernel(const AttnStep a, const T
         const float l = block_sum<4>(w * ls, red);
         wgt[tid] = l > 0.f ? w / l : 0.f;
         __syncthreads();
-        const int nq = V >> 2, ng = 256 / nq, vq = tid % nq, gr = tid / nq;
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         if (gr < ng) {
-            for (int s = gr; s < ns; s += ng) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int s = gr + u * ng;
+                const float f = s < ns ? wgt[s] : 0.f;
+                if (f > 0.f) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = fmaf(z0[u][e], f, v[e]);
+                }
+            }
+            for (int s = gr + U * ng; s < ns; s += ng) {
                 const float f = wgt[s];
                 if (f > 0.f) {                                // (an empty split's partial row was never written)
                     const f32x4 z = *reinterpret_cast<const f32x4*>(a.ws + (at + (int64_t)s * a.H) * V + 4 * vq);
@@ -686,10 +702,8 @@ __global__ __launch_bounds__(256) void step_out_kernel(const AttnStep a, const T
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] += z[e];
             }
-            const int c = head * V + 4 * vq;
-            const f32x4 z = *reinterpret_cast<const f32x4*>(rr + a.gate_off + c);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] *= sigmoid_of<T>(z[e]) * a.out_scale;
+            for (int e = 0; e < 4; ++e) v[e] *= sigmoid_of<T>(zg[e]) * a.out_scale;
             store_quad(dst + (c >> 3) * act_oct + (c & 7), v);
         }
         return;
@@ -701,11 +715,21 @@ __global__ __launch_bounds__(256) void step_out_kernel(const AttnStep a, const T
     float ss = 0.f;
     if (r.V == r.V_real && !(size & 3)) {                     // no padding inside a row: quads, the first HOLD of a thread stay in registers
         constexpr int HOLD = 4;
-        f32x4 held[HOLD];
+        f32x4 held[HOLD], wt[HOLD], gt[HOLD];
+        auto weights = [&](int c) { return *reinterpret_cast<const f32x4*>(r.norm_w + (per_channel ? c : first + c)); };
+        auto gates = [&](int c) { return *reinterpret_cast<const f32x4*>(rr + r.gate_off + first + c); };
 #pragma unroll
         for (int u = 0; u < HOLD; ++u) {
             const int c = 4 * (tid + 256 * u);
-            held[u] = c < size ? *reinterpret_cast<const f32x4*>(src + first + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+            held[u] = wt[u] = gt[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (c < size) {
+                held[u] = *reinterpret_cast<const f32x4*>(src + first + c);
+                wt[u] = weights(c);
+                if (per_channel) gt[u] = gates(c);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < HOLD; ++u) {
             ss += held[u][0] * held[u][0] + held[u][1] * held[u][1] + held[u][2] * held[u][2] + held[u][3] * held[u][3];
         }
         for (int c = 4 * (tid + 256 * HOLD); c < size; c += 1024) {
@@ -714,12 +738,10 @@ __global__ __launch_bounds__(256) void step_out_kernel(const AttnStep a, const T
         }
         ss = block_sum<4>(ss, red);
         const float inv = r.out_scale / sqrtf(ss / (float)size + eps);
-        auto put = [&](int c, f32x4 v) {
-            const f32x4 w = *reinterpret_cast<const f32x4*>(r.norm_w + (per_channel ? c : first + c));
+        auto put = [&](int c, f32x4 v, f32x4 w, f32x4 z) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = v[e] * inv * w[e];
             if (per_channel) {
-                const f32x4 z = *reinterpret_cast<const f32x4*>(rr + r.gate_off + first + c);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] *= silu_of<T>(z[e]);
             }
@@ -728,8 +750,9 @@ __global__ __launch_bounds__(256) void step_out_kernel(const AttnStep a, const T
         };
 #pragma unroll
         for (int u = 0; u < HOLD; ++u)
-            if (4 * (tid + 256 * u) < size) put(4 * (tid + 256 * u), held[u]);
-        for (int c = 4 * (tid + 256 * HOLD); c < size; c += 1024) put(c, *reinterpret_cast<const f32x4*>(src + first + c));
+            if (4 * (tid + 256 * u) < size) put(4 * (tid + 256 * u), held[u], wt[u], gt[u]);
+        for (int c = 4 * (tid + 256 * HOLD); c < size; c += 1024)
+            put(c, *reinterpret_cast<const f32x4*>(src + first + c), weights(c), per_channel ? gates(c) : f32x4{0.f, 0.f, 0.f, 0.f});
         return;
     }
     for (int c = tid; c < size; c += 256) {

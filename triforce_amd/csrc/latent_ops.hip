@@ -80,6 +80,13 @@ __global__ __launch_bounds__(64 * NW) void finish_row_kernel(const T* __restrict
     }
     const Y* yr = y ? y + (int64_t)row * ld_y : nullptr;
     f32x4 v[HOLD], z[HOLD], w[HOLD];
+    // one quad a thread (few rows): nothing is left to be asked for behind a sum
+    constexpr bool EARLY = HOLD == 1;
+    f32x4 t0 = {0.f, 0.f, 0.f, 0.f}, n0 = {0.f, 0.f, 0.f, 0.f};
+    if (EARLY && (int)threadIdx.x < nq) {
+        if (step) t0 = *reinterpret_cast<const f32x4*>(step + 4 * threadIdx.x);
+        n0 = *reinterpret_cast<const f32x4*>(norm_w + 4 * threadIdx.x);
+    }
     float s = 0.f;
 #pragma unroll
     for (int j = 0; j < HOLD; ++j) {
@@ -108,12 +115,12 @@ __global__ __launch_bounds__(64 * NW) void finish_row_kernel(const T* __restrict
         }
         if (q < nq) {
             if (step) {
-                const f32x4 t = *reinterpret_cast<const f32x4*>(step + 4 * q);
+                const f32x4 t = EARLY ? t0 : *reinterpret_cast<const f32x4*>(step + 4 * q);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) v[j][r] += t[r];
             }
             if (er || yr || step) *reinterpret_cast<f32x4*>(xr + 4 * q) = v[j];
-            w[j] = *reinterpret_cast<const f32x4*>(norm_w + 4 * q);
+            w[j] = EARLY ? n0 : *reinterpret_cast<const f32x4*>(norm_w + 4 * q);
         }
         s += v[j][0] * v[j][0] + v[j][1] * v[j][1] + v[j][2] * v[j][2] + v[j][3] * v[j][3];
     }
