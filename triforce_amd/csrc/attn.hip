@@ -471,8 +471,7 @@ __device__ __forceinline__ void attn_split_body(
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         float lsum = st.l[qt];
-        lsum += __shfl_xor(lsum, 16, 64);
-        lsum += __shfl_xor(lsum, 32, 64);
+        lsum = rows_sum(lsum);
 #pragma unroll
         for (int hv = 0; hv < HALVES; ++hv) {
 #pragma unroll
@@ -911,8 +910,7 @@ __global__ __launch_bounds__(256, TF_BLOCK_OCC) void attn_block_kernel(
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         float lsum = st.l[qt];
-        lsum += __shfl_xor(lsum, 16, 64);
-        lsum += __shfl_xor(lsum, 32, 64);
+        lsum = rows_sum(lsum);
         const int64_t row = pbase + qbase + qt * 16 + li;      // lane holds O[q = li][d = 16t + 4g + r]
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) *reinterpret_cast<f32x4*>(ws_o + row * D + 16 * tt + 4 * g) = st.acc[qt][tt];
@@ -1385,8 +1383,7 @@ __device__ __forceinline__ void attn_block_lds_body(
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         float lsum = st.l[qt];
-        lsum += __shfl_xor(lsum, 16, 64);
-        lsum += __shfl_xor(lsum, 32, 64);
+        lsum = rows_sum(lsum);
         const int64_t row = pbase + qbase + qt * 16 + li;
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) *reinterpret_cast<f32x4*>(ws_o + row * D + 16 * tt + 4 * g) = st.acc[qt][tt];
@@ -1674,8 +1671,7 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
             float lsum = st.l[qt];
-            lsum += __shfl_xor(lsum, 16, 64);
-            lsum += __shfl_xor(lsum, 32, 64);
+            lsum = rows_sum(lsum);
             const float inv = 1.0f / lsum;
             const int row = qbase + qt * 16 + li;
             if (row >= sq) continue;
@@ -1697,8 +1693,7 @@ __device__ __forceinline__ void attn_prefill_ahead_body(
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
         float lsum = st.l[qt];
-        lsum += __shfl_xor(lsum, 16, 64);
-        lsum += __shfl_xor(lsum, 32, 64);
+        lsum = rows_sum(lsum);
         const int64_t row = pbase + qbase + qt * 16 + li;
 #pragma unroll
         for (int tt = 0; tt < NT; ++tt) *reinterpret_cast<f32x4*>(ws_o + row * D + 16 * tt + 4 * g) = st.acc[qt][tt];

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "../../include/triforce_hip.h"
+#include "lanes.h"
 
 typedef _Float16 h16;
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -18,14 +19,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
     } while (0)
 
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return lanes_sum(v);
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    return lanes_max(v);
 }
 
 // fp16 product / sum with torch's half semantics: compute in fp32, round once to fp16.

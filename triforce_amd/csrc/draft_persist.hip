@@ -273,8 +273,7 @@ __device__ __forceinline__ bool dp_role_qkv(DpCtx& c, int l, float* sm, float* r
                 const float f = (float)b[u][e];
                 ss = fmaf(f, f, ss);
             }
-        ss += __shfl_xor(ss, 16, 64);
-        ss += __shfl_xor(ss, 32, 64);
+        ss = rows_sum(ss);
         if (g == 0) sm_ss[wave * 16 + li] = ss;
         __syncthreads();
         float tot = 0.f;
@@ -311,7 +310,7 @@ __device__ __forceinline__ bool dp_role_qkv(DpCtx& c, int l, float* sm, float* r
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             val[r] = (h16)S[r];
-            oth[r] = (h16)__shfl_xor((float)val[r], 32, 64);             // rotary partner: lane g <-> g ^ 2 (exact)
+            oth[r] = (h16)other_half((float)val[r]);             // rotary partner: lane g <-> g ^ 2 (exact)
         }
         if (rowv) {
             const int slot = P.slot0 + li;
@@ -397,8 +396,7 @@ __device__ __forceinline__ bool dp_role_plain(DpCtx& c, const half8* wp, const h
         }
         if (rowv) st_half4(P.x + (int64_t)li * HID + y_off, o);
         float qq = s2[0] * s2[0] + s2[1] * s2[1] + s2[2] * s2[2] + s2[3] * s2[3];
-        qq += __shfl_xor(qq, 16, 64);
-        qq += __shfl_xor(qq, 32, 64);
+        qq = rows_sum(qq);
         if (g == 0) st4f(P.ss + panel * 32 + li, qq);
         dp_arrive(c, edge_out, OD_LO, OD_HI, false);
     }

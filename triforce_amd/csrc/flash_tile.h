@@ -166,8 +166,7 @@ template <int KR, int NWV> struct FlashTile {
                 float mx = s[0][u][0];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) mx = fmaxf(fmaxf(fmaxf(mx, s[0][u][r]), fmaxf(s[1][u][r], s[2][u][r])), s[3][u][r]);
-                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                mx = rows_max(mx);
                 top[u] = fmaxf(m[u], mx * sc);
                 if (__builtin_amdgcn_ballot_w64(top[u] != m[u])) {                       // (most tiles leave every maximum where it was)
                     const float alpha = __builtin_amdgcn_exp2f(m[u] - top[u]);
@@ -207,8 +206,7 @@ template <int KR, int NWV> struct FlashTile {
     // Sum of the weights of query u (over the four lanes that hold its keys).
     __device__ __forceinline__ float weight(int u) const {
         float s = l[u];
-        s += __shfl_xor(s, 16, 64);
-        s += __shfl_xor(s, 32, 64);
+        s = rows_sum(s);
         return s;
     }
 };

@@ -490,8 +490,7 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(const half8* __
             }
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                ss[t] += __shfl_xor(ss[t], 16, 64);
-                ss[t] += __shfl_xor(ss[t], 32, 64);
+                ss[t] = rows_sum(ss[t]);
                 if (g == 0) sm_ss[wave][t][li] = ss[t];
             }
             __syncthreads();
@@ -817,7 +816,7 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(const half8* __
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 val[r] = (h16)s[r];
-                oth[r] = (h16)__shfl_xor((float)val[r], 32, 64);         // rotary partner: lane g <-> g ^ 2 (exact)
+                oth[r] = (h16)other_half((float)val[r]);         // rotary partner: lane g <-> g ^ 2 (exact)
             }
             if (m >= M) continue;
             const int slot = (rp.slot0_dev ? *rp.slot0_dev : rp.slot0) + m;
@@ -888,8 +887,7 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_kernel(const half8* __
         }
         if (MODE == SG_PLAIN && ss_out) {            // this panel's share of sum(y^2) per row, for the next norm prologue
             float q = s2[0] * s2[0] + s2[1] * s2[1] + s2[2] * s2[2] + s2[3] * s2[3];
-            q += __shfl_xor(q, 16, 64);
-            q += __shfl_xor(q, 32, 64);
+            q = rows_sum(q);
             if (g == 0) ss_out[(int64_t)panel * 32 + m] = q;
         }
     }
@@ -1069,8 +1067,7 @@ __global__ __launch_bounds__(WAVES * 64) void skinny_gemm_n8_kernel(const half8*
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
                 ss[t] += __shfl_xor(ss[t], 8, 64);              // the two stacked chunks
-                ss[t] += __shfl_xor(ss[t], 16, 64);             // the four k-octets
-                ss[t] += __shfl_xor(ss[t], 32, 64);
+                ss[t] = rows_sum(ss[t]);
                 if (lane < 8) sm_ss[wave][t * 8 + lane] = ss[t];
             }
             __syncthreads();

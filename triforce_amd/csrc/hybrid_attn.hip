@@ -163,8 +163,7 @@ __global__ __launch_bounds__(256, 1) void attn_chunk_kernel(const T* __restrict_
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows_max(mx);
         mx = fmaxf(m_run, mx * scale);
         // a row may have seen no key yet (its chunk starts in a later tile): its maximum is -inf, every weight 0
         const float ref = mx == NEG_INF ? 0.f : mx;
@@ -200,8 +199,7 @@ __global__ __launch_bounds__(256, 1) void attn_chunk_kernel(const T* __restrict_
     }
     const int j = qb + 16 * wave + i;
     float l = l_run;
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = rows_sum(l);
     if (j >= nq) return;
     const float inv = out_scale / l;
     const int64_t tok = q_at + j;

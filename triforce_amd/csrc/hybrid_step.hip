@@ -34,14 +34,8 @@ __device__ __forceinline__ Slots find_slot(const int32_t* klen, int rows, int ns
     const int n = lane < rows ? klen[lane] : 0, t0 = first_visible(n, chunk) / TFL_PAGE;
     const int p = n > 0 ? (n - 1) / TFL_PAGE + 1 - t0 : 0;
     int total = p, most = p;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        if (o < rows) {                                       // (lanes from `rows` on hold zeros)
-            total += __shfl_xor(total, o, 64);
-            most = max(most, __shfl_xor(most, o, 64));
-        }
-    total = __builtin_amdgcn_readfirstlane(total);            // (one number for the wave, and known to be: see attn_part_sized)
-    most = __builtin_amdgcn_readfirstlane(most);
+    total = __builtin_amdgcn_readfirstlane(lanes_sum(total));                            // (one number for the wave, and known to be: see attn_part_sized)
+    most = __builtin_amdgcn_readfirstlane(lanes_max(most));
     const int slots = rows * nsplit, least = max(1, (most + 255) / 256);                     // (the merge weighs 256 slots of a row)
     // sum of ceil(p / q) <= total / q + rows: this q always fits, a smaller one often does
     const int fits = max(least, slots > rows ? (total + slots - rows - 1) / (slots - rows) : most);
@@ -162,8 +156,7 @@ __device__ __forceinline__ void attn_part(const AttnStep& a, const float* raw, i
             s[r] = k < n && k >= first_key ? s[r] * a.scale : NEG_INF;
             mx = fmaxf(mx, s[r]);
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows_max(mx);
         if (g == 0) red[wave * 16 + i] = mx;
         __syncthreads();
         mx = m_run;
@@ -205,8 +198,7 @@ __device__ __forceinline__ void attn_part(const AttnStep& a, const float* raw, i
         }
         __syncthreads();
     }
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = rows_sum(l_run);
     if (g == 0) red[wave * 16 + i] = l_run;
     __syncthreads();
     if (i < nh) {
@@ -429,8 +421,7 @@ __device__ __forceinline__ void attn_part_sized(const AttnStep& a, const float* 
                 s[kt][r] = (!LAST || k < n) && k >= first_key ? s[kt][r] * a.scale : NEG_INF;
                 mx = fmaxf(mx, s[kt][r]);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows_max(mx);
         mx = fmaxf(m_run, mx);                                // (every tile has a visible key: finite)
         const float alpha = __builtin_amdgcn_exp2f((m_run - mx) * LOG2E);
         m_run = mx;
@@ -465,8 +456,7 @@ __device__ __forceinline__ void attn_part_sized(const AttnStep& a, const float* 
         for (; t + 4 < t_end; t += 4) step(t, std::false_type());
         step(t, std::true_type());
     }
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
+    l_run = rows_sum(l_run);
     if (g == 0) {
         red[wave * 16 + i] = m_run;
         red[64 + wave * 16 + i] = l_run;
@@ -665,8 +655,7 @@ __global__ __launch_bounds__(256) void step_out_kernel(const AttnStep a, const T
         const float m_have = ml[2 * (int64_t)min(tid, last) * a.H], l_have = ml[2 * (int64_t)min(tid, last) * a.H + 1];
         const float ls = tid < ns ? l_have : 0.f, ms = ls > 0.f ? m_have : NEG_INF;
         float m = ms;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+        m = lanes_max(m);
         if ((tid & 63) == 0) red[4 + (tid >> 6)] = m;
         __syncthreads();
         m = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));

@@ -94,8 +94,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_latent_kernel(const T* __rest
                 s[h][r] = k0 + 16 * wave + 4 * g + r < n ? s[h][r] * scale : NEG_INF;
                 mx = fmaxf(mx, s[h][r]);
             }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            mx = rows_max(mx);
             if (g == 0) red[wave * 16 * HT + 16 * h + i] = mx;
         }
         __syncthreads();
@@ -152,8 +151,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_latent_kernel(const T* __rest
 #pragma unroll
     for (int h = 0; h < HT; ++h) {
         float l = l_run[h];
-        l += __shfl_xor(l, 16, 64);
-        l += __shfl_xor(l, 32, 64);
+        l = rows_sum(l);
         if (g == 0) red[wave * 16 * HT + 16 * h + i] = l;
     }
     __syncthreads();
@@ -215,8 +213,7 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(const float* __restri
     const float m_have = ml[2 * min(tid, nsplit - 1)], l_have = ml[2 * min(tid, nsplit - 1) + 1];
     const float ls = tid < nsplit ? l_have : 0.f, ms = ls > 0.f ? m_have : NEG_INF;
     float m = ms;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+    m = lanes_max(m);
     if ((tid & 63) == 0) red[4 + (tid >> 6)] = m;
     __syncthreads();
     m = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
@@ -283,8 +280,7 @@ __global__ __launch_bounds__(256) void latent_merge_waves_kernel(const float* __
         for (int u = 0; u < U; ++u) z[u] = *reinterpret_cast<const f32x2*>(src + (int64_t)min(s0 + u, nsplit - 1) * C);
         if (s0 == 0) {                                        // (the statistics arrive under the first partial rows)
             float m = ms;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+            m = lanes_max(m);
             w = ls > 0.f ? exp2f((ms - m) * LOG2E) : 0.f;
             const float l = wave_sum64(w * ls);
             w = l > 0.f ? w / l : 0.f;
@@ -415,8 +411,7 @@ __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ 
         };
         auto largest = [&] {                                  // of these 16 keys, into red
             float x = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-            x = fmaxf(x, __shfl_xor(x, 16, 64));
-            x = fmaxf(x, __shfl_xor(x, 32, 64));
+            x = rows_max(x);
             if (g == 0) red[Z::H * ks + head] = x;
         };
         auto weights = [&](int j) {
@@ -466,8 +461,7 @@ __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ 
             }
             meet<LOADS>();
         }
-        l += __shfl_xor(l, 16, 64);
-        l += __shfl_xor(l, 32, 64);
+        l = rows_sum(l);
         if (g == 0) red[Z::H * ks + head] = l;
         meet<0>();                                            // (no load is under way when the LDS is given back)
         if (writes) {
@@ -834,15 +828,13 @@ __global__ __launch_bounds__(512) void latent_value_kernel(const float* __restri
             m[h] = l[h] > 0.f ? ml[2 * s] : NEG_INF;          // (an empty split: its partial row is not read either)
         }
         float most = fmaxf(m[0], m[1]), all = 0.f;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) most = fmaxf(most, __shfl_xor(most, o, 64));
+        most = lanes_max(most);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             m[h] = l[h] > 0.f ? exp2f((m[h] - most) * LOG2E) : 0.f;
             all += m[h] * l[h];
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) all += __shfl_xor(all, o, 64);
+        all = lanes_sum(all);
 #pragma unroll
         for (int h = 0; h < 2; ++h) weight[wave][lane + 64 * h] = all > 0.f ? m[h] / all : 0.f;
         const uint64_t low = __builtin_amdgcn_ballot_w64(l[0] > 0.f), high = __builtin_amdgcn_ballot_w64(l[1] > 0.f);
@@ -1011,8 +1003,7 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(const T* __restric
         for (int kt = 0; kt < KT / 16; ++kt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) mx = fmaxf(mx, s[kt][r]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows_max(mx);
         mx = fmaxf(m_run, mx * scale);                        // (scale > 0; key 0 is visible to every row: finite from tile 0 on)
         const float alpha = __builtin_amdgcn_exp2f((m_run - mx) * LOG2E), sc = scale * LOG2E, mb = mx * LOG2E;
         m_run = mx;
@@ -1045,8 +1036,7 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_kernel(const T* __restric
         __syncthreads();
     }
     float l = l_run;
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = rows_sum(l);
     if (j >= nq) return;
     const float inv = 1.0f / l;
 #pragma unroll

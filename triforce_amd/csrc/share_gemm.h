@@ -32,8 +32,7 @@ __device__ __forceinline__ void finish_quad(const TflGemm& a, int m, int n, f32x
 template <typename T>
 __device__ __forceinline__ void finish_raw(const TflGemm& a, int m, bool live, int pin, int n, int g, f32x4 s) {
     float q = s[0] * s[0] + s[1] * s[1] + s[2] * s[2] + s[3] * s[3];
-    q += __shfl_xor(q, 16, 64);
-    q += __shfl_xor(q, 32, 64);
+    q = rows_sum(q);
     if (!live) return;
     *reinterpret_cast<f32x4*>(a.out_f + (int64_t)m * a.ld_f + n) = s;
     if (n < a.n_scaled) {
@@ -141,7 +140,7 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
             if constexpr (EPI == TFL_EPI_GLU) {              // lanes g < 2 hold gate rows, g + 2 the same outputs' up rows
                 f32x4 up;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(s[r], 32, 64);
+                for (int r = 0; r < 4; ++r) up[r] = other_half(s[r]);
                 if (live && g < 2) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) s[r] = gelu_tanh(s[r]) * up[r];

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "../../include/triforce_tile.h"
+#include "lanes.h"
 
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -93,9 +94,7 @@ template <typename T> __device__ __forceinline__ float gelu_of(float z) {
 __device__ __forceinline__ float sigmoid(float z) { return 1.0f / (1.0f + expf(-z)); }
 
 __device__ __forceinline__ float wave_sum64(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return lanes_sum(v);
 }
 // Sum over a workgroup of NW waves; red = NW floats of LDS, free again after the call's second barrier.
 template <int NW> __device__ __forceinline__ float block_sum(float v, float* red) {

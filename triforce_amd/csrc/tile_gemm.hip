@@ -131,8 +131,7 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
                 const float2 v = ss[p];
                 q += v.x + v.y;
             }
-            q += __shfl_xor(q, 16, 64);
-            q += __shfl_xor(q, 32, 64);
+            q = rows_sum(q);
             inv = 1.0f / sqrtf(q / (float)a.k_real + a.eps);
         }
     }
@@ -153,8 +152,7 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
     if constexpr (EPI == TFL_EPI_IN) {
         if (16 * pin < a.n_raw) {
             float q = s[0] * s[0] + s[1] * s[1] + s[2] * s[2] + s[3] * s[3];
-            q += __shfl_xor(q, 16, 64);
-            q += __shfl_xor(q, 32, 64);
+            q = rows_sum(q);
             if (live) {
                 *reinterpret_cast<f32x4*>(a.out_f + (int64_t)m * a.ld_f + n) = s;
                 if (n < a.n_scaled) {
@@ -176,7 +174,7 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
     if constexpr (EPI == TFL_EPI_GLU) {                      // lanes g < 2 hold gate rows, g + 2 the same outputs' up rows
         f32x4 up;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) up[r] = __shfl_xor(s[r], 32, 64);
+        for (int r = 0; r < 4; ++r) up[r] = other_half(s[r]);
         if (live && g < 2) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) s[r] = gelu_tanh(s[r]) * up[r];
