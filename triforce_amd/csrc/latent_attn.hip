@@ -597,24 +597,21 @@ __global__ __launch_bounds__(512, 2) void attn_latent_beside_kernel(const bf16* 
     }
     const int lane = threadIdx.x & 63;
     const int pages = lane < rows ? max(1, (len[min(lane, rows - 1)] + 63) >> 6) : 0;        // (a row without keys has one empty split)
-    int total = pages, most = pages;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        total += __shfl_xor(total, o, 64);
-        most = max(most, __shfl_xor(most, o, 64));
-    }
+    const int total = lanes_sum(pages), most = lanes_max(pages);
     int per = max((total + workers - 1) / workers, most > 16 ? 2 : 1), mine, end;
     for (;; ++per) {                                          // (with `most` pages a split there are as many splits as rows)
         mine = lane < rows ? min(nsplit, (pages + per - 1) / per) : 0;
         end = mine;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int v = __shfl_up(end, o, 64);
-            if (lane >= o) end += v;
-        }
-        if (per >= most || __shfl(end, 63, 64) <= workers) break;
+        for (int o = 1; o < 64; o <<= 1)
+            if (o < rows) {                                   // (lanes from `rows` on are not looked at)
+                const int v = __shfl_up(end, o, 64);
+                if (lane >= o) end += v;
+            }
+        if (per >= most || __builtin_amdgcn_readlane(end, rows - 1) <= workers) break;
     }
-    const int row = __popcll(__builtin_amdgcn_ballot_w64(end <= me));            // (lanes past the rows end where the last row does)
+    const uint64_t before = __builtin_amdgcn_ballot_w64(lane < rows && end <= me);
+    const int row = __popcll(before);
     if (row >= rows) return;
     const int have = __builtin_amdgcn_readlane(mine, row), split = me - (__builtin_amdgcn_readlane(end, row) - have), n = len[row];
     const int ntiles = n > 0 ? (n + 63) >> 6 : 0, each = (ntiles + have - 1) / have;
@@ -824,8 +821,9 @@ __global__ __launch_bounds__(512) void latent_value_kernel(const float* __restri
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int s = lane + 64 * h;
-            l[h] = s < nsplit ? ml[2 * s + 1] : 0.f;
-            m[h] = l[h] > 0.f ? ml[2 * s] : NEG_INF;          // (an empty split: its partial row is not read either)
+            const float m_have = ml[2 * min(s, nsplit - 1)], l_have = ml[2 * min(s, nsplit - 1) + 1];         // (both at once)
+            l[h] = s < nsplit ? l_have : 0.f;
+            m[h] = l[h] > 0.f ? m_have : NEG_INF;             // (an empty split: its partial row is not read either)
         }
         float most = fmaxf(m[0], m[1]), all = 0.f;
         most = lanes_max(most);

@@ -5,19 +5,19 @@
 
 // What one lane does with four finished outputs n .. n+3 of batch row m (`s`); panel-wide parts (sums of squares, gate | up pairs) are
 // its caller's.
+// old: RESIDUAL's fp32 residual there.
 template <typename T, int EPI>
-__device__ __forceinline__ void finish_quad(const TflGemm& a, int m, int n, f32x4 s) {
+__device__ __forceinline__ void finish_quad(const TflGemm& a, int m, int n, f32x4 s, f32x4 old) {
     if constexpr (EPI == TFL_EPI_F32) {
         float* y = a.out_f + (int64_t)m * a.ld_f + n;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             if (n + r < a.n_real) y[r] = s[r];
     } else if constexpr (EPI == TFL_EPI_RESIDUAL) {
-        f32x4* y = reinterpret_cast<f32x4*>(a.out_f + (int64_t)m * a.ld_f + n);
-        f32x4 o = *y;
+        f32x4 o = old;
 #pragma unroll
         for (int r = 0; r < 4; ++r) o[r] += s[r];
-        *y = o;
+        *reinterpret_cast<f32x4*>(a.out_f + (int64_t)m * a.ld_f + n) = o;
         if (a.out_t) store_quad((T*)a.out_t + (int64_t)m * a.ld_t + (n >> 3) * a.t_oct + (n & 7), o);
     } else {                                                 // IN behind its raw part
         static_assert(EPI == TFL_EPI_IN, "quad epilogues");
@@ -28,15 +28,14 @@ __device__ __forceinline__ void finish_quad(const TflGemm& a, int m, int n, f32x
     }
 }
 
-// IN's raw part: outputs n .. n+3 of a panel that all lanes of the wave hold (g = quad of the panel, i = row).
+// IN's raw part: outputs n .. n+3 of a panel that all lanes of the wave hold (g = quad of the panel, i = row); w: their norm weights.
 template <typename T>
-__device__ __forceinline__ void finish_raw(const TflGemm& a, int m, bool live, int pin, int n, int g, f32x4 s) {
+__device__ __forceinline__ void finish_raw(const TflGemm& a, int m, bool live, int pin, int n, int g, f32x4 s, f32x4 w) {
     float q = s[0] * s[0] + s[1] * s[1] + s[2] * s[2] + s[3] * s[3];
     q = rows_sum(q);
     if (!live) return;
     *reinterpret_cast<f32x4*>(a.out_f + (int64_t)m * a.ld_f + n) = s;
     if (n < a.n_scaled) {
-        const f32x4 w = *reinterpret_cast<const f32x4*>(a.norm_w + n);
 #pragma unroll
         for (int r = 0; r < 4; ++r) s[r] *= w[r];
         store_quad((T*)a.out_t2 + (int64_t)m * 8 + (n >> 3) * (8 * (int64_t)a.rows) + (n & 7), s);
@@ -108,6 +107,26 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
                     for (int t = 0; t < MT; ++t) acc[p][t] = El<T>::mma(w[u][p], x[u][t], acc[p][t]);
             }
     };
+    // What the epilogue of result tile j (row block t of panel or left-over tile p) reads: of a wave's first one asked for in front of the weights,
+    // not behind the products, where nothing is left to hide it (4 096 x 4 096 onto the residual, 1 / 32 rows: 7.90 -> 7.43 us, 11.83 -> 11.34).
+    auto beside = [&](int j) {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (EPI == TFL_EPI_RESIDUAL || EPI == TFL_EPI_IN) {
+            const int p = j / MT, m = m0 + 16 * (j - p * MT) + i, row = cu * tail_per + 4 * g;
+            const bool whole = !TAIL || p < P;
+            const int n = whole ? 16 * (panel0 + p) + 4 * g : 16 * CUS * P + row;
+            if (j < NP * MT && (whole ? panel0 + p < npan : 4 * g < tail_per && row < tail_rows)) {
+                if constexpr (EPI == TFL_EPI_IN) {
+                    if (whole && n < a.n_scaled) v = *reinterpret_cast<const f32x4*>(a.norm_w + n);
+                } else {
+                    v = *reinterpret_cast<const f32x4*>(a.out_f + (int64_t)min(m, a.rows - 1) * a.ld_f + n);
+                }
+            }
+        }
+        return v;
+    };
+    const f32x4 first = beside(wave);
+    asm volatile("" ::: "memory");
     if (n_own > 0) {
         Frag wa[U][NP], xa[U][MT], wb[U][NP], xb[U][MT];
         load(wa, xa, 0);
@@ -134,6 +153,7 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
             for (int r = 0; r < 4; ++r) s[r] += o[r];
         }
         const bool live = m < a.rows;
+        const f32x4 with = j == wave ? first : beside(j);
         if (!TAIL || p < P) {
             const int panel = panel0 + p, n = 16 * panel + 4 * g;
             if (panel >= npan) continue;
@@ -149,11 +169,11 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
             } else {
                 if constexpr (EPI == TFL_EPI_IN) {
                     if (16 * panel < a.n_raw) {
-                        finish_raw<T>(a, m, live, panel, n, g, s);
+                        finish_raw<T>(a, m, live, panel, n, g, s, with);
                         continue;
                     }
                 }
-                if (live) finish_quad<T, EPI>(a, m, n, s);
+                if (live) finish_quad<T, EPI>(a, m, n, s, with);
             }
         } else {
             const int row = cu * tail_per + 4 * g;   // first of this lane's four left-over rows
@@ -163,7 +183,7 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
                 const Pair y = {(T)(gelu_tanh(s[0]) * s[2]), (T)(gelu_tanh(s[1]) * s[3])};
                 *reinterpret_cast<Pair*>((T*)a.out_t + (int64_t)m * a.ld_t + (CUS * P + (row >> 4)) * a.t_oct + ((row & 15) >> 1)) = y;
             } else {
-                finish_quad<T, EPI>(a, m, 16 * CUS * P + row, s);
+                finish_quad<T, EPI>(a, m, 16 * CUS * P + row, s, with);
             }
         }
     }
