@@ -101,6 +101,30 @@ def test_prefill_attention_order_of_row_blocks(n, past, H):
     assert torch.isfinite(got).all()
 
 
+# row blocks of 256 (640 MB of keys and values, whole rounds of 256 workgroups): one ragged block and two, tiles of one key, of 63 and whole ones,
+# rows H * D apart; scores that rise with the key
+@pytest.mark.parametrize("n,past,H,token_major,rising", [(130, 2431, 512, False, False), (256, 2560, 512, True, True), (257, 4934, 256, True, False),
+                                                         (511, 4672, 256, False, True), (3850, 37111, 32, False, False)])
+def test_prefill_attention_wide_blocks(n, past, H, token_major, rising):
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n)
+    m = past + n
+    k, v = (torch.randn(*((m + 7, H) if token_major else (H, m + 7)), 128, generator=g, device=DEV, dtype=torch.float16) for _ in range(2))
+    kc, vc = (t.transpose(0, 1) if token_major else t for t in (k, v))
+    q = torch.randn(n, H, 128, generator=g, device=DEV, dtype=torch.float16)
+    some = [0, 7, H - 1]
+    if rising:
+        for h in some:
+            kc[h] += (q[:, h].mean(0) * 20 * torch.linspace(0, 1, m + 7, device=DEV)[:, None]).half()
+    kc[:, m:], vc[:, m:] = float("nan"), float("nan")           # behind the keys: never read
+    got = ops.attn_prefill(q, kc, vc, m, 0.088).view(n, H, 128)
+    assert torch.isfinite(got).all()
+    for rows in {(0, min(70, n)), (max(0, n // 2 - 40), n // 2 + 40), (n - min(n, 140), n)}:
+        seen = m - (n - rows[1])
+        want, size = _attention64(q[rows[0]:rows[1], some], kc[some, :seen], vc[some, :seen], 0.088)
+        assert ((got[rows[0]:rows[1], some].double() - want).abs() <= 2.0 ** -10 * size + 2.0 ** -11 * want.abs() + 1e-6).all()       # (as above)
+
+
 # every key alike, rows that do not see all of their last slab: a hidden score of minus infinity times 0 is no number
 @pytest.mark.parametrize("n,past,H", [(130, 0, 8), (200, 2000, 8), (2049, 0, 32)])
 def test_prefill_attention_scale_of_zero(n, past, H):

@@ -1740,6 +1740,51 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(
                                       nullptr, 0, 0, 0, split, h, s_begin, min(nslabs, s_begin + sps));
 }
 
+#include "prefill_wide.h"
+// The same chunk in row blocks of 256 (launch_prefill says where): all of them side by side, the longest first, a head's on one XCD.
+__global__ __launch_bounds__(256, 1) void prefill_wide_kernel(const h16* __restrict__ q, const h16* __restrict__ k, const h16* __restrict__ v,
+                                                              int64_t stride_t, int64_t stride_h, int sq, int sk, int H, float scale,
+                                                              h16* __restrict__ out, int nrb) {
+    extern __shared__ __attribute__((aligned(16))) char wide_smem[];
+    const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3, h = j / nrb * 8 + xcd, rb = nrb - 1 - j % nrb;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, i = lane & 15;
+    const int r0 = rb * 256, rows = min(256, sq - r0), past = sk - sq;
+    PrefillWide f;
+    int lo[4], hi[4];
+    auto load = [&] {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int row = min(r0 + 64 * wave + 16 * u + i, sq - 1);
+            lo[u] = 0;
+            hi[u] = past + row;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) f.q[u][c] = load_half8(q + ((int64_t)row * H + h) * 128 + 32 * c + 8 * g);
+        }
+    };
+    const h16 *kb = k + (int64_t)h * stride_h, *vb = v + (int64_t)h * stride_h;
+    const int wave_first = past + min(r0 + 64 * wave, sq - 1), end = past + r0 + rows;
+    f.run(wide_smem, 0, (end + 63) / 64, (uint32_t)stride_t, scale, lo, hi, load,
+          [&](int t) {
+              const int64_t at = (int64_t)t * 64 * stride_t;
+              return PrefillWide::Tile{kb + at, vb + at, min(64, sk - t * 64) - 1};
+          },
+          [&](int k0) { return k0 + 31 <= wave_first; });
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int row = r0 + 64 * wave + 16 * u + i;
+        const float inv = 1.0f / f.weight(u);
+        if (row >= sq) continue;
+        h16* o = out + ((int64_t)row * H + h) * 128 + 4 * g;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            half4 x;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) x[r] = (h16)(f.acc[u][t][r] * inv);
+            *reinterpret_cast<half4*>(o + 16 * t) = x;
+        }
+    }
+}
+
 template <int D>
 static size_t blk_lds_bytes() {
     return (size_t)2 * (BlkLayout<D>::K_HALFS + BlkLayout<D>::V_HALFS) * sizeof(h16);
@@ -2280,6 +2325,21 @@ static int launch_prefill(const void* q, const void* k, const void* v, void* out
     // all): 32 heads 12 288 684 -> 703, 16 384 (268 MB) 950 -> 938, 32 768 2 060 -> 1 973; 40 heads 12 288 (252 MB) 852 -> 896, 16 384 1 211
     // -> 1 194; 1 400 rows x 20 000 x 32 heads 519 -> 503.
     const bool from_memory = (int64_t)H * sk * D * 4 > (int64_t)256 << 20;
+    // Row blocks of 256 read half as much from LDS, and pay where memory and LDS draw most: past 640 MB of keys and values, in two or more whole rounds
+    // of one workgroup per CU (us, blocks of 128 -> of 256): 4 096 rows x 32 heads 16 400 keys 937 -> 988, 32 768 2 071 -> 2 078, 40 960 (640 MB)
+    // 2 570 -> 2 503, 57 344 3 432 -> 3 341, 65 536 4 118 -> 3 847, 124 928 8 012 -> 7 300; 3 900 rows x 65 536 4 213 -> 3 873; 2 048 x 64 heads x
+    // 40 000 2 533 -> 2 445; but one round, 2 048 x 32 heads x 65 536 2 107 -> 2 120, and two and a half, 4 096 x 40 heads x 16 384 1 166 -> 1 382.
+    if constexpr (D == 128 && TF_PREFILL_AHEAD && TF_BLOCK_P_SPLIT == 0) {
+        const int blocks = (sq + 255) / 256;
+        if (nsplit == 1 && (int64_t)H * sk * D * 4 >= (int64_t)640 << 20 && H % 8 == 0 && H * blocks >= 512 && H * blocks % 256 == 0) {
+            const hipError_t e = hipFuncSetAttribute((const void*)prefill_wide_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PrefillWide::LDS);
+            if (e != hipSuccess) return (int)e;
+            hipLaunchKernelGGL(prefill_wide_kernel, dim3((unsigned)(H * blocks)), dim3(256), PrefillWide::LDS, st, (const h16*)q, (const h16*)k,
+                               (const h16*)v, stride_t, stride_h, sq, sk, H, scale, (h16*)out, blocks);
+            TF_LAUNCH_CHECK();
+            return TF_OK;
+        }
+    }
     const int nrb = (sq + 127) / 128, rbg = nrb < 8 || from_memory ? nrb : 8;
     const int groups = (nrb + rbg - 1) / rbg;
     const int64_t blocks = (int64_t)H * nsplit * rbg * groups;
