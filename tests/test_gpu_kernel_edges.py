@@ -26,6 +26,24 @@ def test_retrieval_topk_against_stable_sort(H, C, sets, ties):
     assert torch.equal(got, torch.cat([torch.zeros(H, 1, dtype=torch.long), want], 1))
 
 
+# keys of the deciding bin: as many as are ranked against each other, one more, all (a second and a third digit); both sides of 8 and of 16 keys a thread
+@pytest.mark.parametrize("C", [8193, 8194, 16385, 16386])
+@pytest.mark.parametrize("crowd", [256, 257, 8000])
+@pytest.mark.parametrize("equal", [True, False])
+def test_retrieval_topk_of_a_crowded_bin(C, crowd, equal):
+    from triforce_amd import ops
+    g = torch.Generator().manual_seed(C + crowd)
+    s = torch.rand(2, C, generator=g) * 0.9                                           # below the bin of 1 to 1 + 1/32
+    for h in range(2):
+        at = torch.randperm(C - 1, generator=g)[:crowd + 10] + 1
+        s[h, at[:crowd]] = 1.0 + (0 if equal else 1) * torch.randint(0, 32, (crowd,), generator=g) / 1024.0
+        s[h, at[crowd:]] = 2.0 + torch.arange(10)
+    for sets in (12, 12 + crowd // 2, 11 + crowd):                                    # one of the bin, half of it, all
+        got = ops.retrieval_topk(s.half().to(DEV), sets).cpu().long()
+        want = torch.argsort(-s.half()[:, 1:].double(), dim=1, stable=True)[:, :sets - 1] + 1
+        assert torch.equal(got, torch.cat([torch.zeros(2, 1, dtype=torch.long), want], 1))
+
+
 # chunks: fewer than a workgroup's groups, one step and a bit, an even and an odd number of steps, one workgroup per CU; both layouts
 @pytest.mark.parametrize("H,C,token_major", [(3, 5, False), (5, 17, True), (32, 257, False), (40, 700, False), (32, 8200, False), (2, 3001, True)])
 def test_retrieval_score_chunks_of_eight(H, C, token_major):

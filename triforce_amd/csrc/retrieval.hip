@@ -12,6 +12,8 @@
 // per 16-lane group), nothing is staged in a temporary, the top-k runs in LDS.
 #include "common.h"
 
+#include <type_traits>
+
 #ifndef TF_RSCORE_CAP_CEIL
 #define TF_RSCORE_CAP_CEIL 0
 #endif
@@ -150,52 +152,76 @@ __global__ __launch_bounds__(1024) void retrieval_topk_kernel(const uint16_t* __
 // deterministic), the m keys >= it are compacted and only those are sorted.  Same output, bit for bit, as the full sort.
 //
 // One workgroup per head; a latency chain, not a bandwidth one (15 615 keys are 31 KB), so every serial piece is what counts:
-//   * three passes of 11 / 11 / 10 bits instead of four of 8: 2 048 bins spread a head's scores (an fp16's sign, exponent and
-//     five mantissa bits) where 256 bins made the waves queue on a handful of LDS counters;
-//   * the bin that holds the m-th key is found by one wave with two 64-wide scans (one lane walking the bins from the top was
-//     the longest piece of the kernel);
-//   * bitonic stages below 64 exchange inside a wave, so 512 winners meet 6 barrier-separated stages of 45.
-// 32 heads x 15 616 chunks, m = 511: 46.9 -> 16.9 us.
-constexpr int kTopkBins = 2048;
+//   * the keys stay in registers (NK a thread), all asked for at once;
+//   * digits of 11 / 11 / 10 bits: 2 048 bins spread a head's scores (an fp16's sign, exponent and five mantissa bits) where 256 bins made
+//     the waves queue on a handful of LDS counters;
+//   * the bin that holds the m-th key is found by one wave with two 64-wide scans, in registers;
+//   * as soon as that bin holds kTopkNear keys at most (nearly always after the first digit: some 65 of 15 615 normal scores) they are ranked
+//     against each other, instead of two more passes over all keys; more of them, and a pass costs less than the ranks;
+//   * a wave counts what it keeps by ballots and takes its places with one atomic;
+//   * bitonic stages below 64 exchange inside a wave, without LDS; the others alternate between two buffers, one barrier each.
+// 32 heads x 15 616 chunks, m = 511: 46.9 us as one sort, 17.0 with three passes over keys in LDS and exchanges through it, 10.7 now; scores that need
+// a second digit 19.5 -> 14.4; 32 x 4 000 12.6 -> 7.9, 32 x 1 000 (m = 255) 9.4 -> 6.5, 32 x 32 768 23.7 -> 16.7, 8 x 20 000 (m = 4 095) 36.9 -> 31.1.
+constexpr int kTopkBins = 2048, kTopkNear = 256;
 __device__ __forceinline__ int topk_bin(int b) { return b + (b >> 5); }      // (a lane sums 32 neighbouring bins: no bank twice)
 
-// The digit (of `bins` of them) at which the count from the top reaches `rem`, and what is left to find inside it.  One wave.
-__device__ __forceinline__ void topk_digit(const int* hist, int bins, int rem, int lane, int* digit, int* left) {
+template <int CTRL, int ROWS = 0xf> __device__ __forceinline__ uint32_t lane_dpp(uint32_t v) {       // 0 from outside
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+// Inclusive sums over the lanes of a wave: 1, 2, 4, 8 places within a row of 16, then a row's last lane for the rows behind it.
+__device__ __forceinline__ int lanes_scan(int v) {
+    v += lane_dpp<0x111>(v);
+    v += lane_dpp<0x112>(v);
+    v += lane_dpp<0x114>(v);
+    v += lane_dpp<0x118>(v);
+    v += lane_dpp<0x142, 0xa>(v);
+    v += lane_dpp<0x143, 0xc>(v);
+    return v;
+}
+// The larger and the smaller key of lanes l and l ^ J.
+template <int J> __device__ __forceinline__ LanePair<uint32_t> lane_order(uint32_t v) {
+    uint32_t b;
+    if constexpr (J == 32 || J == 16) {
+        const LanePair<uint32_t> p = J == 32 ? lane_halves(v) : lane_rows(v);
+        return {max(p.a, p.b), min(p.a, p.b)};
+    } else if constexpr (J == 8) {
+        b = lane_rotated<8>(v);
+    } else if constexpr (J == 4) {
+        b = lane_dpp<0x1b>(lane_dpp<0x141>(v));                          // l ^ 7 (a half row mirrored), then ^ 3
+    } else {
+        b = lane_dpp<J == 2 ? 0x4e : 0xb1>(v);
+    }
+    return {max(v, b), min(v, b)};
+}
+
+// The digit (of `bins` of them) at which the count from the top reaches `rem`, the keys in its bin and what is left to find among them.  One wave.
+__device__ __forceinline__ void topk_digit(const int* hist, int bins, int rem, int lane, int* digit, int* keys, int* left) {
     const int per = bins >> 6;                                           // 32 or 16
     int own = 0;
+#pragma unroll 8
     for (int j = 0; j < per; ++j) own += hist[topk_bin(bins - 1 - (lane * per + j))];
-    int upto = own;                                                      // inclusive count of the lanes before (higher digits)
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(upto, o, 64);
-        if (lane >= o) upto += t;
-    }
+    const int upto = lanes_scan(own);                                    // inclusive count of the lanes before (higher digits)
     const int owner = __ffsll((long long)__ballot(upto >= rem)) - 1;     // (rem <= keys in the histogram: some lane reaches it)
-    const int before = __shfl(upto - own, owner, 64);
+    const int before = __builtin_amdgcn_readlane(upto - own, owner);
     const int cnt = lane < per ? hist[topk_bin(bins - 1 - (owner * per + lane))] : 0;
-    int in = cnt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int t = __shfl_up(in, o, 64);
-        if (lane >= o) in += t;
-    }
+    const int in = lanes_scan(cnt);
     const int at = __ffsll((long long)__ballot(before + in >= rem)) - 1;
     *digit = bins - 1 - (owner * per + at);
-    *left = rem - before - __shfl(in - cnt, at, 64);
+    *keys = __builtin_amdgcn_readlane(cnt, at);
+    *left = rem - before - __builtin_amdgcn_readlane(in - cnt, at);
 }
 
 // E = winners per thread (the sort's size / 1024, at least 1): element e * 1024 + tid sits in register e of thread tid, so stages
 // below 64 are lane exchanges, stages of 1024 and more are register exchanges and only those between go through LDS.
-template <int E>
+// NK = keys per thread (n <= 1024 * NK).
+template <int E, int NK>
 __global__ __launch_bounds__(1024) void retrieval_topk_select_kernel(const uint16_t* __restrict__ scores,
                                                                       int32_t* __restrict__ idx, int C, int sets,
                                                                       int n, int mpow2) {
-    extern __shared__ uint32_t smem_u[];
-    uint32_t* keys = smem_u;                 // [n]   candidate keys (chunks 1..C-1)
-    uint32_t* sel = smem_u + n;              // [mpow2] the winners
-    __shared__ int hist[kTopkBins + kTopkBins / 32];
+    extern __shared__ uint32_t sel[];        // [2][mpow2] the winners
+    __shared__ __align__(16) int hist[kTopkBins + kTopkBins / 32];
     __shared__ uint32_t s_prefix;
-    __shared__ int s_remaining, s_count;
+    __shared__ int s_remaining, s_keys, s_count;
     const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
     constexpr int nt = 1024;
     const uint16_t* sc = scores + (int64_t)h * C;
@@ -203,49 +229,85 @@ __global__ __launch_bounds__(1024) void retrieval_topk_select_kernel(const uint1
     int32_t* out = idx + (int64_t)h * sets;
     if (tid == 0) out[0] = 0;
     if (m == 0) return;
-#pragma unroll 8
-    for (int i = tid; i < n; i += nt) {
-        const int c = i + 1;
-        keys[i] = (sortable_fp16(sc[c]) << 16) | (uint32_t)(65535 - (c & 0xFFFF));
-    }
-    for (int i = tid; i < mpow2; i += nt) sel[i] = 0u;                   // padding sorts last
-    if (tid == 0) { s_prefix = 0u; s_remaining = m; s_count = 0; }
-    uint32_t prefix = 0u, known = 0u;                                    // the bits of the m-th key found so far
+    uint32_t key[NK];                                                    // of chunks 1..C-1; 0 behind the last (no key is 0)
+#pragma unroll
+    for (int u = 0; u < NK; ++u) key[u] = sc[min(tid + u * nt, n - 1) + 1];
+    for (int i = tid + m; i < mpow2; i += nt) sel[i] = 0u;               // padding sorts last
+    if (tid == 0) { s_remaining = m; s_count = 0; }
+    uint32_t prefix = 0u, known = 0u, open = 0u;                         // the bits of the m-th key found so far, and those to find
+    int keys = 0, left = 0;                                              // with these bits, and how many of them win
 #pragma unroll
     for (int pass = 0; pass < 3; ++pass) {
         const int shift = pass == 0 ? 21 : (pass == 1 ? 10 : 0), bins = pass == 2 ? 1024 : kTopkBins;
         for (int i = tid; i < kTopkBins + kTopkBins / 32; i += nt) hist[i] = 0;
         __syncthreads();
-#pragma unroll 4
-        for (int i = tid; i < n; i += nt) {
-            const uint32_t k = keys[i];
-            if ((k & known) == prefix) atomicAdd(&hist[topk_bin((k >> shift) & (bins - 1))], 1);
+        if (pass == 0) {
+#pragma unroll
+            for (int u = 0; u < NK; ++u) {
+                const int i = tid + u * nt;
+                key[u] = i < n ? (sortable_fp16(key[u]) << 16) | (uint32_t)(65535 - ((i + 1) & 0xFFFF)) : 0u;
+            }
         }
+#pragma unroll
+        for (int u = 0; u < NK; ++u)
+            if (key[u] && (key[u] & known) == prefix) atomicAdd(&hist[topk_bin((key[u] >> shift) & (bins - 1))], 1);
         __syncthreads();
         if (tid < 64) {
-            int digit, left;
-            topk_digit(hist, bins, s_remaining, lane, &digit, &left);
+            int digit, in, rest;
+            topk_digit(hist, bins, s_remaining, lane, &digit, &in, &rest);
             if (tid == 0) {
-                s_remaining = left;
+                s_remaining = rest;
+                s_keys = in;
                 s_prefix = prefix | ((uint32_t)digit << shift);
             }
         }
         __syncthreads();
         prefix = s_prefix;
         known |= (uint32_t)(bins - 1) << shift;
+        open = (1u << shift) - 1u;
+        keys = s_keys;
+        left = s_remaining;
+        if (keys <= kTopkNear) break;                                    // (the last digit leaves one key: keys are distinct)
     }
-#pragma unroll 4
-    for (int i = tid; i < n; i += nt) {                                  // prefix is the m-th largest key (keys are distinct)
-        const uint32_t k = keys[i];
-        if (k >= prefix) {
-            const int p = atomicAdd(&s_count, 1);
-            if (p < mpow2) sel[p] = k;
+    uint32_t* near = reinterpret_cast<uint32_t*>(hist);                  // [keys], zeros up to a multiple of 16 (the counts are used up)
+    if (tid < 16) near[keys + tid] = 0u;
+    const uint32_t least = max(prefix, 1u), most = prefix | open;        // keys above `most` win, m - left of them
+    uint32_t total = 0;                                                  // of this wave: winners, and keys of the bin << 16
+#pragma unroll
+    for (int u = 0; u < NK; ++u)
+        total += (uint32_t)__popcll(__ballot(key[u] > most)) + ((uint32_t)__popcll(__ballot(key[u] >= least && key[u] <= most)) << 16);
+    uint32_t at = 0;
+    if (lane == 0 && total) at = (uint32_t)atomicAdd(&s_count, (int)total);
+    at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    uint32_t at_sel = at & 0xFFFFu, at_near = at >> 16;
+    auto below = [](uint64_t b) { return (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(b >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b, 0u)); };
+#pragma unroll
+    for (int u = 0; u < NK; ++u) {
+        const bool wins = key[u] > most, in = key[u] >= least && key[u] <= most;
+        const uint64_t bw = __ballot(wins), bi = __ballot(in);
+        if (wins) sel[at_sel + below(bw)] = key[u];
+        if (in) near[at_near + below(bi)] = key[u];
+        at_sel += (uint32_t)__popcll(bw);
+        at_near += (uint32_t)__popcll(bi);
+    }
+    __syncthreads();
+    if (tid < keys) {
+        const uint32_t own = near[tid];
+        int rank = 0;
+        for (int j = 0; j < keys; j += 16) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint4 v = *reinterpret_cast<const uint4*>(near + j + 4 * e);
+                rank += (int)(v.x > own) + (int)(v.y > own) + (int)(v.z > own) + (int)(v.w > own);
+            }
         }
+        if (rank < left) sel[m - left + rank] = own;
     }
     __syncthreads();
     uint32_t v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = e * nt + tid < mpow2 ? sel[e * nt + tid] : 0u;
+    uint32_t* spare = sel + mpow2;           // a stage's buffer: written before its barrier and read behind it, the next stage takes the other
     for (int kk = 2; kk <= mpow2; kk <<= 1) {
         int j = kk >> 1;
         if constexpr (E > 1) {
@@ -266,29 +328,38 @@ __global__ __launch_bounds__(1024) void retrieval_topk_select_kernel(const uint1
             }
         }
         for (; j >= 64; j >>= 1) {                                       // other waves hold the partners
-            __syncthreads();
 #pragma unroll
             for (int e = 0; e < E; ++e)
-                if (e * nt + tid < mpow2) sel[e * nt + tid] = v[e];
+                if (e * nt + tid < mpow2) spare[e * nt + tid] = v[e];
             __syncthreads();
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 const int i = e * nt + tid;
                 if (i < mpow2) {
-                    const uint32_t b = sel[i ^ j];
+                    const uint32_t b = spare[i ^ j];
                     const bool larger = ((i & kk) == 0) == ((i & j) == 0);   // this place keeps the larger key of the pair
                     v[e] = larger ? max(v[e], b) : min(v[e], b);
                 }
             }
+            spare = spare == sel ? sel + mpow2 : sel;
         }
-        for (; j > 0; j >>= 1) {
+        if (tid < mpow2) {                                               // (whole waves: mpow2 is 64 at least)
+            auto stage = [&](auto J) __attribute__((always_inline)) {
+                constexpr int j = decltype(J)::value;
+                if (kk > j)
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int i = e * nt + tid;
-                const uint32_t b = __shfl_xor(v[e], j, 64);
-                const bool larger = ((i & kk) == 0) == ((i & j) == 0);
-                v[e] = larger ? max(v[e], b) : min(v[e], b);
-            }
+                    for (int e = 0; e < E; ++e) {
+                        const int i = e * nt + tid;
+                        const LanePair<uint32_t> p = lane_order<j>(v[e]);
+                        v[e] = ((i & kk) == 0) == ((i & j) == 0) ? p.a : p.b;
+                    }
+            };
+            stage(std::integral_constant<int, 32>{});
+            stage(std::integral_constant<int, 16>{});
+            stage(std::integral_constant<int, 8>{});
+            stage(std::integral_constant<int, 4>{});
+            stage(std::integral_constant<int, 2>{});
+            stage(std::integral_constant<int, 1>{});
         }
     }
 #pragma unroll
@@ -405,18 +476,19 @@ extern "C" int tf_retrieval_score(const void* k, int64_t stride_t, int64_t strid
     return TF_OK;
 }
 
-template <int E>
-static int launch_topk_select(const void* scores, int32_t* idx, int C, int sets, int H, int mpow2, size_t lds, void* stream) {
+template <int E, int NK>
+static int launch_topk_select(const void* scores, int32_t* idx, int C, int sets, int H, int mpow2, void* stream) {
+    const size_t lds = 2 * (size_t)mpow2 * sizeof(uint32_t);
     if (lds > 48 * 1024) {
         static bool raised = false;
         if (!raised) {
-            hipError_t e = hipFuncSetAttribute((const void*)retrieval_topk_select_kernel<E>,
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024);
+            hipError_t e = hipFuncSetAttribute((const void*)retrieval_topk_select_kernel<E, NK>,
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
             if (e != hipSuccess) return (int)e;
             raised = true;
         }
     }
-    hipLaunchKernelGGL((retrieval_topk_select_kernel<E>), dim3(H), dim3(1024), lds, (hipStream_t)stream,
+    hipLaunchKernelGGL((retrieval_topk_select_kernel<E, NK>), dim3(H), dim3(1024), lds, (hipStream_t)stream,
                        (const uint16_t*)scores, idx, C, sets, C - 1, mpow2);
     TF_LAUNCH_CHECK();
     return TF_OK;
@@ -425,18 +497,20 @@ static int launch_topk_select(const void* scores, int32_t* idx, int C, int sets,
 extern "C" int tf_retrieval_topk(const void* scores, int32_t* idx, int C, int sets, int H, void* stream) {
     if (!scores || !idx || C < 2 || sets < 1 || sets > C || H < 1) return TF_EINVAL;
     if (C > 32768) return TF_ERANGE;
-    // select-then-sort when candidates + winners fit in LDS together (always for the paper's shapes)
+    // select-then-sort up to 8 192 winners (two buffers of them, 64 KB)
     int mpow2 = 64;
     while (mpow2 < sets - 1) mpow2 <<= 1;
-    const size_t lds_sel = (size_t)((C - 1) + mpow2) * sizeof(uint32_t);
-    if (lds_sel <= 150 * 1024 && mpow2 <= 8192) {
-        const int per_thread = mpow2 <= 1024 ? 1 : mpow2 / 1024;
-        switch (per_thread) {
-            case 1: return launch_topk_select<1>(scores, idx, C, sets, H, mpow2, lds_sel, stream);
-            case 2: return launch_topk_select<2>(scores, idx, C, sets, H, mpow2, lds_sel, stream);
-            case 4: return launch_topk_select<4>(scores, idx, C, sets, H, mpow2, lds_sel, stream);
-            default: return launch_topk_select<8>(scores, idx, C, sets, H, mpow2, lds_sel, stream);
+    if (mpow2 <= 8192) {
+#define GO(E, NK) return launch_topk_select<E, NK>(scores, idx, C, sets, H, mpow2, stream)
+#define GO_N(E) do { if (C - 1 <= 8192) GO(E, 8); if (C - 1 <= 16384) GO(E, 16); GO(E, 32); } while (0)
+        switch (mpow2 <= 1024 ? 1 : mpow2 / 1024) {
+            case 1: GO_N(1);
+            case 2: GO_N(2);
+            case 4: GO_N(4);
+            default: GO_N(8);
         }
+#undef GO_N
+#undef GO
     }
     int npow2 = 2;
     while (npow2 < C - 1) npow2 <<= 1;
