@@ -759,3 +759,59 @@ def test_latent_prefill_by_sequence(news, pasts, H):
                                                   ([700, 130, 257, 513], [3000, 1500, 1400, 691], 8192, 32, 32), ([700, 130, 257, 513], [3000, 1500, 1400, 692], 8192, 32, 32)])
 def test_chunked_prefill_by_sequence(news, pasts, chunk, H, G):
     test_chunked_prefill_tiles(news, pasts, chunk, H, G)
+
+
+# more pages in a split than the 64 whose ids a wave holds (tiles at 64 and 65 pages, two fetches of ids, none), and merges of more splits than the
+# ones that are asked for first
+@pytest.mark.parametrize("nsplit", [1, 2, 40])
+@pytest.mark.parametrize("D", [64, 128])
+def test_step_over_many_pages(nsplit, D):
+    from triforce_amd import ops_hybrid as oh
+    g = torch.Generator(device=DEV).manual_seed(D + nsplit)
+    lens, pages, H, G = [4096, 4097, 8450, 70], 133, 4, 1
+    raw = torch.randn(4, 2 * H * D + 2 * G * D, generator=g, device=DEV)
+    cache = _bf(g, 4 * pages * 64, G * 2 * D)
+    table = torch.randperm(4 * pages, generator=torch.Generator().manual_seed(D)).to(torch.int32).view(4, pages).to(DEV)
+    norm = torch.ones(D, device=DEV)
+    angle = torch.arange(8500, device=DEV)[:, None] * 0.01 * torch.arange(1, 9, device=DEV)
+    before = cache.clone().view(-1, 64, G * 2 * D)
+    attn = dict(q_norm=norm, k_norm=norm, cos=angle.cos().float().contiguous(), sin=angle.sin().float().contiguous(), cache=cache, table=table, q_off=0,
+                k_off=H * D, v_off=H * D + G * D, gate_off=H * D + 2 * G * D, half=8, max_pos=8500, H=H, G=G, D=D, D_real=D, V=D, chunk=0, scale=0.1,
+                out_scale=1.0)
+    step = oh.MixerStep(raw, torch.tensor(lens, dtype=torch.int32, device=DEV), 1e-5, torch.bfloat16, attn=attn, max_keys=pages * 64, nsplit=nsplit)
+    got = step.run().operand().permute(1, 0, 2).reshape(4, -1).double()
+
+    def turned(x, at):                                           # norm, then pairs (e, e + 8) by the position's angle
+        x = x / torch.sqrt(x.square().mean(-1, keepdim=True) + 1e-5)
+        c, s = angle[at].cos(), angle[at].sin()
+        return torch.cat([x[:, :8] * c - x[:, 8:16] * s, x[:, 8:16] * c + x[:, :8] * s, x[:, 16:]], 1).bfloat16().double()
+    for b, n in enumerate(lens):
+        old = before[table[b].long()].reshape(-1, G * 2 * D)[:n - 1].double()
+        q, k = turned(raw[b, :H * D].view(H, D), n - 1), turned(raw[b, H * D:H * D + G * D].view(G, D), n - 1)
+        v = raw[b, H * D + G * D:H * D + 2 * G * D].view(G, D).bfloat16().double()
+        keys, vals = torch.cat([old[:, :D], k]), torch.cat([old[:, D:], v])
+        gate = torch.sigmoid(raw[b, H * D + 2 * G * D:].double()).view(H, D)
+        w = torch.softmax(q @ keys.T * 0.1, 1)
+        want, size = gate * (w @ vals), gate * (w @ vals.abs())
+        # the result's rounding to bfloat16; an entry of q or k that rounds the other way moves a score by 2^-8 * 4 * 4 * 0.1 at most
+        assert ((got[b].view(H, D) - want).abs() <= 2.0 ** -8 * want.abs() + (2.0 ** -15 + 0.00625) * size + 1e-6).all()
+        at = table[b, (n - 1) // 64].long()
+        assert torch.equal(cache.view(-1, 64, 2 * D)[at, (n - 1) % 64, D:], v[0].bfloat16())
+
+
+# rows of more quads than threads: the first of a thread is asked for ahead, the others are not
+@pytest.mark.parametrize("streams", [1, 4])
+@pytest.mark.parametrize("width", [4104, 8192])
+def test_connect_of_wide_rows(streams, width):
+    from triforce_amd import ops_hybrid as oh
+    g = torch.Generator(device=DEV).manual_seed(width + streams)
+    x, y, w = (torch.randn(*n, generator=g, device=DEV) for n in ((3, streams, width), (3, width), (width,)))
+    u, out, mix = (torch.randn(*n, generator=g, device=DEV) for n in ((streams,), (streams,), (streams, streams)))
+    got = x.clone()
+    h = oh.connect(got, u, w, 1e-4, width, torch.bfloat16, y=y, out=out, mix=mix)
+    want = torch.matmul(mix.double().T, x.double()) + out.double()[None, :, None] * y.double()[:, None]
+    # at most 2 * streams float32 sums of terms up to 4 * 4: 8 * 16 * 2^-24 each
+    torch.testing.assert_close(got, want.float(), atol=1e-4, rtol=1e-5)
+    v = torch.matmul(u.double(), want)
+    v = v / torch.sqrt(v.square().mean(-1, keepdim=True) + 1e-4) * w.double()
+    assert ((h.double() - v).abs() <= 2.0 ** -8 * v.abs() + 1e-4).all()          # the result's rounding to bfloat16, and the sums above

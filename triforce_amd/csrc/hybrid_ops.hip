@@ -21,8 +21,7 @@ __global__ __launch_bounds__(64 * NW) void connect_kernel(const T* __restrict__ 
     float* xr = x + (int64_t)row * streams * width;
     const Y* yr = y ? y + (int64_t)row * ld_y : nullptr;
     // Few rows are bound by round trips: what a thread's first quad needs is asked for together with the coefficients (8 rows of 4 x 4 096
-    // 6.0 -> 5.0 us).  More rows are bound by memory, and more
-    // streams do not fit the registers.
+    // 6.0 -> 5.3 us).  More rows are bound by memory, and more streams do not fit the registers.
     constexpr bool EARLY = NW == 16 && S <= 4;
     f32x4 x0[S], y0 = {0.f, 0.f, 0.f, 0.f}, w0 = {0.f, 0.f, 0.f, 0.f};
     auto streams_of = [&](f32x4 (&v)[S], int q) {

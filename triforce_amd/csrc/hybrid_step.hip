@@ -266,6 +266,9 @@ template <int D> struct HeadEntries {                         // raw entries, an
 // of behind them.  What is left is a chain of some 12 us (launch, length, page, first rows, norms, merge of the waves) in front of and
 // behind the stream.  Step and merge, 41 KB and dealt slots against 77 KB and nsplit slots a row: 1 x 8 192 keys 23.7 -> 20.9 us, 8 x 4 096 51.3 ->
 // 46.9, 8 rows of 808 to 8 157 keys 59.1 -> 55.5, 32 around 3 000 139.5 -> 123.8.
+// The wave knows that its row, slot and pages are one number (scalar), and holds the ids of 64 pages: an id read in the loop, or a load behind a
+// condition, has the compiler wait for every load in flight, the tile ahead too.  G = 8, H = 32 of 128, step and merge, before -> now: 8 x 4 096 keys
+// 34.5 -> 32.0 us, 1 x 8 000 18.1 -> 16.6, 16 x 3 000 44.3 -> 40.8, 32 x 3 000 82.4 -> 72.1, 64 x 1 000 61.2 -> 55.1.
 template <int DK, int DV>
 struct SizedStep {
     static constexpr int KT = 32, D = 32 * DK, V = 16 * DV, LDK = D + 8, LDV = V + 16, TILE = KT * (LDK > LDV ? LDK : LDV);

@@ -1,10 +1,11 @@
 // Attention of the latent family for gfx950.
 //
-// Decode (attn_latent_kernel): the query has been taken through the key up-projection, so the cached row itself is the key
-// ([latent | rotated]) and its latent part the value, for every head: one KV stream shared by all heads.  A workgroup walks the
-// 64-key pages of its split, staged in LDS.  Scores are computed transposed (S^T = K Q^T: rows keys, columns heads), so that a lane owns one head's statistics;
-// wave w takes keys 16w .. 16w+15.  The weights go to LDS as [head][key] and every wave then accumulates its share of the
-// latent columns, O^T = C^T P^T, with the transposed operand read straight from the key-major page (ds_read_b64_tr_b16).
+// Decode: the query has been taken through the key up-projection, so the cached row itself is the key ([latent | rotated]) and its latent part the
+// value, for every head: one KV stream shared by all heads.  Scores are computed transposed (S^T = K Q^T: rows keys, columns heads), so that a lane
+// owns one head's statistics; the weights go to LDS as [head][key] and every wave accumulates its share of the latent columns, O^T = C^T P^T, with the
+// transposed operand read straight from the key-major page (ds_read_b64_tr_b16).  In bfloat16 of 512 + 64 (attn_latent_sized_body) half of a workgroup's
+// waves score a half page of 32 keys while the other half multiplies the one before; other sizes (attn_latent_kernel) take whole pages, staged in LDS,
+// wave w keys 16w .. 16w+15.
 //
 // Prefill (attn_prefill_kernel): keys and values up-projected once per chunk, flash attention with 16 query rows per wave (2 x 16 in
 // attn_prefill_sized_kernel), the waves of a workgroup sharing the key / value tile.  Also transposed: the S^T result registers of two 16-key tiles ARE the P operand of
