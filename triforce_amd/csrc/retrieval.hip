@@ -368,10 +368,11 @@ __global__ __launch_bounds__(1024) void retrieval_topk_select_kernel(const uint1
 }
 
 // ---- gather ---------------------------------------------------------------------------------
-// One 128-thread workgroup per (slot, head, K | V): a 2-KiB chunk, one 16-byte vector per thread.  In situ 24.9 us for the
-// 134 MB (67 read + 67 written) of a cfg2 layer = 5.4 TB/s.  A coarser form — one workgroup per 8 slots, all chunk ids
-// read first, 8 loads in flight per lane before the 8 stores — measured 26.0 us (round 3, bench.py roofline_stages on two
-// boxes): the copy is bound by the mixed read / write stream, not by loads in flight; the simple form stays.
+// One 128-thread workgroup per (slot, head, K | V): a 2-KiB chunk, one 16-byte vector per thread.  Bound by the mixed stream, not by loads in
+// flight: whole lines that nobody reads soon are written past the caches, whose place the reads keep.  32 heads x 512 chunks of 15 616 (67 MB read and
+// 67 written, four layers in turn) plain -> this way 29.3 -> 22.2 us (6.0 TB/s), 1 536 chunks, two layers 39.4 -> 34.1, 32 x 256 of 1 000
+// 12.3 -> 10.1, 5 x 513 of 5 003 10.2 -> 8.9, one layer from the caches 4.5 -> 4.3 and 2.5 -> 2.2.  Reads past the caches instead 21.7, but 5.3 and
+// 3.0 where the chunks are in them; both 23.3; two, four or eight slots a workgroup 20.5 to 30, the same order.
 __global__ __launch_bounds__(128) void retrieval_gather_kernel(
     const h16* __restrict__ k_src, const h16* __restrict__ v_src, int64_t sst, int64_t ssh,
     const int32_t* __restrict__ idx, h16* __restrict__ k_dst, h16* __restrict__ v_dst, int64_t dst_t, int64_t dsh,
@@ -385,7 +386,7 @@ __global__ __launch_bounds__(128) void retrieval_gather_kernel(
     for (int e = threadIdx.x; e < chunk * vec_per_row; e += blockDim.x) {
         const int r = e / vec_per_row, dv = e - r * vec_per_row;
         const half8 x = load_half8(src + ((int64_t)c * chunk + r) * sst + 8 * dv);
-        store_half8(dst + ((int64_t)slot * chunk + r) * dst_t + 8 * dv, x);
+        __builtin_nontemporal_store(x, reinterpret_cast<half8*>(dst + ((int64_t)slot * chunk + r) * dst_t + 8 * dv));
     }
 }
 
