@@ -44,6 +44,32 @@ def test_retrieval_topk_of_a_crowded_bin(C, crowd, equal):
         assert torch.equal(got, torch.cat([torch.zeros(2, 1, dtype=torch.long), want], 1))
 
 
+# few rows and more, heads of whole 16-byte pieces and not, rows and bases that start on one and not, more pieces than a workgroup's threads; both cache layouts
+@pytest.mark.parametrize("H,D", [(1, 16), (3, 48), (33, 128), (2, 8), (5, 40), (3, 2)])
+@pytest.mark.parametrize("shift,pad", [(0, 0), (0, 4), (1, 7), (8, 8)])
+@pytest.mark.parametrize("token_major", [False, True])
+@pytest.mark.parametrize("rows", [63, 64, 70])
+def test_rope_append_in_pieces(H, D, shift, pad, token_major, rows):
+    from triforce_amd import ops
+    from oracle import ref_ops as R
+    g = torch.Generator().manual_seed(H * D + shift)
+    T = rows + 7
+    wide = torch.randn(rows, shift + 3 * H * D + pad, generator=g).half()
+    qkv = wide.to(DEV)[:, shift:shift + 3 * H * D]
+    cos, sin = torch.randn(40, D, generator=g).half(), torch.randn(40, D, generator=g).half()
+    pos = torch.randint(0, 40, (rows,), generator=g)
+    q, k, v = wide[:, shift:shift + 3 * H * D].view(rows, 3, H, D).unbind(1)
+    for rotate in (True, False):
+        kl, vl = (torch.zeros((T, H, D) if token_major else (H, T, D), dtype=torch.float16, device=DEV) for _ in "kv")
+        if token_major:
+            kl, vl = kl.permute(1, 0, 2), vl.permute(1, 0, 2)
+        got = ops.rope_append(qkv, cos.to(DEV), sin.to(DEV), pos.to(DEV), kl, vl, 4, H, D, rotate_k=rotate)
+        assert torch.equal(got.cpu(), R.apply_rope(q, cos, sin, pos))
+        assert torch.equal(kl[:, 4:4 + rows].permute(1, 0, 2).cpu(), R.apply_rope(k, cos, sin, pos) if rotate else k)
+        assert torch.equal(vl[:, 4:4 + rows].permute(1, 0, 2).cpu(), v)
+        assert not kl[:, :4].any() and not kl[:, 4 + rows:].any() and not vl[:, :4].any() and not vl[:, 4 + rows:].any()
+
+
 # chunks: fewer than a workgroup's groups, one step and a bit, an even and an odd number of steps, one workgroup per CU; both layouts
 @pytest.mark.parametrize("H,C,token_major", [(3, 5, False), (5, 17, True), (32, 257, False), (40, 700, False), (32, 8200, False), (2, 3001, True)])
 def test_retrieval_score_chunks_of_eight(H, C, token_major):
