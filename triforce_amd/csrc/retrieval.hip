@@ -370,7 +370,7 @@ __global__ __launch_bounds__(1024) void retrieval_topk_select_kernel(const uint1
 // ---- gather ---------------------------------------------------------------------------------
 // One 128-thread workgroup per (slot, head, K | V): a 2-KiB chunk, one 16-byte vector per thread.  Bound by the mixed stream, not by loads in
 // flight: whole lines that nobody reads soon are written past the caches, whose place the reads keep.  32 heads x 512 chunks of 15 616 (67 MB read and
-// 67 written, four layers in turn) plain -> this way 29.3 -> 22.2 us (6.0 TB/s), 1 536 chunks, two layers 39.4 -> 34.1, 32 x 256 of 1 000
+// 67 written, four layers in turn) plain -> this way 29.3 -> 22.2 us (6.0 TB/s; behind a build's scores 29.3 -> 25.4), 1 536 chunks, two layers 39.4 -> 34.1, 32 x 256 of 1 000
 // 12.3 -> 10.1, 5 x 513 of 5 003 10.2 -> 8.9, one layer from the caches 4.5 -> 4.3 and 2.5 -> 2.2.  Reads past the caches instead 21.7, but 5.3 and
 // 3.0 where the chunks are in them; both 23.3; two, four or eight slots a workgroup 20.5 to 30, the same order.
 __global__ __launch_bounds__(128) void retrieval_gather_kernel(
