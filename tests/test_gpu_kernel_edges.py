@@ -169,6 +169,24 @@ def test_prefill_attention_wide_blocks(n, past, H, token_major, rising):
         assert ((got[rows[0]:rows[1], some].double() - want).abs() <= 2.0 ** -10 * size + 2.0 ** -11 * want.abs() + 1e-6).all()       # (as above)
 
 
+# a value that is not finite spoils the rows that see it, and by hidden weights of 0 no others than those whose 64 rows walk its tile of 64 keys
+@pytest.mark.parametrize("n,past,H", [(256, 2560, 512), (511, 4672, 256), (3850, 37111, 32)])
+def test_prefill_attention_reach_of_a_value_that_is_not_finite(n, past, H):
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n)
+    k, v = (torch.randn(H, past + n, 128, generator=g, device=DEV, dtype=torch.float16) for _ in range(2))
+    q = torch.randn(n, H, 128, generator=g, device=DEV, dtype=torch.float16)
+    plain = ops.attn_prefill(q, k, v, past + n, 0.088).view(n, H, 128).clone()
+    at = past + torch.linspace(0, n - 1, H, device=DEV).long()  # a key of the chunk for each head
+    v[torch.arange(H, device=DEV), at, 5] = float("inf")
+    got = ops.attn_prefill(q, k, v, past + n, 0.088).view(n, H, 128)
+    row = torch.arange(n, device=DEV)[:, None]
+    walked = 64 * ((past + torch.clamp(64 * (row // 64 + 1), max=n) + 63) // 64)
+    assert not torch.isfinite(got[..., 5])[past + row >= at].any()
+    clean = at[None] >= walked
+    assert clean.any() and torch.equal(got[clean], plain[clean])
+
+
 # every key alike, rows that do not see all of their last slab: a hidden score of minus infinity times 0 is no number
 @pytest.mark.parametrize("n,past,H", [(130, 0, 8), (200, 2000, 8), (2049, 0, 32)])
 def test_prefill_attention_scale_of_zero(n, past, H):

@@ -1762,8 +1762,8 @@ __global__ __launch_bounds__(256, 1) void prefill_wide_kernel(const h16* __restr
         }
     };
     const h16 *kb = k + (int64_t)h * stride_h, *vb = v + (int64_t)h * stride_h;
-    const int wave_first = past + min(r0 + 64 * wave, sq - 1), end = past + r0 + rows;
-    f.run(wide_smem, 0, (end + 63) / 64, (uint32_t)stride_t, scale, lo, hi, load,
+    const int wave_first = past + min(r0 + 64 * wave, sq - 1), wave_last = past + min(r0 + 64 * wave + 63, sq - 1), end = past + r0 + rows;
+    f.run(wide_smem, 0, wave_last / 64 + 1, (end + 63) / 64, (uint32_t)stride_t, scale, lo, hi, load,
           [&](int t) {
               const int64_t at = (int64_t)t * 64 * stride_t;
               return PrefillWide::Tile{kb + at, vb + at, min(64, sk - t * 64) - 1};

@@ -51,8 +51,10 @@ struct PrefillWide {
 
     // tile(t): the Tile; whole(k0): every row of the wave sees all 32 keys from k0 on (wave-uniform); otherwise query u sees lo[u] .. hi[u].
     // load() fills q, lo and hi.  k_ld: elements from row to row (63 rows stay below 2^32 bytes).
+    // A wave multiplies the tiles up to t_own, its last row's (wave-uniform), and brings in its part of the others: a hidden weight of 0 times a value that
+    // is not finite is no number, so what a row does not see must end with its wave's 64 rows and not with the workgroup's 256.
     template <class Load, class Src, class Whole>
-    __device__ __forceinline__ void run(char* smem, int t_beg, int t_end, uint32_t k_ld, float scale, const int (&lo)[QT], const int (&hi)[QT], Load&& load,
+    __device__ __forceinline__ void run(char* smem, int t_beg, int t_own, int t_end, uint32_t k_ld, float scale, const int (&lo)[QT], const int (&hi)[QT], Load&& load,
                                         Src&& tile, Whole&& whole) {
         const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, i = lane & 15;
         const float sc = scale * 1.4426950408889634f;
@@ -289,7 +291,7 @@ struct PrefillWide {
         }
         meet<16>();                                           // V[0]
         uint32_t slot = 0;
-        for (int t = t_beg; t < t_end; ++t) {
+        for (int t = t_beg; t < t_own; ++t) {
             half_step(sa, sb, Num<0>{}, t, slot);
             refer(true);
             half_step(sb, sa, Num<1>{}, t, slot);
@@ -301,6 +303,16 @@ struct PrefillWide {
         for (int u = 0; u < QT; ++u)
 #pragma unroll
             for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(acc[u][t]));
+        for (int t = t_own; t < t_end; ++t) {
+            meet<8>();
+            const Tile a = at_tile(t + 3);
+            const uint4v k0 = source(a.k, a.last), v0 = source(a.v, a.last);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) fetch_k(k0, (slot + 3 * TILE) & (3 * TILE), p);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) fetch_v(v0, (slot + 3 * TILE) & (3 * TILE), p);
+            slot = (slot + TILE) & (3 * TILE);
+        }
         __builtin_amdgcn_s_waitcnt(0x0F70);                   // no load is under way when the LDS is given back
     }
     __device__ __forceinline__ float weight(int u) const {
