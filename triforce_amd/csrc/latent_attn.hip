@@ -313,8 +313,10 @@ static int launch_merge(const float* ws, void* out, int rows, int H, int C, int 
 // The same attention for rows of 512 + 64 in bfloat16, up to 32 heads per workgroup.  Half pages (32 keys) stream through four places in LDS,
 // where LDS-DMA brings them two ahead of their use.  Waves 0 .. 3 score a half page (16 keys x 16 heads each, queries in registers) while waves
 // 4 .. 7 multiply the one before it with its weights (128 of the latent columns each, all heads): one barrier a half page.
-// The weights' reference is a head's largest score of the first half page, and stays: weights go in as value and remainder, whose precision
-// does not depend on the scale, and nothing overflows before a score is 2^100 above it.  Then the reference follows and the sums are scaled.
+// The weights' reference lies ROOM above a head's largest score of the first half page, and stays until a score passes it; then it moves ROOM above that
+// one and the sums are scaled.  So no weight is above 1, and sums of large latents overflow where they do with a running maximum, not before.  The largest
+// weight is at least 2^-8 behind a reference that has just moved: weights go in as value and remainder, whose precision does not depend on the scale,
+// and 8 places leave the smallest normal latents' sums (2^-126 of them, in denormals of 2^-149) more places than the result has.
 // A place holds rows of 1 152 bytes; inside every 128 bytes the pieces of 16 are XORed by swap(row), which leaves the row reads of the scores and
 // the transposing reads of the values without bank conflicts.
 // Bound by what two half pages under way (74 KB a CU) draw, 5.5 TB/s, behind some 9 us of start and end.  Eight waves that took a page together, scored it,
@@ -342,7 +344,7 @@ __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ 
                                                        int row, int h0, int split, int t_beg, int t_end, char* smem) {
     typedef LatentTile Z;
     constexpr int W = Z::W, C = Z::C, LDP = Z::LDP, ROW = 2 * W, PIECES = W / 8, LOADS = Z::BYTES / 4096;
-    constexpr float GROW = 100.0f;
+    constexpr float ROOM = 8.0f / LOG2E;
     typedef __attribute__((address_space(3))) const char* Lds;
     typedef __attribute__((address_space(3))) bf16x4* Lds4;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15, part = wave & 3;
@@ -434,7 +436,7 @@ __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ 
         scores(0);
         largest();
         meet<63>();
-        m = fmaxf(red[head], red[Z::H + head]);               // (the first key is visible: finite)
+        m = fmaxf(red[head], red[Z::H + head]) + ROOM;        // (the first key is visible: finite)
         if (ks == 0 && g == 0) ref[head] = m;
         weights(0);
         meet<LOADS>();
@@ -444,7 +446,7 @@ __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ 
             if (__builtin_amdgcn_readfirstlane(grown)) {      // the half page before this one needs another reference
                 largest();
                 meet<63>();
-                const float to = fmaxf(m, fmaxf(red[head], red[Z::H + head]));
+                const float to = fmaxf(m, fmaxf(red[head], red[Z::H + head]) + ROOM);
                 l *= __builtin_amdgcn_exp2f((m - to) * LOG2E);
                 m = to;
                 weights(j - 1);
@@ -455,7 +457,7 @@ __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ 
             if (j < nt) {
                 scores(j);
                 const float top = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
-                if (__builtin_amdgcn_ballot_w64((top - m) * LOG2E > GROW)) {
+                if (__builtin_amdgcn_ballot_w64(top > m)) {
                     if (lane == 0) grow[j & 1] = 1;
                 }
                 weights(j);
@@ -514,7 +516,7 @@ __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ 
                 meet<63>();
 #pragma unroll
                 for (int h = 0; h < HT; ++h) {
-                    const float was = ref[16 * h + i], to = fmaxf(was, fmaxf(red[16 * h + i], red[Z::H + 16 * h + i]));
+                    const float was = ref[16 * h + i], to = fmaxf(was, fmaxf(red[16 * h + i], red[Z::H + 16 * h + i]) + ROOM);
                     const float f = __builtin_amdgcn_exp2f((was - to) * LOG2E);
 #pragma unroll
                     for (int x = 0; x < NTW; ++x)
