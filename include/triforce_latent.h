@@ -70,8 +70,10 @@ int tfl_attn_decode(const void* q, const void* cache, int n_pages, const int32_t
  * splits dealt over the rows' pages (at most nsplit, 2 .. 128, of a row); the others take panels_each panels (2 .. 4) of the product.
  * out NULL: the splits stay in ws, for tfl_latent_value.
  * tfl_attn_beside_plan: workers, panels_each and nsplit for rows with `pages` pages in all, 0 where the two are better launched apart; parts: how
- * many splits all rows have together. */
+ * many splits all rows have together.  tfl_attn_beside_plan_of: the same, `longest` of the pages in one row. */
 int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages, int n, int k, int32_t* panels_each, int32_t* nsplit, int32_t* parts);
+int tfl_attn_beside_plan_of(int rows, int H, int C, int R, int64_t pages, int64_t longest, int n, int k, int32_t* panels_each, int32_t* nsplit,
+                            int32_t* parts);
 int tfl_attn_decode_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out, float* ws,
                            int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int panels_each, const TflGemm* product, void* stream);
 /* TFL_EPI_GATED in bfloat16 (include/triforce_tile.h; k 512, up to 4 rows) of what the splits in ws merge to: product->x is not read. */

@@ -182,11 +182,11 @@ def test_steps_do_not_depend_on_the_room_in_the_cache(lens):
 def test_a_graph_for_each_form_of_the_step():
     """Few pages and many in turn, by replays and eagerly: the same logits, and a graph for each form, whichever rows are live."""
     model = _model()
-    lens = [60 + 3 * b for b in range(8)] + [8000 - 16 * b for b in range(8)]
+    lens = [60 + 3 * b for b in range(8)] + [16000 - 16 * b for b in range(8)]          # (on either side of a change of the division)
     graphs, eager = (_filled(model, sum(lens) + 1000, lens, g) for g in (True, False))
     few, many = list(range(8)), list(range(8, 16))
     for t, names in enumerate((few, many, few, few, many, few)):
         ids = (torch.arange(8) * 7 + t) % 96
         assert torch.equal(graphs.decode(names, ids), eager.decode(names, ids)), t
     forms = list(graphs._steps[8].graphs)
-    assert forms == [model.decode_form(8, sum(n // 64 + 1 for n in ls)) for ls in (lens[:8], lens[8:])] and len(set(forms)) == 2
+    assert forms == [model.decode_form(8, sum(n // 64 + 1 for n in ls), max(ls) // 64 + 1) for ls in (lens[:8], lens[8:])] and len(set(forms)) == 2

@@ -126,12 +126,45 @@ def test_plan_of_attention_beside_a_product():
     assert ol.beside_plan(1, 20, 512, 32, 64, 4096, 11008) is None and ol.beside_plan(1, 20, 256, 64, 64, 4096, 11008) is None
 
 
-# rows, pages in all -> panels each: where one division was the fastest by 3 % or more (32 heads, 4 096 x 11 008)
+# rows, pages in all -> panels each: the division that was the fastest, mostly by 3 % or more (32 heads, 4 096 x 11 008; rows half to all as long as the longest)
 @pytest.mark.parametrize("rows,pages,each", [(1, 4, 2), (1, 64, 2), (1, 192, 2), (2, 114, 2), (4, 204, 2), (8, 54, 2), (8, 258, 2), (12, 438, 2), (16, 592, 2),
-                                             (24, 596, 2), (24, 1192, 3), (32, 32, 2), (32, 784, 2), (32, 1184, 3), (12, 870, 3), (24, 1788, 4)])
+                                             (24, 596, 2), (24, 1192, 2), (32, 32, 2), (32, 784, 2), (32, 1184, 2), (12, 870, 2), (24, 1788, 3)])
 def test_plan_picks_what_was_measured_fastest(rows, pages, each):
     from triforce_amd import ops_latent as ol
     assert ol.beside_plan(rows, 32, 512, 64, pages, 4096, 11008)[1] == each
+
+
+# the same with the longest row known, others as long, half or an eighth as long; apart (0) where the product's part of the CUs is far the longer side
+@pytest.mark.parametrize("rows,pages,longest,n,k,each", [
+    (20, 1449, 96, 4096, 11008, 2), (14, 980, 70, 4096, 11008, 2), (26, 1040, 40, 4096, 11008, 2), (32, 503, 100, 4096, 11008, 2), (12, 1733, 192, 4096, 11008, 3),
+    (8, 1539, 256, 4096, 11008, 3), (32, 2319, 96, 4096, 11008, 3), (28, 4044, 192, 4096, 11008, 4), (8, 2306, 512, 4096, 11008, 4),
+    (26, 1250, 300, 4096, 11008, 4), (32, 1478, 300, 4096, 11008, 4), (24, 155, 8, 8192, 16384, 0), (24, 155, 8, 4096, 16384, 0), (24, 1163, 64, 4096, 16384, 2)])
+def test_plan_for_a_known_longest_row(rows, pages, longest, n, k, each):
+    from triforce_amd import ops_latent as ol
+    plan = ol.beside_plan(rows, 32, 512, 64, pages, n, k, longest)
+    assert plan is None if each == 0 else plan[1] == each
+
+
+def test_a_step_says_how_long_its_longest_sequence_is():
+    """With the token that it adds: a page's last and its first."""
+    from triforce_amd.utils.batch_infer import _DecodeStep
+    asked = []
+
+    class Model:
+        def decode_form(self, rows, pages, longest):
+            asked.append((rows, pages, longest))
+            raise StopIteration
+
+    class Known:
+        page, length = 64, {"a": 63, "b": 64, "c": 200}
+    step = object.__new__(_DecodeStep)
+    step.model, step.cache, step.use_graph, step.graphs = Model(), Known(), True, {}
+    step.form = step.model.decode_form
+    step.buf = type("Buffers", (), dict(B=2, batch=type("Batch", (), {})()))()
+    for seqs in (["a", "b"], ["a", "a"], ["c", "new"]):
+        with pytest.raises(StopIteration):
+            step(seqs, None)
+    assert asked == [(2, 3, 2), (2, 2, 1), (2, 5, 4)]
 
 
 # ---- configuration and registry -------------------------------------------------------------------------------------------

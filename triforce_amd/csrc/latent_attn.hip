@@ -582,8 +582,8 @@ __global__ __launch_bounds__(512, 2) void attn_latent_sized_kernel(const bf16* _
 // and CU behind 8 us of start, the product up to 50.
 // Splits are dealt: as many pages each, 2 at least where a row has more than 16, as make the splits of all rows fit the workers; a row has
 // nsplit at most, with as many pages each as that takes.  Statistics of splits that a row does not have are zero, which the merge skips.
-// us, 32 heads, attention, merge, value and the output product (shorter by 11 008 of its 15 104), apart -> so: a row of 64 pages 38.2 -> 33.2, 32 rows
-// with 1 184 pages 67.1 -> 64.8 (more beside beside_plan).
+// us, 32 heads, attention, merge, value and the output product (shorter by 11 008 of its 15 104), apart -> so: a row of 64 pages 38.5 -> 33.6, 32 rows
+// with 1 167 pages 68.0 -> 60.1 (more beside beside_plan).
 template <int P, int MT>
 __global__ __launch_bounds__(512, 2) void attn_latent_beside_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages,
                                                                     const int32_t* __restrict__ table, int table_ld, const int32_t* __restrict__ len,
@@ -712,41 +712,45 @@ extern "C" int tfl_attn_decode(const void* q, const void* cache, int n_pages, co
     return TF_EINVAL;
 }
 
-// How the CUs are shared between the attention of `pages` pages in all and a product of n outputs of k, or 0 workers where the two are better one
-// after the other.  The product takes up to half of the CUs, which draw all that memory gives (39 bytes a ns each with their start).  us of a graph of
-// the attention, its merge, latent to value and the whole output product (32 heads, n 4096, k 11 008 of 15 104, rows half to all as long as the longest),
-// apart -> beside with the product on 128 CUs | 86 | 64:
-//   pages in all   one each                ~200                  ~600                  ~1 200                  ~2 350
-//    1 row    31.2->32.6|39.1|44.4   42.8->37.8|44.4|49.3   48.0->41.8|47.0|51.5 (512)
-//    8 rows   37.2->39.7|46.4|51.7   42.1->43.4|50.5|54.5   46.5->45.9|51.9|56.4   53.7->50.8|53.9|59.5   68.7->70.0|64.3|67.6 (16 rows)
-//   16 rows   42.7->42.0|50.2|55.9   44.8->46.1|53.0|57.7   48.9->47.9|55.4|59.8   56.6->50.3|56.4|62.0
-//   32 rows   54.9->53.7|59.8|65.2   54.2->55.1|60.9|66.7   58.7->55.2|63.1|68.4   67.1->57.0|64.8|70.8   79.4->74.4|68.4|75.4
-// The constants were fitted (530 points: 20 and 32 heads, 1 to 32 rows, 1 to 512 pages a row, n 4 096 to 8 192, k 2 048 to 16 384) to the attention before
-// this one, whose page took a CU 4.4 us beside the product and 3.9 on the whole chip, where this one's takes 2.2 and 2.7.  They hold up to some 30 pages
-// a row; behind that they leave the product fewer CUs than it would like (32 rows, 1 200 to 1 600 pages in all: 64.8 and 66.4 on 86, 57.0 and 61.4 on 128).
-// At k 16 384 the product's half of the CUs is by far the longer side.  A row of activations costs 0.5 in either form (each group of panels reads all of x).
-static int beside_plan(int rows, int H, int64_t pages, int n, int k, int* panels_each) {
+// How the CUs are shared between the attention of `pages` pages in all, `longest` of them in one row, and a product of n outputs of k, or 0 workers
+// where the two are better one after the other.  The product takes up to half of the CUs, which draw all that memory gives (38 bytes a ns each).
+// us of a graph of the attention, its merge, latent to value and the whole output product (32 heads, n 4096, k 11 008 of 15 104, rows half to all as long
+// as the longest, weights and keys from memory), apart -> beside with the product on 128 CUs | 86 | 64:
+//   pages in all   one each                 ~60                  ~200                  ~590                 ~1 160                 ~1 550                 ~2 320
+//    1 row    32.0->32.3|41.0|45.0   38.5->33.6|42.2|46.0   41.7->37.7|45.4|49.4   47.3->41.1|47.3|51.0 (512)
+//    4 rows   35.6->36.6|44.3|49.0   39.8->38.3|45.1|49.5   41.9->40.5|48.0|51.9   46.8->44.0|49.8|54.3                          62.2->63.0|56.8|61.6
+//    8 rows   36.7->38.7|46.1|51.3   39.2->40.2|47.1|52.7   41.5->42.6|49.6|54.5   46.2->44.4|51.7|56.9   56.4->54.9|56.7|61.6   61.8->61.9|57.6|64.4
+//   16 rows   41.0->41.3|49.9|55.6   41.6->42.9|50.5|56.6   44.3->45.9|52.4|58.4   49.6->48.0|54.7|60.3   59.3->55.1|59.2|66.0   64.8->61.9|61.9|68.2   75.9->78.4|70.5|72.4
+//   32 rows   52.2->52.3|59.5|66.0   52.5->52.9|59.9|66.4   53.8->54.5|61.3|67.7   58.6->55.3|63.4|69.8   68.0->60.1|68.0|75.5   74.4->67.1|70.4|77.4   84.6->83.0|74.5|81.2
+// The constants are fitted to 1 862 such points: 20 to 32 heads, 1 to 32 rows, 1 to 4 096 pages, n 4 096 to 8 192, k 2 048 to 16 384; rows half to all as
+// long as the longest, all alike, and one eight times as long as the others, whose pages too few splits then share (32 rows with 503 pages, 100 of
+// them in one row: 76.3 apart, 57.3 beside).  What they pick takes 1.008 of the best on average and at most 1.10.  Half of that is short contexts,
+// which stay beside where that costs a tenth at most: apart, the splits follow the cache's room, beside, what is in it.  (Not at k above 12 288, where the
+// product's half of the CUs is by far the longer side.)
+static int beside_plan(int rows, int H, int64_t pages, int64_t longest, int n, int k, int* panels_each) {
     const int panels = n >> 4;
-    if (rows < 1 || rows > 32 || H <= 16 || H > 32 || pages < 1 || pages > (1 << 20) || panels < 256 || panels > 512 || k < 2048) return 0;
-    if (k > 12288 && rows > 4 && pages < 32 * rows) return 0;
-    const int row = (int)((pages + rows - 1) / rows), ns = tfl_attn_decode_splits(rows, H, 512, 64, (int)pages * TFL_PAGE, 0);
-    const double bytes = 2.0 * n * k, heads = H / 32.0, x = rows * k / 11008.0;
-    double least = bytes / 6.2e6 + 13.35 + 3.9 * ((row + ns - 1) / ns) - 0.11 * rows + 0.47 * x + 0.005 * heads * rows * ns;        // (apart)
+    if (rows < 1 || rows > 32 || H <= 16 || H > 32 || pages < 1 || pages > (1 << 20) || longest < 1 || panels < 256 || panels > 512 || k < 2048) return 0;
+    const int ns = tfl_attn_decode_splits(rows, H, 512, 64, (int)(pages < 16 ? 16 : pages) * TFL_PAGE, 0);        // (a cache of what is there, or more)
+    const double mb = 2e-6 * n * k, heads = H / 32.0, x = rows * k / 11008.0;
+    double least = 3.345 + 0.1237 * mb + 0.1656 * rows + 0.4873 * x + 0.0083 * heads * rows * ns + 0.0026 * pages + 2.245 * (double)((longest + ns - 1) / ns);
+    if (pages < 32 * rows && k <= 12288) least *= 1.0 / 0.9;
     int workers = 0;
     for (int p = 2; p <= 4; ++p) {
-        const int g = (panels + p - 1) / p, a = 256 - g;
+        const int g = (panels + p - 1) / p, a = 256 - g, most = 2 * a / rows < 128 ? 2 * a / rows : 128;
         if (g > 128) continue;
-        const double product = 5.5 + bytes / g / 39e3 + 0.51 * x, attention = 7.85 + 4.45 * (double)pages / a + 2.0 * p;
-        const double t = fmax(product, attention) + (0.064 + 0.03 * heads) * rows + 0.005 * heads * (double)(pages < a ? pages : a);
+        const double each = fmax((double)pages / a, (double)((longest + most - 1) / most));
+        const double product = 26.33 * mb / g + 0.527 * x, attention = 3.22 + 2.7475 * each + 0.945 * p;
+        const double t = fmax(product, attention) + 0.25 * heads * rows + 0.0068 * heads * (double)(pages < a ? pages : a) - 1.892 * (rows < 5 ? 5 - rows : 0);
         if (t < least) { least = t; workers = a; *panels_each = p; }
     }
     return workers;
 }
 
-extern "C" int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages, int n, int k, int32_t* panels_each, int32_t* nsplit, int32_t* parts) {
+extern "C" int tfl_attn_beside_plan_of(int rows, int H, int C, int R, int64_t pages, int64_t longest, int n, int k, int32_t* panels_each, int32_t* nsplit,
+                                       int32_t* parts) {
     if (!panels_each || !nsplit || !parts || C != 512 || R != 64) return 0;
     int p = 0;
-    const int a = beside_plan(rows, H, pages, n, k, &p);
+    const int a = beside_plan(rows, H, pages, longest, n, k, &p);
     *panels_each = p;
     *nsplit = rows < 1 ? 0 : 2 * a / rows < 128 ? 2 * a / rows : 128;
     *parts = 0;
@@ -755,6 +759,12 @@ extern "C" int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages
         *parts = (int32_t)(all < a ? all : a);
     }
     return a;
+}
+
+// The same where nobody knows the longest row: rows half to all as long as it.
+extern "C" int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages, int n, int k, int32_t* panels_each, int32_t* nsplit, int32_t* parts) {
+    const int64_t longest = rows < 1 || pages < rows ? 1 : (4 * pages - 1) / (3 * (int64_t)rows) + 1;
+    return tfl_attn_beside_plan_of(rows, H, C, R, pages, rows == 1 ? pages : longest, n, k, panels_each, nsplit, parts);
 }
 
 template <int P, int MT>

@@ -68,14 +68,14 @@ class LatentLayer:
     def weights(self):
         return [self.w_in, self.w_uq, self.w_uk_t, self.w_uv, self.w_out] + ([self.side_gate, self.side_proj] if self.side_dim else [])
 
-    def beside(self, rows, pages):
+    def beside(self, rows, pages, longest=None):
         """How attention and the feed-forward's half of the output product share the chip in a decode step of rows that hold ``pages`` pages in
-        all (ops_latent.beside_plan); None: one after the other, as where nobody knows the pages.  (What they hold, not what the cache could:
+        all, the longest ``longest`` (ops_latent.beside_plan); None: one after the other, as where nobody knows the pages.  (What they hold, not what the cache could:
         for the product a CU too few costs more than a page's attention on one CU more.)"""
         g = self.geom
         if pages is None or not self.ff or not self.w_out.chunk_major or self.w_out.dtype != torch.bfloat16:
             return None
-        return ol.beside_plan(rows, g.H, g.C, g.R, pages, self.w_out.n, self.w_out.k - g.H * g.V)
+        return ol.beside_plan(rows, g.H, g.C, g.R, pages, self.w_out.n, self.w_out.k - g.H * g.V, longest)
 
     # -- the two forms of a layer: h (normed input), x (fp32 residual, updated) -> y (token-side output, added by the next norm) ----
     def decode(self, h, x, ids, side_table, batch, rope, cache_rows, eps):
@@ -85,7 +85,7 @@ class LatentLayer:
         qn, q = ol.query_and_append(xq, raw, ss, self.w_uq, g, self.kv_norm, eps, rope, batch.pos, batch.slot, cache_rows)
         ol.query_to_latent(qn, self.w_uk_t, q, g)
         own = g.H * g.V                                       # act: the attention's columns, then the feed-forward's, which wait for nothing of it
-        plan = self.beside(ids.numel(), batch.pages)
+        plan = self.beside(ids.numel(), batch.pages, batch.longest)
         if plan is None:
             o = ol.attn_decode(q, cache_rows, batch.table, batch.klen, g, self.scale, batch.max_len)
         else:
@@ -159,9 +159,9 @@ class LatentWeights:
         self.kinds = list({(L.geom.H, L.geom.V, L.geom.C, L.geom.R, L.ff, L.w_out.n): L for L in self.layers}.values())
         return self
 
-    def decode_form(self, rows, pages):
+    def decode_form(self, rows, pages, longest=None):
         """What a decode step's launches depend on besides the number of rows: equal for steps that one captured graph serves."""
-        return tuple(L.beside(rows, pages) for L in self.kinds)
+        return tuple(L.beside(rows, pages, longest) for L in self.kinds)
 
     def load_state_dict(self, sd):
         want = self.shapes()

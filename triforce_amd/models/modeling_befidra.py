@@ -70,9 +70,9 @@ class BefidraForCausalLM:
             self._rope = {k: RotaryTable(s, n, self.device) for k, s in specs.items()}
 
     # -- forward -----------------------------------------------------------------------------
-    def decode_form(self, rows, pages):
-        """Key of the decode step's launches for ``rows`` sequences that hold ``pages`` cache pages in all."""
-        return self.weights.decode_form(rows, pages)
+    def decode_form(self, rows, pages, longest=None):
+        """Key of the decode step's launches for ``rows`` sequences that hold ``pages`` cache pages in all, ``longest`` of them in one."""
+        return self.weights.decode_form(rows, pages, longest)
 
     @torch.inference_mode()
     def __call__(self, input_ids, kv_cache=None, graph_cache=None, position_ids=None, **_):

@@ -208,11 +208,13 @@ def _value_merges(rows, H, nsplit, parts):
 
 
 @functools.lru_cache(maxsize=1024)
-def beside_plan(rows, H, C, R, pages, n, k):
-    """(workers, panels each, splits, does latent_to_value merge them) of attn_decode_beside for rows that hold ``pages`` pages in all and a
-    product of n outputs of k, None where the two are better launched apart."""
+def beside_plan(rows, H, C, R, pages, n, k, longest=None):
+    """(workers, panels each, splits, does latent_to_value merge them) of attn_decode_beside for rows that hold ``pages`` pages in all, the longest
+    ``longest`` of them (not known: rows half to all as long as it), and a product of n outputs of k, None where the two are better launched apart."""
     each, nsplit, parts = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
-    workers = hip.latent_lib().tfl_attn_beside_plan(rows, H, C, R, pages, n, k, ctypes.byref(each), ctypes.byref(nsplit), ctypes.byref(parts))
+    to = ctypes.byref(each), ctypes.byref(nsplit), ctypes.byref(parts)
+    L = hip.latent_lib()
+    workers = L.tfl_attn_beside_plan(rows, H, C, R, pages, n, k, *to) if longest is None else L.tfl_attn_beside_plan_of(rows, H, C, R, pages, longest, n, k, *to)
     return (workers, each.value, nsplit.value, _value_merges(rows, H, nsplit.value, parts.value)) if workers > 0 else None
 
 

@@ -72,7 +72,7 @@ class _DecodeStep:
 
     def __init__(self, model, cache, B, use_graph):
         self.model, self.cache, self.buf, self.use_graph = model, cache, _DecodeBuffers(cache, B), use_graph
-        self.form = getattr(model, "decode_form", lambda rows, pages: None)                     # (most models have one form)
+        self.form = getattr(model, "decode_form", lambda rows, pages, longest: None)                     # (most models have one form)
         self.graphs = {}                                        # form -> (graph, logits), in one pool: of these only one runs at a time
 
     def _graph(self, form):
@@ -93,7 +93,8 @@ class _DecodeStep:
         b, c = self.buf, self.cache
         before = tuple(c.length.get(s, 0) for s in seqs)
         b.batch.pages = sum(n // c.page + 1 for n in before)    # with this step's token
-        graph, logits = self._graph(self.form(b.B, b.batch.pages)) if self.use_graph else (None, None)
+        b.batch.longest = max(before, default=0) // c.page + 1
+        graph, logits = self._graph(self.form(b.B, b.batch.pages, b.batch.longest)) if self.use_graph else (None, None)
         c.extend([(s, 1) for s in seqs])
         births = tuple(c.birth[s] for s in seqs)
         if b.current != (births, before):
