@@ -145,10 +145,11 @@ def test_prefill_attention_order_of_row_blocks(n, past, H):
     assert torch.isfinite(got).all()
 
 
-# row blocks of 256 (640 MB of keys and values, whole rounds of 256 workgroups): one ragged block and two, tiles of one key, of 63 and whole ones,
+# row blocks of 256 (640 MB of keys and values, whole rounds of 256 workgroups; 900 MB, more than half a last round): one ragged block and two, tiles of one key, of 63 and whole ones,
 # rows H * D apart; scores that rise with the key
 @pytest.mark.parametrize("n,past,H,token_major,rising", [(130, 2431, 512, False, False), (256, 2560, 512, True, True), (257, 4934, 256, True, False),
-                                                         (511, 4672, 256, False, True), (3850, 37111, 32, False, False)])
+                                                         (511, 4672, 256, False, True), (3850, 37111, 32, False, False),
+                                                         (3300, 54310, 32, True, True), (257, 9100, 200, False, False)])
 def test_prefill_attention_wide_blocks(n, past, H, token_major, rising):
     from triforce_amd import ops
     g = torch.Generator(device=DEV).manual_seed(n)
@@ -170,7 +171,7 @@ def test_prefill_attention_wide_blocks(n, past, H, token_major, rising):
 
 
 # a value that is not finite spoils the rows that see it, and by hidden weights of 0 no others than those whose 64 rows walk its tile of 64 keys
-@pytest.mark.parametrize("n,past,H", [(256, 2560, 512), (511, 4672, 256), (3850, 37111, 32)])
+@pytest.mark.parametrize("n,past,H", [(256, 2560, 512), (511, 4672, 256), (3850, 37111, 32), (3300, 54310, 32)])
 def test_prefill_attention_reach_of_a_value_that_is_not_finite(n, past, H):
     from triforce_amd import ops
     g = torch.Generator(device=DEV).manual_seed(n)

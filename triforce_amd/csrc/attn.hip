@@ -2328,10 +2328,15 @@ static int launch_prefill(const void* q, const void* k, const void* v, void* out
     // Row blocks of 256 read half as much from LDS, and pay where memory and LDS draw most: past 640 MB of keys and values, in two or more whole rounds
     // of one workgroup per CU (us, blocks of 128 -> of 256): 4 096 rows x 32 heads 16 400 keys 937 -> 988, 32 768 2 071 -> 2 078, 40 960 (640 MB)
     // 2 570 -> 2 503, 57 344 3 432 -> 3 341, 65 536 4 118 -> 3 847, 124 928 8 012 -> 7 300; 3 900 rows x 65 536 4 213 -> 3 873; 2 048 x 64 heads x
-    // 40 000 2 533 -> 2 445; but one round, 2 048 x 32 heads x 65 536 2 107 -> 2 120, and two and a half, 4 096 x 40 heads x 16 384 1 166 -> 1 382.
+    // 40 000 2 533 -> 2 445; but one round, 2 048 x 32 heads x 65 536 2 107 -> 2 120.  A last round that is more than half full pays from 900 MB on, as blocks
+    // of 128 leave as many CUs idle there: 1.6 rounds (3 328 x 32 heads) x 65 536 4 060 -> 3 770, 1.9 (3 840) 4 185 -> 3 730, x 124 928 8 110 -> 7 190, 40 heads
+    // x 3 072 x 65 536 4 312 -> 3 880, 2.8 (48 x 3 840) 0.93 of the time, 3.8 (64 x 3 840) 0.955; 645 MB 0.92 to 1.09 of it, 96 heads x 1 700 rows 1.045 at 900 MB,
+    // 0.93 at 2 200.  Half a round or less does not: 1.5 (3 072 x 32) x 65 536 3 360 -> 3 805, 2.5 (4 096 x 40) 5 262 -> 5 760, x 124 928 10 080 -> 11 040, 1.25
+    // (2 560 x 32) 3 100 -> 3 870, 3.5 (64 x 3 584) 1.06 of the time.
     if constexpr (D == 128 && TF_PREFILL_AHEAD && TF_BLOCK_P_SPLIT == 0) {
-        const int blocks = (sq + 255) / 256;
-        if (nsplit == 1 && (int64_t)H * sk * D * 4 >= (int64_t)640 << 20 && H % 8 == 0 && H * blocks >= 512 && H * blocks % 256 == 0) {
+        const int blocks = (sq + 255) / 256, last = H * blocks % 256;
+        const int64_t bytes = (int64_t)H * sk * D * 4;
+        if (nsplit == 1 && H % 8 == 0 && H * blocks > 384 && ((last == 0 && bytes >= (int64_t)640 << 20) || (last > 128 && bytes >= (int64_t)900 << 20))) {
             const hipError_t e = hipFuncSetAttribute((const void*)prefill_wide_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, PrefillWide::LDS);
             if (e != hipSuccess) return (int)e;
             hipLaunchKernelGGL(prefill_wide_kernel, dim3((unsigned)(H * blocks)), dim3(256), PrefillWide::LDS, st, (const h16*)q, (const h16*)k,
