@@ -156,3 +156,32 @@ def test_every_prefill_attention_kernel_takes_the_split_of_its_weights():
     plain, split = products(()), products(("TF_BLOCK_P_SPLIT=1",))
     assert len(plain) == 2 and plain.keys() == split.keys()
     assert all(split[k] > 1.3 * plain[k] for k in plain), (plain, split)
+
+
+def test_counted_waits_leave_what_a_step_issues():
+    """attn_latent_sized_body meets with the youngest half page (9 loads; the first time two) in flight, PrefillWide with the youngest tile (8; the first time the
+    two behind the first).  More would be in flight behind a barrier if a wait counted other loads than a step issues; none may be where the wave ends."""
+    synthetic = """
+_Zk: ; @_Zk
+\tglobal_load_lds_dwordx4 v1, s[0:1]
+\tbuffer_load_dwordx4 v2, s[4:7], 0 offen lds
+\tbuffer_load_dwordx4 v[4:7], v2, s[4:7], 0 offen
+\ts_waitcnt vmcnt(1) lgkmcnt(0)
+\ts_barrier
+\ts_cbranch_scc1 .LBB0_2
+\ts_waitcnt vmcnt(0)
+.LBB0_2:
+\ts_endpgm
+.Lfunc_end0:
+"""
+    assert isa_lint.dma_in_flight(synthetic)["_Zk"] == dict(dma=2, most=2, at_barriers=[1], at_end=1)
+    assert isa_lint.dma_in_flight(synthetic.replace("\ts_cbranch_scc1 .LBB0_2\n", ""))["_Zk"]["at_end"] == 0
+    from triforce_amd.build import FLAGS
+    extra = [f for f in FLAGS if f == "-mllvm" or f.startswith("-amdgpu-")]
+    for source, names, dma, left in (("latent_attn.hip", ("attn_latent_sized_kernel", "attn_latent_beside_kernel"), 36, {0, 9, 18}),
+                                     ("attn.hip", ("prefill_wide_kernel",), 40, {0, 8, 16})):
+        shapes = isa_lint.dma_in_flight(isa_lint.compile_to_asm(os.path.join(CSRC, source), extra=extra))
+        found = {k: v for k, v in shapes.items() if any(n in k for n in names)}
+        assert len(found) >= len(names)
+        for k, v in found.items():
+            assert v["dma"] == dma and set(v["at_barriers"]) <= left and v["at_end"] == 0, (k, v)

@@ -249,3 +249,46 @@ def undrained_dma(text):
                 at += 1
         out[m.group(1)] = dict(dma=dma, undrained_barriers=len(bad))
     return out
+
+
+# ---- fifth check: LDS-DMA behind counted waits (csrc/latent_attn.hip, csrc/prefill_wide.h) --------------------------------------
+# There a barrier leaves the youngest loads in flight, by a number in the source that has to fit how many a step issues.  dma_in_flight() walks
+# every path of a kernel with the most LDS-DMA that can be under way (a wait for all but N loads leaves N at most, whatever else was
+# issued), and says how many that is at the barriers and where the wave ends, whose LDS the next workgroup gets.
+def dma_in_flight(text):
+    out = {}
+    for m in re.finditer(r"^(_Z\w+):\s*;\s*@\1\n([\s\S]*?)\n\.Lfunc_end\d+:", text, re.M):
+        insts, labels = [], {}
+        for line in m.group(2).split("\n"):
+            t = line.strip()
+            lab = re.match(r"^(\.L\w+):", t)
+            if lab:
+                labels[lab.group(1)] = len(insts)
+            elif t and t[0] not in ";.":
+                insts.append(t)
+        is_dma = lambda t: t.startswith("global_load_lds") or (t.startswith("buffer_load") and re.search(r"\blds\b", t))       # noqa: E731
+        barriers, ends, most, work, seen = set(), set(), 0, [(0, 0)], set()
+        while work:
+            at, flying = work.pop()
+            while at < len(insts) and (at, flying) not in seen:
+                seen.add((at, flying))
+                t = insts[at]
+                left = re.search(r"vmcnt\((\d+)\)", t) if t.startswith("s_waitcnt") else None
+                if is_dma(t):
+                    flying = min(flying + 1, 64)
+                    most = max(most, flying)
+                elif left:
+                    flying = min(flying, int(left.group(1)))
+                elif t.startswith("s_barrier"):
+                    barriers.add(flying)
+                elif t.startswith("s_endpgm"):
+                    ends.add(flying)
+                    break
+                jump = re.match(r"^s_c?branch\w*\s+(\.L\w+)", t)
+                if jump:
+                    work.append((labels[jump.group(1)], flying))
+                    if t.startswith("s_branch"):
+                        break
+                at += 1
+        out[m.group(1)] = dict(dma=sum(map(bool, map(is_dma, insts))), most=most, at_barriers=sorted(barriers), at_end=max(ends, default=0))
+    return out

@@ -11,6 +11,7 @@
 // attn_prefill_sized_kernel), the waves of a workgroup sharing the key / value tile.  Also transposed: the S^T result registers of two 16-key tiles ARE the P operand of
 // one PV product (the value operand is read with the matching key order), so the weights never leave the registers.
 #include "flash_tile.h"
+#include "lds_dma.h"
 #include "share_gemm.h"
 
 #define NEG_INF (-__builtin_inff())
@@ -319,24 +320,19 @@ static int launch_merge(const float* ws, void* out, int rows, int H, int C, int 
 // and 8 places leave the smallest normal latents' sums (2^-126 of them, in denormals of 2^-149) more places than the result has.
 // A place holds rows of 1 152 bytes; inside every 128 bytes the pieces of 16 are XORed by swap(row), which leaves the row reads of the scores and
 // the transposing reads of the values without bank conflicts.
-// Bound by what two half pages under way (74 KB a CU) draw, 5.5 TB/s, behind some 9 us of start and end.  Eight waves that took a page together, scored it,
-// met, weighed it, met and multiplied it needed 2.6 us a page from L2 and 3.8 from memory, with the maxima and the scaling in every page; this 2.05 and
-// 3.4.  us with the merge, 32 heads, keys from memory, before -> now: 32 rows of 24 / 48 / 96 pages 28.2 / 40.0 / 62.7 -> 25.5 / 34.8 / 55.1, 8 of 48 / 192
-// 22.3 / 38.3 -> 19.3 / 34.3, one of 64 / 512 18.1 / 28.3 -> 14.3 / 25.7.  More loads under way (one word of each line, 4 to 8 half pages ahead): 62 -> 71
-// to 77.
+// 5.5 TB/s behind some 9 us of start and end, with one half page under way: where a page is looked up the compiler waits for the loads before it.  With
+// that wait in the branch that asks for more ids, and so two under way, 1 204 sizes are the same to 1 % (apart 0.99 to 1.00, beside a product 1.00).
+// Eight waves that took a page together, scored it, met, weighed it, met and multiplied it needed 2.6 us a page from L2 and 3.8 from memory, with the
+// maxima and the scaling in every page; this 2.05 and 3.4.  us with the merge, 32 heads, keys from memory, before -> now: 32 rows of 24 / 48 / 96 pages
+// 28.2 / 40.0 / 62.7 -> 25.5 / 34.8 / 55.1, 8 of 48 / 192 22.3 / 38.3 -> 19.3 / 34.3, one of 64 / 512 18.1 / 28.3 -> 14.3 / 25.7.  More loads under way (one
+// word of each line, 4 to 8 half pages ahead): 62 -> 71 to 77.
 struct LatentTile {
     static constexpr int KT = 32, W = 576, C = 512, H = 32, BYTES = KT * W * 2, RING = 4, LDP = KT + 8, PARTS = 2;
     static constexpr int P_ELEMS = PARTS * H * LDP, RED = RING * BYTES + 2 * P_ELEMS * 2, LDS = RED + 4 * (2 * H + H + 2);
 };
 static_assert(LatentTile::LDS <= 160 * 1024, "LDS");
 
-// All waves are here, this one's LDS accesses are done and all but the LEFT youngest of its loads have landed.
-template <int LEFT> __device__ __forceinline__ void meet() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0x0070 | (LEFT & 15) | (LEFT >> 4 << 14));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
+template <int LEFT> __device__ __forceinline__ void meet() { meet_dma<LEFT, true>(); }
 
 // (everything but the pointers is the same in all lanes)
 __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages, const int32_t* __restrict__ tab,
@@ -385,10 +381,7 @@ __device__ __forceinline__ void attn_latent_sized_body(const bf16* __restrict__ 
             const char* src = (const char*)(cache + (int64_t)(pg < 0 ? 0 : (pg >= n_pages ? n_pages - 1 : pg)) * (64 * W)) + (c & 1) * Z::BYTES;
             const uint32_t dst = lds + (j & 3) * Z::BYTES + 1024 * part;
 #pragma unroll
-            for (int u = 0; u < LOADS; ++u) {                 // (nothing else here uses M0)
-                const uint32_t at = __builtin_amdgcn_readfirstlane(dst + 4096 * u), o = left >= Z::KT - 1 ? off[u] : place(u, left);
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(o), "s"(src) : "memory");
-            }
+            for (int u = 0; u < LOADS; ++u) lds_dma(__builtin_amdgcn_readfirstlane(dst + 4096 * u), left >= Z::KT - 1 ? off[u] : place(u, left), src);
         };
         page_ids();
 #pragma unroll
@@ -635,12 +628,16 @@ extern "C" int64_t tfl_attn_decode_ws_floats(int rows, int H, int C, int nsplit)
     return nsplit == 1 ? 0 : (int64_t)rows * H * nsplit * (C + 2);
 }
 
-// One workgroup per CU (256) as long as a split keeps at least two pages of keys, or one of up to 16: there the second page costs more
-// (2.4 us) than its partial rows (one row, attention and merge: 500 keys 16.7 -> 14.3 us, 1 000 16.8 -> 14.6; 4 000 keys 18.2 either way, two rows of
-// 4 000 19.7 against 20.7).  Two pages are one split where the second one costs less than the merge: always in the form of known sizes (32 heads,
-// one row 12.7 us against 14.1, 64 rows 13.6 against 19.7), in the other bfloat16 forms from 65 workgroups of 16 heads on (256 | 32, 16 heads, 96 rows
-// 11.5 against 12.4; 32 rows 11.5 against 10.6), never in float32 (55 against 35).  Float32 takes 16 heads per workgroup, one to a CU: single pages
-// only where they are no more rounds of 256 than pairs would be (32 heads, 12 rows of 12 pages 86.5 us against 92.8).
+// One workgroup per CU (256) as long as a split keeps at least two pages of keys, or one of up to 16.  us of the attention with its merge, latent to value
+// and an output product of k 6 144, 32 heads, pairs -> single pages: one row of 8 pages 26.0 -> 24.1, of 16 26.2 -> 24.7; of 64 27.2 -> 26.3, of 128
+// 28.1 -> 30.0; 4 rows of 64 30.6 -> 30.8, 8 of 48 31.9 -> 39.2 (more than the CUs).  So the line would lie at 17 to 64 pages for one or two rows
+// (17 pages 26.3 -> 24.7; 16 heads, 32 pages 23.0 -> 21.1), which this rule leaves at pairs, as it does three to eight pages of 32 rows and more at
+// one a split, where one split of all costs less (64 rows of three pages 51.4 -> 46.8, 64 heads 78.1 -> 67.1): over 568 points of 1 to 64 rows, 1 to 512
+// pages and 16 to 64 heads it takes 1.011 of the best, in the worst 1.16.  Two pages are one split where the second one costs less than the merge: always in
+// the form of known sizes (one row 24.0 us in two, 22.8 in one, 64 rows 50.7 and 44.9).  The other forms, attention and merge alone: bfloat16 from 65
+// workgroups of 16 heads on (256 | 32, 16 heads, 96 rows 11.5 against 12.4; 32 rows 11.5 against 10.6), never in float32 (55 against 35).  Float32
+// takes 16 heads per workgroup, one to a CU: single pages only where they are no more rounds of 256 than pairs would be (32 heads, 12 rows of 12 pages
+// 86.5 us against 92.8).
 extern "C" int tfl_attn_decode_splits(int rows, int H, int C, int R, int max_len, int dtype) {
     if (rows < 1 || H < 1 || max_len < 1) return 1;
     const int groups = H <= 16 ? 1 : (H + 31) / 32, pages = (max_len + TFL_PAGE - 1) / TFL_PAGE, pairs = (pages + 1) / 2;

@@ -10,6 +10,7 @@
 // in place by inline asm, which the compiler would copy; a rescale of 128 sums is one block of asm with its own branches for the same reason.
 #pragma once
 #include "common.h"
+#include "lds_dma.h"
 
 typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -35,19 +36,7 @@ struct PrefillWide {
     static __device__ __forceinline__ void more(Frag a, Frag b, f32x4& c) { asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "a"(a), "a"(b)); }
     static __device__ __forceinline__ void value(Frag a, uint4v b, f32x4& c) { asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "a"(a), "v"(b)); }
     static __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
-    // Twelve wait states between products and what else touches their sums.
-    static __device__ __forceinline__ void hold() {
-        fence();
-        asm volatile("s_nop 11" ::: "memory");
-        fence();
-    }
-    // All but the LEFT youngest loads of this wave have landed, and so have every other wave's; no access crosses.
-    template <int LEFT> static __device__ __forceinline__ void meet() {
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(0x0F70 | (LEFT & 15) | (LEFT >> 4 << 14));
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-    }
+    template <int LEFT> static __device__ __forceinline__ void meet() { meet_dma<LEFT, false>(); }
 
     // tile(t): the Tile; whole(k0): every row of the wave sees all 32 keys from k0 on (wave-uniform); otherwise query u sees lo[u] .. hi[u].
     // load() fills q, lo and hi.  k_ld: elements from row to row (63 rows stay below 2^32 bytes).
@@ -69,7 +58,7 @@ struct PrefillWide {
         }
         auto dma = [&](const uint4v& src, uint32_t off, uint32_t dst) __attribute__((always_inline)) {
             const uint32_t at = __builtin_amdgcn_readfirstlane(dst);
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(at), "v"(off), "s"(src) : "memory");
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(at), "v"(off), "s"(src) : "memory", "m0");
         };
         // a tile as a buffer that ends with its last row: what lies behind comes in as zeros
         auto source = [&](const h16* base, int last) __attribute__((always_inline)) {
@@ -280,7 +269,7 @@ struct PrefillWide {
             if (e == 24 || e == 28) read_k(1, (e - 24) / 4);
             fence();
         });
-        hold();
+        hold_sums();
         if (!whole(t_beg * KT)) hide(sa, t_beg * KT);
 #pragma unroll
         for (int u = 0; u < QT; ++u) {
@@ -298,7 +287,7 @@ struct PrefillWide {
             refer(false);
             slot = (slot + TILE) & (3 * TILE);
         }
-        hold();
+        hold_sums();
 #pragma unroll
         for (int u = 0; u < QT; ++u)
 #pragma unroll
@@ -316,10 +305,7 @@ struct PrefillWide {
         __builtin_amdgcn_s_waitcnt(0x0F70);                   // no load is under way when the LDS is given back
     }
     __device__ __forceinline__ float weight(int u) const {
-        float s = l[u];
-        s += __shfl_xor(s, 16, 64);
-        s += __shfl_xor(s, 32, 64);
-        return s;
+        return rows_sum(l[u]);
     }
 };
 

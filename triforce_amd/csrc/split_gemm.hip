@@ -39,6 +39,7 @@
 // an infinity leaves behind in a model, are marked when they are cut and keep their NaN results.  One infinite row of 700 in front of
 // 22 016 x 4 096 costs 600 -> 1 070 us, of 300 in front of 4 096 x 15 104 236 -> 665 (by a thread per result 4 200 and 9 900).  The kernel stores all
 // sums first and walks through a wave's tiles again where one was odd: thirty-two walks in line cost every launch 4 %.  (The scaling is 16 of some 200 VALU operations per step: 22 016 x 4 096 at 700 rows 740 -> 752 us.)
+#include "lds_dma.h"
 #include "tile_common.h"
 #include <type_traits>
 
@@ -73,23 +74,10 @@ __device__ __forceinline__ void cut_store(const f32x4 (&v)[2], bf16* dst) {
     for (int z = 0; z < 3; ++z) *reinterpret_cast<u32x4*>(dst + 512 * z) = out[z];
 }
 
-// 16 bytes a lane from `from` + off to LDS at `to` + 16 * lane.  Not counted by the compiler, which behind its own form waits for all reads of
-// LDS that are under way wherever one is needed: see meet().
-__device__ __forceinline__ void lds_dma(bf16* to, uint32_t off, const bf16* from) {
-    const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)to;
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(at), "v"(off), "s"(from) : "memory");
-}
-
 // A product without the compiler's say in where its sum goes: it moves some of 256 registers of sums through others in every step.  It does not
-// see then what the matrix core still has to read or write: see hold().
+// see then what the matrix core still has to read or write: hold_sums() stands behind the products of a step, inside their loop, so that no copy of a
+// sum can come first.
 __device__ __forceinline__ void add_in_place(bf16x8 a, bf16x8 b, f32x4& c) { asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b)); }
-// Twelve wait states between products and what else touches their sums: behind a 16 x 16 x 32 product (eight passes) eleven are needed.  Behind the
-// products of a step, inside their loop, so that no copy of a sum can come first.
-__device__ __forceinline__ void hold() {
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_nop 11" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-}
 
 // One workgroup: 16 rows, SPLIT_KC columns.  nans[row][part]: the row has a NaN in this part of k.
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, int64_t ld, int rows, int k, bf16* __restrict__ planes,
@@ -227,7 +215,9 @@ __global__ __launch_bounds__(256, 1) void split_gemm_kernel(const SplitGemm a) {
     const bf16* src[PER];                                     // this wave's fragments of x: scalar pointers to their first chunk
     const float* wsrc[4];                                     // this lane's eight weights of four panels
     f32x4 staged[4][2];
-    auto fetch_x = [&](int f, int c, int buf) { lds_dma(tiles + buf * BUF + (3 * NP + wave * PER + f) * 512, 16u * lane, src[f] + (int64_t)c * 1536); };
+    auto fetch_x = [&](int f, int c, int buf) {
+        lds_dma((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(tiles + buf * BUF + (3 * NP + wave * PER + f) * 512), 16u * lane, src[f] + (int64_t)c * 1536);
+    };
     auto fetch_w = [&](int f, int c) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) staged[f][h] = *reinterpret_cast<const f32x4*>(wsrc[f] + 32 * c + 4 * h);
@@ -356,7 +346,7 @@ __global__ __launch_bounds__(256, 1) void split_gemm_kernel(const SplitGemm a) {
             });
 #pragma unroll
             for (int z = 0; z < 3; ++z) read_w(3, z, buf ^ 1);
-            hold();
+            hold_sums();
         }
     };
     const bool half = xpan - mt0 * MT <= MT / 2;
@@ -455,14 +445,15 @@ struct Parts { int whole, splits, sharers, fold; };
 
 // How k is cut: rounds of workgroups, each with the fill of its pipe (4 steps of 32), against what the parts cost on their way through memory
 // (a written and read 128 x 256 part as much as 8 steps).  Rounds are an XCD's: it has 32 CUs and its eighth of the tiles, rounded up (36 tiles in
-// seven parts are 252 workgroups, but 35 on some XCDs: 700 rows, 1 536 x 6 144 in seven 119 us, in six 95).  256 rows, 12 320 x 4 096: 267 us
-// without parts, 159 with two, 171 with four; 700 rows, 4 096 x 8 192: 514, 296 with two, 262 with five, 265 with eight.
-// From 32 tiles an XCD on: whole rounds of whole tiles, and the steps of the others shared by all CUs, 8 or more to each.  A last round of few tiles,
-// or parts of all tiles instead (516 tiles of 22 016 x 4 096 at 700 rows in two parts, 2.5 rounds and 250 MB of parts): 755 -> 665 us; 12 320
-// outputs 425 -> 402, 1 000 rows of them 565 -> 509, 300 rows of 22 016 402 -> 365, 1 500 1 437 -> 1 288.  Below, sharing gains nothing over whole
-// tiles on fewer CUs, which run at a higher clock (256 rows of 22 016, 172 tiles: 317 us alone, 327 shared).
+// seven parts are 252 workgroups, but 35 on some XCDs: 700 rows, 1 536 x 6 144 in seven 126 us, in six 92).  256 rows, 12 320 x 4 096: 240 us
+// without parts, 148 with two, 164 with four; 700 rows, 4 096 x 8 192: 468, 274 with two, 250 with five, 256 with eight.
+// From 32 tiles an XCD on: whole rounds of whole tiles, and the steps of the others shared by all CUs, 8 or more to each.  Whole tiles alone | the best of
+// two to eight parts of all tiles | this: 700 rows of 22 016 x 4 096 757 | 692 | 605 us, of 12 320 499 | 402 | 364, 1 000 rows of them 523 | 531 | 466,
+// 300 rows of 22 016 414 | 349 | 309, 1 500 1 331 | 1 324 | 1 193.  Below, sharing gains nothing over whole tiles on fewer CUs, which run at a higher clock (256
+// rows of 22 016, 172 tiles, with eight waves: 317 us alone, 327 shared).  The constants were fitted to eight waves of 64 x 64 and hold for these four: over 19
+// sizes of 256 to 2 048 rows what they pick takes 1.03 of the best number of parts at most.
 // A running sum of all steps is further off than the parts that k would be in otherwise (absolute values, 4 096 columns: 3.5e-7, two parts 1.8e-7,
-// three 1.1e-7), so it goes to the result as often (`fold`), at 4 steps' cost each: 700 rows of 22 016 637 -> 665 us, error as in two parts.
+// three 1.1e-7), so it goes to the result as often (`fold`), at 4 steps' cost each (eight waves, 700 rows of 22 016: 637 -> 665 us), error as in two parts.
 static Parts pick_parts(int rows, int n, int k) {
     const int tiles = split_tiles(rows, n), per_xcd = (tiles + 7) / 8;
     const double chunks = k / 32;

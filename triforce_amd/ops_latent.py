@@ -201,9 +201,10 @@ def attn_decode(q, cache, table, klen, g, scale, max_len, nsplit=None):
 
 def _value_merges(rows, H, nsplit, parts):
     """Does latent_to_value merge the splits of attn_decode_beside itself (latent_value_kernel) or a launch in front of it?  us of a layer's attention,
-    value and output product, launch -> itself: one row 35.4 -> 33.3 (64 pages), 40.0 -> 39.4 (256); two 36.4 -> 35.5 (46 splits), 36.7 -> 35.9 (60),
-    38.2 -> 39.0 (88); three rows the same to 1 %; four rows of 32 heads, whose merge is a wave for 128 columns (launch_merge: from 128 heads
-    on, up to 64 splits), 40.3 -> 38.8 with 64 splits a row, with 85 48.2 -> 50.4; four of 20 heads 35.2 -> 36.1."""
+    value and output product, launch -> itself: one row 35.5 -> 33.9 (64 pages), 37.7 -> 37.5 (192), the same from there on; two 36.2 -> 35.4 (72 pages),
+    39.6 -> 39.8 (192); three rows the same to 1 %; four rows of 32 heads, whose merge is a wave for 128 columns (launch_merge: from 128 heads
+    on, up to 64 splits), 39.9 -> 39.0 with 64 splits a row (144 pages), with 85 49.8 -> 51.2 (576 pages).  Over 672 points of 1 to 4 rows 1.001 of the
+    better one, at most 1.04."""
     return rows == 1 or (rows == 2 and parts <= 72) or (rows <= 4 and rows * H >= 128 and nsplit <= 64)
 
 

@@ -168,8 +168,10 @@ def linear_rows(x, w):
     split_linear.  Its tiles are 256 x 128: from 256 rows and 2^32 multiply-adds on it is the faster one (256 x 4 096 x 4 096 87 -> 68 us, 2 048 x 2 048 x 1 024
     68 -> 65, 700 x 22 016 x 4 096 917 -> 590), below that it leaves CUs idle (300 x 6 144 x 1 536 47 -> 52, 64 x 22 016 x 4 096
     117 -> 124), as with few results of a long k, whose parts are eight at most (2^19 results: 385 x 1 136 x 15 104 117 -> 135, 512 x 1 136
-    160 -> 143), and with k below 96 the cut and the results are all there is (1 030 x 65 536 x 64 111 -> 127; of 96 151 -> 159, but 3 000 x 16 384 97 -> 93).  Up to k = 65 536 its error is a
-    tenth to a half of the library's; at 2^20, with as few parts, the two are equal."""
+    160 -> 143), and with k below 96 the cut and the results are all there is (1 030 x 65 536 x 64 111 -> 127).  At k = 96 the two are as fast on the
+    whole (300 x 151 552 144 -> 103, 700 x 65 536 100 -> 92, 1 030 x 65 536 143 -> 153, 262 144 x 1 024 505 -> 602), but the library is three times as far off
+    (normals 1.8e-7 against 5.8e-8), so it starts there.  Up to k = 65 536 its error is a tenth to a half of the library's; at 2^20, with as few parts,
+    the two are equal."""
     rows, (n, k) = x.shape[0], w.shape
     if x.dtype == w.dtype == torch.float32 and x.dim() == 2 and x.shape[1] == k and 256 <= rows <= 1 << 24 and rows * n * k >= 1 << 32 \
             and rows * n > 1 << 19 and n % 16 == 0 and k % 32 == 0 and 96 <= k <= 1 << 16 and x.device == w.device and ops_rows.unwatched(x, w) \
