@@ -53,7 +53,7 @@ __device__ __forceinline__ void finish_raw(const TflGemm& a, int m, bool live, i
 //   * one private stream per wave, panels a power of two apart: chunk-major, the chip reads one moving window per wave index.  (The same
 //     kernel on panel-major weights is slower than the old form up to 8 rows: 28.4 us at 1 076 panels.)
 // us before -> now at 1 / 8 / 32 rows, K 4 096: 256 panels 10.5 / 10.4 / 11.9 -> 7.8 / 8.1 / 10.7, 512: 13.9 / 14.8 / 20.5 -> 12.9 / 12.8 /
-// 15.6, 1 076: 27.9 / 29.2 / 39.5 -> 26.1 / 26.3 / 29.2, 1 376: 34.2 / 34.7 / 41.9 -> 31.2 / 31.6 / 34.8, 2 000: 44.6 / 45.9 / 56.5 -> 43.4 /
+// 15.6, 1 076: 27.9 / 29.2 / 39.5 -> 24.5 / 24.3 / 26.6, 1 376: 34.2 / 34.7 / 41.9 -> 30.5 / 29.6 / 31.5, 2 000: 44.6 / 45.9 / 56.5 -> 43.4 /
 // 43.6 / 46.1 (6.0 TB/s); 256 panels of 15 104: 26.9 / 28.7 / 36.5 -> 21.2 / 22.2 / 32.9 (5.8 TB/s).
 // cu: this workgroup's place among those that share the panels, mb: its block of rows.
 template <typename T, int EPI, int P, bool TAIL, int MT, int U>
@@ -71,8 +71,12 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
     const T* wp[NP];
 #pragma unroll
     for (int p = 0; p < P; ++p) wp[p] = (const T*)a.wp + min(panel0 + p, npan - 1) * 512 + lane * 8;
+    // The rows left over are dealt in fours of workgroups on one XCD: four rows are 64 bytes of a chunk's 256, and a cache line that two XCDs ask for is
+    // fetched twice.  us at 1 / 8 / 32 rows, workgroup by workgroup -> here, K 4 096: 1 076 panels 25.1 / 24.9 / 26.9 -> 24.5 / 24.3 / 26.6, 1 172 25.8 /
+    // 26.1 / 28.4 -> 25.0 / 25.3 / 28.0, gate | up of 1 376 31.9 / 31.0 / 32.3 -> 30.5 / 29.6 / 31.5 (5.9 to 6.1 TB/s).
+    const int tail0 = ((cu & ~31) | (cu & 7) << 2 | (cu >> 3 & 3)) * tail_per;
     if constexpr (TAIL) {
-        const int row = min(min(cu * tail_per + i, cu * tail_per + tail_per - 1), tail_rows - 1);
+        const int row = min(min(tail0 + i, tail0 + tail_per - 1), tail_rows - 1);
         int slot = row & 15;
         if constexpr (EPI == TFL_EPI_GLU) slot = ((slot >> 2) << 1) + (slot & 1) + ((slot & 2) << 2);
         wp[P] = (const T*)a.wp + (CUS * P + (row >> 4)) * 512 + g * 128 + slot * 8;
@@ -112,7 +116,7 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
     auto beside = [&](int j) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         if constexpr (EPI == TFL_EPI_RESIDUAL || EPI == TFL_EPI_IN) {
-            const int p = j / MT, m = m0 + 16 * (j - p * MT) + i, row = cu * tail_per + 4 * g;
+            const int p = j / MT, m = m0 + 16 * (j - p * MT) + i, row = tail0 + 4 * g;
             const bool whole = !TAIL || p < P;
             const int n = whole ? 16 * (panel0 + p) + 4 * g : 16 * CUS * P + row;
             if (j < NP * MT && (whole ? panel0 + p < npan : 4 * g < tail_per && row < tail_rows)) {
@@ -176,7 +180,7 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
                 if (live) finish_quad<T, EPI>(a, m, n, s, with);
             }
         } else {
-            const int row = cu * tail_per + 4 * g;   // first of this lane's four left-over rows
+            const int row = tail0 + 4 * g;   // first of this lane's four left-over rows
             if (!live || 4 * g >= tail_per || row >= tail_rows) continue;
             if constexpr (EPI == TFL_EPI_GLU) {              // gate, gate, up, up of outputs 2q, 2q + 1 of a panel's octet
                 typedef T Pair __attribute__((ext_vector_type(2)));
