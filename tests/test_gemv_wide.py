@@ -1,0 +1,167 @@
+"""The one-workgroup-per-CU products of csrc/gemv_wide.hip at the edges of their shares, against float64 with the rounding points of the path, and the rule
+that picks them."""
+import pytest
+import torch
+
+DEV = "cuda:0"
+EPS = 1e-5
+
+
+def test_the_rule_takes_whole_shares_only_where_panels_stay_whole():
+    from triforce_amd import hip
+    takes = hip.lib().tf_wide_gemm_takes
+    for mode, n, k, want in [(0, 4096, 4096, 1), (0, 4096, 11008, 1), (0, 8192, 2048, 1), (0, 5120, 5120, 0), (0, 5120, 13824, 0), (0, 7168, 2048, 1),
+                             (0, 7152, 2048, 0), (0, 4080, 4096, 0), (0, 4096, 2016, 0), (3, 12288, 4096, 1), (3, 15360, 5120, 1), (3, 9216, 4096, 0),
+                             (1, 22016, 4096, 1), (1, 27648, 5120, 1), (1, 4352, 4096, 1), (2, 32000, 4096, 1), (2, 32768, 4096, 1), (2, 33024, 4096, 0),
+                             (2, 32000, 768, 0), (1, 5504, 4096, 1)]:
+        assert takes(mode, n, k) == want, (mode, n, k)
+    for bad in [(-1, 4096, 4096), (4, 4096, 4096), (0, 4100, 4096), (0, 4096, 4100), (0, 0, 4096), (0, 4096, 0)]:
+        assert takes(*bad) == -22
+
+
+def _rnd(g, *shape, std=1.0):
+    return (torch.randn(*shape, generator=g, device=DEV) * std).half()
+
+
+def _block(ops, x, packed):
+    return ops.Act.from_rows(x, x.shape[0] + 3) if packed else x
+
+
+def _rows(y):
+    return y if isinstance(y, torch.Tensor) else y.rows()
+
+
+def _normed(x, ln):
+    inv = 1.0 / torch.sqrt(x.float().square().mean(-1, keepdim=True) + EPS)
+    return ln * (x.float() * inv).half()
+
+
+def _sums(ops, x):
+    ss = ops.ss_buffer(x.shape[1], DEV)
+    ss.fill_(float("nan"))                                     # (rows that are not there are not read)
+    ss[:, :x.shape[0]] = x.float().view(x.shape[0], -1, 16).square().sum(-1).T
+    return ss
+
+
+def _product(h, w):
+    """The product in 64 bits, and how far its fp16 may be: fp32 sums, their rounding, two operand elements on the neighbouring fp16 (the norm's own sum)."""
+    want, size = h.double() @ w.double().T, h.double().abs() @ w.double().abs().T
+    most = float(h.abs().max()) * w.double().abs().max(1).values
+    return want, size * w.shape[1] * 2.0 ** -24 + want.abs() * 2.0 ** -11 + 2 * most * 2.0 ** -10 + 2.0 ** -24
+
+
+def _near(got, want, bound):
+    excess = (got.double() - want).abs() - bound
+    assert bool((excess <= 0).all()), float(excess.max())
+
+
+# batch rows: one, one block full, two blocks, the last row of them; chunks: as many for each wave, 65 (the last wave has 2), 129
+ROWS_K = [(1, 2048), (7, 4128), (16, 2080), (17, 2048), (32, 4096)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K", ROWS_K)
+@pytest.mark.parametrize("N", [4096, 7168, 8192])             # one panel a workgroup, two on 224 CUs, two
+@pytest.mark.parametrize("packed", [False, True])
+def test_residual(M, K, N, packed):
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    w, x, res = _rnd(g, N, K, std=K ** -0.5), _rnd(g, M, K), _rnd(g, M, N)
+    pl = ops.PackedLinear(w, wide="residual")
+    assert pl.wide == "residual"
+    want, bound = _product(x, w)
+    _near(_rows(ops.linear(_block(ops, x, packed), pl)), want, bound)
+    ss, y = torch.full((N // 16, 32), float("nan"), device=DEV), _block(ops, res.clone(), packed)
+    ops.linear(_block(ops, x, packed), pl, resid=y, out=y, ss_out=ss)
+    got, total = _rows(y), want + res.double()
+    _near(got, total, bound + total.abs() * 2.0 ** -11 + 2.0 ** -24)
+    own = got.double().view(M, -1, 16).square().sum(-1).T
+    assert bool(((ss[:, :M].double() - own).abs() <= own * 16 * 2.0 ** -24).all())
+    pl.w.mul_(2.0)                                             # exact in fp16: re-packed in place
+    before = pl.parts[0].data_ptr()
+    assert pl.refresh_().parts[0].data_ptr() == before
+    _near(_rows(ops.linear(_block(ops, x, packed), pl)), 2 * want, 2 * bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K", ROWS_K)
+# pairs of panels: one workgroup's rest of 4 rows (ragged), whole shares, rests of 8 (full and ragged), a share of one more on fewer CUs, the widest
+@pytest.mark.parametrize("I", [2096, 4096, 5120, 11008, 13824, 16384])
+def test_swiglu(M, K, I):
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(I + M)
+    w, x, ln = _rnd(g, 2 * I, K, std=K ** -0.5), _rnd(g, M, K), (1 + 0.1 * torch.randn(K, generator=g, device=DEV)).half()
+    pl = ops.PackedLinear(w, split=2, wide="swiglu")
+    assert pl.wide == "swiglu"
+    want, bound = _product(_normed(x, ln), w)
+    (a, u), (ea, eu) = want.chunk(2, 1), bound.chunk(2, 1)
+    # silu' is below 1.1 and |silu(a)| at most |a|; roundings of silu and of the product, and expf
+    unit = torch.nn.functional.silu(a) * u
+    most = 1.1 * ea * (u.abs() + eu) + a.abs() * eu + unit.abs() * 2.0 ** -9 + 2.0 ** -23 * (1 + u.abs())
+    for packed in (False, True):
+        for ss in (None, _sums(ops, x)):
+            _near(_rows(ops.mlp_act(_block(ops, x, packed), pl, ln=ln, eps=EPS, ss_in=ss)), unit, most)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K", ROWS_K)
+@pytest.mark.parametrize("N", [4096, 4112, 9984, 21504, 32000, 32768])        # whole shares, rests of 4 and 12 rows, a share of one more, the widest
+def test_logits(M, K, N):
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    w, x, ln = _rnd(g, N, K, std=K ** -0.5), _rnd(g, M, K), (1 + 0.1 * torch.randn(K, generator=g, device=DEV)).half()
+    pl = ops.PackedLinear(w, wide="logits")
+    assert pl.wide == "logits"
+    want, bound = _product(x, w)
+    got = ops.linear(x, pl, out_f32=True)
+    assert got.dtype == torch.float32 and torch.equal(got, got.half().float())          # an fp16 product, then the cast
+    _near(got, want, bound)
+    want, bound = _product(_normed(x, ln), w)
+    for ss in (None, _sums(ops, x)):
+        _near(ops.linear(_block(ops, x, ss is None), pl, out_f32=True, ln=ln, eps=EPS, ss_in=ss), want, bound)
+    wide = torch.full((M, N + 5), 7.0, device=DEV)
+    ops.linear(x, pl, out_f32=True, out=wide[:, 2:N + 2])                               # rows at any stride: nothing beside them is written
+    assert torch.equal(wide[:, 2:N + 2], got) and bool((wide[:, :2] == 7).all()) and bool((wide[:, N + 2:] == 7).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K", ROWS_K)
+@pytest.mark.parametrize("H,D", [(32, 128), (40, 128), (20, 128), (64, 64), (56, 128)])   # 3 panels a workgroup, 4 on 240 CUs, 2 on 240, heads of 64, 6 on 224
+@pytest.mark.parametrize("rotate_k", [True, False])
+def test_qkv(M, K, H, D, rotate_k):
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(H + M)
+    w, x, ln = _rnd(g, 3 * H * D, K, std=K ** -0.5), _rnd(g, M, K), (1 + 0.1 * torch.randn(K, generator=g, device=DEV)).half()
+    pl = ops.PackedLinear(w, rope=(H, D), wide="qkv")
+    assert pl.wide == "qkv"
+    a = torch.outer(torch.arange(300, device=DEV).float(), 100.0 ** (-torch.arange(0, D, 2, device=DEV) / D))
+    cos, sin = (torch.cat([t, t], 1).half() for t in (a.cos(), a.sin()))
+    pos = torch.randint(0, 300, (M,), generator=g, device=DEV)
+    want, bound = ([t.view(M, H, D) for t in p.chunk(3, 1)] for p in _product(_normed(x, ln), w))
+    c, s = cos[pos].double()[:, None], sin[pos].double()[:, None]
+
+    def turned(v, e):
+        other, eo = (torch.cat([t[..., D // 2:], t[..., :D // 2]], -1) for t in (v, e))
+        sign = torch.cat([-torch.ones(D // 2), torch.ones(D // 2)]).to(DEV).double()
+        return v * c + sign * other * s, (e * c.abs() + eo * s.abs()) + ((v * c).abs() + (other * s).abs()) * 2.0 ** -10 + 2.0 ** -23
+    for ss, dev in ((None, None), (_sums(ops, x), torch.tensor([9], dtype=torch.int32, device=DEV))):
+        k, v = (torch.full((H, 64, D), 5.0, device=DEV).half() for _ in range(2))
+        q = ops.qkv_rope(_block(ops, x, ss is None), pl, ln, EPS, cos, sin, pos, k, v, 0 if dev is not None else 9, H, D, rotate_k=rotate_k, slot0_dev=dev,
+                         ss_in=ss)
+        _near(q, *turned(want[0], bound[0]))
+        _near(k[:, 9:9 + M].transpose(0, 1), *(turned(want[1], bound[1]) if rotate_k else (want[1], bound[1])))
+        _near(v[:, 9:9 + M].transpose(0, 1), want[2], bound[2])
+        for t in (k, v):
+            assert bool((t[:, :9] == 5).all()) and bool((t[:, 9 + M:] == 5).all())
+
+
+@pytest.mark.gpu
+def test_a_row_that_is_not_finite_stays_its_own():
+    from triforce_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(3)
+    w, x, ln = _rnd(g, 8192, 2048, std=2048 ** -0.5), _rnd(g, 5, 2048), torch.ones(2048, device=DEV).half()
+    pl = ops.PackedLinear(w, wide="logits")
+    good = ops.linear(x, pl, out_f32=True, ln=ln, eps=EPS)
+    x[2, 7], x[4] = float("inf"), 0.0
+    got = ops.linear(x, pl, out_f32=True, ln=ln, eps=EPS)
+    assert torch.equal(got[[0, 1, 3]], good[[0, 1, 3]]) and bool(got[2].isnan().any()) and bool((got[4] == 0).all())

@@ -16,10 +16,10 @@ LIB_PATH = os.path.join(LIB_DIR, "libtriforce_hip.so")
 TILE_LIB_PATH = os.path.join(LIB_DIR, "libtriforce_tile.so")
 LATENT_LIB_PATH = os.path.join(LIB_DIR, "libtriforce_latent.so")
 HYBRID_LIB_PATH = os.path.join(LIB_DIR, "libtriforce_hybrid.so")
-SOURCES = ["attn.hip", "retrieval.hip", "elementwise.hip", "sampling.hip", "offload.hip", "gemv.hip", "rows_gemm.hip", "allreduce.hip", "draft.hip", "draft_persist.hip", "topp_multi.hip", "abi.hip"]
+SOURCES = ["attn.hip", "retrieval.hip", "elementwise.hip", "sampling.hip", "offload.hip", "gemv.hip", "gemv_wide.hip", "rows_gemm.hip", "allreduce.hip", "draft.hip", "draft_persist.hip", "topp_multi.hip", "abi.hip"]
 LIBRARIES = {
-    "core": (LIB_PATH, SOURCES, ["common.h", "lanes.h", "tree_mask.h", "select_common.h", "prefill_wide.h", "lds_dma.h", "rows_gemm.h"], ["triforce_hip.h"]),
-    "tile": (TILE_LIB_PATH, ["tile_gemm.hip", "split_gemm.hip", "tile_rows_gemm.hip", "paged.hip"], ["tile_common.h", "lanes.h", "lds_dma.h", "share_gemm.h", "rows_gemm.h"], ["triforce_tile.h"]),
+    "core": (LIB_PATH, SOURCES, ["common.h", "gemv_common.h", "share_shape.h", "lanes.h", "tree_mask.h", "select_common.h", "prefill_wide.h", "lds_dma.h", "rows_gemm.h"], ["triforce_hip.h"]),
+    "tile": (TILE_LIB_PATH, ["tile_gemm.hip", "split_gemm.hip", "tile_rows_gemm.hip", "paged.hip"], ["tile_common.h", "lanes.h", "lds_dma.h", "share_gemm.h", "share_shape.h", "rows_gemm.h"], ["triforce_tile.h"]),
     "latent": (LATENT_LIB_PATH, ["latent_attn.hip", "latent_ops.hip"], ["tile_common.h", "lanes.h", "lds_dma.h", "flash_tile.h", "share_gemm.h"], ["triforce_tile.h", "triforce_latent.h"]),
     "hybrid": (HYBRID_LIB_PATH, ["hybrid_rec.hip", "hybrid_attn.hip", "hybrid_step.hip", "hybrid_ops.hip"], ["tile_common.h", "lanes.h", "flash_tile.h", "hybrid_common.h"],
                ["triforce_tile.h", "triforce_hybrid.h"]),

@@ -22,7 +22,7 @@
 //   * RoPE + KV-append epilogue (fused q|k|v, :212-238): the packed row order pairs rotary partners d and d + D/2
 //     inside one 16-row panel, so the epilogue rotates q / k in registers (one cross-lane exchange) and writes q
 //     to [M][H][D] and the k / v rows straight into the cache slots.
-#include "common.h"
+#include "gemv_common.h"
 
 #ifdef TF_NO_NT
 #define SG_LOAD(p) (*(p))
@@ -65,8 +65,6 @@
 #define TF_SG_RES_EARLY 1   // residual epilogue operands fetched before the weight loop (0: at the tail, round 2's form)
 #endif
 
-enum { SG_PLAIN = 0, SG_GATEUP = 1, SG_F32 = 2, SG_QKV = 3 };
-
 // Activation layout (round 4).  Every activation operand is addressed through two element strides,
 //     element (m, k) at base[m * sm + (k / 8) * sk + (k % 8)],
 // so one kernel serves the reference's row-major [M][ld] blocks (sm = ld, sk = 8) and the k-octet-major form
@@ -74,9 +72,6 @@ enum { SG_PLAIN = 0, SG_GATEUP = 1, SG_F32 = 2, SG_QKV = 3 };
 // M-row block is ONE contiguous run of 4 * R pieces.  The B operand of a 16-row tile is then 4 runs of 256 B instead of
 // 16 row fragments of 64 B (twice the cache lines per load instruction), which is what bounded the 17...32-row GEMMs of the
 // gamma = 16 verifies (profiles/r03_gemm_rows_ab.jsonl).
-struct SgAct {
-    int64_t sm, sk;
-};
 
 // P = panels per wave: a wave that multiplies P weight panels against ONE B operand reads x once per P KiB of weights
 // (x traffic through L2 -> L1 is panels * M * K * 2 bytes: as large as the weight stream itself at 17 rows with P = 1).
@@ -212,27 +207,6 @@ __device__ __forceinline__ half4 xc_ld8(const h16* p) {
 static int g_sg_p2_rows = 1;       // P = 2 from this many rows (tf_sg_tune key 0; 33 = never)
 static int g_sg_p2_waves = 4;      // waves per workgroup of the P = 2 form (key 1)
 static int g_sg_p2_groups = SG_P_WIDE_MIN_GROUPS;   // ... while panels / 2 >= this (key 2)
-
-struct SgRope {                       // arguments of the RoPE + KV-append epilogue (SG_QKV)
-    const h16* cosb;                  // [max_pos][D] fp16
-    const h16* sinb;
-    const int64_t* positions;         // [M]
-    h16* q_out;                       // [M][H][D]
-    h16* k_cache;                     // layer base, element strides below
-    h16* v_cache;
-    int64_t stride_t, stride_h;
-    const int32_t* slot0_dev;
-    int slot0, H, D, rotate_k;
-};
-
-// h = w_ln * fp16(x * inv): the cast precedes the weight multiply (modeling_llama.py:141-143); the fp16 product of
-// two fp16 values rounded once is the native half multiply.
-__device__ __forceinline__ half8 sg_normalise(half8 xv, half8 wv, float inv) {
-    half8 o;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = hmul_rn(wv[e], (h16)((float)xv[e] * inv));
-    return o;
-}
 
 template <int MT, int MODE, bool NORM, int WAVES, int P, bool KSPLIT, bool XCHG = false, int UX = 1>
 // Argument order: what the PROLOGUE needs comes first, as plain pointers / scalars — weights, x and its two strides, the
@@ -1363,13 +1337,6 @@ static int launch_sg(const SgArgs& a, const SgRope& rp, hipStream_t st) {
     }
     TF_LAUNCH_CHECK();
     return TF_OK;
-}
-
-static bool sg_act_ok(const SgAct& s) { return s.sm > 0 && s.sk > 0 && (s.sm % 8) == 0 && (s.sk % 8) == 0; }
-
-static bool sg_shape_ok(int M, int N, int K, const SgAct& xa) {
-    return M >= 1 && M <= 32 && N >= 16 && (N % 16) == 0 && K >= 32 && (K % 32) == 0 && sg_act_ok(xa) &&
-           xa.sm <= 0x7fffffff && xa.sk <= 0x7fffffff;     // (the kernel takes x's two strides as 32-bit arguments)
 }
 
 // A/B knobs of the launch rule (tools/gemm_layout_ab.py): key 0 = rows from which two panels per wave are used (33:

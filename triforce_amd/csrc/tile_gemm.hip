@@ -16,6 +16,7 @@
 //   F32       the sums themselves
 #include "tile_common.h"
 #include "share_gemm.h"
+#include "share_shape.h"
 
 #ifndef TFL_PAIR_MIN
 #define TFL_PAIR_MIN 420     // panel pairs from which two panels share a workgroup
@@ -307,19 +308,10 @@ static int launch_share(const TflGemm& a, int tail_rows, int tail_per, hipStream
 // TF_ERANGE: not a shape of this form.
 template <typename T, int EPI>
 static int share_gemm(const TflGemm& a, hipStream_t st) {
-    const int panels = a.n >> 4, whole = panels / 256, left = (panels - 256 * whole) * 16, per = (left + 1023) / 1024 * 4;
-    if (!a.chunk_major || panels < 256) return TF_ERANGE;
-    if (EPI == TFL_EPI_IN && per > 0 && per < 16 && 256 * whole * 16 < a.n_raw) return TF_ERANGE;      // sums of squares need whole panels
-    // One panel and a rest of up to 4 rows, from the third (gate | up) or fifth row block on: every block reads the rest again at the price of a
-    // panel.  300 panels, K 4 096, gate | up, 64 / 128 / 256 rows here 26.5 / 48.6 / 92.9 us, panel by panel 25.1 / 39.9 / 76.4; other outputs
-    // 23.5 / 44.5 / 86.8 and 25.6 / 41.8 / 80.8
-    if (whole == 1 && per == 4 && a.rows > (EPI == TFL_EPI_GLU ? 32 : 64)) return TF_ERANGE;
-    // Rests of 9 to 12 rows a workgroup, and of 5 to 8 beside one panel of gate | up, cost as much as a panel of their own or more (gate | up deals
-    // them in pairs of rows, 32 bytes each): whole panels on fewer CUs.  us at one row, K 4 096, gate | up: 448 panels 13.0 panel by panel, 16.3
-    // with a rest, 12.9 on 224 CUs; 688 17.8, 21.9, 16.7; other outputs 448 12.5, 12.7, 12.5; 688 17.0, 18.3, 16.1; 900 21.7, 21.3 and, as 1 024,
-    // 22.7.
-    const bool up = per == 16 || (per == 12 && (EPI == TFL_EPI_GLU || whole <= 2)) || (per == 8 && EPI == TFL_EPI_GLU && whole == 1);
-    if (per == 0 || up) switch (up ? whole + 1 : whole) {
+    if (!a.chunk_major) return TF_ERANGE;
+    const ShareShape f = share_shape(a.n >> 4, EPI == TFL_EPI_GLU, EPI == TFL_EPI_IN ? a.n_raw : 0, a.rows);
+    const int left = f.left, per = f.rest;
+    if (per == 0) switch (f.each) {
         case 1: return launch_share<T, EPI, 1, false>(a, 0, 0, st);
         case 2: return launch_share<T, EPI, 2, false>(a, 0, 0, st);
         case 3: return launch_share<T, EPI, 3, false>(a, 0, 0, st);
@@ -330,7 +322,7 @@ static int share_gemm(const TflGemm& a, hipStream_t st) {
         case 8: return launch_share<T, EPI, 8, false>(a, 0, 0, st);
         default: return TF_ERANGE;
     }
-    switch (whole) {
+    switch (f.each) {
         case 1: return launch_share<T, EPI, 1, true>(a, left, per, st);
         case 2: return launch_share<T, EPI, 2, true>(a, left, per, st);
         case 3: return launch_share<T, EPI, 3, true>(a, left, per, st);

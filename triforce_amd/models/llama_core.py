@@ -71,11 +71,13 @@ class LlamaWeights:
     """Device-resident fp16 weights with fused qkv / gate-up matrices.
 
     rank / world_size select a Megatron-style shard (TP_layers.py:126-147): q/k/v/gate/up rows,
-    o/down columns; embed, norms and lm_head are replicated (TP_llama.py:91-94).
+    o/down columns; embed, norms and lm_head are replicated (TP_llama.py:91-94).  ``wide``: weights that the
+    one-workgroup-per-CU products take are packed for those alone (whole layers on one GPU: no exchange reads them).
     """
 
-    def __init__(self, cfg: LlamaConfig, device, rank=0, world_size=1):
+    def __init__(self, cfg: LlamaConfig, device, rank=0, world_size=1, wide=False):
         self.cfg, self.device, self.rank, self.world_size = cfg, torch.device(device), rank, world_size
+        self.wide = wide and world_size == 1 and ops.FUSE_MODE in ("all", "all2")
         self.L = cfg.num_hidden_layers
         self.H = cfg.num_attention_heads
         self.D = cfg.hidden_size // self.H
@@ -182,13 +184,16 @@ class LlamaWeights:
         if isinstance(self.lm_head, PL):
             return self
         tied = self.lm_head is self.embed
-        self.lm_head = PL(self.lm_head)
+
+        def use(name):
+            return name if self.wide else None
+        self.lm_head = PL(self.lm_head, wide=use("logits"))
         if tied:
             self.embed = self.lm_head.w
-        self.wqkv = [PL(w, rope=(self.H_local, self.D)) for w in self.wqkv]
-        self.wo = [PL(w) for w in self.wo]
-        self.wgu = [PL(w, split=2) for w in self.wgu]
-        self.wd = [PL(w) for w in self.wd]
+        self.wqkv = [PL(w, rope=(self.H_local, self.D), wide=use("qkv")) for w in self.wqkv]
+        self.wo = [PL(w, wide=use("residual")) for w in self.wo]
+        self.wgu = [PL(w, split=2, wide=use("swiglu")) for w in self.wgu]
+        self.wd = [PL(w, wide=use("residual")) for w in self.wd]
         return self
 
     def nbytes(self):

@@ -23,7 +23,7 @@ class LlamaForCausalLM:
         self.config = config
         self.device = torch.device(device)
         self.dtype = torch.float16
-        self.weights = LlamaWeights(config, self.device)
+        self.weights = LlamaWeights(config, self.device, wide=True)
         cos, sin = rope_tables_for(config)
         self.cos, self.sin = cos.to(self.device), sin.to(self.device)
         self.scale = softmax_scale_for(config.hidden_size // config.num_attention_heads)

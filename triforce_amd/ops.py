@@ -139,13 +139,30 @@ def _ensure_sg_workspace(device):
     _SG_WS[device] = ws
 
 
+def pack_weight_wide(w):
+    """pack_weight with the tiles chunk by chunk, [K/32][N/16][4 (g)][16 (i)][8]: the order of csrc/gemv_wide.hip."""
+    N, K = w.shape
+    assert N % 16 == 0 and K % 32 == 0 and w.dtype == _HALF
+    return w.view(N // 16, 16, K // 32, 4, 8).permute(2, 0, 3, 1, 4).contiguous()
+
+
+def _gate_up_eights(w):
+    """[gate | up] rows -> blocks of 8 gate | 8 up rows."""
+    n, k = w.shape[0] // 2, w.shape[1]
+    return torch.stack([w[:n].view(n // 8, 8, k), w[n:].view(n // 8, 8, k)], 1).reshape(2 * n, k)
+
+
 class PackedLinear:
     """A weight matrix with (on a HIP device) its pre-packed copy for the skinny decode GEMM.  ``w`` stays
     available for the >32-row prefill GEMMs (ops_rows).  ``split`` = number of equal row blocks that were
     fused (2 for gate|up) — each block is packed on its own so the SwiGLU kernel can pair them.  ``rope=(H, D)``
-    marks a fused q|k|v weight: a second packed copy in rotary-pair row order feeds tf_skinny_qkv_rope."""
+    marks a fused q|k|v weight: a second packed copy in rotary-pair row order feeds tf_skinny_qkv_rope.
+    ``wide``: what the weight is used for, where the one-workgroup-per-CU form may take it - "residual" (fp16 results, no norm), "swiglu" and "qkv"
+    (behind a norm) or "logits" (fp32) - and one copy in that form's order is all it gets if it does (``self.wide`` is None if not)."""
 
-    def __init__(self, w, split=1, pack=None, rope=None):
+    WIDE = {"residual": 0, "swiglu": 1, "logits": 2, "qkv": 3}
+
+    def __init__(self, w, split=1, pack=None, rope=None, wide=None):
         self.w = w
         self.N, self.K = w.shape
         self.split = split
@@ -153,21 +170,39 @@ class PackedLinear:
         ok = pack and (self.N // split) % 16 == 0 and self.K % 32 == 0
         if ok and w.is_cuda:
             _ensure_sg_workspace(w.device)
+        self.rope = rope
+        self.parts_n8 = self.wp_rope_n8 = None
+        narrow = n8_applies(self.N // split, self.K) if split == 2 or rope is not None else False
+        if wide == "qkv" and not (rope is not None and rope[1] % 32 == 0 and self.N == 3 * rope[0] * rope[1]):
+            wide = None
+        takes = ok and w.is_cuda and wide is not None and not narrow and hip.lib().tf_wide_gemm_takes(self.WIDE[wide], self.N, self.K) == 1
+        self.wide = wide if takes else None
+        if self.wide is not None:
+            self.parts = [pack_weight_wide(self._wide_rows())]
+            self.wp, self.wp_rope = (None, self.parts[0]) if wide == "qkv" else (None if wide == "swiglu" else self.parts[0], None)
+            return
         self.parts = [pack_weight(b) for b in w.chunk(split, dim=0)] if ok else None
         self.wp = self.parts[0] if (ok and split == 1) else None
-        self.rope = rope
         self.wp_rope = None
         if ok and rope is not None and rope[1] % 32 == 0 and self.N == 3 * rope[0] * rope[1]:
             self.wp_rope = pack_weight(w[rope_row_order(rope[0], rope[1], w.device)])
         # narrow-panel copies (few-panel shards only): gate|up streams, and the q|k|v weight in its 8-row rotary order
-        self.parts_n8 = self.wp_rope_n8 = None
         if ok and w.is_cuda and split == 2 and n8_applies(self.N // split, self.K):
             self.parts_n8 = [pack_weight_n8(b) for b in w.chunk(split, dim=0)]
         if self.wp_rope is not None and w.is_cuda and n8_applies(self.N, self.K):
             self.wp_rope_n8 = pack_weight_n8(w[rope_row_order_n8(rope[0], rope[1], w.device)])
 
+    def _wide_rows(self):
+        """The rows in the order of the one-workgroup-per-CU form."""
+        if self.wide == "qkv":
+            return self.w[rope_row_order(self.rope[0], self.rope[1], self.w.device)]
+        return _gate_up_eights(self.w) if self.wide == "swiglu" else self.w
+
     def refresh_(self):
         """Re-pack IN PLACE after ``self.w`` was modified in place (captured hipGraphs keep their pointers)."""
+        if self.wide is not None:
+            self.parts[0].copy_(pack_weight_wide(self._wide_rows()))
+            return self
         if self.parts is not None:
             for dst, blk in zip(self.parts, self.w.chunk(self.split, dim=0)):
                 dst.copy_(pack_weight(blk))
@@ -349,7 +384,7 @@ def linear(x, w, out_f32=False, ln=None, eps=0.0, resid=None, out=None, ss_in=No
     x / resid / out may be ``Act`` blocks (k-octet-major); an Act input gives an Act output unless ``out`` says
     otherwise (fp32 logits are always a row-major tensor)."""
     M = x.shape[0]
-    if isinstance(w, PackedLinear) and w.wp is not None and M <= SKINNY_MAX_ROWS and x.is_cuda:
+    if isinstance(w, PackedLinear) and w.wp is not None and M <= SKINNY_MAX_ROWS and x.is_cuda and (w.wide is None or (w.wide == "logits") == out_f32):
         assert x.dtype == _HALF and x.shape[1] == w.K
         if out is None:
             if out_f32 or not isinstance(x, Act):
@@ -370,9 +405,9 @@ def linear(x, w, out_f32=False, ln=None, eps=0.0, resid=None, out=None, ss_in=No
             yp, ysm, ysk = _ptr(out), out.stride(0), 8
         else:
             yp, ysm, ysk = _lay(out)
-        hip.check(hip.lib().tf_skinny_gemm_act(_ptr(w.wp), xp, xsm, xsk, _ptr(ln), float(eps), _ptr(ss_in), rp, rsm, rsk,
-                                               _ptr(ss_out), yp, ysm, ysk, M, w.N, w.K, 1 if out_f32 else 0, _stream()),
-                  "tf_skinny_gemm_act")
+        form = hip.lib().tf_skinny_gemm_act if w.wide is None else hip.lib().tf_wide_gemm_act
+        hip.check(form(_ptr(w.wp), xp, xsm, xsk, _ptr(ln), float(eps), _ptr(ss_in), rp, rsm, rsk, _ptr(ss_out), yp, ysm, ysk, M, w.N, w.K,
+                       1 if out_f32 else 0, _stream()), "tf_skinny_gemm_act" if w.wide is None else "tf_wide_gemm_act")
         return out
     assert ln is None and resid is None and out is None and ss_in is None and ss_out is None, \
         "fused linear needs the skinny kernel (ops.can_fuse)"
@@ -387,7 +422,7 @@ def mlp_act(h, wgu, ln=None, eps=0.0, ss_in=None):
     An Act input gives an Act output."""
     M = h.shape[0]
     if isinstance(wgu, PackedLinear) and wgu.parts is not None and wgu.split == 2 and M <= SKINNY_MAX_ROWS \
-            and h.is_cuda:
+            and h.is_cuda and (wgu.wide is None or ln is not None):
         I = wgu.N // 2
         act = Act.empty(M, I, h.device) if isinstance(h, Act) else torch.empty(M, I, dtype=_HALF, device=h.device)
         hp, hsm, hsk = _lay(h)
@@ -396,6 +431,10 @@ def mlp_act(h, wgu, ln=None, eps=0.0, ss_in=None):
             hip.check(hip.lib().tf_skinny_gemm_swiglu_n8(_ptr(wgu.parts_n8[0]), _ptr(wgu.parts_n8[1]), hp, hsm, hsk, _ptr(ln),
                                                          float(eps), _ptr(ss_in), ap, asm, ask, M, I, wgu.K, _stream()),
                       "tf_skinny_gemm_swiglu_n8")
+            return act
+        if wgu.wide is not None:
+            hip.check(hip.lib().tf_wide_gemm_swiglu_act(_ptr(wgu.parts[0]), hp, hsm, hsk, _ptr(ln), float(eps), _ptr(ss_in), ap, asm, ask, M, I, wgu.K,
+                                                        _stream()), "tf_wide_gemm_swiglu_act")
             return act
         hip.check(hip.lib().tf_skinny_gemm_swiglu_act(_ptr(wgu.parts[0]), _ptr(wgu.parts[1]), hp, hsm, hsk, _ptr(ln),
                                                       float(eps), _ptr(ss_in), ap, asm, ask, M, I, wgu.K, _stream()),
@@ -433,10 +472,10 @@ def qkv_rope(x, wqkv, ln, eps, cos, sin, positions, k_layer, v_layer, slot0, H, 
                                                   _ptr(v_layer), st, sh, int(slot0), _ptr(slot0_dev), rows, H, D, wqkv.K,
                                                   1 if rotate_k else 0, _stream()), "tf_skinny_qkv_rope_n8")
         return q
-    hip.check(hip.lib().tf_skinny_qkv_rope_act(_ptr(wqkv.wp_rope), xp, xsm, xsk, _ptr(ln), float(eps), _ptr(ss_in),
-                                               _ptr(cos), _ptr(sin), _ptr(positions), _ptr(q), _ptr(k_layer),
-                                               _ptr(v_layer), st, sh, int(slot0), _ptr(slot0_dev), rows, H, D, wqkv.K,
-                                               1 if rotate_k else 0, _stream()), "tf_skinny_qkv_rope_act")
+    form = hip.lib().tf_skinny_qkv_rope_act if wqkv.wide is None else hip.lib().tf_wide_qkv_rope_act
+    hip.check(form(_ptr(wqkv.wp_rope), xp, xsm, xsk, _ptr(ln), float(eps), _ptr(ss_in), _ptr(cos), _ptr(sin), _ptr(positions), _ptr(q), _ptr(k_layer),
+                   _ptr(v_layer), st, sh, int(slot0), _ptr(slot0_dev), rows, H, D, wqkv.K, 1 if rotate_k else 0, _stream()),
+              "tf_skinny_qkv_rope_act" if wqkv.wide is None else "tf_wide_qkv_rope_act")
     return q
 
 
@@ -648,7 +687,7 @@ def draft_model_struct(embed, ln1, wqkv, wo, ln2, wgu, wd, norm, lm_head, cos, s
     packed for the fused kernels (CPU tensors, odd shapes).  The struct holds raw pointers: keep the tensors alive."""
     L = len(wqkv)
     ws = list(wqkv) + list(wo) + list(wgu) + list(wd) + [lm_head]
-    if L > hip.TF_DRAFT_MAX_LAYERS or D != 64 or not all(isinstance(w, PackedLinear) and w.parts is not None for w in ws):
+    if L > hip.TF_DRAFT_MAX_LAYERS or D != 64 or not all(isinstance(w, PackedLinear) and w.parts is not None and w.wide is None for w in ws):
         return None
     if any(w.wp_rope is None for w in wqkv) or any(w.split != 2 for w in wgu) or not embed.is_cuda:
         return None

@@ -324,7 +324,7 @@ class GemmExchange:
         squares of the new x.  a / x: row-major tensors or ops.Act blocks (x's layout is also the staging layout)."""
         from .. import ops
         assert self._stage is not None, "GemmExchange.connect() has not run"
-        assert isinstance(w, ops.PackedLinear) and w.wp is not None
+        assert isinstance(w, ops.PackedLinear) and w.wp is not None and w.wide is None
         M = a.shape[0]
         assert tuple(x.shape) == (M, w.N) and a.shape[1] == w.K and self.fits(M, w.N)
         assert ss_out.dtype == torch.float32 and ss_out.is_contiguous() and ss_out.shape == (w.N // 16, 32)
