@@ -340,10 +340,11 @@ int tf_skinny_qkv_rope_act(const void* wqkv_packed, const void* x, int64_t xs_m,
                            void* q_out, void* k_cache, void* v_cache, int64_t stride_t, int64_t stride_h, int slot0,
                            const int32_t* slot0_dev, int M, int H, int D, int K, int rotate_k, void* stream);
 int tf_sg_tune(int key, int value);
-/* The same products for wide weights, one workgroup per CU (csrc/gemv_wide.hip): operands, rounding points and results as above (the K sum in another order),
- * weights packed chunk-major, [K/32][N/16][64][8], the q|k|v rows in the rotary order of tf_skinny_qkv_rope, gate and up in blocks of 8 gate | 8 up rows
- * (N = 2 I).  tf_wide_gemm_takes(mode, N, K): 1 for a size of this form, 0 for others.  mode 0: fp16 with a residual and sums of squares (no norm), 1: SwiGLU, 2: fp32
- * (logits), 3: q|k|v.  TF_ERANGE otherwise.  16-byte aligned x; 8-byte aligned fp16 results and residuals. */
+/* The same products for wide weights, one workgroup per CU (csrc/gemv_wide.hip): operands, rounding points and bits as above; weights packed chunk-major,
+ * [K/32][N/16][64][8], the chunks of each of 8 (mode 0) or 4 equal parts of K (rounded up to whole chunks) turned by twice the part's number: chunk o
+ * of part p of n chunks lies at (o + 2 p) % n of the part.  q|k|v rows in the rotary order of tf_skinny_qkv_rope, gate and up in blocks of 8 gate |
+ * 8 up rows (N = 2 I).  tf_wide_gemm_takes(mode, N, K): 1 for a size of this form, 0 for others.  mode 0: fp16 with a residual and sums of squares (no
+ * norm), 1: SwiGLU, 2: fp32 (logits), 3: q|k|v.  TF_ERANGE otherwise.  16-byte aligned x; 8-byte aligned fp16 results and residuals. */
 int tf_wide_gemm_takes(int mode, int N, int K);
 int tf_wide_gemm_act(const void* w_packed, const void* x, int64_t xs_m, int64_t xs_k, const void* ln_w, float eps, const float* ss_in,
                      const void* resid, int64_t rs_m, int64_t rs_k, float* ss_out, void* y, int64_t ys_m, int64_t ys_k, int M, int N, int K,

@@ -26,8 +26,8 @@ struct SgRope {                       // arguments of the RoPE + KV-append epilo
 __device__ __forceinline__ half8 sg_normalise(half8 xv, half8 wv, float inv) {
     half8 o;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = hmul_rn(wv[e], (h16)((float)xv[e] * inv));
-    return o;
+    for (int e = 0; e < 8; ++e) o[e] = (h16)((float)xv[e] * inv);
+    return wv * o;
 }
 
 static bool sg_act_ok(const SgAct& s) { return s.sm > 0 && s.sk > 0 && (s.sm % 8) == 0 && (s.sk % 8) == 0; }

@@ -5,31 +5,34 @@
 
 // Bound by the weight stream.  A workgroup per panel (gemv.hip) leaves a few CUs with a panel more than the rest, reads x once per panel and begins with one
 // batch of weights a wave.  Here all CUs have the same share (share_shape.h) and read x once.
-// us in a graph over weights that come from memory, panel by panel -> here, 7 / 17 / 32 rows (a read of the same bytes):
-//   q|k|v   12 288 x  4 096  21.5 -> 16.9, 27.0 -> 19.3, 28.5 -> 19.6 (16.5)      15 360 x 5 120  27.2 -> 26.5, 31.9 -> 27.5 (24.8)
-//   o        4 096 x  4 096   8.6 ->  7.7,  9.8 ->  8.8, 11.5 -> 10.5 (6.7)
-//   gate|up 22 016 x  4 096  32.4 -> 30.9, 40.6 -> 33.1, 41.7 -> 32.3 (28.1)      27 648 x 5 120  49.9 -> 44.5, 53.6 -> 46.5 (43.1)
-//   down     4 096 x 11 008  18.2 -> 16.5, 19.7 -> 18.8, 23.0 -> 22.4 (15.0)
-//   logits  32 000 x  4 096  48.6 -> 41.2, 53.4 -> 42.2, 56.3 -> 42.2 (40.1)      32 000 x 5 120  54.3 -> 50.4, 63.8 -> 52.2 (49.6)
-// A retrieval verification of four 7B layers 476 -> 441 us, the one over 122K tokens 1 604 -> 1 576.
+// us in a graph over weights that come from memory, panel by panel -> here, 7 / 17 rows, k-octet-major x (a read of the same bytes):
+//   q|k|v   12 288 x  4 096  21.2 -> 17.5, 26.6 -> 20.8 (16.5)      15 360 x 5 120  27.7 -> 27.4, 33.4 -> 29.3 (24.8)
+//   o        4 096 x  4 096   8.5 ->  7.8,  9.8 ->  9.0 (6.7)
+//   gate|up 22 016 x  4 096  32.1 -> 31.1, 40.2 -> 33.2 (28.1)      27 648 x 5 120  49.6 -> 45.1, 53.3 -> 46.9 (43.1)
+//   down     4 096 x 11 008  17.6 -> 16.9, 21.0 -> 18.7 (15.0)
+//   logits  32 000 x  4 096  48.4 -> 42.0, 53.3 -> 43.3 (40.1)      32 000 x 5 120  52.9 -> 52.0, 64.2 -> 53.1 (49.6)
 //
-// Weights are packed chunk-major, [K/32][N/16][64][8]: the chip reads one moving window per wave index.  Eight waves split K.  A wave asks for two batches
-// of chunks (weights, operand, norm weights) before anything waits, the norm's sums of squares in front of them, so that the fold of those runs under
-// the stream; after that a batch is asked for whenever one has been used.
-template <int MODE, bool NORM, int P, bool TAIL, int MT, int U>
-__global__ __launch_bounds__(512, 2) void gemv_wide_kernel(const h16* __restrict__ wp, const h16* __restrict__ x, const float* __restrict__ ss_in,
+// The bits are those of the panel form: WAVES parts of K, as many as that form has for these sizes (8 for o and down, 4 for the others), each summed chunk by
+// chunk, and the parts in their order.  (Eight parts everywhere and another order of the chunks: q|k|v 16.9, o 7.7, gate|up 30.9, down 16.5, but which tokens
+// top-p keeps depends on last digits of the logits.)
+// Weights are packed chunk-major, [K/32][N/16][64][8], so that the chip reads one moving window per wave index; as the waves' ranges of K start a power of
+// two apart, the chunks of wave w's range lie turned by 2 w in it (o 8.4 us without, 8.0 with).  A wave asks for two batches of chunks (weights,
+// operand, norm weights) before anything waits, the norm's sums of squares in front of them, so that the fold of those runs under the stream; after
+// that a batch is asked for whenever one has been used.
+template <int MODE, bool NORM, int P, bool TAIL, int MT, int U, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, WAVES / 4) void gemv_wide_kernel(const h16* __restrict__ wp, const h16* __restrict__ x, const float* __restrict__ ss_in,
                                                            const h16* __restrict__ ln_w, int K, int M, int x_sm, int x_sk, float eps, int N,
                                                            const h16* resid, SgAct ra, void* yv, SgAct ya, SgRope rp, float* __restrict__ ss_out,
                                                            int tail_rows, int tail_per) {
-    constexpr int WAVES = 8, NP = P + (TAIL ? 1 : 0), CUS = 256, G = 32, SSB = 8;
+    constexpr int NP = P + (TAIL ? 1 : 0), CUS = 256, G = 4 * WAVES, SSB = 256 / G;
     static_assert(!TAIL || MODE == SG_F32 || MODE == SG_GATEUP, "rotation and sums of squares need whole panels");
     extern __shared__ __align__(16) char wide_smem[];
     f32x4 (*part)[NP * MT][64] = reinterpret_cast<f32x4 (*)[NP * MT][64]>(wide_smem);
-    __shared__ float red[NORM ? MT : 1][G][16];
+    __shared__ float red[NORM ? MT : 1][G][16];             // (G: groups of 16 threads)
     const int cu = blockIdx.x, tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15;
     const int npan = N >> 4, panel0 = cu * P, chunks = K >> 5;
     const int per = (chunks + WAVES - 1) / WAVES, c_beg = wave * per, n_own = min(chunks, c_beg + per) - c_beg;
-    const int rot = n_own > 0 ? 2 * wave % n_own : 0;        // (the waves' ranges start a power of two apart)
+    const int rot = n_own > 0 ? 2 * wave % n_own : 0;
     const int64_t wstep = (int64_t)npan * 512, xstep = 4 * (int64_t)x_sk;
     const h16* w_at[NP];
 #pragma unroll
@@ -48,13 +51,12 @@ __global__ __launch_bounds__(512, 2) void gemv_wide_kernel(const h16* __restrict
     auto load = [&](Batch& b, int c0) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            int c = min(c0 + u, n_own - 1) + rot;
-            c = c_beg + (c >= n_own ? c - n_own : c);
+            const int o = min(c0 + u, n_own - 1), c = c_beg + o, at = c_beg + (o + rot >= n_own ? o + rot - n_own : o + rot);
 #pragma unroll
             for (int t = 0; t < MT; ++t) b.x[u][t] = load_half8(x_at[t] + xstep * c);
             if constexpr (NORM) b.ln[u] = load_half8(ln_w + 32 * c + 8 * g);
 #pragma unroll
-            for (int p = 0; p < NP; ++p) b.w[u][p] = load_half8_stream(w_at[p] + wstep * c);
+            for (int p = 0; p < NP; ++p) b.w[u][p] = load_half8_stream(w_at[p] + wstep * at);
         }
     };
     float inv[MT];
@@ -116,8 +118,7 @@ __global__ __launch_bounds__(512, 2) void gemv_wide_kernel(const h16* __restrict
             for (int t = 0; t < MT; ++t) {
                 float s = 0.f;
 #pragma unroll
-                for (int j = 0; j < SSB; ++j)
-                    if (pg + j * G < nparts) s += ssv[t][j];
+                for (int j = 0; j < SSB; ++j) s += pg + j * G < nparts ? ssv[t][j] : 0.f;
                 for (int p = pg + SSB * G; p < nparts; p += G) s += ss_in[(int64_t)p * 32 + 16 * t + m16];
                 red[t][pg][m16] = s;
             }
@@ -130,16 +131,17 @@ __global__ __launch_bounds__(512, 2) void gemv_wide_kernel(const h16* __restrict
 #pragma unroll
                     for (int e = 0; e < 8; ++e) s = fmaf((float)v[e], (float)v[e], s);
                 }
-                red[t][4 * wave + g][i] = s;
+                s = rows_sum(s);
+                if (g == 0) red[t][wave][i] = s;
             }
         }
         __syncthreads();
+        const int groups = ss_in ? G : WAVES;
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             float s = 0.f;
-#pragma unroll
-            for (int k = 0; k < G / 4; ++k) s += red[t][(G / 4) * g + k][i];
-            inv[t] = 1.0f / sqrtf(rows_sum(s) / (float)K + eps);
+            for (int k = 0; k < groups; ++k) s += red[t][k][i];
+            inv[t] = 1.0f / sqrtf(s / (float)K + eps);
         }
     }
     half4 cs_end = {0, 0, 0, 0}, sn_end = {0, 0, 0, 0};
@@ -221,17 +223,17 @@ __global__ __launch_bounds__(512, 2) void gemv_wide_kernel(const h16* __restrict
             for (int r = 0; r < 4; ++r) dst[r] = (float)(h16)s[r];
         } else if constexpr (MODE == SG_PLAIN) {
             half4 o;
-            float q = 0.f;
+            float y[4];
             if (resid && j != wave) with = residual(panel, min(m, M - 1));
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 o[r] = (h16)s[r];
                 if (resid) o[r] = hadd_rn(with[r], o[r]);
-                q = fmaf((float)o[r], (float)o[r], q);
+                y[r] = live ? (float)o[r] : 0.f;
             }
             if (live) *reinterpret_cast<half4*>((h16*)yv + (int64_t)m * ya.sm + (int64_t)(2 * panel + (g >> 1)) * ya.sk + 4 * (g & 1)) = o;
             if (ss_out) {                                    // this panel's share of sum(y^2) per row, for the next norm
-                q = rows_sum(live ? q : 0.f);
+                const float q = rows_sum(y[0] * y[0] + y[1] * y[1] + y[2] * y[2] + y[3] * y[3]);
                 if (g == 0) ss_out[(int64_t)panel * 32 + m] = q;
             }
         } else {                                             // q and k panels hold rows d0..d0+7 | d0+D/2..d0+D/2+7 of a head
@@ -290,18 +292,19 @@ static ShareShape wide_shape(int mode, int N, int K) {
 
 template <int MODE, bool NORM, int P, bool TAIL, int MT>
 static int launch_wide_rows(const WideArgs& a, const ShareShape& f, hipStream_t st) {
-    constexpr int NP = P + (TAIL ? 1 : 0), LDS = 8 * NP * MT * 64 * (int)sizeof(f32x4);
-    // Chunks of a batch: two batches of 4 to 16 KB a wave, what the registers hold.  More of them (4 up to six tiles, 3 up to nine) gain nothing or cost
-    // (13B q|k|v 26.5 -> 28.1 us), fewer cost (gate | up 30.9 -> 31.6).
-    constexpr int U = NP <= 2 ? 4 : NP * MT <= (NORM ? 11 : 14) ? 2 : 1;
+    constexpr int WAVES = MODE == SG_PLAIN ? 8 : 4;
+    constexpr int NP = P + (TAIL ? 1 : 0), LDS = WAVES * NP * MT * 64 * (int)sizeof(f32x4);
+    // Chunks of a batch.  More gain nothing (q|k|v, three panels, six chunks 17.5 -> 18.3 us; gate | up, six tiles, three 31.1 -> 31.8).
+    constexpr int U = WAVES == 8 ? 4 : NP <= 2 ? 8 : NP <= 4 ? 4 : 2;
     static_assert(LDS <= 152 * 1024, "one workgroup's partial tiles");
+    auto* k = gemv_wide_kernel<MODE, NORM, P, TAIL, MT, U, WAVES>;
     if (LDS > 60 * 1024) {
-        const hipError_t e = hipFuncSetAttribute((const void*)gemv_wide_kernel<MODE, NORM, P, TAIL, MT, U>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
         if (e != hipSuccess) return (int)e;
     }
-    hipLaunchKernelGGL((gemv_wide_kernel<MODE, NORM, P, TAIL, MT, U>), dim3(TAIL ? 256 : (a.N / 16 + P - 1) / P), dim3(512), LDS, st, (const h16*)a.wp,
-                       (const h16*)a.x, a.ss_in, (const h16*)a.ln_w, a.K, a.M, (int)a.xa.sm, (int)a.xa.sk, a.eps, a.N, (const h16*)a.resid, a.ra, a.y,
-                       a.ya, a.rp, a.ss_out, f.left, f.rest);
+    hipLaunchKernelGGL(k, dim3(TAIL ? 256 : (a.N / 16 + P - 1) / P), dim3(64 * WAVES), LDS, st, (const h16*)a.wp, (const h16*)a.x, a.ss_in,
+                       (const h16*)a.ln_w, a.K, a.M, (int)a.xa.sm, (int)a.xa.sk, a.eps, a.N, (const h16*)a.resid, a.ra, a.y, a.ya, a.rp, a.ss_out, f.left,
+                       f.rest);
     TF_LAUNCH_CHECK();
     return TF_OK;
 }

@@ -102,7 +102,7 @@ class LlamaForCausalLM:
         fused = mode in ("all", "all2")
         # the fused layer keeps residual stream / attention output / SwiGLU output k-octet-major (ops.Act): the GEMMs' B
         # operand is then read in 256-byte runs (ops.py, "activation layouts")
-        packed = fused and ops.act_packed(q_len)
+        packed = fused and ops.act_packed(q_len, W.wd[0].wide is not None)
         x = ops.embed_rows(W.embed, input_ids, packed)   # (q, hidden) fp16 gather
         ss = ops.ss_buffer(x.shape[1], x.device) if mode == "all" else None     # sum(x^2) hand-off between GEMMs
         d = None

@@ -139,11 +139,21 @@ def _ensure_sg_workspace(device):
     _SG_WS[device] = ws
 
 
-def pack_weight_wide(w):
-    """pack_weight with the tiles chunk by chunk, [K/32][N/16][4 (g)][16 (i)][8]: the order of csrc/gemv_wide.hip."""
+def pack_weight_wide(w, parts):
+    """pack_weight with the tiles chunk by chunk, [K/32][N/16][4 (g)][16 (i)][8], each of ``parts`` parts of K turned by twice its number
+    (csrc/gemv_wide.hip)."""
     N, K = w.shape
     assert N % 16 == 0 and K % 32 == 0 and w.dtype == _HALF
-    return w.view(N // 16, 16, K // 32, 4, 8).permute(2, 0, 3, 1, 4).contiguous()
+    chunks = K // 32
+    per = -(-chunks // parts)
+    tiles = w.view(N // 16, 16, chunks, 4, 8).permute(2, 0, 3, 1, 4)
+    out = torch.empty(tiles.shape, dtype=w.dtype, device=w.device)
+    for p in range(parts):
+        a, b = p * per, min(chunks, (p + 1) * per)
+        turn = 2 * p % (b - a)
+        out[a + turn:b] = tiles[a:b - turn]
+        out[a:a + turn] = tiles[b - turn:b]
+    return out
 
 
 def _gate_up_eights(w):
@@ -178,7 +188,7 @@ class PackedLinear:
         takes = ok and w.is_cuda and wide is not None and not narrow and hip.lib().tf_wide_gemm_takes(self.WIDE[wide], self.N, self.K) == 1
         self.wide = wide if takes else None
         if self.wide is not None:
-            self.parts = [pack_weight_wide(self._wide_rows())]
+            self.parts = [self._pack_wide()]
             self.wp, self.wp_rope = (None, self.parts[0]) if wide == "qkv" else (None if wide == "swiglu" else self.parts[0], None)
             return
         self.parts = [pack_weight(b) for b in w.chunk(split, dim=0)] if ok else None
@@ -192,16 +202,17 @@ class PackedLinear:
         if self.wp_rope is not None and w.is_cuda and n8_applies(self.N, self.K):
             self.wp_rope_n8 = pack_weight_n8(w[rope_row_order_n8(rope[0], rope[1], w.device)])
 
-    def _wide_rows(self):
-        """The rows in the order of the one-workgroup-per-CU form."""
+    def _pack_wide(self):
+        if self.wide == "residual":
+            return pack_weight_wide(self.w, 8)
         if self.wide == "qkv":
-            return self.w[rope_row_order(self.rope[0], self.rope[1], self.w.device)]
-        return _gate_up_eights(self.w) if self.wide == "swiglu" else self.w
+            return pack_weight_wide(self.w[rope_row_order(self.rope[0], self.rope[1], self.w.device)], 4)
+        return pack_weight_wide(_gate_up_eights(self.w) if self.wide == "swiglu" else self.w, 4)
 
     def refresh_(self):
         """Re-pack IN PLACE after ``self.w`` was modified in place (captured hipGraphs keep their pointers)."""
         if self.wide is not None:
-            self.parts[0].copy_(pack_weight_wide(self._wide_rows()))
+            self.parts[0].copy_(self._pack_wide())
             return self
         if self.parts is not None:
             for dst, blk in zip(self.parts, self.w.chunk(self.split, dim=0)):
@@ -232,15 +243,18 @@ ACT_LAYOUT = _os.environ.get("TRIFORCE_ACT_LAYOUT", "auto")
 # retrieval verify 9 198 -> 8 319 us, target verify 25 640 -> 24 578; 7B gamma = 16 retrieval verify 5 287 -> 5 024; at
 # 7 rows 3 345 -> 3 303 (1 %) and the tensor-parallel shard's eager 1-row step LOSES (host cost of the Act wrappers)
 ACT_PACKED_MIN_ROWS = int(_os.environ.get("TRIFORCE_ACT_PACKED_MIN_ROWS", "17"))
+# Wide weights (csrc/gemv_wide.hip) from 4 rows: their waves read the same columns of all rows together, rows a power of two apart in the row-major
+# form.  us of a 7B layer's four products, rows -> octets: 1 row the same, 7 rows 74.4 -> 73.3, 12 rows 80.0 -> 74.7.
+ACT_PACKED_MIN_ROWS_WIDE = 4
 
 
-def act_packed(rows):
+def act_packed(rows, wide=False):
     """Should a decode forward of ``rows`` rows keep its activations k-octet-major?"""
     if ACT_LAYOUT == "packed":
         return True
     if ACT_LAYOUT == "rows":
         return False
-    return rows >= ACT_PACKED_MIN_ROWS
+    return rows >= (min(ACT_PACKED_MIN_ROWS, ACT_PACKED_MIN_ROWS_WIDE) if wide else ACT_PACKED_MIN_ROWS)
 
 
 class Act:
