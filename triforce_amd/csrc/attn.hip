@@ -63,7 +63,7 @@
 #define FUSED_MERGE_BIG_MAX_WGS 256
 #endif
 #ifndef TF_ATTN_EAGER_TILES
-#define TF_ATTN_EAGER_TILES 16 // splits of up to this many 16-key tiles per wave use the unconditional-prefetch loop
+#define TF_ATTN_EAGER_TILES 128 // splits of up to this many 16-key tiles per wave use the unconditional-prefetch loop
 #endif
 
 // Two deeper load pipelines, MEASURED AND REJECTED in round 3 (profiles/r03_attn_pipeline_ab.jsonl; cold-cache hipGraph
@@ -93,6 +93,16 @@ __device__ __forceinline__ void st_agent(float* p, float v) {
 }
 __device__ __forceinline__ float ld_agent(const float* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Two neighbours at once (8-byte aligned).
+__device__ __forceinline__ void st_agent2(float* p, float a, float b) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), (uint64_t)__float_as_uint(b) << 32 | __float_as_uint(a), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f32x4 ld_agent4(const float* p) {
+    const uint64_t* u = reinterpret_cast<const uint64_t*>(p);
+    const uint64_t a = __hip_atomic_load(u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), b = __hip_atomic_load(u + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return f32x4{__uint_as_float((uint32_t)a), __uint_as_float((uint32_t)(a >> 32)), __uint_as_float((uint32_t)b), __uint_as_float((uint32_t)(b >> 32))};
 }
 
 // max over the 4 lane groups of a wave (lanes i, i^16, i^32, i^48) on the VALU: v_permlane{32,16}_swap + v_max instead of
@@ -351,7 +361,7 @@ __device__ __forceinline__ void attn_split_body(
     // barrier — the merge of the waves' partial results
     constexpr int HALVES = NW > 4 ? 2 : 1, DH = D / HALVES, NTH = NT / HALVES;
     constexpr bool ROWS = TF_ATTN_ROW_LOADS > 0 && NW == 4;
-    constexpr size_t MERGE_BYTES = sizeof(float) * ((size_t)NW * 16 * (DH + 1) + 2 * NW * 16);
+    constexpr size_t MERGE_BYTES = sizeof(float) * ((size_t)NW * 16 * (DH + 4) + 2 * NW * 16);
     constexpr size_t STAGE_BYTES = ROWS ? (size_t)NW * 2 * 16 * (D + 8) * sizeof(h16) : 0;
     __shared__ __attribute__((aligned(16))) unsigned char sm_raw[MERGE_BYTES > STAGE_BYTES ? MERGE_BYTES : STAGE_BYTES];
     h16* stage = reinterpret_cast<h16*>(sm_raw) + (size_t)wave * 2 * 16 * (D + 8);
@@ -381,10 +391,9 @@ __device__ __forceinline__ void attn_split_body(
     // Two forms of the same two-tiles-deep loop.  A load under `if (t1 < t_end)` makes the compiler assume the worst
     // case at the use of the OLDER tile — "no younger load was issued" — so it waits vmcnt(7..0) there, i.e. for the
     // prefetch it has just issued: the wave runs one tile deep.  Issuing the run-ahead loads unconditionally (past the
-    // last tile they re-read it) gives the intended vmcnt(15..8).  Measured (tools/attn_merge_ab.py): short streams gain
-    // (7B retrieval verify 21.0 -> 20.2 us, 4-head TP shard 14.3 -> 13.6, draft-sized 6.9 -> 6.5) but the 125K-key
-    // streams, already bandwidth-bound with 8 MB in flight chip-wide, LOSE 0.7 % (32 heads) to 4 % (16 heads x 17 rows)
-    // with twice as much in flight — so the form is chosen by the length of the wave's stream.
+    // last tile they re-read it) gives the intended vmcnt(15..8).  us, conditional -> unconditional, 7 rows, 32 heads: 12 295 keys 41.6 -> 39.2, 32 768
+    // 89.0 -> 86.5; 16 heads of 65 000 113.4 -> 104.4, 4 of 124 935 50.4 -> 48.0.  From some 130 tiles a wave on the stream is bound by bandwidth either
+    // way (32 heads: 90 000 keys 238 both, 124 935 320 -> 330): the form is chosen by the length of the wave's stream.
     static_assert(NW == 4 || (DEEP == 0 && (QT == 1 ? TF_ATTN_RING_Q1 : TF_ATTN_RING_Q2) == 0), "deep / ring forms: 4 waves");
     int t = t_begin + wave;
     if constexpr (DEEP > 0) {
@@ -460,10 +469,12 @@ __device__ __forceinline__ void attn_split_body(
 #undef ATTN_LOAD_TILE
     // ---- merge the NW waves of this split through LDS, one q-tile at a time (8 waves: one half of D at a time, so the
     // staging stays under the 64 KiB static limit) ----
-    float (*sm_o)[16][DH + 1] = reinterpret_cast<float (*)[16][DH + 1]>(sm_raw);
-    float (*sm_m)[16] = reinterpret_cast<float (*)[16]>(sm_raw + sizeof(float) * (size_t)NW * 16 * (DH + 1));
+    // Every wave weighs its own accumulators, with the maxima of all, before they go to LDS in 16-byte pieces; what is left is a sum in wave order, for the
+    // rows that there are, stored 8 bytes a piece (4-byte elements weighed one by one by their reader, all 16 rows of a tile: 7 rows of 32 heads
+    // over 264 / 1 000 / 4 103 keys 9.1 / 11.8 / 19.8 us, now 7.9 / 9.9 / 17.8; 16 rows over 4 112 keys 21.7 -> 19.0).
+    float (*sm_o)[16][DH + 4] = reinterpret_cast<float (*)[16][DH + 4]>(sm_raw);
+    float (*sm_m)[16] = reinterpret_cast<float (*)[16]>(sm_raw + sizeof(float) * (size_t)NW * 16 * (DH + 4));
     float (*sm_l)[16] = sm_m + NW;
-    if constexpr (ROWS) __syncthreads();               // another wave may still be reading its staging tile where this one is about to write
     float* ws_o = ws;
     float* ws_m = ws + (int64_t)H * nsplit * QR * D;
     float* ws_l = ws_m + (int64_t)H * nsplit * QR;
@@ -472,45 +483,62 @@ __device__ __forceinline__ void attn_split_body(
     for (int qt = 0; qt < QT; ++qt) {
         float lsum = st.l[qt];
         lsum = rows_sum(lsum);
+        if (ROWS || qt > 0) __syncthreads();           // another wave may still be reading what this one is about to overwrite
+        if (g == 0) {
+            sm_m[wave][li] = st.m[qt];
+            sm_l[wave][li] = lsum;
+        }
+        __syncthreads();
+        float mm = sm_m[0][li];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) mm = fmaxf(mm, sm_m[w][li]);
+        const float own = __expf(st.m[qt] - mm);
+        if (wave == 0 && g == 0 && qt * 16 + li < sq) {
+            float lw = 0.f;                            // (wave order)
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const float ww = __expf(sm_m[w][li] - mm);
+                lw = (w == 0) ? sm_l[w][li] * ww : lw + sm_l[w][li] * ww;
+            }
+            float *to_m = &ws_m[pbase + qt * 16 + li], *to_l = &ws_l[pbase + qt * 16 + li];
+            if (tickets == nullptr) {
+                *to_m = mm;
+                *to_l = lw;
+            } else {
+                st_agent(to_m, mm);
+                st_agent(to_l, lw);
+            }
+        }
+        const int rows = min(16, sq - qt * 16);
 #pragma unroll
         for (int hv = 0; hv < HALVES; ++hv) {
+            if (hv > 0) __syncthreads();
 #pragma unroll
-            for (int tt = 0; tt < NTH; ++tt)
+            for (int tt = 0; tt < NTH; ++tt) {
+                f32x4 o = st.acc[qt][hv * NTH + tt];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) sm_o[wave][li][16 * tt + 4 * g + r] = st.acc[qt][hv * NTH + tt][r];
-            if (g == 0) {
-                sm_m[wave][li] = st.m[qt];
-                sm_l[wave][li] = lsum;
+                for (int r = 0; r < 4; ++r) o[r] *= own;
+                *reinterpret_cast<f32x4*>(&sm_o[wave][li][16 * tt + 4 * g]) = o;
             }
             __syncthreads();
-            for (int e = tid; e < 16 * DH; e += 64 * NW) {
-                const int qq = e / DH, dl = e - qq * DH, d = hv * DH + dl;
-                float mm = sm_m[0][qq];
+            for (int e = tid; e < rows * (DH / 4); e += 64 * NW) {
+                const int qq = e / (DH / 4), d4 = e - qq * (DH / 4);
+                // sum over the waves in wave order: ((a0 w0 + a1 w1) + a2 w2) + a3 w3
+                f32x4 o = *reinterpret_cast<const f32x4*>(&sm_o[0][qq][4 * d4]);
 #pragma unroll
-                for (int w = 1; w < NW; ++w) mm = fmaxf(mm, sm_m[w][qq]);
-                // sum over the waves in wave order (for NW = 4 the very expression of round 2: ((a0 w0 + a1 w1) + a2 w2) + a3 w3)
-                float o = 0.f, lw = 0.f;
+                for (int w = 1; w < NW; ++w) {
+                    const f32x4 v = *reinterpret_cast<const f32x4*>(&sm_o[w][qq][4 * d4]);
 #pragma unroll
-                for (int w = 0; w < NW; ++w) {
-                    const float ww = __expf(sm_m[w][qq] - mm);
-                    o = (w == 0) ? sm_o[w][qq][dl] * ww : o + sm_o[w][qq][dl] * ww;
-                    lw = (w == 0) ? sm_l[w][qq] * ww : lw + sm_l[w][qq] * ww;
+                    for (int r = 0; r < 4; ++r) o[r] += v[r];
                 }
+                float* to = ws_o + (pbase + qt * 16 + qq) * D + hv * DH + 4 * d4;
                 if (tickets == nullptr) {
-                    ws_o[(pbase + qt * 16 + qq) * D + d] = o;
-                    if (d == 0) {
-                        ws_m[pbase + qt * 16 + qq] = mm;
-                        ws_l[pbase + qt * 16 + qq] = lw;
-                    }
-                } else {                                   // one-launch form: write-through (sc1) stores, see below
-                    st_agent(&ws_o[(pbase + qt * 16 + qq) * D + d], o);
-                    if (d == 0) {
-                        st_agent(&ws_m[pbase + qt * 16 + qq], mm);
-                        st_agent(&ws_l[pbase + qt * 16 + qq], lw);
-                    }
+                    *reinterpret_cast<f32x4*>(to) = o;
+                } else {                               // one-launch form: write-through (sc1) stores, see below
+                    st_agent2(to, o[0], o[1]);
+                    st_agent2(to + 2, o[2], o[3]);
                 }
             }
-            __syncthreads();
         }
     }
     if (tickets == nullptr) return;                    // two-launch form: attn_combine_kernel merges the splits
@@ -633,7 +661,7 @@ __device__ __forceinline__ void attn_split_body(
         for (int s = 0; s < FUSED_MERGE_MAX_SPLITS; ++s) {
             if (s < nsplit) {
                 const float* xp = ws_o + (hbase + (int64_t)s * QR + r) * D + 4 * d4;
-                px[s] = f32x4{ld_agent(xp), ld_agent(xp + 1), ld_agent(xp + 2), ld_agent(xp + 3)};
+                px[s] = ld_agent4(xp);
                 pm[s] = ld_agent(&ws_m[hbase + (int64_t)s * QR + r]);
                 pl[s] = ld_agent(&ws_l[hbase + (int64_t)s * QR + r]);
             } else {
