@@ -30,6 +30,25 @@ int tfh_connect(const void* embed, const int64_t* ids, int vocab, const float* e
                 const float* out, const float* mix, const float* in, const float* norm_w, float* x, int streams, int keep, void* h,
                 int64_t ld_h, int64_t h_oct, int rows, int width, int width_real, float eps, int dtype, void* stream);
 
+/* tfh_connect of rows whose next reader is a wide product, in that product's launch (bfloat16, one row of up to 4 streams of up to 4 096): every
+ * workgroup makes the normed row for itself, beside the beginning of its weights.  x_out (NULL: the streams are not kept) is another block than x;
+ * product->x is not read.  epilogue TFL_EPI_F32 or TFL_EPI_GLU, chunk-major weights.  TF_ERANGE: not a size of this form (nothing launched);
+ * tfh_connect_gemm_takes says so beforehand. */
+typedef struct TfhConnect {
+    const float* y;                 /* [rows], row stride ld_y */
+    const float* out;               /* [streams] */
+    const float* mix;               /* [streams][streams] */
+    const float* in;                /* [streams] */
+    const float* norm_w;
+    const float* x;                 /* [rows][streams][width] */
+    float* x_out;
+    int64_t ld_y;
+    int32_t streams, width, width_real;
+    float eps;
+} TfhConnect;
+int tfh_connect_gemm_takes(int rows, int streams, int width, int n, int k, int epilogue);
+int tfh_connect_gemm(const TfhConnect* f, const TflGemm* product, int epilogue, void* stream);
+
 /* ---- prefill ----------------------------------------------------------------------------------------------------------- */
 
 /* Queries and keys of new tokens: per head x / rms * norm, then entries i and i + half of the first 2 * half turn at pos[token];

@@ -27,6 +27,23 @@ int tfl_finish(const void* embed, const int64_t* ids, int vocab, const void* y, 
                const float* step, const float* norm_w, float* x, void* h, int64_t ld_h, int64_t h_oct, int rows, int width,
                int width_real, float eps, int dtype, void* stream);
 
+/* tfl_finish of rows whose next reader is a wide product, in that product's launch (bfloat16, up to 2 rows of up to 4 096): every workgroup makes the normed
+ * rows for itself, beside the beginning of its weights.  x_out = x + y / rms(y) * y_w [+ step] is another block than x; product->x is not read.
+ * epilogue TFL_EPI_IN or TFL_EPI_F32, chunk-major weights.  TF_ERANGE: not a size of this form (nothing launched); tfl_finish_gemm_takes says so beforehand. */
+typedef struct TflFinish {
+    const float* y;                 /* [rows], row stride ld_y */
+    const float* y_w;
+    const float* step;              /* NULL: none */
+    const float* norm_w;
+    const float* x;                 /* [rows][width] */
+    float* x_out;
+    int64_t ld_y;
+    int32_t width, width_real;
+    float eps;
+} TflFinish;
+int tfl_finish_gemm_takes(int rows, int width, int n, int k, int epilogue, int n_raw);
+int tfl_finish_gemm(const TflFinish* f, const TflGemm* product, int epilogue, void* stream);
+
 /* x += d (T); xt = T(x)  (xt may be NULL). */
 int tfl_residual(const void* d, float* x, void* xt, int64_t n, int dtype, void* stream);
 

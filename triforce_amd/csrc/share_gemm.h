@@ -56,8 +56,12 @@ __device__ __forceinline__ void finish_raw(const TflGemm& a, int m, bool live, i
 // 15.6, 1 076: 27.9 / 29.2 / 39.5 -> 24.5 / 24.3 / 26.6, 1 376: 34.2 / 34.7 / 41.9 -> 30.5 / 29.6 / 31.5, 2 000: 44.6 / 45.9 / 56.5 -> 43.4 /
 // 43.6 / 46.1 (6.0 TB/s); 256 panels of 15 104: 26.9 / 28.7 / 36.5 -> 21.2 / 22.2 / 32.9 (5.8 TB/s).
 // cu: this workgroup's place among those that share the panels, mb: its block of rows.
-template <typename T, int EPI, int P, bool TAIL, int MT, int U>
-__device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail_rows, const int tail_per, const int cu, const int mb, char* share_smem) {
+// Src: where x comes from.  FromMemory: a.x, asked for with the weights.  Otherwise (INSIDE, one block of rows) the workgroup makes it itself under the first
+// two batches of weights: src.ask() issues its loads in front of them, src.make() leaves x in LDS, octet-major, and ends with a barrier.
+struct FromMemory { static constexpr bool INSIDE = false; };
+template <typename T, int EPI, int P, bool TAIL, int MT, int U, class Src = FromMemory>
+__device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail_rows, const int tail_per, const int cu, const int mb, char* share_smem,
+                                                Src src = Src()) {
     typedef typename El<T>::Frag Frag;
     constexpr int WAVES = 8, NP = P + (TAIL ? 1 : 0), CUS = 256;
     f32x4 (*part)[NP * MT][64] = reinterpret_cast<f32x4 (*)[NP * MT][64]>(share_smem);
@@ -90,15 +94,20 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
     for (int p = 0; p < NP; ++p)
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[p][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto load = [&](Frag (&w)[U][NP], Frag (&x)[U][MT], int c0) {         // (past the end: the last chunk again, not used)
+    auto chunk = [&](int o) {                                // (past the end: the last chunk again, not used)
+        const int c = min(o, n_own - 1) + rot;
+        return c_beg + (c >= n_own ? c - n_own : c);
+    };
+    auto load = [&](Frag (&w)[U][NP], Frag (&x)[U][MT], int c0) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            int c = min(c0 + u, n_own - 1) + rot;
-            c = c_beg + (c >= n_own ? c - n_own : c);
+            const int c = chunk(c0 + u);
 #pragma unroll
             for (int p = 0; p < NP; ++p) w[u][p] = load_frag_stream(wp[p] + wstep * c);
+            if constexpr (!Src::INSIDE) {
 #pragma unroll
-            for (int t = 0; t < MT; ++t) x[u][t] = load_frag(xp[t] + xstep * c);
+                for (int t = 0; t < MT; ++t) x[u][t] = load_frag(xp[t] + xstep * c);
+            }
         }
     };
     auto multiply = [&](const Frag (&w)[U][NP], const Frag (&x)[U][MT], int c0) {
@@ -131,7 +140,38 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
     };
     const f32x4 first = beside(wave);
     asm volatile("" ::: "memory");
-    if (n_own > 0) {
+    if constexpr (Src::INSIDE) {
+        static_assert(MT == 1, "one block of rows");
+        Frag wa[U][NP], wb[U][NP], x[U][MT];
+        src.ask();
+        asm volatile("" ::: "memory");
+        if (n_own > 0) {
+            load(wa, x, 0);
+            load(wb, x, U);
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        const T* xs = src.make(cu) + (g * a.rows + min(i, a.rows - 1)) * 8;
+        auto take = [&](int c0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) x[u][0] = load_frag(xs + chunk(c0 + u) * 32 * a.rows);
+        };
+        if (n_own > 0) {
+            int c0 = 0;
+            for (; c0 + 2 * U < n_own; c0 += 2 * U) {
+                take(c0);
+                multiply(wa, x, c0);
+                load(wa, x, c0 + 2 * U);
+                take(c0 + U);
+                multiply(wb, x, c0 + U);
+                load(wb, x, c0 + 3 * U);
+            }
+            take(c0);
+            multiply(wa, x, c0);
+            take(c0 + U);
+            multiply(wb, x, c0 + U);
+        }
+    } else if (n_own > 0) {
         Frag wa[U][NP], xa[U][MT], wb[U][NP], xb[U][MT];
         load(wa, xa, 0);
         for (int c0 = 0; c0 < n_own; c0 += 2 * U) {

@@ -178,7 +178,14 @@ TILE_ABI_VERSION = 2
 _tile = None
 
 # ---- libtriforce_latent.so (include/triforce_latent.h) ------------------------------------------------------------------
+class TflFinish(_c.Structure):
+    """include/triforce_latent.h: TflFinish."""
+    _fields_ = [(n, _vp) for n in ("y", "y_w", "step", "norm_w", "x", "x_out")] + [("ld_y", _i64), ("width", _i32), ("width_real", _i32), ("eps", _f32)]
+
+
 LATENT_SIGNATURES = {
+    "tfl_finish_gemm_takes": (_i32, [_i32] * 6),
+    "tfl_finish_gemm": (_i32, [_c.POINTER(TflFinish), _c.POINTER(TflGemm), _i32, _vp]),
     "tfl_abi_version": (_i32, []),
     "tfl_finish": (_i32, [_vp, _vp, _i32, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _f32, _i32, _vp]),
     "tfl_residual": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp]),
@@ -226,7 +233,15 @@ class TfhRecStep(_c.Structure):
                 + [(n, _f32) for n in ("inv_tau", "q_scale", "out_scale")])
 
 
+class TfhConnect(_c.Structure):
+    """include/triforce_hybrid.h: TfhConnect."""
+    _fields_ = ([(n, _vp) for n in ("y", "out", "mix", "in", "norm_w", "x", "x_out")] + [("ld_y", _i64)]
+                + [(n, _i32) for n in ("streams", "width", "width_real")] + [("eps", _f32)])
+
+
 HYBRID_SIGNATURES = {
+    "tfh_connect_gemm_takes": (_i32, [_i32] * 6),
+    "tfh_connect_gemm": (_i32, [_c.POINTER(TfhConnect), _c.POINTER(TflGemm), _i32, _vp]),
     "tfh_abi_version": (_i32, []),
     "tfh_connect": (_i32, [_vp, _vp, _i32, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _i64, _i64, _i32, _i32, _i32,
                            _f32, _i32, _vp]),

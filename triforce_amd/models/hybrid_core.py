@@ -2,7 +2,8 @@
 state-space recurrence, or gated linear attention) on the HIP ops (ops_hybrid).
 
 Decode form of a layer (one token per sequence, any number of sequences): eight launches - [streams, norm] [input projections]
-[mixer: attention splits and state updates side by side] [merge, norms, gates] [output projection] [streams, norm] [gated unit] [down].
+[mixer: attention splits and state updates side by side] [merge, norms, gates] [output projection] [streams, norm] [gated unit] [down]; for one
+sequence the products behind [streams, norm] make their row themselves.
 Prefill form: products of many rows (ops_rows) between the row kernels, the paged attention and the segmented recurrence.
 """
 import zlib
@@ -166,7 +167,7 @@ class ParallelMixer:
         return _units(self.right.geom)
 
     def decode(self, h, batch, rope, cache_rows, states, eps):
-        raw = oh.linear_f32(h, self.w_in, self.w_in.n)
+        raw = oh.linear_of(h, self.w_in, self.w_in.n)
         step = oh.MixerStep(raw, batch.klen, eps, h.dtype, attn=self.left.step(batch, rope, cache_rows, self.spec.left_scale),
                             rec=self.right.step(batch, states, self.spec.right_scale), max_keys=batch.max_len)
         return oh.linear_f32(step.run().operand(), self.w_out, self.w_out.n)
@@ -212,7 +213,7 @@ class LinearAttentionMixer:
 
     def decode(self, h, batch, rope, cache_rows, states, eps):
         g = self.geom
-        raw = oh.linear_f32(h, self.w_in, self.w_in.n)
+        raw = oh.linear_of(h, self.w_in, self.w_in.n)
         rec = dict(a2=self.a2, a2_b=self.a2_b, norm_w=self.norm_w, state=states["state"], seat=batch.seat, gate_off=g.gate_off, q_off=g.q_off,
                    k_off=g.k_off, v_off=g.v_off, a_off=g.a_off, rank=g.rank, H=g.H, per_group=1, N=g.N, V=g.V, V_real=g.v_real,
                    norm_groups=g.norm_groups, inv_tau=1.0 / self.spec.tau, q_scale=self.q_scale, out_scale=1.0)
@@ -242,7 +243,7 @@ class GatedFeedForward:
         self.w_down = TileWeight(grow(get("down").to(dtype), W, F))
 
     def decode(self, h):
-        return oh.linear_f32(oh.gelu_glu_linear(h, self.w_gu), self.w_down, self.w_down.n)
+        return oh.linear_f32(oh.gelu_glu_of(h, self.w_gu), self.w_down, self.w_down.n)
 
     def prefill(self, h):
         act = self.w_gu.glu_matmul(h)

@@ -1,6 +1,6 @@
 """Weights and the per-layer compute of a latent-attention decoder on the HIP ops (ops_latent).
 
-Decode form of a layer (one token per sequence, any number of sequences): ten launches - [norm] [input projections, gelu]
+Decode form of a layer (one token per sequence, any number of sequences): ten launches - [norm] [input projections, gelu] (one or two rows: one launch)
 [query up-projection + cache append] [query to latent] [attention (beside it, on CUs of its own, feed-forward down), merge, or the
 merge in the next one] [latent to value, gate] [output (+ feed-forward down), residual] [token gate] [token projection].  Prefill form: products of many
 rows (ops_rows) between the row kernels and the up-projected attention.

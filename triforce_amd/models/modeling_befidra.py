@@ -92,10 +92,19 @@ class BefidraForCausalLM:
         W, eps, width = self.weights, self.config.eps, self.config.hidden_size
         x = torch.empty(ids.numel(), ol.pad32(width), dtype=torch.float32, device=self.device)
         y = y_w = None
+
+        def inside(wt, epi, n_raw=0):
+            """Does the product that reads the next norm make its rows itself?"""
+            return (batch.decode and y is not None and W.capture is None
+                    and ol.Finish.takes(x.shape[0], x.shape[1], wt, epi, n_raw))
         for r, (i, t, first) in enumerate(self.runs):
             L = W.layers[i]
-            h = ol.finish(x, L.norm1, eps, width, self.dtype, embed=W.embed if r == 0 else None, ids=ids if r == 0 else None,
-                          y=y, y_w=y_w, step=W.step[t] if first else None, octets=batch.decode)
+            if inside(L.w_in, "in", L.geom.n_raw):
+                h = ol.Finish(x, L.norm1, eps, width, y, y_w, W.step[t] if first else None)
+                x = h.out
+            else:
+                h = ol.finish(x, L.norm1, eps, width, self.dtype, embed=W.embed if r == 0 else None, ids=ids if r == 0 else None,
+                              y=y, y_w=y_w, step=W.step[t] if first else None, octets=batch.decode)
             if W.capture is not None and r > 0:
                 W.capture.append((x - W.step[t] if first else x.clone())[:, :width])
             layer = L.decode if batch.decode else L.prefill
@@ -105,6 +114,8 @@ class BefidraForCausalLM:
             return None
         if batch.want is not None:
             x, y = x[batch.want], None if y is None else y[batch.want]
+        if inside(W.logits, "f32"):
+            return ol.finish_logits(ol.Finish(x, W.final_norm, eps, width, y, y_w), W.logits, self.vocab_size)
         h = ol.finish(x, W.final_norm, eps, width, self.dtype, y=y, y_w=y_w)
         if W.capture is not None:
             W.capture.append(x[:, :width].clone())

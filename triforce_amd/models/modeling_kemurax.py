@@ -101,23 +101,28 @@ class KemuraxForCausalLM:
         first = dict(embed=W.embed, ids=ids, embed_w=W.embed_norm)
         y = hc = None
 
-        def read(connection, norm):
-            """The last sublayer's result into the streams, the next sublayer's input out of them."""
+        def read(x, connection, norm, wt, epi):
+            """The last sublayer's result into the streams, the next sublayer's input, which goes through wt, out of them: (input, streams)."""
+            if batch.decode and hc is not None and W.capture is None and oh.Connect.takes(x, wt, epi):
+                h = oh.Connect(x, connection.u_in, norm, eps, width, y, hc.out, hc.mix)
+                return h, h.out
             before = first if hc is None else dict(y=y, out=hc.out, mix=hc.mix)
-            return oh.connect(x, connection.u_in, norm, eps, width, self.dtype, octets=batch.decode, **before)
+            return oh.connect(x, connection.u_in, norm, eps, width, self.dtype, octets=batch.decode, **before), x
         for i, L in enumerate(W.layers):
-            h = read(L.hc1, L.norm1)
+            h, x = read(x, L.hc1, L.norm1, L.mixer.w_in, "f32")
             if W.capture is not None and i > 0:
                 W.capture.append(x.sum(1)[:, :width])
             run = L.mixer.decode if batch.decode else L.mixer.prefill
             y, hc = run(h, batch, self._rope_of(L.spec), cache.rows[i], cache.states[i], eps), L.hc1
             if L.ff is not None:
-                h = read(L.hc2, L.norm2)
+                h, x = read(x, L.hc2, L.norm2, L.ff.w_gu, "glu")
                 y, hc = (L.ff.decode if batch.decode else L.ff.prefill)(h), L.hc2
         if batch.want is not None and batch.want.numel() == 0:
             return None
         if batch.want is not None:
             x, y = x[batch.want], y[batch.want]
+        if batch.decode and W.capture is None and oh.Connect.takes(x, W.logits, "f32"):
+            return oh.Connect(x, W.final_in, W.final_norm, eps, width, y, hc.out, hc.mix, keep=False).linear(W.logits, self.vocab_size)
         h = oh.connect(x, W.final_in, W.final_norm, eps, width, self.dtype, y=y, out=hc.out, mix=hc.mix, keep=W.capture is not None)
         if W.capture is not None:
             W.capture.append(x.sum(1)[:, :width])

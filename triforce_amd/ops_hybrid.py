@@ -40,6 +40,60 @@ def connect(x, u_in, norm_w, eps, width, dtype, embed=None, ids=None, embed_w=No
     return h
 
 
+class Connect:
+    """connect() of decode rows that the product which reads them makes for itself (tfh_connect_gemm): stands for its activation block; ``out`` holds the
+    updated streams."""
+
+    def __init__(self, x, u_in, norm_w, eps, width, y, out, mix, keep=True):
+        _need(x, u_in, norm_w, y, out, mix)
+        _f32(x, u_in, norm_w, y, out, mix)
+        rows, streams, wp = x.shape
+        assert x.is_contiguous() and norm_w.numel() == wp and u_in.numel() == streams == out.numel() and mix.shape == (streams, streams) and mix.is_contiguous()
+        assert y.shape == (rows, wp) and y.stride(1) == 1
+        self.out, self.rows, self.dtype, self.device = torch.empty_like(x) if keep else None, rows, torch.bfloat16, x.device
+        self.keep = (x, u_in, norm_w, y, out, mix)
+        f = self.c = hip.TfhConnect()
+        for name, t in (("y", y), ("out", out), ("mix", mix), ("in", u_in), ("norm_w", norm_w), ("x", x), ("x_out", self.out)):
+            setattr(f, name, None if t is None else t.data_ptr())
+        f.ld_y, f.streams, f.width, f.width_real, f.eps = y.stride(0), streams, wp, width, eps
+
+    @staticmethod
+    def takes(x, wt, epi):
+        """Does the product of wt with this epilogue ("f32", "glu") make the rows of x itself?"""
+        rows, streams, wp = x.shape
+        return wt.chunk_major and wt.dtype == torch.bfloat16 and wt.k == wp and _lib().tfh_connect_gemm_takes(rows, streams, wp, wt.n, wt.k, hip.TFL_EPI[epi]) == 1
+
+    def _product(self, wt, epi, **kw):
+        assert wt.dtype == self.dtype
+        a = hip.TflGemm()
+        a.wp, a.rows, a.n, a.k, a.groups, a.x_oct, a.t_oct, a.ld_x, a.chunk_major = wt.packed.data_ptr(), self.rows, wt.n, wt.k, 1, 8, 8, 8, 1
+        for name, v in kw.items():
+            setattr(a, name, v.data_ptr() if isinstance(v, torch.Tensor) else v)
+        hip.check(_lib().tfh_connect_gemm(ctypes.byref(self.c), ctypes.byref(a), hip.TFL_EPI[epi], _stream()), "tfh_connect_gemm " + epi)
+
+    def linear(self, wt, n_real):
+        """linear_f32 of the rows."""
+        out = torch.empty(self.rows, n_real, dtype=torch.float32, device=self.device)
+        self._product(wt, "f32", out_f=out, ld_f=n_real, n_real=n_real)
+        return out
+
+    def gelu_glu(self, wt):
+        """gelu_glu_linear of the rows."""
+        out = empty_act(self.rows, wt.n // 2, wt.dtype, self.device)
+        self._product(wt, "glu", out_t=out, ld_t=8, t_oct=8 * self.rows)
+        return out
+
+
+def linear_of(h, wt, n_real):
+    """linear_f32 of an activation block or a Connect."""
+    return h.linear(wt, n_real) if isinstance(h, Connect) else linear_f32(h, wt, n_real)
+
+
+def gelu_glu_of(h, wt):
+    """gelu_glu_linear of an activation block or a Connect."""
+    return h.gelu_glu(wt) if isinstance(h, Connect) else gelu_glu_linear(h, wt)
+
+
 def qkv_prepare(y, g, q_norm, k_norm, eps, rope, pos, slot, cache):
     """Norm and rotation of new queries (in place) and keys; keys and values into the cache rows ``slot``."""
     _need(y, pos, slot, cache)

@@ -13,12 +13,41 @@ from . import hip
 from .ops_tile import (_CODE, PAGE, TileWeight, _f32, _gemm, _i32, _lay, _need, _p, _stream, _tail, act_rows, decode_prep, empty_act, linear_rows,  # noqa: F401
                        linear_f32, pack_tiles, pad32)
 
+class Finish:
+    """finish() of decode rows that the product which reads them makes for itself (tfl_finish_gemm): stands for its activation block; ``out`` is the
+    updated residual."""
+
+    def __init__(self, x, norm_w, eps, width, y, y_w, step=None):
+        _need(x, norm_w, y, y_w, step)
+        _f32(x, norm_w, y, y_w, step)
+        rows, wp = x.shape
+        assert x.is_contiguous() and norm_w.numel() == wp == y_w.numel() and y.shape == (rows, wp) and y.stride(1) == 1 and (step is None or step.numel() == wp)
+        self.out, self.dtype, self.is_cuda, self.shape = torch.empty_like(x), torch.bfloat16, True, (rows, wp)
+        self.device, self.keep = x.device, (x, norm_w, y, y_w, step)
+        f = self.c = hip.TflFinish()
+        f.y, f.y_w, f.step, f.norm_w, f.x, f.x_out = y.data_ptr(), y_w.data_ptr(), None if step is None else step.data_ptr(), norm_w.data_ptr(), x.data_ptr(), self.out.data_ptr()
+        f.ld_y, f.width, f.width_real, f.eps = y.stride(0), wp, width, eps
+
+    @staticmethod
+    def takes(rows, wp, wt, epi, n_raw=0):
+        """Does the product of wt with this epilogue ("in", "f32") make ``rows`` rows itself?"""
+        return wt.chunk_major and wt.dtype == torch.bfloat16 and wt.k == wp and hip.latent_lib().tfl_finish_gemm_takes(rows, wp, wt.n, wt.k, hip.TFL_EPI[epi], n_raw) == 1
+
+    def product(self, wt, epi, **kw):
+        a = hip.TflGemm()
+        a.wp, a.rows, a.n, a.k, a.groups, a.x_oct, a.t_oct, a.ld_x, a.chunk_major = wt.packed.data_ptr(), self.shape[0], wt.n, wt.k, 1, 8, 8, 8, 1
+        for name, v in kw.items():
+            setattr(a, name, v.data_ptr() if isinstance(v, torch.Tensor) else v)
+        hip.check(hip.latent_lib().tfl_finish_gemm(ctypes.byref(self.c), ctypes.byref(a), hip.TFL_EPI[epi], _stream()), "tfl_finish_gemm " + epi)
+
+
 def input_projection(h, wt, n_raw, q_norm, act, act_off):
-    """All projections of the layer's one norm (h, act: activation blocks).  Returns (raw fp32 [rows, n_raw], per-panel sums of
+    """All projections of the layer's one norm (h, act: activation blocks, h also a Finish).  Returns (raw fp32 [rows, n_raw], per-panel sums of
     squares, the first len(q_norm) outputs times q_norm as an octet-major block); gelu of the outputs behind n_raw goes to the
     columns of act from act_off on."""
-    _need(h, act)
-    rows, k, ld, octet = _lay(h)
+    inside = isinstance(h, Finish)
+    _need(None if inside else h, act)
+    rows, k, ld, octet = (*h.shape, 8, 8) if inside else _lay(h)
     act_rows_, act_k, act_ld, act_oct = _lay(act)
     assert h.dtype == wt.dtype == act.dtype and k == wt.k and act_rows_ == rows and act_k >= act_off + wt.n - n_raw and act_off % 8 == 0
     raw = torch.empty(rows, n_raw, dtype=torch.float32, device=h.device)
@@ -26,9 +55,21 @@ def input_projection(h, wt, n_raw, q_norm, act, act_off):
     _f32(q_norm)
     xq = empty_act(rows, q_norm.numel(), wt.dtype, h.device)
     tail = _tail(act, act_off) if wt.n > n_raw else act
-    _gemm(wt, h, "in", rows, ld_x=ld, x_oct=octet, out_f=raw, ld_f=n_raw, ss_out=ss, ss_ld=n_raw // 16, n_raw=n_raw,
-          out_t=tail, ld_t=act_ld, t_oct=act_oct, out_t2=xq, norm_w=q_norm, n_scaled=q_norm.numel())
+    to = dict(out_f=raw, ld_f=n_raw, ss_out=ss, ss_ld=n_raw // 16, n_raw=n_raw, out_t=tail, ld_t=act_ld, t_oct=act_oct, out_t2=xq, norm_w=q_norm,
+              n_scaled=q_norm.numel())
+    if inside:
+        h.product(wt, "in", **to)
+    else:
+        _gemm(wt, h, "in", rows, ld_x=ld, x_oct=octet, **to)
     return raw, ss, xq
+
+
+def finish_logits(h, wt, n_real):
+    """linear_f32 of a Finish."""
+    assert h.dtype == wt.dtype
+    out = torch.empty(h.shape[0], n_real, dtype=torch.float32, device=h.device)
+    h.product(wt, "f32", out_f=out, ld_f=n_real, n_real=n_real)
+    return out
 
 
 def query_and_append(xq, raw, ss, wt, g, kv_norm, eps, rope, pos, slot, cache):
