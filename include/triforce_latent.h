@@ -51,6 +51,14 @@ int tfl_residual(const void* d, float* x, void* xt, int64_t n, int dtype, void* 
 int tfl_token_gate(const void* s, int64_t ld_s, const void* tok_table, int64_t ld_tok, const int64_t* ids, int vocab, void* out,
                    int rows, int n, int n_real, int dtype, void* stream);
 
+/* Both products of a token's side input for up to 16 rows in bfloat16: out[m*ld_out + n] = sum over s of (gelu_tanh(x . Wg^T)[m][s] * tok_table[ids[m]*ld_tok
+ * + s]) * Wp[n][s], n < n_real (TFL_EPI_TOKEN, then TFL_EPI_F32).  gate_packed [side, width] and proj_packed [width, side] panel-major; x an activation block;
+ * ws: tfl_token_side_ws_floats(rows, side) floats. */
+int64_t tfl_token_side_ws_floats(int rows, int side);
+int tfl_token_side(const void* gate_packed, const void* proj_packed, const void* x, int64_t ld_x, int64_t x_oct, const void* table,
+                   int64_t ld_tok, const int64_t* ids, int vocab, float* out, int64_t ld_out, float* ws, int64_t ws_floats, int rows,
+                   int width, int side, int side_real, int n_real, void* stream);
+
 /* Prefill half of the input projection: y [rows][q + C + R + gate + up] (T) ->
  *   cq [rows][q] = y_q / rms * q_norm;  cache row slot[m] = latent / rms * kv_norm | rotated key;  ck [rows][C + R] the same
  *   row again (NULL: not wanted);  act [rows] at stride ld_act = gelu_tanh(up) (n_up = 0: none). */

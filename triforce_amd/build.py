@@ -20,7 +20,7 @@ SOURCES = ["attn.hip", "retrieval.hip", "elementwise.hip", "sampling.hip", "offl
 LIBRARIES = {
     "core": (LIB_PATH, SOURCES, ["common.h", "gemv_common.h", "share_shape.h", "lanes.h", "tree_mask.h", "select_common.h", "prefill_wide.h", "lds_dma.h", "rows_gemm.h"], ["triforce_hip.h"]),
     "tile": (TILE_LIB_PATH, ["tile_gemm.hip", "split_gemm.hip", "tile_rows_gemm.hip", "paged.hip"], ["tile_common.h", "lanes.h", "lds_dma.h", "share_gemm.h", "share_shape.h", "rows_gemm.h"], ["triforce_tile.h"]),
-    "latent": (LATENT_LIB_PATH, ["latent_attn.hip", "latent_ops.hip", "latent_finish.hip"], ["tile_common.h", "lanes.h", "lds_dma.h", "flash_tile.h", "share_gemm.h", "share_shape.h", "row_source.h"], ["triforce_tile.h", "triforce_latent.h"]),
+    "latent": (LATENT_LIB_PATH, ["latent_attn.hip", "latent_ops.hip", "latent_finish.hip", "latent_token.hip"], ["tile_common.h", "lanes.h", "lds_dma.h", "flash_tile.h", "share_gemm.h", "share_shape.h", "row_source.h"], ["triforce_tile.h", "triforce_latent.h"]),
     "hybrid": (HYBRID_LIB_PATH, ["hybrid_rec.hip", "hybrid_attn.hip", "hybrid_step.hip", "hybrid_ops.hip", "hybrid_connect.hip"],
                ["tile_common.h", "lanes.h", "flash_tile.h", "hybrid_common.h", "share_gemm.h", "share_shape.h", "row_source.h"],
                ["triforce_tile.h", "triforce_hybrid.h"]),

@@ -184,6 +184,8 @@ class TflFinish(_c.Structure):
 
 
 LATENT_SIGNATURES = {
+    "tfl_token_side_ws_floats": (_i64, [_i32, _i32]),
+    "tfl_token_side": (_i32, [_vp, _vp, _vp, _i64, _i64, _vp, _i64, _vp, _i32, _vp, _i64, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _vp]),
     "tfl_finish_gemm_takes": (_i32, [_i32] * 6),
     "tfl_finish_gemm": (_i32, [_c.POINTER(TflFinish), _c.POINTER(TflGemm), _i32, _vp]),
     "tfl_abi_version": (_i32, []),

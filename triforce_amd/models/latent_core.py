@@ -94,7 +94,7 @@ class LatentLayer:
         xt = ol.add_linear(act, self.w_out, x, want_copy=bool(self.side_dim), k=None if plan is None else own)
         if not self.side_dim:
             return None
-        return ol.linear_f32(ol.token_gate_linear(xt, self.side_gate, side_table, ids, self.side_dim), self.side_proj, self.width)
+        return ol.token_side(xt, self.side_gate, self.side_proj, side_table, ids, self.side_dim, self.width)
 
     def prefill(self, h, x, ids, side_table, batch, rope, cache_rows, eps):
         g = self.geom

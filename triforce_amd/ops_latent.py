@@ -143,6 +143,27 @@ def token_gate_linear(x, wt, table, ids, n_real):
     return out
 
 
+# Every workgroup of the projection reads all parts of all rows: us of eight steps of six layer runs, panels -> parts, 1 row 4 296 -> 4 187, 2 4 506 ->
+# 4 420, 4 4 768 -> 4 674, 8 4 968 -> 4 925, 12 the same, 16 5 378 -> 5 402.
+TOKEN_SIDE_ROWS = 10
+
+
+def token_side(x, gate, proj, table, ids, n_real, width):
+    """linear_f32(token_gate_linear(x, gate, table, ids, n_real), proj, width), for a few rows of bfloat16 with the gate's K cut over the grid (tfl_token_side)."""
+    rows, k, ld, octet = _lay(x)
+    if x.dtype != torch.bfloat16 or rows > TOKEN_SIDE_ROWS or proj.chunk_major or gate.chunk_major:
+        return linear_f32(token_gate_linear(x, gate, table, ids, n_real), proj, width)
+    _need(x, table, ids)
+    assert ids.dtype == torch.int64 and ids.numel() == rows and k == gate.k == proj.n and gate.n == proj.k and x.dtype == table.dtype == gate.dtype == proj.dtype
+    assert table.shape[1] == n_real and ids.is_contiguous()
+    L = hip.latent_lib()
+    out = torch.empty(rows, width, dtype=torch.float32, device=x.device)
+    ws = torch.empty(L.tfl_token_side_ws_floats(rows, gate.n), dtype=torch.float32, device=x.device)
+    hip.check(L.tfl_token_side(_p(gate.packed), _p(proj.packed), _p(x), ld, octet, _p(table), table.stride(0), _p(ids), table.shape[0], _p(out), out.stride(0), _p(ws),
+                               ws.numel(), rows, gate.k, gate.n, n_real, width, _stream()), "tfl_token_side")
+    return out
+
+
 def finish(x, norm_w, eps, width, dtype, embed=None, ids=None, y=None, y_w=None, step=None, octets=False):
     """Residual bookkeeping between two layers and the next norm; see tfl_finish.  x fp32 [rows, padded width] is updated in
     place; returns h in ``dtype``, row-major or (``octets``) octet-major."""
