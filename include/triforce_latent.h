@@ -101,6 +101,9 @@ int tfl_attn_beside_plan_of(int rows, int H, int C, int R, int64_t pages, int64_
                             int32_t* parts);
 int tfl_attn_decode_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out, float* ws,
                            int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int panels_each, const TflGemm* product, void* stream);
+/* Columns of the product (n of k) beside the attention, from the last on, that the query to latent product in front of it carries (tfl_gemm_carry); 0: none. */
+int tfl_latent_carry(int rows, int H, int C, int R, int64_t pages, int64_t longest, int n, int k);
+
 /* TFL_EPI_GATED in bfloat16 (include/triforce_tile.h; k 512, up to 4 rows) of what the splits in ws merge to: product->x is not read. */
 int tfl_latent_value(const float* ws, int64_t ws_floats, int nsplit, const TflGemm* product, void* stream);
 

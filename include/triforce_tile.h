@@ -73,6 +73,10 @@ typedef struct TflGemm {
 
 int tfl_gemm(const TflGemm* a, int dtype, int epilogue, void* stream);
 
+/* tfl_gemm in bfloat16 with LATENT, up to 16 rows and n a multiple of 64, and beside it, on workgroups of their own in the same launch, another product
+ * that waits for nothing of it: carried->out_f += carried->x . W^T (chunk-major weights, one group, as many rows, no out_t). */
+int tfl_gemm_carry(const TflGemm* a, const TflGemm* carried, void* stream);
+
 /* Start of a decode step: pos = len; slot = table[len/64]*64 + len%64; klen = len + 1; len += 1.  Rows with len < 0 (or past
  * their table) stay idle: pos 0, slot -1, klen 0. */
 int tfl_decode_prep(int32_t* len, const int32_t* table, int table_ld, int table_cols, int32_t* pos, int32_t* slot, int32_t* klen,

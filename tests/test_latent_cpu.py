@@ -145,6 +145,25 @@ def test_plan_for_a_known_longest_row(rows, pages, longest, n, k, each):
     assert plan is None if each == 0 else plan[1] == each
 
 
+def test_carried_columns():
+    """What query to latent carries of that product: whole thousands that leave a product the attention runs beside, none where that one is the shorter side, and
+    as picked where it was measured."""
+    from triforce_amd import ops_latent as ol
+    for rows in (0, 1, 2, 7, 16, 17, 32):
+        for heads in (16, 17, 32, 33):
+            for pages in (0, 1, 64, 500, 2016, 1 << 21):
+                for n, k in ((4096, 11008), (4096, 5120), (4096, 6144), (4096, 14336), (8192, 8192), (6160, 8224)):
+                    for longest in (None, max(1, pages // 2)):
+                        c = ol.carry_plan(rows, heads, 512, 64, pages, n, k, longest)
+                        assert c in (0, 4096, 5120, 6144)
+                        if c:
+                            assert 1 <= rows <= 16 and 16 < heads <= 32 and pages >= 1 and ol.beside_plan(rows, heads, 512, 64, pages, n, k - c, longest)
+    assert ol.carry_plan(1, 32, 256, 64, 64, 4096, 11008) == ol.carry_plan(1, 32, 512, 32, 64, 4096, 11008) == 0
+    pick = [ol.carry_plan(rows, 32, 512, 64, pages, 4096, 11008, longest) for rows, pages, longest in
+            ((1, 63, 63), (2, 112, 63), (4, 204, 63), (8, 396, 63), (16, 810, 63), (1, 7, 7), (16, 90, 7), (2, 560, 313), (8, 1950, 313))]
+    assert pick == [5120, 5120, 5120, 4096, 0, 5120, 6144, 0, 0]
+
+
 def test_a_step_says_how_long_its_longest_sequence_is():
     """With the token that it adds: a page's last and its first."""
     from triforce_amd.utils.batch_infer import _DecodeStep

@@ -724,6 +724,15 @@ extern "C" int tfl_attn_decode(const void* q, const void* cache, int n_pages, co
 // them in one row: 76.3 apart, 57.3 beside).  What they pick takes 1.008 of the best on average and at most 1.10.  Half of that is short contexts,
 // which stay beside where that costs a tenth at most: apart, the splits follow the cache's room, beside, what is in it.  (Not at k above 12 288, where the
 // product's half of the CUs is by far the longer side.)
+struct BesideTime { int workers; double product, attention, all; };
+static BesideTime beside_time(int rows, int H, int64_t pages, int64_t longest, int n, int k, int p) {
+    const int g = ((n >> 4) + p - 1) / p, a = 256 - g, most = 2 * a / rows < 128 ? 2 * a / rows : 128;
+    if (g > 128) return {0, 0., 0., 0.};
+    const double heads = H / 32.0, each = fmax((double)pages / a, (double)((longest + most - 1) / most));
+    const double product = 26.33 * 2e-6 * n * k / g + 0.527 * rows * k / 11008.0, attention = 3.22 + 2.7475 * each + 0.945 * p;
+    return {a, product, attention, fmax(product, attention) + 0.25 * heads * rows + 0.0068 * heads * (double)(pages < a ? pages : a) - 1.892 * (rows < 5 ? 5 - rows : 0)};
+}
+
 static int beside_plan(int rows, int H, int64_t pages, int64_t longest, int n, int k, int* panels_each) {
     const int panels = n >> 4;
     if (rows < 1 || rows > 32 || H <= 16 || H > 32 || pages < 1 || pages > (1 << 20) || longest < 1 || panels < 256 || panels > 512 || k < 2048) return 0;
@@ -733,12 +742,8 @@ static int beside_plan(int rows, int H, int64_t pages, int64_t longest, int n, i
     if (pages < 32 * rows && k <= 12288) least *= 1.0 / 0.9;
     int workers = 0;
     for (int p = 2; p <= 4; ++p) {
-        const int g = (panels + p - 1) / p, a = 256 - g, most = 2 * a / rows < 128 ? 2 * a / rows : 128;
-        if (g > 128) continue;
-        const double each = fmax((double)pages / a, (double)((longest + most - 1) / most));
-        const double product = 26.33 * mb / g + 0.527 * x, attention = 3.22 + 2.7475 * each + 0.945 * p;
-        const double t = fmax(product, attention) + 0.25 * heads * rows + 0.0068 * heads * (double)(pages < a ? pages : a) - 1.892 * (rows < 5 ? 5 - rows : 0);
-        if (t < least) { least = t; workers = a; *panels_each = p; }
+        const BesideTime b = beside_time(rows, H, pages, longest, n, k, p);
+        if (b.workers > 0 && b.all < least) { least = b.all; workers = b.workers; *panels_each = p; }
     }
     return workers;
 }
@@ -756,6 +761,29 @@ extern "C" int tfl_attn_beside_plan_of(int rows, int H, int C, int R, int64_t pa
         *parts = (int32_t)(all < a ? all : a);
     }
     return a;
+}
+
+// Columns of that product's k, from the last on, that the query to latent product in front of the attention carries (latent_carry_kernel in tile_gemm.hip): as
+// long as what is left still outlasts the attention, in steps of 1 024 from 4 096 on (below that a carried panel costs its start more than the
+// other one saves: eight steps of six layer runs, one row of 4 000 keys, 2 048 -36 us, 3 072 +10, 4 096 -65, 5 120 -82, 6 144 -48).  The cost of carrying is
+// fitted to 90 points of 1 to 16 rows, contexts of 300 to 20 000; of 54 others none is slower for the pick.  us of query to latent, attention, value and output
+// product (32 heads, n 4 096, k 11 008), none -> as picked, at 300 / 2 000 / 4 000 keys: 1 row 34.7 -> 33.4, 35.5 -> 34.3, 36.0 -> 35.0; 4 rows 39.6 -> 37.6,
+// 40.9 -> 39.7, 43.1 -> 40.9; 8 rows 42.0 -> 39.3, 45.2 -> 41.6, 45.7 -> 43.4; 16 rows 46.4 -> 42.7, 48.8 -> 45.5, not picked (51.7, carrying 54.5).
+// Up to 16 rows: of 32 rows a carried panel reads twice its weights' bytes of x (6 664 us of eight steps -> 6 924).
+extern "C" int tfl_latent_carry(int rows, int H, int C, int R, int64_t pages, int64_t longest, int n, int k) {
+    if (C != 512 || R != 64 || rows < 1 || rows > 16 || longest < 1 || k > (1 << 20)) return 0;
+    int p = 0, q = 0, best = 0;
+    if (beside_plan(rows, H, pages, longest, n, k, &p) == 0) return 0;
+    const double apart = beside_time(rows, H, pages, longest, n, k, p).all;
+    double gain = 0.8;
+    for (int c = 4096; c <= 6144 && k - c >= 2048; c += 1024) {
+        if (beside_plan(rows, H, pages, longest, n, k - c, &q) == 0) break;
+        const BesideTime b = beside_time(rows, H, pages, longest, n, k - c, q);
+        const double saved = apart - b.all - (0.55 + 3.2e-7 * c * n + 0.11 * rows);
+        if (b.product < b.attention + 1.0 - 0.06 * rows) break;
+        if (saved > gain) { gain = saved; best = c; }
+    }
+    return best;
 }
 
 // The same where nobody knows the longest row: rows half to all as long as it.

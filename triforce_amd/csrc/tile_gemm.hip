@@ -24,16 +24,15 @@
 
 // P panels per workgroup (they share the operand rows), MT 16-row blocks, U tiles of 32 per batch; AHEAD: the next batch's weights
 // are requested before the current one is used (long K), otherwise a wave's whole K range should fit one or two batches.
+// bx, rb of blocks: this workgroup's place (a WAVES-wide half of one may stand for it, tid within it), part: its LDS.
 template <typename T, int EPI, int P, int MT, int WAVES, int U, bool AHEAD>
-__global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a) {
+__device__ __forceinline__ void latent_gemm_body(const TflGemm& a, const int tid, const int bx, const int blocks, const int rb, f32x4 (*part)[P * MT][64]) {
     typedef typename El<T>::Frag Frag;
     static_assert(P * MT <= WAVES, "one wave finishes one 16x16 tile");
-    __shared__ f32x4 part[WAVES][P * MT][64];
     const int ppg = a.n >> 4, npan = ppg * a.groups;
-    const int tid = threadIdx.x;
     if constexpr (EPI == TFL_EPI_QUERY) {
-        if ((int)blockIdx.x >= npan) {                       // the cache row of one batch row
-            const int m = blockIdx.y * (gridDim.x - npan) + blockIdx.x - npan;
+        if (bx >= npan) {                                    // the cache row of one batch row
+            const int m = rb * (blocks - npan) + bx - npan;
             if (m >= a.rows) return;
             const int slot = a.slot[m];
             if (slot < 0 || slot >= a.cache_rows) return;
@@ -47,8 +46,8 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
         }
     }
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, g = lane >> 4, i = lane & 15;
-    const int panel0 = blockIdx.x * P, grp = P == 1 ? panel0 / ppg : 0;
-    const int m0 = blockIdx.y * 16 * MT;
+    const int panel0 = bx * P, grp = panel0 / ppg;            // (several groups: their panels come in whole P)
+    const int m0 = rb * 16 * MT;
     const int chunks = a.k >> 5;
     const int per = (chunks + WAVES - 1) / WAVES;
     const int c_beg = wave * per, c_end = min(chunks, c_beg + per), last = c_end - 1;
@@ -76,7 +75,7 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
         for (int t = 0; t < MT; ++t) acc[p][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     // What the epilogue reads is asked for in front of the weights by the wave that finishes a tile, not behind the products, where nothing is
     // left to hide it (us: QUERY at one row 6.85 -> 6.62; at 32 rows TOKEN 8.97 -> 8.50, GATED 5.62 -> 5.21).
-    const int t_end = wave % MT, panel_end = panel0 + wave / MT, pin_end = P == 1 ? panel_end - grp * ppg : panel_end;
+    const int t_end = wave % MT, panel_end = panel0 + wave / MT, pin_end = panel_end - grp * ppg;
     const int m_end = min(m0 + 16 * t_end + i, a.rows - 1), n_end = 16 * pin_end + 4 * g;
     const bool ends = wave < P * MT && panel_end < npan;
     [[maybe_unused]] f32x4 with = {0.f, 0.f, 0.f, 0.f};
@@ -184,7 +183,7 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
     }
     __syncthreads();
     if (wave >= P * MT) return;                              // wave p * MT + t finishes row block t of panel p
-    const int t = wave % MT, panel = panel0 + wave / MT, pin = P == 1 ? panel - grp * ppg : panel;
+    const int t = wave % MT, panel = panel0 + wave / MT, pin = panel - grp * ppg;
     if (panel >= npan) return;
     f32x4 s = part[0][wave][lane];
 #pragma unroll
@@ -273,6 +272,28 @@ __global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a
         for (int r = 0; r < 4; ++r) s[r] = n + r < a.n_real ? gelu_tanh(s[r]) * (float)row4[r] : 0.f;
         store_quad((T*)a.out_t + (int64_t)m * a.ld_t + n, s);
     }
+}
+
+template <typename T, int EPI, int P, int MT, int WAVES, int U, bool AHEAD>
+__global__ __launch_bounds__(WAVES * 64) void latent_gemm_kernel(const TflGemm a) {
+    __shared__ f32x4 part[WAVES][P * MT][64];
+    latent_gemm_body<T, EPI, P, MT, WAVES, U, AHEAD>(a, threadIdx.x, blockIdx.x, gridDim.x, blockIdx.y, part);
+}
+
+// LATENT of up to 16 rows, and in front of it, on workgroups of their own, panels of another product that waits for nothing of it: out_f += x . W^T.
+// The decode step's query to latent is 4 MB of weights in a launch of 4.9 us, most of which is the launch's own start and end, while the feed-forward's down
+// product (90 MB) runs on half of the CUs beside the attention.  With 33 MB of it in here this launch takes 8.5 us, 0.6 more than those alone would, and
+// the attention's 14.4 instead of 20.0 (one row of 4 000 keys).  As many columns as tfl_latent_carry says.  Both workgroups are 512 threads of up
+// to 128 registers, so that every CU holds one of each; the carried ones are the longer and come first.  Half a workgroup is a workgroup of
+// latent_gemm_kernel: the same sums in the same order.
+__global__ __launch_bounds__(512, 4) void latent_carry_kernel(const TflGemm a, const TflGemm g, const int carried, const int blocks) {
+    __shared__ __align__(16) f32x4 part[8][2][64];
+    if ((int)blockIdx.x < carried) {
+        share_gemm_body<bf16, TFL_EPI_RESIDUAL, 1, false, 1, 4>(g, 0, 0, blockIdx.x, 0, (char*)part);
+        return;
+    }
+    const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    latent_gemm_body<bf16, TFL_EPI_LATENT, 2, 1, 4, 8, false>(a, threadIdx.x & 255, 2 * ((int)blockIdx.x - carried) + half, blocks, 0, part + 4 * half);
 }
 
 template <typename T, int EPI, int P, bool TAIL, int MT, int U>
@@ -382,14 +403,8 @@ static int dispatch_gemm(const TflGemm& a, int epi, hipStream_t st) {
     return TF_EINVAL;
 }
 
-extern "C" int tfl_gemm(const TflGemm* p, int dtype, int epi, void* stream) {
-    if (!p || !p->wp || !p->x) return TF_EINVAL;
-    const TflGemm a = *p;
-    if (a.rows < 1 || a.rows > (1 << 20) || a.n < 16 || (a.n & 15) || a.k < 32 || (a.k & 31) || a.groups < 1) return TF_EINVAL;
-    if ((a.ld_x & 7) || (a.x_group & 7) || a.x_oct < 8 || (a.x_oct & 7) || a.ld_x < 8) return TF_EINVAL;
-    if (a.chunk_major != 0 && (a.chunk_major != 1 || a.groups != 1)) return TF_EINVAL;
-    if (a.out_t && (a.t_oct < 8 || (a.t_oct & 7))) return TF_EINVAL;
-    if (dtype != 0 && dtype != 1) return TF_EINVAL;
+// What an epilogue asks of its operands.
+static int check_gemm(const TflGemm& a, int epi) {
     switch (epi) {
         case TFL_EPI_F32:
             if (!a.out_f || a.groups != 1 || a.n_real < 1 || a.n_real > a.n || a.ld_f < a.n_real) return TF_EINVAL;
@@ -427,5 +442,33 @@ extern "C" int tfl_gemm(const TflGemm* p, int dtype, int epi, void* stream) {
         default:
             return TF_EINVAL;
     }
+    return TF_OK;
+}
+
+extern "C" int tfl_gemm(const TflGemm* p, int dtype, int epi, void* stream) {
+    if (!p || !p->wp || !p->x) return TF_EINVAL;
+    const TflGemm a = *p;
+    if (a.rows < 1 || a.rows > (1 << 20) || a.n < 16 || (a.n & 15) || a.k < 32 || (a.k & 31) || a.groups < 1) return TF_EINVAL;
+    if ((a.ld_x & 7) || (a.x_group & 7) || a.x_oct < 8 || (a.x_oct & 7) || a.ld_x < 8) return TF_EINVAL;
+    if (a.chunk_major != 0 && (a.chunk_major != 1 || a.groups != 1)) return TF_EINVAL;
+    if (a.out_t && (a.t_oct < 8 || (a.t_oct & 7))) return TF_EINVAL;
+    if (dtype != 0 && dtype != 1) return TF_EINVAL;
+    const int rc = check_gemm(a, epi);
+    if (rc != TF_OK) return rc;
     return dtype == 0 ? dispatch_gemm<bf16>(a, epi, (hipStream_t)stream) : dispatch_gemm<float>(a, epi, (hipStream_t)stream);
+}
+
+extern "C" int tfl_gemm_carry(const TflGemm* p, const TflGemm* carried, void* stream) {
+    if (!p || !p->wp || !p->x || !carried) return TF_EINVAL;
+    const TflGemm a = *p, g = *carried;
+    if (a.rows < 1 || a.rows > 16 || a.n < 64 || (a.n & 63) || a.n > (1 << 16) || a.k < 32 || (a.k & 31) || a.groups < 1 || a.groups > 4096 || a.chunk_major != 0
+        || (a.ld_x & 7) || (a.x_group & 7) || a.x_oct < 8 || (a.x_oct & 7) || a.ld_x < 8) return TF_EINVAL;
+    if (!g.wp || !g.x || !g.out_f || g.out_t || g.rows != a.rows || g.n < 16 || (g.n & 15) || g.n > (1 << 16) || g.k < 32 || (g.k & 31) || g.groups != 1 || g.chunk_major != 1
+        || (g.ld_x & 7) || g.ld_x < 8 || g.x_oct < 8 || (g.x_oct & 7) || g.ld_f < g.n || (g.ld_f & 3)) return TF_EINVAL;
+    const int rc = check_gemm(a, TFL_EPI_LATENT);
+    if (rc != TF_OK) return rc;
+    const int blocks = (a.n >> 5) * a.groups, carry = g.n >> 4;            // (an even number of pairs of panels: n in 64s)
+    hipLaunchKernelGGL(latent_carry_kernel, dim3(carry + blocks / 2), dim3(512), 0, (hipStream_t)stream, a, g, carry, blocks);
+    TFL_LAUNCH_CHECK();
+    return TF_OK;
 }

@@ -167,6 +167,7 @@ class TflGemm(_c.Structure):
 TILE_SIGNATURES = {
     "tfl_tile_abi_version": (_i32, []),
     "tfl_gemm": (_i32, [_c.POINTER(TflGemm), _i32, _i32, _vp]),
+    "tfl_gemm_carry": (_i32, [_c.POINTER(TflGemm), _c.POINTER(TflGemm), _vp]),
     "tfl_split_gemm_ws_floats": (_i64, [_i32, _i32, _i32, _i32]),
     "tfl_split_gemm": (_i32, [_vp, _vp, _i64, _vp, _i64, _vp, _i64, _i32, _i32, _i32, _i32, _vp]),
     "tfl_rows_gemm_plan": (_i64, [_i32, _i32, _i32, _c.POINTER(_c.c_int32), _c.POINTER(_c.c_int32)]),
@@ -202,6 +203,7 @@ LATENT_SIGNATURES = {
     "tfl_attn_decode_pick_nsplit": (_i32, [_i32, _i32, _i32]),
     "tfl_attn_beside_plan": (_i32, [_i32, _i32, _i32, _i32, _i64, _i32, _i32] + 3 * [_c.POINTER(_c.c_int32)]),
     "tfl_attn_beside_plan_of": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i32, _i32] + 3 * [_c.POINTER(_c.c_int32)]),
+    "tfl_latent_carry": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i32, _i32]),
     "tfl_latent_value": (_i32, [_vp, _i64, _i32, _c.POINTER(TflGemm), _vp]),
     "tfl_attn_decode_beside": (_i32, [_vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _f32, _i32, _i32, _i32, _c.POINTER(TflGemm), _vp]),
     "tfl_attn_decode": (_i32, [_vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _vp]),

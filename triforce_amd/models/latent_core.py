@@ -1,7 +1,7 @@
 """Weights and the per-layer compute of a latent-attention decoder on the HIP ops (ops_latent).
 
 Decode form of a layer (one token per sequence, any number of sequences): ten launches - [norm] [input projections, gelu] (one or two rows: one launch)
-[query up-projection + cache append] [query to latent] [attention (beside it, on CUs of its own, feed-forward down), merge, or the
+[query up-projection + cache append] [query to latent (+ a part of feed-forward down)] [attention (beside it, on CUs of its own, feed-forward down), merge, or the
 merge in the next one] [latent to value, gate] [output (+ feed-forward down), residual] [token gate] [token projection].  Prefill form: products of many
 rows (ops_rows) between the row kernels and the up-projected attention.
 """
@@ -70,26 +70,32 @@ class LatentLayer:
 
     def beside(self, rows, pages, longest=None):
         """How attention and the feed-forward's half of the output product share the chip in a decode step of rows that hold ``pages`` pages in
-        all, the longest ``longest`` (ops_latent.beside_plan); None: one after the other, as where nobody knows the pages.  (What they hold, not what the cache could:
+        all, the longest ``longest`` (ops_latent.beside_plan, carry_plan); None: one after the other, as where nobody knows the pages.  (What they hold, not what the cache could:
         for the product a CU too few costs more than a page's attention on one CU more.)"""
         g = self.geom
         if pages is None or not self.ff or not self.w_out.chunk_major or self.w_out.dtype != torch.bfloat16:
             return None
-        return ol.beside_plan(rows, g.H, g.C, g.R, pages, self.w_out.n, self.w_out.k - g.H * g.V, longest)
+        k = self.w_out.k - g.H * g.V
+        carried = ol.carry_plan(rows, g.H, g.C, g.R, pages, self.w_out.n, k, longest)
+        plan = ol.beside_plan(rows, g.H, g.C, g.R, pages, self.w_out.n, k - carried, longest)
+        return plan and (plan, carried)
 
     # -- the two forms of a layer: h (normed input), x (fp32 residual, updated) -> y (token-side output, added by the next norm) ----
     def decode(self, h, x, ids, side_table, batch, rope, cache_rows, eps):
         g = self.geom
         act = ol.empty_act(ids.numel(), self.w_out.k, h.dtype, h.device)
         raw, ss, xq = ol.input_projection(h, self.w_in, g.n_raw, self.q_norm, act, g.H * g.V)
-        qn, q = ol.query_and_append(xq, raw, ss, self.w_uq, g, self.kv_norm, eps, rope, batch.pos, batch.slot, cache_rows)
-        ol.query_to_latent(qn, self.w_uk_t, q, g)
         own = g.H * g.V                                       # act: the attention's columns, then the feed-forward's, which wait for nothing of it
         plan = self.beside(ids.numel(), batch.pages, batch.longest)
+        qn, q = ol.query_and_append(xq, raw, ss, self.w_uq, g, self.kv_norm, eps, rope, batch.pos, batch.slot, cache_rows)
         if plan is None:
+            ol.query_to_latent(qn, self.w_uk_t, q, g)
             o = ol.attn_decode(q, cache_rows, batch.table, batch.klen, g, self.scale, batch.max_len)
         else:
-            o = ol.attn_decode_beside(q, cache_rows, batch.table, batch.klen, g, self.scale, plan, act, self.w_out, x, own)
+            beside, carried = plan
+            rest = self.w_out.k - carried
+            ol.query_to_latent(qn, self.w_uk_t, q, g, ol.part_of(act, self.w_out, x, rest, self.w_out.k) if carried else None)
+            o = ol.attn_decode_beside(q, cache_rows, batch.table, batch.klen, g, self.scale, beside, act, self.w_out, x, own, rest)
         ol.latent_to_value(o, self.w_uv, raw, g.gate_off, act, g)
         xt = ol.add_linear(act, self.w_out, x, want_copy=bool(self.side_dim), k=None if plan is None else own)
         if not self.side_dim:

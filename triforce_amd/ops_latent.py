@@ -11,7 +11,7 @@ import torch
 
 from . import hip
 from .ops_tile import (_CODE, PAGE, TileWeight, _f32, _gemm, _i32, _lay, _need, _p, _stream, _tail, act_rows, decode_prep, empty_act, linear_rows,  # noqa: F401
-                       linear_f32, pack_tiles, pad32)
+                       linear_f32, pack_tiles, pad32, part_of)
 
 class Finish:
     """finish() of decode rows that the product which reads them makes for itself (tfl_finish_gemm): stands for its activation block; ``out`` is the
@@ -93,12 +93,12 @@ def query_and_append(xq, raw, ss, wt, g, kv_norm, eps, rope, pos, slot, cache):
     return qn, q
 
 
-def query_to_latent(qn, wt, q, g):
-    """q[:, h, :C] = qn[:, h] . Wuk_h (wt: groups of [C, N])."""
+def query_to_latent(qn, wt, q, g, carried=None):
+    """q[:, h, :C] = qn[:, h] . Wuk_h (wt: groups of [C, N]).  ``carried``: a product (part_of) in the same launch."""
     _need(qn, q)
     rows = qn.shape[0]
     assert (wt.groups, wt.n, wt.k) == (g.H, g.C, g.N) and qn.dtype == q.dtype == wt.dtype
-    _gemm(wt, qn, "latent", rows, ld_x=g.H * g.N, x_group=g.N, out_t=q, H=g.H, C=g.C, R=g.R)
+    _gemm(wt, qn, "latent", rows, carried, ld_x=g.H * g.N, x_group=g.N, out_t=q, H=g.H, C=g.C, R=g.R)
     return q
 
 
@@ -281,6 +281,14 @@ def beside_plan(rows, H, C, R, pages, n, k, longest=None):
     return (workers, each.value, nsplit.value, _value_merges(rows, H, nsplit.value, parts.value)) if workers > 0 else None
 
 
+@functools.lru_cache(maxsize=1024)
+def carry_plan(rows, H, C, R, pages, n, k, longest=None):
+    """Columns of such a product, from the last on, that query_to_latent carries (0: none); what is left goes beside the attention as its own beside_plan says."""
+    if longest is None:
+        longest = pages if rows <= 1 else (4 * pages - 1) // (3 * rows) + 1
+    return hip.latent_lib().tfl_latent_carry(rows, H, C, R, pages, longest, n, k)
+
+
 class Splits:
     """What attn_decode_beside leaves to latent_to_value: unmerged splits of [rows, H, C]."""
 
@@ -288,24 +296,18 @@ class Splits:
         self.ws, self.nsplit, self.shape, self.dtype, self.is_cuda = ws, nsplit, shape, dtype, ws.is_cuda
 
 
-def attn_decode_beside(q, cache, table, klen, g, scale, plan, act, wt, x, k0):
-    """attn_decode of bfloat16 rows of 512 + 64 with x += act . W^T over the columns from k0 on in the same launch.  Splits as the plan says."""
-    _need(q, cache, table, klen, act, x)
+def attn_decode_beside(q, cache, table, klen, g, scale, plan, act, wt, x, k0, k1=None):
+    """attn_decode of bfloat16 rows of 512 + 64 with x += act . W^T over the columns from k0 on (to k1) in the same launch.  Splits as the plan says."""
+    product = part_of(act, wt, x, k0, wt.k if k1 is None else k1)
+    _need(q, cache, table, klen)
     _i32(table, klen)
-    _f32(x)
     rows, (workers, each, nsplit, later) = q.shape[0], plan
-    assert q.dtype == cache.dtype == act.dtype == wt.dtype == torch.bfloat16 and q.is_contiguous() and q.shape[1:] == (g.H, 576) and (g.C, g.R) == (512, 64)
+    assert q.dtype == cache.dtype == torch.bfloat16 and product.rows == rows and q.is_contiguous() and q.shape[1:] == (g.H, 576) and (g.C, g.R) == (512, 64)
     assert cache.is_contiguous() and cache.shape[1] == 576 and cache.shape[0] % PAGE == 0
     assert table.shape[0] == rows and table.stride(1) == 1 and klen.numel() == rows
-    assert act.dim() == 3 and act.is_contiguous() and act.shape[:2] == (wt.k // 8, rows) and x.shape == (rows, wt.n) and x.is_contiguous()
-    assert wt.chunk_major and 0 <= k0 < wt.k and k0 % 32 == 0
     L = hip.latent_lib()
     ws = torch.empty(L.tfl_attn_decode_ws_floats(rows, g.H, g.C, nsplit), dtype=torch.float32, device=q.device)
     out = None if later else torch.empty(rows, g.H, g.C, dtype=q.dtype, device=q.device)
-    a = hip.TflGemm()
-    a.wp, a.x, a.out_f = wt.packed.data_ptr() + 2 * k0 * wt.n, act[k0 // 8:].data_ptr(), x.data_ptr()
-    a.rows, a.n, a.k, a.groups, a.chunk_major, a.ld_f = rows, wt.n, wt.k - k0, 1, 1, x.stride(0)
-    a.ld_x, a.x_oct, a.t_oct = 8, 8 * rows, 8
     hip.check(L.tfl_attn_decode_beside(_p(q), _p(cache), cache.shape[0] // PAGE, _p(table), table.stride(0), _p(klen), _p(out), _p(ws), ws.numel(), rows, g.H,
-                                       float(scale), nsplit, workers, each, ctypes.byref(a), _stream()), "tfl_attn_decode_beside")
+                                       float(scale), nsplit, workers, each, ctypes.byref(product), _stream()), "tfl_attn_decode_beside")
     return Splits(ws, nsplit, (rows, g.H, g.C), q.dtype) if later else out

@@ -124,7 +124,22 @@ def _tail(x, k):
     return x[k // 8:] if x.dim() == 3 else x[:, k:]
 
 
-def _gemm(wt, x, epi, rows, **kw):
+def part_of(act, wt, x, k0, k1):
+    """x (fp32) += act . W^T over the columns k0 .. k1 - 1 of both, as a product that another launch carries (_gemm, tfl_attn_decode_beside): the octet-major
+    block act, chunk-major weights.  The tensors have to outlive the launch's enqueueing only."""
+    _need(act, x)
+    _f32(x)
+    assert act.dim() == 3 and act.is_contiguous() and act.dtype == wt.dtype == torch.bfloat16 and wt.chunk_major
+    rows = act.shape[1]
+    assert act.shape[0] == wt.k // 8 and x.shape == (rows, wt.n) and x.is_contiguous() and 0 <= k0 < k1 <= wt.k and k0 % 32 == 0 and k1 % 32 == 0
+    a = hip.TflGemm()
+    a.wp, a.x, a.out_f = wt.packed.data_ptr() + 2 * k0 * wt.n, act[k0 // 8:].data_ptr(), x.data_ptr()
+    a.rows, a.n, a.k, a.groups, a.chunk_major, a.ld_f = rows, wt.n, k1 - k0, 1, 1, x.stride(0)
+    a.ld_x, a.x_oct, a.t_oct = 8, 8 * rows, 8
+    return a
+
+
+def _gemm(wt, x, epi, rows, carried=None, **kw):
     a = hip.TflGemm()
     a.wp, a.x = wt.packed.data_ptr(), x.data_ptr()
     a.rows, a.n, a.k, a.groups = rows, wt.n, wt.k, wt.groups
@@ -132,6 +147,10 @@ def _gemm(wt, x, epi, rows, **kw):
     a.chunk_major = int(wt.chunk_major)
     for name, v in kw.items():
         setattr(a, name, v.data_ptr() if isinstance(v, torch.Tensor) else v)
+    if carried is not None:
+        assert wt.dtype == torch.bfloat16 and epi == "latent"
+        hip.check(hip.tile_lib().tfl_gemm_carry(ctypes.byref(a), ctypes.byref(carried), _stream()), "tfl_gemm_carry")
+        return
     hip.check(hip.tile_lib().tfl_gemm(ctypes.byref(a), _CODE[wt.dtype], hip.TFL_EPI[epi], _stream()), "tfl_gemm " + epi)
 
 
