@@ -49,6 +49,17 @@ typedef struct TfhConnect {
 int tfh_connect_gemm_takes(int rows, int streams, int width, int n, int k, int epilogue);
 int tfh_connect_gemm(const TfhConnect* f, const TflGemm* product, int epilogue, void* stream);
 
+/* The same between two wide products of any number of rows, up to 4 streams, without a launch of its own (bfloat16, chunk-major weights).
+ * tfh_streams_gemm: y = product->x . W^T of a sublayer's last product (n = width) goes into the streams (f->y is not read; f->x_out: x itself, another block, or
+ *   NULL), product->out_t = u * norm_w, an activation block without the norm's scale, and product->ss_out[m*ss_ld + n/16] = sums of u^2 over each panel.
+ * tfh_scaled_gemm: TFL_EPI_F32 or TFL_EPI_GLU of rows that are scaled by 1 / sqrt(sum(ss_in[m][:ss_n]) / k_real + eps) behind the product; ss_n and ss_ld in fours,
+ *   up to 512.
+ * TF_ERANGE: not a size of these forms; the _takes functions say so beforehand. */
+int tfh_streams_gemm_takes(int rows, int streams, int n, int k);
+int tfh_streams_gemm(const TfhConnect* f, const TflGemm* product, void* stream);
+int tfh_scaled_gemm_takes(int rows, int n, int epilogue);
+int tfh_scaled_gemm(const TflGemm* a, int epilogue, void* stream);
+
 /* ---- prefill ----------------------------------------------------------------------------------------------------------- */
 
 /* Queries and keys of new tokens: per head x / rms * norm, then entries i and i + half of the first 2 * half turn at pos[token];

@@ -21,7 +21,7 @@ LIBRARIES = {
     "core": (LIB_PATH, SOURCES, ["common.h", "gemv_common.h", "share_shape.h", "lanes.h", "tree_mask.h", "select_common.h", "prefill_wide.h", "lds_dma.h", "rows_gemm.h"], ["triforce_hip.h"]),
     "tile": (TILE_LIB_PATH, ["tile_gemm.hip", "split_gemm.hip", "tile_rows_gemm.hip", "paged.hip"], ["tile_common.h", "lanes.h", "lds_dma.h", "share_gemm.h", "share_shape.h", "rows_gemm.h"], ["triforce_tile.h"]),
     "latent": (LATENT_LIB_PATH, ["latent_attn.hip", "latent_ops.hip", "latent_finish.hip", "latent_token.hip"], ["tile_common.h", "lanes.h", "lds_dma.h", "flash_tile.h", "share_gemm.h", "share_shape.h", "row_source.h"], ["triforce_tile.h", "triforce_latent.h"]),
-    "hybrid": (HYBRID_LIB_PATH, ["hybrid_rec.hip", "hybrid_attn.hip", "hybrid_step.hip", "hybrid_ops.hip", "hybrid_connect.hip"],
+    "hybrid": (HYBRID_LIB_PATH, ["hybrid_rec.hip", "hybrid_attn.hip", "hybrid_step.hip", "hybrid_ops.hip", "hybrid_connect.hip", "hybrid_streams.hip"],
                ["tile_common.h", "lanes.h", "flash_tile.h", "hybrid_common.h", "share_gemm.h", "share_shape.h", "row_source.h"],
                ["triforce_tile.h", "triforce_hybrid.h"]),
 }

@@ -4,13 +4,14 @@
 #include "share_shape.h"
 #include "row_source.h"
 
-// connect_kernel (hybrid_ops.hip) between two sublayers as a product's source of x: up to S streams of rows of up to 4 096.
+// connect_kernel (hybrid_ops.hip) between two sublayers as a product's source of x: up to S streams of rows of up to 4 096.  For widths whose last products are not
+// whole panels of every CU (4 096 is, see hybrid_streams.hip, and is faster there: eight steps of four layers 3 670 -> 3 609).
 // A launch of its own is 5 us of round trips in which memory idles; here they run under the first 160 KB of weights of every CU.  One row, apart -> together:
 // 18 752 x 4 096 5.0 + 26.3 -> 28.2 us, gate | up of 22 016 5.0 + 30.5 -> 32.1; eight steps of four layers 3 831 -> 3 683.  Two rows of four streams are 160 KB
 // for every workgroup and take longer than the launch that they save (3 905 -> 3 986).
 template <int S>
 struct ConnectSource {
-    static constexpr bool INSIDE = true;
+    static constexpr bool INSIDE = true, SCALED = false, TILE = false;
     static constexpr int ROWS = 1;
     const TfhConnect& f;
     bf16* xs;                                                 // [width / 8][rows][8]

@@ -58,7 +58,10 @@ __device__ __forceinline__ void finish_raw(const TflGemm& a, int m, bool live, i
 // cu: this workgroup's place among those that share the panels, mb: its block of rows.
 // Src: where x comes from.  FromMemory: a.x, asked for with the weights.  Otherwise (INSIDE, one block of rows) the workgroup makes it itself under the first
 // two batches of weights: src.ask() issues its loads in front of them, src.make() leaves x in LDS, octet-major, and ends with a barrier.
-struct FromMemory { static constexpr bool INSIDE = false; };
+// SCALED: row m of the result is a.x's times 1 / sqrt(sum(a.ss_in[m]) / a.k_real + a.eps) before anything else is done with it; what is asked for in front of
+// the weights is added up while the first of them come.  TILE: src.ask_tile() and src.put_tile() in the place of an epilogue (one tile a wave, whole panels).
+struct FromMemory { static constexpr bool INSIDE = false, SCALED = false, TILE = false; };
+struct FromMemoryScaled { static constexpr bool INSIDE = false, SCALED = true, TILE = false; };
 template <typename T, int EPI, int P, bool TAIL, int MT, int U, class Src = FromMemory>
 __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail_rows, const int tail_per, const int cu, const int mb, char* share_smem,
                                                 Src src = Src()) {
@@ -139,6 +142,31 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
         return v;
     };
     const f32x4 first = beside(wave);
+    if constexpr (Src::TILE)
+        if (wave < NP * MT) src.ask_tile(min(m0 + 16 * (wave % MT) + i, a.rows - 1), 16 * (panel0 + min(wave / MT, NP - 1)) + 4 * g);
+    constexpr int TPR = 512 / (16 * MT), SQ = 128 / TPR;      // SCALED: threads a row, quads of its sums of squares each (512 sums)
+    [[maybe_unused]] f32x4 sq[SQ];
+    [[maybe_unused]] float* const scale = reinterpret_cast<float*>(share_smem + sizeof(f32x4) * WAVES * NP * MT * 64);
+    if constexpr (Src::SCALED) {
+        const float* ss = a.ss_in + (int64_t)min(m0 + tid / TPR, a.rows - 1) * a.ss_ld;
+#pragma unroll
+        for (int u = 0; u < SQ; ++u) sq[u] = *reinterpret_cast<const f32x4*>(ss + 4 * min(tid % TPR + u * TPR, (a.ss_n >> 2) - 1));
+    }
+    [[maybe_unused]] auto row_scales = [&] {
+        float q = 0.f;
+#pragma unroll
+        for (int u = 0; u < SQ; ++u)
+            if (tid % TPR + u * TPR < a.ss_n >> 2) q += (sq[u][0] + sq[u][1]) + (sq[u][2] + sq[u][3]);
+        q += lane_rotated<8>(q);
+        q += lane_rotated<4>(q);
+        q += lane_rotated<2>(q);
+        q += lane_rotated<1>(q);
+        if constexpr (TPR == 32) {
+            const LanePair<float> r = lane_rows(q);
+            q = r.a + r.b;
+        }
+        if (tid % TPR == 0) scale[tid / TPR] = 1.0f / sqrtf(q / (float)a.k_real + a.eps);
+    };
     asm volatile("" ::: "memory");
     if constexpr (Src::INSIDE) {
         static_assert(MT == 1, "one block of rows");
@@ -171,9 +199,13 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
             take(c0 + U);
             multiply(wb, x, c0 + U);
         }
-    } else if (n_own > 0) {
+    } else {
         Frag wa[U][NP], xa[U][MT], wb[U][NP], xb[U][MT];
-        load(wa, xa, 0);
+        if (n_own > 0) load(wa, xa, 0);
+        if constexpr (Src::SCALED) {
+            __builtin_amdgcn_sched_barrier(0);
+            row_scales();
+        }
         for (int c0 = 0; c0 < n_own; c0 += 2 * U) {
             load(wb, xb, c0 + U);
             multiply(wa, xa, c0);
@@ -196,7 +228,17 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
 #pragma unroll
             for (int r = 0; r < 4; ++r) s[r] += o[r];
         }
+        if constexpr (Src::SCALED) {
+            const float by = scale[16 * t + i];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) s[r] *= by;
+        }
         const bool live = m < a.rows;
+        if constexpr (Src::TILE) {
+            static_assert(!TAIL && NP * MT <= WAVES, "one tile a wave");
+            src.put_tile(m, live, panel0 + p, npan, g, s);
+            continue;
+        }
         const f32x4 with = j == wave ? first : beside(j);
         if (!TAIL || p < P) {
             const int panel = panel0 + p, n = 16 * panel + 4 * g;

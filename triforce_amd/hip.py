@@ -245,6 +245,10 @@ class TfhConnect(_c.Structure):
 
 HYBRID_SIGNATURES = {
     "tfh_connect_gemm_takes": (_i32, [_i32] * 6),
+    "tfh_streams_gemm_takes": (_i32, [_i32] * 4),
+    "tfh_streams_gemm": (_i32, [_c.POINTER(TfhConnect), _c.POINTER(TflGemm), _vp]),
+    "tfh_scaled_gemm_takes": (_i32, [_i32] * 3),
+    "tfh_scaled_gemm": (_i32, [_c.POINTER(TflGemm), _i32, _vp]),
     "tfh_connect_gemm": (_i32, [_c.POINTER(TfhConnect), _c.POINTER(TflGemm), _i32, _vp]),
     "tfh_abi_version": (_i32, []),
     "tfh_connect": (_i32, [_vp, _vp, _i32, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _vp, _i64, _i64, _i32, _i32, _i32,

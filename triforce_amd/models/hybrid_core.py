@@ -166,11 +166,11 @@ class ParallelMixer:
     def recurrence_units(self):
         return _units(self.right.geom)
 
-    def decode(self, h, batch, rope, cache_rows, states, eps):
+    def decode(self, h, batch, rope, cache_rows, states, eps, to=None):
         raw = oh.linear_of(h, self.w_in, self.w_in.n)
         step = oh.MixerStep(raw, batch.klen, eps, h.dtype, attn=self.left.step(batch, rope, cache_rows, self.spec.left_scale),
                             rec=self.right.step(batch, states, self.spec.right_scale), max_keys=batch.max_len)
-        return oh.linear_f32(step.run().operand(), self.w_out, self.w_out.n)
+        return oh.result_of(step.run().operand(), self.w_out, to)
 
     def prefill(self, h, batch, rope, cache_rows, states, eps):
         y = self.w_in.matmul(h)
@@ -211,13 +211,13 @@ class LinearAttentionMixer:
     def recurrence_units(self):
         return _units(self.geom)
 
-    def decode(self, h, batch, rope, cache_rows, states, eps):
+    def decode(self, h, batch, rope, cache_rows, states, eps, to=None):
         g = self.geom
         raw = oh.linear_of(h, self.w_in, self.w_in.n)
         rec = dict(a2=self.a2, a2_b=self.a2_b, norm_w=self.norm_w, state=states["state"], seat=batch.seat, gate_off=g.gate_off, q_off=g.q_off,
                    k_off=g.k_off, v_off=g.v_off, a_off=g.a_off, rank=g.rank, H=g.H, per_group=1, N=g.N, V=g.V, V_real=g.v_real,
                    norm_groups=g.norm_groups, inv_tau=1.0 / self.spec.tau, q_scale=self.q_scale, out_scale=1.0)
-        return oh.linear_f32(oh.MixerStep(raw, batch.klen, eps, h.dtype, rec=rec).run().operand(), self.w_out, self.w_out.n)
+        return oh.result_of(oh.MixerStep(raw, batch.klen, eps, h.dtype, rec=rec).run().operand(), self.w_out, to)
 
     def prefill(self, h, batch, rope, cache_rows, states, eps):
         g = self.geom
@@ -242,8 +242,8 @@ class GatedFeedForward:
         self.w_gu = TileWeight(oh.interleave_glu(grow(get("gate").to(dtype), F, W), grow(get("up").to(dtype), F, W)))
         self.w_down = TileWeight(grow(get("down").to(dtype), W, F))
 
-    def decode(self, h):
-        return oh.linear_f32(oh.gelu_glu_of(h, self.w_gu), self.w_down, self.w_down.n)
+    def decode(self, h, to=None):
+        return oh.result_of(oh.gelu_glu_of(h, self.w_gu), self.w_down, to)
 
     def prefill(self, h):
         act = self.w_gu.glu_matmul(h)

@@ -108,15 +108,29 @@ class KemuraxForCausalLM:
                 return h, h.out
             before = first if hc is None else dict(y=y, out=hc.out, mix=hc.mix)
             return oh.connect(x, connection.u_in, norm, eps, width, self.dtype, octets=batch.decode, **before), x
+        fused = batch.decode and W.capture is None and batch.want is None
+
+        def goes(hc, wt, following):
+            """Where the sublayer that ends with wt takes its result if that is the next one's input already (ops_hybrid.Streams)."""
+            if not fused:
+                return {}
+            connection, norm, after, epi = following
+            ok = oh.Streams.takes(x, wt, after, epi)
+            return dict(to=oh.Streams(x, hc.out, hc.mix, connection, norm, eps, width, keep=after is not W.logits)) if ok else {}
+        last = (W.final_in, W.final_norm, W.logits, "f32")
         for i, L in enumerate(W.layers):
-            h, x = read(x, L.hc1, L.norm1, L.mixer.w_in, "f32")
+            following = (W.layers[i + 1].hc1.u_in, W.layers[i + 1].norm1, W.layers[i + 1].mixer.w_in, "f32") if i + 1 < len(W.layers) else last
+            h, x = (y, x) if isinstance(y, oh.Scaled) else read(x, L.hc1, L.norm1, L.mixer.w_in, "f32")
             if W.capture is not None and i > 0:
                 W.capture.append(x.sum(1)[:, :width])
             run = L.mixer.decode if batch.decode else L.mixer.prefill
-            y, hc = run(h, batch, self._rope_of(L.spec), cache.rows[i], cache.states[i], eps), L.hc1
+            to = goes(L.hc1, L.mixer.w_out, following if L.ff is None else (L.hc2.u_in, L.norm2, L.ff.w_gu, "glu"))
+            y, hc = run(h, batch, self._rope_of(L.spec), cache.rows[i], cache.states[i], eps, **to), L.hc1
             if L.ff is not None:
-                h, x = read(x, L.hc2, L.norm2, L.ff.w_gu, "glu")
-                y, hc = (L.ff.decode if batch.decode else L.ff.prefill)(h), L.hc2
+                h, x = (y, x) if isinstance(y, oh.Scaled) else read(x, L.hc2, L.norm2, L.ff.w_gu, "glu")
+                y, hc = (L.ff.decode if batch.decode else L.ff.prefill)(h, **goes(L.hc2, L.ff.w_down, following)), L.hc2
+        if isinstance(y, oh.Scaled):
+            return y.linear(W.logits, self.vocab_size)
         if batch.want is not None and batch.want.numel() == 0:
             return None
         if batch.want is not None:

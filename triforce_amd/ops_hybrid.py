@@ -84,14 +84,88 @@ class Connect:
         return out
 
 
+class Streams:
+    """Where a sublayer's last product takes its result (tfh_streams_gemm): into the residual streams x (in place; not kept unless ``keep``), and on as the
+    next sublayer's input."""
+
+    def __init__(self, x, out, mix, u_in, norm_w, eps, width, keep=True):
+        _need(x, u_in, norm_w, out, mix)
+        _f32(x, u_in, norm_w, out, mix)
+        rows, streams, wp = x.shape
+        assert x.is_contiguous() and norm_w.numel() == wp and u_in.numel() == streams == out.numel() and mix.shape == (streams, streams) and mix.is_contiguous()
+        self.keep, self.rows, self.eps, self.width = (x, u_in, norm_w, out, mix), rows, eps, width
+        f = self.c = hip.TfhConnect()
+        for name, t in (("out", out), ("mix", mix), ("in", u_in), ("norm_w", norm_w), ("x", x), ("x_out", x if keep else None)):
+            setattr(f, name, None if t is None else t.data_ptr())
+        f.streams, f.width, f.width_real, f.eps = streams, wp, width, eps
+
+    @staticmethod
+    def takes(x, wt, after, epi):
+        """Do the product of wt into the streams x and the one of ``after`` with this epilogue ("f32", "glu") behind it have these forms?"""
+        rows, streams, wp = x.shape
+        L = _lib()
+        return (wt.chunk_major and after.chunk_major and wt.dtype == after.dtype == torch.bfloat16 and wt.n == wp == after.k
+                and L.tfh_streams_gemm_takes(rows, streams, wt.n, wt.k) == 1 and L.tfh_scaled_gemm_takes(rows, after.n, hip.TFL_EPI[epi]) == 1)
+
+    def result(self, act, wt):
+        """The input (a Scaled) that comes out of the streams behind act . W^T."""
+        _need(act)
+        rows, k, ld, octet = _lay(act)
+        assert act.dtype == wt.dtype and k == wt.k and rows == self.rows
+        h = empty_act(rows, wt.n, wt.dtype, act.device)
+        ss = torch.empty(rows, wt.n // 16, dtype=torch.float32, device=act.device)
+        a = hip.TflGemm()
+        a.wp, a.x, a.out_t, a.ss_out = wt.packed.data_ptr(), act.data_ptr(), h.data_ptr(), ss.data_ptr()
+        a.rows, a.n, a.k, a.groups, a.chunk_major, a.ld_x, a.x_oct, a.ld_t, a.t_oct, a.ss_ld = rows, wt.n, wt.k, 1, 1, ld, octet, 8, 8 * rows, wt.n // 16
+        hip.check(_lib().tfh_streams_gemm(ctypes.byref(self.c), ctypes.byref(a), _stream()), "tfh_streams_gemm")
+        return Scaled(h, ss, self.width, self.eps)
+
+
+class Scaled:
+    """An activation block whose rows still miss their norm's scale, which the next product makes of their sums of squares (tfh_scaled_gemm)."""
+
+    def __init__(self, h, ss, width, eps):
+        self.h, self.ss, self.width, self.eps, self.dtype, self.device = h, ss, width, eps, h.dtype, h.device
+
+    def _product(self, wt, epi, **kw):
+        rows, k, ld, octet = _lay(self.h)
+        assert wt.dtype == self.dtype and k == wt.k and wt.chunk_major
+        a = hip.TflGemm()
+        a.wp, a.x, a.ss_in = wt.packed.data_ptr(), self.h.data_ptr(), self.ss.data_ptr()
+        a.rows, a.n, a.k, a.groups, a.chunk_major, a.ld_x, a.x_oct, a.t_oct = rows, wt.n, wt.k, 1, 1, ld, octet, 8
+        a.ss_n = a.ss_ld = self.ss.shape[1]
+        a.k_real, a.eps = self.width, self.eps
+        for name, v in kw.items():
+            setattr(a, name, v.data_ptr() if isinstance(v, torch.Tensor) else v)
+        hip.check(_lib().tfh_scaled_gemm(ctypes.byref(a), hip.TFL_EPI[epi], _stream()), "tfh_scaled_gemm " + epi)
+
+    def linear(self, wt, n_real):
+        """linear_f32 of the rows."""
+        out = torch.empty(self.h.shape[1], n_real, dtype=torch.float32, device=self.device)
+        self._product(wt, "f32", out_f=out, ld_f=n_real, n_real=n_real)
+        return out
+
+    def gelu_glu(self, wt):
+        """gelu_glu_linear of the rows."""
+        rows = self.h.shape[1]
+        out = empty_act(rows, wt.n // 2, wt.dtype, self.device)
+        self._product(wt, "glu", out_t=out, ld_t=8, t_oct=8 * rows)
+        return out
+
+
 def linear_of(h, wt, n_real):
-    """linear_f32 of an activation block or a Connect."""
-    return h.linear(wt, n_real) if isinstance(h, Connect) else linear_f32(h, wt, n_real)
+    """linear_f32 of an activation block, a Connect or a Scaled."""
+    return h.linear(wt, n_real) if isinstance(h, (Connect, Scaled)) else linear_f32(h, wt, n_real)
 
 
 def gelu_glu_of(h, wt):
-    """gelu_glu_linear of an activation block or a Connect."""
-    return h.gelu_glu(wt) if isinstance(h, Connect) else gelu_glu_linear(h, wt)
+    """gelu_glu_linear of an activation block, a Connect or a Scaled."""
+    return h.gelu_glu(wt) if isinstance(h, (Connect, Scaled)) else gelu_glu_linear(h, wt)
+
+
+def result_of(act, wt, to):
+    """A sublayer's result: fp32 act . W^T, or with ``to`` (Streams) the next sublayer's input."""
+    return linear_f32(act, wt, wt.n) if to is None else to.result(act, wt)
 
 
 def qkv_prepare(y, g, q_norm, k_norm, eps, rope, pos, slot, cache):
