@@ -101,6 +101,12 @@ int tfl_attn_beside_plan_of(int rows, int H, int C, int R, int64_t pages, int64_
                             int32_t* parts);
 int tfl_attn_decode_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out, float* ws,
                            int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int panels_each, const TflGemm* product, void* stream);
+/* The same for 17 to 32 rows with the product's panels in eights over `parts` (1 .. 4) ranges of k each, whose sums go to product->out_f [parts][rows][n]
+ * (product->n_real = ld_f = n): parts * ceil(n / 128) workgroups.  tfl_beside_parts: how many parts, with the workers and nsplit to them, 0 where that is not the faster way.  TFL_EPI_RESIDUAL of a later product adds them (TflGemm.also). */
+int tfl_beside_parts(int rows, int H, int C, int R, int64_t pages, int64_t longest, int n, int k, int32_t* workers, int32_t* nsplit);
+int tfl_attn_decode_beside_parts(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out, float* ws,
+                                 int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int parts, const TflGemm* product, void* stream);
+
 /* Columns of the product (n of k) beside the attention, from the last on, that the query to latent product in front of it carries (tfl_gemm_carry); 0: none. */
 int tfl_latent_carry(int rows, int H, int C, int R, int64_t pages, int64_t longest, int n, int k);
 

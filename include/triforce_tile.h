@@ -69,6 +69,8 @@ typedef struct TflGemm {
     int32_t H, N, R, C, half, c_real, max_pos, cache_rows, vocab;
     float eps;
     int32_t chunk_major;            /* packed weights as [k/32][n/16][64][8] (one group) */
+    int32_t n_also;                 /* RESIDUAL of the one-workgroup-per-CU form, 17 rows and more: also[p][m][n] is added too, p < n_also (0 .. 4), blocks of [rows][n] */
+    const float* also;
 } TflGemm;
 
 int tfl_gemm(const TflGemm* a, int dtype, int epilogue, void* stream);

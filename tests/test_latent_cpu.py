@@ -164,6 +164,26 @@ def test_carried_columns():
     assert pick == [5120, 5120, 5120, 4096, 0, 5120, 6144, 0, 0]
 
 
+def test_plan_of_a_product_cut_over_k():
+    """Whatever the sizes: panels in eights over 3 or 4 ranges and the workers share 256 CUs, two workers a row at least; picked where it was measured the fastest way."""
+    from triforce_amd import ops_latent as ol
+    for rows in (1, 16, 17, 25, 32, 33):
+        for heads in (16, 17, 32, 33):
+            for pages in (0, 1, 40, 500, 2016, 100000, 1 << 21):
+                for n, k in ((4096, 11008), (4096, 4064), (4080, 11008), (8192, 8192), (8208, 8192), (6160, 4128), (4096, 14368)):
+                    for longest in (None, max(1, pages // 3)):
+                        plan = ol.parts_plan(rows, heads, 512, 64, pages, n, k, longest)
+                        if plan is None:
+                            continue
+                        workers, parts, splits = plan
+                        assert 17 <= rows <= 32 and 16 < heads <= 32 and 4096 <= n <= 8192 and 4096 <= k <= 14336 and parts in (3, 4)
+                        assert workers >= 2 * rows and workers + parts * -(-n // 128) == 256 and 2 <= splits <= 128
+    assert ol.parts_plan(20, 32, 256, 64, 64, 4096, 11008) is None and ol.parts_plan(20, 32, 512, 32, 64, 4096, 11008) is None
+    pick = [(ol.parts_plan(rows, 32, 512, 64, pages, 4096, 11008, longest) or (0, 0))[1] for rows, pages, longest in
+            ((17, 70, 5), (17, 629, 47), (20, 1457, 94), (24, 596, 32), (32, 130, 5), (32, 784, 32), (32, 1546, 63), (32, 2312, 94))]
+    assert pick == [4, 4, 3, 4, 4, 4, 3, 0]
+
+
 def test_a_step_says_how_long_its_longest_sequence_is():
     """With the token that it adds: a page's last and its first."""
     from triforce_amd.utils.batch_infer import _DecodeStep

@@ -11,7 +11,7 @@
 // for every workgroup and take longer than the launch that they save (3 905 -> 3 986).
 template <int S>
 struct ConnectSource {
-    static constexpr bool INSIDE = true, SCALED = false, TILE = false;
+    static constexpr bool INSIDE = true, SCALED = false, TILE = false, ALSO = false;
     static constexpr int ROWS = 1;
     const TfhConnect& f;
     bf16* xs;                                                 // [width / 8][rows][8]

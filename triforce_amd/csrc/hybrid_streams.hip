@@ -11,7 +11,7 @@
 // hybrid_connect.hip) 3 670 -> 3 609, 2 3 906 -> 3 680, 4 3 943 -> 3 716, 8 4 891 -> 4 603, 16 5 429 -> 5 147, 32 6 940 -> 6 641, 48 9 574 -> 9 445, 64 10 019 -> 9 893.
 template <int S>
 struct StreamsTile {
-    static constexpr bool INSIDE = false, SCALED = false, TILE = true;
+    static constexpr bool INSIDE = false, SCALED = false, TILE = true, ALSO = false;
     const TfhConnect& f;
     const TflGemm& a;
     f32x4 x[S], w;

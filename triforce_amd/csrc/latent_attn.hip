@@ -577,17 +577,32 @@ __global__ __launch_bounds__(512, 2) void attn_latent_sized_kernel(const bf16* _
 // nsplit at most, with as many pages each as that takes.  Statistics of splits that a row does not have are zero, which the merge skips.
 // us, 32 heads, attention, merge, value and the output product (shorter by 11 008 of its 15 104), apart -> so: a row of 64 pages 38.5 -> 33.6, 32 rows
 // with 1 167 pages 68.0 -> 60.1 (more beside beside_plan).
-template <int P, int MT>
+// SPLIT: the product's workgroups take P panels over one of `parts` ranges of k each and leave the range's sums in g.out_f [parts][rows][n], for the output
+// product to add.  Above 16 rows a workgroup reads as much of x as of the weights where it has two panels of all of k (704 KB each of 32 rows and k
+// 11 008), and is the longer side for it (figures at tfl_beside_parts).
+template <int P, int MT, bool SPLIT>
 __global__ __launch_bounds__(512, 2) void attn_latent_beside_kernel(const bf16* __restrict__ q, const bf16* __restrict__ cache, int n_pages,
                                                                     const int32_t* __restrict__ table, int table_ld, const int32_t* __restrict__ len,
                                                                     float* __restrict__ ws, int H, float scale, int nsplit, int rows, int workers,
-                                                                    const TflGemm g) {
+                                                                    const TflGemm g, const int parts) {
     extern __shared__ __align__(16) char smem[];
     // which of the two start first: on 128 CUs the product is the longer side up to 1 200 pages (one row of 64 pages 33.4 -> 33.2 us with it first, 32
     // rows of 1 568 61.6 -> 61.2), on 86 and 64 it is slower for it (40.0 -> 41.5, 45.1 -> 45.7)
     constexpr bool FIRST = P == 2;
     const int me = (int)blockIdx.x - (FIRST ? (int)gridDim.x - workers : 0), group = (int)blockIdx.x - (FIRST ? 0 : workers);
-    if (FIRST ? me < 0 : group >= 0) {
+    if constexpr (SPLIT) {
+        if (group >= 0) {
+            const int npan = g.n >> 4, groups = (npan + P - 1) / P, part = group / groups, chunks = g.k >> 5;
+            const int c_beg = chunks * part / parts, c_end = chunks * (part + 1) / parts;
+            TflGemm own = g;
+            own.wp = (const bf16*)g.wp + (int64_t)c_beg * npan * 512;
+            own.x = (const bf16*)g.x + 4 * g.x_oct * c_beg;
+            own.k = 32 * (c_end - c_beg);
+            own.out_f = g.out_f + (int64_t)part * g.rows * g.n;
+            share_gemm_body<bf16, TFL_EPI_F32, P, false, MT, 1>(own, 0, 0, group - part * groups, 0, smem);
+            return;
+        }
+    } else if (FIRST ? me < 0 : group >= 0) {
         share_gemm_body<bf16, TFL_EPI_RESIDUAL, P, false, MT, 2>(g, 0, 0, group, 0, smem);
         return;
     }
@@ -786,28 +801,62 @@ extern "C" int tfl_latent_carry(int rows, int H, int C, int R, int64_t pages, in
     return best;
 }
 
+// Ranges of k (3 or 4; 0: none) into which 17 to 32 rows' product is cut where that is faster than beside_plan's division or the two apart.  The times of query to
+// latent, attention, value and output product as fitted to 720 measured ones (17, 20, 24, 28, 32 rows of 300 to 6 000 keys; 17, 20, 24, 32 heads; n 4 096 to 8 192, k 4 096
+// to 14 336): 2.5 % off on average, so 2 % have to be in it.  At those 180 sizes that picks 4.5 % on average, nowhere slower, 0.3 % behind the best.  us, 32 heads,
+// n 4 096, k 11 008, as before -> cut in 3 | in 4, the pick marked: 17 rows of 300 keys 45.5 -> 47.8 | 42.2*, of 4 000 51.5 -> 54.9 | 50.2*; 32 rows of 300 53.0 -> 52.8 |
+// 47.5*, of 2 000 56.9 -> 57.2 | 52.4*, of 3 000 58.8* -> 59.7 | 60.3, of 4 000 65.4 -> 63.0* | 67.2, of 6 000 72.3* -> 75.1 | 83.1.  Up to 16 rows it is never faster (16 rows of 300
+// 43.2 -> 48.6 | 46.3), nor in one or two ranges, which leave the product too few CUs.
+extern "C" int tfl_beside_parts(int rows, int H, int C, int R, int64_t pages, int64_t longest, int n, int k, int32_t* workers, int32_t* nsplit) {
+    if (!workers || !nsplit || C != 512 || R != 64 || rows < 17 || rows > 32 || H <= 16 || H > 32 || pages < 1 || pages > (1 << 20) || longest < 1 || n < 4096 || n > 8192 || (n & 15)
+        || k < 4096 || k > 14336) return 0;
+    const double mb = 2e-6 * n * k, x = rows * k / 11008.0, heads = rows * H / 32.0, out = 2.56e-4 * n * H;
+    auto load = [&](int a) {                                  // pages of the busiest worker
+        const int most = 2 * a / rows < 128 ? 2 * a / rows : 128;
+        return fmax((double)pages / a, (double)((longest + most - 1) / most));
+    };
+    int p = 0, best = 0;
+    double least;
+    if (beside_plan(rows, H, pages, longest, n, k, &p)) {
+        const int g = ((n >> 4) + p - 1) / p;
+        const double product = 24.79 * mb / g + 0.190 * x, attention = 2.44 + 2.477 * load(256 - g);
+        least = fmax(product, attention) + 0.295 * fmin(product, attention) + 0.320 * heads + 0.163 * out + 17.15;
+    } else {
+        least = 0.4464 * mb - 1.623 * rows + 0.6034 * x * n / 4096.0 + 0.017 * pages + 1.276 * heads - 0.279 * out;
+    }
+    least *= 0.98;
+    for (int c = 3; c <= 4; ++c) {
+        const int g = c * ((n + 127) / 128), a = 256 - g;
+        if (a < 64 || a < 2 * rows) continue;
+        const double product = 22.23 * mb / g + (0.0332 * c - 0.0462) * x, attention = 2.31 + 2.568 * load(a);
+        const double t = fmax(product, attention) + 0.417 * fmin(product, attention) + 0.320 * heads + 0.163 * out + 17.15;
+        if (t < least) { least = t; best = c; *workers = a; *nsplit = 2 * a / rows < 128 ? 2 * a / rows : 128; }
+    }
+    return best;
+}
+
 // The same where nobody knows the longest row: rows half to all as long as it.
 extern "C" int tfl_attn_beside_plan(int rows, int H, int C, int R, int64_t pages, int n, int k, int32_t* panels_each, int32_t* nsplit, int32_t* parts) {
     const int64_t longest = rows < 1 || pages < rows ? 1 : (4 * pages - 1) / (3 * (int64_t)rows) + 1;
     return tfl_attn_beside_plan_of(rows, H, C, R, pages, rows == 1 ? pages : longest, n, k, panels_each, nsplit, parts);
 }
 
-template <int P, int MT>
+template <int P, int MT, bool SPLIT = false>
 static int launch_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, float* ws, int rows, int H,
-                         float scale, int nsplit, int workers, const TflGemm& g, hipStream_t st) {
+                         float scale, int nsplit, int workers, const TflGemm& g, hipStream_t st, int parts = 1) {
     constexpr int LDS = LatentTile::LDS;
     static_assert(8 * P * MT * 64 * (int)sizeof(f32x4) <= LDS, "LDS");
-    const hipError_t e = hipFuncSetAttribute((const void*)attn_latent_beside_kernel<P, MT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    const hipError_t e = hipFuncSetAttribute((const void*)attn_latent_beside_kernel<P, MT, SPLIT>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((attn_latent_beside_kernel<P, MT>), dim3(workers + ((g.n >> 4) + P - 1) / P), dim3(512), LDS, st, (const bf16*)q, (const bf16*)cache,
-                       n_pages, table, table_ld, len, ws, H, scale, nsplit, rows, workers, g);
+    hipLaunchKernelGGL((attn_latent_beside_kernel<P, MT, SPLIT>), dim3(workers + ((g.n >> 4) + P - 1) / P * parts), dim3(512), LDS, st, (const bf16*)q, (const bf16*)cache,
+                       n_pages, table, table_ld, len, ws, H, scale, nsplit, rows, workers, g, parts);
     TFL_LAUNCH_CHECK();
     return TF_OK;
 }
 
-extern "C" int tfl_attn_decode_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out,
-                                      float* ws, int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int panels_each,
-                                      const TflGemm* product, void* stream) {
+static int attn_decode_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out,
+                              float* ws, int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int panels_each,
+                                      int parts, const TflGemm* product, void* stream) {
     if (!q || !cache || !table || !len || !ws || !product || rows < 1 || rows > 32 || H <= 16 || H > 32 || n_pages < 1 || table_ld < 1) return TF_EINVAL;
     if (nsplit < 2 || nsplit > 128 || workers < 2 * rows || workers > 255) return TF_EINVAL;
     if (ws_floats < tfl_attn_decode_ws_floats(rows, H, 512, nsplit)) return TF_ENOSPC;
@@ -818,13 +867,29 @@ extern "C" int tfl_attn_decode_beside(const void* q, const void* cache, int n_pa
     int rc = TF_EINVAL;
 #define GO(P) rc = rows <= 16 ? launch_beside<P, 1>(q, cache, n_pages, table, table_ld, len, ws, rows, H, scale, nsplit, workers, g, st) \
                               : launch_beside<P, 2>(q, cache, n_pages, table, table_ld, len, ws, rows, H, scale, nsplit, workers, g, st)
-    switch (panels_each) {
+    if (parts > 0) {
+        if (panels_each == 8 && parts <= 4 && rows > 16 && g.k >= 32 * parts && g.ld_f == g.n)
+            rc = launch_beside<8, 2, true>(q, cache, n_pages, table, table_ld, len, ws, rows, H, scale, nsplit, workers, g, st, parts);
+    } else switch (panels_each) {
         case 2: GO(2); break;
         case 3: GO(3); break;
         case 4: GO(4); break;
     }
 #undef GO
     return rc == TF_OK && out ? launch_merge<bf16>(ws, out, rows, H, 512, nsplit, st) : rc;
+}
+
+extern "C" int tfl_attn_decode_beside(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out,
+                                      float* ws, int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int panels_each,
+                                      const TflGemm* product, void* stream) {
+    return attn_decode_beside(q, cache, n_pages, table, table_ld, len, out, ws, ws_floats, rows, H, scale, nsplit, workers, panels_each, 0, product, stream);
+}
+
+extern "C" int tfl_attn_decode_beside_parts(const void* q, const void* cache, int n_pages, const int32_t* table, int table_ld, const int32_t* len, void* out,
+                                            float* ws, int64_t ws_floats, int rows, int H, float scale, int nsplit, int workers, int parts,
+                                            const TflGemm* product, void* stream) {
+    if (parts < 1 || !product || product->n_real != product->n) return TF_EINVAL;
+    return attn_decode_beside(q, cache, n_pages, table, table_ld, len, out, ws, ws_floats, rows, H, scale, nsplit, workers, 8, parts, product, stream);
 }
 
 // The merge of the splits in front of latent to value: out = (merged . W_head^T) * sigmoid(gate) for up to 4 rows of 512 latents, one panel of

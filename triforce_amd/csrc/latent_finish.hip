@@ -11,7 +11,7 @@
 // rows it takes longer than the launch that it saves (4 704 -> 4 761, 4 756 -> 4 834).
 template <int ROWS>
 struct FinishSource {
-    static constexpr bool INSIDE = true, SCALED = false, TILE = false;
+    static constexpr bool INSIDE = true, SCALED = false, TILE = false, ALSO = false;
     const TflFinish& f;
     bf16* xs;                                                 // [width / 8][rows][8]
     float* red;                                               // [2][ROWS][8]

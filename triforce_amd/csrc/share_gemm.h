@@ -60,8 +60,10 @@ __device__ __forceinline__ void finish_raw(const TflGemm& a, int m, bool live, i
 // two batches of weights: src.ask() issues its loads in front of them, src.make() leaves x in LDS, octet-major, and ends with a barrier.
 // SCALED: row m of the result is a.x's times 1 / sqrt(sum(a.ss_in[m]) / a.k_real + a.eps) before anything else is done with it; what is asked for in front of
 // the weights is added up while the first of them come.  TILE: src.ask_tile() and src.put_tile() in the place of an epilogue (one tile a wave, whole panels).
-struct FromMemory { static constexpr bool INSIDE = false, SCALED = false, TILE = false; };
-struct FromMemoryScaled { static constexpr bool INSIDE = false, SCALED = true, TILE = false; };
+// ALSO: RESIDUAL adds a.n_also further parts of the sum.
+struct FromMemory { static constexpr bool INSIDE = false, SCALED = false, TILE = false, ALSO = false; };
+struct FromMemoryScaled { static constexpr bool INSIDE = false, SCALED = true, TILE = false, ALSO = false; };
+struct FromMemoryAlso { static constexpr bool INSIDE = false, SCALED = false, TILE = false, ALSO = true; };
 template <typename T, int EPI, int P, bool TAIL, int MT, int U, class Src = FromMemory>
 __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail_rows, const int tail_per, const int cu, const int mb, char* share_smem,
                                                 Src src = Src()) {
@@ -142,6 +144,19 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
         return v;
     };
     const f32x4 first = beside(wave);
+    [[maybe_unused]] f32x4 more[4];                           // ALSO: of the wave's first tile
+    [[maybe_unused]] auto also_at = [&](int j, int q) {
+        const int p = j / MT, m = m0 + 16 * (j - p * MT) + i;
+        const int n = !TAIL || p < P ? min(16 * (panel0 + p) + 4 * g, a.n - 4) : min(16 * CUS * P + tail0 + 4 * g, a.n - 4);
+        return *reinterpret_cast<const f32x4*>(a.also + ((int64_t)q * a.rows + min(m, a.rows - 1)) * a.n + n);
+    };
+    if constexpr (Src::ALSO) {
+        static_assert(EPI == TFL_EPI_RESIDUAL, "sums to be added");
+        if (wave < NP * MT) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) more[q] = also_at(wave, min(q, a.n_also - 1));
+        }
+    }
     if constexpr (Src::TILE)
         if (wave < NP * MT) src.ask_tile(min(m0 + 16 * (wave % MT) + i, a.rows - 1), 16 * (panel0 + min(wave / MT, NP - 1)) + 4 * g);
     constexpr int TPR = 512 / (16 * MT), SQ = 128 / TPR;      // SCALED: threads a row, quads of its sums of squares each (512 sums)
@@ -240,6 +255,15 @@ __device__ __forceinline__ void share_gemm_body(const TflGemm& a, const int tail
             continue;
         }
         const f32x4 with = j == wave ? first : beside(j);
+        if constexpr (Src::ALSO) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (q < a.n_also) {
+                    const f32x4 o = j == wave ? more[q] : also_at(j, q);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s[r] += o[r];
+                }
+        }
         if (!TAIL || p < P) {
             const int panel = panel0 + p, n = 16 * panel + 4 * g;
             if (panel >= npan) continue;

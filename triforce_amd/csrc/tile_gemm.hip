@@ -296,13 +296,13 @@ __global__ __launch_bounds__(512, 4) void latent_carry_kernel(const TflGemm a, c
     latent_gemm_body<bf16, TFL_EPI_LATENT, 2, 1, 4, 8, false>(a, threadIdx.x & 255, 2 * ((int)blockIdx.x - carried) + half, blocks, 0, part + 4 * half);
 }
 
-template <typename T, int EPI, int P, bool TAIL, int MT, int U>
+template <typename T, int EPI, int P, bool TAIL, int MT, int U, class Src = FromMemory>
 __global__ __launch_bounds__(512, 2) void share_gemm_kernel(const TflGemm a, const int tail_rows, const int tail_per) {
     extern __shared__ __align__(16) char share_smem[];
-    share_gemm_body<T, EPI, P, TAIL, MT, U>(a, tail_rows, tail_per, blockIdx.x, blockIdx.y, share_smem);
+    share_gemm_body<T, EPI, P, TAIL, MT, U, Src>(a, tail_rows, tail_per, blockIdx.x, blockIdx.y, share_smem);
 }
 
-template <typename T, int EPI, int P, bool TAIL, int MT>
+template <typename T, int EPI, int P, bool TAIL, int MT, class Src = FromMemory>
 static int launch_share_rows(const TflGemm& a, int tail_rows, int tail_per, hipStream_t st) {
     constexpr int NP = P + (TAIL ? 1 : 0), LDS = 8 * NP * MT * 64 * (int)sizeof(f32x4);
     // Chunks asked for ahead: what the registers hold (seven panels and two row blocks 221; with one chunk ahead 1 792 panels of 4 096 took 51.8
@@ -310,18 +310,21 @@ static int launch_share_rows(const TflGemm& a, int tail_rows, int tail_per, hipS
     constexpr int U = NP == 1 ? 4 : NP * MT <= 14 ? 2 : 1;
     static_assert(LDS <= 160 * 1024, "one workgroup's partial tiles");
     if (LDS > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute((const void*)share_gemm_kernel<T, EPI, P, TAIL, MT, U>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+        const hipError_t e = hipFuncSetAttribute((const void*)share_gemm_kernel<T, EPI, P, TAIL, MT, U, Src>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
         if (e != hipSuccess) return (int)e;
     }
     const int panels = a.n >> 4;
     const dim3 grid(TAIL ? 256 : (panels + P - 1) / P, (a.rows + 16 * MT - 1) / (16 * MT));
-    hipLaunchKernelGGL((share_gemm_kernel<T, EPI, P, TAIL, MT, U>), grid, dim3(512), LDS, st, a, tail_rows, tail_per);
+    hipLaunchKernelGGL((share_gemm_kernel<T, EPI, P, TAIL, MT, U, Src>), grid, dim3(512), LDS, st, a, tail_rows, tail_per);
     TFL_LAUNCH_CHECK();
     return TF_OK;
 }
 
 template <typename T, int EPI, int P, bool TAIL>
 static int launch_share(const TflGemm& a, int tail_rows, int tail_per, hipStream_t st) {
+    if constexpr (EPI == TFL_EPI_RESIDUAL) {                  // (forms of their own: asked about in these, one row, six layer runs, eight steps 4 134 -> 4 162 us)
+        if (a.n_also > 0) return launch_share_rows<T, EPI, P, TAIL, 2, FromMemoryAlso>(a, tail_rows, tail_per, st);
+    }
     return a.rows <= 16 ? launch_share_rows<T, EPI, P, TAIL, 1>(a, tail_rows, tail_per, st)
                         : launch_share_rows<T, EPI, P, TAIL, 2>(a, tail_rows, tail_per, st);
 }
@@ -404,7 +407,8 @@ static int dispatch_gemm(const TflGemm& a, int epi, hipStream_t st) {
 }
 
 // What an epilogue asks of its operands.
-static int check_gemm(const TflGemm& a, int epi) {
+static int check_gemm(const TflGemm& a, int dtype, int epi) {
+    if (a.n_also && (epi != TFL_EPI_RESIDUAL || dtype != 0)) return TF_EINVAL;
     switch (epi) {
         case TFL_EPI_F32:
             if (!a.out_f || a.groups != 1 || a.n_real < 1 || a.n_real > a.n || a.ld_f < a.n_real) return TF_EINVAL;
@@ -430,6 +434,7 @@ static int check_gemm(const TflGemm& a, int epi) {
             if (!a.out_t || !a.gate || a.ld_t < 8 || a.ld_gate < (int64_t)a.groups * a.n || (a.ld_t & 7) || (a.ld_gate & 3)) return TF_EINVAL;
             break;
         case TFL_EPI_RESIDUAL:
+            if (a.n_also < 0 || a.n_also > 4 || (a.n_also && (a.rows <= 16 || !a.also || !a.chunk_major || share_shape(a.n >> 4, false, 0, a.rows).each == 0))) return TF_EINVAL;
             if (!a.out_f || a.groups != 1 || a.ld_f < a.n || (a.ld_f & 3) || (a.out_t && (a.ld_t < 8 || (a.ld_t & 7)))) return TF_EINVAL;
             break;
         case TFL_EPI_TOKEN:
@@ -453,7 +458,7 @@ extern "C" int tfl_gemm(const TflGemm* p, int dtype, int epi, void* stream) {
     if (a.chunk_major != 0 && (a.chunk_major != 1 || a.groups != 1)) return TF_EINVAL;
     if (a.out_t && (a.t_oct < 8 || (a.t_oct & 7))) return TF_EINVAL;
     if (dtype != 0 && dtype != 1) return TF_EINVAL;
-    const int rc = check_gemm(a, epi);
+    const int rc = check_gemm(a, dtype, epi);
     if (rc != TF_OK) return rc;
     return dtype == 0 ? dispatch_gemm<bf16>(a, epi, (hipStream_t)stream) : dispatch_gemm<float>(a, epi, (hipStream_t)stream);
 }
@@ -465,7 +470,7 @@ extern "C" int tfl_gemm_carry(const TflGemm* p, const TflGemm* carried, void* st
         || (a.ld_x & 7) || (a.x_group & 7) || a.x_oct < 8 || (a.x_oct & 7) || a.ld_x < 8) return TF_EINVAL;
     if (!g.wp || !g.x || !g.out_f || g.out_t || g.rows != a.rows || g.n < 16 || (g.n & 15) || g.n > (1 << 16) || g.k < 32 || (g.k & 31) || g.groups != 1 || g.chunk_major != 1
         || (g.ld_x & 7) || g.ld_x < 8 || g.x_oct < 8 || (g.x_oct & 7) || g.ld_f < g.n || (g.ld_f & 3)) return TF_EINVAL;
-    const int rc = check_gemm(a, TFL_EPI_LATENT);
+    const int rc = check_gemm(a, 0, TFL_EPI_LATENT);
     if (rc != TF_OK) return rc;
     const int blocks = (a.n >> 5) * a.groups, carry = g.n >> 4;            // (an even number of pairs of panels: n in 64s)
     hipLaunchKernelGGL(latent_carry_kernel, dim3(carry + blocks / 2), dim3(512), 0, (hipStream_t)stream, a, g, carry, blocks);

@@ -161,7 +161,7 @@ class TflGemm(_c.Structure):
                 + [(n, _i64) for n in ("ld_x", "x_oct", "x_group", "ld_t", "t_oct", "ld_f", "ld_gate", "ld_tok", "ld_kv")]
                 + [(n, _i32) for n in ("rows", "n", "k", "groups", "n_real", "k_real", "n_raw", "n_scaled", "ss_n", "ss_ld", "H", "N", "R", "C",
                                        "half", "c_real", "max_pos", "cache_rows", "vocab")]
-                + [("eps", _f32), ("chunk_major", _i32)])
+                + [("eps", _f32), ("chunk_major", _i32), ("n_also", _i32), ("also", _vp)])
 
 
 TILE_SIGNATURES = {
@@ -203,6 +203,8 @@ LATENT_SIGNATURES = {
     "tfl_attn_decode_pick_nsplit": (_i32, [_i32, _i32, _i32]),
     "tfl_attn_beside_plan": (_i32, [_i32, _i32, _i32, _i32, _i64, _i32, _i32] + 3 * [_c.POINTER(_c.c_int32)]),
     "tfl_attn_beside_plan_of": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i32, _i32] + 3 * [_c.POINTER(_c.c_int32)]),
+    "tfl_attn_decode_beside_parts": (_i32, [_vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _f32, _i32, _i32, _i32, _c.POINTER(TflGemm), _vp]),
+    "tfl_beside_parts": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i32, _i32, _c.POINTER(_c.c_int32), _c.POINTER(_c.c_int32)]),
     "tfl_latent_carry": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i32, _i32]),
     "tfl_latent_value": (_i32, [_vp, _i64, _i32, _c.POINTER(TflGemm), _vp]),
     "tfl_attn_decode_beside": (_i32, [_vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _f32, _i32, _i32, _i32, _c.POINTER(TflGemm), _vp]),

@@ -70,15 +70,18 @@ class LatentLayer:
 
     def beside(self, rows, pages, longest=None):
         """How attention and the feed-forward's half of the output product share the chip in a decode step of rows that hold ``pages`` pages in
-        all, the longest ``longest`` (ops_latent.beside_plan, carry_plan); None: one after the other, as where nobody knows the pages.  (What they hold, not what the cache could:
+        all, the longest ``longest`` ((ops_latent.beside_plan, columns by carry_plan, False) or (parts_plan, 0, True)); None: one after the other, as where nobody knows the pages.  (What they hold, not what the cache could:
         for the product a CU too few costs more than a page's attention on one CU more.)"""
         g = self.geom
         if pages is None or not self.ff or not self.w_out.chunk_major or self.w_out.dtype != torch.bfloat16:
             return None
         k = self.w_out.k - g.H * g.V
+        parts = ol.parts_plan(rows, g.H, g.C, g.R, pages, self.w_out.n, k, longest)
+        if parts is not None:
+            return parts, 0, True
         carried = ol.carry_plan(rows, g.H, g.C, g.R, pages, self.w_out.n, k, longest)
         plan = ol.beside_plan(rows, g.H, g.C, g.R, pages, self.w_out.n, k - carried, longest)
-        return plan and (plan, carried)
+        return plan and (plan, carried, False)
 
     # -- the two forms of a layer: h (normed input), x (fp32 residual, updated) -> y (token-side output, added by the next norm) ----
     def decode(self, h, x, ids, side_table, batch, rope, cache_rows, eps):
@@ -88,16 +91,20 @@ class LatentLayer:
         own = g.H * g.V                                       # act: the attention's columns, then the feed-forward's, which wait for nothing of it
         plan = self.beside(ids.numel(), batch.pages, batch.longest)
         qn, q = ol.query_and_append(xq, raw, ss, self.w_uq, g, self.kv_norm, eps, rope, batch.pos, batch.slot, cache_rows)
+        sums = None
         if plan is None:
             ol.query_to_latent(qn, self.w_uk_t, q, g)
             o = ol.attn_decode(q, cache_rows, batch.table, batch.klen, g, self.scale, batch.max_len)
         else:
-            beside, carried = plan
+            beside, carried, cut = plan
             rest = self.w_out.k - carried
             ol.query_to_latent(qn, self.w_uk_t, q, g, ol.part_of(act, self.w_out, x, rest, self.w_out.k) if carried else None)
-            o = ol.attn_decode_beside(q, cache_rows, batch.table, batch.klen, g, self.scale, beside, act, self.w_out, x, own, rest)
+            if cut:
+                o, sums = ol.attn_decode_beside_parts(q, cache_rows, batch.table, batch.klen, g, self.scale, beside, act, self.w_out, own, rest)
+            else:
+                o = ol.attn_decode_beside(q, cache_rows, batch.table, batch.klen, g, self.scale, beside, act, self.w_out, x, own, rest)
         ol.latent_to_value(o, self.w_uv, raw, g.gate_off, act, g)
-        xt = ol.add_linear(act, self.w_out, x, want_copy=bool(self.side_dim), k=None if plan is None else own)
+        xt = ol.add_linear(act, self.w_out, x, want_copy=bool(self.side_dim), k=None if plan is None else own, also=sums)
         if not self.side_dim:
             return None
         return ol.token_side(xt, self.side_gate, self.side_proj, side_table, ids, self.side_dim, self.width)

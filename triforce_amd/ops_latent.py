@@ -118,17 +118,18 @@ def latent_to_value(ol, wt, raw, gate_off, act, g):
           ld_t=act_ld, t_oct=act_oct)
 
 
-def add_linear(act, wt, x, want_copy=False, k=None):
+def add_linear(act, wt, x, want_copy=False, k=None, also=None):
     """x (fp32) += act . W^T, over the first ``k`` columns of both if given (chunk-major weights); returns the sum as an octet-major
-    block of act's type when ``want_copy``."""
-    _need(act, x)
-    _f32(x)
+    block of act's type when ``want_copy``.  ``also``: fp32 [parts][rows][n] to be added too (attn_decode_beside_parts)."""
+    _need(act, x, also)
+    _f32(x, also)
     rows, have, ld, octet = _lay(act)
     assert act.dtype == wt.dtype and have == wt.k and x.shape == (rows, wt.n) and x.is_contiguous()
     assert k is None or (wt.chunk_major and 0 < k <= have and k % 32 == 0)
+    assert also is None or (also.shape[1:] == x.shape and also.is_contiguous() and 1 <= also.shape[0] <= 4)
     xt = empty_act(rows, wt.n, wt.dtype, x.device) if want_copy else None
     _gemm(wt, act, "residual", rows, ld_x=ld, x_oct=octet, out_f=x, ld_f=x.stride(0), k=have if k is None else k,
-          **(dict(out_t=xt, ld_t=8, t_oct=8 * rows) if want_copy else {}))
+          **(dict(out_t=xt, ld_t=8, t_oct=8 * rows) if want_copy else {}), **(dict(also=also, n_also=also.shape[0]) if also is not None else {}))
     return xt
 
 
@@ -284,9 +285,20 @@ def beside_plan(rows, H, C, R, pages, n, k, longest=None):
 @functools.lru_cache(maxsize=1024)
 def carry_plan(rows, H, C, R, pages, n, k, longest=None):
     """Columns of such a product, from the last on, that query_to_latent carries (0: none); what is left goes beside the attention as its own beside_plan says."""
-    if longest is None:
-        longest = pages if rows <= 1 else (4 * pages - 1) // (3 * rows) + 1
-    return hip.latent_lib().tfl_latent_carry(rows, H, C, R, pages, longest, n, k)
+    return hip.latent_lib().tfl_latent_carry(rows, H, C, R, pages, _longest(rows, pages, longest), n, k)
+
+
+def _longest(rows, pages, longest):
+    """As tfl_attn_beside_plan takes it where nobody knows: rows half to all as long as it."""
+    return longest if longest is not None else pages if rows <= 1 else (4 * pages - 1) // (3 * rows) + 1
+
+
+@functools.lru_cache(maxsize=1024)
+def parts_plan(rows, H, C, R, pages, n, k, longest=None):
+    """(workers, parts, splits) of attn_decode_beside_parts, None where beside_plan's division, or the two apart, are the faster way."""
+    workers, nsplit = ctypes.c_int32(), ctypes.c_int32()
+    parts = hip.latent_lib().tfl_beside_parts(rows, H, C, R, pages, _longest(rows, pages, longest), n, k, ctypes.byref(workers), ctypes.byref(nsplit))
+    return (workers.value, parts, nsplit.value) if parts else None
 
 
 class Splits:
@@ -311,3 +323,22 @@ def attn_decode_beside(q, cache, table, klen, g, scale, plan, act, wt, x, k0, k1
     hip.check(L.tfl_attn_decode_beside(_p(q), _p(cache), cache.shape[0] // PAGE, _p(table), table.stride(0), _p(klen), _p(out), _p(ws), ws.numel(), rows, g.H,
                                        float(scale), nsplit, workers, each, ctypes.byref(product), _stream()), "tfl_attn_decode_beside")
     return Splits(ws, nsplit, (rows, g.H, g.C), q.dtype) if later else out
+
+
+def attn_decode_beside_parts(q, cache, table, klen, g, scale, plan, act, wt, k0, k1):
+    """attn_decode_beside of 17 to 32 rows with the product cut over k too: (attention, the parts' sums fp32 [parts][rows][n]) for add_linear.  plan: parts_plan."""
+    _need(q, cache, table, klen)
+    _i32(table, klen)
+    rows, (workers, parts, nsplit) = q.shape[0], plan
+    sums = torch.empty(parts, rows, wt.n, dtype=torch.float32, device=q.device)
+    product = part_of(act, wt, sums[0], k0, k1)
+    product.n_real = wt.n
+    assert q.dtype == cache.dtype == torch.bfloat16 and product.rows == rows and q.is_contiguous() and q.shape[1:] == (g.H, 576) and (g.C, g.R) == (512, 64)
+    assert cache.is_contiguous() and cache.shape[1] == 576 and cache.shape[0] % PAGE == 0
+    assert table.shape[0] == rows and table.stride(1) == 1 and klen.numel() == rows
+    L = hip.latent_lib()
+    ws = torch.empty(L.tfl_attn_decode_ws_floats(rows, g.H, g.C, nsplit), dtype=torch.float32, device=q.device)
+    out = torch.empty(rows, g.H, g.C, dtype=q.dtype, device=q.device)
+    hip.check(L.tfl_attn_decode_beside_parts(_p(q), _p(cache), cache.shape[0] // PAGE, _p(table), table.stride(0), _p(klen), _p(out), _p(ws), ws.numel(), rows, g.H,
+                                             float(scale), nsplit, workers, parts, ctypes.byref(product), _stream()), "tfl_attn_decode_beside_parts")
+    return out, sums
