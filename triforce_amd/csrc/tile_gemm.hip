@@ -361,7 +361,12 @@ static int share_gemm(const TflGemm& a, hipStream_t st) {
 template <typename T, int EPI, int P, int WAVES, int U, bool AHEAD>
 static int launch_form(const TflGemm& a, hipStream_t st) {
     const int panels = (a.n >> 4) * a.groups;
-    const int mt = a.rows <= 16 ? 1 : 2, rb = (a.rows + 16 * mt - 1) / (16 * mt);
+    // Two row blocks of 16 share a workgroup's weights, and take its CU's time for twice the rows of x.  Where a few panels leave CUs idle they go to workgroups of
+    // their own, up to 64 rows.  us at 17 / 32 / 64 rows, together -> apart: TOKEN of 256 x 4 096 5.6 / 5.7 / 6.6 -> 4.6 / 4.6 / 5.3, of 1 024 x 4 096 7.3 / 7.9 / 7.7 -> 6.3 / 6.6 / 6.6,
+    // of 256 x 8 192 8.3 / 9.8 / 12.1 -> 6.5 / 7.5 / 8.9; GATED of 256 panels, eight steps of six layer runs, 32 rows 6 519 -> 6 508.  QUERY of 384 panels is slower
+    // for it (6 519 -> 6 578), LATENT of 1 024 too (6 571).
+    const bool apart = a.rows <= 64 && ((EPI == TFL_EPI_TOKEN && panels <= 64) || (EPI == TFL_EPI_GATED && panels <= 256));
+    const int mt = a.rows <= 16 || apart ? 1 : 2, rb = (a.rows + 16 * mt - 1) / (16 * mt);
     const int extra = EPI == TFL_EPI_QUERY && a.kv_raw ? (a.rows + rb - 1) / rb : 0;
     const dim3 grid((panels + P - 1) / P + extra, rb), block(64 * WAVES);
     if (mt == 1) hipLaunchKernelGGL((latent_gemm_kernel<T, EPI, P, 1, WAVES, U, AHEAD>), grid, block, 0, st, a);
