@@ -29,6 +29,9 @@ int tfh_abi_version(void);
 int tfh_connect(const void* embed, const int64_t* ids, int vocab, const float* embed_w, const void* y, int y_f32, int64_t ld_y,
                 const float* out, const float* mix, const float* in, const float* norm_w, float* x, int streams, int keep, void* h,
                 int64_t ld_h, int64_t h_oct, int rows, int width, int width_real, float eps, int dtype, void* stream);
+/* The first of a decode step (embed given, y not, x kept), with tfl_decode_prep of its rows in the same launch. */
+int tfh_connect_first(const void* embed, const int64_t* ids, int vocab, const float* embed_w, const float* in, const float* norm_w, float* x, int streams, void* h,
+                      int64_t ld_h, int64_t h_oct, int rows, int width, int width_real, float eps, const TflDecodePrep* prep, int dtype, void* stream);
 
 /* tfh_connect of rows whose next reader is a wide product, in that product's launch (bfloat16, one row of up to 4 streams of up to 4 096): every
  * workgroup makes the normed row for itself, beside the beginning of its weights.  x_out (NULL: the streams are not kept) is another block than x;

@@ -26,6 +26,9 @@ int tfl_abi_version(void);
 int tfl_finish(const void* embed, const int64_t* ids, int vocab, const void* y, int y_f32, int64_t ld_y, const float* y_w,
                const float* step, const float* norm_w, float* x, void* h, int64_t ld_h, int64_t h_oct, int rows, int width,
                int width_real, float eps, int dtype, void* stream);
+/* The first of a decode step (embed given, y not), with tfl_decode_prep of its rows in the same launch. */
+int tfl_finish_first(const void* embed, const int64_t* ids, int vocab, const float* step, const float* norm_w, float* x, void* h, int64_t ld_h, int64_t h_oct,
+                     int rows, int width, int width_real, float eps, const TflDecodePrep* prep, int dtype, void* stream);
 
 /* tfl_finish of rows whose next reader is a wide product, in that product's launch (bfloat16, up to 2 rows of up to 4 096): every workgroup makes the normed
  * rows for itself, beside the beginning of its weights.  x_out = x + y / rms(y) * y_w [+ step] is another block than x; product->x is not read.

@@ -83,6 +83,12 @@ int tfl_gemm_carry(const TflGemm* a, const TflGemm* carried, void* stream);
  * their table) stay idle: pos 0, slot -1, klen 0. */
 int tfl_decode_prep(int32_t* len, const int32_t* table, int table_ld, int table_cols, int32_t* pos, int32_t* slot, int32_t* klen,
                     int rows, void* stream);
+typedef struct TflDecodePrep {      /* the same as part of a step's first launch (tfl_finish_first, tfh_connect_first) */
+    int32_t* len;
+    const int32_t* table;
+    int32_t *pos, *slot, *klen;
+    int32_t table_ld, table_cols, rows;
+} TflDecodePrep;
 
 /* float32 products of many rows on the bfloat16 matrix cores (csrc/split_gemm.hip): out[m*ld_out + n] = sum over k of x[m*ld_x + k] * w[n*k_total + k].
  * n % 16 == 0, k % 32 == 0, 16-byte aligned pointers and rows; k is cut into `splits` parts (0: the library's choice).

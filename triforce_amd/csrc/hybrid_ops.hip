@@ -6,14 +6,21 @@ extern "C" int tfh_abi_version(void) { return 1; }
 
 // ------------------------------------------------------------------------------------------------------------ streams
 // One workgroup per row.  S streams at most (streams is the real number); the sublayer input u stays in LDS between its two uses.
-template <typename T, typename Y, int S, int NW>
+// PREP: a step's first launch, with decode_prep_row() of all rows as one more workgroup.
+template <typename T, typename Y, int S, int NW, bool PREP = false>
 __global__ __launch_bounds__(64 * NW) void connect_kernel(const T* __restrict__ embed, const int64_t* __restrict__ ids, int vocab,
                                                           const float* __restrict__ embed_w, const Y* __restrict__ y, int64_t ld_y,
                                                           const float* __restrict__ out, const float* __restrict__ mix,
                                                           const float* __restrict__ in, const float* __restrict__ norm_w,
                                                           float* __restrict__ x, int streams, int keep, T* __restrict__ h, int64_t ld_h,
-                                                          int64_t h_oct, int width, int width_real, float eps) {
+                                                          int64_t h_oct, int width, int width_real, float eps, const TflDecodePrep prep) {
     constexpr int NT = 64 * NW;
+    if constexpr (PREP) {
+        if ((int)blockIdx.x == prep.rows) {
+            for (int m = threadIdx.x; m < prep.rows; m += NT) decode_prep_row(prep, m);
+            return;
+        }
+    }
     extern __shared__ __align__(16) float us[];              // [width]
     __shared__ float red[NW];
     __shared__ float cf[S * S + 2 * S];                      // mix | out | in
@@ -121,26 +128,26 @@ __global__ __launch_bounds__(64 * NW) void connect_kernel(const T* __restrict__ 
     }
 }
 
-template <typename T, typename Y, int S, int NW>
+template <typename T, typename Y, int S, int NW, bool PREP>
 static int launch_connect(const void* embed, const int64_t* ids, int vocab, const float* embed_w, const void* y, int64_t ld_y, const float* out,
                           const float* mix, const float* in, const float* norm_w, float* x, int streams, int keep, void* h, int64_t ld_h,
-                          int64_t h_oct, int rows, int width, int width_real, float eps, hipStream_t st) {
-    auto k = connect_kernel<T, Y, S, NW>;
+                          int64_t h_oct, int rows, int width, int width_real, float eps, const TflDecodePrep& prep, hipStream_t st) {
+    auto k = connect_kernel<T, Y, S, NW, PREP>;
     static bool attr = false;
     if (!attr) {
         const hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 144 * 1024);
         if (e != hipSuccess) return (int)e;
         attr = true;
     }
-    hipLaunchKernelGGL(k, dim3(rows), dim3(64 * NW), sizeof(float) * width, st, (const T*)embed, ids, vocab, embed_w, (const Y*)y, ld_y, out, mix,
-                       in, norm_w, x, streams, keep, (T*)h, ld_h, h_oct, width, width_real, eps);
+    hipLaunchKernelGGL(k, dim3(rows + PREP), dim3(64 * NW), sizeof(float) * width, st, (const T*)embed, ids, vocab, embed_w, (const Y*)y, ld_y, out, mix,
+                       in, norm_w, x, streams, keep, (T*)h, ld_h, h_oct, width, width_real, eps, prep);
     TFL_LAUNCH_CHECK();
     return TF_OK;
 }
 
-extern "C" int tfh_connect(const void* embed, const int64_t* ids, int vocab, const float* embed_w, const void* y, int y_f32, int64_t ld_y,
+static int connect(const void* embed, const int64_t* ids, int vocab, const float* embed_w, const void* y, int y_f32, int64_t ld_y,
                            const float* out, const float* mix, const float* in, const float* norm_w, float* x, int streams, int keep,
-                           void* h, int64_t ld_h, int64_t h_oct, int rows, int width, int width_real, float eps, int dtype, void* stream) {
+                           void* h, int64_t ld_h, int64_t h_oct, int rows, int width, int width_real, float eps, const TflDecodePrep* prep, int dtype, void* stream) {
     if (!x || !h || !norm_w || !in || rows < 1 || width < 8 || (width & 7) || ld_h < 8 || (ld_h & 7) || h_oct < 8 || (h_oct & 7)
         || width_real < 1 || width_real > width || streams < 1) return TF_EINVAL;
     if (embed && (!ids || !embed_w || vocab < 1 || y)) return TF_EINVAL;
@@ -148,17 +155,34 @@ extern "C" int tfh_connect(const void* embed, const int64_t* ids, int vocab, con
     if ((dtype != 0 && dtype != 1) || (dtype == 1 && y && !y_f32)) return TF_EINVAL;
     if (streams > 16 || width > 32768) return TF_ERANGE;
     hipStream_t st = (hipStream_t)stream;
-#define GO(T, Y, S, NW) \
-    return launch_connect<T, Y, S, NW>(embed, ids, vocab, embed_w, y, ld_y, out, mix, in, norm_w, x, streams, keep, h, ld_h, h_oct, rows, \
-                                       width, width_real, eps, st)
-#define GO_S(T, Y, NW) do { if (streams <= 2) GO(T, Y, 2, NW); if (streams <= 4) GO(T, Y, 4, NW); if (streams <= 8) GO(T, Y, 8, NW); GO(T, Y, 16, NW); } while (0)
-#define GO_W(T, Y) do { if (rows <= 256 && width >= 2048) GO_S(T, Y, 16); GO_S(T, Y, 4); } while (0)
-    if (dtype == 1) GO_W(float, float);
-    if (y_f32) GO_W(bf16, float);
-    GO_W(bf16, bf16);
+    const TflDecodePrep d = prep ? *prep : TflDecodePrep{};
+#define GO(T, Y, S, NW, PREP) \
+    return launch_connect<T, Y, S, NW, PREP>(embed, ids, vocab, embed_w, y, ld_y, out, mix, in, norm_w, x, streams, keep, h, ld_h, h_oct, rows, \
+                                       width, width_real, eps, d, st)
+#define GO_S(T, Y, NW, PREP) do { if (streams <= 2) GO(T, Y, 2, NW, PREP); if (streams <= 4) GO(T, Y, 4, NW, PREP); if (streams <= 8) GO(T, Y, 8, NW, PREP); GO(T, Y, 16, NW, PREP); } while (0)
+#define GO_W(T, Y, PREP) do { if (rows <= 256 && width >= 2048) GO_S(T, Y, 16, PREP); GO_S(T, Y, 4, PREP); } while (0)
+    if (prep) {
+        if (dtype == 1) GO_W(float, float, true);
+        GO_W(bf16, bf16, true);
+    }
+    if (dtype == 1) GO_W(float, float, false);
+    if (y_f32) GO_W(bf16, float, false);
+    GO_W(bf16, bf16, false);
 #undef GO_W
 #undef GO_S
 #undef GO
+}
+
+extern "C" int tfh_connect(const void* embed, const int64_t* ids, int vocab, const float* embed_w, const void* y, int y_f32, int64_t ld_y,
+                           const float* out, const float* mix, const float* in, const float* norm_w, float* x, int streams, int keep,
+                           void* h, int64_t ld_h, int64_t h_oct, int rows, int width, int width_real, float eps, int dtype, void* stream) {
+    return connect(embed, ids, vocab, embed_w, y, y_f32, ld_y, out, mix, in, norm_w, x, streams, keep, h, ld_h, h_oct, rows, width, width_real, eps, nullptr, dtype, stream);
+}
+
+extern "C" int tfh_connect_first(const void* embed, const int64_t* ids, int vocab, const float* embed_w, const float* in, const float* norm_w, float* x, int streams,
+                                 void* h, int64_t ld_h, int64_t h_oct, int rows, int width, int width_real, float eps, const TflDecodePrep* prep, int dtype, void* stream) {
+    if (!embed || !decode_prep_ok(prep, rows)) return TF_EINVAL;
+    return connect(embed, ids, vocab, embed_w, nullptr, 0, 0, nullptr, nullptr, in, norm_w, x, streams, 1, h, ld_h, h_oct, rows, width, width_real, eps, prep, dtype, stream);
 }
 
 // ------------------------------------------------------------------------------------------------------------ q | k | v

@@ -4,12 +4,19 @@
 
 extern "C" int tfl_abi_version(void) { return 1; }
 
-template <typename T, typename Y>
+// PREP: a step's first launch, with decode_prep_row() of all rows as one more workgroup (a launch of its own is 4.3 us of a step of one row of 516).
+template <typename T, typename Y, bool PREP = false>
 __global__ __launch_bounds__(256) void finish_kernel(const T* __restrict__ embed, const int64_t* __restrict__ ids, int vocab,
                                                      const Y* __restrict__ y, int64_t ld_y, const float* __restrict__ y_w,
                                                      const float* __restrict__ step, const float* __restrict__ norm_w,
                                                      float* __restrict__ x, T* __restrict__ h, int64_t ld_h, int64_t h_oct,
-                                                     int width, int width_real, float eps) {
+                                                     int width, int width_real, float eps, const TflDecodePrep prep) {
+    if constexpr (PREP) {
+        if ((int)blockIdx.x == prep.rows) {
+            for (int m = threadIdx.x; m < prep.rows; m += 256) decode_prep_row(prep, m);
+            return;
+        }
+    }
     __shared__ float red[4];
     const int row = blockIdx.x, nq = width >> 2;             // elements in groups of 4
     float* xr = x + (int64_t)row * width;
@@ -63,12 +70,18 @@ __global__ __launch_bounds__(256) void finish_kernel(const T* __restrict__ embed
 // 3.9 us, 32 rows 5.4 -> 4.1, 4 000 rows 40.6 -> 33.4 (5.9 TB/s).  Narrow rows take no more waves than they have quads (4 000 rows of 192 with four
 // times four 8.6 us, with one wave 4.3, in the form above 6.7); 4 000 rows of 1 025 to 2 048, which leave half the four quads empty, are
 // faster above (2 048 16.5 us and 18.6).
-template <typename T, typename Y, int NW, int HOLD>
+template <typename T, typename Y, int NW, int HOLD, bool PREP = false>
 __global__ __launch_bounds__(64 * NW) void finish_row_kernel(const T* __restrict__ embed, const int64_t* __restrict__ ids, int vocab,
                                                              const Y* __restrict__ y, int64_t ld_y, const float* __restrict__ y_w,
                                                              const float* __restrict__ step, const float* __restrict__ norm_w,
                                                              float* __restrict__ x, T* __restrict__ h, int64_t ld_h, int64_t h_oct,
-                                                             int width, int width_real, float eps) {
+                                                             int width, int width_real, float eps, const TflDecodePrep prep) {
+    if constexpr (PREP) {
+        if ((int)blockIdx.x == prep.rows) {
+            for (int m = threadIdx.x; m < prep.rows; m += 64 * NW) decode_prep_row(prep, m);
+            return;
+        }
+    }
     __shared__ float red[NW];
     const int row = blockIdx.x, nq = width >> 2;
     float* xr = x + (int64_t)row * width;
@@ -135,29 +148,43 @@ __global__ __launch_bounds__(64 * NW) void finish_row_kernel(const T* __restrict
     }
 }
 
-extern "C" int tfl_finish(const void* embed, const int64_t* ids, int vocab, const void* y, int y_f32, int64_t ld_y,
+static int finish(const void* embed, const int64_t* ids, int vocab, const void* y, int y_f32, int64_t ld_y,
                           const float* y_w, const float* step, const float* norm_w, float* x, void* h, int64_t ld_h, int64_t h_oct,
-                          int rows, int width, int width_real, float eps, int dtype, void* stream) {
+                          int rows, int width, int width_real, float eps, const TflDecodePrep* prep, int dtype, void* stream) {
     if (!x || !h || !norm_w || rows < 1 || width < 8 || (width & 7) || ld_h < 8 || (ld_h & 7) || h_oct < 8 || (h_oct & 7) || width_real < 1 || width_real > width) return TF_EINVAL;
     if (embed && (!ids || vocab < 1)) return TF_EINVAL;
     if (y && (!y_w || ld_y < width || (ld_y & 3))) return TF_EINVAL;
     hipStream_t st = (hipStream_t)stream;
-#define ARGS(T, Y) 0, st, (const T*)embed, ids, vocab, (const Y*)y, ld_y, y_w, step, norm_w, x, (T*)h, ld_h, h_oct, width, width_real, eps
-#define GO(T, Y)                                                                                                                              \
+    const TflDecodePrep d = prep ? *prep : TflDecodePrep{};
+#define ARGS(T, Y) 0, st, (const T*)embed, ids, vocab, (const Y*)y, ld_y, y_w, step, norm_w, x, (T*)h, ld_h, h_oct, width, width_real, eps, d
+#define GO(T, Y, PREP)                                                                                                                              \
     do {                                                                                                                                      \
-        if (width > 4096 || (width > 1024 && width <= 2048 && rows > 1024)) hipLaunchKernelGGL((finish_kernel<T, Y>), dim3(rows), dim3(256), ARGS(T, Y)); \
-        else if (width <= 256) hipLaunchKernelGGL((finish_row_kernel<T, Y, 1, 1>), dim3(rows), dim3(64), ARGS(T, Y));                          \
-        else if (width <= 1024) hipLaunchKernelGGL((finish_row_kernel<T, Y, 4, 1>), dim3(rows), dim3(256), ARGS(T, Y));                        \
-        else if (rows <= 256) hipLaunchKernelGGL((finish_row_kernel<T, Y, 16, 1>), dim3(rows), dim3(1024), ARGS(T, Y));  /* a row per CU */    \
-        else hipLaunchKernelGGL((finish_row_kernel<T, Y, 4, 4>), dim3(rows), dim3(256), ARGS(T, Y));                                          \
+        if (width > 4096 || (width > 1024 && width <= 2048 && rows > 1024)) hipLaunchKernelGGL((finish_kernel<T, Y, PREP>), dim3(rows + PREP), dim3(256), ARGS(T, Y)); \
+        else if (width <= 256) hipLaunchKernelGGL((finish_row_kernel<T, Y, 1, 1, PREP>), dim3(rows + PREP), dim3(64), ARGS(T, Y));                          \
+        else if (width <= 1024) hipLaunchKernelGGL((finish_row_kernel<T, Y, 4, 1, PREP>), dim3(rows + PREP), dim3(256), ARGS(T, Y));                        \
+        else if (rows <= 256) hipLaunchKernelGGL((finish_row_kernel<T, Y, 16, 1, PREP>), dim3(rows + PREP), dim3(1024), ARGS(T, Y));  /* a row per CU */    \
+        else hipLaunchKernelGGL((finish_row_kernel<T, Y, 4, 4, PREP>), dim3(rows + PREP), dim3(256), ARGS(T, Y));                                          \
     } while (0)
-    if (dtype == 0) { if (y_f32) GO(bf16, float); else GO(bf16, bf16); }
-    else if (dtype == 1) GO(float, float);
+    if (prep) { if (dtype == 0) GO(bf16, bf16, true); else if (dtype == 1) GO(float, float, true); else return TF_EINVAL; }
+    else if (dtype == 0) { if (y_f32) GO(bf16, float, false); else GO(bf16, bf16, false); }
+    else if (dtype == 1) GO(float, float, false);
     else return TF_EINVAL;
 #undef GO
 #undef ARGS
     TFL_LAUNCH_CHECK();
     return TF_OK;
+}
+
+extern "C" int tfl_finish(const void* embed, const int64_t* ids, int vocab, const void* y, int y_f32, int64_t ld_y,
+                          const float* y_w, const float* step, const float* norm_w, float* x, void* h, int64_t ld_h, int64_t h_oct,
+                          int rows, int width, int width_real, float eps, int dtype, void* stream) {
+    return finish(embed, ids, vocab, y, y_f32, ld_y, y_w, step, norm_w, x, h, ld_h, h_oct, rows, width, width_real, eps, nullptr, dtype, stream);
+}
+
+extern "C" int tfl_finish_first(const void* embed, const int64_t* ids, int vocab, const float* step, const float* norm_w, float* x, void* h, int64_t ld_h, int64_t h_oct,
+                                int rows, int width, int width_real, float eps, const TflDecodePrep* prep, int dtype, void* stream) {
+    if (!embed || !decode_prep_ok(prep, rows)) return TF_EINVAL;
+    return finish(embed, ids, vocab, nullptr, 0, 0, nullptr, step, norm_w, x, h, ld_h, h_oct, rows, width, width_real, eps, prep, dtype, stream);
 }
 
 template <typename T>

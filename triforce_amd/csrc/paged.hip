@@ -6,13 +6,7 @@ extern "C" int tfl_tile_abi_version(void) { return 2; }
 __global__ void decode_prep_kernel(int32_t* __restrict__ len, const int32_t* __restrict__ table, int table_ld, int table_cols,
                                    int32_t* __restrict__ pos, int32_t* __restrict__ slot, int32_t* __restrict__ klen, int rows) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= rows) return;
-    const int l = len[m];
-    const bool live = l >= 0 && l / TFL_PAGE < table_cols;
-    pos[m] = live ? l : 0;
-    slot[m] = live ? table[(int64_t)m * table_ld + l / TFL_PAGE] * TFL_PAGE + l % TFL_PAGE : -1;
-    klen[m] = live ? l + 1 : 0;
-    if (live) len[m] = l + 1;
+    if (m < rows) decode_prep_row(TflDecodePrep{len, table, pos, slot, klen, table_ld, table_cols, rows}, m);
 }
 
 extern "C" int tfl_decode_prep(int32_t* len, const int32_t* table, int table_ld, int table_cols, int32_t* pos, int32_t* slot,

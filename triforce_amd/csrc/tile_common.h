@@ -138,6 +138,19 @@ __device__ __forceinline__ void cache_row(Src src, int C, int c_real, int R, con
     }
 }
 
+// Where row m of a decode step stands: its position, cache row and visible keys, and its length one further.
+__device__ __forceinline__ void decode_prep_row(const TflDecodePrep& d, int m) {
+    const int l = d.len[m];
+    const bool live = l >= 0 && l / TFL_PAGE < d.table_cols;
+    d.pos[m] = live ? l : 0;
+    d.slot[m] = live ? d.table[(int64_t)m * d.table_ld + l / TFL_PAGE] * TFL_PAGE + l % TFL_PAGE : -1;
+    d.klen[m] = live ? l + 1 : 0;
+    if (live) d.len[m] = l + 1;
+}
+static inline bool decode_prep_ok(const TflDecodePrep* d, int rows) {
+    return d && d->len && d->table && d->pos && d->slot && d->klen && d->rows == rows && d->table_cols >= 1 && d->table_ld >= d->table_cols;
+}
+
 #define TFL_LAUNCH_CHECK()                      \
     do {                                        \
         hipError_t e__ = hipGetLastError();     \

@@ -154,6 +154,11 @@ TFL_MAX_ENTRIES = 64
 TFL_EPI = {n: i for i, n in enumerate(("f32", "in", "query", "latent", "gated", "residual", "token", "glu"))}
 
 
+class TflDecodePrep(_c.Structure):
+    """include/triforce_tile.h: TflDecodePrep."""
+    _fields_ = [(n, _vp) for n in ("len", "table", "pos", "slot", "klen")] + [(n, _i32) for n in ("table_ld", "table_cols", "rows")]
+
+
 class TflGemm(_c.Structure):
     """include/triforce_tile.h: TflGemm."""
     _fields_ = ([(n, _vp) for n in ("wp", "x", "norm_w", "ss_in", "out_t", "out_t2", "out_f", "ss_out", "gate", "tok_table", "ids",
@@ -204,6 +209,7 @@ LATENT_SIGNATURES = {
     "tfl_attn_beside_plan": (_i32, [_i32, _i32, _i32, _i32, _i64, _i32, _i32] + 3 * [_c.POINTER(_c.c_int32)]),
     "tfl_attn_beside_plan_of": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i32, _i32] + 3 * [_c.POINTER(_c.c_int32)]),
     "tfl_attn_decode_beside_parts": (_i32, [_vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _f32, _i32, _i32, _i32, _c.POINTER(TflGemm), _vp]),
+    "tfl_finish_first": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _f32, _c.POINTER(TflDecodePrep), _i32, _vp]),
     "tfl_beside_parts": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i32, _i32, _c.POINTER(_c.c_int32), _c.POINTER(_c.c_int32)]),
     "tfl_latent_carry": (_i32, [_i32, _i32, _i32, _i32, _i64, _i64, _i32, _i32]),
     "tfl_latent_value": (_i32, [_vp, _i64, _i32, _c.POINTER(TflGemm), _vp]),
@@ -247,6 +253,7 @@ class TfhConnect(_c.Structure):
 
 HYBRID_SIGNATURES = {
     "tfh_connect_gemm_takes": (_i32, [_i32] * 6),
+    "tfh_connect_first": (_i32, [_vp, _vp, _i32, _vp, _vp, _vp, _vp, _i32, _vp, _i64, _i64, _i32, _i32, _i32, _f32, _c.POINTER(TflDecodePrep), _i32, _vp]),
     "tfh_streams_gemm_takes": (_i32, [_i32] * 4),
     "tfh_streams_gemm": (_i32, [_c.POINTER(TfhConnect), _c.POINTER(TflGemm), _vp]),
     "tfh_scaled_gemm_takes": (_i32, [_i32] * 3),

@@ -570,7 +570,8 @@ class PagedBatch:
     """What one forward over several sequences needs besides the token ids; device tensors unless said otherwise.
 
     decode (one token per sequence): pos / slot / klen / seat int32 [B], table int32 [B, columns], max_len (host int: what the cache holds),
-      pages, longest (host ints: what these sequences hold of it in all, and one of them at most; None where that is not known).
+      pages, longest (host ints: what these sequences hold of it in all, and one of them at most; None where that is not known),
+      prep (the arguments of ops_tile.decode_prep where the forward's first launch is to do that; None where it has been done).
     prefill: pos / slot int32 [tokens]; max_new (host int); seq int32 [sequences, 4], its columns depend on the cache:
       LatentCache: first new token, new tokens, first key, keys; key_rows int32 [keys] = cache rows of every visible key, or None
         when no sequence has a past.
@@ -579,12 +580,12 @@ class PagedBatch:
     want: rows whose logits are asked for (int64), None = all."""
 
     def __init__(self, decode, pos, slot, want=None, table=None, klen=None, seat=None, max_len=0, seq=None, max_new=0, key_rows=None,
-                 seg=None, span=None, max_segs=0, pages=None, longest=None):
+                 seg=None, span=None, max_segs=0, pages=None, longest=None, prep=None):
         self.decode, self.pos, self.slot, self.want = decode, pos, slot, want
         self.table, self.klen, self.seat, self.max_len = table, klen, seat, max_len
         self.seq, self.max_new, self.key_rows = seq, max_new, key_rows
         self.seg, self.span, self.max_segs = seg, span, max_segs
-        self.pages, self.longest = pages, longest
+        self.pages, self.longest, self.prep = pages, longest, prep
 
 
 class PagedCache(Cache):

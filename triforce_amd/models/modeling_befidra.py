@@ -16,6 +16,7 @@ from .rotary import RotaryTable
 
 class BefidraForCausalLM:
     supports_speculation = False                   # no retrieval cache over latents: the engines serve it autoregressively
+    prepares_steps = True                          # a decode step's first launch takes PagedBatch.prep
 
     def __init__(self, config: BefidraConfig, device="cuda:0", dtype=torch.bfloat16):
         if dtype not in (torch.bfloat16, torch.float32):
@@ -104,7 +105,7 @@ class BefidraForCausalLM:
                 x = h.out
             else:
                 h = ol.finish(x, L.norm1, eps, width, self.dtype, embed=W.embed if r == 0 else None, ids=ids if r == 0 else None,
-                              y=y, y_w=y_w, step=W.step[t] if first else None, octets=batch.decode)
+                              y=y, y_w=y_w, step=W.step[t] if first else None, octets=batch.decode, prep=batch.prep if r == 0 else None)
             if W.capture is not None and r > 0:
                 W.capture.append((x - W.step[t] if first else x.clone())[:, :width])
             layer = L.decode if batch.decode else L.prefill

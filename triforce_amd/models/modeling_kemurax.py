@@ -17,6 +17,7 @@ from .rotary import RotaryTable
 
 class KemuraxForCausalLM:
     supports_speculation = False                   # a recurrent state cannot be rolled back to an accepted prefix: served autoregressively
+    prepares_steps = True                          # a decode step's first launch takes PagedBatch.prep
 
     def __init__(self, config: KemuraxConfig, device="cuda:0", dtype=torch.bfloat16):
         if dtype not in (torch.bfloat16, torch.float32):
@@ -106,7 +107,7 @@ class KemuraxForCausalLM:
             if batch.decode and hc is not None and W.capture is None and oh.Connect.takes(x, wt, epi):
                 h = oh.Connect(x, connection.u_in, norm, eps, width, y, hc.out, hc.mix)
                 return h, h.out
-            before = first if hc is None else dict(y=y, out=hc.out, mix=hc.mix)
+            before = dict(first, prep=batch.prep) if hc is None else dict(y=y, out=hc.out, mix=hc.mix)
             return oh.connect(x, connection.u_in, norm, eps, width, self.dtype, octets=batch.decode, **before), x
         fused = batch.decode and W.capture is None and batch.want is None
 

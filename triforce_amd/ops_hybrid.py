@@ -10,7 +10,7 @@ import ctypes
 import torch
 
 from . import hip
-from .ops_tile import (_CODE, PAGE, TileWeight, _f32, _i32, _lay, _need, _p, _stream, decode_prep, empty_act, gelu_glu_linear,  # noqa: F401
+from .ops_tile import (_CODE, PAGE, TileWeight, _f32, _i32, _lay, _need, _p, _stream, decode_prep, decode_prep_of, empty_act, gelu_glu_linear,  # noqa: F401
                        grow, interleave_glu, linear_f32, pad32)
 
 CHUNK = 64                     # tokens a recurrence takes at a time in prefill (TFH_CHUNK)
@@ -20,9 +20,11 @@ def _lib():
     return hip.hybrid_lib()
 
 
-def connect(x, u_in, norm_w, eps, width, dtype, embed=None, ids=None, embed_w=None, y=None, out=None, mix=None, keep=True, octets=False):
+def connect(x, u_in, norm_w, eps, width, dtype, embed=None, ids=None, embed_w=None, y=None, out=None, mix=None, keep=True, octets=False,
+            prep=None):
     """Residual streams between two sublayers; see tfh_connect.  x fp32 [rows, streams, padded width] is updated in place (unless
-    not ``keep``); returns the sublayer's normed input in ``dtype``, row-major or (``octets``) octet-major."""
+    not ``keep``); returns the sublayer's normed input in ``dtype``, row-major or (``octets``) octet-major.  ``prep``: decode_prep() of these tensors in the same
+    launch (embed, kept)."""
     _need(x, u_in, norm_w, embed, ids, embed_w, y, out, mix)
     _f32(x, u_in, norm_w, embed_w, out, mix)
     rows, streams, wp = x.shape
@@ -33,6 +35,12 @@ def connect(x, u_in, norm_w, eps, width, dtype, embed=None, ids=None, embed_w=No
                          and mix.shape == (streams, streams) and mix.is_contiguous())
     h = empty_act(rows, wp, dtype, x.device) if octets else torch.empty(rows, wp, dtype=dtype, device=x.device)
     _, _, ld, octet = _lay(h)
+    if prep is not None:
+        assert embed is not None and y is None and keep
+        d = decode_prep_of(*prep)
+        hip.check(_lib().tfh_connect_first(_p(embed), _p(ids), embed.shape[0], _p(embed_w), _p(u_in), _p(norm_w), _p(x), streams, _p(h), ld, octet, rows, wp, width,
+                                           float(eps), ctypes.byref(d), _CODE[dtype], _stream()), "tfh_connect_first")
+        return h
     hip.check(_lib().tfh_connect(_p(embed), _p(ids), 0 if embed is None else embed.shape[0], _p(embed_w), _p(y),
                                  int(y is not None and y.dtype == torch.float32), 0 if y is None else y.stride(0), _p(out), _p(mix), _p(u_in),
                                  _p(norm_w), _p(x), streams, int(keep), _p(h), ld, octet, rows, wp, width, float(eps), _CODE[dtype], _stream()),

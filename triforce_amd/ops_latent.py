@@ -10,7 +10,7 @@ import functools
 import torch
 
 from . import hip
-from .ops_tile import (_CODE, PAGE, TileWeight, _f32, _gemm, _i32, _lay, _need, _p, _stream, _tail, act_rows, decode_prep, empty_act, linear_rows,  # noqa: F401
+from .ops_tile import (_CODE, PAGE, TileWeight, _f32, _gemm, _i32, _lay, _need, _p, _stream, _tail, act_rows, decode_prep, decode_prep_of, empty_act, linear_rows,  # noqa: F401
                        linear_f32, pack_tiles, pad32, part_of)
 
 class Finish:
@@ -165,9 +165,9 @@ def token_side(x, gate, proj, table, ids, n_real, width):
     return out
 
 
-def finish(x, norm_w, eps, width, dtype, embed=None, ids=None, y=None, y_w=None, step=None, octets=False):
+def finish(x, norm_w, eps, width, dtype, embed=None, ids=None, y=None, y_w=None, step=None, octets=False, prep=None):
     """Residual bookkeeping between two layers and the next norm; see tfl_finish.  x fp32 [rows, padded width] is updated in
-    place; returns h in ``dtype``, row-major or (``octets``) octet-major."""
+    place; returns h in ``dtype``, row-major or (``octets``) octet-major.  ``prep``: decode_prep() of these tensors in the same launch (embed, no y)."""
     _need(x, norm_w, embed, ids, y, y_w, step)
     _f32(x, norm_w, y_w, step)
     rows, wp = x.shape
@@ -177,6 +177,12 @@ def finish(x, norm_w, eps, width, dtype, embed=None, ids=None, y=None, y_w=None,
     assert y is None or (y.shape == (rows, wp) and y_w.numel() == wp and y.dtype in (dtype, torch.float32) and y.stride(1) == 1)
     h = empty_act(rows, wp, dtype, x.device) if octets else torch.empty(rows, wp, dtype=dtype, device=x.device)
     _, _, ld, octet = _lay(h)
+    if prep is not None:
+        assert embed is not None and y is None
+        d = decode_prep_of(*prep)
+        hip.check(hip.latent_lib().tfl_finish_first(_p(embed), _p(ids), embed.shape[0], _p(step), _p(norm_w), _p(x), _p(h), ld, octet, rows, wp, width, float(eps),
+                                                    ctypes.byref(d), _CODE[dtype], _stream()), "tfl_finish_first")
+        return h
     hip.check(hip.latent_lib().tfl_finish(_p(embed), _p(ids), 0 if embed is None else embed.shape[0], _p(y),
                                           int(y is not None and y.dtype == torch.float32), 0 if y is None else y.stride(0), _p(y_w),
                                           _p(step), _p(norm_w), _p(x), _p(h), ld, octet, rows, wp, width, float(eps), _CODE[dtype], _stream()),

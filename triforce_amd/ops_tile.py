@@ -224,6 +224,15 @@ def set_pages(table, entries):
         hip.check(hip.tile_lib().tfl_set_pages(_p(table), table.stride(0), table.shape[0], table.shape[1], flat, len(part), _stream()), "tfl_set_pages")
 
 
+def decode_prep_of(lens, table, pos, slot, klen):
+    """decode_prep() as an argument of a step's first launch (ops_latent.finish, ops_hybrid.connect)."""
+    _need(lens, table, pos, slot, klen)
+    _i32(lens, table, pos, slot, klen)
+    rows = lens.numel()
+    assert table.shape[0] == rows and table.stride(1) == 1 and pos.numel() == rows and slot.numel() == rows and klen.numel() == rows
+    return hip.TflDecodePrep(_p(lens), _p(table), _p(pos), _p(slot), _p(klen), table.stride(0), table.shape[1], rows)
+
+
 def decode_prep(lens, table, pos, slot, klen):
     _need(lens, table, pos, slot, klen)
     _i32(lens, table, pos, slot, klen)

@@ -73,6 +73,7 @@ class _DecodeStep:
     def __init__(self, model, cache, B, use_graph):
         self.model, self.cache, self.buf, self.use_graph = model, cache, _DecodeBuffers(cache, B), use_graph
         self.form = getattr(model, "decode_form", lambda rows, pages, longest: None)                     # (most models have one form)
+        self.prepares = getattr(model, "prepares_steps", False)                                          # (decode_prep in the forward's first launch)
         self.graphs = {}                                        # form -> (graph, logits), in one pool: of these only one runs at a time
 
     def _graph(self, form):
@@ -84,7 +85,11 @@ class _DecodeStep:
 
     def _run(self):
         b = self.buf
-        ops_tile.decode_prep(b.lens, b.table, b.pos, b.slot, b.klen)
+        prep = (b.lens, b.table, b.pos, b.slot, b.klen)
+        if self.prepares:
+            b.batch.prep = prep
+        else:
+            ops_tile.decode_prep(*prep)
         return self.model.forward_batch(b.ids, b.batch, self.cache)
 
     def __call__(self, seqs, ids):
