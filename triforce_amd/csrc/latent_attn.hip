@@ -748,12 +748,17 @@ static BesideTime beside_time(int rows, int H, int64_t pages, int64_t longest, i
     return {a, product, attention, fmax(product, attention) + 0.25 * heads * rows + 0.0068 * heads * (double)(pages < a ? pages : a) - 1.892 * (rows < 5 ? 5 - rows : 0)};
 }
 
+// The two one after the other.
+static double apart_time(int rows, int H, int64_t pages, int64_t longest, int n, int k) {
+    const int ns = tfl_attn_decode_splits(rows, H, 512, 64, (int)(pages < 16 ? 16 : pages) * TFL_PAGE, 0);        // (a cache of what is there, or more)
+    const double mb = 2e-6 * n * k, heads = H / 32.0, x = rows * k / 11008.0;
+    return 3.345 + 0.1237 * mb + 0.1656 * rows + 0.4873 * x + 0.0083 * heads * rows * ns + 0.0026 * pages + 2.245 * (double)((longest + ns - 1) / ns);
+}
+
 static int beside_plan(int rows, int H, int64_t pages, int64_t longest, int n, int k, int* panels_each) {
     const int panels = n >> 4;
     if (rows < 1 || rows > 32 || H <= 16 || H > 32 || pages < 1 || pages > (1 << 20) || longest < 1 || panels < 256 || panels > 512 || k < 2048) return 0;
-    const int ns = tfl_attn_decode_splits(rows, H, 512, 64, (int)(pages < 16 ? 16 : pages) * TFL_PAGE, 0);        // (a cache of what is there, or more)
-    const double mb = 2e-6 * n * k, heads = H / 32.0, x = rows * k / 11008.0;
-    double least = 3.345 + 0.1237 * mb + 0.1656 * rows + 0.4873 * x + 0.0083 * heads * rows * ns + 0.0026 * pages + 2.245 * (double)((longest + ns - 1) / ns);
+    double least = apart_time(rows, H, pages, longest, n, k);
     if (pages < 32 * rows && k <= 12288) least *= 1.0 / 0.9;
     int workers = 0;
     for (int p = 2; p <= 4; ++p) {
@@ -778,35 +783,37 @@ extern "C" int tfl_attn_beside_plan_of(int rows, int H, int C, int R, int64_t pa
     return a;
 }
 
-// Columns of that product's k, from the last on, that the query to latent product in front of the attention carries (latent_carry_kernel in tile_gemm.hip): as
-// long as what is left still outlasts the attention, in steps of 1 024 from 4 096 on (below that a carried panel costs its start more than the
-// other one saves: eight steps of six layer runs, one row of 4 000 keys, 2 048 -36 us, 3 072 +10, 4 096 -65, 5 120 -82, 6 144 -48).  The cost of carrying is
-// fitted to 90 points of 1 to 16 rows, contexts of 300 to 20 000; of 54 others none is slower for the pick.  us of query to latent, attention, value and output
-// product (32 heads, n 4 096, k 11 008), none -> as picked, at 300 / 2 000 / 4 000 keys: 1 row 34.7 -> 33.4, 35.5 -> 34.3, 36.0 -> 35.0; 4 rows 39.6 -> 37.6,
-// 40.9 -> 39.7, 43.1 -> 40.9; 8 rows 42.0 -> 39.3, 45.2 -> 41.6, 45.7 -> 43.4; 16 rows 46.4 -> 42.7, 48.8 -> 45.5, not picked (51.7, carrying 54.5).
+// Columns of that product's k, from the last on, that the query to latent product in front of the attention carries (latent_carry_kernel in tile_gemm.hip): one
+// amount for a product's k, or none.  An amount that followed the context would be a captured step of its own in each of its ranges, 65 to 110 ms of
+// capture while an answer grows (8 rows changed it at 2 048, 3 072 and 4 032 tokens), for up to 1 us a layer run: us of query to latent, attention, value and
+// output product (32 heads, n 4 096, k 11 008), none | 4 096 | 5 120 | 6 144 columns, the longest row of 300, 2 000, 4 000, 9 000, 16 000 keys:
+//    1 row   34.7|33.7|33.4|33.0  35.2|34.4|34.2|34.5  36.1|35.3|35.0|35.4  39.0|38.0|37.8|38.2  41.7|40.3|40.5|40.9, of 20 000 41.7|40.9|41.7|42.6
+//    4 rows  39.5|38.5|38.1|37.6  41.0|39.7|39.2|39.5  43.0|41.3|41.0|41.1  45.4|44.8|45.6|45.0
+//    8 rows  42.1|40.6|39.8|39.2  45.3|42.7|42.0|41.9  45.9|44.1|44.9|45.8
+//   16 rows  46.5|44.0|43.4|42.8  49.0|46.3|45.9|47.1  51.9|55.1|54.6|55.4
+// Carried as long as the fitted times save 0.8 us by it, also where the two without it would go one after the other: 131 of 218 points (1 to 16 rows, 300 to
+// 28 000 keys, 20 to 32 heads, n 4 096 and 6 144), 1.6 us or 3.8 % faster on average, one of them slower (0.12 us).
 // Up to 16 rows: of 32 rows a carried panel reads twice its weights' bytes of x (6 664 us of eight steps -> 6 924).
 extern "C" int tfl_latent_carry(int rows, int H, int C, int R, int64_t pages, int64_t longest, int n, int k) {
-    if (C != 512 || R != 64 || rows < 1 || rows > 16 || longest < 1 || k > (1 << 20)) return 0;
-    int p = 0, q = 0, best = 0;
-    if (beside_plan(rows, H, pages, longest, n, k, &p) == 0) return 0;
-    const double apart = beside_time(rows, H, pages, longest, n, k, p).all;
-    double gain = 0.8;
-    for (int c = 4096; c <= 6144 && k - c >= 2048; c += 1024) {
-        if (beside_plan(rows, H, pages, longest, n, k - c, &q) == 0) break;
-        const BesideTime b = beside_time(rows, H, pages, longest, n, k - c, q);
-        const double saved = apart - b.all - (0.55 + 3.2e-7 * c * n + 0.11 * rows);
-        if (b.product < b.attention + 1.0 - 0.06 * rows) break;
-        if (saved > gain) { gain = saved; best = c; }
-    }
-    return best;
+    const int columns = k >= 5120 + 2048 ? 5120 : 4096;       // (4 096: a carried panel of less costs its start more than the other one saves)
+    if (C != 512 || R != 64 || rows < 1 || rows > 16 || longest < 1 || k > (1 << 20) || k - columns < 2048) return 0;
+    int p = 0, q = 0;
+    if (beside_plan(rows, H, pages, longest, n, k - columns, &q) == 0) return 0;
+    const double without = beside_plan(rows, H, pages, longest, n, k, &p) ? beside_time(rows, H, pages, longest, n, k, p).all : apart_time(rows, H, pages, longest, n, k);
+    const double with = beside_time(rows, H, pages, longest, n, k - columns, q).all + 0.55 + 3.2e-7 * columns * n + 0.11 * rows;
+    return without - with > 0.8 && (p == 0 || p == q) ? columns : 0;
 }
 
-// Ranges of k (3 or 4; 0: none) into which 17 to 32 rows' product is cut where that is faster than beside_plan's division or the two apart.  The times of query to
-// latent, attention, value and output product as fitted to 720 measured ones (17, 20, 24, 28, 32 rows of 300 to 6 000 keys; 17, 20, 24, 32 heads; n 4 096 to 8 192, k 4 096
-// to 14 336): 2.5 % off on average, so 2 % have to be in it.  At those 180 sizes that picks 4.5 % on average, nowhere slower, 0.3 % behind the best.  us, 32 heads,
-// n 4 096, k 11 008, as before -> cut in 3 | in 4, the pick marked: 17 rows of 300 keys 45.5 -> 47.8 | 42.2*, of 4 000 51.5 -> 54.9 | 50.2*; 32 rows of 300 53.0 -> 52.8 |
-// 47.5*, of 2 000 56.9 -> 57.2 | 52.4*, of 3 000 58.8* -> 59.7 | 60.3, of 4 000 65.4 -> 63.0* | 67.2, of 6 000 72.3* -> 75.1 | 83.1.  Up to 16 rows it is never faster (16 rows of 300
-// 43.2 -> 48.6 | 46.3), nor in one or two ranges, which leave the product too few CUs.
+// Ranges of k (4, or 3 where the attention would be left with too few CUs; 0: none) into which 17 to 32 rows' product is cut where that is faster than
+// beside_plan's division or the two apart.  The times of query to latent, attention, value and output product as fitted to 720 measured ones (17, 20, 24, 28, 32 rows
+// of 300 to 6 000 keys; 17, 20, 24, 32 heads; n 4 096 to 8 192, k 4 096 to 14 336): 2.5 % off on average, so 2 % have to be in it.  Every division is a captured step of
+// its own, 65 to 110 ms of capture while an answer grows, so there is the one cut of short contexts and no other between it and whole panels (three
+// ranges besides: 0.3 % on average).  Of 226 other points (17 to 32 rows, 20 to 32 heads, k 8 192 to 14 336) it is 1.85 % faster on average than without, 2 are more than 1 %
+// slower (1.5 %).  us, 32 heads, n 4 096, k 11 008, rows half to all as long as the longest, 2 | 3 whole panels, 3 | 4 ranges, * the pick:
+//   17 rows of   300 49.6|56.6|52.2|46.8*  2 000 51.5|59.6|54.7|49.3*  3 500 53.9|62.7|58.5|53.6*  5 000 56.6*|65.3|60.5|58.4   6 000 61.4*|65.9|61.8|62.9
+//   24 rows of   300 53.3|59.1|53.8|49.7*  2 000 55.1|63.3|56.7|52.5*  3 500 57.5*|67.3|61.7|59.0  5 000 66.1*|67.8|64.3|68.1   6 000 73.0|70.2*|69.0|74.9
+//   32 rows of   300 56.5|64.5|57.2|51.7*  2 000 60.9|69.7|61.7|57.2*  3 000 63.0*|70.7|64.5|64.8  4 000 69.6*|72.6|67.9|71.8   5 000 79.1|74.3*|74.5|81.0
+// Up to 16 rows it is never faster (16 rows of 300 43.2 -> 48.6 in three ranges, 46.3 in four), nor in one or two ranges, which leave the product too few CUs.
 extern "C" int tfl_beside_parts(int rows, int H, int C, int R, int64_t pages, int64_t longest, int n, int k, int32_t* workers, int32_t* nsplit) {
     if (!workers || !nsplit || C != 512 || R != 64 || rows < 17 || rows > 32 || H <= 16 || H > 32 || pages < 1 || pages > (1 << 20) || longest < 1 || n < 4096 || n > 8192 || (n & 15)
         || k < 4096 || k > 14336) return 0;
@@ -815,7 +822,9 @@ extern "C" int tfl_beside_parts(int rows, int H, int C, int R, int64_t pages, in
         const int most = 2 * a / rows < 128 ? 2 * a / rows : 128;
         return fmax((double)pages / a, (double)((longest + most - 1) / most));
     };
-    int p = 0, best = 0;
+    const int eights = (n + 127) / 128;
+    const bool four = 256 - 4 * eights >= 64 && 256 - 4 * eights >= 2 * rows;
+    int p = 0;
     double least;
     if (beside_plan(rows, H, pages, longest, n, k, &p)) {
         const int g = ((n >> 4) + p - 1) / p;
@@ -824,15 +833,13 @@ extern "C" int tfl_beside_parts(int rows, int H, int C, int R, int64_t pages, in
     } else {
         least = 0.4464 * mb - 1.623 * rows + 0.6034 * x * n / 4096.0 + 0.017 * pages + 1.276 * heads - 0.279 * out;
     }
-    least *= 0.98;
-    for (int c = 3; c <= 4; ++c) {
-        const int g = c * ((n + 127) / 128), a = 256 - g;
-        if (a < 64 || a < 2 * rows) continue;
-        const double product = 22.23 * mb / g + (0.0332 * c - 0.0462) * x, attention = 2.31 + 2.568 * load(a);
-        const double t = fmax(product, attention) + 0.417 * fmin(product, attention) + 0.320 * heads + 0.163 * out + 17.15;
-        if (t < least) { least = t; best = c; *workers = a; *nsplit = 2 * a / rows < 128 ? 2 * a / rows : 128; }
-    }
-    return best;
+    const int c = four ? 4 : 3, g = c * eights, a = 256 - g;
+    if (a < 64 || a < 2 * rows) return 0;
+    const double product = 22.23 * mb / g + (0.0332 * c - 0.0462) * x, attention = 2.31 + 2.568 * load(a);
+    if (fmax(product, attention) + 0.417 * fmin(product, attention) + 0.320 * heads + 0.163 * out + 17.15 >= 0.98 * least) return 0;
+    *workers = a;
+    *nsplit = 2 * a / rows < 128 ? 2 * a / rows : 128;
+    return c;
 }
 
 // The same where nobody knows the longest row: rows half to all as long as it.

@@ -70,7 +70,8 @@ class LatentLayer:
 
     def beside(self, rows, pages, longest=None):
         """How attention and the feed-forward's half of the output product share the chip in a decode step of rows that hold ``pages`` pages in
-        all, the longest ``longest`` ((ops_latent.beside_plan, columns by carry_plan, False) or (parts_plan, 0, True)); None: one after the other, as where nobody knows the pages.  (What they hold, not what the cache could:
+        all, the longest ``longest`` ((ops_latent.beside_plan, columns by carry_plan, False) or (parts_plan, 0, True)); None: one after the other, as where nobody knows the pages.
+        Every distinct answer is a captured step of its own.  (What they hold, not what the cache could:
         for the product a CU too few costs more than a page's attention on one CU more.)"""
         g = self.geom
         if pages is None or not self.ff or not self.w_out.chunk_major or self.w_out.dtype != torch.bfloat16:

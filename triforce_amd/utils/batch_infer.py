@@ -67,7 +67,7 @@ class _DecodeBuffers:
 
 class _DecodeStep:
     """The lockstep decode forward of B sequences: eager, or captured and replayed.  How the launches share the chip may depend on how
-    many pages the sequences hold: there is a graph for each of the model's ``decode_form``s (a handful), captured when a step first asks for
+    many pages the sequences hold: there is a graph for each of the model's ``decode_form``s (five at most), captured when a step first asks for
     it, as the first one is for a new B."""
 
     def __init__(self, model, cache, B, use_graph):
