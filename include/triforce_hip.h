@@ -340,7 +340,8 @@ int tf_skinny_qkv_rope_act(const void* wqkv_packed, const void* x, int64_t xs_m,
                            void* q_out, void* k_cache, void* v_cache, int64_t stride_t, int64_t stride_h, int slot0,
                            const int32_t* slot0_dev, int M, int H, int D, int K, int rotate_k, void* stream);
 int tf_sg_tune(int key, int value);
-/* The same products for wide weights, one workgroup per CU (csrc/gemv_wide.hip): operands, rounding points and bits as above; weights packed chunk-major,
+/* The same products for wide weights, one workgroup per CU (csrc/gemv_wide.hip): operands and rounding points as above, and the same bits but for sizes whose K
+ * the panel forms cut into eight (logits and q|k|v of up to 8 192 outputs, SwiGLU of more than 16 rows with I up to 3 200).  Weights packed chunk-major,
  * [K/32][N/16][64][8], the chunks of each of 8 (mode 0) or 4 equal parts of K (rounded up to whole chunks) turned by twice the part's number: chunk o
  * of part p of n chunks lies at (o + 2 p) % n of the part.  q|k|v rows in the rotary order of tf_skinny_qkv_rope, gate and up in blocks of 8 gate |
  * 8 up rows (N = 2 I).  tf_wide_gemm_takes(mode, N, K): 1 for a size of this form, 0 for others.  mode 0: fp16 with a residual and sums of squares (no

@@ -4,11 +4,11 @@
 #include "share_shape.h"
 #include "row_source.h"
 
-// connect_kernel (hybrid_ops.hip) between two sublayers as a product's source of x: up to S streams of rows of up to 4 096.  For widths whose last products are not
-// whole panels of every CU (4 096 is, see hybrid_streams.hip, and is faster there: eight steps of four layers 3 670 -> 3 609).
-// A launch of its own is 5 us of round trips in which memory idles; here they run under the first 160 KB of weights of every CU.  One row, apart -> together:
-// 18 752 x 4 096 5.0 + 26.3 -> 28.2 us, gate | up of 22 016 5.0 + 30.5 -> 32.1; eight steps of four layers 3 831 -> 3 683.  Two rows of four streams are 160 KB
-// for every workgroup and take longer than the launch that they save (3 905 -> 3 986).
+// connect_kernel (hybrid_ops.hip) between two sublayers as a product's source of x: up to S streams of a row of up to 4 096.  It serves widths whose last products
+// are not whole panels of every CU, 2 048 to 4 064 (4 096 is, see hybrid_streams.hip).
+// A launch of its own is 5 us of round trips in which memory idles; here they run under the first 160 KB of weights of every CU.  One row, twelve layers of a parallel
+// mixer and a gated unit, four streams, a step apart -> together: width 2 048 704 -> 688 us, 2 560 863 -> 829, 3 072 1 028 -> 981, 3 584 1 218 -> 1 185; one stream of
+// 3 072 1 015 -> 970.  Two rows of four streams are 160 KB for every workgroup and take longer than the launch that they save.
 template <int S>
 struct ConnectSource {
     static constexpr bool INSIDE = true, SCALED = false, TILE = false, ALSO = false;

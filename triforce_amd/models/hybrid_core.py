@@ -1,9 +1,10 @@
 """Weights and the per-layer compute of a decoder with several residual streams and hybrid mixers (chunked attention beside a
 state-space recurrence, or gated linear attention) on the HIP ops (ops_hybrid).
 
-Decode form of a layer (one token per sequence, any number of sequences): eight launches - [streams, norm] [input projections]
-[mixer: attention splits and state updates side by side] [merge, norms, gates] [output projection] [streams, norm] [gated unit] [down]; for one
-sequence the products behind [streams, norm] make their row themselves.
+Decode form of a layer (one token per sequence, any number of sequences): [input projections] [mixer: attention splits and state updates side by side]
+[merge, norms, gates] [output projection] [gated unit] [down] and, in front of the input projections and of the gated unit, [streams, norm].  In bfloat16
+with up to four streams the two are no launches of their own where the width is 4 096, or 7 232 to 8 192 in 64s (ops_hybrid.Streams: the product in front of
+them brings the streams on, the one behind scales), nor, with one sequence, where it is 2 048 to 4 064 (ops_hybrid.Connect: the product behind makes its row).
 Prefill form: products of many rows (ops_rows) between the row kernels, the paged attention and the segmented recurrence.
 """
 import zlib
