@@ -176,3 +176,62 @@ def test_a_row_that_is_not_finite_stays_its_own():
     x[2, 7], x[4] = float("inf"), 0.0
     got = ops.linear(x, pl, out_f32=True, ln=ln, eps=EPS)
     assert torch.equal(got[[0, 1, 3]], good[[0, 1, 3]]) and bool(got[2].isnan().any()) and bool((got[4] == 0).all())
+
+
+# What the form does not have goes to the panel form, not to a library, and gives its bits; eagerly, in a captured graph, and after the weight has changed.
+CALLS = {
+    "residual": [lambda o, w, x, ln, r: o.linear(x, w, ln=ln, eps=EPS), lambda o, w, x, ln, r: o.linear(x, w, out_f32=True),
+                 lambda o, w, x, ln, r: o.linear(x, w, resid=r[:, :w.N], out=r.clone()[:, 1:w.N + 1]),
+                 lambda o, w, x, ln, r: o.linear(_beside(x), w)],
+    "logits": [lambda o, w, x, ln, r: o.linear(x, w), lambda o, w, x, ln, r: o.linear(x, w, ln=ln, eps=EPS, resid=r[:, :w.N].contiguous())],
+    "swiglu": [lambda o, w, x, ln, r: o.mlp_act(x, w), lambda o, w, x, ln, r: o.mlp_act(o.Act.from_rows(x), w).rows(),
+               lambda o, w, x, ln, r: o.mlp_act(_beside(x), w, ln=ln, eps=EPS)],
+    "qkv": [lambda o, w, x, ln, r: o.linear(x, w), lambda o, w, x, ln, r: _turned(o, w, x)],
+}
+
+
+def _beside(x):
+    """x at 8 bytes behind a boundary of 16."""
+    return torch.cat([x[:, :4], x, x[:, :4]], 1)[:, 4:-4]
+
+
+def _turned(ops, w, x):
+    H, D = w.rope
+    cos = torch.ones(64, D, device=DEV).half()
+    k, v = torch.zeros(H, 64, D, device=DEV).half(), torch.zeros(H, 64, D, device=DEV).half()
+    q = ops.qkv_rope(x, w, None, 0.0, cos, cos * 0.5, torch.arange(x.shape[0], device=DEV), k, v, 3, H, D)
+    return torch.cat([q.flatten(), k.flatten(), v.flatten()])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 7, 32])
+@pytest.mark.parametrize("use", sorted(CALLS))
+def test_other_calls_of_a_wide_weight(monkeypatch, use, M):
+    from triforce_amd import ops, ops_rows
+    monkeypatch.setattr(ops_rows, "linear", lambda *a, **k: pytest.fail("library product"))
+    monkeypatch.setattr(ops_rows, "glu_linear", lambda *a, **k: pytest.fail("product of many rows"))
+    g = torch.Generator(device=DEV).manual_seed(M)
+    kw = dict(swiglu=dict(split=2), qkv=dict(rope=(32, 128))).get(use, {})
+    N, K = {"residual": 4096, "logits": 32000, "swiglu": 22016, "qkv": 12288}[use], 4096
+    w, x, ln, r = _rnd(g, N, K, std=K ** -0.5), _rnd(g, M, K), (1 + 0.1 * torch.randn(K, generator=g, device=DEV)).half(), _rnd(g, M, N + 8)
+    for call in CALLS[use]:
+        pl, plain = ops.PackedLinear(w, wide=use, **kw), ops.PackedLinear(w, **kw)
+        assert pl.wide == use and plain.wide is None
+        want = call(ops, plain, x, ln, r)
+        for eager_first in (False, True):
+            graph = torch.cuda.CUDAGraph()
+            if eager_first:
+                assert torch.equal(call(ops, pl, x, ln, r), want)
+                assert pl.panels() is pl.panels() is not pl
+            with torch.cuda.graph(graph):
+                out = call(ops, pl, x, ln, r)
+            for _ in range(3):
+                out.zero_()
+                graph.replay()
+                assert torch.equal(out, want) and torch.equal(call(ops, pl, x, ln, r), want)
+        w.mul_(0.5)
+        pl.refresh_(), plain.refresh_()
+        want = call(ops, plain, x, ln, r)
+        graph.replay()
+        assert torch.equal(call(ops, pl, x, ln, r), want) and torch.equal(out, want)
+        w.mul_(2.0)

@@ -168,7 +168,8 @@ class PackedLinear:
     fused (2 for gate|up) — each block is packed on its own so the SwiGLU kernel can pair them.  ``rope=(H, D)``
     marks a fused q|k|v weight: a second packed copy in rotary-pair row order feeds tf_skinny_qkv_rope.
     ``wide``: what the weight is used for, where the one-workgroup-per-CU form may take it - "residual" (fp16 results, no norm), "swiglu" and "qkv"
-    (behind a norm) or "logits" (fp32) - and one copy in that form's order is all it gets if it does (``self.wide`` is None if not)."""
+    (behind a norm) or "logits" (fp32) - and one copy in that form's order is all it gets if it does (``self.wide`` is None if not), until a call comes
+    that the form does not have (``panels``)."""
 
     WIDE = {"residual": 0, "swiglu": 1, "logits": 2, "qkv": 3}
 
@@ -181,7 +182,7 @@ class PackedLinear:
         if ok and w.is_cuda:
             _ensure_sg_workspace(w.device)
         self.rope = rope
-        self.parts_n8 = self.wp_rope_n8 = None
+        self.parts_n8 = self.wp_rope_n8 = self._panels = None
         narrow = n8_applies(self.N // split, self.K) if split == 2 or rope is not None else False
         if wide == "qkv" and not (rope is not None and rope[1] % 32 == 0 and self.N == 3 * rope[0] * rope[1]):
             wide = None
@@ -209,8 +210,21 @@ class PackedLinear:
             return pack_weight_wide(self.w[rope_row_order(self.rope[0], self.rope[1], self.w.device)], 4)
         return pack_weight_wide(_gate_up_eights(self.w) if self.wide == "swiglu" else self.w, 4)
 
+    def panels(self):
+        """The weight as it is without ``wide``, for a call that the one-workgroup-per-CU form does not have; packed when the first one comes, and kept.  (While a
+        graph is captured nothing is: the graph would be what fills it.)"""
+        if self.wide is None or self._panels is not None:
+            return self._panels or self
+        made = PackedLinear(self.w, self.split, rope=self.rope)
+        if not torch.cuda.is_current_stream_capturing():
+            torch.cuda.current_stream(self.w.device).synchronize()        # (any stream may read it next)
+            self._panels = made
+        return made
+
     def refresh_(self):
         """Re-pack IN PLACE after ``self.w`` was modified in place (captured hipGraphs keep their pointers)."""
+        if self._panels is not None:
+            self._panels.refresh_()
         if self.wide is not None:
             self.parts[0].copy_(self._pack_wide())
             return self
@@ -388,6 +402,16 @@ def can_fuse_rows(rows, embed, *ws):
             and all(isinstance(w, PackedLinear) and w.parts is not None for w in ws))
 
 
+def _form_of(w, x, form, resid=None, out=None):
+    """w in the order for a call of up to SKINNY_MAX_ROWS rows: its own where the call is the one that it is packed for (``form``) and what the wide products read and
+    write in pieces is aligned, else the panels."""
+    if not isinstance(w, PackedLinear) or w.wide is None or x.shape[0] > SKINNY_MAX_ROWS or not x.is_cuda:
+        return w
+    if w.wide == form and x.data_ptr() % 16 == 0 and all(t is None or (t.data_ptr() % 8 == 0 and _lay(t)[1] % 4 == 0) for t in (resid, out)):
+        return w
+    return w.panels()
+
+
 def linear(x, w, out_f32=False, ln=None, eps=0.0, resid=None, out=None, ss_in=None, ss_out=None):
     """y = x . W^T, fp16 with fp32 accumulation — the reference's nn.Linear / F.linear.  <=32 rows against a
     PackedLinear run the hand-written weight-streaming kernel; larger blocks (prefill) go to ops_rows.linear.
@@ -398,7 +422,8 @@ def linear(x, w, out_f32=False, ln=None, eps=0.0, resid=None, out=None, ss_in=No
     x / resid / out may be ``Act`` blocks (k-octet-major); an Act input gives an Act output unless ``out`` says
     otherwise (fp32 logits are always a row-major tensor)."""
     M = x.shape[0]
-    if isinstance(w, PackedLinear) and w.wp is not None and M <= SKINNY_MAX_ROWS and x.is_cuda and (w.wide is None or (w.wide == "logits") == out_f32):
+    w = _form_of(w, x, "logits") if out_f32 else _form_of(w, x, None if ln is not None else "residual", resid, out)
+    if isinstance(w, PackedLinear) and w.wp is not None and M <= SKINNY_MAX_ROWS and x.is_cuda:
         assert x.dtype == _HALF and x.shape[1] == w.K
         if out is None:
             if out_f32 or not isinstance(x, Act):
@@ -435,8 +460,9 @@ def mlp_act(h, wgu, ln=None, eps=0.0, ss_in=None):
     RMSNorm of h folded in, ``ln``), the product of many rows with the unit in its epilogue (or GEMM + silu_mul) otherwise.
     An Act input gives an Act output."""
     M = h.shape[0]
+    wgu = _form_of(wgu, h, None if ln is None else "swiglu")
     if isinstance(wgu, PackedLinear) and wgu.parts is not None and wgu.split == 2 and M <= SKINNY_MAX_ROWS \
-            and h.is_cuda and (wgu.wide is None or ln is not None):
+            and h.is_cuda:
         I = wgu.N // 2
         act = Act.empty(M, I, h.device) if isinstance(h, Act) else torch.empty(M, I, dtype=_HALF, device=h.device)
         hp, hsm, hsk = _lay(h)
@@ -471,6 +497,7 @@ def qkv_rope(x, wqkv, ln, eps, cos, sin, positions, k_layer, v_layer, slot0, H, 
     (ln = input_layernorm weight, or None when x is already normalised; a row-major tensor or an Act); q (rows,H,D)
     is returned rotated, the k (rotated unless rotate_k is False) and v rows land in the cache at slot0+i."""
     _dev(ln, cos, sin, positions, k_layer, v_layer, slot0_dev)
+    wqkv = _form_of(wqkv, x, None if ln is None else "qkv")
     assert isinstance(wqkv, PackedLinear) and wqkv.wp_rope is not None and wqkv.rope == (H, D)
     rows = x.shape[0]
     assert x.is_cuda and x.dtype == _HALF and x.shape[1] == wqkv.K and rows <= SKINNY_MAX_ROWS
