@@ -1,5 +1,9 @@
 """The one-workgroup-per-CU products of csrc/gemv_wide.hip at the edges of their shares, against float64 with the rounding points of the path and bit for bit
 against the panel form, and the rule that picks them."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -17,6 +21,15 @@ def test_the_rule_takes_whole_shares_only_where_panels_stay_whole():
         assert takes(mode, n, k) == want, (mode, n, k)
     for bad in [(-1, 4096, 4096), (4, 4096, 4096), (0, 4100, 4096), (0, 4096, 4100), (0, 0, 4096), (0, 4096, 0)]:
         assert takes(*bad) == -22
+
+
+def test_a_line_that_was_asked_for_is_the_line():
+    """Rows from which activations are octet-major: TRIFORCE_ACT_PACKED_MIN_ROWS where it is set, upwards too, whatever form the weights have."""
+    show = "from triforce_amd import ops; print([[n for n in range(1, 40) if ops.act_packed(n, wide)][:1] for wide in (False, True)])"
+    for line, want in ((None, "[[17], [4]]"), ("33", "[[33], [33]]"), ("9", "[[9], [9]]"), ("17", "[[17], [17]]"), ("2", "[[2], [2]]")):
+        env = {k: v for k, v in os.environ.items() if not k.startswith("TRIFORCE_ACT")}
+        env.update({} if line is None else {"TRIFORCE_ACT_PACKED_MIN_ROWS": line})
+        assert subprocess.run([sys.executable, "-c", show], env=env, capture_output=True, text=True, check=True).stdout.strip() == want, line
 
 
 def _rnd(g, *shape, std=1.0):

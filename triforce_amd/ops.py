@@ -259,7 +259,7 @@ ACT_LAYOUT = _os.environ.get("TRIFORCE_ACT_LAYOUT", "auto")
 ACT_PACKED_MIN_ROWS = int(_os.environ.get("TRIFORCE_ACT_PACKED_MIN_ROWS", "17"))
 # Wide weights (csrc/gemv_wide.hip) from 4 rows: their waves read the same columns of all rows together, rows a power of two apart in the row-major
 # form.  us of a 7B layer's four products, rows -> octets: 1 row the same, 7 rows 74.4 -> 73.3, 12 rows 80.0 -> 74.7.
-ACT_PACKED_MIN_ROWS_WIDE = 4
+ACT_PACKED_MIN_ROWS_WIDE = int(_os.environ.get("TRIFORCE_ACT_PACKED_MIN_ROWS", "4"))         # (a line that was asked for is the line)
 
 
 def act_packed(rows, wide=False):
@@ -268,7 +268,7 @@ def act_packed(rows, wide=False):
         return True
     if ACT_LAYOUT == "rows":
         return False
-    return rows >= (min(ACT_PACKED_MIN_ROWS, ACT_PACKED_MIN_ROWS_WIDE) if wide else ACT_PACKED_MIN_ROWS)
+    return rows >= (ACT_PACKED_MIN_ROWS_WIDE if wide else ACT_PACKED_MIN_ROWS)
 
 
 class Act:
