@@ -15,7 +15,7 @@
 extern "C" {
 #endif
 
-int tfl_abi_version(void);
+int tfl_abi_version(void);          /* 2: as tfl_tile_abi_version 3 */
 
 /* x (fp32 residual) of one row per workgroup, in this order, each part optional:
  *   x = embed[ids]            (embed != NULL)

@@ -24,7 +24,7 @@ extern "C" {
 
 #define TFL_PAGE 64                 /* cache rows per page */
 
-int tfl_tile_abi_version(void);
+int tfl_tile_abi_version(void);     /* 3: TflGemm with n_also and also */
 
 /* Activation blocks: element (m, k) lives at m*ld + (k/8)*oct + k%8.  Row-major rows have oct = 8; decode keeps its norm output
  * and the output projection's input octet-major (ld = 8, oct = 8 * rows), where a 16-row operand is four contiguous runs. */

@@ -26,6 +26,14 @@ def test_library_exports_every_declared_symbol():
     assert lib.tf_abi_version() == hip.ABI_VERSION
 
 
+def test_a_longer_struct_is_another_version():
+    """A caller built against an older header passes a shorter TflGemm: the versions that its libraries give have to differ from those that it knows."""
+    from triforce_amd import hip
+    versions = hip.tile_lib().tfl_tile_abi_version(), hip.latent_lib().tfl_abi_version()
+    assert versions == (hip.TILE_ABI_VERSION, hip.LATENT_ABI_VERSION)
+    assert versions == {312: (3, 2), 304: (2, 1)}[ctypes.sizeof(hip.TflGemm)]          # (the shorter one ended with chunk_major)
+
+
 def test_host_side_helpers():
     from triforce_amd import hip
     lib = hip.lib()

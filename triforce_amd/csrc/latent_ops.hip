@@ -2,7 +2,7 @@
 // (norms, rotation, cache append, gelu), the per-layer token gate, and the cache-row gather.
 #include "tile_common.h"
 
-extern "C" int tfl_abi_version(void) { return 1; }
+extern "C" int tfl_abi_version(void) { return 2; }
 
 // PREP: a step's first launch, with decode_prep_row() of all rows as one more workgroup (a launch of its own is 4.3 us of a step of one row of 516).
 template <typename T, typename Y, bool PREP = false>

@@ -1,7 +1,8 @@
 // Set-up of a paged decode step on the device (no host upload while neither the sequences nor their pages change).
 #include "tile_common.h"
 
-extern "C" int tfl_tile_abi_version(void) { return 2; }
+static_assert(sizeof(TflGemm) == 312, "another struct is another version, here and in latent_ops.hip and hybrid_ops.hip");
+extern "C" int tfl_tile_abi_version(void) { return 3; }
 
 __global__ void decode_prep_kernel(int32_t* __restrict__ len, const int32_t* __restrict__ table, int table_ld, int table_cols,
                                    int32_t* __restrict__ pos, int32_t* __restrict__ slot, int32_t* __restrict__ klen, int rows) {

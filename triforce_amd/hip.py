@@ -180,7 +180,7 @@ TILE_SIGNATURES = {
     "tfl_set_pages": (_i32, [_vp, _i32, _i32, _i32, _c.POINTER(_c.c_int32), _i32, _vp]),
     "tfl_decode_prep": (_i32, [_vp, _vp, _i32, _i32, _vp, _vp, _vp, _i32, _vp]),
 }
-TILE_ABI_VERSION = 2
+TILE_ABI_VERSION = 3
 _tile = None
 
 # ---- libtriforce_latent.so (include/triforce_latent.h) ------------------------------------------------------------------
@@ -216,7 +216,7 @@ LATENT_SIGNATURES = {
     "tfl_attn_decode_beside": (_i32, [_vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _f32, _i32, _i32, _i32, _c.POINTER(TflGemm), _vp]),
     "tfl_attn_decode": (_i32, [_vp, _vp, _i32, _vp, _i32, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _vp]),
 }
-LATENT_ABI_VERSION = 1
+LATENT_ABI_VERSION = 2
 _latent = None
 
 
