@@ -49,7 +49,8 @@ int tf_abi_version(void);
  *   sk_dev   optional device int32: if non-NULL the key count is read from it at run time (lets a
  *            captured hipGraph follow a growing cache); `sk` is then the upper bound used to size
  *            the launch
- *   ws       float workspace, at least tf_attn_decode_ws_floats(H, sq, D, nsplit) floats
+ *   ws       float workspace, at least tf_attn_decode_ws_floats(H, sq, D, nsplit) floats (8-byte aligned for the one-launch merge
+ *            of tf_attn_decode_fused / _act; at another float's address they take two launches, with the same bits)
  *   nsplit   number of KV splits per head (>=1); tf_attn_decode_pick_nsplit gives a default
  * D must be 64 or 128.
  * ------------------------------------------------------------------------------------------- */

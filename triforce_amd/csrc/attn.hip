@@ -105,6 +105,9 @@ __device__ __forceinline__ f32x4 ld_agent4(const float* p) {
     return f32x4{__uint_as_float((uint32_t)a), __uint_as_float((uint32_t)(a >> 32)), __uint_as_float((uint32_t)b), __uint_as_float((uint32_t)(b >> 32))};
 }
 
+// Four neighbours at any float's address (what a caller's workspace begins at is its own business; the hardware takes dwords).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 // max over the 4 lane groups of a wave (lanes i, i^16, i^32, i^48) on the VALU: v_permlane{32,16}_swap + v_max instead of
 // two ds_bpermute round trips through the LDS queue (and their lgkmcnt(0) waits in the middle of the softmax chain).
 __device__ __forceinline__ float vmax_raw(float a, float b) {          // plain v_max_f32: no canonicalising pre-ops
@@ -533,7 +536,7 @@ __device__ __forceinline__ void attn_split_body(
                 }
                 float* to = ws_o + (pbase + qt * 16 + qq) * D + hv * DH + 4 * d4;
                 if (tickets == nullptr) {
-                    *reinterpret_cast<f32x4*>(to) = o;
+                    *reinterpret_cast<f32x4_any*>(to) = o;
                 } else {                               // one-launch form: write-through (sc1) stores, see below
                     st_agent2(to, o[0], o[1]);
                     st_agent2(to + 2, o[2], o[3]);
@@ -2192,6 +2195,7 @@ static int launch_attn(const void* q, const void* k, const void* v, void* out, i
                        int nsplit, float* ws, unsigned* tickets, hipStream_t st) {
     dim3 grid(nsplit, H), block(256);
     if (stride_t > 0x7fffffff || stride_h > 0x7fffffff) return TF_EINVAL;   // (the kernels take the two strides as 32-bit arguments)
+    if (reinterpret_cast<uintptr_t>(ws) % 8) tickets = nullptr;             // (the one-launch merge goes through ws two floats at a time; the same bits)
     // many splits on a big grid: the parallel merge kernel wins; on a small grid (few heads) the last workgroup of a head
     // folds them inside the launch (see FUSED_MERGE_BIG_SPLITS)
     if (tickets && nsplit > FUSED_MERGE_MAX_SPLITS &&
