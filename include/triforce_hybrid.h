@@ -35,7 +35,7 @@ int tfh_connect_first(const void* embed, const int64_t* ids, int vocab, const fl
 
 /* tfh_connect of rows whose next reader is a wide product, in that product's launch (bfloat16, one row of up to 4 streams of up to 4 096): every
  * workgroup makes the normed row for itself, beside the beginning of its weights.  x_out (NULL: the streams are not kept) is another block than x;
- * product->x is not read.  epilogue TFL_EPI_F32 or TFL_EPI_GLU, chunk-major weights.  TF_ERANGE: not a size of this form (nothing launched);
+ * product->x is not read.  epilogue TFL_EPI_F32 or TFL_EPI_GLU, chunk-major weights, 16-byte aligned pointers.  TF_ERANGE: not a size of this form (nothing launched);
  * tfh_connect_gemm_takes says so beforehand. */
 typedef struct TfhConnect {
     const float* y;                 /* [rows], row stride ld_y */
@@ -52,7 +52,7 @@ typedef struct TfhConnect {
 int tfh_connect_gemm_takes(int rows, int streams, int width, int n, int k, int epilogue);
 int tfh_connect_gemm(const TfhConnect* f, const TflGemm* product, int epilogue, void* stream);
 
-/* The same between two wide products of any number of rows, up to 4 streams, without a launch of its own (bfloat16, chunk-major weights).
+/* The same between two wide products of any number of rows, up to 4 streams, without a launch of its own (bfloat16, chunk-major weights, 16-byte aligned pointers).
  * tfh_streams_gemm: y = product->x . W^T of a sublayer's last product (n = width) goes into the streams (f->y is not read; f->x_out: x itself, another block, or
  *   NULL), product->out_t = u * norm_w, an activation block without the norm's scale, and product->ss_out[m*ss_ld + n/16] = sums of u^2 over each panel.
  * tfh_scaled_gemm: TFL_EPI_F32 or TFL_EPI_GLU of rows that are scaled by 1 / sqrt(sum(ss_in[m][:ss_n]) / k_real + eps) behind the product; ss_n and ss_ld in fours,

@@ -32,7 +32,7 @@ int tfl_finish_first(const void* embed, const int64_t* ids, int vocab, const flo
 
 /* tfl_finish of rows whose next reader is a wide product, in that product's launch (bfloat16, up to 2 rows of up to 4 096): every workgroup makes the normed
  * rows for itself, beside the beginning of its weights.  x_out = x + y / rms(y) * y_w [+ step] is another block than x; product->x is not read.
- * epilogue TFL_EPI_IN or TFL_EPI_F32, chunk-major weights.  TF_ERANGE: not a size of this form (nothing launched); tfl_finish_gemm_takes says so beforehand. */
+ * epilogue TFL_EPI_IN or TFL_EPI_F32, chunk-major weights, 16-byte aligned pointers.  TF_ERANGE: not a size of this form (nothing launched); tfl_finish_gemm_takes says so beforehand. */
 typedef struct TflFinish {
     const float* y;                 /* [rows], row stride ld_y */
     const float* y_w;

@@ -86,6 +86,47 @@ def test_bad_arguments_are_refused_before_any_launch():
                 assert 1 <= s <= 256 and (s == 1 or s <= math.ceil(n / 128))
 
 
+def test_rows_inside_a_product_are_read_in_pieces_of_16_bytes():
+    """The entries that make a product's rows, streams or scales refuse an address that is not one of theirs before any launch."""
+    from triforce_amd import hip
+    L, Y = hip.latent_lib(), hip.hybrid_lib()
+    at = 1 << 20
+
+    def gemm(**kw):
+        a = hip.TflGemm()
+        for key, v in dict(dict(wp=at, x=at, rows=1, n=16384, k=4096, groups=1, chunk_major=1, ld_x=8, x_oct=8, ld_f=16384, n_real=16384, ld_t=8, t_oct=8, out_f=at,
+                                out_t=at, out_t2=at, norm_w=at, ss_out=at, ss_in=at, ss_n=256, ss_ld=1024, k_real=4096, n_raw=2048, n_scaled=512), **kw).items():
+            setattr(a, key, v)
+        return ctypes.byref(a)
+
+    def rows(cls, **kw):
+        f = cls()
+        for name, kind in cls._fields_:
+            setattr(f, name, dict(ld_y=4096, width=4096, width_real=4096, streams=4, eps=1e-5, x_out=2 * at).get(name, at))
+        for key, v in kw.items():
+            setattr(f, key, v)
+        return ctypes.byref(f)
+    epi = hip.TFL_EPI
+    for off in (4, 8):
+        for key in ("y", "y_w", "step", "norm_w", "x", "x_out"):
+            assert L.tfl_finish_gemm(rows(hip.TflFinish, **{key: at + off}), gemm(), epi["f32"], None) == -22, key
+        for key in ("out_f", "out_t", "out_t2", "norm_w", "wp"):
+            assert L.tfl_finish_gemm(rows(hip.TflFinish), gemm(**{key: at + off}), epi["in"], None) == -22, key
+        for key in ("y", "norm_w", "x", "x_out"):
+            assert Y.tfh_connect_gemm(rows(hip.TfhConnect, **{key: at + off}), gemm(), epi["glu"], None) == -22, key
+        assert Y.tfh_connect_gemm(rows(hip.TfhConnect), gemm(out_t=at + off), epi["glu"], None) == -22
+        for key in ("norm_w", "x", "x_out"):
+            assert Y.tfh_streams_gemm(rows(hip.TfhConnect, **{key: at + off}), gemm(n=4096), None) == -22, key
+        for key in ("wp", "x", "out_t"):
+            assert Y.tfh_streams_gemm(rows(hip.TfhConnect), gemm(n=4096, **{key: at + off}), None) == -22, key
+        for key in ("wp", "x", "ss_in", "out_t"):
+            assert Y.tfh_scaled_gemm(gemm(**{key: at + off}), epi["glu"], None) == -22, key
+        for places in (1, 2, 5, 10):
+            args = [at, at, at, 8, 8, at, 256, at, 100, at, 4096, at, 1 << 30, 1, 4096, 256, 256, 4096, None]
+            args[{1: 0, 2: 1, 5: 2, 10: 11}[places]] += off
+            assert L.tfl_token_side(*args) == -22, places
+
+
 def test_decode_splits_by_form():
     """Two pages: one split where the merge costs more than the second page; float32 (one workgroup of 16 heads per CU): single pages only
     where they are no more rounds of 256 workgroups than pairs."""

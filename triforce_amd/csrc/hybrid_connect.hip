@@ -141,11 +141,11 @@ extern "C" int tfh_connect_gemm(const TfhConnect* pf, const TflGemm* pa, int epi
     const TfhConnect f = *pf;
     const TflGemm a = *pa;
     if (a.rows < 1 || a.groups != 1 || a.chunk_major != 1 || f.width < 4 || (f.width & 3) || f.width_real < 1 || f.width_real > f.width || f.ld_y < f.width
-        || (f.ld_y & 3) || (a.n & 15) || a.n < 16) return TF_EINVAL;
+        || (f.ld_y & 3) || (a.n & 15) || a.n < 16 || !at16(a.wp, f.y, f.norm_w, f.x, f.x_out)) return TF_EINVAL;
     if (epilogue == TFL_EPI_F32) {
         if (!a.out_f || a.n_real < 1 || a.n_real > a.n || a.ld_f < a.n_real) return TF_EINVAL;
         return connect_gemm<TFL_EPI_F32>(f, a, (hipStream_t)stream);
     }
-    if (epilogue != TFL_EPI_GLU || !a.out_t || a.ld_t < 8 || (a.ld_t & 7) || a.t_oct < 8 || (a.t_oct & 7)) return TF_EINVAL;
+    if (epilogue != TFL_EPI_GLU || !a.out_t || !at16(a.out_t) || a.ld_t < 8 || (a.ld_t & 7) || a.t_oct < 8 || (a.t_oct & 7)) return TF_EINVAL;
     return connect_gemm<TFL_EPI_GLU>(f, a, (hipStream_t)stream);
 }

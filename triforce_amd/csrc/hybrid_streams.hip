@@ -144,7 +144,8 @@ extern "C" int tfh_streams_gemm(const TfhConnect* pf, const TflGemm* pa, void* s
     const TfhConnect f = *pf;
     const TflGemm a = *pa;
     if (a.rows < 1 || a.groups != 1 || a.chunk_major != 1 || a.n != f.width || (a.n & 15) || a.n < 16 || a.k < 32 || (a.k & 31) || a.ld_x < 8 || (a.ld_x & 7) || a.x_oct < 8
-        || (a.x_oct & 7) || !a.out_t || a.ld_t < 8 || (a.ld_t & 7) || a.t_oct < 8 || (a.t_oct & 7) || !a.ss_out || a.ss_ld < a.n >> 4) return TF_EINVAL;
+        || (a.x_oct & 7) || !a.out_t || a.ld_t < 8 || (a.ld_t & 7) || a.t_oct < 8 || (a.t_oct & 7) || !a.ss_out || a.ss_ld < a.n >> 4
+        || !at16(a.wp, a.x, a.out_t, f.norm_w, f.x, f.x_out)) return TF_EINVAL;
     const int each = streams_panels(a.rows, f.streams, a.n, a.k);
     hipStream_t st = (hipStream_t)stream;
     if (each == 1) return a.rows <= 16 ? launch_streams<1, 1>(f, a, st) : launch_streams<1, 2>(f, a, st);
@@ -156,10 +157,10 @@ extern "C" int tfh_scaled_gemm(const TflGemm* pa, int epilogue, void* stream) {
     if (!pa || !pa->wp || !pa->x || !pa->ss_in) return TF_EINVAL;
     const TflGemm a = *pa;
     if (a.rows < 1 || a.groups != 1 || a.chunk_major != 1 || (a.n & 15) || a.n < 16 || a.k < 32 || (a.k & 31) || a.ld_x < 8 || (a.ld_x & 7) || a.x_oct < 8 || (a.x_oct & 7)
-        || a.ss_n < 4 || (a.ss_n & 3) || a.ss_n > 512 || a.ss_ld < a.ss_n || (a.ss_ld & 3) || a.k_real < 1) return TF_EINVAL;
+        || a.ss_n < 4 || (a.ss_n & 3) || a.ss_n > 512 || a.ss_ld < a.ss_n || (a.ss_ld & 3) || a.k_real < 1 || !at16(a.wp, a.x, a.ss_in)) return TF_EINVAL;
     if (epilogue == TFL_EPI_F32) {
         if (!a.out_f || a.n_real < 1 || a.n_real > a.n || a.ld_f < a.n_real) return TF_EINVAL;
-    } else if (epilogue != TFL_EPI_GLU || !a.out_t || a.ld_t < 8 || (a.ld_t & 7) || a.t_oct < 8 || (a.t_oct & 7)) {
+    } else if (epilogue != TFL_EPI_GLU || !a.out_t || !at16(a.out_t) || a.ld_t < 8 || (a.ld_t & 7) || a.t_oct < 8 || (a.t_oct & 7)) {
         return TF_EINVAL;
     }
     if (!tfh_scaled_gemm_takes(a.rows, a.n, epilogue)) return TF_ERANGE;

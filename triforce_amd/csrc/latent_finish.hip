@@ -124,12 +124,12 @@ extern "C" int tfl_finish_gemm(const TflFinish* pf, const TflGemm* pa, int epilo
     const TflFinish f = *pf;
     const TflGemm a = *pa;
     if (a.rows < 1 || a.groups != 1 || a.chunk_major != 1 || f.width < 4 || (f.width & 3) || f.width_real < 1 || f.width_real > f.width || f.ld_y < f.width
-        || (f.ld_y & 3) || !a.out_f || (a.n & 15) || a.n < 16) return TF_EINVAL;
+        || (f.ld_y & 3) || !a.out_f || (a.n & 15) || a.n < 16 || !at16(a.wp, f.y, f.y_w, f.step, f.norm_w, f.x, f.x_out)) return TF_EINVAL;
     if (epilogue == TFL_EPI_F32) {
         if (a.n_real < 1 || a.n_real > a.n || a.ld_f < a.n_real) return TF_EINVAL;
         return finish_gemm<TFL_EPI_F32>(f, a, (hipStream_t)stream);
     }
-    if (epilogue != TFL_EPI_IN || !a.ss_out || a.n_raw < 16 || (a.n_raw & 15) || a.n_raw > a.n || a.ld_f < a.n_raw || (a.ld_f & 3) || a.ss_ld < a.n_raw / 16
+    if (epilogue != TFL_EPI_IN || !a.ss_out || !at16(a.out_f, a.out_t, a.out_t2, a.norm_w) || a.n_raw < 16 || (a.n_raw & 15) || a.n_raw > a.n || a.ld_f < a.n_raw || (a.ld_f & 3) || a.ss_ld < a.n_raw / 16
         || a.n_scaled < 0 || (a.n_scaled & 15) || a.n_scaled > a.n_raw || (a.n_scaled && (!a.norm_w || !a.out_t2))
         || (a.n_raw < a.n && (!a.out_t || a.t_oct < 8 || (a.t_oct & 7) || (a.ld_t & 7) || a.ld_t < 8))) return TF_EINVAL;
     return finish_gemm<TFL_EPI_IN>(f, a, (hipStream_t)stream);

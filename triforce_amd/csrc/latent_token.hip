@@ -95,7 +95,7 @@ extern "C" int tfl_token_side(const void* gate_packed, const void* proj_packed, 
                               int vocab, float* out, int64_t ld_out, float* ws, int64_t ws_floats, int rows, int width, int side, int side_real, int n_real, void* stream) {
     if (!gate_packed || !proj_packed || !x || !table || !ids || !out || !ws || rows < 1 || rows > 16 || width < 32 || (width & 31) || width > (1 << 20) || side < 32 || (side & 31)
         || side > 4096 || side_real < 1 || side_real > side || n_real < 1 || n_real > width || vocab < 1 || ld_tok < side_real || ld_out < n_real || ld_x < 8 || (ld_x & 7)
-        || x_oct < 8 || (x_oct & 7) || (reinterpret_cast<uintptr_t>(x) & 15) || (reinterpret_cast<uintptr_t>(ws) & 15)) return TF_EINVAL;
+        || x_oct < 8 || (x_oct & 7) || !at16(gate_packed, proj_packed, x, ws)) return TF_EINVAL;
     if (ws_floats < tfl_token_side_ws_floats(rows, side)) return TF_ENOSPC;
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(token_parts_kernel, dim3(side / 16, PARTS), dim3(64 * WAVES), 0, st, (const bf16*)gate_packed, (const bf16*)x, ld_x, x_oct, ws, rows, side, width / 32);

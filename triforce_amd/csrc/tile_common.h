@@ -147,6 +147,10 @@ __device__ __forceinline__ void decode_prep_row(const TflDecodePrep& d, int m) {
     d.klen[m] = live ? l + 1 : 0;
     if (live) d.len[m] = l + 1;
 }
+// Addresses of what is read or written in 16-byte pieces (NULL is one).
+template <typename... P>
+static inline bool at16(P... p) { return (((uintptr_t)p | ...) & 15) == 0; }
+
 static inline bool decode_prep_ok(const TflDecodePrep* d, int rows) {
     return d && d->len && d->table && d->pos && d->slot && d->klen && d->rows == rows && d->table_cols >= 1 && d->table_ld >= d->table_cols;
 }
