@@ -361,11 +361,12 @@ static int share_gemm(const TflGemm& a, hipStream_t st) {
 template <typename T, int EPI, int P, int WAVES, int U, bool AHEAD>
 static int launch_form(const TflGemm& a, hipStream_t st) {
     const int panels = (a.n >> 4) * a.groups;
-    // Two row blocks of 16 share a workgroup's weights, and take its CU's time for twice the rows of x.  Where a few panels leave CUs idle they go to workgroups of
-    // their own, up to 64 rows.  us at 17 / 32 / 64 rows, together -> apart: TOKEN of 256 x 4 096 5.6 / 5.7 / 6.6 -> 4.6 / 4.6 / 5.3, of 1 024 x 4 096 7.3 / 7.9 / 7.7 -> 6.3 / 6.6 / 6.6,
-    // of 256 x 8 192 8.3 / 9.8 / 12.1 -> 6.5 / 7.5 / 8.9; GATED of 256 panels, eight steps of six layer runs, 32 rows 6 519 -> 6 508.  QUERY of 384 panels is slower
-    // for it (6 519 -> 6 578), LATENT of 1 024 too (6 571).
-    const bool apart = a.rows <= 64 && ((EPI == TFL_EPI_TOKEN && panels <= 64) || (EPI == TFL_EPI_GATED && panels <= 256));
+    // Two row blocks of 16 share a workgroup's weights, and take its CU's time for twice the rows of x.  Up to 64 rows they go to workgroups of their own as long as
+    // there is a CU for each.  us, bfloat16 | float32, together -> apart: TOKEN at 17 / 32 / 64 rows, 256 x 4 096 7.1 / 7.6 / 7.4 -> 6.0 / 6.3 / 6.1 | 23.1 / 23.7 / 21.3 -> 11.9 /
+    // 12.9 / 12.1, 256 x 8 192 11.7 / 13.8 / 12.8 -> 9.0 / 9.7 / 9.3; GATED of 64 panels 3.5 / 3.8 / 3.8 -> 3.4 / 3.4 / 3.4 | 5.4 / 5.9 / 5.6 -> 4.4 / 4.4 / 4.3, of 128 at 17 / 32 rows
+    // 3.6 / 3.9 -> 3.5 / 3.5 | 5.6 / 6.0 -> 4.5 / 4.6.  With fewer CUs than workgroups GATED is slower for it: 128 panels at 33 / 64 rows 3.9 / 4.0 -> 5.4 / 5.4 | 5.6 / 5.9 -> 6.1 / 6.7,
+    // 256 at 17 / 64 3.7 / 6.1 -> 3.7 / 6.2 | 6.1 / 12.0 -> 7.0 / 15.0.  QUERY of 384 panels and LATENT of 1 024 too (befidra decode 32 6 519 -> 6 578, 6 571).
+    const bool apart = a.rows <= 64 && ((EPI == TFL_EPI_TOKEN && panels <= 64) || (EPI == TFL_EPI_GATED && panels * ((a.rows + 15) / 16) <= 256));
     const int mt = a.rows <= 16 || apart ? 1 : 2, rb = (a.rows + 16 * mt - 1) / (16 * mt);
     const int extra = EPI == TFL_EPI_QUERY && a.kv_raw ? (a.rows + rb - 1) / rb : 0;
     const dim3 grid((panels + P - 1) / P + extra, rb), block(64 * WAVES);
