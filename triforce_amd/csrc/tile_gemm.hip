@@ -125,6 +125,11 @@ __device__ __forceinline__ void latent_gemm_body(const TflGemm& a, const int tid
         }
         asm volatile("" ::: "memory");
     }
+    // float32: where the loads of a batch stand is no longer the scheduler's choice, which put those of its second operand behind the first one's products and
+    // changed with the code around (up to 20 % either way).  One row block: the next weights in front of this batch's products too, two: among them.  us at 1 /
+    // 16 / 17 / 32 rows, scheduled -> so: 4 096 x 15 104 61.4 / 64.7 / 88.9 / 93.7 -> 45.9 / 54.9 / 60.6 / 66.1, 17 216 x 4 096 63.8 / 81.3 / 94.8 / 111.5 -> 63.1 / 76.2 / 83.6 / 92.1,
+    // gate | up of 4 096 x 4 096 19.3 / 20.2 / 26.7 / 27.9 -> 16.5 / 19.2 / 19.2 / 20.2.  (LATENT, a chunk or two a wave, is slower for either: 32 rows 8.8 -> 9.4.)
+    constexpr bool HOLD = AHEAD && sizeof(T) == 4 && EPI != TFL_EPI_LATENT;
     if (c_beg < c_end) {
         Frag w[P][U], wn[P][U];
         load_w(w, c_beg);
@@ -136,7 +141,9 @@ __device__ __forceinline__ void latent_gemm_body(const TflGemm& a, const int tid
 #pragma unroll
                     for (int t = 0; t < MT; ++t) x[u][t] = load_frag((const T*)a.x + xoff[t] + xstep * min(c0 + u, last));
                 }
+            if constexpr (HOLD && MT > 1) __builtin_amdgcn_sched_barrier(0);
             if constexpr (AHEAD) load_w(wn, c0 + U);
+            if constexpr (HOLD && MT == 1) __builtin_amdgcn_sched_barrier(0);
             if constexpr (EPI == TFL_EPI_QUERY) {
                 if (c0 == c_beg) second();
             }
