@@ -329,7 +329,7 @@ static int launch_share_rows(const TflGemm& a, int tail_rows, int tail_per, hipS
 
 template <typename T, int EPI, int P, bool TAIL>
 static int launch_share(const TflGemm& a, int tail_rows, int tail_per, hipStream_t st) {
-    if constexpr (EPI == TFL_EPI_RESIDUAL) {                  // (forms of their own: asked about in these, one row, six layer runs, eight steps 4 134 -> 4 162 us)
+    if constexpr (EPI == TFL_EPI_RESIDUAL && sizeof(T) == 2) { // (forms of their own: asked about in these, one row, six layer runs, eight steps 4 134 -> 4 162 us)
         if (a.n_also > 0) return launch_share_rows<T, EPI, P, TAIL, 2, FromMemoryAlso>(a, tail_rows, tail_per, st);
     }
     return a.rows <= 16 ? launch_share_rows<T, EPI, P, TAIL, 1>(a, tail_rows, tail_per, st)
@@ -447,7 +447,7 @@ static int check_gemm(const TflGemm& a, int dtype, int epi) {
             if (!a.out_t || !a.gate || a.ld_t < 8 || a.ld_gate < (int64_t)a.groups * a.n || (a.ld_t & 7) || (a.ld_gate & 3)) return TF_EINVAL;
             break;
         case TFL_EPI_RESIDUAL:
-            if (a.n_also < 0 || a.n_also > 4 || (a.n_also && (a.rows <= 16 || !a.also || !a.chunk_major || share_shape(a.n >> 4, false, 0, a.rows).each == 0))) return TF_EINVAL;
+            if (a.n_also < 0 || a.n_also > 4 || (a.n_also && (a.rows <= 16 || !a.also || !at16(a.also) || !a.chunk_major || share_shape(a.n >> 4, false, 0, a.rows).each == 0))) return TF_EINVAL;
             if (!a.out_f || a.groups != 1 || a.ld_f < a.n || (a.ld_f & 3) || (a.out_t && (a.ld_t < 8 || (a.ld_t & 7)))) return TF_EINVAL;
             break;
         case TFL_EPI_TOKEN:
