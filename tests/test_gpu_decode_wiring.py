@@ -74,7 +74,7 @@ def test_decode_steps(made, monkeypatch, name, rows):
     monkeypatch.setattr(oh.Streams, "takes", staticmethod(lambda *a: False))
     monkeypatch.setattr(oh.Connect, "takes", staticmethod(lambda *a: False))
     monkeypatch.setattr(ol.Finish, "takes", staticmethod(lambda *a: False))
-    monkeypatch.setattr(ol, "TOKEN_SIDE_ROWS", 0)
+    monkeypatch.setattr(ol, "token_side_pays", lambda *a: False)
     apart = _steps(model, prompts, then, False)
     worst = 0.0
     with torch.device("cuda"):

@@ -10,8 +10,9 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("rows", [1, 2, 7, 10, 11, 16])
 @pytest.mark.parametrize("width,real", [(4096, 4096), (192, 180), (2080, 2080), (8224, 8223)])
 @pytest.mark.parametrize("side,side_real", [(32, 20), (64, 64), (256, 256), (256, 250), (544, 544)])
-def test_token_side(rows, width, real, side, side_real):
+def test_token_side(monkeypatch, rows, width, real, side, side_real):
     from triforce_amd import ops_latent as ol, ops_tile as ot
+    monkeypatch.setattr(ol, "token_side_pays", lambda *a: rows <= 10)      # (the kernels at all of these, not only where they are the faster way)
     g = torch.Generator(device=DEV).manual_seed(rows * width + side)
 
     def rnd(*shape, std=1.0):

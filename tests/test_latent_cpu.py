@@ -127,6 +127,15 @@ def test_rows_inside_a_product_are_read_in_pieces_of_16_bytes():
             assert L.tfl_token_side(*args) == -22, places
 
 
+def test_large_sides_stay_panels():
+    """Where it was measured the slower way, and more than the kernel takes: any side of a model's configuration is one."""
+    from triforce_amd import ops_latent as ol
+    for rows, width, side, want in ((1, 4096, 256, True), (10, 4096, 256, True), (11, 4096, 256, False), (1, 4096, 512, False), (1, 8192, 512, False), (10, 8192, 256, True),
+                                    (4, 6144, 256, True), (8, 6144, 256, False), (1, 2048, 256, False), (10, 2048, 128, True), (4, 1024, 128, True), (8, 1024, 128, False),
+                                    (10, 1024, 64, True), (1, 2048, 1024, False), (1, 2048, 4128, False)):
+        assert ol.token_side_pays(rows, width, side) == want, (rows, width, side)
+
+
 def test_decode_splits_by_form():
     """Two pages: one split where the merge costs more than the second page; float32 (one workgroup of 16 heads per CU): single pages only
     where they are no more rounds of 256 workgroups than pairs."""

@@ -144,15 +144,25 @@ def token_gate_linear(x, wt, table, ids, n_real):
     return out
 
 
-# Every workgroup of the projection reads all parts of all rows: us of eight steps of six layer runs, panels -> parts, 1 row 4 296 -> 4 187, 2 4 506 ->
-# 4 420, 4 4 768 -> 4 674, 8 4 968 -> 4 925, 12 the same, 16 5 378 -> 5 402.
 TOKEN_SIDE_ROWS = 10
+
+
+def token_side_pays(rows, width, side):
+    """Is the gate's K cut over the grid the faster way?  Every workgroup of the projection then reads all parts of all rows, which has to be little beside what the gate
+    gains by more CUs.  us of the two launches, panels -> parts, at 1 / 4 / 10 rows: side 64 of 1 024 6.3 / 6.3 / 6.3 -> 5.6 / 5.8 / 6.2, of 4 096 8.4 / 8.4 / 8.9 -> 6.2 / 6.4 / 6.6;
+    128 of 1 024 6.4 / 6.7 / 6.8* -> 6.0 / 6.4 / 7.2, of 8 192 11.9 / 12.1 / 13.2 -> 7.8 / 8.6 / 10.2; 256 of 2 048 7.6* / 7.9* / 8.2* -> 7.2 / 8.0 / 9.5, of 4 096 9.1 / 9.4 / 9.9 ->
+    7.4 / 8.2 / 9.7, of 6 144 11.8 / 12.2 / 13.1* -> 9.5 / 11.2 / 14.2; 512 of 4 096 9.4* / 9.7* / 10.2* -> 9.6 / 10.9 / 13.9, 1 024 10.4* / 10.7* / 11.0* -> 15.2 / 16.8 / 24.0 (*: stays
+    panels).  Eight steps of six layer runs, side 256 of 4 096, 1 row 4 296 -> 4 187, 8 4 968 -> 4 925, 12 the same, 16 5 378 -> 5 402."""
+    if rows > TOKEN_SIDE_ROWS or side > 256 or (side > 128 and width < 4096):
+        return False
+    rounds = 1 if width <= 4096 or width % 4096 == 0 else 2          # (of the projection's workgroups over the CUs, and one that is half empty)
+    return 8 * rows * side * rounds <= 5 * width
 
 
 def token_side(x, gate, proj, table, ids, n_real, width):
     """linear_f32(token_gate_linear(x, gate, table, ids, n_real), proj, width), for a few rows of bfloat16 with the gate's K cut over the grid (tfl_token_side)."""
     rows, k, ld, octet = _lay(x)
-    if x.dtype != torch.bfloat16 or rows > TOKEN_SIDE_ROWS or proj.chunk_major or gate.chunk_major:
+    if x.dtype != torch.bfloat16 or not token_side_pays(rows, k, gate.n) or proj.chunk_major or gate.chunk_major:
         return linear_f32(token_gate_linear(x, gate, table, ids, n_real), proj, width)
     _need(x, table, ids)
     assert ids.dtype == torch.int64 and ids.numel() == rows and k == gate.k == proj.n and gate.n == proj.k and x.dtype == table.dtype == gate.dtype == proj.dtype
