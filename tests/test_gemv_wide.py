@@ -14,10 +14,12 @@ EPS = 1e-5
 def test_the_rule_takes_whole_shares_only_where_panels_stay_whole():
     from triforce_amd import hip
     takes = hip.lib().tf_wide_gemm_takes
-    for mode, n, k, want in [(0, 4096, 4096, 1), (0, 4096, 11008, 1), (0, 8192, 2048, 1), (0, 5120, 5120, 0), (0, 5120, 13824, 0), (0, 7168, 2048, 1),
-                             (0, 7152, 2048, 0), (0, 4080, 4096, 0), (0, 4096, 2016, 0), (3, 12288, 4096, 1), (3, 15360, 5120, 1), (3, 9216, 4096, 0),
-                             (1, 22016, 4096, 1), (1, 27648, 5120, 1), (1, 4352, 4096, 1), (2, 32000, 4096, 1), (2, 32768, 4096, 1), (2, 33024, 4096, 0),
-                             (2, 32000, 768, 0), (1, 5504, 4096, 1)]:
+    for mode, n, k, want in [(0, 4096, 4096, 1), (0, 4096, 11008, 1), (0, 8192, 2048, 1), (0, 5120, 5120, 0), (0, 5120, 13824, 0), (0, 7168, 7168, 1),
+                             (0, 7152, 7168, 0), (0, 7168, 4096, 0), (0, 7680, 4096, 0), (0, 8192, 2560, 1), (0, 4080, 4096, 0), (0, 4096, 2016, 0),
+                             (3, 12288, 4096, 1), (3, 15360, 5120, 1), (3, 9216, 4096, 0),
+                             (1, 22016, 4096, 1), (1, 27648, 5120, 1), (1, 4352, 4096, 0), (1, 8176, 4096, 0), (1, 8192, 2048, 1), (2, 4352, 4096, 0), (2, 5136, 4096, 1), (2, 4096, 4096, 1),
+                             (2, 32000, 4096, 1), (2, 32768, 4096, 1), (2, 33024, 4096, 0),
+                             (2, 32000, 768, 0), (1, 5504, 4096, 0)]:
         assert takes(mode, n, k) == want, (mode, n, k)
     for bad in [(-1, 4096, 4096), (4, 4096, 4096), (0, 4100, 4096), (0, 4096, 4100), (0, 0, 4096), (0, 4096, 0)]:
         assert takes(*bad) == -22
@@ -78,6 +80,7 @@ ROWS_K = [(1, 2048), (7, 4128), (16, 2080), (17, 2048), (32, 4096)]
 @pytest.mark.parametrize("packed", [False, True])
 def test_residual(M, K, N, packed):
     from triforce_amd import ops
+    K += 5120 if N == 7168 else 0                              # (a part of the CUs: from 7 168 on)
     g = torch.Generator(device=DEV).manual_seed(N + M)
     w, x, res = _rnd(g, N, K, std=K ** -0.5), _rnd(g, M, K), _rnd(g, M, N)
     pl = ops.PackedLinear(w, wide="residual")
@@ -100,7 +103,7 @@ def test_residual(M, K, N, packed):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K", ROWS_K)
 # pairs of panels: one workgroup's rest of 4 rows (ragged), whole shares, rests of 8 (full and ragged), a share of one more on fewer CUs, the widest
-@pytest.mark.parametrize("I", [2096, 4096, 5120, 11008, 13824, 16384])
+@pytest.mark.parametrize("I", [4120, 4096, 5120, 11008, 13824, 16384])
 def test_swiglu(M, K, I):
     from triforce_amd import ops
     g = torch.Generator(device=DEV).manual_seed(I + M)
@@ -122,7 +125,7 @@ def test_swiglu(M, K, I):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K", ROWS_K)
-@pytest.mark.parametrize("N", [4096, 4112, 9984, 21504, 32000, 32768])        # whole shares, rests of 4 and 12 rows, a share of one more, the widest
+@pytest.mark.parametrize("N", [4096, 5136, 8208, 9984, 21504, 32000, 32768])  # whole shares, rests of 8 beside one panel, 4 and 12 rows, a share of one more, the widest
 def test_logits(M, K, N):
     from triforce_amd import ops
     g = torch.Generator(device=DEV).manual_seed(N + M)

@@ -278,16 +278,25 @@ struct WideArgs {
 };
 
 // The shape of a product in this form; each == 0: gemv.hip's.  Rotation and sums of squares come in whole panels: there a share of a panel more is taken
-// where it leaves no more than an eighth of the CUs without work.
+// where it leaves no more than an eighth of the CUs without work.  Which form a weight has is settled when it is packed, for all rows, so the sizes that are slower
+// at few of them stay panels; us, panels -> here, at 1 / 2 / 7 / 17 rows:
+//   gate | up below two panels a CU: 4 352 x 2 048 7.6 / 7.7 / 8.0 / 9.5 -> 8.8 / 8.9 / 8.8 / 10.7, 5 120 x 4 096 11.9 / 12.0 / 12.3 / 15.0 -> 11.7 / 11.7 / 12.0 / 14.9 (32 rows
+//     15.6 -> 15.9), 6 144 x 2 048 8.2 / 8.2 / 8.6 / 9.9 -> 8.3 / 8.3 / 8.4 / 10.1; from there on 8 192 x 2 048 9.3 / 9.0 / 9.3 / 11.3 -> 9.1 / 9.1 / 9.1 / 10.5;
+//   logits with one panel and up to four rows: 4 352 x 2 048 8.0 / 8.0 / 8.5 / 12.9 -> 8.6 / 8.6 / 8.4 / 10.3; 5 120 x 2 048 is 8.2 / 8.2 / 8.7 / 13.1 -> 7.4 / 7.4 / 7.5 / 9.4;
+//   o and down on a part of the CUs over a short K: 7 424 x 2 560 8.9 / 8.6 / 9.8 / 11.2 -> 9.1 / 9.2 / 9.3 / 10.0, 7 168 x 4 096 12.2 / 11.7 / 12.6 / 14.6 -> 12.0 / 12.1 / 12.1 / 12.5;
+//     7 168 x 7 168 is 19.3 / 18.3 / 20.2 / 23.8 -> 18.5 / 18.5 / 18.3 / 19.7, 7 680 x 7 680 22.5 / 21.9 / 22.9 / 26.3 -> 20.2 / 20.1 / 20.0 / 20.9.
+// Taken although slower at up to four rows, beside gate | up of the same layer: q|k|v 15 360 x 5 120 26.3 / 26.6 / 27.3 / 32.1 -> 27.2 / 27.4 / 26.8 / 29.6 (27 648 x 5 120 49.6 /
+// 48.1 / 48.6 / 51.8 -> 45.5 / 44.6 / 43.6 / 45.5).
 static ShareShape wide_shape(int mode, int N, int K) {
     if (K < 2048 || K > (1 << 20) || (K % 32) || N < 4096 || (N % 16) || N > (1 << 20)) return {0, 0, 0};
     const int panels = N / 16;
-    ShareShape s = share_shape(panels, mode == SG_GATEUP, 0, 32);
     if (mode == SG_PLAIN || mode == SG_QKV) {
         const int each = (panels + 255) / 256;
-        s = each <= (mode == SG_QKV ? 6 : 2) && panels * 8 >= each * 256 * 7 ? ShareShape{each, 0, 0} : ShareShape{0, 0, 0};
+        if (mode == SG_PLAIN && panels != each * 256 && K < 7168) return {0, 0, 0};
+        return each <= (mode == SG_QKV ? 6 : 2) && panels * 8 >= each * 256 * 7 ? ShareShape{each, 0, 0} : ShareShape{0, 0, 0};
     }
-    return s;
+    const ShareShape s = share_shape(panels, mode == SG_GATEUP, 0, 32);
+    return (mode == SG_GATEUP && panels < 512) || (s.each == 1 && s.rest == 4) ? ShareShape{0, 0, 0} : s;
 }
 
 template <int MODE, bool NORM, int P, bool TAIL, int MT>
@@ -324,8 +333,11 @@ static int wide(const WideArgs& a, hipStream_t st) {
     } else if constexpr (MODE == SG_QKV) {
         switch (f.each) { WIDE(1); WIDE(2); WIDE(3); WIDE(4); WIDE(5); WIDE(6); }
     } else {
-        if (f.rest) switch (f.each) { WIDE_TAIL(1); WIDE_TAIL(2); WIDE_TAIL(3); WIDE_TAIL(4); WIDE_TAIL(5); WIDE_TAIL(6); WIDE_TAIL(7); }
-        else switch (f.each) { WIDE(1); WIDE(2); WIDE(3); WIDE(4); WIDE(5); WIDE(6); WIDE(7); WIDE(8); }
+        if constexpr (MODE == SG_F32) {
+            if (f.each == 1) return f.rest ? launch_wide<MODE, NORM, 1, true>(a, f, st) : launch_wide<MODE, NORM, 1, false>(a, f, st);
+        }
+        if (f.rest) switch (f.each) { WIDE_TAIL(2); WIDE_TAIL(3); WIDE_TAIL(4); WIDE_TAIL(5); WIDE_TAIL(6); WIDE_TAIL(7); }
+        else switch (f.each) { WIDE(2); WIDE(3); WIDE(4); WIDE(5); WIDE(6); WIDE(7); WIDE(8); }
     }
 #undef WIDE
 #undef WIDE_TAIL
