@@ -103,7 +103,7 @@ def test_residual(M, K, N, packed):
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,K", ROWS_K)
 # pairs of panels: one workgroup's rest of 4 rows (ragged), whole shares, rests of 8 (full and ragged), a share of one more on fewer CUs, the widest
-@pytest.mark.parametrize("I", [4120, 4096, 5120, 11008, 13824, 16384])
+@pytest.mark.parametrize("I", [4128, 4096, 5120, 11008, 13824, 16384])
 def test_swiglu(M, K, I):
     from triforce_amd import ops
     g = torch.Generator(device=DEV).manual_seed(I + M)
